@@ -1,10 +1,11 @@
 // Matrix products of the projections: Y[M, N] = X[M, K] * W[N, K]^T, the weight
 // in the checkpoint's [out, in] orientation (K contiguous in both operands).
 //
-// gemm_ordered_kernel is the 32-bit path: operands of either storage type are
-// widened exactly, every output element is one fused-multiply-add chain over
-// ascending k that starts at +0, as in the reference's kernels
-// (/root/reference/crates/nnis-kernels/src/gemm.rs:16-64, gemv.rs:45-62), so a
+// gemm_ordered_kernel takes any sizes and types (32-bit products whose rows can be
+// loaded 16 bytes at a time run on the matrix cores, gemm_f32.hip): operands of
+// either storage type are widened exactly, every output element is one
+// fused-multiply-add chain over ascending k that starts at +0, as in the
+// reference's kernels (/root/reference/crates/nnis-kernels/src/gemm.rs:16-64, gemv.rs:45-62), so a
 // row's result depends neither on the other rows nor on where the tile lies.
 #include "common.h"
 

@@ -50,6 +50,7 @@ _CORE_SIGNATURES = {
     "nnis_argmax": [_VOID, _VOID, _INT, _INT, _VOID, _VOID],
     "nnis_argmax_scratch": [_INT, _INT],
     "nnis_argmax_static": [_VOID, _VOID, _INT, _INT, _VOID],
+    "nnis_gemm_f32": [_VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_ordered": [_VOID, _INT, _VOID, _INT, _VOID, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_bf16": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID, _SIZE, _VOID],
     "nnis_gemm_fused": [_VOID, _VOID, _VOID, _VOID, _INT, _FLT, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT,
@@ -567,6 +568,29 @@ def gemm_ordered(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
     lib = core()
     _check(lib, lib.nnis_gemm_ordered(x.data_ptr(), _code(x), w.data_ptr(), _code(w), out.data_ptr(), _code(out), m, n, k,
                                       _stream()))
+    return out
+
+
+GEMM_F32_VARIANTS = 16  # kHints of csrc/gemm_f32.hip
+
+
+def gemm_f32_takes(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """Whether ``gemm_f32`` takes this product: 32-bit weights in the checkpoint's order whose rows, and those of x, can
+    be loaded 16 bytes (four channels) at a time."""
+    return w.dtype == torch.float32 and w.shape[1] % 4 == 0 and not (x.data_ptr() | w.data_ptr() | out.data_ptr()) & 15
+
+
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, variant: int = -1) -> torch.Tensor:
+    """out[M, N] = x[M, K] @ w[N, K]^T on the matrix cores in 32 bits: w float32, x and out float32 or bfloat16 (x
+    widened exactly), K a multiple of 4, operands on 16-byte boundaries.  ``variant``: one of the kernel's forms
+    (-1: chosen by the sizes)."""
+    _dev(x, "x"), _dev(w, "weight"), _dev(out, "out")
+    m, k = x.shape
+    n = w.shape[0]
+    if w.dtype != torch.float32 or w.shape[1] != k or out.shape != (m, n):
+        raise KernelError(f"gemm_f32: x {tuple(x.shape)} w {tuple(w.shape)} {w.dtype} out {tuple(out.shape)} do not fit")
+    lib = core()
+    _check(lib, lib.nnis_gemm_f32(x.data_ptr(), _code(x), w.data_ptr(), out.data_ptr(), _code(out), m, n, k, int(variant), _stream()))
     return out
 
 
@@ -1135,12 +1159,14 @@ def unit_rows(device) -> torch.Tensor:
 
 def linear(x: torch.Tensor, weight, out: torch.Tensor) -> torch.Tensor:
     """out = x @ weight^T.  A packed weight (bfloat16) takes the matrix-core
-    kernels; a weight as the checkpoint has it (32-bit, or a width the 16-byte
-    loads cannot take) the ordered 32-bit product."""
+    kernels, a 32-bit weight those for 32-bit operands; a weight of a width
+    the 16-byte loads cannot take the ordered 32-bit product."""
     if isinstance(weight, PackedWeight):
         if x.dtype != torch.bfloat16 or x.data_ptr() % 16 != 0 or out.data_ptr() % 16 != 0:
             raise KernelError(f"linear: a packed weight multiplies bfloat16 rows on 16-byte boundaries, got {x.dtype}")
         return gemm_bf16(x, weight, out)
+    if gemm_f32_takes(x, weight, out):
+        return gemm_f32(x, weight, out)
     return gemm_ordered(x, weight, out)
 
 

@@ -1,6 +1,6 @@
 """A projection y = W x with the checkpoint's [out, in] weight and no bias
 (/root/reference/crates/nnis-model/src/runtime.rs:402-426).  The kernel is
-chosen by the types at hand: a 32-bit weight takes the ordered 32-bit product;
+chosen by the types at hand: a 32-bit weight takes the 32-bit products;
 a bfloat16 weight is packed once, when it is bound, into the order the
 matrix-core kernels read, and takes those.
 """
@@ -16,8 +16,7 @@ class Projection:
     def __init__(self, weight: torch.Tensor, rt=None):
         """``rt``: the runtime the projection will run under; with a bfloat16
         one, a bfloat16 weight is kept packed only (the checkpoint's order is
-        dropped).  Without it the weight stays as it is and takes the ordered
-        product."""
+        dropped).  Without it the weight stays as it is."""
         if weight.dim() != 2:
             raise ValueError(f"a projection weight is a matrix, got shape {tuple(weight.shape)}")
         self.out_features, self.in_features = weight.shape

@@ -12,7 +12,8 @@ nothing narrows unless the caller asks for it: ``narrow_to_bfloat16`` rounds
 32-bit tensors to bfloat16 (nearest, ties to even) as they are loaded, so that
 a 32-bit checkpoint under a bfloat16 runtime runs on the matrix cores.  Without
 it such a checkpoint keeps its 32-bit weights and every projection takes the
-ordered 32-bit product, much slower; the loader says so in one line.  A table
+32-bit products, which read twice the bytes and multiply at a sixteenth of the
+rate; the loader says so in one line.  A table
 of integers (a part declares it so) is kept as int32 on either path.
 Everything wrong with a folder is reported in one error: missing tensors,
 tensors nobody asked for, wrong shapes, unsupported stored types
@@ -179,6 +180,6 @@ def load_weights(model_dir: str, specs: Sequence[TensorSpec], device, widen_to_f
         handle.close()
     if kept_wide:
         print(f"[nnis_amd] {model_dir}: {kept_wide} tensors are stored in 32-bit and stay so; under bfloat16 their products "
-              "take the ordered 32-bit kernel (slow).  narrow_to_bfloat16 / --narrow-to-bfloat16 rounds them at load.",
+              "take the 32-bit kernels (slow).  narrow_to_bfloat16 / --narrow-to-bfloat16 rounds them at load.",
               file=sys.stderr, flush=True)
     return out

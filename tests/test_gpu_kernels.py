@@ -82,6 +82,51 @@ def test_gemm_ordered(m, n, k, x_dtype, w_dtype, y_dtype):
         assert torch.equal(alone[0], y[m - 1])
 
 
+@pytest.mark.parametrize("variant", range(-1, 16))
+@pytest.mark.parametrize("m, n, k", [(1, 1, 4), (8, 40, 52), (7, 130, 548), (17, 33, 100), (65, 130, 176), (131, 257, 612), (5, 17, 2052)])
+def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
+    """Every form of the product at sizes with tails in every dimension (K a multiple of 4 and of nothing more), against 64
+    bits: a sum of k products in chains is off by at most k roundings of the sum of magnitudes, sqrt(k) where they are
+    as random as here."""
+    ops = _ops()
+    if variant == 13 and m > 8:
+        with pytest.raises(KernelError, match="no variant"):
+            ops.gemm_f32(torch.zeros(m, k, device="cuda"), torch.zeros(n, k, device="cuda"), torch.zeros(m, n, device="cuda"), variant)
+        return
+    torch.manual_seed(m + n + k)
+    x, w = torch.randn(m, k), torch.randn(n, k)
+    want, scale = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    y = torch.full((m + 1, n), 7.0, device="cuda")
+    ops.gemm_f32(x.cuda(), w.cuda(), y[:m], variant)
+    assert ((y[:m].cpu().double() - want).abs() <= 2e-7 * math.sqrt(k) * scale).all() and (y[m] == 7).all()
+    if 4 <= variant <= 12:
+        return  # tiles take 32-bit rows
+    x = x.bfloat16()
+    for dtype, tol in ((torch.float32, 2e-7 * math.sqrt(k)), (torch.bfloat16, 4e-3)):
+        y = torch.empty(m, n, dtype=dtype, device="cuda")
+        ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
+        assert ((y.cpu().double() - x.double() @ w.double().t()).abs() <= tol * (x.double().abs() @ w.double().abs().t())).all()
+
+
+def test_a_32_bit_product_whose_rows_cannot_be_loaded_16_bytes_at_a_time_takes_the_ordered_kernel():
+    ops = _ops()
+    w = torch.randn(24, 36, device="cuda")
+    for x, weight in ((torch.randn(5, 34, device="cuda"), w.flatten()[:24 * 34].view(24, 34)),  # a width that is no multiple of 4
+                      (torch.randn(5 * 36 + 1, device="cuda")[1:].view(5, 36), w)):  # rows on no 16-byte boundary
+        y, ordered = torch.empty(5, 24, device="cuda"), torch.empty(5, 24, device="cuda")
+        assert not ops.gemm_f32_takes(x, weight, y)
+        ops.linear(x, weight, y)
+        assert torch.equal(y, ops.gemm_ordered(x, weight, ordered))
+        with pytest.raises(KernelError):
+            ops.gemm_f32(x, weight, y)
+    for count in (5, 70):  # the last chunk's lanes beyond K count as zeros whatever the row begins with
+        x = torch.randn(count, 36, device="cuda")
+        x[2, 0] = float("inf")
+        y = torch.empty(count, 24, device="cuda")
+        ops.linear(x, w, y)
+        assert torch.isfinite(y[[0, 1, 3, 4]]).all() and torch.isinf(y[2]).all()
+
+
 @pytest.mark.parametrize("m", [1, 8, 16, 17, 40, 64, 65, 130, 300])
 @pytest.mark.parametrize("n, k", [(576, 576), (960, 576), (1000, 96), (70, 176), (3072, 64), (64, 1536), (17, 8), (200, 1096),
                                   (2050, 2312)])  # the last: large weights, few columns -- K is cut among blocks beyond 16 tokens
