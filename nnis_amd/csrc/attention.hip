@@ -1497,6 +1497,8 @@ __global__ void attention_combine_kernel(const float* __restrict__ partial, bf16
   }
 }
 
+#include "attention_f32.h"
+
 #endif  // NNIS_MATRIX_CORES
 
 }  // namespace
@@ -1515,13 +1517,11 @@ static int fill_terms(NnisHeadTerms& into, const NnisHeadTerms* terms, int heads
   return 0;
 }
 
-extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, int out_dtype, const void* k_pages,
-                                          const void* v_pages, int cache_dtype, const int* block_table, int max_pages,
-                                          const int* tok_slot, const int* tok_pos, int tokens, int heads, int kv_heads,
-                                          int head_dim, int window, float scale, int value_dim, float softcap, int keep_first,
-                                          const float* bias, int reach, const float* sink, const void* pool_k,
-                                          const void* pool_v, const int* pool_table, int pool_max_pages, int pool,
-                                          const NnisHeadTerms* terms, void* stream) {
+static int fill_args(AttnArgs& a, const void* q, int q_dtype, void* out, int out_dtype, const void* k_pages, const void* v_pages,
+                     int cache_dtype, const int* block_table, int max_pages, const int* tok_slot, const int* tok_pos, int tokens, int heads,
+                     int kv_heads, int head_dim, int window, float scale, int value_dim, float softcap, int keep_first,
+                     const float* bias, int reach, const float* sink, const void* pool_k, const void* pool_v, const int* pool_table,
+                     int pool_max_pages, int pool, const NnisHeadTerms* terms) {
   NNIS_REQUIRE(pool >= 0 && (pool == 0 || (window > 0 && pool_k && pool_v && pool_table && pool_max_pages > 0)),
                "attention: pooled blocks (%d tokens each) need a window and pages of their own", pool);
   NNIS_REQUIRE(head_dim == HD, "attention: this module is compiled for head_dim %d, got %d", HD, head_dim);
@@ -1533,8 +1533,6 @@ extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, 
                heads, kv_heads);
   NNIS_REQUIRE(window > -(1 << 30) && max_pages > 0, "attention: bad window %d or block table width %d", window, max_pages);
   NNIS_REQUIRE(keep_first >= 0 && (bias == nullptr || reach >= 0), "attention: bad keep_first %d or reach %d", keep_first, reach);
-  if (tokens <= 0) return 0;
-  AttnArgs a;
   a.q = q; a.q_dtype = q_dtype; a.out = out; a.out_dtype = out_dtype;
   a.k_pages = k_pages; a.v_pages = v_pages; a.cache_dtype = cache_dtype;
   a.block_table = block_table; a.max_pages = max_pages; a.tok_slot = tok_slot; a.tok_pos = tok_pos;
@@ -1542,6 +1540,20 @@ extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, 
   a.keep_first = window > 0 ? keep_first : 0; a.bias = bias; a.reach = reach; a.sink = sink;
   a.pool_k = pool_k; a.pool_v = pool_v; a.pool_table = pool_table; a.pool_max_pages = pool_max_pages; a.pool = pool;
   if (fill_terms(a.terms, terms, heads)) return 1;
+  return 0;
+}
+
+extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, int out_dtype, const void* k_pages,
+                                          const void* v_pages, int cache_dtype, const int* block_table, int max_pages,
+                                          const int* tok_slot, const int* tok_pos, int tokens, int heads, int kv_heads,
+                                          int head_dim, int window, float scale, int value_dim, float softcap, int keep_first,
+                                          const float* bias, int reach, const float* sink, const void* pool_k,
+                                          const void* pool_v, const int* pool_table, int pool_max_pages, int pool,
+                                          const NnisHeadTerms* terms, void* stream) {
+  AttnArgs a;
+  if (fill_args(a, q, q_dtype, out, out_dtype, k_pages, v_pages, cache_dtype, block_table, max_pages, tok_slot, tok_pos, tokens, heads, kv_heads,
+                head_dim, window, scale, value_dim, softcap, keep_first, bias, reach, sink, pool_k, pool_v, pool_table, pool_max_pages, pool, terms)) return 1;
+  if (tokens <= 0) return 0;
   const long long items = (long long)tokens * heads;
   const unsigned blocks = (unsigned)((items + 3) / 4);
   if (cache_dtype == NNIS_F32) {
@@ -1552,6 +1564,50 @@ extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, 
   NNIS_LAUNCH_CHECK("attention_rows");
   return 0;
 }
+
+#if NNIS_MATRIX_CORES
+extern "C" int nnis_attention_f32_tile_rows(int heads, int kv_heads) { return heads == kv_heads ? 16 * kF32Columns : 16; }
+extern "C" int nnis_attention_f32_most_splits() { return kF32MostSplits; }
+
+// Everything in 32 bits.  tile_seq null: one token a sequence (tok_slot, tok_pos), its keys cut into `splits` blocks whose
+// outputs meet in `partial` (tokens * heads * splits * (HDV + 4) floats, with splits > 1).  Else `tiles` items of a step of prompts.
+extern "C" int nnis_attention_f32(const void* q, void* out, const void* k_pages, const void* v_pages, const int* block_table, int max_pages,
+                                  const int* tok_slot, const int* tok_pos, int tokens, int heads, int kv_heads, int head_dim, int window,
+                                  float scale, int value_dim, float softcap, int keep_first, const float* bias, int reach, const float* sink,
+                                  const void* pool_k, const void* pool_v, const int* pool_table, int pool_max_pages, int pool,
+                                  const NnisHeadTerms* terms, const int* tile_seq, const int* tile_row0, int tiles, const int* seq_slot,
+                                  const int* seq_start, const int* seq_pos0, int splits, float* partial, void* stream) {
+  AttnArgs a;
+  if (fill_args(a, q, NNIS_F32, out, NNIS_F32, k_pages, v_pages, NNIS_F32, block_table, max_pages, tok_slot, tok_pos, tokens, heads, kv_heads,
+                head_dim, window, scale, value_dim, softcap, keep_first, bias, reach, sink, pool_k, pool_v, pool_table, pool_max_pages, pool, terms)) return 1;
+  NNIS_REQUIRE(((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)pool_k | (uintptr_t)pool_v | (uintptr_t)partial) % 16 == 0,
+               "attention: operands must be 16-byte aligned");
+  const bool single = tile_seq == nullptr;
+  NNIS_REQUIRE(single ? splits >= 1 && splits <= kF32MostSplits && (splits == 1 || partial) : splits == 1 && tile_row0 && seq_slot && seq_start && seq_pos0,
+               "attention: %d blocks of keys an item (up to %d, for single tokens), or a part of the items' places missing", splits, kF32MostSplits);
+  const int items = single ? tokens : tiles;
+  if (tokens <= 0 || items <= 0) return 0;
+  const int group = heads / kv_heads;
+  F32Step step;
+  step.tile_seq = tile_seq; step.tile_row0 = tile_row0; step.seq_slot = seq_slot; step.seq_start = seq_start; step.seq_pos0 = seq_pos0;
+  step.chunks = single ? (group + 15) / 16 : (group == 1 ? 1 : (group + kF32Columns - 1) / kF32Columns);
+  step.splits = splits; step.partial = partial;
+  const long long blocks = (long long)items * kv_heads * step.chunks;
+  NNIS_REQUIRE(blocks < (1LL << 31), "attention: %d items of %d heads exceed the grid limit", items, heads);
+  hipStream_t s = (hipStream_t)stream;
+  if (single) {
+    hipLaunchKernelGGL((attention_f32_kernel<1, true>), dim3((unsigned)blocks, splits), dim3(kWave * kF32Waves), 0, s, a, step);
+  } else {
+    hipLaunchKernelGGL((attention_f32_kernel<kF32Columns, false>), dim3((unsigned)blocks), dim3(kWave * kF32Waves), 0, s, a, step);
+  }
+  NNIS_LAUNCH_CHECK("attention_f32");
+  if (splits > 1) {
+    hipLaunchKernelGGL(attention_f32_combine_kernel, dim3(tokens, heads), dim3(HDV < 64 ? 64 : (HDV > 256 ? 256 : HDV)), 0, s, a, step);
+    NNIS_LAUNCH_CHECK("attention_f32_combine");
+  }
+  return 0;
+}
+#endif
 
 extern "C" int nnis_attention_rows_pooled(const void* q, int q_dtype, void* out, int out_dtype, const void* k_pages,
                                           const void* v_pages, int cache_dtype, const int* block_table, int max_pages,

@@ -154,7 +154,7 @@ def _attention_recipe(rest: str) -> ModuleRecipe:
         defines.append(("NNIS_SCORE_EXTRAS", "1"))
     if pooled:
         defines.append(("NNIS_POOLED_BLOCKS", "1"))
-    return ModuleRecipe(("attention.hip",), ("common.h",), tuple(defines), (("attention.hip", tuple(_VECTOR_SUMS)),))
+    return ModuleRecipe(("attention.hip",), ("common.h", "attention_f32.h"), tuple(defines), (("attention.hip", tuple(_VECTOR_SUMS)),))
 
 
 # the library's own modules: ``core`` holds the kernels whose sizes are run-time arguments; attention is compiled per head size

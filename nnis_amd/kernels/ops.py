@@ -90,6 +90,9 @@ _ATTN_SIGNATURES = {
     "nnis_attention_decode_bf16_terms": [_VOID, _VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _FLT,
                                          _INT, _INT, _VOID, _INT, _INT, _INT, _FLT, _INT, _VOID, _INT, _VOID,
                                          _VOID, _VOID, _VOID, _INT, _INT, _VOID, _VOID],
+    "nnis_attention_f32": [_VOID, _VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _FLT, _INT, _FLT, _INT, _VOID,
+                           _INT, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _VOID, _INT, _VOID, _VOID],
+    "nnis_attention_f32_tile_rows": [_INT, _INT],
     "nnis_attention_prefill_tile_rows": [_INT, _INT, _INT],
     "nnis_attention_prefill_bf16": [_VOID, _VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _VOID, _VOID, _VOID, _INT,
                                     _INT, _INT, _INT, _FLT, _INT, _INT, _FLT, _VOID],
@@ -804,6 +807,65 @@ def attention_rows(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_
                                         tok_slot.data_ptr(), tok_pos.data_ptr(), tokens, heads, kv_heads, head_dim,
                                         int(window), float(scale), int(value_dim), float(softcap), _stream()))
     return out
+
+
+ATTENTION_F32_MOST_SPLITS = 16  # kF32MostSplits of csrc/attention_f32.h
+
+
+def attention_f32(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
+                  tok_slot: torch.Tensor, tok_pos: torch.Tensor, heads: int, kv_heads: int, head_dim: int, scale: float, window: int = 0,
+                  value_dim: Optional[int] = None, softcap: float = 0.0, extras: Optional[ScoreExtras] = None,
+                  pooled: Optional["PooledBlocks"] = None, terms: Optional[HeadTerms] = None, tiles=None, splits: int = 1) -> torch.Tensor:
+    """``attention_rows`` on the matrix cores, everything in 32 bits, for heads
+    whose keys and values come in steps of 16 channels up to 256.  ``tiles``:
+    (items, seq_slot, seq_start, seq_pos0) of a step of prompts, the items as
+    ``prefill_tile_list`` makes them for ``attention_f32_tile_rows`` rows; None
+    for one token a sequence, whose keys go to ``splits`` blocks."""
+    tokens = q.shape[0]
+    value_dim = value_dim or head_dim
+    if q.shape != (tokens, heads * head_dim) or out.shape != (tokens, heads * value_dim):
+        raise KernelError(f"attention: q {tuple(q.shape)} / out {tuple(out.shape)} do not fit {heads} heads of {head_dim} "
+                          f"with values of {value_dim}")
+    for t, what in ((q, "q"), (out, "out"), (k_pages, "k_pages"), (v_pages, "v_pages"), (block_table, "block_table")):
+        _dev(t, what)
+        if t.dtype != (torch.int32 if t is block_table else torch.float32):
+            raise KernelError(f"attention: the 32-bit kernels do not take {what} of {t.dtype}")
+    if not _pages_fit(k_pages, v_pages, kv_heads, head_dim, value_dim) or block_table.dim() != 2:
+        raise KernelError(f"attention: page shapes {tuple(k_pages.shape)} / {tuple(v_pages.shape)} / {tuple(block_table.shape)} do not fit")
+    items, where = None, (None, None, None)
+    if tiles is not None:
+        items, where = tiles[0], tiles[1:]
+    for t in (tok_slot, tok_pos) if tiles is None else (items, *where):
+        _dev(t, "step metadata")
+        if t.dtype != torch.int32:
+            raise KernelError("attention: a step's metadata must be int32")
+    if tiles is None and min(tok_slot.numel(), tok_pos.numel()) < tokens:
+        raise KernelError("attention: tok_slot / tok_pos must have one entry per token")
+    # (a call's own: calls on other streams may run beside this one)
+    partial = torch.empty(tokens * heads * splits * (value_dim + 4), dtype=torch.float32, device=q.device) if splits > 1 else None
+    held = terms.struct(tokens, heads) if terms else None
+    lib = attention_module(head_dim, value_dim, softcap, extras, pooled, terms)
+    _check(lib, lib.nnis_attention_f32(
+        q.data_ptr(), out.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), block_table.data_ptr(), block_table.shape[1], tok_slot.data_ptr(),
+        tok_pos.data_ptr(), tokens, heads, kv_heads, head_dim, int(window), float(scale), int(value_dim), float(softcap),
+        *_more_arguments(heads, k_pages, v_pages, kv_heads, head_dim, value_dim, window, extras, pooled), ctypes.addressof(held) if held else None,
+        *((items[0].data_ptr(), items[1].data_ptr(), items.shape[1]) if items is not None else (None, None, 0)), *map(_ptr, where), int(splits),
+        _ptr(partial), _stream()))
+    return out
+
+
+def attention_f32_splits(tokens: int, heads: int, kv_heads: int, window: int, longest: int) -> int:
+    """The blocks that a step of single tokens cuts an item's keys into: as many as bring the step to F32_BLOCKS blocks
+    of 4 waves, of which each gets a tile of 16 keys where a sequence has as many as it may come to have (``longest``, or
+    the window).  It does not go by the step's own lengths, so that a captured step serves them all."""
+    # Microseconds with 1 / 4 / 8 / 16 blocks an item (a second kernel sums them): 1 token of 1,000 keys on 3 key/value heads of
+    # 64 21 / 12 / 10 / 9, 8 of 2,000 37 / 17 / 13 / 13, 32 of 60 to 1,610 32 / 19.5 / 21 / 23; 8 of 2,000 on 32 heads 42 / 50 / 51 / 58.
+    items = tokens * kv_heads * ((heads // kv_heads + 15) // 16)
+    keys = longest if window == 0 else min(longest, abs(window) + 15)
+    return max(1, min(F32_BLOCKS // max(items, 1), (keys + 63) // 64, ATTENTION_F32_MOST_SPLITS))
+
+
+F32_BLOCKS = 384
 
 
 # ---------------------------------------------------------------------------
@@ -1556,6 +1618,15 @@ def attention(q: torch.Tensor, out: torch.Tensor, view, ctx, heads: int, kv_head
     for the last n keys, or n < 0 for the keys of the query's own chunk of -n
     positions."""
     value_dim = value_dim or head_dim
+    if attention_f32_takes(q, out, view.k_pages, view.v_pages, head_dim, value_dim):
+        if ctx.decode:
+            tiles, splits = None, attention_f32_splits(q.shape[0], heads, kv_heads, window, 64 * view.block_table.shape[1])
+        else:
+            rows = attention_module(head_dim, value_dim, softcap, extras, pooled, terms).nnis_attention_f32_tile_rows(heads, kv_heads)
+            items = ctx.lists.device_list(("attention_tiles", rows), lambda new, first, padded: prefill_tile_list(new, first, padded, rows))
+            tiles, splits = (items, ctx.seq_slot, ctx.seq_start, ctx.seq_pos0), 1
+        return attention_f32(q, out, view.k_pages, view.v_pages, view.block_table, ctx.tok_slot, ctx.tok_pos, heads, kv_heads, head_dim, scale,
+                             window, value_dim, softcap, extras, pooled, terms, tiles, splits)
     fast = attention_on_matrix_cores(q.dtype, view.k_pages.dtype, head_dim, value_dim, softcap, extras)
     size = max(head_dim, value_dim)  # what a wave's registers are sized by
     if fast and ctx.decode and heads // kv_heads <= 16 * (4 if size <= 64 else (2 if size <= 128 else 1)):
@@ -1588,6 +1659,12 @@ def attention_on_matrix_cores(q_dtype, cache_dtype, head_dim: int, value_dim: Op
     """Whether ``attention`` takes the matrix-core kernels for these types and sizes (else the 32-bit row kernel)."""
     return (q_dtype == torch.bfloat16 and cache_dtype == torch.bfloat16 and head_dim % 16 == 0
             and (value_dim or head_dim) % 16 == 0 and max(head_dim, value_dim or head_dim) <= ATTENTION_MOST_CHANNELS)
+
+
+def attention_f32_takes(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, head_dim: int, value_dim: int) -> bool:
+    """Whether ``attention`` takes ``attention_f32`` for 32-bit operands of these sizes (else the row kernel)."""
+    return (q.dtype == out.dtype == k_pages.dtype == torch.float32 and head_dim % 16 == 0 and value_dim % 16 == 0
+            and max(head_dim, value_dim) <= ATTENTION_MOST_CHANNELS and not (q.data_ptr() | out.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) & 15)
 
 
 def sample(logits: torch.Tensor, weights: torch.Tensor, row_slot: torch.Tensor, rng: torch.Tensor,

@@ -1025,3 +1025,62 @@ def test_the_tiles_that_products_are_given():
         (2048, 3072, 576): T.TILE_64x128,
     }.items():
         assert ops.gemm_tile(m, n, k) == tile, (m, n, k, ops.gemm_tile(m, n, k))
+
+
+F32_ATTENTION = [
+    # heads, key/value heads, key channels, value channels, options
+    (9, 3, 64, 64, {}), (4, 4, 16, 16, {}), (32, 1, 64, 64, {}), (40, 2, 16, 16, {}), (5, 5, 80, 80, {}), (8, 2, 128, 128, {}), (3, 3, 256, 256, {}),
+    (6, 2, 48, 48, dict(window=70)), (4, 1, 112, 112, dict(window=-96)), (6, 3, 32, 16, dict(window=33, keep_first=21, bias=True, sink=True)),
+    (4, 2, 16, 48, dict(window=64, softcap=3.0, sink=True, pool=16)), (8, 2, 32, 16, dict(softcap=2.0, bias=True, decay=True, gated=True)),
+    (4, 4, 96, 64, dict(bias=True, sink=True)),
+]
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim, value_dim, options", F32_ATTENTION)
+def test_attention_in_32_bits_on_the_matrix_cores(heads, kv_heads, head_dim, value_dim, options):
+    """Single tokens (their keys in one block or several) and a step of prompts, some behind tokens held already, in every
+    option, against the row kernel.  Both are 32-bit: a score below 16 is rounded at each of its ``head_dim`` products, by up
+    to 2^-21 a time, of which about the square root adds up, and moves an output by as much of the values' spread, 4."""
+    ops = _ops()
+    torch.manual_seed(heads * head_dim + value_dim)
+    rand = lambda *shape: torch.randn(*shape)  # noqa: E731
+    first, new = [0, 250, 63, 0], [37, 50, 1, 130]
+    ends = [f + n for f, n in zip(first, new)]
+    k_pages, v_pages, table = _paged([rand(n, kv_heads, head_dim) for n in ends], [rand(n, kv_heads, value_dim) for n in ends], torch.float32,
+                                     kv_heads, head_dim) if value_dim == head_dim else (None, None, None)
+    if k_pages is None:
+        k_pages, _, table = _paged([rand(n, kv_heads, head_dim) for n in ends], [rand(n, kv_heads, head_dim) for n in ends], torch.float32, kv_heads, head_dim)
+        _, v_pages, _ = _paged([rand(n, kv_heads, value_dim) for n in ends], [rand(n, kv_heads, value_dim) for n in ends], torch.float32, kv_heads, value_dim)
+    pooled = terms = None
+    extras = ops.ScoreExtras(options.get("keep_first", 0), rand(heads, 41).cuda() if options.get("bias") else None,
+                             rand(heads).cuda() if options.get("sink") else None)
+    if options.get("pool"):
+        pk = _paged([rand(64, kv_heads, head_dim) for _ in ends], [rand(64, kv_heads, head_dim) for _ in ends], torch.float32, kv_heads, head_dim)
+        pv = _paged([rand(64, kv_heads, value_dim) for _ in ends], [rand(64, kv_heads, value_dim) for _ in ends], torch.float32, kv_heads, value_dim)
+        pooled = ops.PooledBlocks(pk[0], pv[1], pk[2], options["pool"])
+    if options.get("decay"):
+        terms = ops.HeadTerms((torch.rand(heads).cuda(), torch.rand(heads).cuda()), gated=options.get("gated", False))
+    common = (heads, kv_heads, head_dim, head_dim ** -0.5, options.get("window", 0), value_dim, options.get("softcap", 0.0), extras, pooled)
+
+    def both(slots, positions, tiles=None, splits=1):
+        tokens = len(slots)
+        q = 3.0 * rand(tokens, heads * head_dim).cuda()  # (scores large enough for the softmax reference to move)
+        own = terms.with_gate(rand(tokens, heads).cuda()) if terms is not None and terms.gated else terms
+        want = torch.empty(tokens, heads * value_dim, device="cuda")
+        got = torch.full((tokens, heads * value_dim), 9.0, device="cuda")
+        ops.attention_rows(q, want, k_pages, v_pages, table, _i32(slots), _i32(positions), *common, own)
+        ops.attention_f32(q, got, k_pages, v_pages, table, _i32(slots), _i32(positions), *common, own, tiles, splits)
+        assert (got - want).abs().max().item() <= 4 * 2.0 ** -21 * max(head_dim, 32) ** 0.5, (tiles is not None, splits)
+        return got
+
+    for splits in (1, 3, ops.ATTENTION_F32_MOST_SPLITS):
+        got = both([3, 1, -1, 0, 2], [129, 299, 0, 0, 63], splits=splits)
+        assert (got[2] == 0).all()  # a padding row
+    rows = ops.attention_module(head_dim, value_dim, options.get("softcap", 0.0), extras, pooled, terms).nnis_attention_f32_tile_rows(heads, kv_heads)
+    starts = [0, *np.cumsum(new).tolist()]
+    for padded in (None, (4, 256)):
+        items = torch.from_numpy(ops.prefill_tile_list(new, first, padded, rows)).cuda()
+        both([s for s, n in enumerate(new) for _ in range(n)], [f + i for f, n in zip(first, new) for i in range(n)],
+             (items, _i32([0, 1, 2, 3]), _i32(starts), _i32(first)))
+    with pytest.raises(KernelError):
+        both([0], [0], splits=ops.ATTENTION_F32_MOST_SPLITS + 1)
