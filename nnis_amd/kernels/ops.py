@@ -50,6 +50,8 @@ _CORE_SIGNATURES = {
     "nnis_argmax": [_VOID, _VOID, _INT, _INT, _VOID, _VOID],
     "nnis_argmax_scratch": [_INT, _INT],
     "nnis_argmax_static": [_VOID, _VOID, _INT, _INT, _VOID],
+    "nnis_gemm_f32_fused": [_VOID, _INT, _VOID, _FLT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _VOID, _VOID, _VOID,
+                            _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
     "nnis_gemm_f32": [_VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_ordered": [_VOID, _INT, _VOID, _INT, _VOID, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_bf16": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID, _SIZE, _VOID],
@@ -1035,6 +1037,43 @@ def gemm_fused(x_in: torch.Tensor, delta: Optional[torch.Tensor], x_out: Optiona
     return y
 
 
+EPILOGUE_RESIDUAL = 3  # of ``gemm_f32_fused``
+GEMM_F32_NORM_ROWS = 16  # NNIS_GEMM_F32_NORM_ROWS of csrc/gemm_f32.hip
+
+
+def gemm_f32_fused(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, epilogue: int = EPILOGUE_STORE, norm_weight: Optional[torch.Tensor] = None,
+                   eps: float = 0.0, rope: Optional[dict] = None, variant: int = -1) -> torch.Tensor:
+    """``gemm_f32`` on 32-bit rows with what comes behind the product in its
+    kernel: stored (y [m, n]); SiLU(gate) * up for a weight of gate rows
+    followed by up rows (y [m, n / 2]); rotate-half RoPE with the write of keys
+    and values into 32-bit pages (``rope`` as for ``gemm_fused``; y [m, heads *
+    head_dim]); or added to y [m, n], the residual stream.  With
+    ``norm_weight`` (float32 [k]; up to ``GEMM_F32_NORM_ROWS`` rows, not with
+    the sum) x stands for its RMS norm."""
+    _dev(x, "x"), _dev(w, "weight"), _dev(y, "y")
+    m, k = x.shape
+    n = w.shape[0]
+    if not x.dtype == w.dtype == y.dtype == torch.float32 or w.shape[1] != k:
+        raise KernelError(f"gemm_f32: x {tuple(x.shape)} {x.dtype} w {tuple(w.shape)} {w.dtype} y {y.dtype} do not fit")
+    if norm_weight is not None:
+        _dev(norm_weight, "norm weight")
+        if norm_weight.dtype != torch.float32 or norm_weight.numel() != k:
+            raise KernelError(f"gemm_f32: norm weight {tuple(norm_weight.shape)} {norm_weight.dtype} for width {k}")
+    r = {}
+    if epilogue == EPILOGUE_RESIDUAL:
+        if y.shape != (m, n):
+            raise KernelError(f"gemm_f32: a stream {tuple(y.shape)} for a product of {m} x {n}")
+    else:
+        r = _check_epilogue("gemm_f32", m, n, y, epilogue, rope, pages=torch.float32)
+    bt = r.get("block_table")
+    lib = core()
+    _check(lib, lib.nnis_gemm_f32_fused(
+        x.data_ptr(), 0, _ptr(norm_weight), float(eps), w.data_ptr(), y.data_ptr(), 0, m, n, k, int(epilogue), _ptr(r.get("cos")), _ptr(r.get("sin")),
+        _ptr(r.get("tok_slot")), _ptr(r.get("tok_pos")), _ptr(r.get("k_pages")), _ptr(r.get("v_pages")), _ptr(bt), bt.shape[1] if bt is not None else 0,
+        r.get("heads", 0), r.get("kv_heads", 0), r.get("head_dim", 0), *_step_table_pointers(r), int(variant), _stream()))
+    return y
+
+
 def _step_table_pointers(rope: dict):
     """(tok_cos, tok_sin, tok_page) of a rotating epilogue's ``tables`` (a ``StepTables``), or three nulls."""
     tables = rope.get("tables")
@@ -1043,8 +1082,9 @@ def _step_table_pointers(rope: dict):
     return tables.cos.data_ptr(), tables.sin.data_ptr(), tables.page.data_ptr()
 
 
-def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, rope: Optional[dict]) -> dict:
-    """Checks y and the rotating epilogue's arguments against the sizes; returns the arguments (or {})."""
+def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, rope: Optional[dict], pages: torch.dtype = torch.bfloat16) -> dict:
+    """Checks y and the rotating epilogue's arguments against the sizes; returns the arguments (or {}).  ``pages``: the
+    type of y and of the cache's pages."""
     expect = {EPILOGUE_STORE: (m, n), EPILOGUE_SILU: (m, n // 2)}.get(epilogue & 0xff if epilogue > 0 else epilogue)
     if epilogue >> 8 and ((epilogue & 0xff) != EPILOGUE_SILU or epilogue >> 8 not in ACTIVATIONS.values()):
         raise KernelError(f"{what}: unknown epilogue {epilogue}")
@@ -1065,11 +1105,11 @@ def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, r
         if r.get("k_pages") is not None:
             kp, vp, bt = r["k_pages"], r["v_pages"], r["block_table"]
             _dev(kp, "k_pages"), _dev(vp, "v_pages"), _dev(bt, "block_table")
-            if (kp.dtype != torch.bfloat16 or vp.dtype != torch.bfloat16 or bt.dtype != torch.int32
+            if (kp.dtype != pages or vp.dtype != pages or bt.dtype != torch.int32
                     or not _pages_fit(kp, vp, r["kv_heads"], r["head_dim"])):
-                raise KernelError(f"{what}: cache pages must be bfloat16 in the cache's layout, the block table int32")
-    if expect is None or tuple(y.shape) != expect or y.dtype != torch.bfloat16 or not y.is_contiguous():
-        raise KernelError(f"{what}: y {tuple(y.shape)} {y.dtype} does not fit epilogue {epilogue} (expected bfloat16 {expect})")
+                raise KernelError(f"{what}: cache pages must be {pages} in the cache's layout, the block table int32")
+    if expect is None or tuple(y.shape) != expect or y.dtype != pages or not y.is_contiguous():
+        raise KernelError(f"{what}: y {tuple(y.shape)} {y.dtype} does not fit epilogue {epilogue} (expected {pages} {expect})")
     return r
 
 

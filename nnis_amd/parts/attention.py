@@ -241,7 +241,7 @@ class CausalSelfAttention(Mixer):
             qkv = x.fused(self.qkv.weight, rt.empty(x.rows, self.qkv.out_features), rt.ops.EPILOGUE_STORE)
         elif isinstance(x, PendingNorm):
             if (self._plain and x.can_fuse(self.qkv.weight) and tables is not None and tables.rot_dim == self.head_dim
-                    and self.head_dim % 32 == 0 and view.k_pages.dtype == torch.bfloat16):
+                    and self.head_dim % 32 == 0 and view.k_pages.dtype == rt.dtype):
                 # residual sum, norm, the three projections, the rotation and the cache write in one kernel
                 rope = dict(cos=tables.cos, sin=tables.sin, tok_slot=ctx.tok_slot, tok_pos=ctx.tok_pos,
                             tables=ctx.step_tables(rt, tables, view.block_table),

@@ -65,6 +65,9 @@ class PendingNorm:
         ops = self.rt.ops
         if self.ready is not None:
             return False
+        if self.rt.is_fp32:
+            return (getattr(self.norm, "fusable_rms", False) and self.norm.weight.dtype == torch.float32 and self.x.dtype == torch.float32
+                    and self.x.is_contiguous() and isinstance(weight, torch.Tensor) and ops.gemm_f32_takes(self.x, weight, self.norm.weight))
         fits = (
             getattr(self.norm, "fusable_rms", False)
             and self.x.dtype == torch.float32
@@ -76,7 +79,15 @@ class PendingNorm:
         return fits and self.rows <= ops.FUSED_MAX_TOKENS and (self.delta is None or self.delta.dtype == torch.bfloat16)
 
     def fused(self, weight, y: torch.Tensor, epilogue: int, rope=None) -> torch.Tensor:
-        """y = epilogue(weight . norm(x + delta)) in one kernel."""
+        """y = epilogue(weight . norm(x + delta)) in one kernel (under a 32-bit runtime behind the norm's own, where the
+        rows are many or the sum is still to be taken)."""
+        ops = self.rt.ops
+        if self.rt.is_fp32:
+            if self.delta is not None or self.rows > ops.GEMM_F32_NORM_ROWS:
+                return ops.gemm_f32_fused(self.materialize(), weight, y, epilogue, rope=rope)
+            ops.gemm_f32_fused(self.x, weight, y, epilogue, self.norm.weight, self.norm.eps, rope)
+            self.residual = self.x
+            return y
         if self.scaled is not None:
             return self.rt.ops.gemm_scaled(self.scaled, self.ss, self.parts, self.norm.eps, weight, y, epilogue, rope)
         x_out = None
@@ -99,6 +110,12 @@ class ResidualInto:
         self.rt = rt
 
     def can_take(self, x: torch.Tensor, weight) -> bool:
+        if self.rt.is_fp32:
+            residual = self.source.residual
+            return (getattr(self.norm, "fusable_rms", False) and residual is not None and residual.dtype == torch.float32
+                    and residual.is_contiguous() and isinstance(x, torch.Tensor) and x.dtype == torch.float32 and x.is_contiguous()
+                    and isinstance(weight, torch.Tensor) and weight.shape[0] == residual.shape[1]
+                    and self.rt.ops.gemm_f32_takes(x, weight, residual))
         return getattr(self.norm, "fusable_rms", False) and self._fits(x, weight)
 
     def _fits(self, x: torch.Tensor, weight) -> bool:
@@ -114,7 +131,10 @@ class ResidualInto:
         )
 
     def take(self, x: torch.Tensor, weight) -> PendingNorm:
-        """residual += x @ weight^T; returns the next norm, prepared."""
+        """residual += x @ weight^T; returns the next norm, prepared (under a 32-bit runtime pending, with nothing to add)."""
+        if self.rt.is_fp32:
+            self.rt.ops.gemm_f32_fused(x, weight, self.source.residual, self.rt.ops.EPILOGUE_RESIDUAL)
+            return PendingNorm(self.norm, self.source.residual, None, self.rt)
         return self.take_by(lambda residual, gain, scaled, ss: self.rt.ops.gemm_residual(x, weight, residual, gain, scaled, ss))
 
     def take_by(self, write) -> PendingNorm:

@@ -108,6 +108,69 @@ def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
         assert ((y.cpu().double() - x.double() @ w.double().t()).abs() <= tol * (x.double().abs() @ w.double().abs().t())).all()
 
 
+@pytest.mark.parametrize("variant", [-1, 1, 2, 3, 4, 5, 7, 9, 10, 12, 13, 14, 15])
+@pytest.mark.parametrize("normed", [False, True])
+@pytest.mark.parametrize("m, n, k", [(1, 2, 4), (8, 70, 52), (5, 2 * 130, 548), (16, 34, 100), (65, 2 * 67, 176), (131, 256, 612)])
+def test_gemm_f32_with_what_comes_behind_it(m, n, k, normed, variant):
+    """The gate, the sum into the stream and the plain store behind the product, with the norm before it or without, in
+    every form that takes them, against 64 bits: the bound of the plain product, carried through the gate (whose slopes
+    are below 1.1 times the other factor) and with the norm's own few roundings."""
+    ops = _ops()
+    few = variant in (1, 13, 14, 15, -1)
+    if (variant == 13 and m > 8) or (normed and (m > 16 or not few)):
+        return
+    torch.manual_seed(m + n + k)
+    x, w, gain = torch.randn(m, k), torch.randn(n, k), 1 + 0.2 * torch.randn(k)
+    rows = P.rms_norm(x.double(), gain.double(), 1e-5) if normed else x.double()
+    product, scale = rows @ w.double().t(), 4e-7 * math.sqrt(k) * (rows.abs() @ w.double().abs().t()) + 1e-7
+    norm = (gain.cuda(), 1e-5) if normed else ()
+    out = torch.full((m + 1, n // 2), 7.0, device="cuda")
+    ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_SILU, *norm, variant=variant)
+    gate, up = product[:, :n // 2], product[:, n // 2:]
+    bound = 1.1 * (scale[:, :n // 2] * up.abs() + gate.abs() * scale[:, n // 2:]) + 1e-6 * (1 + (gate * up).abs()) + scale[:, :n // 2] * scale[:, n // 2:]
+    assert ((out[:m].cpu().double() - gate * torch.sigmoid(gate) * up).abs() <= bound).all() and (out[m] == 7).all()
+    if variant in (2, 3, 4, 5, 7, 9, 10, 12, -1) or few:
+        out = torch.full((m + 1, n), 7.0, device="cuda")
+        ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_STORE, *norm, variant=variant)
+        assert ((out[:m].cpu().double() - product).abs() <= scale).all() and (out[m] == 7).all()
+    if not normed:
+        stream = torch.randn(m + 1, n)
+        out = stream.cuda()
+        ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_RESIDUAL, variant=variant)
+        assert ((out[:m].cpu().double() - stream[:m].double() - product).abs() <= scale + 1e-6).all() and torch.equal(out[m].cpu(), stream[m])
+
+
+@pytest.mark.parametrize("variant", [-1, 1, 2, 4, 5, 12, 13, 14])
+@pytest.mark.parametrize("tokens, heads, kv_heads, head_dim, normed, tables", [(1, 9, 3, 64, True, True), (7, 3, 1, 32, True, False), (13, 4, 4, 96, False, True),
+                                                                              (70, 4, 2, 64, False, False)])
+def test_gemm_f32_rotates_and_writes_the_cache(tokens, heads, kv_heads, head_dim, normed, tables, variant):
+    """The rotation and the cache write behind the product against the kernels of their own on the plain product."""
+    ops = _ops()
+    if (variant == 13 and tokens > 8) or (normed and variant not in (-1, 1, 13, 14)):
+        return
+    torch.manual_seed(tokens + head_dim)
+    k, n = 100, (heads + 2 * kv_heads) * head_dim
+    x, w, gain = torch.randn(tokens, k).cuda(), torch.randn(n, k).cuda(), (1 + 0.2 * torch.randn(k)).cuda()
+    cos, sin = (torch.from_numpy(t).cuda() for t in P.rope_tables(256, head_dim, 10000.0))
+    slots = [t % 3 if t % 5 != 4 else -1 for t in range(tokens)]
+    positions = [(t // 3) * 3 + 60 for t in range(tokens)]
+    table = torch.tensor([[3, 0], [9, 4], [2, 7]], dtype=torch.int32).cuda()
+    slot, pos = _i32(slots), _i32(positions)
+    pages = [_empty_pages(10, kv_heads, head_dim, torch.float32, 7.0, 7.0, "cuda") for _ in range(2)]
+    rows = ops.rmsnorm(x, gain, 1e-5, torch.empty_like(x)) if normed else x
+    plain, want, got = torch.empty(tokens, n, device="cuda"), torch.zeros(tokens, heads * head_dim, device="cuda"), torch.zeros(tokens, heads * head_dim, device="cuda")
+    ops.gemm_f32(rows, w, plain)
+    ops.rope_kv_write(plain, want, cos, sin, head_dim, slot, pos, *pages[0], table, heads, kv_heads, head_dim)
+    rope = dict(cos=cos, sin=sin, tok_slot=slot, tok_pos=pos, k_pages=pages[1][0], v_pages=pages[1][1], block_table=table, heads=heads,
+                kv_heads=kv_heads, head_dim=head_dim, tables=ops.step_tables(slot, pos, tokens, cos, sin, table) if tables else None)
+    ops.gemm_f32_fused(x, w, got, ops.EPILOGUE_ROPE, *((gain, 1e-5) if normed else ()), rope=rope, variant=variant)
+    live = torch.tensor([s >= 0 for s in slots])
+    bound = 1e-6 * k  # both sides sum k products of normal values in 32 bits
+    assert (got - want)[live.cuda()].abs().max().item() <= bound
+    for mine, theirs in zip(pages[1], pages[0]):
+        assert (mine - theirs).abs().max().item() <= bound
+
+
 def test_a_32_bit_product_whose_rows_cannot_be_loaded_16_bytes_at_a_time_takes_the_ordered_kernel():
     ops = _ops()
     w = torch.randn(24, 36, device="cuda")
