@@ -1248,16 +1248,23 @@ __global__ __launch_bounds__(256) void gated_delta_kernel(DeltaArgs a) {
 
 }  // namespace
 
+// over a step's prompts, in chunks of tokens (chunked_state.hip)
+int nnis_gated_delta_chunks(const float* unit, const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
+                            float* state, const int* seq_slot, const int* seq_start, int batch, int tokens, int heads, int groups, int key_dim,
+                            int value_dim, float* out, float* scratch, hipStream_t s);
+
 // Floats of scratch that nnis_gated_delta needs for `tokens` rows: the unit vectors, the gates and the products q . k.
 extern "C" long long nnis_gated_delta_scratch(int tokens, int heads, int groups, int key_dim) {
   return (long long)tokens * ((long long)groups * 2 * key_dim + 2 * heads + groups);
 }
 
 // rows [tokens, stride] hold [q | k | v] behind the convolution; ba float32 [tokens, 2 * heads]; out float32 [tokens, heads *
-// value_dim]; scratch: nnis_gated_delta_scratch floats
+// value_dim]; scratch: nnis_gated_delta_scratch floats; chunk_scratch: null, or nnis_chunked_scratch floats, and the
+// sequences are walked in chunks of 64 tokens (sizes that nnis_chunked_takes)
 extern "C" int nnis_gated_delta(const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
                                 float q_scale, float unit_eps, float* state, const int* seq_slot, const int* seq_start, int batch,
-                                int tokens, int heads, int groups, int key_dim, int value_dim, float* out, float* scratch, void* stream) {
+                                int tokens, int heads, int groups, int key_dim, int value_dim, float* out, float* scratch, float* chunk_scratch,
+                                void* stream) {
   NNIS_REQUIRE(nnis_dtype_ok(dtype), "gated_delta: unknown dtype %d", dtype);
   NNIS_REQUIRE(heads > 0 && groups > 0 && heads % groups == 0 && key_dim > 0 && key_dim <= 256 && value_dim > 0 && batch >= 0 && tokens >= 0,
                "gated_delta: bad sizes (heads %d on %d query/key heads, key channels %d: up to 256 are taken, value channels %d)", heads,
@@ -1275,6 +1282,9 @@ extern "C" int nnis_gated_delta(const void* rows, int dtype, int stride, const f
   hipStream_t s = (hipStream_t)stream;
   const int items = tokens * groups;
   hipLaunchKernelGGL(delta_prepare_kernel, dim3((items + 3) / 4), dim3(256), 0, s, a);
+  if (chunk_scratch)
+    return nnis_gated_delta_chunks(a.unit, rows, dtype, stride, ba, rate, dt_bias, state, seq_slot, seq_start, batch, tokens, heads, groups,
+                                   key_dim, value_dim, out, chunk_scratch, s);
   const int need = (key_dim + 7) / 8;  // a thread keeps 8 key rows
   const int lane_groups = need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : (need <= 8 ? 8 : (need <= 16 ? 16 : 32))));
   const int cols = 4 * (kWave / lane_groups);

@@ -162,7 +162,7 @@ register_module("core", ["elementwise.hip", "residual.hip", "gemm.hip", "gemm_f3
                 headers=["common.h", "epilogue.h", "product.h", "nnis_noalloc.h"], source_flags={"gemm_mfma.hip": _VECTOR_SUMS, "gemm_f32.hip": _VECTOR_SUMS})
 register_module_family("attn_hd", _attention_recipe)
 # the mixers that carry a state of fixed size (convolution, selective scan, gated linear attention and retention, minGRU, gated delta rule)
-register_module("recurrent", ["recurrent.hip"], headers=["common.h"])
+register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
 # the real-gated linear recurrent unit
 register_module("gated_unit", ["gated_unit.hip"], headers=["common.h"], source_flags={"gated_unit.hip": _VECTOR_SUMS})
 # Mamba-2's state spaces

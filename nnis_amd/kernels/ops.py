@@ -119,7 +119,10 @@ _RECURRENT_SIGNATURES = {
     "nnis_gla_scan_turned": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _FLT, _VOID,
                              _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _INT, _VOID, _VOID, _VOID],
     "nnis_gated_delta": [_VOID, _INT, _INT, _VOID, _VOID, _VOID, _FLT, _FLT, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _INT, _VOID,
-                         _VOID, _VOID],
+                         _VOID, _VOID, _VOID],
+    "nnis_retention_chunks": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _FLT, _VOID, _VOID, _VOID,
+                              _INT, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID],
+    "nnis_chunked_takes": [_INT, _INT],
     "nnis_gla_decays": [_VOID, _VOID, _INT, _INT, _FLT, _VOID],
     "nnis_head_norm_gate": [_VOID, _VOID, _INT, _INT, _VOID, _INT, _VOID, _INT, _INT, _INT, _INT, _FLT, _VOID],
     "nnis_min_gru": [_VOID, _INT, _INT, _VOID, _VOID, _INT, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _INT, _INT, _INT, _VOID, _VOID, _VOID],
@@ -239,6 +242,8 @@ def recurrent():
     global _recurrent
     if _recurrent is None:
         _recurrent = _bind("recurrent", _RECURRENT_SIGNATURES)
+        _recurrent.nnis_chunked_scratch.argtypes = [_INT] * 6
+        _recurrent.nnis_chunked_scratch.restype = ctypes.c_longlong
     return _recurrent
 
 
@@ -1895,6 +1900,25 @@ def run_pieces(ctx, state_bytes: int):
     return (piece, pieces) if pieces > 1 else (0, 1)
 
 
+# The most scratch that a step's chunks take (147 KB a chunk and head of 128 x 256); steps beyond, of 28,000 tokens on 64
+# such heads, go a token at a time.
+CHUNKED_MOST_BYTES = 4 << 30
+
+
+def chunked_scratch(ctx, tokens: int, heads: int, key_dim: int, value_dim: int, delta: bool, device) -> Optional[torch.Tensor]:
+    """Scratch for a step whose sequences a matrix-state recurrence walks in chunks of 64 tokens (csrc/chunked_state.hip);
+    None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts too short."""
+    # Microseconds a token at a time and in chunks, by sequences x tokens.  Delta rule, 16 heads of 128 x 128: 1 x 96 48 / 41, 1 x 64 35 /
+    # 38; 4 x 96 60 / 64, 4 x 128 76 / 67; 8 x 128 103 / 117, 8 x 192 149 / 133; 16 x 128 199 / 192.  Retention, 8 heads of 128 x 256: 1 x 16
+    # 25 / 14; 8 x 16 26 / 30, 8 x 32 42 / 31; 16 x 32 48 / 51, 16 x 64 178 / 55.  (Its token at a time is split into pieces.)
+    least = 96 + 8 * min(ctx.batch, 8) if delta else 16 + 2 * min(ctx.batch, 16)
+    lib = recurrent()
+    if ctx.decode or tokens < least * max(ctx.batch, 1) or not lib.nnis_chunked_takes(key_dim, value_dim):
+        return None
+    floats = lib.nnis_chunked_scratch(tokens, ctx.batch, heads, key_dim, value_dim, 1 if delta else 0)
+    return torch.empty(floats, dtype=torch.float32, device=device) if 4 * floats <= CHUNKED_MOST_BYTES else None
+
+
 def _step_arrays(ctx, what: str):
     for t in (ctx.tok_slot, ctx.tok_pos, ctx.seq_slot, ctx.seq_start):
         _dev(t, "step metadata")
@@ -2185,6 +2209,19 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay_logs: Opti
         raise KernelError("gla_scan: out must be float32 [tokens, heads * value channels]")
     _step_arrays(ctx, "gla_scan")
     stride = lambda t: t.stride(0) if tokens > 1 else t.shape[1]  # noqa: E731
+    quarter = 4 * q.element_size()  # a prompt's rows and tables are loaded four channels at a time
+    chunks = None
+    if (head_decay is not None and not (q.data_ptr() | k.data_ptr()) % quarter and stride(q) % 4 == 0 and stride(k) % 4 == 0 and rot_dim % 8 == 0
+            and (rotation is None or not (cos.data_ptr() | sin.data_ptr()) % 16)):
+        chunks = chunked_scratch(ctx, tokens, heads, key_dim, value_dim, False, out.device)
+    if chunks is not None:
+        lib = recurrent()
+        _check(lib, lib.nnis_retention_chunks(q.data_ptr(), k.data_ptr(), v.data_ptr(), _code(q), stride(q), stride(k), stride(v),
+                                              head_decay.data_ptr(), _ptr(cos), _ptr(sin), rot_dim, cos.shape[0] if cos is not None else 0,
+                                              ctx.tok_pos.data_ptr(), float(scale), state.data_ptr(), ctx.seq_slot.data_ptr(),
+                                              ctx.seq_start.data_ptr(), ctx.batch, tokens, heads, key_dim, value_dim, out.data_ptr(),
+                                              chunks.data_ptr(), _stream()))
+        return out
     piece, pieces = run_pieces(ctx, heads * key_dim * value_dim * 4)
     carried = decayed = None
     if pieces > 1:
@@ -2243,11 +2280,13 @@ def gated_delta(rows: torch.Tensor, ba: torch.Tensor, rate: torch.Tensor, dt_bia
     _step_arrays(ctx, "gated_delta")
     # between the two kernels: the unit vectors, g and beta, and the products q . k, all 32-bit
     scratch = torch.empty(max(1, tokens * (groups * 2 * key_dim + 2 * heads + groups)), dtype=torch.float32, device=out.device)
+    chunks = chunked_scratch(ctx, tokens, heads, key_dim, value_dim, True, out.device)
     lib = recurrent()
     _check(lib, lib.nnis_gated_delta(rows.data_ptr(), _code(rows), rows.stride(0) if tokens > 1 else rows.shape[1], ba.data_ptr(),
                                      rate.data_ptr(), dt_bias.data_ptr(), float(q_scale), float(unit_eps), state.data_ptr(),
                                      ctx.seq_slot.data_ptr(), ctx.seq_start.data_ptr(), ctx.batch, tokens, heads, groups, key_dim,
-                                     value_dim, out.data_ptr(), scratch.data_ptr(), _stream()))
+                                     value_dim, out.data_ptr(), scratch.data_ptr(),
+                                     _ptr(chunks), _stream()))
     return out
 
 

@@ -1147,3 +1147,86 @@ def test_attention_in_32_bits_on_the_matrix_cores(heads, kv_heads, head_dim, val
              (items, _i32([0, 1, 2, 3]), _i32(starts), _i32(first)))
     with pytest.raises(KernelError):
         both([0], [0], splits=ops.ATTENTION_F32_MOST_SPLITS + 1)
+
+
+def _delta_in_64_bits(rows, ba, rate, dt_bias, q_scale, state, starts, heads, groups, d, e):
+    rows, ba, S = rows.double(), ba.double(), state.double().transpose(-1, -2).clone()
+    unit = lambda x: x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    q, k = (unit(rows[:, i * groups * d:(i + 1) * groups * d].view(-1, groups, d)).repeat_interleave(heads // groups, 1) for i in (0, 1))
+    v = rows[:, 2 * groups * d:2 * groups * d + heads * e].view(-1, heads, e)
+    beta, g = torch.sigmoid(ba[:, :heads]), torch.exp(-rate.double() * torch.log1p(torch.exp(ba[:, heads:] + dt_bias.double())))
+    out = torch.empty(len(rows), heads, e, dtype=torch.float64)
+    for b in range(len(starts) - 1):
+        for t in range(starts[b], starts[b + 1]):
+            S[b] *= g[t][:, None, None]
+            S[b] += k[t][:, :, None] * (beta[t][:, None] * (v[t] - torch.bmm(k[t][:, None], S[b])[:, 0]))[:, None]
+            out[t] = torch.bmm(q[t][:, None] * q_scale, S[b])[:, 0]
+    return out.view(len(rows), -1), S.transpose(-1, -2)
+
+
+def _retention_in_64_bits(q, k, v, decay, scale, state, starts, positions, rotation, heads, d, e):
+    S, out = state.double().clone(), torch.empty(len(q), heads, e, dtype=torch.float64)
+    cos, sin = (table.double()[positions][:, None] for table in rotation[:2])
+    half = rotation[2] // 2
+
+    def turned(x):
+        x = x.double().view(-1, heads, d)
+        a, b = x[..., :half], x[..., half:2 * half]
+        return torch.cat([a * cos - b * sin, b * cos + a * sin, x[..., 2 * half:]], dim=-1)
+
+    q, k, v = turned(q), turned(k), v.double().view(-1, heads, e)
+    for b in range(len(starts) - 1):
+        for t in range(starts[b], starts[b + 1]):
+            S[b] = decay.double()[:, None, None] * S[b] + k[t][:, :, None] * v[t][:, None]
+            out[t] = torch.bmm(q[t][:, None] * scale, S[b])[:, 0]
+    return out.view(len(q), -1), S
+
+
+@pytest.mark.parametrize("lengths", [(63,), (64, 65, 1), (200, 7, 128, 2), (130,)])
+@pytest.mark.parametrize("heads, groups, d, e, dtype", [(4, 2, 128, 128, torch.bfloat16), (2, 2, 16, 48, torch.float32), (3, 1, 112, 16, torch.bfloat16), (2, 1, 64, 256, torch.bfloat16)])
+@pytest.mark.parametrize("delta", [True, False])
+def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, monkeypatch):
+    """The delta rule (decays from slow to a state that is gone at once) and retention over prompts in chunks of 64 tokens and
+    a token at a time, from states that hold something, against 64 bits.  A result is a sum over up to 64 tokens or 128
+    channels that is rounded at each: 2^-24 of it, the square root of their number adding up."""
+    import types
+
+    ops = _ops()
+    torch.manual_seed(sum(lengths) + d)
+    tokens, batch, starts = sum(lengths), len(lengths), [0, *np.cumsum(lengths).tolist()]
+    positions = [40 + i for n in lengths for i in range(n)]
+    slots = list(range(batch, 0, -1))
+    ctx = types.SimpleNamespace(decode=False, batch=batch, tokens=tokens, max_new=max(lengths), planned_rows=max(lengths), seq_slot=_i32(slots), seq_start=_i32(starts),
+                                tok_slot=_i32([s for s, n in zip(slots, lengths) for _ in range(n)]), tok_pos=_i32(positions))
+    state = 0.3 * torch.randn(batch + 1, heads, *((e, d) if delta else (d, e)))
+    if delta:
+        wide = torch.randn(tokens, 2 * groups * d + heads * e + 8).to(dtype)  # (rows may be longer than what they hold)
+        ba, rate, dt_bias = torch.randn(tokens, 2 * heads), 1 + torch.rand(heads), torch.linspace(-4.0, 3.0, heads)
+        ba[tokens // 2, heads:] = 80.0  # (nothing of what was there before is left)
+        want, after = _delta_in_64_bits(wide, ba, rate, dt_bias, d ** -0.5, state[slots], starts, heads, groups, d, e)
+    else:
+        wide = torch.randn(tokens, heads * (2 * d + e) + 8).to(dtype)
+        q, k, v = wide[:, :heads * d], wide[:, heads * d:2 * heads * d], wide[:, 2 * heads * d:heads * (2 * d + e)]
+        decay = torch.tensor([1 - 2.0 ** (-1 - 3 * h) for h in range(heads)])
+        angle = torch.rand(300, d // 4 if d > 16 else 4) * 6
+        rotation = (torch.cos(angle), torch.sin(angle), 2 * angle.shape[1])
+        want, after = _retention_in_64_bits(q, k, v, decay, d ** -0.5, state[slots], starts, positions, rotation, heads, d, e)
+    made = ops.chunked_scratch
+
+    def in_chunks(ctx, tokens, *sizes):  # (whatever the lengths)
+        return made(types.SimpleNamespace(decode=False, batch=ctx.batch), tokens if tokens >= 160 * ctx.batch else 160 * ctx.batch, *sizes)
+
+    for form in (in_chunks, lambda *sizes: None):
+        monkeypatch.setattr(ops, "chunked_scratch", form)
+        held, out = state.cuda(), torch.full((tokens, heads * e), 9.0, device="cuda")
+        rows = wide.cuda()
+        if delta:
+            ops.gated_delta(rows, ba.cuda(), rate.cuda(), dt_bias.cuda(), d ** -0.5, held, ctx, heads, groups, d, e, out)
+        else:
+            q, k, v = rows[:, :heads * d], rows[:, heads * d:2 * heads * d], rows[:, 2 * heads * d:heads * (2 * d + e)]
+            ops.gla_scan(q, k, v, None, d ** -0.5, held, ctx, heads, out, head_decay=torch.stack([decay, torch.log(decay)]).cuda(),
+                         rotation=(rotation[0].cuda(), rotation[1].cuda(), rotation[2]))
+        for got, exact in ((out.cpu(), want), (held.cpu()[slots], after)):
+            error = (got.double() - exact).square().mean().sqrt() / exact.square().mean().sqrt()
+            assert error.item() <= 2.0 ** -24 * 128 ** 0.5, form
+        assert (held.cpu()[0] == state[0]).all()  # a slot that no sequence has
