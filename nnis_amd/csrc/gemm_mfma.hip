@@ -333,6 +333,13 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 template <int N>
 __device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
+// (A buffer load: of one through a global address the compiler thinks that it may come back out of order with every
+// other, and then waits for all reads and loads in flight wherever it needs one of them.)
+__device__ __forceinline__ void load_to_lds(const void* base, int offset, int uniform_offset, char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00027000), (lds_ptr_t)to, 16, offset,
+                                           uniform_offset, 0, 0);
+}
+
 extern __shared__ __align__(16) char tile_lds[];  // NS stages of BM + BN rows of BK
 
 #ifndef NNIS_TILE_GROUP_ROWS
@@ -349,10 +356,16 @@ extern __shared__ __align__(16) char tile_lds[];  // NS stages of BM + BN rows o
 // SPLIT: K is cut into ksplit parts, a block leaves its part's sums in `partial` and gemm_reduce_kernel does the
 // rest (a variant of its own, so that the other has no branch around the loads that prepare its epilogue).
 // WGM x WGN: the block's waves, each with BM / WGM rows and BN / WGN columns of the tile.  2 x 2 for the tiles of 64
-// rows; 4 x 2 for the tile of 256 x 256, which a product takes when it still gives most compute units a block: a
-// step of such a tile brings 64 KB from L2 for 8.4 MFLOP where four tiles of 64 x 128 bring 96 KB for 2.1 (measured
-// on 2048 x 16384 x 2048: 117 us against 171; 2048 x 6144 x 2048: 57 against 68; 6224 x 2048 x 8192: 188 against 308).
-template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2>
+// rows; 4 x 2 for the others of 8 waves but the tile of 256 x 256.
+// DIRECT, the tile of 256 x 256: only the activations go through LDS; a wave has 128 rows x 64 columns (2 x 4 waves)
+// and loads its columns' weights, which lie as the matrix instruction takes them, into registers a step ahead.  With both
+// operands in LDS (4 x 2 waves of 64 x 128) a step's reads and fills took LDS as long as its products the matrix units,
+// 2,048 cycles each, and two stages of 64 KB left the loads of a step half a step to arrive; now LDS has 1,280, the
+// L1 the weights' 64 KB beside the fills, and four stages fit.  Microseconds before and after, gated products: 2048 x 16384 x
+// 2048 132 / 120, 12288 x 11264 x 2048 515 / 482, 4096 x 28672 x 4096 835 / 765, 8192 x 8192 x 8192 902 / 820 (1.34 PFLOP/s; without
+// the buffer loads of load_to_lds it was no faster than before).  What bounds it now: the fill of each block, its epilogue,
+// and the clock under matrix load.
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2, bool DIRECT = false>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                     OutT y, int m, int n, int k, int col_blocks, int ksplit,
                                                                     float* __restrict__ partial) {
@@ -367,10 +380,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   constexpr int A_LOADS = BM / (8 * W), B_LOADS = BN / (8 * W);  // a wave's load instructions per step (8 rows each)
   static_assert(A_LOADS * 8 * W == BM && B_LOADS * 8 * W == BN && (64 * W) % BM == 0, "the tile must divide among the waves");
   constexpr int LOADS = A_LOADS + B_LOADS;
-  constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = (BM + BN) * BK * 2;
+  constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = (BM + (DIRECT ? 0 : BN)) * BK * 2;
 
   const int tid = threadIdx.x;
-  const int wave = tid / kWave, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;  // (the wave's number as a scalar)
   const int wave_m = wave / WGN, wave_n = wave % WGN;
   const int r = lane % 16, g = lane / 16;
   // Blocks go to the chip's 8 dies in turn (block i to die i % 8), and each die has an L2 of its own: the
@@ -402,34 +415,45 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 
-  // what this lane loads: its chunk (the same for every load: rows 8 apart) of rows 8 (W o + wave) + lane / 8
-  const bf16_t* a_src[A_LOADS];
-  const bf16_t* b_src[B_LOADS];
+  // What this lane loads: its chunk (the same for every load: rows 8 apart) of rows 8 (W o + wave) + lane / 8, as bytes
+  // from the tile's first row, which is the same in every lane.
+  const bf16_t* a_base = x + (size_t)row0 * k;
+  int a_off[A_LOADS];
   const int chunk_k = ((lane % 8) ^ (lane / 8)) * 8;
 #pragma unroll
   for (int o = 0; o < A_LOADS; ++o) {
-    int row = row0 + (o * W + wave) * 8 + lane / 8;
-    row = row < m ? row : m - 1;
-    a_src[o] = x + (size_t)row * k + chunk_k;
+    const int row = (o * W + wave) * 8 + lane / 8;
+    a_off[o] = ((row0 + row < m ? row : m - 1 - row0) * k + chunk_k) * 2;
   }
   constexpr int EPI = scaled_epilogue<OutT>::value;  // -1: the product is stored or added as it is
   constexpr bool kPaired = EPI == EPI_SILU || EPI == EPI_ROPE;
   // The weights are packed in the order the matrix instruction takes them: a load instruction copies one half of
-  // a strip's chunk (1 KB, lane l's 16 bytes to place l) and the stage holds [strip of the tile][half][lane].
+  // a strip's chunk (1 KB, lane l's 16 bytes to place l) and the stage holds [strip of the tile][half][lane].  DIRECT: they
+  // go into registers, one half of each strip of the wave's own columns a load.  Bytes from the wave's first row (of
+  // its pairs' lower or upper rows: a wave's loads into LDS all take the one or all the other).
   const int chunks = nnis_packed_chunks(k);
+  constexpr int B_PIECES = DIRECT ? TN : B_LOADS;
+  int b_off[B_PIECES], base_row[DIRECT && kPaired ? 2 : 1];
+  const bf16_t* b_base[DIRECT && kPaired ? 2 : 1];
 #pragma unroll
-  for (int o = 0; o < B_LOADS; ++o) {
-    const int piece = o * W + wave;  // (strip of the tile, half)
+  for (int o = 0; o < B_PIECES; ++o) {
+    const int piece = DIRECT ? 2 * (wave_n * TN + o) : o * W + wave;  // (strip of the tile, half)
     const int tile_row = (piece / 2) * 16 + r;
+    const int which = DIRECT && kPaired ? o % 2 : 0;  // (strips of lower and upper rows alternate)
     int row;
     if constexpr (kPaired) {
       row = paired_weight_row<EPI, BN, WGN>(y.rope, col_block, tile_row, n);
-      row = row >= 0 ? row : 0;  // rows beyond the end read a valid row and are not stored
     } else {
       row = col0 + tile_row;
       row = row < n ? row : n - 1;
     }
-    b_src[o] = w + nnis_packed_lane(row, g, k) + (piece % 2) * kPackedHalfElems;
+    if (o == which) {
+      const int first = __builtin_amdgcn_readfirstlane(row);
+      base_row[which] = first >= 0 ? first : 0;
+      b_base[which] = w + nnis_packed_lane(base_row[which], 0, k);
+    }
+    row = row >= 0 ? row : base_row[which];  // rows beyond the end read a valid row and are not stored
+    b_off[o] = (int)(w + nnis_packed_lane(row, g, k) - b_base[which] + (DIRECT ? 0 : (piece % 2) * kPackedHalfElems)) * 2;
   }
   // Step s lies in stage s % NS.  A step first asks for the step NS - 1 ahead, into the
   // stage that was read a step ago (every wave is past the barrier that ended that step, and what it read
@@ -451,13 +475,24 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
     const int from = k0 <= last_chunk ? k0 : last_chunk;
 #pragma unroll
     for (int o = 0; o < A_LOADS; ++o)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(a_src[o] + from), (lds_ptr_t)(base + o * W * 1024), 16, 0, 0);
+      load_to_lds(a_base, a_off[o] + from * 2, 0, base + o * W * 1024);
+    if constexpr (DIRECT) return;
     const size_t from_chunk = (size_t)(step < chunks ? step : chunks - 1) * kPackedChunkElems;
 #pragma unroll
     for (int o = 0; o < B_LOADS; ++o)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(b_src[o] + from_chunk), (lds_ptr_t)(base + A_BYTES + o * W * 1024), 16, 0, 0);
+      load_to_lds(b_base[0], b_off[o], (int)(from_chunk * 2), base + A_BYTES + o * W * 1024);
   };
 
+  bf16x8 direct[DIRECT ? 2 : 1][DIRECT ? 2 : 1][DIRECT ? TN : 1];  // the weights of two steps: [step % 2][half]
+  auto ask_direct = [&](int step, int half, bf16x8 (&into)[DIRECT ? TN : 1]) {
+    const size_t from = (size_t)(step < chunks ? step : chunks - 1) * kPackedChunkElems + half * kPackedHalfElems;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) into[j] = *(const bf16x8*)((const char*)(b_base[DIRECT && kPaired ? j % 2 : 0] + from) + (unsigned)b_off[j]);
+  };
+  if constexpr (DIRECT) {
+    ask_direct(step0, 0, direct[0][0]);
+    ask_direct(step0, 1, direct[0][1]);
+  }
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) ask(step0 + s, s);
 
@@ -466,6 +501,16 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   constexpr int PG = 64 * W / BM;  // threads a row of the tile has for the parts of its sum of squares
   __shared__ float row_scale[EPI >= 0 ? PG : 1][EPI >= 0 ? BM : 1];  // each thread's share of a row's sum of squares
   int tok_pos[TM], tok_page[TM];
+  auto ask_places = [&](const auto& to) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      int token = row0 + wave_m * WM + i * 16 + r;
+      token = token < m ? token : m - 1;
+      const int slot = to.rope.tok_page ? 0 : to.rope.tok_slot[token];
+      tok_pos[i] = to.rope.tok_pos[token];
+      tok_page[i] = rope_page(to.rope, token, slot, tok_pos[i]);
+    }
+  };
   if constexpr (EPI >= 0 && !SPLIT) {  // (with K in parts the reduce kernel does this)
     // a thread takes the parts pg, pg + PG, .. of its row: eight loads at a time, none waiting for another
     const int tile_row = tid % BM, pg = tid / BM;
@@ -495,16 +540,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       }
     }
     row_scale[pg][tile_row] = total;
-    if constexpr (EPI == EPI_ROPE) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        int token = row0 + wave_m * WM + i * 16 + r;
-        token = token < m ? token : m - 1;
-        const int slot = y.rope.tok_page ? 0 : y.rope.tok_slot[token];
-        tok_pos[i] = y.rope.tok_pos[token];
-        tok_page[i] = rope_page(y.rope, token, slot, tok_pos[i]);
-      }
-    }
+    if constexpr (EPI == EPI_ROPE && !DIRECT) ask_places(y);
   }
 
   // a residual epilogue asks for the stream and the gain before the product (small tiles: registers)
@@ -524,7 +560,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       }
   }
 
-  wait_loads_but<(NS - 2) * LOADS>();
+  wait_loads_but<DIRECT ? 0 : (NS - 2) * LOADS>();  // (DIRECT: the loop counts whole steps' loads from its first on)
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   int stage = 0;
@@ -535,7 +571,62 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   // read of a stage is still waited for before the barrier that lets the stage be filled again, and a sum takes
   // its halves in the same order as before.
   constexpr bool kCarry = TM * TN <= 16 && W == 8;
-  if constexpr (kCarry) {
+  if constexpr (DIRECT) {
+    // A step in four groups of products, half by half and TM / 2 row tiles each.  A group's rows are read under the
+    // products of the group before it, the last group is multiplied behind the step's barrier; the next step's weights are
+    // asked for in the first two groups, the activations NS - 1 steps ahead in the third.
+    constexpr int Q = TM / 2;  // rows of a quarter step: a half's tiles in two groups
+    bf16x8 a[2][Q];
+    auto read = [&](int from, int half, int group, bf16x8 (&into)[Q]) {
+      const bf16x8* a_tile = (const bf16x8*)(tile_lds + from * STAGE_BYTES);
+#pragma unroll
+      for (int i = 0; i < Q; ++i) into[i] = a_tile[swizzled<CH>(wave_m * WM + (group * Q + i) * 16 + r, g * 2 + half)];
+    };
+    auto multiply = [&](const bf16x8 (&rows)[Q], int group, const bf16x8 (&b)[TN]) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < Q; ++i) acc[group * Q + i][j] = mfma(b[j], rows[i], acc[group * Q + i][j]);
+      __builtin_amdgcn_s_setprio(0);
+    };
+    auto run = [&](int step, bf16x8 (&here)[2][TN], bf16x8 (&next)[2][TN]) {
+      ask_direct(step + 1, 0, next[0]);
+      read(stage, 0, 1, a[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(a[0], 0, here[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      ask_direct(step + 1, 1, next[1]);
+      read(stage, 1, 0, a[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(a[1], 1, here[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
+      read(stage, 1, 1, a[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(a[0], 0, here[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      wait_loads_but<(NS - 2) * (A_LOADS + 2 * TN)>();  // the activations of the step behind the barrier have arrived
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      stage = stage + 1 == NS ? 0 : stage + 1;
+      read(stage, 0, 0, a[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(a[1], 1, here[1]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    read(0, 0, 0, a[0]);
+    int step = step0;
+    for (; step + 1 < step1; step += 2) {
+      run(step, direct[0], direct[1]);
+      run(step + 1, direct[1], direct[0]);
+    }
+    if (step < step1) run(step, direct[0], direct[1]);
+    if constexpr (EPI == EPI_ROPE) ask_places(y);
+  } else if constexpr (kCarry) {
     static_assert(BK == 64, "two halves of 32 k a step");
     bf16x8 a0[TM], b0[TN], a1[TM], b1[TN];
     auto read_half = [&](int from, int half, bf16x8 (&a)[TM], bf16x8 (&b)[TN]) {
@@ -581,11 +672,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
     }
   } else {
   for (int step = step0; step < step1; ++step) {
-    // The tile of 256 x 256 asks for the next step between its two halves, under the first half's products
-    // (2048 x 16384 x 2048 137 us against 141, 6224 x 11264 x 2048 277 against 294); the tile of 256 x 192, whose
-    // steps are shorter, loses by the later start of its loads (2048 x 11264 x 2048 105 against 95).
-    constexpr bool kAskBetween = TM * TN > 16 && BN >= 256;
-    if constexpr (!kAskBetween) ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
+    ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
     const bf16x8* a_tile = (const bf16x8*)(tile_lds + stage * STAGE_BYTES);
     const bf16x8* b_tile = (const bf16x8*)(tile_lds + stage * STAGE_BYTES + A_BYTES);
     static_assert(BK == 64, "two halves of 32 k a step");
@@ -614,9 +701,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       }
       __builtin_amdgcn_sched_group_barrier(0x008, 2 * TM * TN - (TM + TN), 0);
     } else {
-      // a wave tile of 64 x 128: the operands of one half at a time (registers); the other wave of the SIMD
-      // multiplies while this one reads.  (The reads of a half spread between its products, each two groups of
-      // four products ahead of its use, by scheduling barriers: 136 us against 139 on 2048 x 16384 x 2048.)
+      // a wave tile of 64 x 96: the operands of one half at a time (registers); the other wave of the SIMD
+      // multiplies while this one reads
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         bf16x8 a_frag[TM], b_frag[TN];
@@ -628,9 +714,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
         for (int jj = 0; jj < TN; ++jj)
 #pragma unroll
           for (int i = 0; i < TM; ++i) acc[i][jj] = mfma(b_frag[jj], a_frag[i], acc[i][jj]);
-        if constexpr (kAskBetween) {
-          if (half == 0) ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
-        }
       }
     }
     // what this wave read of its stage has arrived too: the stage is the next step's to fill
@@ -667,6 +750,15 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       return 1.0f / sqrtf(total / (float)k + y.eps);
     } else {
       return 1.0f;
+    }
+  };
+  // A part of a row's sum of squares covers half the tile's columns: one wave column of two, or two of DIRECT's four
+  __shared__ float squares[kResidual && DIRECT ? WGN : 1][kResidual && DIRECT ? BM : 1];
+  auto put_squares = [&](int i, int token, float sq) {
+    if (g != 0) return;
+    if constexpr (kResidual && DIRECT) squares[wave_n][wave_m * WM + i * 16 + r] = sq;
+    else if constexpr (kResidual) {
+      if (token < m) y.ss[(size_t)(col_block * WGN + wave_n) * m + token] = sq;
     }
   };
   // first operand = weight rows: lane holds D[n = 4g + e][token = r]
@@ -723,9 +815,15 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       // a part of the row's sum of squares: this wave's columns
       sq += __shfl_xor(sq, 16, kWave);
       sq += __shfl_xor(sq, 32, kWave);
-      if (g == 0 && token < m) y.ss[(size_t)(col_block * WGN + wave_n) * m + token] = sq;
+      put_squares(i, token, sq);
     }
   }
+  }
+  if constexpr (kResidual && DIRECT) {
+    static_assert(WGN == 4 && 64 * W == 2 * BM, "a thread has one part of one row");
+    __syncthreads();
+    const int row = tid % BM, part_of = tid / BM;
+    if (row0 + row < m) y.ss[(size_t)(col_block * 2 + part_of) * m + row0 + row] = squares[2 * part_of][row] + squares[2 * part_of + 1][row];
   }
   }  // !SPLIT
 }
@@ -935,15 +1033,15 @@ int tiled_ksplit(int tiles, int m, int width, int k, size_t workspace_bytes) {
   return ksplit;
 }
 
-template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2>
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2, bool DIRECT = false>
 void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int col_blocks, int row_blocks, int ksplit,
                          Workspace ws, hipStream_t stream) {
-  constexpr int lds_bytes = NS * (BM + BN) * BK * 2;
+  constexpr int lds_bytes = NS * (BM + (DIRECT ? 0 : BN)) * BK * 2;
   // beyond 64 KB a kernel has to be told once; a refusal shows as the launch's failure
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN>,
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, DIRECT>,
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
   (void)allowed;
-  hipLaunchKernelGGL((gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN>), dim3((unsigned)col_blocks * row_blocks * ksplit),
+  hipLaunchKernelGGL((gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, DIRECT>), dim3((unsigned)col_blocks * row_blocks * ksplit),
                      dim3(64 * WGM * WGN), lds_bytes, stream, x, w, y, m, n, k, col_blocks, ksplit, ws.floats);
 }
 
@@ -952,7 +1050,11 @@ void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n,
 template <int BN, typename OutT>
 int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
   const int col_blocks = (columns + BN - 1) / BN, row_blocks = (m + 255) / 256;
-  launch_tiled_kernel<256, BN, 64, 2, false, OutT, 4, 2>(x, w, y, m, n, k, col_blocks, row_blocks, 1, {nullptr, 0}, stream);
+  if constexpr (BN == 256) {
+    launch_tiled_kernel<256, 256, 64, 4, false, OutT, 2, 4, true>(x, w, y, m, n, k, col_blocks, row_blocks, 1, {nullptr, 0}, stream);
+  } else {
+    launch_tiled_kernel<256, BN, 64, 2, false, OutT, 4, 2>(x, w, y, m, n, k, col_blocks, row_blocks, 1, {nullptr, 0}, stream);
+  }
   return 2 * col_blocks;
 }
 
@@ -1006,19 +1108,12 @@ int launch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, 
 // stages, a step's second half multiplied behind the barrier).
 //
 // Among the five the one whose rounds of blocks (blocks / 256 compute units, rounded up) come to the least tile area
-// over the tile's rate.  Rates, from full rounds at K = 2048 over weights from memory, relative to 256x128 (32768
-// outputs in 35.5 us): 256x256 1.10, 256x192 1.08, 128x192 0.91, 128x128 0.82.  The rule names the fastest tile, or
-// one within a few per cent of it, on all of 77 products of 256 to 4,096 rows with 2,048 to 16,384 columns (auto
-// against each tile asked for); a few of them, microseconds: 2048 x 16384 in 512 tiles of 256x256 128 (256x128: 141);
-// 2048 x 6144 in 256 of 256x192 49 (256x256, 192 tiles: 56); 3072 x 6144 in 768 of 128x192 80 (384 of 256x192: 92);
-// 1536 x 16384 in 768 of 256x128 99 (384 of 256x256: 113); 4096 x 2048 in 256 of 256x128 35.5 (512 of 128x128: 43);
-// 2048 x 2560 in 224 of 128x192 26.5 (64x128: 29); 2048 x 2048 in 256 of 128x128 21.6 (64x128: 23.6).  At a K of
-// 8,192 the three-stage tiles gain on the others (4096 x 2048 x 8192 in 256 of 256x128: 117 us, 1.18 PFLOP/s): from
-// a K of 8,192 on the rates are 256x256 0.97, 256x192 0.93, 128x192 0.90, 128x128 0.80 of 256x128, from 4,096 on
-// the same but 256x256 1.03 (4096 x 6144 x 8192 in 768 tiles of 256x128 347 us against 383 in 512 of 256x192; 2048 x 28672 x
-// 4096 in 1792 of them 438 against 473 in 896 of 256x256); there the rule is within a tenth of the fastest tile on
-// the same 77 products but one (1536 x 6144 x 8192: 190 in 192 tiles of 256x192, 162 in 384 of 128x192, a round and
-// a half that the rule below keeps out).
+// over the tile's rate.  Rates, from full rounds over weights from memory, relative to 256x128 (32768 outputs in 33 us at a K
+// of 2,048, 60 at 4,096, 112 at 8,192): 256x256 1.10, 1.08 and 1.05, 256x192 1.01, 0.90 and 0.93, 128x192 0.90, 128x128
+// 0.81.  A few of them, microseconds, gated products: 2048 x 16384 in 512 tiles of 256x256 120 (256x128: 133); 2048 x 6144
+// in 256 of 256x192 47 (256x256, 192 tiles: 51; 512 of 128x192: 55); 4096 x 2048 in 256 of 256x128 34 (512 of 128x128:
+// 41); 4096 x 2048 x 8192 110 (128x128: 136); 12288 x 2048 x 5632 in 768 of 256x128 232 (384 of 256x256, a round and a
+// half: 241); 4096 x 28672 x 4096 in 1792 of 256x256 765 (256x128: 817).
 //
 // What keeps a tile out:
 //  * rows that do not fill its row blocks: 300 rows would be multiplied as 512.  Three quarters for the three-stage
@@ -1041,7 +1136,7 @@ int pick_tile(int m, int columns, int k, int tile_hint) {
   struct Candidate { int tile, rows, width, rate[3], stages; };  // rates for a K below 4,096, below 8,192, and beyond
   const int depth = k >= 8192 ? 2 : (k >= 4096 ? 1 : 0);
   long long best = 0;
-  for (const Candidate c : {Candidate{4, 256, 256, {110, 103, 97}, 2}, Candidate{5, 256, 192, {108, 93, 93}, 2},
+  for (const Candidate c : {Candidate{4, 256, 256, {110, 108, 105}, 2}, Candidate{5, 256, 192, {101, 90, 93}, 2},
                             Candidate{7, 256, 128, {100, 100, 100}, 3}, Candidate{8, 128, 192, {91, 90, 90}, 3},
                             Candidate{6, 128, 128, {82, 80, 80}, 3}}) {
     const long long row_blocks = (m + c.rows - 1) / c.rows;
