@@ -793,6 +793,43 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
         }
       }
     }
+  } else if (kResidual && !kAskEarly && vector_ok && col0 + BN <= n) {
+    // Whole columns: up to four row tiles of the stream asked for ahead, nothing behind a branch, the gains once.  (Each
+    // tile of 16 x 16 asked for and waited for by itself cost a block 35 us where its product took 50.  Microseconds before
+    // and after: 12288 x 2048 x 2048 140 / 122, 12288 x 2048 x 5632 317 / 286, 2048 x 8192 x 2048 97 / 79, 8192 x 8192 x 8192 1041 / 987.)
+    if constexpr (kResidual) {
+      constexpr int kAhead = TM < 4 ? TM : 4;
+      f32x4 stream[kAhead][TN];
+      ResidualHeld taken[TN];
+      auto row_of = [&](int i) { return row0 + wave_m * WM + i * 16 + r; };
+      const int n0 = col0 + wave_n * WN + g * 4;
+      auto ask_row = [&](int i) {
+        const int token = row_of(i) < m ? row_of(i) : m - 1;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) stream[i % kAhead][j] = *(const f32x4*)(y.resid + (size_t)token * n + n0 + j * 16);
+      };
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) ask_row(i);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) taken[j] = residual_ask_gain(y, n0 + j * 16);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int token = row_of(i);
+        float sq = 0.0f;
+        if (token < m) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            taken[j].v = stream[i % kAhead][j];
+            sq += residual_take(y, taken[j], (size_t)token * n + n0 + j * 16, acc[i][j], 4, true);
+          }
+        }
+        if (i + kAhead < TM) ask_row(i + kAhead);
+        sq += __shfl_xor(sq, 16, kWave);
+        sq += __shfl_xor(sq, 32, kWave);
+        put_squares(i, token, sq);
+      }
+    }
   } else {
 #pragma unroll
   for (int i = 0; i < TM; ++i) {

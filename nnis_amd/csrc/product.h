@@ -72,19 +72,28 @@ struct ResidualHeld {
   f32x4 v, g;
 };
 
+// the gains of four whole columns
+__device__ __forceinline__ ResidualHeld residual_ask_gain(const ResidualOut& o, int column) {
+  ResidualHeld h;
+  h.v = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  h.g = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  if (o.gain_dtype == NNIS_F32) {
+    h.g = *(const f32x4*)((const float*)o.gain + column);
+  } else {
+    const float2 packed = *(const float2*)((const bf16_t*)o.gain + column);
+    h.g[0] = packed.x;
+    h.g[1] = packed.y;
+  }
+  return h;
+}
+
 __device__ __forceinline__ ResidualHeld residual_ask(const ResidualOut& o, size_t index, int column, int valid, bool vector_ok) {
   ResidualHeld h;
   h.v = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   h.g = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   if (valid == 4 && vector_ok) {
+    h = residual_ask_gain(o, column);
     h.v = *(const f32x4*)(o.resid + index);
-    if (o.gain_dtype == NNIS_F32) {
-      h.g = *(const f32x4*)((const float*)o.gain + column);
-    } else {
-      const float2 packed = *(const float2*)((const bf16_t*)o.gain + column);
-      h.g[0] = packed.x;
-      h.g[1] = packed.y;
-    }
   } else {
     for (int e = 0; e < valid; ++e) {
       h.v[e] = o.resid[index + e];
