@@ -26,7 +26,6 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((address_space(1))) const void* global_ptr_t;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 template <int N>
@@ -347,6 +346,14 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_few_kernel(const XT* __restri
 constexpr int kStepK = 32;      // k of a step: 128 bytes of a row, 8 chunks of 16 bytes
 constexpr int kFlushSteps = 8;  // a chain of sums is this many steps long, then goes into the total
 
+// (A buffer load: of one through a global address the compiler thinks that it may come back out of order with every
+// other, and then waits for all reads and loads in flight wherever it needs one of them.  A prompt of 509 tokens through a
+// 1.1B model 10.39 -> 9.97 ms.)
+__device__ __forceinline__ void load_to_lds(const void* base, int offset, char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00027000), (lds_ptr_t)to, 16, offset, 0,
+                                           0, 0);
+}
+
 extern __shared__ __align__(16) char f32_lds[];  // NS stages of BM rows of X and BN rows of W
 
 // 4 waves, 2 x 2, each with BM / 2 rows and BN / 2 columns.  A load instruction of a wave brings 8 rows of 128 bytes
@@ -361,7 +368,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   constexpr int TM = BM / 32, TN = BN / 32;  // tiles of 16 x 16 a wave has, each way
   constexpr int A_LOADS = BM / 32, B_LOADS = BN / 32, LOADS = A_LOADS + B_LOADS;  // load instructions a wave and step
   constexpr int A_BYTES = BM * kStepK * 4, STAGE_BYTES = (BM + BN) * kStepK * 4;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int wave_m = wave / 2, wave_n = wave % 2;
   const int r = lane % 16, g = lane / 16;
   // blocks go to the 8 dies in turn: a die's blocks are consecutive tiles, rows fastest, so that its L2 holds a few
@@ -378,12 +385,15 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   const int row0 = row_block * BM, col0 = col_block * BN;
 
   const int chunk_k = ((lane % 8) ^ (lane / 8)) * 4;  // the first k of this lane's chunk of a step
-  const float* a_src[A_LOADS];
-  const float* b_src[B_LOADS];
+  // rows in bytes from the tile's first row, and from the first of the wave's weight rows (of its pairs' lower or upper rows:
+  // a wave's loads take the one or all the other), which are the same in every lane
+  const float* a_base = x + (size_t)row0 * k;
+  const float* b_base = w;
+  int a_off[A_LOADS], b_off[B_LOADS], base_row = 0;
 #pragma unroll
   for (int o = 0; o < A_LOADS; ++o) {
-    const int row = row0 + (o * 4 + wave) * 8 + lane / 8;
-    a_src[o] = x + (size_t)(row < m ? row : m - 1) * k;
+    const int row = (o * 4 + wave) * 8 + lane / 8;
+    a_off[o] = (row0 + row < m ? row : m - 1 - row0) * k * 4;
   }
 #pragma unroll
   for (int o = 0; o < B_LOADS; ++o) {
@@ -391,7 +401,12 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
     int row;
     if constexpr (kPaired) row = paired_row<EPI, 16>(f, col_block * (BN / 32) + in_tile / 32, in_tile / 16 % 2, in_tile % 16, n);
     else row = col0 + in_tile;
-    b_src[o] = w + (size_t)(row >= 0 && row < n ? row : n - 1) * k;
+    if (o == 0) {
+      const int first = __builtin_amdgcn_readfirstlane(row);
+      base_row = first >= 0 && first < n ? first : n - 1;
+      b_base = w + (size_t)base_row * k;
+    }
+    b_off[o] = (row >= 0 && row < n ? row - base_row : 0) * k * 4;  // (rows beyond the end: a valid one, not stored)
   }
   // Step s lies in stage s % NS.  A step beyond the end, and the last step's chunks beyond K, are asked for from the
   // row's first chunk: valid memory; the former nobody reads, the latter count as zeros.
@@ -399,13 +414,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   auto ask = [&](int step, int stage) {
     char* base = f32_lds + stage * STAGE_BYTES + wave * 1024;
     const int at = step * kStepK + chunk_k;
-    const int from = at < k ? at : 0;
+    const int from = (at < k ? at : 0) * 4;
 #pragma unroll
-    for (int o = 0; o < A_LOADS; ++o)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(a_src[o] + from), (lds_ptr_t)(base + o * 4096), 16, 0, 0);
+    for (int o = 0; o < A_LOADS; ++o) load_to_lds(a_base, a_off[o] + from, base + o * 4096);
 #pragma unroll
-    for (int o = 0; o < B_LOADS; ++o)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(b_src[o] + from), (lds_ptr_t)(base + A_BYTES + o * 4096), 16, 0, 0);
+    for (int o = 0; o < B_LOADS; ++o) load_to_lds(b_base, b_off[o] + from, base + A_BYTES + o * 4096);
   };
 
   f32x4 sum[TM][TN], total[TM][TN];
