@@ -16,7 +16,8 @@
 //    waves, or, where a product still fills the chip with them, 256x256 or
 //    256x192 tiles of 8 waves; K in steps of 64 that go from memory straight
 //    into LDS, a ring of stages deep, with an XOR swizzle of the 16-byte
-//    chunks so that operand reads are free of bank conflicts.
+//    chunks so that operand reads are free of bank conflicts (the 256x256
+//    tile's weights go into registers).
 //
 // Both need K % 8 == 0 and 16-byte aligned operands (the host checks) and take
 // any M and N.
@@ -752,13 +753,24 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
       return 1.0f;
     }
   };
-  // A part of a row's sum of squares covers half the tile's columns: one wave column of two, or two of DIRECT's four
-  __shared__ float squares[kResidual && DIRECT ? WGN : 1][kResidual && DIRECT ? BM : 1];
+  // A part of a row's sum of squares covers half the tile's columns: a wave column of two, or two of DIRECT's four.  The
+  // latter leave what each lane took, tile by tile, in LDS, and are added as one wave over both would: left to right, then
+  // over the lane groups, so that a row's norm does not depend on how a tile's waves lie.
+  constexpr bool kMeet = kResidual && DIRECT;
+  float* squares = (float*)tile_lds;  // kMeet: [row][part][lane group][8 column tiles]
+  if constexpr (kMeet) {
+    static_assert(WGN == 4 && TN == 4 && 64 * W >= 2 * BM && BM * 64 * 4 <= NS * STAGE_BYTES, "a part is the eight column tiles of two waves");
+    __syncthreads();  // (all loads have arrived, and nobody reads a stage any more)
+  }
+  auto take_square = [&](int i, int j, float& sq, float of_tile) {
+    if constexpr (kMeet) squares[(wave_m * WM + i * 16 + r) * 64 + (((wave_n / 2) * 4 + g) * 8 + wave_n % 2 * 4 + j ^ (r % 8) * 4)] = of_tile;
+    else sq += of_tile;
+  };
   auto put_squares = [&](int i, int token, float sq) {
-    if (g != 0) return;
-    if constexpr (kResidual && DIRECT) squares[wave_n][wave_m * WM + i * 16 + r] = sq;
-    else if constexpr (kResidual) {
-      if (token < m) y.ss[(size_t)(col_block * WGN + wave_n) * m + token] = sq;
+    if constexpr (kResidual && !kMeet) {
+      sq += __shfl_xor(sq, 16, kWave);
+      sq += __shfl_xor(sq, 32, kWave);
+      if (g == 0 && token < m) y.ss[(size_t)(col_block * WGN + wave_n) * m + token] = sq;
     }
   };
   // first operand = weight rows: lane holds D[n = 4g + e][token = r]
@@ -821,12 +833,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             taken[j].v = stream[i % kAhead][j];
-            sq += residual_take(y, taken[j], (size_t)token * n + n0 + j * 16, acc[i][j], 4, true);
+            take_square(i, j, sq, residual_take(y, taken[j], (size_t)token * n + n0 + j * 16, acc[i][j], 4, true));
           }
         }
         if (i + kAhead < TM) ask_row(i + kAhead);
-        sq += __shfl_xor(sq, 16, kWave);
-        sq += __shfl_xor(sq, 32, kWave);
         put_squares(i, token, sq);
       }
     }
@@ -841,26 +851,34 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
     for (int j = 0; j < TN; ++j) {
       const int n0 = col0 + wave_n * WN + j * 16 + g * 4;
       const int valid = n - n0 >= 4 ? 4 : (n - n0 > 0 ? n - n0 : 0);
-      if (token >= m || valid <= 0) continue;
+      if (token >= m || valid <= 0) {
+        if constexpr (kMeet) take_square(i, j, sq, 0.0f);
+        continue;
+      }
       if constexpr (kResidual) {
-        if constexpr (kAskEarly) sq += residual_take(y, held[i][j], (size_t)token * n + n0, acc[i][j], valid, vector_ok);
-        else sq += residual_take(y, residual_ask(y, (size_t)token * n + n0, n0, valid, vector_ok), (size_t)token * n + n0, acc[i][j], valid, vector_ok);
+        if constexpr (kAskEarly) take_square(i, j, sq, residual_take(y, held[i][j], (size_t)token * n + n0, acc[i][j], valid, vector_ok));
+        else take_square(i, j, sq, residual_take(y, residual_ask(y, (size_t)token * n + n0, n0, valid, vector_ok), (size_t)token * n + n0, acc[i][j], valid, vector_ok));
       } else if constexpr (EPI == EPI_STORE) store4(y.y, (size_t)token * n + n0, acc[i][j] * scale, valid, vector_ok);
       else store4(y, (size_t)token * n + n0, acc[i][j], valid, vector_ok);
     }
     if constexpr (kResidual) {
-      // a part of the row's sum of squares: this wave's columns
-      sq += __shfl_xor(sq, 16, kWave);
-      sq += __shfl_xor(sq, 32, kWave);
       put_squares(i, token, sq);
     }
   }
   }
-  if constexpr (kResidual && DIRECT) {
-    static_assert(WGN == 4 && 64 * W == 2 * BM, "a thread has one part of one row");
+  if constexpr (kMeet) {
     __syncthreads();
     const int row = tid % BM, part_of = tid / BM;
-    if (row0 + row < m) y.ss[(size_t)(col_block * 2 + part_of) * m + row0 + row] = squares[2 * part_of][row] + squares[2 * part_of + 1][row];
+    if (part_of < 2 && row0 + row < m) {
+      float lanes[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        lanes[q] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) lanes[q] += squares[row * 64 + ((part_of * 4 + q) * 8 + t ^ (row % 8) * 4)];
+      }
+      y.ss[(size_t)(col_block * 2 + part_of) * m + row0 + row] = (lanes[0] + lanes[1]) + (lanes[2] + lanes[3]);
+    }
   }
   }  // !SPLIT
 }
@@ -1082,7 +1100,7 @@ void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n,
                      dim3(64 * WGM * WGN), lds_bytes, stream, x, w, y, m, n, k, col_blocks, ksplit, ws.floats);
 }
 
-// the tile of 256 x 256 (8 waves, 2 stages of 64 KB, one block a compute unit); returns the parts of a row's sum of
+// the tiles of 256 x 256 (DIRECT, 4 stages of 32 KB) and 256 x 192 (2 of 56 KB), 8 waves, one block a compute unit; returns the parts of a row's sum of
 // squares that a residual epilogue wrote: one per wave column
 template <int BN, typename OutT>
 int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
@@ -1150,14 +1168,17 @@ int launch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, 
 // 0.81.  A few of them, microseconds, gated products: 2048 x 16384 in 512 tiles of 256x256 120 (256x128: 133); 2048 x 6144
 // in 256 of 256x192 47 (256x256, 192 tiles: 51; 512 of 128x192: 55); 4096 x 2048 in 256 of 256x128 34 (512 of 128x128:
 // 41); 4096 x 2048 x 8192 110 (128x128: 136); 12288 x 2048 x 5632 in 768 of 256x128 232 (384 of 256x256, a round and a
-// half: 241); 4096 x 28672 x 4096 in 1792 of 256x256 765 (256x128: 817).
+// half: 241); 4096 x 28672 x 4096 in 1792 of 256x256 765 (256x128: 817).  A product into the stream leaves its rows' sums
+// of squares in parts of a wave's columns, so another tile is another rounding of the norm: it goes by rates of its own
+// (256x256 1.10, 1.03, 0.97 and 256x192 1.08, 0.93, 0.93, from tiles whose epilogue waited for each load), which name
+// the fastest tile or one within 7% of it (8192 x 8192 x 8192 1,008 us in tiles of 256x128, 987 in 256x256).
 //
 // What keeps a tile out:
 //  * rows that do not fill its row blocks: 300 rows would be multiplied as 512.  Three quarters for the three-stage
 //    tiles (384 x 16384 x 4096 as 512 rows in 256 tiles of 256x128: 61 us against 75 in tiles of 64x128); for the two-stage ones three quarters from 1,024 rows on and fifteen sixteenths below (384 x 16384 x
 //    2048 as 512 rows of 256x192 took 44.5 us against 34.2 in tiles of 64x128);
 //  * blocks too few for the chip, against the 4-wave tiles, which several of fit a compute unit: the two-stage tiles
-//    want 160 blocks (1024 x 6144 x 2048 in 128 tiles: 44 us against 34), a single round of the others five eighths
+//    (256x256 with them) want 160 blocks (1024 x 6144 x 2048 in 128 tiles: 44 us against 34), a single round of the others five eighths
 //    of the compute units (1024 x 2560 x 2048 in 160 tiles of 128x128: 20.0 against 21.6; 1024 x 2048 x 8192 in 128:
 //    58 against 51; in 144, 768 x 3072 60 against 67 but 384 x 6144 77 against 68), two rounds seven eighths of them (3072 x 2048 x 4096 in 384 tiles of 128x128: 81 against 69),
 //    more rounds a last one that is half full (1280 x 16384 x 8192 in 640 tiles of 256x128: 334 against 372);
@@ -1167,13 +1188,14 @@ int launch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, 
 #ifndef NNIS_LARGE_TILE_BLOCKS
 #define NNIS_LARGE_TILE_BLOCKS 160
 #endif
-int pick_tile(int m, int columns, int k, int tile_hint) {
+int pick_tile(int m, int columns, int k, int tile_hint, bool residual = false) {
   const long long blocks_64_128 = (long long)((m + 63) / 64) * ((columns + 127) / 128);
   int tile = blocks_64_128 > 256 ? 2 : 3;
   struct Candidate { int tile, rows, width, rate[3], stages; };  // rates for a K below 4,096, below 8,192, and beyond
   const int depth = k >= 8192 ? 2 : (k >= 4096 ? 1 : 0);
   long long best = 0;
-  for (const Candidate c : {Candidate{4, 256, 256, {110, 108, 105}, 2}, Candidate{5, 256, 192, {101, 90, 93}, 2},
+  for (const Candidate c : {residual ? Candidate{4, 256, 256, {110, 103, 97}, 2} : Candidate{4, 256, 256, {110, 108, 105}, 2},
+                            residual ? Candidate{5, 256, 192, {108, 93, 93}, 2} : Candidate{5, 256, 192, {101, 90, 93}, 2},
                             Candidate{7, 256, 128, {100, 100, 100}, 3}, Candidate{8, 128, 192, {91, 90, 90}, 3},
                             Candidate{6, 128, 128, {82, 80, 80}, 3}}) {
     const long long row_blocks = (m + c.rows - 1) / c.rows;
@@ -1198,7 +1220,7 @@ int pick_tile(int m, int columns, int k, int tile_hint) {
 
 // the most parts of a row's sum of squares that a residual epilogue of the tiled kernel writes for these sizes
 int tiled_parts(int m, int columns, int k, int tile_hint) {
-  const int tile = pick_tile(m, columns, k, tile_hint);
+  const int tile = pick_tile(m, columns, k, tile_hint, true);
   const int width = tile == 4 ? 256 : (tile == 5 || tile == 8 ? 192 : (tile == 2 || tile == 6 || tile == 7 ? 128 : 64));
   return 2 * ((columns + width - 1) / width);  // with K in parts: one per 64 columns, which is no more
 }
@@ -1208,7 +1230,7 @@ template <typename OutT>
 int dispatch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int tile_hint, Workspace ws, hipStream_t stream,
                    int columns = 0) {
   if (columns <= 0) columns = n;
-  const int tile = pick_tile(m, columns, k, tile_hint);
+  const int tile = pick_tile(m, columns, k, tile_hint, std::is_same<OutT, ResidualOut>::value);
   if (tile == 4) return launch_tiled_large<256, OutT>(x, w, y, m, n, k, columns, stream);
   if (tile == 5) return launch_tiled_large<192, OutT>(x, w, y, m, n, k, columns, stream);
   if (tile == 6) return launch_tiled_medium<128, 128, OutT>(x, w, y, m, n, k, columns, stream);

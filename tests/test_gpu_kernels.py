@@ -1230,3 +1230,27 @@ def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, mon
             error = (got.double() - exact).square().mean().sqrt() / exact.square().mean().sqrt()
             assert error.item() <= 2.0 ** -24 * 128 ** 0.5, form
         assert (held.cpu()[0] == state[0]).all()  # a slot that no sequence has
+
+
+@pytest.mark.parametrize("m, k", [(70, 72), (300, 392), (530, 8), (257, 136)])
+@pytest.mark.parametrize("epilogue", ["store", "silu", "rope"])
+def test_the_tile_whose_weights_go_into_registers(epilogue, m, k):
+    """The 256 x 256 tile behind a prepared norm, at ragged rows and columns, gate rows that share a strip with up rows, and K
+    of one step to seven: every sum takes its terms in the order of the other tiles, so the rows are the 64 x 128 tile's."""
+    ops = _ops()
+    torch.manual_seed(m + k)
+    rope, heads, kv_heads, head_dim = None, 6, 2, 64
+    n = {"store": 596, "silu": 2 * 300, "rope": (heads + 2 * kv_heads) * head_dim}[epilogue]
+    code, width = {"store": (ops.EPILOGUE_STORE, n), "silu": (ops.EPILOGUE_SILU, n // 2), "rope": (ops.EPILOGUE_ROPE, heads * head_dim)}[epilogue]
+    if epilogue == "rope":
+        angle = torch.rand(64, head_dim // 2, device="cuda") * 6
+        rope = dict(cos=torch.cos(angle), sin=torch.sin(angle), tok_slot=_i32([0] * m), tok_pos=_i32([i % 64 for i in range(m)]), heads=heads,
+                    kv_heads=kv_heads, head_dim=head_dim)
+    x, weight = torch.randn(m, k).bfloat16().cuda(), ops.pack_weight((torch.randn(n, k) / math.sqrt(k)).bfloat16().cuda())
+    ss = (1.0 + torch.rand(1, m)).cuda() * k
+    rows = []
+    for tile in (ops.TILE_256x256, ops.TILE_64x128):
+        y = torch.full((m, width), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_scaled(x, ss, 1, 1e-5, weight, y, code, rope, 16 * tile)
+        rows.append(y)
+    assert torch.equal(*rows)
