@@ -1211,10 +1211,12 @@ def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, mon
         angle = torch.rand(300, d // 4 if d > 16 else 4) * 6
         rotation = (torch.cos(angle), torch.sin(angle), 2 * angle.shape[1])
         want, after = _retention_in_64_bits(q, k, v, decay, d ** -0.5, state[slots], starts, positions, rotation, heads, d, e)
-    made = ops.chunked_scratch
+    rooms = []
 
-    def in_chunks(ctx, tokens, *sizes):  # (whatever the lengths)
-        return made(types.SimpleNamespace(decode=False, batch=ctx.batch), tokens if tokens >= 160 * ctx.batch else 160 * ctx.batch, *sizes)
+    def in_chunks(ctx, tokens, *sizes):  # (whatever the lengths; the floats that such a step asks for, and three chunks' behind them)
+        need = lambda rows: ops.recurrent().nnis_chunked_scratch(rows, ctx.batch, *sizes[:4])  # noqa: E731
+        rooms.append((torch.full((need(tokens + 192),), 7.0, device=sizes[4]), need(tokens)))
+        return rooms[-1][0][:need(tokens)]
 
     for form in (in_chunks, lambda *sizes: None):
         monkeypatch.setattr(ops, "chunked_scratch", form)
@@ -1230,6 +1232,7 @@ def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, mon
             error = (got.double() - exact).square().mean().sqrt() / exact.square().mean().sqrt()
             assert error.item() <= 2.0 ** -24 * 128 ** 0.5, form
         assert (held.cpu()[0] == state[0]).all()  # a slot that no sequence has
+    assert len(rooms) == 1 and (rooms[0][0][rooms[0][1]:] == 7).all()  # nothing was written beyond what the step asks for
 
 
 @pytest.mark.parametrize("m, k", [(70, 72), (300, 392), (530, 8), (257, 136)])
