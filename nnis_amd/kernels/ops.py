@@ -1900,23 +1900,28 @@ def run_pieces(ctx, state_bytes: int):
     return (piece, pieces) if pieces > 1 else (0, 1)
 
 
-# The most scratch that a step's chunks take (147 KB a chunk and head of 128 x 256); steps beyond, of 28,000 tokens on 64
-# such heads, go a token at a time.
+# The most scratch that a step's chunks take (a chunk and head of 128 x 128 147 KB with the delta rule, of 128 x 256 82 KB with
+# retention); steps beyond, of 29,000 and 52,000 tokens on 64 such heads, go a token at a time.
 CHUNKED_MOST_BYTES = 4 << 30
 
 
 def chunked_scratch(ctx, tokens: int, heads: int, key_dim: int, value_dim: int, delta: bool, device) -> Optional[torch.Tensor]:
-    """Scratch for a step whose sequences a matrix-state recurrence walks in chunks of 64 tokens (csrc/chunked_state.hip);
-    None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts too short."""
-    # Microseconds a token at a time and in chunks, by sequences x tokens.  Delta rule, 16 heads of 128 x 128: 1 x 96 48 / 41, 1 x 64 35 /
-    # 38; 4 x 96 60 / 64, 4 x 128 76 / 67; 8 x 128 103 / 117, 8 x 192 149 / 133; 16 x 128 199 / 192.  Retention, 8 heads of 128 x 256: 1 x 16
-    # 25 / 14; 8 x 16 26 / 30, 8 x 32 42 / 31; 16 x 32 48 / 51, 16 x 64 178 / 55.  (Its token at a time is split into pieces.)
+    """Scratch for a step of ``tokens`` rows whose sequences a matrix-state recurrence walks in chunks of 64 tokens
+    (csrc/chunked_state.hip); None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts too
+    short.  Which of the two goes by the rows that the step plans for, not by those at hand: a step that is launched and the same step
+    replayed from a graph's rows take the same form (their results are rounded differently)."""
+    # Microseconds a token at a time and in chunks, by sequences x tokens; an engine's steps plan for their tokens rounded up to 64 and
+    # more, so the first of a pair that a rule takes in is given.  Delta rule, 16 heads of 128 x 128: 1 x 65 35 / 40 (planned for 128), 1 x
+    # 80 41 / 40, 1 x 128 59 / 42; 2 x 97 51 / 44; 4 x 113 68 / 66; 8 x 145 118 / 127, 8 x 192 149 / 133; 16 x 161 238 / 240.  Retention, 8
+    # heads of 128 x 256: 1 x 2 9 / 12 (planned for 64), 1 x 8 14 / 12, 1 x 16 21 / 13, 1 x 64 46 / 14; 4 x 25 29 / 19; 8 x 25 30 / 29; 16 x 33
+    # 43 / 48, 16 x 48 140 / 49.  (Its token at a time is split into pieces.)
     least = 96 + 8 * min(ctx.batch, 8) if delta else 16 + 2 * min(ctx.batch, 16)
     lib = recurrent()
-    if ctx.decode or tokens < least * max(ctx.batch, 1) or not lib.nnis_chunked_takes(key_dim, value_dim):
+    planned = max(tokens, ctx.planned_rows)
+    if ctx.decode or planned < least * max(ctx.batch, 1) or not lib.nnis_chunked_takes(key_dim, value_dim):
         return None
-    floats = lib.nnis_chunked_scratch(tokens, ctx.batch, heads, key_dim, value_dim, 1 if delta else 0)
-    return torch.empty(floats, dtype=torch.float32, device=device) if 4 * floats <= CHUNKED_MOST_BYTES else None
+    floats = lambda rows: lib.nnis_chunked_scratch(rows, ctx.batch, heads, key_dim, value_dim, 1 if delta else 0)  # noqa: E731
+    return torch.empty(floats(tokens), dtype=torch.float32, device=device) if 4 * floats(planned) <= CHUNKED_MOST_BYTES else None
 
 
 def _step_arrays(ctx, what: str):

@@ -563,6 +563,39 @@ def test_prompts_whole_in_portions_and_token_by_token(folders, name, dtype):
             yard.check(got[place], ids, dtype, f"{name} cuts {cuts[:3]}.. position {place}", rows=place)
 
 
+def test_a_prompt_launched_captured_and_replayed_takes_the_same_recurrences(tmp_path, monkeypatch):
+    """Prompts of lengths on both sides of what the delta rule and retention take in chunks at the rows a replay has (64, 128): the
+    first pass is launched, the second captured, the third replayed, and all three answer alike."""
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    config = mafalorn(vocab=200, width=64, logit_scale=1.5, layers=[
+        layer("parallel", parallel(softmax(2, 1, 16, scale=0.3), delta(2, 1, 16, 16, 4), 0.7, 0.9)), layer("retention", retention(2, 16, 16, (0.99, 0.8)))])
+    folder = _folder(tmp_path / "m", config, 7)
+    engine = nnis_amd.load_engine(folder, dtype="float32", max_tokens=512)
+    yard, forms, made = Yardstick(P.PlainMafalorn(folder)), [], ops.chunked_scratch
+
+    def watched(*args):
+        scratch = made(*args)
+        forms.append(scratch is not None)
+        return scratch
+
+    monkeypatch.setattr(ops, "chunked_scratch", watched)
+    for length, chunks in ((10, [False, True]), (60, [False, True]), (70, [True, True]), (103, [True, True]), (128, [True, True])):
+        engine._prefill_graphs = None
+        ids = _ids(length, config["vocab"], length)
+        for turn in ("launched", "captured", "replayed"):
+            forms.clear()
+            slot = engine.start_sequence()
+            rows = engine.step([StepEntry(slot, ids, [0, length - 1])]).cpu()
+            engine.end_sequence(slot)
+            # (a capture runs the step once to find its lists; a replay asks for nothing)
+            assert forms == {"launched": chunks, "captured": 2 * chunks, "replayed": []}[turn], (length, turn)
+            for row, place in zip(rows, (0, length - 1)):
+                yard.check(row, ids, "float32", f"{length} tokens {turn} place {place}", rows=place)
+        assert len(engine._prefill_graphs.graphs) == 1
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_unequal_batches_equal_each_request_alone(folders, name, dtype):

@@ -75,3 +75,32 @@ def test_prefill_plan_by_class_and_size():
     # a group of 3 heads: items of three columns (no two-column plans), one wave an item from twice the chip's waves of them
     assert prefill_plan(8192, 8192, 24, 64, 8) == (1, 0) and prefill_plan(1216, 1216, 24, 64, 8) == (4, 0)
     assert prefill_plan(3072, 3072, 32, 64, 32) == (4, 0)
+
+
+@pytest.mark.parametrize("delta, least", [(True, {1: 128, 4: 512, 8: 1280, 16: 2560}), (False, {1: 64, 4: 128, 16: 768})])
+def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(delta, least):
+    """Chunks or a token at a time by the rows that a step plans for (64 and more, ``prompt_rows``): the same at the tokens that are
+    launched and at the rows that are replayed, and scratch for no more rows than are there."""
+    import types
+
+    from nnis_amd.engine.graph import prompt_rows
+    from nnis_amd.kernels import ops
+
+    def scratch(batch, tokens, planned, decode=False, heads=4):
+        ctx = types.SimpleNamespace(decode=decode, batch=batch, planned_rows=planned)
+        return ops.chunked_scratch(ctx, tokens, heads, 64, 128, delta, "meta")
+
+    for batch, first in least.items():
+        for total in [batch, batch + 1, 63, 65, 100, 103, 104, first - 128, first - 64, first - 63, first - 1, first, first + 1, 4 * first]:
+            if total < batch:
+                continue
+            rows = prompt_rows(total)
+            launched, replayed = scratch(batch, total, rows), scratch(batch, rows, rows)
+            assert (launched is not None) == (replayed is not None) == (rows >= first), (batch, total)
+            if launched is not None:
+                assert launched.numel() == ops.recurrent().nnis_chunked_scratch(total, batch, 4, 64, 128, int(delta)) <= replayed.numel()
+    # whether there is memory enough goes by the planned rows too
+    heads = ops.CHUNKED_MOST_BYTES // (4 * ops.recurrent().nnis_chunked_scratch(1280, 1, 1, 64, 128, int(delta)))
+    assert scratch(1, 1279, 1280, heads=heads) is not None and scratch(1, 1280, 1280, heads=heads) is not None
+    assert scratch(1, 1279, 1280, heads=heads + 1) is None and scratch(1, 1280, 1280, heads=heads + 1) is None
+    assert scratch(8, 8, 4096, decode=True) is None  # single tokens
