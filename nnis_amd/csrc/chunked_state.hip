@@ -270,7 +270,9 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
       const float* ba = a.ba + (size_t)(first + lane) * 2 * heads;
       const float z = ba[heads + head] + a.dt_bias[head];
       log_g = -a.rate[head] * (z > 20.0f ? z : log1pf(expf(z)));
-      log_g = log_g < -1e30f ? -1e30f : log_g;  // (a decay to zero: differences of infinite logarithms would be no numbers)
+      // (a decay to zero: differences of infinite logarithms would be no numbers, and the decays behind a very large one would
+      // drown in the sum; expf gives zero from -104 on)
+      log_g = log_g < -1000.0f ? -1000.0f : log_g;
       beta = 1.0f / (1.0f + expf(-ba[head]));
     }
     double total = (double)log_g;

@@ -1235,6 +1235,39 @@ def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, mon
     assert len(rooms) == 1 and (rooms[0][0][rooms[0][1]:] == 7).all()  # nothing was written beyond what the step asks for
 
 
+def _in_chunks(ops, monkeypatch):
+    """Every step's matrix recurrences in chunks, whatever its lengths."""
+    monkeypatch.setattr(ops, "chunked_scratch", lambda ctx, tokens, *sizes: torch.empty(
+        ops.recurrent().nnis_chunked_scratch(tokens, ctx.batch, *sizes[:4]), device=sizes[4]))
+
+
+def _prompts(lengths):
+    import types
+
+    starts = [0, *np.cumsum(lengths).tolist()]
+    return types.SimpleNamespace(
+        decode=False, batch=len(lengths), tokens=sum(lengths), max_new=max(lengths), planned_rows=sum(lengths), seq_slot=_i32(range(len(lengths))),
+        seq_start=_i32(starts), tok_slot=_i32([s for s, n in enumerate(lengths) for _ in range(n)]), tok_pos=_i32([i for n in lengths for i in range(n)]))
+
+
+@pytest.mark.parametrize("logit", [200.0, 1e16, 1e20, float("inf")])
+def test_decays_behind_a_decay_to_zero(logit, monkeypatch):
+    """A decay of a chunk that is zero, however far below what a float holds, leaves the decays behind it as they are."""
+    ops = _ops()
+    torch.manual_seed(3)
+    heads, d, e, lengths = 2, 32, 16, [64, 100]
+    rows, ba, rate, dt_bias = torch.randn(164, 2 * heads * d + heads * e), torch.randn(164, 2 * heads), 1 + torch.rand(heads), torch.randn(heads)
+    ba[[5, 6, 64 + 30, 64 + 70], heads:] = logit
+    state = torch.randn(2, heads, e, d)
+    want, after = _delta_in_64_bits(rows, ba, rate, dt_bias, d ** -0.5, state, [0, 64, 164], heads, heads, d, e)
+    _in_chunks(ops, monkeypatch)
+    held, out = state.cuda(), torch.empty(164, heads * e, device="cuda")
+    ops.gated_delta(rows.cuda(), ba.cuda(), rate.cuda(), dt_bias.cuda(), d ** -0.5, held, _prompts(lengths), heads, heads, d, e, out)
+    for got, exact in ((out.cpu(), want), (held.cpu(), after)):
+        error = (got.double() - exact).square().mean().sqrt() / exact.square().mean().sqrt()
+        assert error.item() <= 2.0 ** -24 * 64 ** 0.5  # sums over up to 64 tokens, rounded at each
+
+
 @pytest.mark.parametrize("m, k", [(70, 72), (300, 392), (530, 8), (257, 136)])
 @pytest.mark.parametrize("epilogue", ["store", "silu", "rope"])
 def test_the_tile_whose_weights_go_into_registers(epilogue, m, k):
