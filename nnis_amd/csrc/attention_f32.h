@@ -9,11 +9,12 @@
 //
 // Measured, microseconds, against a wave a (token, head) (attention_rows_kernel): 8 single tokens of 100 to 905 keys on 9/3
 // heads of 64 10.4 (31), 8 of 2,000 keys on 32/32 heads 42 (84; 48 at 5.5 TB/s if nothing came from a cache); a prompt of
-// 509 tokens on 32/4 heads of 64 27 (155), of 2,000 on 32/8 heads of 128 413 (4,990; 80 TFLOP/s counted causally).  Over a
-// prompt the products bound it (a tile of keys is 32 instructions of 32 cycles a column tile at 64 channels, beside 130
-// vector instructions); over single tokens the trips to memory.  Measured and no faster: 8 waves a block (28 and 204
-// against 26 and 200 at 509 and 2,000 tokens), three and four tiles in registers, a tile's scores taken ahead of the softmax
-// of the tile before it (31 and 255).
+// 509 tokens on 32/4 heads of 64 28 (155), of 2,000 on 32/8 heads of 128 450 (4,990; 73 TFLOP/s counted causally; 27 and 416
+// without the search for values that are no numbers).  Over a prompt the products bound it (a tile of keys is 32
+// instructions of 32 cycles a column tile at 64 channels, beside 130 vector instructions); over single tokens the trips to
+// memory.  Measured and no faster: 8 waves a block (28 and 204 against 26 and 200 at 509 and 2,000 tokens), three and four
+// tiles in registers, a tile's scores taken ahead of the softmax of the tile before it (31 and 255), such values added behind
+// the products from memory again (31 fewer registers; 28 and 453 where this takes 28 and 450).
 #pragma once
 
 typedef __attribute__((ext_vector_type(4))) float attn_f32x4;
@@ -37,8 +38,9 @@ struct F32Step {
 };
 constexpr int kF32Partial = HDV + 4;
 
+// (two waves a SIMD up to 64 channels: left to itself the compiler takes 260 registers)
 template <int C, bool SINGLE>
-__global__ __launch_bounds__(kWave * kF32Waves) void attention_f32_kernel(AttnArgs a, F32Step step) {
+__global__ __launch_bounds__(kWave * kF32Waves, kF32Ahead ? 2 : 1) void attention_f32_kernel(AttnArgs a, F32Step step) {
   constexpr int KC = HD / 16, VC = HDV / 16;
   constexpr int kOutRow = 64 + 4;  // floats of a column's 64 channels in LDS
   __shared__ float merged[kF32Waves][16][kOutRow];
@@ -167,6 +169,7 @@ __global__ __launch_bounds__(kWave * kF32Waves) void attention_f32_kernel(AttnAr
         for (int c = 0; c < VC; ++c) kv.v[c][e] = held ? kv.v[c][e] : 0.0f;
       }
     }
+    auto seen = [&](int t, int key) { return near ? key <= pos[t] && (key >= lo[t] || key < a.keep_first) : key < lo[t] / a.pool; };
     bool rises = false;
 #pragma unroll
     for (int t = 0; t < C; ++t) {
@@ -186,9 +189,7 @@ __global__ __launch_bounds__(kWave * kF32Waves) void attention_f32_kernel(AttnAr
       if (masked) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int key = key0 + 4 * g + e;
-          const bool seen = near ? key <= pos[t] && (key >= lo[t] || key < a.keep_first) : key < lo[t] / a.pool;
-          s[t][e] = seen ? s[t][e] : -INFINITY;
+          s[t][e] = seen(t, key0 + 4 * g + e) ? s[t][e] : -INFINITY;
         }
       }
       rises |= fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])) > ref[t] + kF32Rise;
@@ -212,6 +213,36 @@ __global__ __launch_bounds__(kWave * kF32Waves) void attention_f32_kernel(AttnAr
 #pragma unroll
       for (int e = 0; e < 4; ++e) s[t][e] = expf(s[t][e] - against);
       sum[t] += (s[t][0] + s[t][1]) + (s[t][2] + s[t][3]);
+    }
+    // A value that is infinite or no number, times the weight of a row that does not see its key, zero, would be no number: of a
+    // tile that some rows see a part of, such values are added to the rows that see them here, and count as zeros below.
+    if (masked) {
+      attn_f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < VC; ++c) none += kv.v[c] * 0.0f;
+      if (__builtin_expect(__any(!((none[0] + none[1]) + (none[2] + none[3]) == 0.0f)), 0)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll 1
+          for (int k4 = 0; k4 < 4; ++k4)  // the key 4 k4 + e: its weights lie in the lane group k4, as its values do
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+              const float weight = __shfl(s[t][e], k4 * 16 + r, kWave);
+              const bool counts = seen(t, key0 + 4 * k4 + e);
+#pragma unroll
+              for (int c = 0; c < VC; ++c) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  const float value = __shfl(kv.v[c][e], k4 * 16 + 4 * g + i, kWave);
+                  out[t][c][i] = counts && !(value * 0.0f == 0.0f) ? fmaf(weight, value, out[t][c][i]) : out[t][c][i];
+                }
+                __builtin_amdgcn_sched_barrier(0);  // (one channel tile after another: registers)
+              }
+            }
+#pragma unroll
+          for (int c = 0; c < VC; ++c) kv.v[c][e] = kv.v[c][e] * 0.0f == 0.0f ? kv.v[c][e] : 0.0f;
+        }
+      }
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e)

@@ -1149,6 +1149,45 @@ def test_attention_in_32_bits_on_the_matrix_cores(heads, kv_heads, head_dim, val
         both([0], [0], splits=ops.ATTENTION_F32_MOST_SPLITS + 1)
 
 
+@pytest.mark.parametrize("heads, kv_heads, head_dim, options", [
+    (4, 4, 64, {}), (6, 2, 64, dict(window=20)), (2, 1, 128, dict(window=-24)), (3, 3, 256, {}), (20, 1, 16, dict(window=7, keep_first=5)),
+    (4, 2, 32, dict(window=16, pool=8)), (8, 2, 80, {})])
+def test_32_bit_attention_keeps_rows_from_values_that_they_do_not_see(heads, kv_heads, head_dim, options):
+    """Values that are infinite or no numbers reach the rows that see their keys and no others, as in the row kernel, over a prompt and
+    for single tokens: the same outputs are numbers, and those are equal to rounding (the bound of the test above)."""
+    ops = _ops()
+    torch.manual_seed(heads + head_dim)
+    ends, window = [37, 50, 5], options.get("window", 0)
+    keys, values = ([torch.randn(n, kv_heads, head_dim) for n in ends] for _ in range(2))
+    values[0][20, 0, 3], values[0][22, -1, head_dim - 1], values[1][33, 0, 5], values[1][2, :, 1], values[2][4, 0, 0] = (
+        float("nan"), float("inf"), float("-inf"), float("nan"), float("inf"))
+    keys[1][40, 0, 2] = float("nan")
+    k_pages, v_pages, table = _paged(keys, values, torch.float32, kv_heads, head_dim)
+    pooled = None
+    if options.get("pool"):
+        entries = [torch.randn(8, kv_heads, head_dim) for _ in ends]
+        entries[0][1, 0, 1] = float("inf")  # (a block that the first of a tile's rows do not see yet)
+        pooled = ops.PooledBlocks(*_paged(entries, entries, torch.float32, kv_heads, head_dim), options["pool"])
+    extras = ops.ScoreExtras(options.get("keep_first", 0), None, None)
+    common = (heads, kv_heads, head_dim, head_dim ** -0.5, window, head_dim, 0.0, extras, pooled)
+
+    def both(slots, positions, tiles=None, splits=1):
+        q = torch.randn(len(slots), heads * head_dim).cuda()
+        want, got = torch.empty_like(q), torch.empty_like(q)
+        ops.attention_rows(q, want, k_pages, v_pages, table, _i32(slots), _i32(positions), *common)
+        ops.attention_f32(q, got, k_pages, v_pages, table, _i32(slots), _i32(positions), *common, None, tiles, splits)
+        numbers = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), numbers) and numbers.any() and not numbers.all()
+        assert (got - want)[numbers].abs().max().item() <= 4 * 2.0 ** -21 * max(head_dim, 32) ** 0.5
+
+    rows = ops.attention_module(head_dim, head_dim, 0.0, extras, pooled, None).nnis_attention_f32_tile_rows(heads, kv_heads)
+    everywhere = [s for s, n in enumerate(ends) for _ in range(n)], [i for n in ends for i in range(n)]
+    items = torch.from_numpy(ops.prefill_tile_list(ends, [0, 0, 0], None, rows)).cuda()
+    both(*everywhere, (items, _i32([0, 1, 2]), _i32([0, *np.cumsum(ends).tolist()]), _i32([0, 0, 0])))
+    for splits in (1, 2):
+        both(*everywhere, splits=splits)
+
+
 def _delta_in_64_bits(rows, ba, rate, dt_bias, q_scale, state, starts, heads, groups, d, e):
     rows, ba, S = rows.double(), ba.double(), state.double().transpose(-1, -2).clone()
     unit = lambda x: x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)  # noqa: E731
