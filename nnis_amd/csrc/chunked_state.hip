@@ -46,6 +46,30 @@ __device__ __forceinline__ f32x4 multiply16(f32x4 a, f32x4 b, f32x4 sum) {
 
 __device__ __forceinline__ f32x4 sum8(const f32x4 (&p)[8]) { return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])); }
 
+// Products with a tile on the diagonal, whose first operand is zero above it: a token that is infinite or no number must not
+// reach the tokens before it (zero times it would be no number), so a tile that holds one is added up element by element.
+// `a` as a first operand, `b` and the sum as results; STRICT: below the diagonal only.
+template <bool STRICT>
+__device__ __forceinline__ f32x4 multiply_below(f32x4 a, f32x4 b, int lane) {
+  const f32x4 none = b * 0.0f;
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (__builtin_expect(!__any(!((none[0] + none[1]) + (none[2] + none[3]) == 0.0f)), 1)) return multiply16(a, b, sum);
+  const int r = lane % 16, g = lane / 16;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll 1
+    for (int from = 0; from < 4; ++from) {  // column 4 from + e of a, row 4 from + e of b
+      const float right = __shfl(b[e], from * 16 + r, kWave);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 4 * g + i, column = 4 * from + e;
+        const float left = __shfl(a[e], from * 16 + row, kWave);
+        sum[i] = column < row || (!STRICT && column == row) ? fmaf(left, right, sum[i]) : sum[i];
+      }
+    }
+  return sum;
+}
+
 __device__ __forceinline__ f32x4 load4(const float* p) { return *(const f32x4*)p; }
 __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
   const bf16x4 v = *(const bf16x4*)p;
@@ -141,7 +165,7 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        // (values of tokens beyond the end meet zeros in K~, and rows of M that nobody stores)
+        // (tokens beyond the end: a value that is there, zeroed where it is used)
         const int token = min(begin + chunk * kChunk + tile * 16 + g * 4 + i, end - 1);
         o.v[i] = to_f32(((const V*)a.v)[(size_t)token * a.v_stride + (size_t)head * e + column]);
       }
@@ -161,7 +185,13 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
         for (int i = 0; i < 4; ++i) part[t % 2 * 4 + i] = mfma(o.rows[t][i], S[t][i], part[t % 2 * 4 + i]);
       sum = sum8(part);
     }
-    if constexpr (!OUTPUTS) u_shared[tile][lane] = o.v + sum;
+    if constexpr (!OUTPUTS && DELTA) u_shared[tile][lane] = o.v + sum;
+    if constexpr (!OUTPUTS && !DELTA) {
+      f32x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = begin + chunk * kChunk + tile * 16 + g * 4 + i < end ? o.v[i] : 0.0f;
+      u_shared[tile][lane] = v;
+    }
     __syncthreads();
     f32x4 U[kTiles];
 #pragma unroll
@@ -175,7 +205,10 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
       f32x4 within = zero;
 #pragma unroll
       for (int s = 0; s < kTiles; ++s)
-        if (s <= tile) within += multiply16(o.m[s], U[s], zero);
+        if (s < tile) within += multiply16(o.m[s], U[s], zero);
+#pragma unroll
+      for (int s = 0; s < kTiles; ++s)
+        if (s == tile) within += multiply_below<false>(o.m[s], U[s], lane);
       const f32x4 out = sum * o.v + within;
       const int token = begin + chunk * kChunk + tile * 16 + g * 4;
       float* to = a.out + ((size_t)token * a.heads + head) * e + column;
@@ -319,9 +352,10 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
       for (int i = 0; i < 4; ++i) {
         const int token = row_tile * 16 + g * 4 + i;
         const bool live = token < count && column < count;
-        const float ratio = live && column <= token ? expf((float)(logs[token] - logs[column])) : 0.0f;
-        A[token][column] = column < token ? -betas[token] * ratio * kk[i] : 0.0f;
-        a.c.within[((at * kTiles + row_tile) * kTiles + s) * kTileFloats + operand_at(g * 4 + i, r)] = ratio * qk[i];
+        const bool met = live && column <= token;
+        const float ratio = met ? expf((float)(logs[token] - logs[column])) : 0.0f;
+        A[token][column] = met && column < token ? -betas[token] * ratio * kk[i] : 0.0f;
+        a.c.within[((at * kTiles + row_tile) * kTiles + s) * kTileFloats + operand_at(g * 4 + i, r)] = met ? ratio * qk[i] : 0.0f;
       }
     }
   }
@@ -366,9 +400,10 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
     for (int i = 0; i < kTiles; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int token = i * 16 + g * 4 + j;  // (beyond the end the factors are zero)
-        right[i][j] = is_key ? unit_row(token, 1)[column]
-                             : load_as_f32(a.rows, a.dtype, (size_t)(first + min(token, count - 1)) * a.stride + a.v_at + (size_t)head * e + column);
+        const int token = i * 16 + g * 4 + j;  // (beyond the end: zeros)
+        const float v = is_key ? unit_row(token, 1)[column]
+                               : load_as_f32(a.rows, a.dtype, (size_t)(first + min(token, count - 1)) * a.stride + a.v_at + (size_t)head * e + column);
+        right[i][j] = token < count ? v : 0.0f;
       }
 #pragma unroll
     for (int i = 0; i < kTiles; ++i) {
@@ -377,7 +412,7 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
 #pragma unroll
       for (int j = 0; j < i; ++j) above += multiply16(a_rows[i][j], x[j], zero);
       above += right[i] * (is_key ? key_factor[i] : value_factor[i]);
-      x[i] = above + multiply16(t_rows[i], above, zero);
+      x[i] = above + multiply_below<true>(t_rows[i], above, lane);
       if (is_key) {
         float* to = a.c.keys + ((at * kTiles + i) * KT + tile) * kTileFloats;
 #pragma unroll

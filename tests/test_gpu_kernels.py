@@ -1289,6 +1289,47 @@ def _prompts(lengths):
         seq_start=_i32(starts), tok_slot=_i32([s for s, n in enumerate(lengths) for _ in range(n)]), tok_pos=_i32([i for n in lengths for i in range(n)]))
 
 
+@pytest.mark.parametrize("delta", [True, False])
+def test_states_in_chunks_keep_tokens_from_those_behind_them(delta, monkeypatch):
+    """Queries, keys, values and decays that are infinite or no numbers show in the outputs that they show in a token at a time, those
+    from their token on, and in the same states; the others are equal to rounding."""
+    ops = _ops()
+    torch.manual_seed(5)
+    heads, d, e, lengths = 3, 32, 48, [64, 100, 21, 130]
+    tokens = sum(lengths)
+    wide, ba = torch.randn(tokens, heads * (2 * d + e)), torch.randn(tokens, 2 * heads)
+    q, k, v = wide[:, :heads * d], wide[:, heads * d:2 * heads * d], wide[:, 2 * heads * d:]
+    nan, inf = float("nan"), float("inf")
+    v[9, 3], v[60, e + 7], v[64 + 70, 2 * e + 1] = nan, inf, nan
+    q[64 + 40, 5], k[64 + 90, d + 2] = nan, nan
+    v[64 + 100 + 20, 2] = -inf  # (a sequence's last)
+    if delta:
+        ba[64 + 100 + 21 + 85, 0], ba[64 + 100 + 21 + 95, heads + 1] = nan, nan
+    else:
+        k[64 + 100 + 21 + 85, 3], v[64 + 100 + 21 + 95, e] = inf, inf
+    rate, dt_bias, decay = 0.2 + torch.rand(heads).cuda(), torch.randn(heads).cuda(), torch.tensor([0.9, 0.99, 0.5])
+    results = []
+    for chunks in (True, False):
+        if chunks:
+            _in_chunks(ops, monkeypatch)
+        else:
+            monkeypatch.setattr(ops, "chunked_scratch", lambda *sizes: None)
+        torch.manual_seed(6)
+        held, out = torch.randn(4, heads, *((e, d) if delta else (d, e))).cuda(), torch.empty(tokens, heads * e, device="cuda")
+        rows = wide.cuda()
+        if delta:
+            ops.gated_delta(rows, ba.cuda(), rate, dt_bias, d ** -0.5, held, _prompts(lengths), heads, heads, d, e, out)
+        else:
+            ops.gla_scan(*rows.split([heads * d, heads * d, heads * e], dim=1), None, d ** -0.5, held, _prompts(lengths), heads, out,
+                         head_decay=torch.stack([decay, torch.log(decay)]).cuda())
+        results.append((out, held))
+    for got, want in zip(*results):
+        numbers = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), numbers) and numbers.any() and not numbers.all()
+        error = (got - want)[numbers].double().square().mean().sqrt() / want[numbers].double().square().mean().sqrt()
+        assert error.item() <= 2 * 2.0 ** -24 * 64 ** 0.5  # both sides sum over up to 64 tokens or channels, rounded at each
+
+
 @pytest.mark.parametrize("logit", [200.0, 1e16, 1e20, float("inf")])
 def test_decays_behind_a_decay_to_zero(logit, monkeypatch):
     """A decay of a chunk that is zero, however far below what a float holds, leaves the decays behind it as they are."""
