@@ -19,11 +19,14 @@
 //
 // Why: the recurrence a token at a time is a chain of 0.39 us a token and sequence for the delta rule, whatever the chip
 // has free; a chunk of 64 is one of 4 us, beside 30 us for the first kernel and the ends.  Microseconds, a prompt of 300 /
-// 1,500 tokens: the delta rule on 16 heads of 128 x 128 55 / 131 (130 / 602 a token at a time), retention on 8 heads of
-// 128 x 256 27 / 74 (78 / 187, in pieces); 8 prompts of 2,048: 990 (1,500) and 430 (1,480).  What bounds the walk is the
+// 1,500 tokens: the delta rule on 16 heads of 128 x 128 57 / 135 (130 / 602 a token at a time), retention on 8 heads of
+// 128 x 256 25 / 74 (78 / 187, in pieces); 8 prompts of 2,048: 1,020 (1,500) and 421 (1,480).  What bounds the walk is the
 // chain of a chunk: two products that wait for each other over U, two barriers, and a state that goes round through LDS.
-// Error against 64 bits, root mean square over the result's: delta rule 1.5e-7 (1.8e-7 a token at a time; equal within 2%
-// where a state is forgotten within a few tokens), retention 2.0e-7 (5.1e-7).
+// Error of the outputs against 64 bits, 1e-7 of their root mean square, and of a token at a time: delta rule, 16 heads of 128 x
+// 128, decays of which most are forgotten within a few tokens 1.17 (1.17), slow ones 1.63 (2.52), between 1.38 (1.36); 4 heads of 16
+// x 48 between 1.31 (1.25); retention 1.95 (5.11) over 1,500 tokens, 1.11 (1.15) over 20.  The states' are within 1% of a token
+// at a time's, 1% above at fast decays, and half as large at slow ones.  (With a token's own M_tt u_t among the products, a twentieth
+// of the time less, fast decays 1.20, between 1.41, 20 tokens of retention 1.20.)
 #include "common.h"
 
 namespace {
@@ -33,7 +36,7 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 
 constexpr int kChunk = 64;       // tokens of a chunk: four tiles of 16, one a wave
 constexpr int kTiles = kChunk / 16;
-constexpr int kGates = kChunk + 16;  // floats a (chunk, head) has for c_t, and for c_64 behind them
+constexpr int kGates = 2 * kChunk + 16;  // floats a (chunk, head) has for c_t, M_tt and c_64
 
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -48,12 +51,15 @@ __device__ __forceinline__ f32x4 sum8(const f32x4 (&p)[8]) { return ((p[0] + p[1
 
 // Products with a tile on the diagonal, whose first operand is zero above it: a token that is infinite or no number must not
 // reach the tokens before it (zero times it would be no number), so a tile that holds one is added up element by element.
-// `a` as a first operand, `b` and the sum as results; STRICT: below the diagonal only.
-template <bool STRICT>
+// `a` as a first operand, `b` and the sum as results; what `a` holds on and above its diagonal is zero.
 __device__ __forceinline__ f32x4 multiply_below(f32x4 a, f32x4 b, int lane) {
   const f32x4 none = b * 0.0f;
   f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (__builtin_expect(!__any(!((none[0] + none[1]) + (none[2] + none[3]) == 0.0f)), 1)) return multiply16(a, b, sum);
+  if (__builtin_expect(!__any(!((none[0] + none[1]) + (none[2] + none[3]) == 0.0f)), 1)) {
+    // (four chains: a row's nearest tokens, the largest terms, come last in one of them and not in the middle of a long one)
+    const f32x4 p0 = mfma(a[0], b[0], sum), p1 = mfma(a[1], b[1], sum), p2 = mfma(a[2], b[2], sum), p3 = mfma(a[3], b[3], sum);
+    return (p0 + p1) + (p2 + p3);
+  }
   const int r = lane % 16, g = lane / 16;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
@@ -64,7 +70,7 @@ __device__ __forceinline__ f32x4 multiply_below(f32x4 a, f32x4 b, int lane) {
       for (int i = 0; i < 4; ++i) {
         const int row = 4 * g + i, column = 4 * from + e;
         const float left = __shfl(a[e], from * 16 + row, kWave);
-        sum[i] = column < row || (!STRICT && column == row) ? fmaf(left, right, sum[i]) : sum[i];
+        sum[i] = column < row ? fmaf(left, right, sum[i]) : sum[i];
       }
     }
   return sum;
@@ -84,9 +90,9 @@ struct ChunkArgs {
   // second kernel's waves load them: tiles of 16 x 16 as first operands, `operand_at`, 1 KB of consecutive memory a load.
   // (In rows, the step's stride of 4 and 8 KB between tokens put a load's 16 rows on one channel of the L2: 3.2 and 5 us a
   // chunk for retention and the delta rule.)
-  float* within;   // [4 tiles of rows][4 of columns]: M
+  float* within;   // [4 tiles of rows][4 of columns]: M below its diagonal
   float* keys_t;   // [key_dim / 16][4 tiles of tokens]: K~
-  float* gates;    // [kGates]: c_t, then c_64
+  float* gates;    // [kGates]: c_t, then M_tt, then c_64
   float* queries;  // [4 tiles of tokens][key_dim / 16]
   float* keys;     // [4][key_dim / 16]: -K'  (delta rule)
   float* values;   // [value_dim / 16][4]: V' (delta rule), tiles as results
@@ -141,7 +147,7 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
   }
 
   struct Operands {
-    f32x4 rows[kRows ? KT : 1], kt[kTiles], m[OUTPUTS ? kTiles : 1], v;  // v: the values, or c_t of the outputs' rows
+    f32x4 rows[kRows ? KT : 1], kt[kTiles], m[OUTPUTS ? kTiles : 1], own, v;  // v: the values, or c_t of the outputs' rows; own: their M_tt
     float c_end;
   };
   // (no load behind a branch: it would be waited for at once)
@@ -158,8 +164,9 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
     if constexpr (OUTPUTS) {
       const float* m = a.within + ((at * kTiles + tile) * kTiles * kWave + lane) * 4;
 #pragma unroll
-      for (int s = 0; s < kTiles; ++s) o.m[s] = load4(m + min(s, tile) * kTileFloats);
+      for (int s = 0; s < kTiles; ++s) o.m[s] = load4(m + (s == kTiles - 1 ? tile : min(s, tile)) * kTileFloats);  // (the last: on the diagonal)
       o.v = load4(a.gates + at * kGates + tile * 16 + g * 4);
+      o.own = load4(a.gates + at * kGates + kChunk + tile * 16 + g * 4);
     } else if constexpr (DELTA) {
       o.v = load4(a.values + (((at * (e / 16) + column / 16) * kTiles + tile) * kWave + lane) * 4);
     } else {
@@ -170,7 +177,7 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
         o.v[i] = to_f32(((const V*)a.v)[(size_t)token * a.v_stride + (size_t)head * e + column]);
       }
     }
-    o.c_end = *(const __attribute__((address_space(4))) float*)(uintptr_t)(a.gates + at * kGates + kChunk);  // (a scalar load)
+    o.c_end = *(const __attribute__((address_space(4))) float*)(uintptr_t)(a.gates + at * kGates + 2 * kChunk);  // (a scalar load)
   };
   auto step = [&](const Operands& o, int chunk) {
     f32x4 sum = zero;
@@ -196,20 +203,20 @@ __device__ __forceinline__ void walk_chunks(const ChunkArgs& a, int head, int co
     f32x4 U[kTiles];
 #pragma unroll
     for (int s = 0; s < kTiles; ++s) U[s] = u_shared[s][lane];
+    const f32x4 u = u_shared[tile][lane];  // (of the outputs' own tokens)
     f32x4 part[kTiles];
 #pragma unroll
     for (int s = 0; s < kTiles; ++s) part[s] = multiply16(o.kt[s], U[s], zero);
     mine = mine * o.c_end + ((part[0] + part[1]) + (part[2] + part[3]));
     if (wave < KT) s_shared[wave][lane] = mine;
     if constexpr (OUTPUTS) {
+      // a token's own update comes last and once: where states are forgotten within a few tokens it is most of the output
       f32x4 within = zero;
 #pragma unroll
-      for (int s = 0; s < kTiles; ++s)
+      for (int s = 0; s < kTiles - 1; ++s)
         if (s < tile) within += multiply16(o.m[s], U[s], zero);
-#pragma unroll
-      for (int s = 0; s < kTiles; ++s)
-        if (s == tile) within += multiply_below<false>(o.m[s], U[s], lane);
-      const f32x4 out = sum * o.v + within;
+      within += multiply_below(o.m[kTiles - 1], u, lane);
+      const f32x4 out = o.own * u + (sum * o.v + within);
       const int token = begin + chunk * kChunk + tile * 16 + g * 4;
       float* to = a.out + ((size_t)token * a.heads + head) * e + column;
 #pragma unroll
@@ -262,6 +269,7 @@ __global__ __launch_bounds__(kWave * kScanWaves) void chunk_scan_kernel(ChunkArg
 struct DeltaChunkArgs {
   ChunkArgs c;
   const float* unit;  // [tokens, groups, 2, key_dim]: q (scaled) then k, unit vectors
+  const float* dots;  // [tokens, groups]: q . k
   const void* rows;   // v of token t, head h at rows + t * stride + v_at + h * value_dim
   int dtype, stride, v_at, groups;
   const float* ba;  // [tokens, 2 * heads]
@@ -317,7 +325,9 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
     logs[lane] = total;
     betas[lane] = beta;
     a.c.gates[at * kGates + lane] = expf((float)total);
-    if (lane == kChunk - 1) a.c.gates[at * kGates + kChunk] = expf((float)total);
+    // (the one that a token at a time takes: summed with less rounding than M's products)
+    a.c.gates[at * kGates + kChunk + lane] = lane < count ? a.dots[(size_t)(first + lane) * a.groups + qk_head] : 0.0f;
+    if (lane == kChunk - 1) a.c.gates[at * kGates + 2 * kChunk] = expf((float)total);
   }
   __syncthreads();
 
@@ -352,9 +362,9 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
       for (int i = 0; i < 4; ++i) {
         const int token = row_tile * 16 + g * 4 + i;
         const bool live = token < count && column < count;
-        const bool met = live && column <= token;
+        const bool met = live && column < token;
         const float ratio = met ? expf((float)(logs[token] - logs[column])) : 0.0f;
-        A[token][column] = met && column < token ? -betas[token] * ratio * kk[i] : 0.0f;
+        A[token][column] = met ? -betas[token] * ratio * kk[i] : 0.0f;
         a.c.within[((at * kTiles + row_tile) * kTiles + s) * kTileFloats + operand_at(g * 4 + i, r)] = met ? ratio * qk[i] : 0.0f;
       }
     }
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(kWave * kPrepareWaves) void chunk_delta_prepare_ker
 #pragma unroll
       for (int j = 0; j < i; ++j) above += multiply16(a_rows[i][j], x[j], zero);
       above += right[i] * (is_key ? key_factor[i] : value_factor[i]);
-      x[i] = above + multiply_below<true>(t_rows[i], above, lane);
+      x[i] = above + multiply_below(t_rows[i], above, lane);
       if (is_key) {
         float* to = a.c.keys + ((at * kTiles + i) * KT + tile) * kTileFloats;
 #pragma unroll
@@ -492,7 +502,7 @@ __global__ __launch_bounds__(256) void chunk_retention_prepare_kernel(RetentionC
   }
   if (wave == 0) {
     a.c.gates[at * kGates + lane] = expf((float)(lane + 1) * log_a);
-    if (lane == 0) a.c.gates[at * kGates + kChunk] = expf((float)count * log_a);
+    if (lane == 0) a.c.gates[at * kGates + 2 * kChunk] = expf((float)count * log_a);
   }
   __syncthreads();
   {
@@ -504,22 +514,25 @@ __global__ __launch_bounds__(256) void chunk_retention_prepare_kernel(RetentionC
     for (int s = 0; s < kTiles; ++s) {
       if (s > wave) break;
       const float* k_row = ks + (s * 16 + r) * kRow + g * 4;
-      f32x4 part[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) part[i] = zero;
+      f32x4 qk = zero, part[8];
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
+        if (t % 4 == 0) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) part[i] = zero;
+        }
         const f32x4 right = load4(k_row + t * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) part[t % 2 * 4 + i] = mfma(q[t][i], right[i], part[t % 2 * 4 + i]);
+        if (t % 4 == 3 || t == KT - 1) qk += sum8(part);
       }
-      const f32x4 qk = sum8(part);
       const int column = s * 16 + r;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int token = wave * 16 + g * 4 + i;
         a.c.within[((at * kTiles + wave) * kTiles + s) * kTileFloats + operand_at(g * 4 + i, r)] =
-            column <= token ? expf((float)(token - column) * log_a) * qk[i] : 0.0f;
+            column < token ? expf((float)(token - column) * log_a) * qk[i] : 0.0f;
+        if (column == token) a.c.gates[at * kGates + kChunk + token] = qk[i];
       }
     }
   }
@@ -571,7 +584,7 @@ extern "C" long long nnis_chunked_scratch(int tokens, int batch, int heads, int 
   }
 
 // The gated delta rule over a step's prompts, behind delta_prepare_kernel (nnis_gated_delta has the operands).
-int nnis_gated_delta_chunks(const float* unit, const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
+int nnis_gated_delta_chunks(const float* unit, const float* dots, const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
                             float* state, const int* seq_slot, const int* seq_start, int batch, int tokens, int heads, int groups, int key_dim,
                             int value_dim, float* out, float* scratch, hipStream_t s) {
   NNIS_REQUIRE(nnis_chunked_takes(key_dim, value_dim), "gated_delta: heads of %d and %d channels are not taken in chunks", key_dim, value_dim);
@@ -582,7 +595,7 @@ int nnis_gated_delta_chunks(const float* unit, const void* rows, int dtype, int 
   lay_out(c, scratch, chunks, true);
   c.v = nullptr; c.v_stride = 0;
   c.state = state; c.state_row = 1; c.state_column = key_dim; c.out = out;
-  a.unit = unit; a.rows = rows; a.dtype = dtype; a.stride = stride; a.v_at = 2 * groups * key_dim; a.groups = groups;
+  a.unit = unit; a.dots = dots; a.rows = rows; a.dtype = dtype; a.stride = stride; a.v_at = 2 * groups * key_dim; a.groups = groups;
   a.ba = ba; a.rate = rate; a.dt_bias = dt_bias;
   const size_t lds = 2 * kChunk * (size_t)(key_dim + 4) * sizeof(float);
 #define NNIS_RUN(KT)                                                                                                                       \

@@ -1249,7 +1249,7 @@ __global__ __launch_bounds__(256) void gated_delta_kernel(DeltaArgs a) {
 }  // namespace
 
 // over a step's prompts, in chunks of tokens (chunked_state.hip)
-int nnis_gated_delta_chunks(const float* unit, const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
+int nnis_gated_delta_chunks(const float* unit, const float* dots, const void* rows, int dtype, int stride, const float* ba, const float* rate, const float* dt_bias,
                             float* state, const int* seq_slot, const int* seq_start, int batch, int tokens, int heads, int groups, int key_dim,
                             int value_dim, float* out, float* scratch, hipStream_t s);
 
@@ -1283,7 +1283,7 @@ extern "C" int nnis_gated_delta(const void* rows, int dtype, int stride, const f
   const int items = tokens * groups;
   hipLaunchKernelGGL(delta_prepare_kernel, dim3((items + 3) / 4), dim3(256), 0, s, a);
   if (chunk_scratch)
-    return nnis_gated_delta_chunks(a.unit, rows, dtype, stride, ba, rate, dt_bias, state, seq_slot, seq_start, batch, tokens, heads, groups,
+    return nnis_gated_delta_chunks(a.unit, a.gates + 2 * (size_t)tokens * heads, rows, dtype, stride, ba, rate, dt_bias, state, seq_slot, seq_start, batch, tokens, heads, groups,
                                    key_dim, value_dim, out, chunk_scratch, s);
   const int need = (key_dim + 7) / 8;  // a thread keeps 8 key rows
   const int lane_groups = need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : (need <= 8 ? 8 : (need <= 16 ? 16 : 32))));

@@ -1900,7 +1900,7 @@ def run_pieces(ctx, state_bytes: int):
     return (piece, pieces) if pieces > 1 else (0, 1)
 
 
-# The most scratch that a step's chunks take (a chunk and head of 128 x 128 147 KB with the delta rule, of 128 x 256 82 KB with
+# The most scratch that a step's chunks take (a chunk and head of 128 x 128 148 KB with the delta rule, of 128 x 256 82 KB with
 # retention); steps beyond, of 29,000 and 52,000 tokens on 64 such heads, go a token at a time.
 CHUNKED_MOST_BYTES = 4 << 30
 

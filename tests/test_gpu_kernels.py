@@ -1289,6 +1289,40 @@ def _prompts(lengths):
         seq_start=_i32(starts), tok_slot=_i32([s for s, n in enumerate(lengths) for _ in range(n)]), tok_pos=_i32([i for n in lengths for i in range(n)]))
 
 
+@pytest.mark.parametrize("rule", ["delta", "retention"])
+def test_chunks_round_no_more_than_a_token_at_a_time(rule, monkeypatch):
+    """Where states are forgotten within a few tokens, and over a prompt of a few, most of an output is its token's own update, which
+    a chunk rounds as often as a token at a time does: the errors against 64 bits are equal (to 1%: both are averages over 2,000
+    and more outputs of a few equal roundings and some that differ)."""
+    ops = _ops()
+    torch.manual_seed(11)
+    heads, groups, d, e, tokens = (8, 4, 64, 128, 300) if rule == "delta" else (8, 8, 128, 256, 20)
+    wide = torch.randn(tokens, 2 * groups * d + heads * e).bfloat16()
+    if rule == "delta":
+        ba, rate, dt_bias = 0.9 * torch.randn(tokens, 2 * heads), torch.arange(1.0, heads + 1), 2 + torch.randn(heads)
+        state = 0.3 * torch.randn(1, heads, e, d)
+        want = _delta_in_64_bits(wide, ba, rate, dt_bias, d ** -0.5, state, [0, tokens], heads, groups, d, e)[0]
+    else:
+        decay, state = torch.tensor([1 - 2.0 ** (-5 - h) for h in range(heads)]), 0.3 * torch.randn(1, heads, d, e)
+        q, k, v = wide.split([heads * d, heads * d, heads * e], dim=1)
+        still = (torch.ones(tokens, 0), torch.zeros(tokens, 0), 0)
+        want = _retention_in_64_bits(q, k, v, decay, d ** -0.5, state, [0, tokens], list(range(tokens)), still, heads, d, e)[0]
+    errors = []
+    for chunks in (True, False):
+        if chunks:
+            _in_chunks(ops, monkeypatch)
+        else:
+            monkeypatch.setattr(ops, "chunked_scratch", lambda *sizes: None)
+        held, out, rows = state.cuda(), torch.empty(tokens, heads * e, device="cuda"), wide.cuda()
+        if rule == "delta":
+            ops.gated_delta(rows, ba.cuda(), rate.cuda(), dt_bias.cuda(), d ** -0.5, held, _prompts([tokens]), heads, groups, d, e, out)
+        else:
+            ops.gla_scan(*rows.split([heads * d, heads * d, heads * e], dim=1), None, d ** -0.5, held, _prompts([tokens]), heads, out,
+                         head_decay=torch.stack([decay, torch.log(decay)]).cuda())
+        errors.append((out.cpu().double() - want).square().mean().sqrt().item())
+    assert errors[0] <= 1.01 * errors[1]
+
+
 @pytest.mark.parametrize("delta", [True, False])
 def test_states_in_chunks_keep_tokens_from_those_behind_them(delta, monkeypatch):
     """Queries, keys, values and decays that are infinite or no numbers show in the outputs that they show in a token at a time, those
