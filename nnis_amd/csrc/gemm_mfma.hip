@@ -1336,8 +1336,10 @@ extern "C" int nnis_gemm_bf16(const void* x, const void* w, void* y, int y_dtype
 }
 
 // The tile that the tiled kernel takes for m rows, `columns` weight rows and a depth of k (2: 64 x 128, 3: 64 x 64,
-// 4: 256 x 256, 5: 256 x 192, 6: 128 x 128, 7: 256 x 128, 8: 128 x 192): for tests and tuning.
+// 4: 256 x 256, 5: 256 x 192, 6: 128 x 128, 7: 256 x 128, 8: 128 x 192): for tests and tuning.  The second: of a product into the
+// residual stream.
 extern "C" int nnis_gemm_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0); }
+extern "C" int nnis_gemm_residual_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0, true); }
 
 // 1 if nnis_gemm_residual gives these sizes to two blocks a strip (with a workspace of `workspace_bytes` and counts
 // behind it), 0 if to another kernel: for callers and tests that have to know which kernel ran.

@@ -59,6 +59,7 @@ _CORE_SIGNATURES = {
                         _VOID, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
     "nnis_gemm_residual_parts": [_INT, _INT],
     "nnis_gemm_tile": [_INT, _INT, _INT],
+    "nnis_gemm_residual_tile": [_INT, _INT, _INT],
     "nnis_gemm_takes_pair": [_INT, _INT, _INT, _SIZE],
     "nnis_gemm_residual": [_VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _VOID, _SIZE, _VOID, _VOID],
     "nnis_gemm_residual_tanh": [_VOID, _VOID, _VOID, _VOID, _VOID, _FLT, _VOID, _VOID, _FLT, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT,
@@ -1122,9 +1123,11 @@ def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, r
 TILE_64x128, TILE_64x64, TILE_256x256, TILE_256x192, TILE_128x128, TILE_256x128, TILE_128x192 = 2, 3, 4, 5, 6, 7, 8
 
 
-def gemm_tile(m: int, n: int, k: int) -> int:
-    """The tile (``TILE_*``) that the tiled kernel takes for a product of m rows with n weight rows of k."""
-    return core().nnis_gemm_tile(int(m), int(n), int(k))
+def gemm_tile(m: int, n: int, k: int, residual: bool = False) -> int:
+    """The tile (``TILE_*``) that the tiled kernel takes for a product of m rows with n weight rows of k; ``residual``: for
+    one into the residual stream, which goes by rates of its own."""
+    lib = core()
+    return (lib.nnis_gemm_residual_tile if residual else lib.nnis_gemm_tile)(int(m), int(n), int(k))
 
 
 def gemm_residual_parts(m: int, n: int) -> int:

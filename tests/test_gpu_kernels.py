@@ -1090,6 +1090,17 @@ def test_the_tiles_that_products_are_given():
         assert ops.gemm_tile(m, n, k) == tile, (m, n, k, ops.gemm_tile(m, n, k))
 
 
+def test_the_tile_of_a_product_into_the_stream_by_the_parts_it_leaves():
+    ops = _ops()
+    for m, n, k, width in ((4096, 4096, 14336, 128), (2048, 8192, 2048, 256)):  # (another tile than a product that is stored takes, and the same)
+        assert {ops.TILE_256x128: 128, ops.TILE_256x256: 256}[ops.gemm_tile(m, n, k, residual=True)] == width
+        x, w = torch.zeros(m, k, dtype=torch.bfloat16, device="cuda"), ops.pack_weight(torch.zeros(n, k, dtype=torch.bfloat16, device="cuda"))
+        resid, scaled = torch.ones(m, n, device="cuda"), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        ss = torch.empty(ops.gemm_residual_parts(m, n), m, device="cuda")
+        parts = ops.gemm_residual(x, w, resid, torch.ones(n, dtype=torch.bfloat16, device="cuda"), scaled, ss)
+        assert parts == 2 * (n // width) and (ss[:parts].sum(0) == n).all()
+
+
 F32_ATTENTION = [
     # heads, key/value heads, key channels, value channels, options
     (9, 3, 64, 64, {}), (4, 4, 16, 16, {}), (32, 1, 64, 64, {}), (40, 2, 16, 16, {}), (5, 5, 80, 80, {}), (8, 2, 128, 128, {}), (3, 3, 256, 256, {}),

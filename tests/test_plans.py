@@ -104,3 +104,21 @@ def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(d
     assert scratch(1, 1279, 1280, heads=heads) is not None and scratch(1, 1280, 1280, heads=heads) is not None
     assert scratch(1, 1279, 1280, heads=heads + 1) is None and scratch(1, 1280, 1280, heads=heads + 1) is None
     assert scratch(8, 8, 4096, decode=True) is None  # single tokens
+
+
+def test_the_tiles_of_products_into_the_stream():
+    """A product into the residual stream goes by rates of its own (the parts of its rows' sums of squares follow the tile)."""
+    from nnis_amd.kernels import ops
+
+    width = {ops.TILE_64x128: 128, ops.TILE_64x64: 64, ops.TILE_256x256: 256, ops.TILE_256x192: 192, ops.TILE_128x128: 128, ops.TILE_256x128: 128,
+             ops.TILE_128x192: 192}
+    for (m, n, k), (tile, stream) in {
+        (2048, 8192, 2048): (ops.TILE_256x256, ops.TILE_256x256),
+        (2048, 2048, 8192): (ops.TILE_128x128, ops.TILE_128x128),
+        (8192, 8192, 8192): (ops.TILE_256x256, ops.TILE_256x128),
+        (4096, 4096, 14336): (ops.TILE_256x256, ops.TILE_256x128),
+        (12288, 2048, 5632): (ops.TILE_256x128, ops.TILE_256x128),
+        (2048, 576, 1536): (ops.TILE_64x64, ops.TILE_64x64),
+    }.items():
+        assert (ops.gemm_tile(m, n, k), ops.gemm_tile(m, n, k, residual=True)) == (tile, stream), (m, n, k)
+        assert ops.core().nnis_gemm_residual_parts(m, n) >= 2 * -(-n // width[stream])  # (the room that any tile asks for)
