@@ -11,6 +11,7 @@ import torch
 
 import plain_llama as P
 from nnis_amd.errors import KernelError
+from nnis_amd.kernels.ops import GEMM_F32_NORM_ROWS, GEMM_F32_VARIANTS
 
 pytestmark = pytest.mark.gpu
 DT = {"float32": torch.float32, "bfloat16": torch.bfloat16}
@@ -82,7 +83,7 @@ def test_gemm_ordered(m, n, k, x_dtype, w_dtype, y_dtype):
         assert torch.equal(alone[0], y[m - 1])
 
 
-@pytest.mark.parametrize("variant", range(-1, 16))
+@pytest.mark.parametrize("variant", range(-1, GEMM_F32_VARIANTS))
 @pytest.mark.parametrize("m, n, k", [(1, 1, 4), (8, 40, 52), (7, 130, 548), (17, 33, 100), (65, 130, 176), (131, 257, 612), (5, 17, 2052)])
 def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
     """Every form of the product at sizes with tails in every dimension (K a multiple of 4 and of nothing more), against 64
@@ -108,31 +109,40 @@ def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
         assert ((y.cpu().double() - x.double() @ w.double().t()).abs() <= tol * (x.double().abs() @ w.double().abs().t())).all()
 
 
-@pytest.mark.parametrize("variant", [-1, 1, 2, 3, 4, 5, 7, 9, 10, 12, 13, 14, 15])
-@pytest.mark.parametrize("normed", [False, True])
-@pytest.mark.parametrize("m, n, k", [(1, 2, 4), (8, 70, 52), (5, 2 * 130, 548), (16, 34, 100), (65, 2 * 67, 176), (131, 256, 612)])
+def _f32_forms(rows, normed):
+    """The forms that take a product of so many 32-bit rows, with the norm before it or without."""
+    few = (-1, 0, 1, 13, 14, 15)  # (13: half strips, up to 8 rows)
+    return [v for v in range(-1, GEMM_F32_VARIANTS) if (v != 13 or rows <= 8) and not (normed and (rows > GEMM_F32_NORM_ROWS or v not in few))]
+
+
+UNPAIRED_F32_FORMS = (0, 6, 8, 11)  # a wave of theirs has no whole pair of strips: no gate, no rotation
+
+
+@pytest.mark.parametrize("m, n, k, normed, variant", [
+    (*sizes, normed, variant) for sizes in [(1, 2, 4), (8, 70, 52), (5, 2 * 130, 548), (16, 34, 100), (65, 2 * 67, 176), (131, 256, 612)]
+    for normed in (False, True) for variant in _f32_forms(sizes[0], normed)])
 def test_gemm_f32_with_what_comes_behind_it(m, n, k, normed, variant):
     """The gate, the sum into the stream and the plain store behind the product, with the norm before it or without, in
     every form that takes them, against 64 bits: the bound of the plain product, carried through the gate (whose slopes
     are below 1.1 times the other factor) and with the norm's own few roundings."""
     ops = _ops()
-    few = variant in (1, 13, 14, 15, -1)
-    if (variant == 13 and m > 8) or (normed and (m > 16 or not few)):
-        return
     torch.manual_seed(m + n + k)
     x, w, gain = torch.randn(m, k), torch.randn(n, k), 1 + 0.2 * torch.randn(k)
     rows = P.rms_norm(x.double(), gain.double(), 1e-5) if normed else x.double()
     product, scale = rows @ w.double().t(), 4e-7 * math.sqrt(k) * (rows.abs() @ w.double().abs().t()) + 1e-7
     norm = (gain.cuda(), 1e-5) if normed else ()
     out = torch.full((m + 1, n // 2), 7.0, device="cuda")
-    ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_SILU, *norm, variant=variant)
-    gate, up = product[:, :n // 2], product[:, n // 2:]
-    bound = 1.1 * (scale[:, :n // 2] * up.abs() + gate.abs() * scale[:, n // 2:]) + 1e-6 * (1 + (gate * up).abs()) + scale[:, :n // 2] * scale[:, n // 2:]
-    assert ((out[:m].cpu().double() - gate * torch.sigmoid(gate) * up).abs() <= bound).all() and (out[m] == 7).all()
-    if variant in (2, 3, 4, 5, 7, 9, 10, 12, -1) or few:
-        out = torch.full((m + 1, n), 7.0, device="cuda")
-        ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_STORE, *norm, variant=variant)
-        assert ((out[:m].cpu().double() - product).abs() <= scale).all() and (out[m] == 7).all()
+    if variant in UNPAIRED_F32_FORMS:
+        with pytest.raises(KernelError, match="no variant"):
+            ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_SILU, *norm, variant=variant)
+    else:
+        ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_SILU, *norm, variant=variant)
+        gate, up = product[:, :n // 2], product[:, n // 2:]
+        bound = 1.1 * (scale[:, :n // 2] * up.abs() + gate.abs() * scale[:, n // 2:]) + 1e-6 * (1 + (gate * up).abs()) + scale[:, :n // 2] * scale[:, n // 2:]
+        assert ((out[:m].cpu().double() - gate * torch.sigmoid(gate) * up).abs() <= bound).all() and (out[m] == 7).all()
+    out = torch.full((m + 1, n), 7.0, device="cuda")
+    ops.gemm_f32_fused(x.cuda(), w.cuda(), out[:m], ops.EPILOGUE_STORE, *norm, variant=variant)
+    assert ((out[:m].cpu().double() - product).abs() <= scale).all() and (out[m] == 7).all()
     if not normed:
         stream = torch.randn(m + 1, n)
         out = stream.cuda()
@@ -140,14 +150,12 @@ def test_gemm_f32_with_what_comes_behind_it(m, n, k, normed, variant):
         assert ((out[:m].cpu().double() - stream[:m].double() - product).abs() <= scale + 1e-6).all() and torch.equal(out[m].cpu(), stream[m])
 
 
-@pytest.mark.parametrize("variant", [-1, 1, 2, 4, 5, 12, 13, 14])
-@pytest.mark.parametrize("tokens, heads, kv_heads, head_dim, normed, tables", [(1, 9, 3, 64, True, True), (7, 3, 1, 32, True, False), (13, 4, 4, 96, False, True),
-                                                                              (70, 4, 2, 64, False, False)])
+@pytest.mark.parametrize("tokens, heads, kv_heads, head_dim, normed, tables, variant", [
+    (*case, variant) for case in [(1, 9, 3, 64, True, True), (7, 3, 1, 32, True, False), (13, 4, 4, 96, False, True), (70, 4, 2, 64, False, False)]
+    for variant in _f32_forms(case[0], case[4]) if variant not in UNPAIRED_F32_FORMS])
 def test_gemm_f32_rotates_and_writes_the_cache(tokens, heads, kv_heads, head_dim, normed, tables, variant):
     """The rotation and the cache write behind the product against the kernels of their own on the plain product."""
     ops = _ops()
-    if (variant == 13 and tokens > 8) or (normed and variant not in (-1, 1, 13, 14)):
-        return
     torch.manual_seed(tokens + head_dim)
     k, n = 100, (heads + 2 * kv_heads) * head_dim
     x, w, gain = torch.randn(tokens, k).cuda(), torch.randn(n, k).cuda(), (1 + 0.2 * torch.randn(k)).cuda()
@@ -659,7 +667,7 @@ def test_residual_projection_with_every_tile(tile, m, n, k):
     rows = ops.gemm_residual_parts(m, n)
     ss = torch.full((rows + 1, m), 7.0, device="cuda")
     parts = ops.gemm_residual(x.cuda(), ops.pack_weight(w.cuda()), resid_gpu, gain.cuda(), scaled, ss, getattr(ops, tile))
-    width = {"TILE_64x128": 64, "TILE_64x64": 32, "TILE_256x256": 128, "TILE_256x192": 96, "TILE_128x128": 64, "TILE_256x128": 64, "TILE_128x192": 96}[tile]  # columns of a wave
+    width = {"TILE_64x128": 64, "TILE_64x64": 32, "TILE_256x256": 128, "TILE_256x192": 96, "TILE_128x128": 64, "TILE_256x128": 64, "TILE_128x192": 96}[tile]  # columns of a part
     if parts != 2 * ((n + 2 * width - 1) // (2 * width)):  # few tiles and a long K: K went in parts, summed per 64 columns
         assert tile in ("TILE_64x128", "TILE_64x64") and k >= 512 and parts == (n + 63) // 64
         width = 64
