@@ -1567,7 +1567,6 @@ extern "C" int nnis_attention_rows_terms(const void* q, int q_dtype, void* out, 
 
 #if NNIS_MATRIX_CORES
 extern "C" int nnis_attention_f32_tile_rows(int heads, int kv_heads) { return heads == kv_heads ? 16 * kF32Columns : 16; }
-extern "C" int nnis_attention_f32_most_splits() { return kF32MostSplits; }
 
 // Everything in 32 bits.  tile_seq null: one token a sequence (tok_slot, tok_pos), its keys cut into `splits` blocks whose
 // outputs meet in `partial` (tokens * heads * splits * (HDV + 4) floats, with splits > 1).  Else `tiles` items of a step of prompts.

@@ -17,8 +17,11 @@
 //
 //  * gemm_f32_few_kernel: few rows of X (a decode step, a short prompt), or too few tiles to fill the chip.  The
 //    weight is streamed straight into operand registers; the waves of a block share K and meet in LDS.
-//  * gemm_f32_tiled_kernel: tiles of 64, 96 or 128 rows and columns, K in steps of 32 through a ring of stages in LDS.
+//  * gemm_f32_tiled_kernel: tiles of 32 to 128 rows and 64 to 128 columns, K in steps of 32 through a ring of stages in LDS.
+// Which of them, and so which chains, goes by the sizes: a row's last bits depend on how many rows the product has, where
+// the ordered kernel's do not.
 #include "common.h"
+#include "lds_loads.h"
 
 #include <type_traits>
 
@@ -26,10 +29,6 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-template <int N>
-__device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 __device__ __forceinline__ f32x4 load4(const float* p) { return *(const f32x4*)p; }
 __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
@@ -346,14 +345,6 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_few_kernel(const XT* __restri
 constexpr int kStepK = 32;      // k of a step: 128 bytes of a row, 8 chunks of 16 bytes
 constexpr int kFlushSteps = 8;  // a chain of sums is this many steps long, then goes into the total
 
-// (A buffer load: of one through a global address the compiler thinks that it may come back out of order with every
-// other, and then waits for all reads and loads in flight wherever it needs one of them.  A prompt of 509 tokens through a
-// 1.1B model 10.39 -> 9.97 ms.)
-__device__ __forceinline__ void load_to_lds(const void* base, int offset, char* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00027000), (lds_ptr_t)to, 16, offset, 0,
-                                           0, 0);
-}
-
 extern __shared__ __align__(16) char f32_lds[];  // NS stages of BM rows of X and BN rows of W
 
 // 4 waves, 2 x 2, each with BM / 2 rows and BN / 2 columns.  A load instruction of a wave brings 8 rows of 128 bytes
@@ -416,9 +407,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
     const int at = step * kStepK + chunk_k;
     const int from = (at < k ? at : 0) * 4;
 #pragma unroll
-    for (int o = 0; o < A_LOADS; ++o) load_to_lds(a_base, a_off[o] + from, base + o * 4096);
+    for (int o = 0; o < A_LOADS; ++o) load_to_lds(a_base, a_off[o] + from, 0, base + o * 4096);
 #pragma unroll
-    for (int o = 0; o < B_LOADS; ++o) load_to_lds(b_base, b_off[o] + from, base + A_BYTES + o * 4096);
+    for (int o = 0; o < B_LOADS; ++o) load_to_lds(b_base, b_off[o] + from, 0, base + A_BYTES + o * 4096);
   };
 
   f32x4 sum[TM][TN], total[TM][TN];
@@ -552,13 +543,13 @@ int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, i
 // 576 27.7 against 29.1, 32000 x 2048 59.1 against 61.5.  Pairs of strips, with the norm before them: half strips up to 8 rows
 // (576 wide, gated 3072 rows 6.0 against 7.2, rotated 960 6.5 against 7.4; 2048 wide, gated 11264 24.2 against 28.1; a 30-layer decode step of 8 sequences, 576 wide,
 // 1.51 -> 1.12 ms with the norms, gates, rotations and sums in the products), then two strips up to 8192 rows of weight (16
-// rows of 6144 x 2048 19.3 against 20.6).  Beyond 16 rows a variant's time is close to its rounds of blocks on 256
-// compute units times its blocks' time, which is a slope times K and a start: the least of these is taken.  Measured:
+// rows of 6144 x 2048 19.3 against 20.6).  Beyond 16 rows a variant's time is close to a start and, for every
+// round of its blocks on 256 compute units, a slope times K: the least of these is taken.  Measured:
 // 64 x 2048 x 2048 14.0 us (two strips, one tile a block), 128 x 2048 x 2048 18.7 (2 x 2), 128 x 11264 x 2048 60 (tiles of 64 x 96; 75
 // in 64 x 64), 509 x 2048 x 5632 112 (64 x 64), 4000 x 11264 x 2048 1,443 (128 x 128; 128 TFLOP/s of the instruction's 157).
 struct Variant {
   int rows, columns;  // of a block
-  float slope, start; // microseconds: slope * K + start for a round of blocks
+  float slope, start; // microseconds: slope * K for each round of blocks, and start
 };
 constexpr Variant kVariants[] = {
     {16, 16, 0.0050f, 2.0f}, {16, 32, 0.0064f, 2.0f}, {32, 32, 0.0083f, 2.0f}, {64, 32, 0.0135f, 2.0f},

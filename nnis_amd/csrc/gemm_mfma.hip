@@ -23,6 +23,7 @@
 // any M and N.
 #include "common.h"
 #include "epilogue.h"
+#include "lds_loads.h"
 #include "product.h"
 
 #include <type_traits>
@@ -327,19 +328,6 @@ __global__ __launch_bounds__(KSPLIT > 4 ? 64 * KSPLIT : 256) void gemm_skinny_ke
 // chunk c of row `row` of a staged tile (CHUNKS chunks of 16 bytes a row) lives at chunk c ^ (row % CHUNKS)
 template <int CHUNKS>
 __device__ __forceinline__ int swizzled(int row, int chunk) { return row * CHUNKS + (chunk ^ (row & (CHUNKS - 1))); }
-
-typedef __attribute__((address_space(1))) const void* global_ptr_t;
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-// The loads into LDS are not the compiler's to wait for: the kernel counts them itself.
-template <int N>
-__device__ __forceinline__ void wait_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
-// (A buffer load: of one through a global address the compiler thinks that it may come back out of order with every
-// other, and then waits for all reads and loads in flight wherever it needs one of them.)
-__device__ __forceinline__ void load_to_lds(const void* base, int offset, int uniform_offset, char* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00027000), (lds_ptr_t)to, 16, offset,
-                                           uniform_offset, 0, 0);
-}
 
 extern __shared__ __align__(16) char tile_lds[];  // NS stages of BM + BN rows of BK
 
@@ -1101,7 +1089,7 @@ void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n,
 }
 
 // the tiles of 256 x 256 (DIRECT, 4 stages of 32 KB) and 256 x 192 (2 of 56 KB), 8 waves, one block a compute unit; returns the parts of a row's sum of
-// squares that a residual epilogue wrote: one per wave column
+// squares that a residual epilogue wrote: two a column block
 template <int BN, typename OutT>
 int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
   const int col_blocks = (columns + BN - 1) / BN, row_blocks = (m + 255) / 256;
@@ -1355,7 +1343,7 @@ extern "C" int nnis_gemm_takes_pair(int m, int n, int k, size_t workspace_bytes)
 // nnis_gemm_residual_parts(m, n) are always enough.
 extern "C" int nnis_gemm_residual_parts(int m, int n) {
   (void)m;
-  // the kernel for few tokens: a part per strip of 16 columns; the tiled one a part per wave column of its tiles,
+  // the kernel for few tokens: a part per strip of 16 columns; the tiled one two parts a column of its tiles,
   // which is fewer from 17 columns on and two for a single tile
   return n > 16 ? (n + 15) / 16 : 2;
 }
