@@ -6,6 +6,7 @@ runs hand-written device code; none has a host or library stand-in.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional
 
 import torch
@@ -1908,20 +1909,40 @@ def run_pieces(ctx, state_bytes: int):
 CHUNKED_MOST_BYTES = 4 << 30
 
 
+def _delta_chunks_pay(mean: float, items: int, key_dim: int, value_dim: int) -> bool:
+    """Whether ``items`` (sequences x heads) walks of the gated delta rule over ``mean`` tokens each take less time in chunks than a
+    token at a time.  Either form's time, in microseconds, is the larger of its chain, one sequence's way through its tokens or
+    chunks, and of its work on the whole chip (between the two where they are alike)."""
+    # Fitted to 602 steps measured in both forms: heads of 32 x 64 to 128 x 256, 4 to 32 of them, 1 to 64 sequences of 65 to 1,300 tokens,
+    # unequal by up to 20; a standard deviation of 9% and 7%.  By the rule no step is more than 4% slower in chunks but those planned
+    # for nearly twice their tokens (1 x 65: 36 / 42) and 256 and more walks of 64 x 128 over 450 to 1,300 tokens (16 x 16 x 700 449 / 526), and none
+    # that stays with its tokens gives away more than 16%.  Microseconds a token at a time / in chunks: 16 heads of 128 x 128, 1 x 128 59 / 42, 2 x 112 56 /
+    # 45, 4 x 113 68 / 66, 8 x 145 118 / 127, 8 x 192 149 / 133, 16 x 101 164 / 191, 32 x 200 575 / 659, 64 x 300 1,788 / 1,646; 16 heads of 64 x 64, 64 x 200
+    # 270 / 524; 8 of 64 x 128, 4 x 120 52 / 34, 64 x 170 219 / 345.  (A rule by tokens a sequence alone, 160 from 8 sequences on, took up to
+    # twice the time where walks are many.)
+    if mean <= 64:
+        return False  # (a step planned for 64 rows may have two)
+    area, chunks = key_dim * value_dim / 16384, mean / 64 + 0.5
+    chain, work = 17 + 0.35 * mean, items * mean * (0.0056 * area + 0.00006)
+    token = (chain ** 3 + work ** 3) ** (1 / 3)
+    chunk = math.hypot(16 + key_dim / 5.8 + chunks * (1.5 + key_dim / 116), items * (chunks * (0.06 + 0.16 * area) + 0.29 * area + 0.08))
+    return chunk < 0.95 * token
+
+
 def chunked_scratch(ctx, tokens: int, heads: int, key_dim: int, value_dim: int, delta: bool, device) -> Optional[torch.Tensor]:
     """Scratch for a step of ``tokens`` rows whose sequences a matrix-state recurrence walks in chunks of 64 tokens
     (csrc/chunked_state.hip); None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts too
     short.  Which of the two goes by the rows that the step plans for, not by those at hand: a step that is launched and the same step
     replayed from a graph's rows take the same form (their results are rounded differently)."""
-    # Microseconds a token at a time and in chunks, by sequences x tokens; an engine's steps plan for their tokens rounded up to 64 and
-    # more, so the first of a pair that a rule takes in is given.  Delta rule, 16 heads of 128 x 128: 1 x 65 35 / 40 (planned for 128), 1 x
-    # 80 41 / 40, 1 x 128 59 / 42; 2 x 97 51 / 44; 4 x 113 68 / 66; 8 x 145 118 / 127, 8 x 192 149 / 133; 16 x 161 238 / 240.  Retention, 8
-    # heads of 128 x 256: 1 x 2 9 / 12 (planned for 64), 1 x 8 14 / 12, 1 x 16 21 / 13, 1 x 64 46 / 14; 4 x 25 29 / 19; 8 x 25 30 / 29; 16 x 33
-    # 43 / 48, 16 x 48 140 / 49.  (Its token at a time is split into pieces.)
-    least = 96 + 8 * min(ctx.batch, 8) if delta else 16 + 2 * min(ctx.batch, 16)
     lib = recurrent()
+    if ctx.decode or ctx.batch == 0 or not lib.nnis_chunked_takes(key_dim, value_dim):
+        return None
     planned = max(tokens, ctx.planned_rows)
-    if ctx.decode or planned < least * max(ctx.batch, 1) or not lib.nnis_chunked_takes(key_dim, value_dim):
+    # Retention, microseconds a token at a time and in chunks, by sequences x tokens, 8 heads of 128 x 256: 1 x 2 9 / 12 (planned for 64), 1 x
+    # 8 14 / 12, 1 x 16 21 / 13, 1 x 64 46 / 14; 4 x 25 29 / 19; 8 x 25 30 / 29; 16 x 33 43 / 48, 16 x 48 140 / 49; 64 x 50 536 / 218, 128 x 48 922 / 578.
+    # (Its token at a time is split into pieces from 48 tokens on.)
+    if not (_delta_chunks_pay(planned / ctx.batch, ctx.batch * heads, key_dim, value_dim) if delta
+            else planned >= (16 + 2 * min(ctx.batch, 16)) * ctx.batch):
         return None
     floats = lambda rows: lib.nnis_chunked_scratch(rows, ctx.batch, heads, key_dim, value_dim, 1 if delta else 0)  # noqa: E731
     return torch.empty(floats(tokens), dtype=torch.float32, device=device) if 4 * floats(planned) <= CHUNKED_MOST_BYTES else None

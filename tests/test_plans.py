@@ -77,7 +77,7 @@ def test_prefill_plan_by_class_and_size():
     assert prefill_plan(3072, 3072, 32, 64, 32) == (4, 0)
 
 
-@pytest.mark.parametrize("delta, least", [(True, {1: 128, 4: 512, 8: 1280, 16: 2560}), (False, {1: 64, 4: 128, 16: 768})])
+@pytest.mark.parametrize("delta, least", [(True, {1: 128, 4: 320, 16: 1280}), (False, {1: 64, 4: 128, 16: 768})])
 def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(delta, least):
     """Chunks or a token at a time by the rows that a step plans for (64 and more, ``prompt_rows``): the same at the tokens that are
     launched and at the rows that are replayed, and scratch for no more rows than are there."""
@@ -104,6 +104,21 @@ def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(d
     assert scratch(1, 1279, 1280, heads=heads) is not None and scratch(1, 1280, 1280, heads=heads) is not None
     assert scratch(1, 1279, 1280, heads=heads + 1) is None and scratch(1, 1280, 1280, heads=heads + 1) is None
     assert scratch(8, 8, 4096, decode=True) is None  # single tokens
+
+
+@pytest.mark.parametrize("heads, key_dim, value_dim, sequences, tokens, chunks", [
+    (16, 128, 128, 1, 128, True), (16, 128, 128, 1, 1500, True), (16, 128, 128, 8, 2048, True), (16, 128, 128, 64, 300, True),  # 59 / 42, 602 / 135, 1,500 / 1,020, 1,788 / 1,646
+    (16, 128, 128, 16, 101, False), (16, 128, 128, 32, 200, False), (16, 128, 128, 64, 170, False),  # 164 / 191, 575 / 659, 978 / 1,142
+    (16, 64, 64, 64, 200, False), (8, 64, 128, 64, 170, False), (8, 32, 64, 64, 180, False), (8, 64, 128, 32, 200, False),  # 270 / 524, 219 / 345, 108 / 201, 140 / 196
+    (8, 64, 128, 4, 120, True), (4, 32, 32, 16, 170, True), (4, 64, 64, 1, 64, False)])  # 52 / 34, 65 / 37; a chunk may hold two tokens
+def test_the_delta_rule_goes_in_chunks_where_that_is_faster(heads, key_dim, value_dim, sequences, tokens, chunks):
+    """Measured steps, microseconds a token at a time / in chunks: many walks fill the chip a token at a time."""
+    import types
+
+    from nnis_amd.kernels import ops
+
+    ctx = types.SimpleNamespace(decode=False, batch=sequences, planned_rows=sequences * tokens)
+    assert (ops.chunked_scratch(ctx, sequences * tokens, heads, key_dim, value_dim, True, "meta") is not None) == chunks
 
 
 def test_the_tiles_of_products_into_the_stream():
