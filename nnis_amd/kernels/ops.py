@@ -863,14 +863,19 @@ def attention_f32(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_p
     return out
 
 
-def attention_f32_splits(tokens: int, heads: int, kv_heads: int, window: int, longest: int) -> int:
+def attention_f32_splits(tokens: int, heads: int, kv_heads: int, window: int, longest: int, size: int = 64) -> int:
     """The blocks that a step of single tokens cuts an item's keys into: as many as bring the step to F32_BLOCKS blocks
     of 4 waves, of which each gets a tile of 16 keys where a sequence has as many as it may come to have (``longest``, or
-    the window).  It does not go by the step's own lengths, so that a captured step serves them all."""
+    the window).  It does not go by the step's own lengths, so that a captured step serves them all.  ``size``: a head's channels (of
+    keys or values, the larger)."""
     # Microseconds with 1 / 4 / 8 / 16 blocks an item (a second kernel sums them): 1 token of 1,000 keys on 3 key/value heads of
     # 64 21 / 12 / 10 / 9, 8 of 2,000 37 / 17 / 13 / 13, 32 of 60 to 1,610 32 / 19.5 / 21 / 23; 8 of 2,000 on 32 heads 42 / 50 / 51 / 58.
+    # Heads of up to 32 channels over up to 256 keys (1 block / 2 / 4, and the row kernel): 16 channels, 100 keys 5.8 / 8.4 / 8.2 (5.7), 200 7.2 / 9.1
+    # / 8.4 (7.0); 32 channels, 100 keys 6.1 / 8.5 / 8.7 (7.6), 200 7.8 / 9.6 / 8.5 (9.7), 300 8.6 / 10.2 / 9.4 and 8.7 with 8 (10.3).
     items = tokens * kv_heads * ((heads // kv_heads + 15) // 16)
     keys = longest if window == 0 else min(longest, abs(window) + 15)
+    if size <= 32 and keys <= 256:
+        return 1
     return max(1, min(F32_BLOCKS // max(items, 1), (keys + 63) // 64, ATTENTION_F32_MOST_SPLITS))
 
 
@@ -1667,9 +1672,10 @@ def attention(q: torch.Tensor, out: torch.Tensor, view, ctx, heads: int, kv_head
     for the last n keys, or n < 0 for the keys of the query's own chunk of -n
     positions."""
     value_dim = value_dim or head_dim
-    if attention_f32_takes(q, out, view.k_pages, view.v_pages, head_dim, value_dim):
+    if (attention_f32_takes(q, out, view.k_pages, view.v_pages, head_dim, value_dim)
+            and (ctx.decode or ctx.planned_rows * heads >= attention_f32_least(head_dim, value_dim))):
         if ctx.decode:
-            tiles, splits = None, attention_f32_splits(q.shape[0], heads, kv_heads, window, 64 * view.block_table.shape[1])
+            tiles, splits = None, attention_f32_splits(q.shape[0], heads, kv_heads, window, 64 * view.block_table.shape[1], max(head_dim, value_dim))
         else:
             rows = attention_module(head_dim, value_dim, softcap, extras, pooled, terms).nnis_attention_f32_tile_rows(heads, kv_heads)
             items = ctx.lists.device_list(("attention_tiles", rows), lambda new, first, padded: prefill_tile_list(new, first, padded, rows))
@@ -1714,6 +1720,15 @@ def attention_f32_takes(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tenso
     """Whether ``attention`` takes ``attention_f32`` for 32-bit operands of these sizes (else the row kernel)."""
     return (q.dtype == out.dtype == k_pages.dtype == torch.float32 and head_dim % 16 == 0 and value_dim % 16 == 0
             and max(head_dim, value_dim) <= ATTENTION_MOST_CHANNELS and not (q.data_ptr() | out.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) & 15)
+
+
+def attention_f32_least(head_dim: int, value_dim: int) -> int:
+    """Query rows x heads that a step of prompts has to plan for to take ``attention_f32``; below it the row kernel is faster."""
+    # Microseconds, rows / matrix cores: 16 channels, 4 heads 64 tokens 5.4 / 7.2, 300 8.1 / 11.5, 1,200 27.3 / 26.2; 9 heads 300 9.4 / 11.4, 600
+    # 18.9 / 17.0, 8 prompts of 64 9.9 / 7.3; 32 heads 64 6.4 / 7.3, 150 10.3 / 9.4.  32 channels, 4 heads 150 9.2 / 10.3, 300 11.6 / 12.8, 600 20.5 / 19.4; 9
+    # heads 64 7.2 / 7.7, 300 14.4 / 12.9; 32 heads 64 9.2 / 7.7.  48 channels, 4 heads 64 8.9 / 8.2, 300 15.9 / 14.5.
+    size = max(head_dim, value_dim)
+    return 4096 if size <= 16 else (2048 if size <= 32 else 0)
 
 
 def sample(logits: torch.Tensor, weights: torch.Tensor, row_slot: torch.Tensor, rng: torch.Tensor,

@@ -121,6 +121,18 @@ def test_the_delta_rule_goes_in_chunks_where_that_is_faster(heads, key_dim, valu
     assert (ops.chunked_scratch(ctx, sequences * tokens, heads, key_dim, value_dim, True, "meta") is not None) == chunks
 
 
+def test_32_bit_attention_of_small_heads():
+    """One block for single tokens of small heads over few keys, and the row kernel for few rows of them, as measured."""
+    from nnis_amd.kernels import ops
+
+    for size, keys, splits in ((16, 100, 1), (32, 256, 1), (32, 320, 5), (16, 2048, 16), (48, 100, 2), (64, 1024, 16)):
+        assert ops.attention_f32_splits(1, 9, 3, 0, keys, size) == splits
+        assert ops.attention_f32_splits(1, 9, 3, keys - 15, 8192, size) == ops.attention_f32_splits(1, 9, 3, 15 - keys, 8192, size) == splits
+    assert ops.attention_f32_least(16, 16) > 300 * 9 and ops.attention_f32_least(16, 16) < 600 * 9 and ops.attention_f32_least(16, 16) < 150 * 32
+    assert ops.attention_f32_least(32, 16) == ops.attention_f32_least(16, 32) > 300 * 4 and ops.attention_f32_least(32, 32) <= 64 * 32
+    assert ops.attention_f32_least(48, 16) == ops.attention_f32_least(64, 64) == 0
+
+
 def test_the_tiles_of_products_into_the_stream():
     """A product into the residual stream goes by rates of its own (the parts of its rows' sums of squares follow the tile)."""
     from nnis_amd.kernels import ops
