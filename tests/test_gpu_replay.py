@@ -128,7 +128,7 @@ def test_measured_shapes_agree_with_the_plain_model(tmp_path, shape, dtype):
         part = {(n[1:], p): row for (n, p), row in rows.items() if n[0] == tag}
         assert len(part) == total
         if dtype == "float32" and config["hidden_size"] > 2048:
-            # sums of up to 14,336 terms: the engine's one chain a sum against the plain model's sums in blocks
+            # sums of up to 14,336 terms: against 64 bits, by what the plain model in 32-bit is off
             if wide is None:
                 plain64 = P.PlainLlama(str(folder), torch.float64)
                 wide = Fp32Yardstick(plain64, plain, [requests["r3"], requests["r4"]])
