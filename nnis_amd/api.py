@@ -18,7 +18,7 @@ def load_model(model_dir: str, dtype="bfloat16", device="cuda:0", narrow_to_bflo
     tensors by name and binds them to the parts.  Returns (model, runtime).
     ``narrow_to_bfloat16``: a checkpoint stored in 32-bit is rounded to
     bfloat16 as it is loaded (only with ``dtype`` bfloat16); without it its
-    weights stay 32-bit and take the slow ordered product."""
+    weights stay 32-bit and take the slower 32-bit products."""
     raw = read_config_json(model_dir)
     _, spec = spec_from_config(raw)
     rt = Runtime(device=device, dtype=dtype)
