@@ -119,9 +119,11 @@ class StepContext:
     host_new: Optional[List[int]] = field(default_factory=list)
     host_pos0: Optional[List[int]] = field(default_factory=list)
     # What the parts plan their launches for, where it is not the step itself (a captured step is replayed for
-    # other lengths and fewer rows than it was captured with): the longest sequence, and the step's rows.
+    # other lengths and fewer rows than it was captured with): the longest sequence, the step's rows, and the most tokens that
+    # a sequence brings.
     plan_len: int = 0
     plan_rows: int = 0
+    plan_new: int = 0
     options: dict = field(default_factory=dict)  # launch options by part kind, for tests and tuning: {"causal_attention": {...}}
     lists: Optional[StepLists] = None  # the parts' host-made work lists (``StepLists``)
     ids: Optional[torch.Tensor] = None  # int32 [tokens]: the step's tokens, for parts that read them beside the stream
@@ -138,6 +140,10 @@ class StepContext:
     @property
     def planned_rows(self) -> int:
         return self.plan_rows or self.tokens
+
+    @property
+    def planned_new(self) -> int:
+        return self.plan_new or self.max_new
 
     def step_tables(self, rt, rotary=None, block_table=None):
         """Each token's rows of the rotation tables ``rotary`` and its pages

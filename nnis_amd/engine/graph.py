@@ -172,11 +172,12 @@ def prompt_rows(total: int) -> int:
 
 
 class PrefillGraph:
-    def __init__(self, engine, batch: int, total: int, wanted: int, plan_len: int):
+    def __init__(self, engine, batch: int, total: int, wanted: int, plan_len: int, plan_new: int = 0):
         """``total``: the rows of the step (``prompt_rows`` of its tokens), ``batch``: its sequences,
-        ``plan_len``: a longest sequence for which the parts plan as they do for this shape."""
+        ``plan_len``, ``plan_new``: a longest sequence and a most tokens that one brings for which the parts plan as they do for this
+        shape."""
         self.engine = engine if isinstance(engine, weakref.ProxyTypes) else weakref.proxy(engine)
-        self.batch, self.total, self.plan_len = batch, total, plan_len
+        self.batch, self.total, self.plan_len, self.plan_new = batch, total, plan_len, plan_new
         # the step's arrays in one buffer, in the order the step function stages them
         self.sizes = [total, total, total, batch, batch + 1, batch, wanted]
         self.lists = None  # the parts' work lists: who makes which, as the first run found them
@@ -207,7 +208,7 @@ class PrefillGraph:
         self.ctx = StepContext(
             tokens=self.total, batch=self.batch, tok_slot=views[1], tok_pos=views[2], seq_slot=views[3], seq_start=views[4],
             seq_pos0=views[5], decode=False, max_new=self.total, max_len=self.plan_len, host_new=None, host_pos0=None,
-            plan_len=self.plan_len, plan_rows=self.total, lists=self.lists)
+            plan_len=self.plan_len, plan_rows=self.total, plan_new=self.plan_new, lists=self.lists)
 
     def fill(self, arrays, counts: Sequence[int], first_positions: Sequence[int]) -> None:
         """The step's data into the buffers: ``arrays`` as the step function stages them (ids, slot and position
@@ -300,7 +301,7 @@ class PrefillGraphs:
         if times < 2:
             return None
         batch, total, wanted, _ = key
-        graph = PrefillGraph(self.engine, batch, total, wanted, longest)
+        graph = PrefillGraph(self.engine, batch, total, wanted, longest, max(counts))
         logits = graph.first_run(arrays, counts, first_positions)
         if graph.graph is None:
             self.refused.add(key)

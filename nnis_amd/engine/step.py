@@ -185,7 +185,7 @@ class Engine:
         if (self.use_graphs and total <= PREFILL_GRAPH_MOST_TOKENS and want_rows
                 and total * float(self.model.spec.width) ** 2 <= PREFILL_GRAPH_MOST_WORK):
             # a shape that comes again is replayed from a graph (engine/graph.py)
-            shape = (len(counts), rows, len(want_rows), self.model.prompt_plan(len(counts), rows, longest, self.rt))
+            shape = (len(counts), rows, len(want_rows), self.model.prompt_plan(len(counts), rows, longest, self.rt, max(counts)))
             if self._prefill_graphs is None:
                 self._prefill_graphs = PrefillGraphs(self)
             done = self._prefill_graphs.step(shape, arrays, counts, pos0, longest)

@@ -1924,40 +1924,48 @@ def run_pieces(ctx, state_bytes: int):
 CHUNKED_MOST_BYTES = 4 << 30
 
 
-def _delta_chunks_pay(mean: float, items: int, key_dim: int, value_dim: int) -> bool:
-    """Whether ``items`` (sequences x heads) walks of the gated delta rule over ``mean`` tokens each take less time in chunks than a
-    token at a time.  Either form's time, in microseconds, is the larger of its chain, one sequence's way through its tokens or
-    chunks, and of its work on the whole chip (between the two where they are alike)."""
+def chunks_pay(delta: bool, batch: int, rows: int, longest: int, heads: int, key_dim: int, value_dim: int) -> bool:
+    """Whether a matrix-state recurrence of ``heads`` heads (``delta``: the gated delta rule, else retention) walks a step of ``batch``
+    sequences, planned for ``rows`` tokens in all and ``longest`` in one of them, in less time in chunks than a token at a time."""
+    if not delta:
+        # Retention, microseconds a token at a time and in chunks, by sequences x tokens, 8 heads of 128 x 256: 1 x 2 9 / 12 (planned for 64), 1 x
+        # 8 14 / 12, 1 x 16 21 / 13, 1 x 64 46 / 14; 4 x 25 29 / 19; 8 x 25 30 / 29; 16 x 33 43 / 48, 16 x 48 140 / 49; 64 x 50 536 / 218, 128 x 48 922 / 578.
+        # Unequal ones: 400 and 15 x 16 136 / 61, 100 and 7 x 2 79 / 34, 1,500 and 63 x 16 968 / 244; 47 and 15 x 10 50 / 52.  (A step with a run of
+        # RUN_PIECE_FROM tokens goes through three passes over pieces a token at a time, all its sequences.)  Of 119 steps measured, equal and
+        # not, one was more than 8% slower in the form that this gives (2 sequences of 12 and 10, planned for 64: 19 / 22).
+        return longest >= RUN_PIECE_FROM or rows >= (16 + 2 * min(batch, 16)) * batch
+    # Either form's time, in microseconds, is the larger of its chain, a sequence's way through its tokens or chunks, and of its work on the
+    # whole chip (between the two where they are alike), and what the longest sequence has to go alone once the others are through.
     # Fitted to 602 steps measured in both forms: heads of 32 x 64 to 128 x 256, 4 to 32 of them, 1 to 64 sequences of 65 to 1,300 tokens,
     # unequal by up to 20; a standard deviation of 9% and 7%.  By the rule no step is more than 4% slower in chunks but those planned
-    # for nearly twice their tokens (1 x 65: 36 / 42) and 256 and more walks of 64 x 128 over 450 to 1,300 tokens (16 x 16 x 700 449 / 526), and none
+    # for nearly twice their tokens and 256 and more walks of 64 x 128 over 450 to 1,300 tokens (16 x 16 x 700 449 / 526), and none
     # that stays with its tokens gives away more than 16%.  Microseconds a token at a time / in chunks: 16 heads of 128 x 128, 1 x 128 59 / 42, 2 x 112 56 /
     # 45, 4 x 113 68 / 66, 8 x 145 118 / 127, 8 x 192 149 / 133, 16 x 101 164 / 191, 32 x 200 575 / 659, 64 x 300 1,788 / 1,646; 16 heads of 64 x 64, 64 x 200
     # 270 / 524; 8 of 64 x 128, 4 x 120 52 / 34, 64 x 170 219 / 345.  (A rule by tokens a sequence alone, 160 from 8 sequences on, took up to
-    # twice the time where walks are many.)
-    if mean <= 64:
-        return False  # (a step planned for 64 rows may have two)
-    area, chunks = key_dim * value_dim / 16384, mean / 64 + 0.5
-    chain, work = 17 + 0.35 * mean, items * mean * (0.0056 * area + 0.00006)
-    token = (chain ** 3 + work ** 3) ** (1 / 3)
-    chunk = math.hypot(16 + key_dim / 5.8 + chunks * (1.5 + key_dim / 116), items * (chunks * (0.06 + 0.16 * area) + 0.29 * area + 0.08))
-    return chunk < 0.95 * token
+    # twice the time where walks are many.)  Unequal lengths, 211 more steps, none more than 12% slower in the form that this gives than in
+    # the other but for 27 / 24 of one prompt of 56: 16 heads of 128 x 128, 1,500 and 15 x 100 658 / 288, 1,500 and 15 x 16 608 / 225, 1,500 and 63 x 16 635 / 687,
+    # 400 and 15 x 16 181 / 168; 8 of 64 x 128, 700 and 15 x 30 264 / 68.  (By the mean length alone the first took its tokens one at a time.)
+    if longest <= 64:
+        return False
+    mean, items, area = rows / batch, batch * heads, key_dim * value_dim / 16384
+    like = min(mean, longest)
+    per_chunk, alone = 1.5 + key_dim / 116, longest - like
+    chain, work = 17 + 0.35 * like, items * mean * (0.0056 * area + 0.00006)
+    token = (chain ** 3 + work ** 3) ** (1 / 3) + 0.3 * alone
+    chunk = math.hypot(16 + key_dim / 5.8 + (like / 64 + 0.5) * per_chunk, items * ((mean / 64 + 0.5) * (0.06 + 0.16 * area) + 0.29 * area + 0.08))
+    return chunk + alone / 64 * per_chunk < 0.95 * token
 
 
 def chunked_scratch(ctx, tokens: int, heads: int, key_dim: int, value_dim: int, delta: bool, device) -> Optional[torch.Tensor]:
     """Scratch for a step of ``tokens`` rows whose sequences a matrix-state recurrence walks in chunks of 64 tokens
-    (csrc/chunked_state.hip); None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts too
-    short.  Which of the two goes by the rows that the step plans for, not by those at hand: a step that is launched and the same step
-    replayed from a graph's rows take the same form (their results are rounded differently)."""
+    (csrc/chunked_state.hip); None for a step that goes a token at a time: single tokens, other sizes of heads, and prompts for
+    which chunks do not pay.  Which of the two goes by what the step plans for, not by the rows at hand: a step that is launched and the
+    same step replayed from a graph's rows take the same form (their results are rounded differently)."""
     lib = recurrent()
     if ctx.decode or ctx.batch == 0 or not lib.nnis_chunked_takes(key_dim, value_dim):
         return None
     planned = max(tokens, ctx.planned_rows)
-    # Retention, microseconds a token at a time and in chunks, by sequences x tokens, 8 heads of 128 x 256: 1 x 2 9 / 12 (planned for 64), 1 x
-    # 8 14 / 12, 1 x 16 21 / 13, 1 x 64 46 / 14; 4 x 25 29 / 19; 8 x 25 30 / 29; 16 x 33 43 / 48, 16 x 48 140 / 49; 64 x 50 536 / 218, 128 x 48 922 / 578.
-    # (Its token at a time is split into pieces from 48 tokens on.)
-    if not (_delta_chunks_pay(planned / ctx.batch, ctx.batch * heads, key_dim, value_dim) if delta
-            else planned >= (16 + 2 * min(ctx.batch, 16)) * ctx.batch):
+    if not chunks_pay(delta, ctx.batch, planned, ctx.planned_new, heads, key_dim, value_dim):
         return None
     floats = lambda rows: lib.nnis_chunked_scratch(rows, ctx.batch, heads, key_dim, value_dim, 1 if delta else 0)  # noqa: E731
     return torch.empty(floats(tokens), dtype=torch.float32, device=device) if 4 * floats(planned) <= CHUNKED_MOST_BYTES else None

@@ -81,15 +81,18 @@ class DecoderModel:
         """What the parts' kernels keep between calls and a captured step has baked in (``Part.held_buffers``)."""
         return [buffer for part in self.parts() for buffer in part.held_buffers(rt)]
 
-    def prompt_plan(self, batch: int, rows: int, longest: int, rt):
-        """The plans of every run of the schedule for a step of prompts (``Part.prompt_plan``)."""
-        key = (batch, rows, longest)
+    def prompt_plan(self, batch: int, rows: int, longest: int, rt, most_new: int = 0):
+        """The plans of every run of the schedule for a step of prompts (``Part.prompt_plan``, ``Part.run_plan``);
+        ``most_new``: the most tokens that a sequence brings (0: all rows of a step of one, their mean of several)."""
+        most_new = most_new or -(-rows // max(batch, 1))
+        key = (batch, rows, longest, most_new)
         plans = self._prompt_plans.get(key)
         if plans is None:
             if len(self._prompt_plans) > 4096:
                 self._prompt_plans.clear()
             plans = self._prompt_plans[key] = tuple(
-                self.layers[entry.layer].prompt_plan(batch, rows, longest, rt) for entry in self.spec.schedule)
+                plan for layer in (self.layers[entry.layer] for entry in self.spec.schedule)
+                for plan in (layer.prompt_plan(batch, rows, longest, rt), layer.run_plan(batch, rows, most_new, rt)))
         return plans
 
     def decode_plan(self, batch: int, longest: int, rt):

@@ -24,7 +24,7 @@ The interfaces:
     ``forward(x, ctx, view, rt)`` -> y, where ``x`` is ``[tokens, width]`` in
     the activation type, ``ctx`` is the step's ``StepContext`` and ``view``
     is the cache's view for this schedule entry.  A mixer whose launches
-    depend on the step's lengths says how (``decode_plan``, ``prompt_plan``);
+    depend on the step's lengths says how (``decode_plan``, ``prompt_plan``, ``run_plan``);
     lists that it makes on the host for a step of prompts go through
     ``ctx.lists`` (``StepLists``), which is what lets the step be replayed.  A mixer that sets
     ``takes_pending_norm = True`` is handed a ``PendingNorm`` instead of ``x``
@@ -147,6 +147,11 @@ class Part:
         """The same for a step of prompts: ``batch`` sequences that bring
         ``rows`` tokens between them (rounded up as the engine rounds a
         replayed step's rows), the longest of ``longest`` tokens after it."""
+        return None
+
+    def run_plan(self, batch: int, rows: int, most_new: int, rt):
+        """The same where a part's launches for a step of prompts depend on
+        the most tokens that a sequence brings, ``most_new``."""
         return None
 
     def held_buffers(self, rt):

@@ -78,6 +78,9 @@ class PreNormBlock(Block):
     def prompt_plan(self, batch, rows, longest, rt):
         return _joined(part.prompt_plan(batch, rows, longest, rt) for part in self._parts)
 
+    def run_plan(self, batch, rows, most_new, rt):
+        return _joined(part.run_plan(batch, rows, most_new, rt) for part in self._parts)
+
     def held_buffers(self, rt):
         return [buffer for part in self._parts for buffer in part.held_buffers(rt)]
 
@@ -196,6 +199,9 @@ class HyperConnectionBlock(Block):
     def prompt_plan(self, batch, rows, longest, rt):
         return _joined(part.prompt_plan(batch, rows, longest, rt) for part in self._parts)
 
+    def run_plan(self, batch, rows, most_new, rt):
+        return _joined(part.run_plan(batch, rows, most_new, rt) for part in self._parts)
+
     def held_buffers(self, rt):
         return [buffer for part in self._parts for buffer in part.held_buffers(rt)]
 
@@ -284,6 +290,9 @@ class PrePostNormBlock(Block):
 
     def prompt_plan(self, batch, rows, longest, rt):
         return _joined(part.prompt_plan(batch, rows, longest, rt) for part in self._parts)
+
+    def run_plan(self, batch, rows, most_new, rt):
+        return _joined(part.run_plan(batch, rows, most_new, rt) for part in self._parts)
 
     def held_buffers(self, rt):
         return [buffer for part in self._parts for buffer in part.held_buffers(rt)]
@@ -411,6 +420,9 @@ class PostNormBlock(Block):
 
     def prompt_plan(self, batch, rows, longest, rt):
         return _joined(part.prompt_plan(batch, rows, longest, rt) for part in self._parts)
+
+    def run_plan(self, batch, rows, most_new, rt):
+        return _joined(part.run_plan(batch, rows, most_new, rt) for part in self._parts)
 
     def held_buffers(self, rt):
         return [buffer for part in self._parts for buffer in part.held_buffers(rt)]

@@ -217,6 +217,9 @@ class Retention(Mixer):
     def weight_bytes(self):
         return self.qkvg.weight_bytes() + self.out.weight_bytes()
 
+    def run_plan(self, batch, rows, most_new, rt):
+        return rt.ops.chunks_pay(False, batch, rows, most_new, self.heads, self.key_dim, self.value_dim)
+
     def cache_request(self):
         return StateRequest((self.heads, self.key_dim, self.value_dim))
 
@@ -291,6 +294,9 @@ class GatedDeltaRule(Mixer):
     def weight_bytes(self):
         small = sum(t.numel() * t.element_size() for t in (self.conv, self.rate, self.dt_bias, self.norm))
         return small + sum(p.weight_bytes() for p in (self.qkvg, self.ba, self.out))
+
+    def run_plan(self, batch, rows, most_new, rt):
+        return rt.ops.chunks_pay(True, batch, rows, most_new, self.heads, self.key_dim, self.value_dim)
 
     def cache_request(self):
         # (the matrix state lies column by column: a value channel's key rows are consecutive)
@@ -571,6 +577,10 @@ class SideBySide(Mixer):
 
     def prompt_plan(self, batch, rows, longest, rt):
         plans = tuple(branch.prompt_plan(batch, rows, longest, rt) for branch in self.branches)
+        return None if all(plan is None for plan in plans) else plans
+
+    def run_plan(self, batch, rows, most_new, rt):
+        plans = tuple(branch.run_plan(batch, rows, most_new, rt) for branch in self.branches)
         return None if all(plan is None for plan in plans) else plans
 
     def held_buffers(self, rt):

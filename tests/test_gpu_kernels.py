@@ -1254,7 +1254,7 @@ def test_matrix_states_in_chunks(delta, heads, groups, d, e, dtype, lengths, mon
     tokens, batch, starts = sum(lengths), len(lengths), [0, *np.cumsum(lengths).tolist()]
     positions = [40 + i for n in lengths for i in range(n)]
     slots = list(range(batch, 0, -1))
-    ctx = types.SimpleNamespace(decode=False, batch=batch, tokens=tokens, max_new=max(lengths), planned_rows=max(lengths), seq_slot=_i32(slots), seq_start=_i32(starts),
+    ctx = types.SimpleNamespace(decode=False, batch=batch, tokens=tokens, max_new=max(lengths), planned_new=max(lengths), planned_rows=max(lengths), seq_slot=_i32(slots), seq_start=_i32(starts),
                                 tok_slot=_i32([s for s, n in zip(slots, lengths) for _ in range(n)]), tok_pos=_i32(positions))
     state = 0.3 * torch.randn(batch + 1, heads, *((e, d) if delta else (d, e)))
     if delta:
@@ -1304,7 +1304,7 @@ def _prompts(lengths):
 
     starts = [0, *np.cumsum(lengths).tolist()]
     return types.SimpleNamespace(
-        decode=False, batch=len(lengths), tokens=sum(lengths), max_new=max(lengths), planned_rows=sum(lengths), seq_slot=_i32(range(len(lengths))),
+        decode=False, batch=len(lengths), tokens=sum(lengths), max_new=max(lengths), planned_new=max(lengths), planned_rows=sum(lengths), seq_slot=_i32(range(len(lengths))),
         seq_start=_i32(starts), tok_slot=_i32([s for s, n in enumerate(lengths) for _ in range(n)]), tok_pos=_i32([i for n in lengths for i in range(n)]))
 
 

@@ -596,6 +596,39 @@ def test_a_prompt_launched_captured_and_replayed_takes_the_same_recurrences(tmp_
         assert len(engine._prefill_graphs.graphs) == 1
 
 
+def test_steps_of_one_size_and_other_lengths_keep_their_recurrences_when_replayed(tmp_path, monkeypatch):
+    """Two steps of three prompts and 128 tokens, one with a long prompt, that take different forms of the delta rule: each is launched,
+    captured and replayed in its own."""
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    config = mafalorn(vocab=200, width=64, logit_scale=1.5, layers=[
+        layer("parallel", parallel(softmax(2, 1, 16, scale=0.3), delta(2, 1, 16, 16, 4), 0.7, 0.9)),
+        layer("parallel", parallel(softmax(2, 2, 16, scale=0.3), delta(2, 2, 16, 16, 2)))])
+    folder = _folder(tmp_path / "m", config, 7)
+    engine = nnis_amd.load_engine(folder, dtype="float32", max_tokens=512)
+    yard, forms, made = Yardstick(P.PlainMafalorn(folder)), [], ops.chunked_scratch
+
+    def watched(*args):
+        scratch = made(*args)
+        forms.append(scratch is not None)
+        return scratch
+
+    monkeypatch.setattr(ops, "chunked_scratch", watched)
+    for turn in ("launched", "captured", "replayed", "replayed"):
+        for lengths, chunks in (((100, 20, 8), True), ((43, 43, 42), False)):
+            forms.clear()
+            prompts = [_ids(n, config["vocab"], n) for n in lengths]
+            slots = [engine.start_sequence() for _ in prompts]
+            rows = engine.step([StepEntry(slot, ids, [len(ids) - 1]) for slot, ids in zip(slots, prompts)]).cpu()
+            for slot in slots:
+                engine.end_sequence(slot)
+            assert forms == {"launched": [chunks] * 2, "captured": [chunks] * 4, "replayed": []}[turn], (lengths, turn)
+            for row, ids in zip(rows, prompts):
+                yard.check(row, ids, "float32", f"{lengths} {turn}", rows=len(ids) - 1)
+    assert len(engine._prefill_graphs.graphs) == 2
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_unequal_batches_equal_each_request_alone(folders, name, dtype):

@@ -86,8 +86,8 @@ def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(d
     from nnis_amd.engine.graph import prompt_rows
     from nnis_amd.kernels import ops
 
-    def scratch(batch, tokens, planned, decode=False, heads=4):
-        ctx = types.SimpleNamespace(decode=decode, batch=batch, planned_rows=planned)
+    def scratch(batch, tokens, planned, decode=False, heads=4, longest=1279):
+        ctx = types.SimpleNamespace(decode=decode, batch=batch, planned_rows=planned, planned_new=longest)
         return ops.chunked_scratch(ctx, tokens, heads, 64, 128, delta, "meta")
 
     for batch, first in least.items():
@@ -95,7 +95,8 @@ def test_a_step_launched_and_replayed_takes_one_form_of_the_matrix_recurrences(d
             if total < batch:
                 continue
             rows = prompt_rows(total)
-            launched, replayed = scratch(batch, total, rows), scratch(batch, rows, rows)
+            longest = -(-rows // batch)
+            launched, replayed = scratch(batch, total, rows, longest=longest), scratch(batch, rows, rows, longest=longest)
             assert (launched is not None) == (replayed is not None) == (rows >= first), (batch, total)
             if launched is not None:
                 assert launched.numel() == ops.recurrent().nnis_chunked_scratch(total, batch, 4, 64, 128, int(delta)) <= replayed.numel()
@@ -117,8 +118,22 @@ def test_the_delta_rule_goes_in_chunks_where_that_is_faster(heads, key_dim, valu
 
     from nnis_amd.kernels import ops
 
-    ctx = types.SimpleNamespace(decode=False, batch=sequences, planned_rows=sequences * tokens)
+    ctx = types.SimpleNamespace(decode=False, batch=sequences, planned_rows=sequences * tokens, planned_new=tokens)
     assert (ops.chunked_scratch(ctx, sequences * tokens, heads, key_dim, value_dim, True, "meta") is not None) == chunks
+
+
+@pytest.mark.parametrize("delta, heads, key_dim, value_dim, lengths, chunks", [
+    (True, 16, 128, 128, [1500] + [100] * 15, True), (True, 16, 128, 128, [1500] + [16] * 15, True),  # 658 / 288, 608 / 225
+    (True, 16, 128, 128, [700] + [30] * 15, True), (True, 8, 64, 128, [700] + [30] * 15, True),  # 305 / 178, 264 / 68
+    (True, 16, 128, 128, [1500] + [16] * 63, False), (True, 16, 64, 64, [135] + [6] * 13, False),  # 635 / 687, 57 / 64
+    (False, 8, 128, 256, [400] + [16] * 15, True), (False, 8, 128, 256, [1500] + [16] * 63, True),  # 136 / 61, 968 / 244
+    (False, 8, 128, 256, [33] + [4] * 15, False), (False, 8, 128, 256, [47] + [10] * 15, False)])  # 38 / 51, 50 / 52
+def test_matrix_recurrences_of_unequal_sequences_go_by_the_longest(delta, heads, key_dim, value_dim, lengths, chunks):
+    """Measured steps, microseconds a token at a time / in chunks: a step lasts as long as its longest sequence's walk."""
+    from nnis_amd.engine.graph import prompt_rows
+    from nnis_amd.kernels import ops
+
+    assert ops.chunks_pay(delta, len(lengths), prompt_rows(sum(lengths)), max(lengths), heads, key_dim, value_dim) == chunks
 
 
 def test_32_bit_attention_of_small_heads():
