@@ -1726,7 +1726,9 @@ def attention_f32_least(head_dim: int, value_dim: int) -> int:
     """Query rows x heads that a step of prompts has to plan for to take ``attention_f32``; below it the row kernel is faster."""
     # Microseconds, rows / matrix cores: 16 channels, 4 heads 64 tokens 5.4 / 7.2, 300 8.1 / 11.5, 1,200 27.3 / 26.2; 9 heads 300 9.4 / 11.4, 600
     # 18.9 / 17.0, 8 prompts of 64 9.9 / 7.3; 32 heads 64 6.4 / 7.3, 150 10.3 / 9.4.  32 channels, 4 heads 150 9.2 / 10.3, 300 11.6 / 12.8, 600 20.5 / 19.4; 9
-    # heads 64 7.2 / 7.7, 300 14.4 / 12.9; 32 heads 64 9.2 / 7.7.  48 channels, 4 heads 64 8.9 / 8.2, 300 15.9 / 14.5.
+    # heads 64 7.2 / 7.7, 300 14.4 / 12.9; 32 heads 64 9.2 / 7.7.  48 channels, 4 heads 64 8.9 / 8.2, 300 15.9 / 14.5.  Behind 4,000 cached keys (with the
+    # launch): 16 channels, 4 heads 64 43 / 74, 600 81 / 83; 32 channels, 9 heads 64 68 / 89, 150 98 / 90; 64 channels, 9/3 heads 16 124 / 124, 32/8 heads 16
+    # 100 / 124 and 64 189 / 126; 128 channels, 9/3 heads 16 414 / 204.
     size = max(head_dim, value_dim)
     return 4096 if size <= 16 else (2048 if size <= 32 else 0)
 
