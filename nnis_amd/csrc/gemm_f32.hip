@@ -1,14 +1,15 @@
 // 32-bit matrix products on the matrix cores: Y[M, N] = X[M, K] * W[N, K]^T for 32-bit weights in the
-// checkpoint's order (K contiguous in both operands), with v_mfma_f32_16x16x4_f32: lane l holds row l % 16 of
+// checkpoint's order (K contiguous in both operands).  For few rows with v_mfma_f32_16x16x4_f32: lane l holds row l % 16 of
 // either operand at k = l / 16, and D[4 * (l / 16) + e][l % 16] of the result, e = 0..3.  Which k a (lane group,
 // instruction) stands for is free as long as both operands agree: lane group g loads 4 consecutive k, 16 bytes,
-// and instruction j of four takes the group's j-th, so that 16 bytes a lane are 16 k of 16 rows.
+// and instruction j of four takes the group's j-th, so that 16 bytes a lane are 16 k of 16 rows.  For tiles with
+// v_mfma_f32_16x16x32_bf16 on operands split into three bfloat16 numbers each, whose sum they are (below).
 //
-// The instruction multiplies and adds in 32 bits; nothing is rounded to fewer on the way.  A sum's terms come in
+// Nothing is rounded to fewer than 32 bits on the way.  A sum's terms come in
 // another order than in the ordered kernel (gemm.hip), in several shorter chains (a wave's share of K, or runs of
 // kFlushSteps steps), so its error against 64 bits is smaller than the one long chain's: 509 x 2048 x 5632 of
-// normal values, root mean square error over that of the result 4.8e-7 (few rows) and 3.0e-7 (tiles) against 1.3e-6,
-// 8 x 960 x 576 1.6e-7 and 2.8e-7 against 4.3e-7.
+// normal values, root mean square error over that of the result 4.8e-7 (few rows) and 2.5e-7 (tiles; 3.0e-7 with the 32-bit
+// instruction, whose chains round 8 times in 32 k instead of 6) against 1.3e-6, 8 x 960 x 576 1.6e-7 and 2.2e-7 against 4.3e-7.
 //
 // What a product does with its sums: stores them, adds them to the residual stream, or, with strips of weight rows that
 // belong together taken in pairs, gates them (silu(gate) * up) or rotates queries and keys and writes the cache
@@ -29,6 +30,7 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 __device__ __forceinline__ f32x4 load4(const float* p) { return *(const f32x4*)p; }
 __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
@@ -342,25 +344,82 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_few_kernel(const XT* __restri
 }
 
 // ---- tiles --------------------------------------------------------------------------------------------------------
-constexpr int kStepK = 32;      // k of a step: 128 bytes of a row, 8 chunks of 16 bytes
+constexpr int kStepK = 32;      // k of a step: 128 bytes of a row
 constexpr int kFlushSteps = 8;  // a chain of sums is this many steps long, then goes into the total
 
-extern __shared__ __align__(16) char f32_lds[];  // NS stages of BM rows of X and BN rows of W
+extern __shared__ __align__(16) char f32_lds[];  // two stages of BM rows of X in three parts
 
-// 4 waves, 2 x 2, each with BM / 2 rows and BN / 2 columns.  A load instruction of a wave brings 8 rows of 128 bytes
-// straight into LDS, lane l's 16 bytes to row l / 8, place l % 8; place p of row r holds chunk p ^ (r % 8), so that
-// the 16 rows which a lane group reads together lie in different banks.  The matrix instructions bound the kernel (a
-// step of a wave tile of 32 x 32 is 32 of them, 1,024 cycles, for 8 KB read from LDS and a quarter of 16 KB loaded).
-template <int BM, int BN, int NS, int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, Fused f, int m, int n,
-                                                             int k, int col_blocks) {
+// A 32-bit number as the sum of three of 8 significant bits: x = hi + mid + lo, exactly, wherever the last of its 24 bits
+// is at least bfloat16's smallest number (x from 2^-110 on; below, it keeps the bits that are).  Both differences are
+// exact.  A number that is none, or that rounds up to infinity, leaves parts that make its product one that is none.
+template <int COUNT>
+struct Split {
+  typedef __attribute__((ext_vector_type(COUNT))) __bf16 part;
+  part hi, mid, lo;
+};
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+__device__ __forceinline__ f32x2 widen(bf16x2 v) {
+  const unsigned both = __builtin_bit_cast(unsigned, v);
+  return (f32x2){__uint_as_float(both << 16), __uint_as_float(both & 0xffff0000u)};
+}
+__device__ __forceinline__ Split<4> split4(f32x4 v) {
+  Split<4> out;
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {  // (two at a time: one conversion for both)
+    const f32x2 x = {v[e], v[e + 1]};
+    const bf16x2 hi = __builtin_convertvector(x, bf16x2);
+    const f32x2 rest = x - widen(hi);
+    const bf16x2 mid = __builtin_convertvector(rest, bf16x2);
+    const bf16x2 lo = __builtin_convertvector(rest - widen(mid), bf16x2);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      out.hi[e + i] = hi[i];
+      out.mid[e + i] = mid[i];
+      out.lo[e + i] = lo[i];
+    }
+  }
+  return out;
+}
+
+// What a sum of parts may not stand for: no number, infinity, and sums so small that their terms' last parts may be
+// missing (a zero stays).  One chain in 32 bits over the operands as they are.
+__device__ __noinline__ float chain_of(const float* x, const float* w, int k) {
+  float sum = 0.0f;
+  for (int i = 0; i < k; ++i) sum = fmaf(x[i], w[i], sum);
+  return sum;
+}
+__device__ __forceinline__ bool parts_hold(float v) {
+  const unsigned magnitude = __float_as_uint(v) & 0x7fffffffu;
+  return magnitude == 0u || (magnitude >= 0x12000000u && magnitude < 0x7f800000u);  // from 2^-91 on
+}
+
+// KG groups of WGM x WGN waves; a wave has BM / WGM rows and BN / WGN columns, a group every KG-th run of 32 k.  On the 16-bit
+// matrix instruction a term x w of a sum is the six products of the operands' parts that are not below 2^-25 of it: x_hi w_hi,
+// x_hi w_mid, x_mid w_hi, x_mid w_mid, x_hi w_lo and x_lo w_hi, six times the work at sixteen times the 32-bit instruction's
+// rate.  The block's threads split each number once, on its way into LDS, where a stage has three planes of 16 rows by 32 k; a
+// lane's 8 k of a step are the 16 bytes at k = 4 g and those at 16 + 4 g, g = l / 16, in both operands, and are read as one
+// operand.  What bounds the kernel is the sum of what a SIMD issues: a step of a wave tile of 64 x 32 is 48 matrix instructions
+// of 16 cycles, about 75 vector instructions (11 for two numbers split) and 26 of LDS, 2,600 cycles for two waves of the 3,050
+// measured; neither half the conversions, loads that hit nearer, operands read a step ahead nor two groups that take turns
+// (products of one beside reads of the other) changed it by more than 5%.  Where a block has a compute unit to itself two groups
+// share K, so that a SIMD has two waves: 509 x 2048 x 5632 in 64 x 64 114 -> 90 us (106 with the 32-bit instruction);
+// with several blocks a unit one group is as fast and meets less.  2000 x 11264 x 2048 in 128 x 128: 501 us, 184 TFLOP/s (the
+// 32-bit instruction's peak is 157, its kernel reached 128); 509 x 11264 x 2048 196 -> 150; 509 x 2560 x 2048 57 -> 41.
+template <int BM, int BN, int WGM, int WGN, int KG, int EPI>
+__global__ __launch_bounds__(64 * WGM * WGN * KG, 2) void gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, Fused f, int m, int n,
+                                                                int k, int col_blocks) {
   constexpr bool kPaired = EPI == F32_SILU || EPI == F32_ROPE;
-  static_assert(!kPaired || BN % 64 == 0, "a wave has whole pairs of strips");
-  constexpr int TM = BM / 32, TN = BN / 32;  // tiles of 16 x 16 a wave has, each way
-  constexpr int A_LOADS = BM / 32, B_LOADS = BN / 32, LOADS = A_LOADS + B_LOADS;  // load instructions a wave and step
-  constexpr int A_BYTES = BM * kStepK * 4, STAGE_BYTES = (BM + BN) * kStepK * 4;
+  constexpr int THREADS = 64 * WGM * WGN * KG, WM = BM / WGM, WN = BN / WGN;
+  static_assert(!kPaired || WN % 32 == 0, "a wave has whole pairs of strips");
+  constexpr int TM = WM / 16, TN = WN / 16;  // tiles of 16 x 16 a wave has, each way
+  constexpr int ROW_CHUNKS = 8 * KG, BLOCK_K = kStepK * KG;  // a step of the block
+  constexpr int LOAD_ROWS = THREADS / ROW_CHUNKS;  // rows that one load of every thread brings
+  constexpr int A_LOADS = (BM + LOAD_ROWS - 1) / LOAD_ROWS, B_LOADS = (BN + LOAD_ROWS - 1) / LOAD_ROWS;
+  constexpr int PLANE = 512, TILE = 3 * PLANE;  // 16 rows of a part and of all parts, in elements
+  constexpr int GROUP = (BM + BN) / 16 * TILE, STAGE = KG * GROUP;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-  const int wave_m = wave / 2, wave_n = wave % 2;
+  const int k_group = wave / (WGM * WGN), wave_m = wave / WGN % WGM, wave_n = wave % WGN;
   const int r = lane % 16, g = lane / 16;
   // blocks go to the 8 dies in turn: a die's blocks are consecutive tiles, rows fastest, so that its L2 holds a few
   // column blocks of W and the rows of X
@@ -374,42 +433,75 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
     col_block = tile / row_blocks;
   }
   const int row0 = row_block * BM, col0 = col_block * BN;
+  // the weight row at place `place` of the block's BN (pairs: strips 2 u and 2 u + 1 of 16 are unit u's); -1 or from n on: none
+  auto weight_row = [&](int place) {
+    if constexpr (kPaired) return paired_row<EPI, 16>(f, col_block * (BN / 32) + place / 32, place / 16 % 2, place % 16, n);
+    else return col0 + place;
+  };
 
-  const int chunk_k = ((lane % 8) ^ (lane / 8)) * 4;  // the first k of this lane's chunk of a step
-  // rows in bytes from the tile's first row, and from the first of the wave's weight rows (of its pairs' lower or upper rows:
-  // a wave's loads take the one or all the other), which are the same in every lane
-  const float* a_base = x + (size_t)row0 * k;
-  const float* b_base = w;
-  int a_off[A_LOADS], b_off[B_LOADS], base_row = 0;
+  // Rows beyond the end: a valid one, not stored.  Loads go by a base that is the same in every lane (the tile's first row; the
+  // first of the 8 weight rows of a wave's load, which follow one another) and an offset in bytes, and give zeros from the base's
+  // limit on: that is where the last step's chunks beyond K are asked for, and the limit is the operand's end, which steps
+  // beyond the last reach (what they bring is not multiplied).
+  constexpr unsigned kNowhere = 0xfffffff0u;
+  auto limit_of = [](size_t elements) { return elements * 4 < kNowhere ? (unsigned)(elements * 4) : kNowhere; };
+  const int steps = (k + BLOCK_K - 1) / BLOCK_K, full = k / BLOCK_K;
+  const auto a_base = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (size_t)row0 * k), 0, limit_of((size_t)(m - row0) * k), 0x00027000);
+  const int load_row = threadIdx.x / ROW_CHUNKS, chunk = threadIdx.x % ROW_CHUNKS, group = chunk % 4;
+  // chunk c (of 8) is half c / 4 of the 8 k of lane group c % 4; 16 rows' chunks of a group lie together, row ^ 2 group, so that the
+  // two rows that 16 lanes write, and the 8 rows that 8 lanes read, lie in different banks
+  const int place_in_tile = chunk / 8 * GROUP + group * 128 + chunk / 4 % 2 * 4;
+  auto place_of_row = [&](int row) { return row / 16 * TILE + place_in_tile + (row % 16 ^ group * 2) * 8; };
+  unsigned a_from[A_LOADS], b_from[B_LOADS];
+  __amdgpu_buffer_rsrc_t b_base[B_LOADS];
 #pragma unroll
   for (int o = 0; o < A_LOADS; ++o) {
-    const int row = (o * 4 + wave) * 8 + lane / 8;
-    a_off[o] = (row0 + row < m ? row : m - 1 - row0) * k * 4;
+    const int row = row0 + o * LOAD_ROWS + load_row;
+    a_from[o] = (unsigned)(((row < m ? row : m - 1) - row0) * k + chunk * 4) * 4u;
   }
 #pragma unroll
   for (int o = 0; o < B_LOADS; ++o) {
-    const int in_tile = (o * 4 + wave) * 8 + lane / 8;  // (pairs: strips 2 u and 2 u + 1 of the tile are unit u's)
-    int row;
-    if constexpr (kPaired) row = paired_row<EPI, 16>(f, col_block * (BN / 32) + in_tile / 32, in_tile / 16 % 2, in_tile % 16, n);
-    else row = col0 + in_tile;
-    if (o == 0) {
-      const int first = __builtin_amdgcn_readfirstlane(row);
-      base_row = first >= 0 && first < n ? first : n - 1;
-      b_base = w + (size_t)base_row * k;
-    }
-    b_off[o] = (row >= 0 && row < n ? row - base_row : 0) * k * 4;  // (rows beyond the end: a valid one, not stored)
+    const int row = weight_row(o * LOAD_ROWS + load_row), first = __builtin_amdgcn_readfirstlane(row);
+    const int start = first >= 0 && first < n ? first : 0;
+    b_base[o] = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)start * k), 0, limit_of((size_t)(n - start) * k), 0x00027000);
+    b_from[o] = (unsigned)((row >= 0 && row < n ? row - start : 0) * k + chunk * 4) * 4u;
   }
-  // Step s lies in stage s % NS.  A step beyond the end, and the last step's chunks beyond K, are asked for from the
-  // row's first chunk: valid memory; the former nobody reads, the latter count as zeros.
-  const int steps = (k + kStepK - 1) / kStepK;
-  auto ask = [&](int step, int stage) {
-    char* base = f32_lds + stage * STAGE_BYTES + wave * 1024;
-    const int at = step * kStepK + chunk_k;
-    const int from = (at < k ? at : 0) * 4;
+  __bf16* stages = (__bf16*)f32_lds;
+
+  // (the step's place in the vector offset: the check against the limit takes no other into account for certain)
+  const bool there = full * BLOCK_K + chunk * 4 < k;  // in a last, short step
+  auto load = [&](__amdgpu_buffer_rsrc_t base, unsigned from, int step) {
+    const unsigned at = step != full || there ? from + (unsigned)step * (BLOCK_K * 4) : kNowhere;
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(base, (int)at, 0, 0));
+  };
+  auto in_tile = [&](int o, int rows) { return rows % LOAD_ROWS == 0 || o * LOAD_ROWS + load_row < rows; };
+  struct Raw {
+    f32x4 a[A_LOADS], b[B_LOADS];
+  };
+  auto ask = [&](Raw& v, int step) {
 #pragma unroll
-    for (int o = 0; o < A_LOADS; ++o) load_to_lds(a_base, a_off[o] + from, 0, base + o * 4096);
+    for (int o = 0; o < A_LOADS; ++o)
+      if (in_tile(o, BM)) v.a[o] = load(a_base, a_from[o], step);
 #pragma unroll
-    for (int o = 0; o < B_LOADS; ++o) load_to_lds(b_base, b_off[o] + from, 0, base + A_BYTES + o * 4096);
+    for (int o = 0; o < B_LOADS; ++o)
+      if (in_tile(o, BN)) v.b[o] = load(b_base[o], b_from[o], step);
+  };
+  auto put = [&](f32x4 v, __bf16* to) {
+    // (two groups: a step's numbers are not to be waited for, and split, together with the step's before it: 41 -> 37 us; one: 4% slower)
+    if constexpr (KG > 1) asm volatile("" : "+v"(v));
+    const Split<4> parts = split4(v);
+    *(bf16x4*)to = parts.hi;
+    *(bf16x4*)(to + PLANE) = parts.mid;
+    *(bf16x4*)(to + 2 * PLANE) = parts.lo;
+  };
+  auto stage_step = [&](const Raw& v, int stage) {
+    __bf16* to = stages + stage * STAGE;
+#pragma unroll
+    for (int o = 0; o < A_LOADS; ++o)
+      if (in_tile(o, BM)) put(v.a[o], to + place_of_row(o * LOAD_ROWS + load_row));
+#pragma unroll
+    for (int o = 0; o < B_LOADS; ++o)
+      if (in_tile(o, BN)) put(v.b[o], to + BM / 16 * TILE + place_of_row(o * LOAD_ROWS + load_row));
   };
 
   f32x4 sum[TM][TN], total[TM][TN];
@@ -418,51 +510,57 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) sum[i][j] = total[i][j] = zero;
-
-  auto read_half = [&](int from, int half, f32x4 (&a)[TM], f32x4 (&b)[TN]) {
-    const f32x4* a_tile = (const f32x4*)(f32_lds + from * STAGE_BYTES);
-    const f32x4* b_tile = (const f32x4*)(f32_lds + from * STAGE_BYTES + A_BYTES);
-    const int place = (half * 4 + g) ^ (r % 8);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) a[i] = a_tile[(wave_m * (BM / 2) + i * 16 + r) * 8 + place];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b[j] = b_tile[(wave_n * (BN / 2) + j * 16 + r) * 8 + place];
+  auto product = [](bf16x8 b, bf16x8 a, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, c, 0, 0, 0); };
+  auto read_part = [&](Split<8>& v, const __bf16* tile) {
+    const __bf16* at = tile + g * 128 + (r ^ g * 2) * 8;
+    v.hi = *(const bf16x8*)at;
+    v.mid = *(const bf16x8*)(at + PLANE);
+    v.lo = *(const bf16x8*)(at + 2 * PLANE);
   };
-  auto multiply = [&](const f32x4 (&a)[TM], const f32x4 (&b)[TN]) {
+  auto meet = [] {  // every wave's reads and writes of LDS so far are done
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  struct Operands {
+    Split<8> rows[TM], weights[TN];
+  };
+  auto read_step = [&](Operands& v, int stage) {
+    const __bf16* from = stages + stage * STAGE + k_group * GROUP;
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int j = 0; j < TN; ++j) read_part(v.weights[j], from + BM / 16 * TILE + (wave_n * TN + j) * TILE);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) read_part(v.rows[i], from + (wave_m * TM + i) * TILE);
+  };
+  auto multiply = [&](const Operands& v) {
+#pragma unroll
+    for (int term = 0; term < 6; ++term)  // the small ones first
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][q], a[i][q], sum[i][j], 0, 0, 0);
+        for (int j = 0; j < TN; ++j) {
+          const bf16x8 of_w = term == 1 ? v.weights[j].lo : (term == 2 || term == 4 ? v.weights[j].mid : v.weights[j].hi);
+          const bf16x8 of_x = term == 0 ? v.rows[i].lo : (term == 2 || term == 3 ? v.rows[i].mid : v.rows[i].hi);
+          sum[i][j] = product(of_w, of_x, sum[i][j]);
+        }
   };
 
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s) ask(s, s);
-  wait_loads_but<(NS - 2) * LOADS>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  int stage = 0;
-  f32x4 a0[TM], b0[TN], a1[TM], b1[TN];
-  // A step asks for the step NS - 1 ahead into the stage that was read a step ago, reads its second half under the
-  // first half's products, and multiplies the second half behind the barrier, while the next step's first half is read.
-  // Every read of a stage is waited for before the barrier that lets the stage be filled again.
-  read_half(0, 0, a0, b0);
-  const int full = k % kStepK == 0 ? steps : steps - 1;  // steps without chunks beyond K
+  // Step s lies in stage s % 2.  It is asked for three steps ahead, split and put there one ahead.  A stage is filled again
+  // behind the barrier behind its last reads.
+  Raw raw[2];
+  ask(raw[0], 0);
+  ask(raw[1], 1);
+  stage_step(raw[0], 0);
+  ask(raw[0], 2);
+  meet();
   int run = 0;
-  for (int step = 0; step < full; ++step) {
-    ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
-    read_half(stage, 1, a1, b1);
-    multiply(a0, b0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wait_loads_but<(NS - 2) * LOADS>();
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("" ::: "memory");
-    stage = stage + 1 == NS ? 0 : stage + 1;
-    read_half(stage, 0, a0, b0);  // (behind the last step: of a stage that nobody multiplies)
-    multiply(a1, b1);
+  auto one_step = [&](int step, Raw& next, int stage) {
+    Operands here;
+    read_step(here, stage);
+    multiply(here);
+    stage_step(next, 1 - stage);
+    ask(next, step + 3);
     if (++run == kFlushSteps) {
       run = 0;
 #pragma unroll
@@ -473,41 +571,58 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
           sum[i][j] = zero;
         }
     }
+    meet();
+  };
+  int step = 0;
+  for (; step + 1 < steps; step += 2) {
+    one_step(step, raw[1], 0);
+    one_step(step + 1, raw[0], 1);
   }
-  if (full < steps) {  // the last step: its chunks beyond K count as zeros
-    const int k0 = full * kStepK + g * 4;
-    read_half(stage, 1, a1, b1);
+  if (step < steps) one_step(step, raw[1], 0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      a0[i] = k0 < k ? a0[i] : zero;
-      a1[i] = k0 + 16 < k ? a1[i] : zero;
-    }
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      b0[j] = k0 < k ? b0[j] : zero;
-      b1[j] = k0 + 16 < k ? b1[j] : zero;
-    }
-    multiply(a0, b0);
-    multiply(a1, b1);
+    for (int j = 0; j < TN; ++j) total[i][j] += sum[i][j];
+  if constexpr (KG > 1) {  // the groups' sums meet in LDS (all reads of the stages are behind the last barrier)
+    f32x4* sums = (f32x4*)f32_lds + (size_t)(wave % (WGM * WGN)) * TM * TN * kWave + lane;
+    if (k_group != 0)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sums[(i * TN + j) * kWave] = total[i][j];
+    meet();
+    if (k_group != 0) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) total[i][j] += sums[(i * TN + j) * kWave];
   }
-  wait_loads_but<0>();  // the steps asked for beyond the end: nothing of this block is in flight when it ends
 
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int row = row0 + wave_m * (BM / 2) + i * 16 + r;
+    const int row = row0 + wave_m * WM + i * 16 + r;
     if (row >= m) continue;
+    auto finished = [&](int j) {
+      f32x4 v = total[i][j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!parts_hold(v[e])) {
+          const int of = weight_row(wave_n * WN + j * 16 + g * 4 + e);
+          if (of >= 0 && of < n) v[e] = chain_of(x + (size_t)row * k, w + (size_t)of * k, k);
+        }
+      return v;
+    };
     if constexpr (kPaired) {
       TokenPlace place = {0, -1};
       if constexpr (EPI == F32_ROPE) place = place_of(f, row);
 #pragma unroll
       for (int u = 0; u < TN / 2; ++u)
-        finish_pair<EPI, 16>(f, row, place, col_block * (BN / 32) + wave_n * (TN / 2) + u, g * 4, n, total[i][2 * u] + sum[i][2 * u],
-                             total[i][2 * u + 1] + sum[i][2 * u + 1]);
+        finish_pair<EPI, 16>(f, row, place, (col0 + wave_n * WN) / 32 + u, g * 4, n, finished(2 * u), finished(2 * u + 1));
     } else {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int column = col0 + wave_n * (BN / 2) + j * 16 + g * 4;
-        f32x4 v = total[i][j] + sum[i][j];
+        const int column = col0 + wave_n * WN + j * 16 + g * 4;
+        f32x4 v = finished(j);
         if constexpr (EPI == F32_RESIDUAL) v += ask_columns((const float*)f.y, row, column, n);
         store_columns(f.y, EPI == F32_RESIDUAL ? (int)NNIS_F32 : f.y_dtype, row, column, n, v);
       }
@@ -522,17 +637,17 @@ void launch_few(const XT* x, const float* w, const Fused& f, int m, int n, int k
   hipLaunchKernelGGL((gemm_f32_few_kernel<XT, S, NT, W, U, HALF, NORM, EPI>), grid, dim3(64 * W), 0, stream, x, w, f, m, n, k);
 }
 
-template <int EPI, int BM, int BN, int NS>
+template <int EPI, int BM, int BN, int WGM, int WGN, int KG>
 int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, int k, hipStream_t stream) {
-  constexpr int lds = NS * (BM + BN) * kStepK * 4;
-  static_assert(lds <= 160 * 1024, "a compute unit has 160 KB");
-  auto kernel = gemm_f32_tiled_kernel<BM, BN, NS, EPI>;
+  constexpr int lds = 2 * KG * (BM + BN) * kStepK * 3 * (int)sizeof(__bf16);
+  static_assert(lds <= 160 * 1024 && lds >= BM * BN * 4, "a compute unit has 160 KB; the groups' sums fit");
+  auto kernel = gemm_f32_tiled_kernel<BM, BN, WGM, WGN, KG, EPI>;
   NNIS_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess,
                "gemm_f32: %d bytes of LDS were refused", lds);
   const int col_blocks = (n + BN - 1) / BN;
   const long long blocks = (long long)col_blocks * ((m + BM - 1) / BM);
   NNIS_REQUIRE(blocks < (1LL << 31), "gemm_f32: %d rows exceed the grid limit", m);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, stream, x, w, f, m, n, k, col_blocks);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64 * WGM * WGN * KG), lds, stream, x, w, f, m, n, k, col_blocks);
   return 0;
 }
 
@@ -545,16 +660,17 @@ int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, i
 // 1.51 -> 1.12 ms with the norms, gates, rotations and sums in the products), then two strips up to 8192 rows of weight (16
 // rows of 6144 x 2048 19.3 against 20.6).  Beyond 16 rows a variant's time is close to a start and, for every
 // round of its blocks on 256 compute units, a slope times K: the least of these is taken.  Measured:
-// 64 x 2048 x 2048 14.0 us (two strips, one tile a block), 128 x 2048 x 2048 18.7 (2 x 2), 128 x 11264 x 2048 60 (tiles of 64 x 96; 75
-// in 64 x 64), 509 x 2048 x 5632 112 (64 x 64), 4000 x 11264 x 2048 1,443 (128 x 128; 128 TFLOP/s of the instruction's 157).
+// 64 x 2048 x 2048 13.4 us (two strips, one tile a block), 100 x 2048 x 2048 18.1 (2 x 2; 23.9 in tiles of 32 x 64), 100 x 11264 x 2048
+// 45.6 (tiles of 64 x 96; 52.7 in 128 x 64), 509 x 2048 x 5632 90 (64 x 64; 103 in 32 x 64), 2000 x 11264 x 2048 501 (128 x 128; 558 in 64 x 128).
+// Over 8 weights from 576 x 576 to 11264 x 2048 at 20 to 2,000 rows the form taken is 0.4% slower than the best on average.
 struct Variant {
   int rows, columns;  // of a block
   float slope, start; // microseconds: slope * K for each round of blocks, and start
 };
 constexpr Variant kVariants[] = {
     {16, 16, 0.0050f, 2.0f}, {16, 32, 0.0064f, 2.0f}, {32, 32, 0.0083f, 2.0f}, {64, 32, 0.0135f, 2.0f},
-    {32, 64, 0.0105f, 3.5f}, {64, 64, 0.0189f, 3.5f}, {64, 96, 0.0280f, 3.5f}, {96, 64, 0.0280f, 3.5f}, {96, 96, 0.0405f, 3.5f},
-    {64, 128, 0.0365f, 3.5f}, {128, 64, 0.0365f, 3.5f}, {128, 96, 0.0540f, 3.5f}, {128, 128, 0.0700f, 3.5f}};
+    {32, 64, 0.0095f, 4.0f}, {64, 64, 0.0145f, 4.5f}, {64, 96, 0.0185f, 4.5f}, {96, 64, 0.0190f, 4.5f}, {96, 96, 0.0285f, 3.5f},
+    {64, 128, 0.0235f, 4.5f}, {128, 64, 0.0209f, 5.8f}, {128, 96, 0.0315f, 4.8f}, {128, 128, 0.0364f, 6.9f}};
 constexpr int kFewVariants = 4, kCountVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 enum : int { kHalfStrips = kCountVariants, kFourWaves, kTwoStrips, kHints };
 
@@ -587,7 +703,7 @@ template <int EPI, bool NORM, typename XT>
 int run_variant(int variant, const XT* x, const float* w, const Fused& f, int m, int n, int k, hipStream_t s) {
   constexpr bool kPaired = EPI == F32_SILU || EPI == F32_ROPE;
   constexpr int S = kPaired ? 2 : 1;
-  // (strips, tiles, waves, chunks in flight); (rows, columns, stages)
+  // (strips, tiles, waves, chunks in flight); (rows, columns, waves along either, groups)
   switch (variant) {
     case kHalfStrips: launch_few<EPI, NORM, XT, S, 1, 8, 4, true>(x, w, f, m, n, k, s); return 0;
     case kFourWaves: launch_few<EPI, NORM, XT, S, 1, 4, 8>(x, w, f, m, n, k, s); return 0;
@@ -611,18 +727,18 @@ int run_variant(int variant, const XT* x, const float* w, const Fused& f, int m,
     }
     if constexpr (std::is_same<XT, float>::value) {
       switch (variant) {
-        case 4: return launch_tiled<EPI, 32, 64, 3>(x, w, f, m, n, k, s);
-        case 5: return launch_tiled<EPI, 64, 64, 3>(x, w, f, m, n, k, s);
-        case 7: return launch_tiled<EPI, 96, 64, 3>(x, w, f, m, n, k, s);
-        case 9: return launch_tiled<EPI, 64, 128, 3>(x, w, f, m, n, k, s);
-        case 10: return launch_tiled<EPI, 128, 64, 3>(x, w, f, m, n, k, s);
-        case 12: return launch_tiled<EPI, 128, 128, 2>(x, w, f, m, n, k, s);
+        case 4: return launch_tiled<EPI, 32, 64, 2, 2, 2>(x, w, f, m, n, k, s);
+        case 5: return launch_tiled<EPI, 64, 64, 2, 2, 2>(x, w, f, m, n, k, s);
+        case 7: return launch_tiled<EPI, 96, 64, 2, 2, 2>(x, w, f, m, n, k, s);
+        case 9: return launch_tiled<EPI, 64, 128, 1, 4, 1>(x, w, f, m, n, k, s);
+        case 10: return launch_tiled<EPI, 128, 64, 2, 2, 2>(x, w, f, m, n, k, s);
+        case 12: return launch_tiled<EPI, 128, 128, 2, 4, 1>(x, w, f, m, n, k, s);
       }
       if constexpr (!kPaired) {
         switch (variant) {
-          case 6: return launch_tiled<EPI, 64, 96, 3>(x, w, f, m, n, k, s);
-          case 8: return launch_tiled<EPI, 96, 96, 3>(x, w, f, m, n, k, s);
-          case 11: return launch_tiled<EPI, 128, 96, 3>(x, w, f, m, n, k, s);
+          case 6: return launch_tiled<EPI, 64, 96, 2, 2, 2>(x, w, f, m, n, k, s);
+          case 8: return launch_tiled<EPI, 96, 96, 3, 2, 1>(x, w, f, m, n, k, s);
+          case 11: return launch_tiled<EPI, 128, 96, 4, 2, 1>(x, w, f, m, n, k, s);
         }
       }
     }

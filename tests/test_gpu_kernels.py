@@ -109,6 +109,46 @@ def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
         assert ((y.cpu().double() - x.double() @ w.double().t()).abs() <= tol * (x.double().abs() @ w.double().abs().t())).all()
 
 
+@pytest.mark.parametrize("variant", range(4, 13))
+@pytest.mark.parametrize("k", [36, 100, 612])
+def test_gemm_f32_tiles_split_any_number(k, variant):
+    """The tiles multiply the bfloat16 parts that a 32-bit number is the sum of.  Rows of every magnitude come out as
+    accurate as ordinary ones: the bound as above, the smallest 32-bit number for each product that falls below it, and
+    what a last part below bfloat16's smallest number, 2^-133, may lack, half of that times the other operand (which
+    only a far larger other operand lets anyone see; small sums are taken again).  Numbers that are none and sums beyond the largest number come out where the 32-bit chain has them, in their rows and
+    columns alone."""
+    ops = _ops()
+    torch.manual_seed(k)
+    m, n = 70, 65
+    x, w = torch.randn(m, k), torch.randn(n, k)
+    x[1] *= 1e-36  # (their last parts are below bfloat16's smallest number)
+    x[2] *= 1e-25
+    x[3] *= 1e30
+    x[4] = torch.where(x[4] > 0, 3.4e38, -3.4e38) * (torch.arange(k) == k - 1)  # rounds up to infinity in bfloat16
+    x[5] = 0.0
+    w[3] *= 1e-20
+    w[4] *= torch.logspace(-18, 18, k)
+    want, scale = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    y = torch.empty(m, n, device="cuda")
+    ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
+    got = y.cpu().double()
+    scale = 2e-7 * math.sqrt(k) * scale + 1.5e-45 * k + 2.0 ** -134 * (x.double().abs().sum(1)[:, None] + w.double().abs().sum(1))
+    fits = scale < 3.4e38 * 2e-7  # (a sum of terms beyond it may be infinite, or cancel, in one order and not in another)
+    bad = ((got - want).abs() > scale) & fits
+    assert not bad.any() and (got[5] == 0).all(), (bad.nonzero()[:8], (got - want)[bad][:8], scale[bad][:8], want[bad][:8])
+    x[6, k - 1], x[7, 3], w[9, 0] = float("inf"), float("nan"), float("-inf")
+    ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
+    now, chain = y.cpu(), torch.empty(m, n, device="cuda")
+    ops.gemm_ordered(x.cuda(), w.cuda(), chain)
+    for row in (6, 7):
+        assert torch.equal(now[row].isnan(), chain[row].cpu().isnan()) and torch.equal(now[row].isinf(), chain[row].cpu().isinf())
+        assert torch.equal(now[row].sign()[now[row].isinf()], chain[row].cpu().sign()[now[row].isinf()])
+    assert torch.equal(now[:, 9].nan_to_num(), chain[:, 9].cpu().nan_to_num()) or not now[:, 9].isfinite().any()
+    rest = [r for r in range(m) if r not in (6, 7)]
+    columns = [c for c in range(n) if c != 9]
+    assert torch.equal(now[rest][:, columns], got.float()[rest][:, columns])
+
+
 def _f32_forms(rows, normed):
     """The forms that take a product of so many 32-bit rows, with the norm before it or without."""
     few = (-1, 0, 1, 13, 14, 15)  # (13: half strips, up to 8 rows)
