@@ -1463,3 +1463,24 @@ def test_the_tile_whose_weights_go_into_registers(epilogue, m, k):
         ops.gemm_scaled(x, ss, 1, 1e-5, weight, y, code, rope, 16 * tile)
         rows.append(y)
     assert torch.equal(*rows)
+
+
+@pytest.mark.parametrize("lengths", [[1, 1, 1], [5, 1, 9], [150, 1, 70]])
+@pytest.mark.parametrize("channels, states", [(70, 4), (300, 16), (33, 20), (40, 6), (40, 128)])
+def test_selective_scan_states_off_16_byte_boundaries(channels, states, lengths):
+    """States and rates that lie where 16 bytes can be loaded at a time, and the same ones 4 bytes further on: equal results,
+    with single tokens, whole runs and runs in pieces."""
+    ops = _ops()
+    torch.manual_seed(channels + states)
+    tokens, slots = sum(lengths), len(lengths) + 1
+    x, z, dt, bc = torch.randn(tokens, channels).cuda(), torch.randn(tokens, channels).cuda(), torch.randn(tokens, channels).cuda(), torch.randn(tokens, 2 * states).cuda()
+    rates, D, bias, state = -torch.rand(channels, states).cuda(), torch.randn(channels).cuda(), torch.randn(channels).cuda(), torch.randn(slots, channels, states).cuda()
+    results = []
+    for shift in (0, 1):
+        held, A = (torch.cat([t.new_zeros(shift), t.flatten()])[shift:].view(t.shape) for t in (state, rates))
+        assert held.data_ptr() % 16 == 4 * shift
+        out = torch.empty(tokens, channels, device="cuda")
+        ops.selective_scan(x, dt, bc, z, A, D, bias, held, _prompts(lengths), out)
+        results.append((out, held))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert torch.equal(results[0][1][-1], state[-1]) and not torch.equal(results[0][1][0], state[0])
