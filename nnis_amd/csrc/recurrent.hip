@@ -658,6 +658,71 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(GlaArgs a) {
   }
 }
 
+// A step of single tokens.  Nothing of the state serves a second token, so the kernel is the state's way through: a block
+// takes LANES x 4 value columns of one head of one sequence, a thread 4 neighbouring columns (16 bytes) of every
+// (256 / LANES)-th key row, LANES threads a row's consecutive memory.  (The scan above has 8 lanes of 4 bytes on a row for heads of
+// 128 x 256, and walks its tokens' loop for one.)  The rows' parts of o are added by lane exchanges and through LDS.
+// One sequence, 8 heads of 128 x 256: STEP1
+template <int ROWS, int LANES>
+__global__ __launch_bounds__(256) void gla_step_kernel(GlaArgs a) {
+  constexpr int kRowsApart = 256 / LANES;  // ROWS of them a thread: key channels up to ROWS * kRowsApart
+  __shared__ float qs[ROWS * kRowsApart], ks[ROWS * kRowsApart], as[ROWS * kRowsApart];
+  __shared__ float4 parts[4][LANES];
+  const int b = blockIdx.z, head = blockIdx.y;
+  const int slot = a.seq_slot[b];
+  if (slot < 0) return;
+  const int t = a.seq_start[b];
+  const int d = a.key_dim, e = a.value_dim;
+  const int lane = threadIdx.x % LANES, row0 = threadIdx.x / LANES;
+  const int col = (blockIdx.x * LANES + lane) * 4;
+  const bool live = col < e;  // (e is a multiple of 4)
+  float* state = a.state + ((size_t)slot * a.heads + head) * d * e + (live ? col : 0);
+  float4 S[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int row = row0 + i * kRowsApart;
+    S[i] = *(const float4*)(state + (size_t)(row < d ? row : 0) * e);
+  }
+  float v[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = load_as_f32(a.v, a.qkv_dtype, (size_t)t * a.v_stride + head * e + (live ? col : 0) + c);
+  for (int ch = threadIdx.x; ch < d; ch += 256) {
+    qs[ch] = gla_turned(a, a.q, a.q_stride, t, head, ch) * a.scale;
+    ks[ch] = gla_turned(a, a.k, a.k_stride, t, head, ch);
+    as[ch] = a.zd ? exp2_fast(a.zd[((size_t)t * a.heads + head) * d + ch] * kLog2e) : a.head_decay[head];
+  }
+  __syncthreads();
+  float o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int row = row0 + i * kRowsApart;
+    if (row >= d) break;
+    const float decay = as[row], k = ks[row], q = qs[row];
+    float* s = (float*)&S[i];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      s[c] = fmaf(decay, s[c], k * v[c]);
+      o[c] = fmaf(s[c], q, o[c]);
+    }
+    if (live) *(float4*)(state + (size_t)row * e) = S[i];
+  }
+#pragma unroll
+  for (int offset = LANES; offset < kWave; offset *= 2)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] += __shfl_xor(o[c], offset, kWave);
+  if (threadIdx.x % kWave < LANES) parts[threadIdx.x / kWave][lane] = make_float4(o[0], o[1], o[2], o[3]);
+  __syncthreads();
+  if (threadIdx.x < LANES && live) {
+    float4 sum = parts[0][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      const float4 more = parts[w][lane];
+      sum.x += more.x; sum.y += more.y; sum.z += more.z; sum.w += more.w;
+    }
+    *(float4*)(a.out + ((size_t)t * a.heads + head) * e + col) = sum;
+  }
+}
+
 // between the passes: a thread an element of a sequence's state walks the pieces, I_(k+1) = P_k I_k + E_k with P_k the
 // product of piece k's decays of the element's key channel, and leaves I_k in E_k's place
 __global__ void gla_carry_kernel(GlaArgs a) {
@@ -799,12 +864,13 @@ extern "C" int nnis_selective_scan(const void* x, int x_dtype, const float* dt_p
 // piece, pieces: as nnis_selective_scan's (`carried`: batch * pieces * heads * key_dim * value_dim floats, `decayed`:
 // batch * pieces * heads * key_dim)
 // Without `zd`: `head_decay` [2, heads], one fixed decay a head and its logarithm.  rot_dim > 0: q's and k's first
-// rot_dim channels of a head are turned by tok_pos[row] while staged (tables [rot_positions, rot_dim / 2]).
+// rot_dim channels of a head are turned by tok_pos[row] while staged (tables [rot_positions, rot_dim / 2]).  `single`: every
+// sequence brings one token.
 extern "C" int nnis_gla_scan_turned(const void* q, const void* k, const void* v, int qkv_dtype, int q_stride, int k_stride, int v_stride,
                                     const float* zd, const float* head_decay, const float* rot_cos, const float* rot_sin,
                                     int rot_dim, int rot_positions, const int* tok_pos, float scale, float* state,
                                     const int* seq_slot, const int* seq_start, int batch, int heads, int key_dim, int value_dim,
-                                    float* out, int piece, int pieces, float* carried, float* decayed, void* stream);
+                                    float* out, int piece, int pieces, float* carried, float* decayed, int single, void* stream);
 
 extern "C" int nnis_gla_scan(const void* q, const void* k, const void* v, int qkv_dtype, int q_stride, int k_stride, int v_stride,
                              const float* zd, float scale, float* state, const int* seq_slot, const int* seq_start,
@@ -812,14 +878,14 @@ extern "C" int nnis_gla_scan(const void* q, const void* k, const void* v, int qk
                              float* decayed, void* stream) {
   NNIS_REQUIRE(zd, "gla_scan: the decays' logarithms are missing");
   return nnis_gla_scan_turned(q, k, v, qkv_dtype, q_stride, k_stride, v_stride, zd, nullptr, nullptr, nullptr, 0, 0, nullptr, scale,
-                              state, seq_slot, seq_start, batch, heads, key_dim, value_dim, out, piece, pieces, carried, decayed, stream);
+                              state, seq_slot, seq_start, batch, heads, key_dim, value_dim, out, piece, pieces, carried, decayed, 0, stream);
 }
 
 extern "C" int nnis_gla_scan_turned(const void* q, const void* k, const void* v, int qkv_dtype, int q_stride, int k_stride, int v_stride,
                                     const float* zd, const float* head_decay, const float* rot_cos, const float* rot_sin,
                                     int rot_dim, int rot_positions, const int* tok_pos, float scale, float* state,
                                     const int* seq_slot, const int* seq_start, int batch, int heads, int key_dim, int value_dim,
-                                    float* out, int piece, int pieces, float* carried, float* decayed, void* stream) {
+                                    float* out, int piece, int pieces, float* carried, float* decayed, int single, void* stream) {
   NNIS_REQUIRE(nnis_dtype_ok(qkv_dtype), "gla_scan: unknown dtype %d", qkv_dtype);
   NNIS_REQUIRE((zd != nullptr) != (head_decay != nullptr), "gla_scan: decays a token and channel, or one a head");
   NNIS_REQUIRE(rot_dim >= 0 && rot_dim % 2 == 0 && rot_dim <= key_dim, "gla_scan: %d turned channels in heads of %d", rot_dim, key_dim);
@@ -836,6 +902,23 @@ extern "C" int nnis_gla_scan_turned(const void* q, const void* k, const void* v,
   a.scale = scale; a.state = state; a.seq_slot = seq_slot; a.seq_start = seq_start; a.heads = heads;
   a.key_dim = key_dim; a.value_dim = value_dim; a.out = out; a.piece = piece; a.pieces = pieces; a.carried = carried; a.decayed = decayed;
   a.head_decay = head_decay; a.rot_cos = rot_cos; a.rot_sin = rot_sin; a.tok_pos = tok_pos; a.rot_dim = rot_dim; a.rot_positions = rot_positions;
+  if (single && value_dim % 4 == 0 && ((uintptr_t)state | (uintptr_t)out) % 16 == 0) {
+    // 8 threads a row (a line of 128 bytes): four times the blocks of 32, while those leave compute units without one
+    const bool narrow = (long long)batch * heads * ((value_dim + 127) / 128) < 256;
+    const int cols = narrow ? 32 : 128;
+    const dim3 grid((value_dim + cols - 1) / cols, heads, batch);
+    if (narrow) {
+      if (key_dim <= 64) hipLaunchKernelGGL((gla_step_kernel<2, 8>), grid, dim3(256), 0, (hipStream_t)stream, a);
+      else if (key_dim <= 128) hipLaunchKernelGGL((gla_step_kernel<4, 8>), grid, dim3(256), 0, (hipStream_t)stream, a);
+      else hipLaunchKernelGGL((gla_step_kernel<8, 8>), grid, dim3(256), 0, (hipStream_t)stream, a);
+    } else {
+      if (key_dim <= 64) hipLaunchKernelGGL((gla_step_kernel<8, 32>), grid, dim3(256), 0, (hipStream_t)stream, a);
+      else if (key_dim <= 128) hipLaunchKernelGGL((gla_step_kernel<16, 32>), grid, dim3(256), 0, (hipStream_t)stream, a);
+      else hipLaunchKernelGGL((gla_step_kernel<32, 32>), grid, dim3(256), 0, (hipStream_t)stream, a);
+    }
+    NNIS_LAUNCH_CHECK("gla_step");
+    return 0;
+  }
   const int need = (key_dim + 15) / 16;
   const int groups = need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : (need <= 8 ? 8 : 16)));
   const int span = 4 * (kWave / groups);

@@ -119,7 +119,7 @@ _RECURRENT_SIGNATURES = {
     "nnis_gla_scan": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _FLT, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT,
                       _VOID, _INT, _INT, _VOID, _VOID, _VOID],
     "nnis_gla_scan_turned": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _FLT, _VOID,
-                             _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _INT, _VOID, _VOID, _VOID],
+                             _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _INT, _VOID, _VOID, _INT, _VOID],
     "nnis_gated_delta": [_VOID, _INT, _INT, _VOID, _VOID, _VOID, _FLT, _FLT, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _INT, _VOID,
                          _VOID, _VOID, _VOID],
     "nnis_retention_chunks": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _INT, _VOID, _FLT, _VOID, _VOID, _VOID,
@@ -2286,7 +2286,8 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay_logs: Opti
                                          _ptr(decay_logits), _ptr(head_decay), _ptr(cos), _ptr(sin), rot_dim,
                                          cos.shape[0] if cos is not None else 0, ctx.tok_pos.data_ptr(), float(scale),
                                          state.data_ptr(), ctx.seq_slot.data_ptr(), ctx.seq_start.data_ptr(), ctx.batch, heads,
-                                         key_dim, value_dim, out.data_ptr(), piece, pieces, _ptr(carried), _ptr(decayed), _stream()))
+                                         key_dim, value_dim, out.data_ptr(), piece, pieces, _ptr(carried), _ptr(decayed),
+                                         1 if (ctx.decode and tokens == ctx.batch) else 0, _stream()))
     return out
 
 

@@ -1484,3 +1484,33 @@ def test_selective_scan_states_off_16_byte_boundaries(channels, states, lengths)
         results.append((out, held))
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
     assert torch.equal(results[0][1][-1], state[-1]) and not torch.equal(results[0][1][0], state[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch, heads, d, e", [(1, 8, 128, 256), (3, 2, 64, 36), (2, 3, 20, 4), (70, 4, 72, 132), (40, 8, 256, 64), (2, 2, 65, 30), (66, 4, 48, 128)])
+def test_gla_single_tokens(batch, heads, d, e, dtype):
+    """A step of single tokens against the scan over runs of one token: equal states, and outputs within the roundings of a
+    sum of d products in another order; sequences without a slot leave everything as it was."""
+    ops = _ops()
+    torch.manual_seed(batch + d + e)
+    rows = torch.randn(batch, heads * (2 * d + e) + 8).to(dtype).cuda()
+    q, k, v = rows[:, :heads * d], rows[:, heads * d:2 * heads * d], rows[:, 2 * heads * d:heads * (2 * d + e)]
+    state = torch.randn(batch + 1, heads, d, e).cuda()
+    ctx = _prompts([1] * batch)
+    ctx.seq_slot = _i32([-1 if b == 1 and batch > 2 else batch - b for b in range(batch)])
+    ctx.tok_pos = _i32([(7 * b) % 50 for b in range(batch)])
+    angle = torch.rand(50, d // 4).cuda() * 6
+    fixed = torch.rand(heads).cuda()
+    for decays in (dict(decay_logs=-torch.rand(batch, heads * d).cuda()),
+                   dict(decay_logs=None, head_decay=torch.stack([fixed, fixed.log()]), rotation=(angle.cos(), angle.sin(), 2 * (d // 4)))):
+        results = []
+        for ctx.decode in (False, True):
+            held, out = state.clone(), torch.full((batch, heads * e), 9.0, device="cuda")
+            ops.gla_scan(q, k, v, scale=d ** -0.5, state=held, ctx=ctx, heads=heads, out=out, **decays)
+            results.append((out, held))
+        assert torch.equal(results[0][1], results[1][1]) and torch.equal(results[0][1][0], state[0])
+        slots = ctx.seq_slot.long()
+        live = slots >= 0
+        size = torch.einsum("bhd,bhde->bhe", q.float().abs().reshape(batch, heads, d) * 1.5, results[0][1][slots.clamp(min=0)].abs()).reshape(batch, heads * e)
+        error = (results[0][0] - results[1][0]).abs()  # (a rotation makes a channel at most sqrt(2) as large)
+        assert (error[live] <= 2.0 ** -23 * (4 + d ** 0.5) * d ** -0.5 * size[live] + 1e-6).all() and (results[1][0][~live] == 9.0).all()
