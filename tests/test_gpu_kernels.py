@@ -1514,3 +1514,29 @@ def test_gla_single_tokens(batch, heads, d, e, dtype):
         size = torch.einsum("bhd,bhde->bhe", q.float().abs().reshape(batch, heads, d) * 1.5, results[0][1][slots.clamp(min=0)].abs()).reshape(batch, heads * e)
         error = (results[0][0] - results[1][0]).abs()  # (a rotation makes a channel at most sqrt(2) as large)
         assert (error[live] <= 2.0 ** -23 * (4 + d ** 0.5) * d ** -0.5 * size[live] + 1e-6).all() and (results[1][0][~live] == 9.0).all()
+
+
+@pytest.mark.parametrize("width", [1028, 2048, 4096, 5000, 8192])
+@pytest.mark.parametrize("count", [1, 5, 1023, 1024])
+def test_rmsnorm_of_few_rows(width, count):
+    """Rows that a block each norms (up to 1,023) and rows that a wave each does: with a row list, with a sum written back, with
+    both, in both types; the last rows of the list out of order."""
+    ops = _ops()
+    torch.manual_seed(width + count)
+    x, delta, weight = torch.randn(count + 3, width), torch.randn(count + 3, width), 1 + 0.2 * torch.randn(width)
+    for dtype in (torch.float32, torch.bfloat16):
+        d, w = delta.to(dtype), weight.to(dtype)
+        rows = torch.arange(count + 2, 2, -1, dtype=torch.int32)
+        total = x.double() + d.double()
+        for picked, added in ((rows, None), (rows, d), (None, d), (None, None)):
+            held = x.cuda()
+            out = torch.full((count + 1 if picked is not None else count + 3, width), 9.0, device="cuda")
+            ops.rmsnorm(held, w.cuda(), 1e-6, out[:count] if picked is not None else out, delta=None if added is None else added.cuda(),
+                        rows=None if picked is None else picked.cuda())
+            source = (total if added is not None else x.double())[picked.long() if picked is not None else slice(None)]
+            want = source / torch.sqrt((source * source).mean(1, keepdim=True) + 1e-6) * w.double()
+            got = out[:len(want)].cpu().double()
+            assert ((got - want).abs() <= 2e-6 * (1 + want.abs())).all()
+            assert picked is None or (out[count] == 9).all()
+            written = added is not None and picked is None
+            assert torch.equal(held.cpu(), (x + d.float()) if written else x)
