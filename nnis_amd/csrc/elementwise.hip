@@ -26,6 +26,21 @@ __global__ void embed_kernel(const int* __restrict__ ids, const void* __restrict
     return;
   }
   const size_t base = (size_t)id * width;
+  if (width % 4 == 0 && ((uintptr_t)table | (uintptr_t)out) % 16 == 0) {  // four channels at a time
+    for (int c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
+      float v[4];
+      if (table_dtype == NNIS_F32) {
+        const float4 four = *(const float4*)((const float*)table + base + c);
+        v[0] = four.x; v[1] = four.y; v[2] = four.z; v[3] = four.w;
+      } else {
+        const uint2 four = *(const uint2*)((const bf16_t*)table + base + c);
+        v[0] = __uint_as_float(four.x << 16); v[1] = __uint_as_float(four.x & 0xffff0000u);
+        v[2] = __uint_as_float(four.y << 16); v[3] = __uint_as_float(four.y & 0xffff0000u);
+      }
+      *(float4*)(dst + c) = make_float4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+    }
+    return;
+  }
   for (int c = threadIdx.x; c < width; c += blockDim.x) dst[c] = load_as_f32(table, table_dtype, base + c) * scale;
 }
 
@@ -34,7 +49,7 @@ extern "C" int nnis_embed(const int* ids, const void* table, int table_dtype, fl
   NNIS_REQUIRE(nnis_dtype_ok(table_dtype), "embed: unknown table dtype %d", table_dtype);
   NNIS_REQUIRE(tokens >= 0 && width > 0 && vocab > 0, "embed: bad sizes tokens=%d width=%d vocab=%d", tokens, width, vocab);
   if (tokens == 0) return 0;
-  hipLaunchKernelGGL(embed_kernel, dim3(tokens), dim3(256), 0, (hipStream_t)stream, ids, table, table_dtype, out,
+  hipLaunchKernelGGL(embed_kernel, dim3(tokens), dim3(width >= 2048 ? 512 : 256), 0, (hipStream_t)stream, ids, table, table_dtype, out,
                      width, vocab, scale);
   NNIS_LAUNCH_CHECK("embed");
   return 0;

@@ -5,6 +5,26 @@
 // Storage types are chosen at run time; every sum and statistic is 32-bit.
 #include "common.h"
 
+typedef __attribute__((ext_vector_type(4))) float f32x4_r;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_r;
+
+__device__ __forceinline__ f32x4_r load4_r(const void* base, int dtype, size_t index) {
+  if (dtype == NNIS_F32) return *(const f32x4_r*)((const float*)base + index);
+  const bf16x4_r v = *(const bf16x4_r*)((const bf16_t*)base + index);
+  return (f32x4_r){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+
+__device__ __forceinline__ void store4_r(void* base, int dtype, size_t index, f32x4_r v) {
+  if (dtype == NNIS_F32) {
+    *(f32x4_r*)((float*)base + index) = v;
+  } else {
+    bf16x4_r packed;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) packed[e] = (__bf16)v[e];
+    *(bf16x4_r*)((bf16_t*)base + index) = packed;
+  }
+}
+
 // -----------------------------------------------------------------------------
 // Embedding with a table of token pairs: out[c][t, :] = table[id] + pairs[row], the same in every one of
 // `copies` copies.  row = (previous * mul_prev + id * mul_cur) % buckets, or `buckets` (the table's last
@@ -41,6 +61,13 @@ __global__ void embed_pair_kernel(const int* __restrict__ ids, const int* __rest
   long long row = buckets;
   if (pos > 0 && before >= 0) row = ((long long)before * mul_prev + (long long)id * mul_cur) % buckets;
   const size_t base = (size_t)id * width, pair_base = (size_t)row * width;
+  if (width % 4 == 0 && ((uintptr_t)table | (uintptr_t)pairs | (uintptr_t)out) % 16 == 0) {  // four channels at a time
+    for (int c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
+      const f32x4_r v = load4_r(table, table_dtype, base + c) + load4_r(pairs, pairs_dtype, pair_base + c);
+      for (int s = 0; s < copies; ++s) *(f32x4_r*)(dst + s * plane + c) = v;
+    }
+    return;
+  }
   for (int c = threadIdx.x; c < width; c += blockDim.x) {
     const float v = load_as_f32(table, table_dtype, base + c) + load_as_f32(pairs, pairs_dtype, pair_base + c);
     for (int s = 0; s < copies; ++s) dst[s * plane + c] = v;
@@ -55,7 +82,7 @@ extern "C" int nnis_embed_pair(const int* ids, const int* tok_slot, const int* t
   NNIS_REQUIRE(mul_prev >= 0 && mul_cur >= 0, "embed_pair: the multipliers must not be negative");
   NNIS_REQUIRE(ids && tok_slot && tok_pos && last_token && out, "embed_pair: a pointer is missing");
   if (tokens == 0) return 0;
-  hipLaunchKernelGGL(embed_pair_kernel, dim3(tokens), dim3(width >= 1024 ? 256 : 64), 0, (hipStream_t)stream, ids, tok_slot,
+  hipLaunchKernelGGL(embed_pair_kernel, dim3(tokens), dim3(width >= 2048 ? 512 : (width >= 1024 ? 256 : 64)), 0, (hipStream_t)stream, ids, tok_slot,
                      tok_pos, tokens, table, table_dtype, vocab, pairs, pairs_dtype, buckets, mul_prev, mul_cur, last_token, out,
                      copies, width);
   NNIS_LAUNCH_CHECK("embed_pair");
@@ -160,26 +187,6 @@ __global__ void stream_kernel(StreamArgs a) {
 // The same with a row in registers: a thread takes CH pieces of 4 channels of every stream, asks for all of them at
 // once (the loop above waits for memory once a piece), and keeps u in registers.  Widths in steps of 4 up to
 // 4096 * CH... channels a block of up to 1024 threads covers.
-typedef __attribute__((ext_vector_type(4))) float f32x4_r;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_r;
-
-__device__ __forceinline__ f32x4_r load4_r(const void* base, int dtype, size_t index) {
-  if (dtype == NNIS_F32) return *(const f32x4_r*)((const float*)base + index);
-  const bf16x4_r v = *(const bf16x4_r*)((const bf16_t*)base + index);
-  return (f32x4_r){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-}
-
-__device__ __forceinline__ void store4_r(void* base, int dtype, size_t index, f32x4_r v) {
-  if (dtype == NNIS_F32) {
-    *(f32x4_r*)((float*)base + index) = v;
-  } else {
-    bf16x4_r packed;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) packed[e] = (__bf16)v[e];
-    *(bf16x4_r*)((bf16_t*)base + index) = packed;
-  }
-}
-
 template <int CH, int SMAX>
 __global__ __launch_bounds__(1024) void stream_wide_kernel(StreamArgs a) {
   __shared__ float scratch[16];
@@ -188,12 +195,14 @@ __global__ __launch_bounds__(1024) void stream_wide_kernel(StreamArgs a) {
   const int S = a.streams;
   const size_t plane = (size_t)a.tokens * a.width;
   float* x = a.x + (size_t)row * a.width;
-  f32x4_r v[SMAX][CH], y[CH];
+  f32x4_r v[SMAX][CH], y[CH], weight[CH], bias[CH];
   bool inside[CH];
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int col = 4 * (threadIdx.x + i * blockDim.x);
     inside[i] = col < a.width;
+    weight[i] = a.weight ? load4_r(a.weight, a.weight_dtype, inside[i] ? col : 0) : (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
+    bias[i] = a.bias ? load4_r(a.bias, a.weight_dtype, inside[i] ? col : 0) : (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int s = 0; s < SMAX; ++s) v[s][i] = (inside[i] && s < S) ? *(const f32x4_r*)(x + s * plane + col) : (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
     y[i] = (a.y && inside[i]) ? load4_r(a.y, a.y_dtype, (size_t)row * a.width + col) : (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
@@ -255,8 +264,8 @@ __global__ __launch_bounds__(1024) void stream_wide_kernel(StreamArgs a) {
     if (!inside[i]) continue;
     f32x4_r out = u[i];
     if (a.weight) {
-      out = ((u[i] - mean) * scale) * load4_r(a.weight, a.weight_dtype, col);
-      if (a.bias) out += load4_r(a.bias, a.weight_dtype, col);
+      out = ((u[i] - mean) * scale) * weight[i];
+      if (a.bias) out += bias[i];
     }
     store4_r(a.h, a.h_dtype, out_base + col, out);
   }
@@ -358,13 +367,14 @@ __global__ __launch_bounds__(1024) void branch_mean_wide_kernel(BranchArgs a) {
   const size_t base = (size_t)blockIdx.x * a.width;
   const int col = 4 * threadIdx.x;
   const bool inside = col < a.width;
-  f32x4_r v[kMostBranches];
+  f32x4_r v[kMostBranches], weight[kMostBranches];
   float squares[kMostBranches];
 #pragma unroll
   for (int i = 0; i < kMostBranches; ++i) {
-    v[i] = (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
+    v[i] = weight[i] = (f32x4_r){0.0f, 0.0f, 0.0f, 0.0f};
     if (i < a.count && inside) {
       v[i] = load4_r(a.y[i], a.y_dtype, base + col);
+      weight[i] = load4_r(a.weight[i], a.weight_dtype, col);
       if (a.bias[i]) v[i] += load4_r(a.bias[i], a.weight_dtype, col);
     }
     squares[i] = (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
@@ -374,7 +384,7 @@ __global__ __launch_bounds__(1024) void branch_mean_wide_kernel(BranchArgs a) {
   for (int i = 0; i < kMostBranches; ++i)
     if (i < a.count) {
       const float scale = 1.0f / sqrtf(block_sum(squares[i], scratch) / (float)a.width + a.eps);
-      if (inside) acc += (v[i] * scale) * load4_r(a.weight[i], a.weight_dtype, col);
+      acc += (v[i] * scale) * weight[i];
     }
   if (inside) store4_r(a.out, a.out_dtype, base + col, acc * (1.0f / (float)a.count));
 }

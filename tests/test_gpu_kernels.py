@@ -1540,3 +1540,25 @@ def test_rmsnorm_of_few_rows(width, count):
             assert picked is None or (out[count] == 9).all()
             written = added is not None and picked is None
             assert torch.equal(held.cpu(), (x + d.float()) if written else x)
+
+
+@pytest.mark.parametrize("width, shift", [(24, 0), (24, 1), (2052, 0), (2052, 4), (30, 0), (4100, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_embeddings_four_channels_at_a_time(width, shift, dtype):
+    """Rows that can be loaded four channels at a time, tables that lie off such places, and widths that cannot: exact copies,
+    and with a table of pairs exact sums, in every copy; ids outside the table give zeros."""
+    ops = _ops()
+    torch.manual_seed(width)
+    table, pairs = torch.randn(shift + 40 * width).to(dtype)[shift:].view(40, width), torch.randn(6, width).to(dtype)
+    held = torch.empty(shift + 40 * width, dtype=dtype, device="cuda")[shift:].view(40, width)
+    held.copy_(table)
+    ids = _i32([3, 39, -1, 40, 0])
+    out = torch.full((5, width), 9.0, device="cuda")
+    ops.embed(ids, held, out, scale=0.5)
+    want = table.float()[[3, 39, 0, 0, 0]] * torch.tensor([0.5, 0.5, 0.0, 0.0, 0.5])[:, None]
+    assert torch.equal(out.cpu(), want)
+    both = torch.full((3, 5, width), 9.0, device="cuda")
+    ops.embed_pair(ids, _i32([0, 1, 2, 3, -1]), _i32([0, 0, 0, 0, 0]), held, pairs.cuda(), 3, 5, _i32([-1] * 4), both)
+    want = torch.zeros(5, width)
+    want[:2] = table.float()[[3, 39]] + pairs.float()[5]
+    assert torch.equal(both.cpu(), want.expand(3, 5, width))
