@@ -345,8 +345,21 @@ __device__ __forceinline__ void load_lane(float (&into)[PER], const float* row, 
   }
 }
 
+// A token's B or C, the same in every lane of a channel's one: through the scalar cache (16 words an instruction; as vector loads
+// a token's two rows are 8 instructions of a wave, whose lanes all ask for the same words).
+// 4,096 channels of 16 states, a token of 4 sequences 5.1 -> 4.5 us, the last pass over pieces of 16 tokens of 4 prompts of 90 to
+// 700 63 -> 50; the first, which has no C, 36 -> 42: it keeps the vector loads.
+template <int PER>
+__device__ __forceinline__ void load_uniform(float (&into)[PER], const float* row) {
+  typedef const __attribute__((address_space(4))) float constant_float;
+  constant_float* from = (constant_float*)(uintptr_t)row;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) into[j] = from[j];
+}
+
 // PER: states a lane keeps (8, or 16: one lane a channel up to 16 states, half the lanes and none of the exchanges)
-template <int LANES, int PASS, int PER>
+// UNIFORM: one lane a channel with PER states, no fewer
+template <int LANES, int PASS, int PER, bool UNIFORM>
 __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
   const int b = blockIdx.z, piece = blockIdx.y;
   const int slot = a.seq_slot[b];
@@ -364,7 +377,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
   const int c = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES;
   const bool live = c < a.channels;
   const int cc = live ? c : 0;
-  const int N = a.states;
+  const int N = UNIFORM ? PER : a.states;
   // (a lane's values lie within the row, on 16-byte boundaries: one by one, neighbouring lanes' loads and stores are 64 bytes
   // apart and take a line each, 32 a wave for 16 states: a token for 4 sequences of 4,096 channels 10.7 -> 5.1 us; the passes over pieces of
   // 4 prompts of 90 to 700 tokens 66 -> 36 and 87 -> 63)
@@ -386,10 +399,20 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
   float z_next = PASS == 1 ? 0.0f : load_as_f32(a.z, a.z_dtype, (size_t)first * a.z_stride + cc);
   float B_next[PER], C_next[PER];
   const bool wide = N % 4 == 0 && ((uintptr_t)a.bc % 16 == 0);  // a lane's 8 values lie within the row, on 16-byte boundaries
-  load_lane<PER>(B_next, a.bc + (size_t)first * 2 * N, part, N, wide);
+  static_assert(!UNIFORM || LANES == 1, "every lane takes the same words");
+  auto load_bc = [&](int t) {
+    const float* row = a.bc + (size_t)t * 2 * N;
+    if constexpr (UNIFORM) {
+      load_uniform<PER>(B_next, row);
+      if (PASS != 1) load_uniform<PER>(C_next, row + PER);
+    } else {
+      load_lane<PER>(B_next, row, part, N, wide);
+      if (PASS != 1) load_lane<PER>(C_next, row + N, part, N, wide);
+    }
+  };
 #pragma unroll
   for (int j = 0; j < PER; ++j) C_next[j] = 0.0f;
-  if (PASS != 1) load_lane<PER>(C_next, a.bc + (size_t)first * 2 * N + N, part, N, wide);
+  load_bc(first);
   for (int t = first; t < last; ++t) {
     const float x = x_next, z = z_next;
     // (the step size is the same in all lanes of a channel: one of them takes the logarithm)
@@ -405,8 +428,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
     x_next = load_as_f32(a.x, a.x_dtype, (size_t)ahead * a.channels + cc);
     dt_next = a.dt_pre[(size_t)ahead * a.channels + cc];
     if (PASS != 1) z_next = load_as_f32(a.z, a.z_dtype, (size_t)ahead * a.z_stride + cc);
-    load_lane<PER>(B_next, a.bc + (size_t)ahead * 2 * N, part, N, wide);
-    if (PASS != 1) load_lane<PER>(C_next, a.bc + (size_t)ahead * 2 * N + N, part, N, wide);
+    load_bc(ahead);
     const float dx = dt * x;
     steps += dt;
     float acc = 0.0f;
@@ -837,16 +859,18 @@ extern "C" int nnis_selective_scan(const void* x, int x_dtype, const float* dt_p
   hipStream_t s = (hipStream_t)stream;
   // blocks of one wave while larger ones would leave compute units without any (single tokens, short runs)
   const int threads = pieces <= 1 && (long long)batch * channels * (need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : 8))) < 256 * 1024 ? 64 : 256;
-#define NNIS_SCAN(LANES_, PASS_, PIECES_, PER_)                                                                            \
-  hipLaunchKernelGGL((selective_scan_kernel<LANES_, PASS_, PER_>),                                                         \
+#define NNIS_SCAN(LANES_, PASS_, PIECES_, PER_, UNIFORM_)                                                                  \
+  hipLaunchKernelGGL((selective_scan_kernel<LANES_, PASS_, PER_, UNIFORM_>),                                               \
                      dim3((channels + threads / LANES_ - 1) / (threads / LANES_), PIECES_, batch), dim3(threads), 0, s, a)
-#define NNIS_SCAN_PASS(PASS_, PIECES_)                     \
-  do {                                                     \
-    if (states <= 8) NNIS_SCAN(1, PASS_, PIECES_, 8);      \
-    else if (need <= 1) NNIS_SCAN(1, PASS_, PIECES_, 16);  \
-    else if (need <= 2) NNIS_SCAN(2, PASS_, PIECES_, 16);  \
-    else if (need <= 4) NNIS_SCAN(4, PASS_, PIECES_, 16);  \
-    else NNIS_SCAN(8, PASS_, PIECES_, 16);                 \
+#define NNIS_SCAN_PASS(PASS_, PIECES_)                               \
+  do {                                                               \
+    if (states == 8) NNIS_SCAN(1, PASS_, PIECES_, 8, PASS_ != 1);          \
+    else if (states < 8) NNIS_SCAN(1, PASS_, PIECES_, 8, false);     \
+    else if (states == 16) NNIS_SCAN(1, PASS_, PIECES_, 16, PASS_ != 1);   \
+    else if (need <= 1) NNIS_SCAN(1, PASS_, PIECES_, 16, false);     \
+    else if (need <= 2) NNIS_SCAN(2, PASS_, PIECES_, 16, false);     \
+    else if (need <= 4) NNIS_SCAN(4, PASS_, PIECES_, 16, false);     \
+    else NNIS_SCAN(8, PASS_, PIECES_, 16, false);                    \
   } while (0)
   if (pieces <= 1) {
     NNIS_SCAN_PASS(0, 1);
