@@ -125,11 +125,13 @@ __global__ __launch_bounds__(KSPLIT > 4 ? 64 * KSPLIT : 256) void gemm_fused_ker
   // has asked for its weights.  The same goes for the parts of a prepared norm's sums of squares.
   int tok_slot[MT], tok_pos[MT], tok_page[MT];
   f32x4 tok_cos[MT], tok_sin[MT];
-  constexpr int kPartRegs = 8;  // parts of a row's sum of squares a lane keeps in flight (4 lane groups share a row)
+  // Parts of a row's sum of squares a lane keeps in flight (4 lane groups share a row): 9 take the 36 of a row of 576 columns in
+  // one trip to memory (with 8 the last four were another, behind the products: a decode step of 30 layers, 8 sequences, 891 -> 882 us)
+  constexpr int kPartRegs = DEAL ? 8 : 9;
   float ss_held[MT][kPartRegs];
   const bool ends_unit = active && part == 0;
   // The parts of a prepared row's sum of squares: a narrow row's few (up to 64) are all asked for by the lane
-  // groups of the wave that ends the unit, eight in flight each.  DEAL: a wide row's (a hundred and more) are
+  // groups of the wave that ends the unit, nine in flight each.  DEAL: a wide row's (a hundred and more) are
   // dealt to the lane groups of all the waves that share the unit's K, so that they are one round trip too and
   // not a chain of them (2048 columns, 8 tokens: the gate/up product 24.9 -> 16 us, the QKV product 14.2 -> 9).
   // The waves' sums meet in LDS with the products' (part_ss), the lane groups' in the shuffles below.  A
