@@ -1562,3 +1562,39 @@ def test_embeddings_four_channels_at_a_time(width, shift, dtype):
     want = torch.zeros(5, width)
     want[:2] = table.float()[[3, 39]] + pairs.float()[5]
     assert torch.equal(both.cpu(), want.expand(3, 5, width))
+
+
+@pytest.mark.parametrize("kernel, heads, kv_heads", [("columns", 16, 2), ("keys", 9, 3)])
+@pytest.mark.parametrize("splits, waves", [(1, 4), (2, 2), (8, 4), (1, 1)])
+def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves):
+    """Runs of keys that end within a sequence's first 64 pages, at the 64th, behind it and begin behind it, whole and in a
+    window that leaves the first pages out."""
+    ops = _ops()
+    torch.manual_seed(splits * 8 + waves)
+    head_dim, lengths = 64, [4200, 4096, 4097, 8300, 63 * 64, 5]
+    ks = [torch.randn(n, kv_heads, head_dim).bfloat16().float() for n in lengths]
+    vs = [torch.randn(n, kv_heads, head_dim).bfloat16().float() for n in lengths]
+    scale = 1.0 / math.sqrt(head_dim)
+    k_pages, v_pages, table = _paged(ks, vs, torch.bfloat16, kv_heads, head_dim, pages=420, max_pages=131)
+    rows = [(s, n - 1, torch.randn(heads, head_dim).bfloat16().float()) for s, n in enumerate(lengths)]
+    q = torch.stack([r[2] for r in rows]).bfloat16().reshape(len(rows), -1).cuda()
+    out = torch.empty(len(rows), heads * head_dim, dtype=torch.bfloat16, device="cuda")
+    partial = torch.full((len(rows) * heads * splits * (head_dim + 4),), float("nan"), dtype=torch.float32, device="cuda")
+    for window in (0, 4300):
+        ops.attention_decode_bf16(q, out, k_pages, v_pages, table, _i32([s for s, _, _ in rows]), _i32([p for _, p, _ in rows]),
+                                  heads, kv_heads, head_dim, scale, window, splits, partial, waves, kernel)
+        want = _plain_rows(rows, ks, vs, scale, window=window) if window else _plain_rows(rows, ks, vs, scale)
+        assert (out.cpu().float().view(len(rows), heads, head_dim) - want).abs().max().item() <= 1e-2
+
+
+@pytest.mark.parametrize("m, n, k", [(70, 576, 576), (128, 700, 1024), (128, 576, 1032), (65, 576, 1208), (130, 2048, 1792), (130, 2000, 1832)])
+def test_products_around_the_k_from_which_it_goes_in_parts(m, n, k):
+    """Products whose K is just too short to go in two, four or eight parts, and just long enough: against 64 bits, and the
+    parts' own rows, as ops.linear and into the stream."""
+    ops = _ops()
+    torch.manual_seed(m + k)
+    x, w = torch.randn(m, k).bfloat16(), (torch.randn(n, k) / math.sqrt(k)).bfloat16()
+    want, scale = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    y = torch.full((m + 1, n), 7.0, device="cuda")
+    ops.linear(x.cuda(), ops.pack_weight(w.cuda()), y[:m])
+    assert ((y[:m].cpu().double() - want).abs() <= 2e-7 * math.sqrt(k) * scale + 1e-6).all() and (y[m] == 7).all()
