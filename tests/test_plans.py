@@ -164,3 +164,15 @@ def test_the_tiles_of_products_into_the_stream():
     }.items():
         assert (ops.gemm_tile(m, n, k), ops.gemm_tile(m, n, k, residual=True)) == (tile, stream), (m, n, k)
         assert ops.core().nnis_gemm_residual_parts(m, n) >= 2 * -(-n // width[stream])  # (the room that any tile asks for)
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim", [(9, 3, 64), (32, 4, 64), (32, 32, 64), (16, 1, 256)])
+def test_prefill_plans_of_short_prompts(heads, kv_heads, head_dim):
+    """Up to 127 tokens: items of one column while a step has few, by the rows planned for and not by the length, which a replayed
+    step knows by its class alone."""
+    from nnis_amd.kernels.ops import prefill_plan
+
+    for longest in (1, 24, 64, 65, 127):
+        assert prefill_plan(longest, 64, heads, head_dim, kv_heads) == prefill_plan(longest, 128, heads, head_dim, kv_heads) == (1, 1)
+        assert prefill_plan(longest, 65536, heads, head_dim, kv_heads) == (1, 0)
+    assert prefill_plan(128, 128, heads, head_dim, kv_heads) == (2, 1)
