@@ -623,9 +623,11 @@ struct PageRun {
   int max_pages;
   int first, stride;  // lane i holds the page at index first + i * stride of the sequence's block-table row
   int cached;
-  // `early`: null, or lane i's page i of the row, asked for before the run's bounds were known (decode: the bounds hang on the
+  // `early`: null, or lane i's page i of the row, asked for before the run's bounds were known (they hang on the
   // token's position, a trip to memory; a run of `count` pages that ends within the row's first 64 then needs no further one:
-  // a decode step of 30 layers, 1 / 8 sequences, 800 -> 797 / 882 -> 879 us)
+  // a decode step of 30 layers, 1 / 8 sequences, 800 -> 797 / 882 -> 879 us;
+  // the kernel for groups of more than 4 heads, which begins with more, was slower so: a step of 22 layers of 32/4
+  // heads, 1 / 11 / 40 sequences, 924 / 1,118 / 1,368 us without and 934 / 1,127 / 1,378 with)
   __device__ __forceinline__ void fill(int lane, int count, const int* early) {
     int index = first + lane * stride;
     if (early && first + (count - 1) * stride < kWave) {
@@ -792,8 +794,7 @@ __device__ __forceinline__ bool merge_group(AttnState<C>& st, float* slots, int 
 template <int C, int RING>
 __device__ __forceinline__ void attend_run(AttnState<C>& st, const QFrag (&q)[C], const MfmaArgs& a, const int* pages,
                                            int kv_head, int first, int stride, int mine, int last_key,
-                                           const int (&lo)[C], const int (&hi)[C], int lane, const More<C>& more,
-                                           const int* early = nullptr) {
+                                           const int (&lo)[C], const int (&hi)[C], int lane, const More<C>& more) {
   // (The run's bounds are the same in every lane -- they come from sums over the wave -- but the compiler has them
   // in vector registers unless it is told: as scalars the loop's counters, the pages' numbers and the pages'
   // addresses cost no vector instruction, of which the loop has none to spare.)
@@ -807,7 +808,7 @@ __device__ __forceinline__ void attend_run(AttnState<C>& st, const QFrag (&q)[C]
   const bf16_t* v_base = v_page_ptr(a, 0, kv_head);
   const size_t k_page_stride = (size_t)a.kv_heads * nnis_k_page_elems(HD), v_page_stride = (size_t)a.kv_heads * nnis_v_page_elems(HDV);
   PageRun run = {pages, a.max_pages, first, stride, 0};
-  run.fill(lane, mine, early);
+  run.fill(lane, mine, nullptr);
   // block b of the run: page index first + (b / 2) * stride, half b % 2
   int blocks = 2 * mine;
   if ((first + (mine - 1) * stride) * kPageTokens + 32 > last_key) --blocks;  // the last page's second half is beyond the keys
@@ -1203,7 +1204,6 @@ __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(Mfma
   const int pos = a.tok_pos[token];
   const int first_key = first_seen(a.window, pos);
   const int* pages = a.block_table + (size_t)(a.rows_by_token ? token : slot) * a.max_pages;
-  const int early = pages[lane < a.max_pages ? lane : a.max_pages - 1];
 
   QFrag q[C];
   int lo[C], hi[C];
@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(Mfma
   }
 #endif
   const int mine = end > begin + wave ? (end - begin - wave + waves - 1) / waves : 0;  // pages of this wave
-  attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2)>(st, q, a, pages, kv_head, begin + wave, waves, mine, pos, lo, hi, lane, more, &early);
+  attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2)>(st, q, a, pages, kv_head, begin + wave, waves, mine, pos, lo, hi, lane, more);
 #if NNIS_POOLED_BLOCKS
   // the pooled blocks go with the first run of the keys (with the step's tables the pooled pages are still the slot's)
   if (a.pool > 0 && split == 0) {
