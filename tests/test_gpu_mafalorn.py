@@ -795,3 +795,18 @@ def test_other_sizes_drawn_from_a_seed(tmp_path):
         slot = engine.start_sequence()
         got = _collect(engine, slot, ids, [66, 70] + list(range(71, 81)))
         assert _relative(got, want) < 5e-5, f"seed {seed}: {config}"
+
+
+@pytest.mark.parametrize("tokens, heads, n, k", [(1, 16, 130, 192), (17, 3, 64, 40), (3, 2, 65, 512), (33, 100, 200, 24)])
+def test_a_map_for_every_head_over_several_blocks(tokens, heads, n, k):
+    """Few rows, whose strips of outputs lie in blocks of their own, and rows enough that one block takes them all."""
+    from nnis_amd.kernels import ops
+
+    torch.manual_seed(tokens + n)
+    x, w, gate = torch.randn(tokens, heads, k).bfloat16(), (torch.randn(heads, n, k) / k ** 0.5).bfloat16(), torch.rand(tokens, heads, n)
+    want = (w.double()[None] * x.double()[:, :, None]).sum(-1)
+    for g in (None, gate):
+        out = torch.full((tokens + 1, heads * n), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.heads_linear(x.reshape(tokens, -1).cuda(), w.cuda(), None if g is None else g.reshape(tokens, -1).cuda(), heads, out[:tokens])
+        exact = (want if g is None else want * g.double()).reshape(tokens, -1)
+        assert ((out[:tokens].cpu().double() - exact).abs() <= 2.0 ** -8 * exact.abs() + 1e-5).all() and (out[tokens] == 7).all()
