@@ -662,7 +662,7 @@ int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, i
 // round of its blocks on 256 compute units, a slope times K: the least of these is taken.  Measured:
 // 64 x 2048 x 2048 13.4 us (two strips, one tile a block), 100 x 2048 x 2048 18.1 (2 x 2; 23.9 in tiles of 32 x 64), 100 x 11264 x 2048
 // 45.6 (tiles of 64 x 96; 52.7 in 128 x 64), 509 x 2048 x 5632 90 (64 x 64; 103 in 32 x 64), 2000 x 11264 x 2048 501 (128 x 128; 558 in 64 x 128).
-// Over 8 weights from 576 x 576 to 11264 x 2048 at 20 to 2,000 rows the form taken is 0.4% slower than the best on average.
+// Over 8 weights from 576 x 576 to 11264 x 2048 at 20 to 2,000 rows the form taken is 0.2% slower than the best on average.
 struct Variant {
   int rows, columns;  // of a block
   float slope, start; // microseconds: slope * K for each round of blocks, and start
@@ -670,7 +670,7 @@ struct Variant {
 constexpr Variant kVariants[] = {
     {16, 16, 0.0050f, 2.0f}, {16, 32, 0.0064f, 2.0f}, {32, 32, 0.0083f, 2.0f}, {64, 32, 0.0135f, 2.0f},
     {32, 64, 0.0095f, 4.0f}, {64, 64, 0.0145f, 4.5f}, {64, 96, 0.0185f, 4.5f}, {96, 64, 0.0190f, 4.5f}, {96, 96, 0.0285f, 3.5f},
-    {64, 128, 0.0235f, 4.5f}, {128, 64, 0.0209f, 5.8f}, {128, 96, 0.0315f, 4.8f}, {128, 128, 0.0364f, 6.9f}};
+    {64, 128, 0.0224f, 12.5f}, {128, 64, 0.0235f, 6.0f}, {128, 96, 0.0315f, 4.8f}, {128, 128, 0.0353f, 5.9f}};
 constexpr int kFewVariants = 4, kCountVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 enum : int { kHalfStrips = kCountVariants, kFourWaves, kTwoStrips, kHints };
 
