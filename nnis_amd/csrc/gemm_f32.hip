@@ -18,11 +18,10 @@
 //
 //  * gemm_f32_few_kernel: few rows of X (a decode step, a short prompt), or too few tiles to fill the chip.  The
 //    weight is streamed straight into operand registers; the waves of a block share K and meet in LDS.
-//  * gemm_f32_tiled_kernel: tiles of 32 to 128 rows and 64 to 128 columns, K in steps of 32 through a ring of stages in LDS.
+//  * gemm_f32_tiled_kernel: tiles of 32 to 128 rows and 64 to 128 columns, K in steps of 32 through two stages in LDS.
 // Which of them, and so which chains, goes by the sizes: a row's last bits depend on how many rows the product has, where
 // the ordered kernel's do not.
 #include "common.h"
-#include "lds_loads.h"
 
 #include <type_traits>
 
