@@ -381,17 +381,89 @@ __device__ __forceinline__ Split<4> split4(f32x4 v) {
   return out;
 }
 
-// What a sum of parts may not stand for: no number, infinity, and sums so small that their terms' last parts may be
-// missing (a zero stays).  One chain in 32 bits over the operands as they are.
-__device__ __noinline__ float chain_of(const float* x, const float* w, int k) {
-  float sum = 0.0f;
-  for (int i = 0; i < k; ++i) sum = fmaf(x[i], w[i], sum);
-  return sum;
+// TN tiles of one 16 rows of X in 32 bits throughout, operands straight from memory (row, weights[j]: this lane's row of each): for
+// what a sum of parts may not stand for.  In runs of kFlushSteps steps of 32 k like the parts' sums, DEPTH steps' operands in flight.
+template <int TN, int DEPTH>
+__device__ __forceinline__ void multiply_in_32_bits(const float* row, const float* const (&weights)[TN], int k, f32x4 (&total)[TN]) {
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int first = threadIdx.x % kWave / 16 * 4, full = k / kStepK;  // this lane group's k of 16; steps without k beyond the last
+  struct Operands {
+    f32x4 a[2], b[2][TN];
+  };
+  auto multiply = [&](const Operands& v, f32x4 (&sum)[TN]) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.b[half][j][q], v.a[half][q], sum[j], 0, 0, 0);
+  };
+  f32x4 sum[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) sum[j] = total[j] = zero;
+  if (full > 0) {
+    auto ask = [&](Operands& v, int step) {  // (beyond the last full one: that one, which is not multiplied again)
+      const int at = (step < full ? step : full - 1) * kStepK + first;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        v.a[half] = load4(row + at + half * 16);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) v.b[half][j] = load4(weights[j] + at + half * 16);
+      }
+    };
+    Operands ring[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) ask(ring[d], d);
+    int run = 0;
+    auto flush = [&] {
+      if (++run < kFlushSteps) return;
+      run = 0;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        total[j] += sum[j];
+        sum[j] = zero;
+      }
+    };
+    int step = 0;
+#pragma unroll 1
+    for (; step + DEPTH <= full; step += DEPTH)
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        multiply(ring[d], sum);
+        ask(ring[d], step + d + DEPTH);
+        flush();
+      }
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (step + d < full) {
+        multiply(ring[d], sum);
+        flush();
+      }
+  }
+  if (full * kStepK < k) {
+    Operands last;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int at = full * kStepK + half * 16 + first;
+      last.a[half] = at < k ? load4(row + at) : zero;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) last.b[half][j] = at < k ? load4(weights[j] + at) : zero;
+    }
+    multiply(last, sum);
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) total[j] += sum[j];
 }
+
+// Whether a sum of parts stands: not if it is no number or infinite, nor so small that its terms' last parts may be missing (a zero stays).
 __device__ __forceinline__ bool parts_hold(float v) {
   const unsigned magnitude = __float_as_uint(v) & 0x7fffffffu;
   return magnitude == 0u || (magnitude >= 0x12000000u && magnitude < 0x7f800000u);  // from 2^-91 on
 }
+
+// Bytes of LDS of a tile's two stages, and the waves of a SIMD that they leave room for (and the registers have to).
+constexpr int tile_lds(int rows, int columns, int groups) { return 2 * groups * (rows + columns) * kStepK * 3 * (int)sizeof(__bf16); }
+constexpr int tile_waves(int lds, int waves) { return 160 * 1024 / lds * waves / 4; }
 
 // KG groups of WGM x WGN waves; a wave has BM / WGM rows and BN / WGN columns, a group every KG-th run of 32 k.  On the 16-bit
 // matrix instruction a term x w of a sum is the six products of the operands' parts that are not below 2^-25 of it: x_hi w_hi,
@@ -406,8 +478,8 @@ __device__ __forceinline__ bool parts_hold(float v) {
 // with several blocks a unit one group is as fast and meets less.  2000 x 11264 x 2048 in 128 x 128: 501 us, 184 TFLOP/s (the
 // 32-bit instruction's peak is 157, its kernel reached 128); 509 x 11264 x 2048 196 -> 150; 509 x 2560 x 2048 57 -> 41.
 template <int BM, int BN, int WGM, int WGN, int KG, int EPI>
-__global__ __launch_bounds__(64 * WGM * WGN * KG, 2) void gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, Fused f, int m, int n,
-                                                                int k, int col_blocks) {
+__global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG), WGM * WGN * KG)) void gemm_f32_tiled_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, Fused f, int m, int n, int k, int col_blocks) {
   constexpr bool kPaired = EPI == F32_SILU || EPI == F32_ROPE;
   constexpr int THREADS = 64 * WGM * WGN * KG, WM = BM / WGM, WN = BN / WGN;
   static_assert(!kPaired || WN % 32 == 0, "a wave has whole pairs of strips");
@@ -597,31 +669,48 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, 2) void gemm_f32_tiled_kernel(
       for (int j = 0; j < TN; ++j) total[i][j] += sums[(i * TN + j) * kWave];
   }
 
+  // A wave that has sums which do not stand takes their 16 rows again in 32 bits, and those sums from there: 509 x 11264 x
+  // 2048 with one row of X that is no number 212 us, with nothing else 590, without 173.  (One lane's chain for each such sum, one
+  // after the other: 3,716 and 22,655.)
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    bool stand = true;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) stand = stand && parts_hold(total[i][j][e]);
+    const int row = row0 + wave_m * WM + i * 16 + r;
+    if (row - r >= m || !__any(!stand)) continue;  // (rows beyond the end, here and below: a valid one, not stored)
+    const float* weights[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int of = weight_row(wave_n * WN + j * 16 + r);
+      weights[j] = w + (size_t)(of >= 0 && of < n ? of : 0) * k;
+    }
+    f32x4 again[TN];
+    multiply_in_32_bits<TN, 2>(x + (size_t)(row < m ? row : m - 1) * k, weights, k, again);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!parts_hold(total[i][j][e])) total[i][j][e] = again[j][e];
+  }
+
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int row = row0 + wave_m * WM + i * 16 + r;
     if (row >= m) continue;
-    auto finished = [&](int j) {
-      f32x4 v = total[i][j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (!parts_hold(v[e])) {
-          const int of = weight_row(wave_n * WN + j * 16 + g * 4 + e);
-          if (of >= 0 && of < n) v[e] = chain_of(x + (size_t)row * k, w + (size_t)of * k, k);
-        }
-      return v;
-    };
     if constexpr (kPaired) {
       TokenPlace place = {0, -1};
       if constexpr (EPI == F32_ROPE) place = place_of(f, row);
 #pragma unroll
       for (int u = 0; u < TN / 2; ++u)
-        finish_pair<EPI, 16>(f, row, place, (col0 + wave_n * WN) / 32 + u, g * 4, n, finished(2 * u), finished(2 * u + 1));
+        finish_pair<EPI, 16>(f, row, place, (col0 + wave_n * WN) / 32 + u, g * 4, n, total[i][2 * u], total[i][2 * u + 1]);
     } else {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const int column = col0 + wave_n * WN + j * 16 + g * 4;
-        f32x4 v = finished(j);
+        f32x4 v = total[i][j];
         if constexpr (EPI == F32_RESIDUAL) v += ask_columns((const float*)f.y, row, column, n);
         store_columns(f.y, EPI == F32_RESIDUAL ? (int)NNIS_F32 : f.y_dtype, row, column, n, v);
       }
@@ -638,7 +727,7 @@ void launch_few(const XT* x, const float* w, const Fused& f, int m, int n, int k
 
 template <int EPI, int BM, int BN, int WGM, int WGN, int KG>
 int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, int k, hipStream_t stream) {
-  constexpr int lds = 2 * KG * (BM + BN) * kStepK * 3 * (int)sizeof(__bf16);
+  constexpr int lds = tile_lds(BM, BN, KG);
   static_assert(lds <= 160 * 1024 && lds >= BM * BN * 4, "a compute unit has 160 KB; the groups' sums fit");
   auto kernel = gemm_f32_tiled_kernel<BM, BN, WGM, WGN, KG, EPI>;
   NNIS_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess,

@@ -146,7 +146,34 @@ def test_gemm_f32_tiles_split_any_number(k, variant):
     assert torch.equal(now[:, 9].nan_to_num(), chain[:, 9].cpu().nan_to_num()) or not now[:, 9].isfinite().any()
     rest = [r for r in range(m) if r not in (6, 7)]
     columns = [c for c in range(n) if c != 9]
-    assert torch.equal(now[rest][:, columns], got.float()[rest][:, columns])
+    # (bits: a sum whose terms are beyond the largest number with either sign is none, in both)
+    assert torch.equal(now[rest][:, columns].view(torch.int32), got.float()[rest][:, columns].view(torch.int32))
+
+
+@pytest.mark.parametrize("variant", range(4, 13))
+def test_gemm_f32_tiles_of_no_numbers_take_no_age(variant):
+    """Rows that are no numbers, and tiny sums, are multiplied again in 32 bits by the whole wave.  A product of nothing else reads
+    its operands twice and multiplies them a second time at the 32-bit instruction's rate: a few times as long as an ordinary one
+    (about 4 here), where one lane's chain for each sum took 80 to 208 times."""
+    ops = _ops()
+    torch.manual_seed(variant)
+    m, n, k = 256, 512, 2048
+    w, y = torch.randn(n, k).cuda(), torch.empty(m, n, device="cuda")
+    times = []
+    for x in (torch.randn(m, k).cuda(), torch.full((m, k), float("nan"), device="cuda"), 1e-30 * torch.randn(m, k).cuda()):
+        for _ in range(3):
+            ops.gemm_f32(x, w, y, variant)
+        best = math.inf
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                ops.gemm_f32(x, w, y, variant)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 100)
+        times.append(best)
+    assert max(times[1:]) < 10 * times[0], times
 
 
 def _f32_forms(rows, normed):
