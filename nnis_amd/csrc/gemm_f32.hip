@@ -5,7 +5,9 @@
 // and instruction j of four takes the group's j-th, so that 16 bytes a lane are 16 k of 16 rows.  For tiles with
 // v_mfma_f32_16x16x32_bf16 on operands split into three bfloat16 numbers each, whose sum they are (below).
 //
-// Nothing is rounded to fewer than 32 bits on the way.  A sum's terms come in
+// Operands enter with all their 24 bits and sums are 32-bit.  (Tiles leave the three smallest of the nine products of a term's parts
+// out: 2^-24 of the term at most, 2^-27.5 in the root mean square, what rounding it once would take; what the parts do not hold
+// goes through the 32-bit instruction.)  A sum's terms come in
 // another order than in the ordered kernel (gemm.hip), in several shorter chains (a wave's share of K, or runs of
 // kFlushSteps steps), so its error against 64 bits is smaller than the one long chain's: 509 x 2048 x 5632 of
 // normal values, root mean square error over that of the result 4.8e-7 (few rows) and 2.5e-7 (tiles; 3.0e-7 with the 32-bit
@@ -348,9 +350,12 @@ constexpr int kFlushSteps = 8;  // a chain of sums is this many steps long, then
 
 extern __shared__ __align__(16) char f32_lds[];  // two stages of BM rows of X in three parts
 
-// A 32-bit number as the sum of three of 8 significant bits: x = hi + mid + lo, exactly, wherever the last of its 24 bits
-// is at least bfloat16's smallest number (x from 2^-110 on; below, it keeps the bits that are).  Both differences are
-// exact.  A number that is none, or that rounds up to infinity, leaves parts that make its product one that is none.
+// A 32-bit number as the sum of three of 8 significant bits: x = hi + mid + lo, exactly, wherever the last of its bits is at least
+// bfloat16's smallest number, 2^-133: from 2^-110 on, and for whoever ends early.  Both differences are exact, and what lo stands
+// for has bits behind the first 16 of its word just where lo does not hold it whole: `left` collects these words, and is 0 in
+// its lower half as long as every number was the sum of its parts.  AT_ONCE: into `left` right behind the conversions; the compiler by
+// itself keeps the words to the end of a step, which takes up to 36 registers more.  A number that is none, or that rounds up to
+// infinity, leaves parts that make its product one that is none.
 template <int COUNT>
 struct Split {
   typedef __attribute__((ext_vector_type(COUNT))) __bf16 part;
@@ -362,7 +367,8 @@ __device__ __forceinline__ f32x2 widen(bf16x2 v) {
   const unsigned both = __builtin_bit_cast(unsigned, v);
   return (f32x2){__uint_as_float(both << 16), __uint_as_float(both & 0xffff0000u)};
 }
-__device__ __forceinline__ Split<4> split4(f32x4 v) {
+template <bool AT_ONCE>
+__device__ __forceinline__ Split<4> split4(f32x4 v, unsigned& left) {
   Split<4> out;
 #pragma unroll
   for (int e = 0; e < 4; e += 2) {  // (two at a time: one conversion for both)
@@ -370,7 +376,10 @@ __device__ __forceinline__ Split<4> split4(f32x4 v) {
     const bf16x2 hi = __builtin_convertvector(x, bf16x2);
     const f32x2 rest = x - widen(hi);
     const bf16x2 mid = __builtin_convertvector(rest, bf16x2);
-    const bf16x2 lo = __builtin_convertvector(rest - widen(mid), bf16x2);
+    const f32x2 last = rest - widen(mid);
+    const bf16x2 lo = __builtin_convertvector(last, bf16x2);
+    if constexpr (AT_ONCE) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(left) : "v"(last[0]), "v"(last[1]));
+    else left |= __float_as_uint(last[0]) | __float_as_uint(last[1]);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       out.hi[e + i] = hi[i];
@@ -455,19 +464,22 @@ __device__ __forceinline__ void multiply_in_32_bits(const float* row, const floa
   for (int j = 0; j < TN; ++j) total[j] += sum[j];
 }
 
-// Whether a sum of parts stands: not if it is no number or infinite, nor so small that its terms' last parts may be missing (a zero stays).
+// Whether a sum of parts stands: not if it is no number or infinite, nor so small that parts of its terms may be missing, which are no
+// numbers below 2^-149 (a zero stays).
 __device__ __forceinline__ bool parts_hold(float v) {
   const unsigned magnitude = __float_as_uint(v) & 0x7fffffffu;
   return magnitude == 0u || (magnitude >= 0x12000000u && magnitude < 0x7f800000u);  // from 2^-91 on
 }
 
-// Bytes of LDS of a tile's two stages, and the waves of a SIMD that they leave room for (and the registers have to).
-constexpr int tile_lds(int rows, int columns, int groups) { return 2 * groups * (rows + columns) * kStepK * 3 * (int)sizeof(__bf16); }
+// Bytes of LDS of a tile's two stages and of its rows' and columns' marks, and the waves of a SIMD that they leave room for (and the
+// registers have to).
+constexpr int tile_stages(int rows, int columns, int groups) { return 2 * groups * (rows + columns) * kStepK * 3 * (int)sizeof(__bf16); }
+constexpr int tile_lds(int rows, int columns, int groups) { return tile_stages(rows, columns, groups) + (rows + columns) * (int)sizeof(unsigned); }
 constexpr int tile_waves(int lds, int waves) { return 160 * 1024 / lds * waves / 4; }
 
 // KG groups of WGM x WGN waves; a wave has BM / WGM rows and BN / WGN columns, a group every KG-th run of 32 k.  On the 16-bit
-// matrix instruction a term x w of a sum is the six products of the operands' parts that are not below 2^-25 of it: x_hi w_hi,
-// x_hi w_mid, x_mid w_hi, x_mid w_mid, x_hi w_lo and x_lo w_hi, six times the work at sixteen times the 32-bit instruction's
+// matrix instruction a term x w of a sum is the six largest products of the operands' parts: x_hi w_hi,
+// x_hi w_mid, x_mid w_hi, x_mid w_mid, x_hi w_lo and x_lo w_hi (of x_mid w_lo, x_lo w_mid and x_lo w_lo none is above 2^-25 of it), six times the work at sixteen times the 32-bit instruction's
 // rate.  The block's threads split each number once, on its way into LDS, where a stage has three planes of 16 rows by 32 k; a
 // lane's 8 k of a step are the 16 bytes at k = 4 g and those at 16 + 4 g, g = l / 16, in both operands, and are read as one
 // operand.  What bounds the kernel is the sum of what a SIMD issues: a step of a wave tile of 64 x 32 is 48 matrix instructions
@@ -476,7 +488,9 @@ constexpr int tile_waves(int lds, int waves) { return 160 * 1024 / lds * waves /
 // (products of one beside reads of the other) changed it by more than 5%.  Where a block has a compute unit to itself two groups
 // share K, so that a SIMD has two waves: 509 x 2048 x 5632 in 64 x 64 114 -> 90 us (106 with the 32-bit instruction);
 // with several blocks a unit one group is as fast and meets less.  2000 x 11264 x 2048 in 128 x 128: 501 us, 184 TFLOP/s (the
-// 32-bit instruction's peak is 157, its kernel reached 128); 509 x 11264 x 2048 196 -> 150; 509 x 2560 x 2048 57 -> 41.
+// 32-bit instruction's peak is 157, its kernel reached 128); 509 x 11264 x 2048 196 -> 150; 509 x 2560 x 2048 57 -> 41.  The
+// marks of rows whose numbers are not the sum of their parts are 1 to 4% of these times (side by side, without and with: 90.9 and 94.0, 507 and 514,
+// 151 and 151, 42.8 and 43.5).
 template <int BM, int BN, int WGM, int WGN, int KG, int EPI>
 __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG), WGM * WGN * KG)) void gemm_f32_tiled_kernel(
     const float* __restrict__ x, const float* __restrict__ w, Fused f, int m, int n, int k, int col_blocks) {
@@ -512,8 +526,8 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
 
   // Rows beyond the end: a valid one, not stored.  Loads go by a base that is the same in every lane (the tile's first row; the
   // first of the 8 weight rows of a wave's load, which follow one another) and an offset in bytes, and give zeros from the base's
-  // limit on: that is where the last step's chunks beyond K are asked for, and the limit is the operand's end, which steps
-  // beyond the last reach (what they bring is not multiplied).
+  // limit on, the operand's end at most: that is where the last step's chunks beyond K are asked for, and steps beyond the last (they
+  // are not multiplied, and zeros are the sum of their parts).
   constexpr unsigned kNowhere = 0xfffffff0u;
   auto limit_of = [](size_t elements) { return elements * 4 < kNowhere ? (unsigned)(elements * 4) : kNowhere; };
   const int steps = (k + BLOCK_K - 1) / BLOCK_K, full = k / BLOCK_K;
@@ -538,11 +552,19 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
     b_from[o] = (unsigned)((row >= 0 && row < n ? row - start : 0) * k + chunk * 4) * 4u;
   }
   __bf16* stages = (__bf16*)f32_lds;
+  // which rows of X, and behind them which weight rows, hold numbers that are not the sum of their parts
+  unsigned* lossy = (unsigned*)(f32_lds + tile_stages(BM, BN, KG));
+  for (int i = threadIdx.x; i < BM + BN; i += THREADS) lossy[i] = 0u;
+  unsigned a_left[A_LOADS], b_left[B_LOADS];
+#pragma unroll
+  for (int o = 0; o < A_LOADS; ++o) a_left[o] = 0u;
+#pragma unroll
+  for (int o = 0; o < B_LOADS; ++o) b_left[o] = 0u;
 
   // (the step's place in the vector offset: the check against the limit takes no other into account for certain)
-  const bool there = full * BLOCK_K + chunk * 4 < k;  // in a last, short step
+  const int steps_there = full + (full * BLOCK_K + chunk * 4 < k ? 1 : 0);  // (a last, short one counts where this thread's chunk is in it)
   auto load = [&](__amdgpu_buffer_rsrc_t base, unsigned from, int step) {
-    const unsigned at = step != full || there ? from + (unsigned)step * (BLOCK_K * 4) : kNowhere;
+    const unsigned at = step < steps_there ? from + (unsigned)step * (BLOCK_K * 4) : kNowhere;
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(base, (int)at, 0, 0));
   };
   auto in_tile = [&](int o, int rows) { return rows % LOAD_ROWS == 0 || o * LOAD_ROWS + load_row < rows; };
@@ -557,10 +579,11 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
     for (int o = 0; o < B_LOADS; ++o)
       if (in_tile(o, BN)) v.b[o] = load(b_base[o], b_from[o], step);
   };
-  auto put = [&](f32x4 v, __bf16* to) {
+  auto put = [&](f32x4 v, __bf16* to, unsigned& left) {
     // (two groups: a step's numbers are not to be waited for, and split, together with the step's before it: 41 -> 37 us; one: 4% slower)
     if constexpr (KG > 1) asm volatile("" : "+v"(v));
-    const Split<4> parts = split4(v);
+    // (two groups have registers for it and are 3% faster without; one: 96 x 96 would keep some in scratch memory)
+    const Split<4> parts = split4<KG == 1>(v, left);
     *(bf16x4*)to = parts.hi;
     *(bf16x4*)(to + PLANE) = parts.mid;
     *(bf16x4*)(to + 2 * PLANE) = parts.lo;
@@ -569,10 +592,10 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
     __bf16* to = stages + stage * STAGE;
 #pragma unroll
     for (int o = 0; o < A_LOADS; ++o)
-      if (in_tile(o, BM)) put(v.a[o], to + place_of_row(o * LOAD_ROWS + load_row));
+      if (in_tile(o, BM)) put(v.a[o], to + place_of_row(o * LOAD_ROWS + load_row), a_left[o]);
 #pragma unroll
     for (int o = 0; o < B_LOADS; ++o)
-      if (in_tile(o, BN)) put(v.b[o], to + BM / 16 * TILE + place_of_row(o * LOAD_ROWS + load_row));
+      if (in_tile(o, BN)) put(v.b[o], to + BM / 16 * TILE + place_of_row(o * LOAD_ROWS + load_row), b_left[o]);
   };
 
   f32x4 sum[TM][TN], total[TM][TN];
@@ -651,10 +674,17 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
   }
   if (step < steps) one_step(step, raw[1], 0);
 #pragma unroll
+  for (int o = 0; o < A_LOADS; ++o)
+    if (in_tile(o, BM) && (a_left[o] & 0xffffu)) lossy[o * LOAD_ROWS + load_row] = 1u;
+#pragma unroll
+  for (int o = 0; o < B_LOADS; ++o)
+    if (in_tile(o, BN) && (b_left[o] & 0xffffu)) lossy[BM + o * LOAD_ROWS + load_row] = 1u;
+  meet();
+#pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) total[i][j] += sum[i][j];
-  if constexpr (KG > 1) {  // the groups' sums meet in LDS (all reads of the stages are behind the last barrier)
+  if constexpr (KG > 1) {  // the groups' sums meet in LDS (all reads of the stages are behind the barrier)
     f32x4* sums = (f32x4*)f32_lds + (size_t)(wave % (WGM * WGN)) * TM * TN * kWave + lane;
     if (k_group != 0)
 #pragma unroll
@@ -669,31 +699,37 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG, tile_waves(tile_lds(BM, BN, KG
       for (int j = 0; j < TN; ++j) total[i][j] += sums[(i * TN + j) * kWave];
   }
 
-  // A wave that has sums which do not stand takes their 16 rows again in 32 bits, and those sums from there: 509 x 11264 x
-  // 2048 with one row of X that is no number 212 us, with nothing else 590, without 173.  (One lane's chain for each such sum, one
-  // after the other: 3,716 and 22,655.)
+  // A wave that has sums which do not stand, or rows or columns of numbers that are not the sum of their parts, takes their 16 rows
+  // again in 32 bits, and those sums from there: 509 x 11264 x 2048 with one row of X that is no number 212 us, with nothing
+  // else 590, without 173.  (One lane's chain for each such sum, one after the other: 3,716 and 22,655.)
+  static_assert(TN * 4 <= 32, "a bit for each of a lane's sums of a row");
+  unsigned lossy_columns = 0u;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) lossy_columns |= lossy[BM + wave_n * WN + j * 16 + g * 4 + e] << (j * 4 + e);
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    bool stand = true;
+    unsigned again = lossy[wave_m * WM + i * 16 + r] ? ~0u : lossy_columns;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) stand = stand && parts_hold(total[i][j][e]);
+      for (int e = 0; e < 4; ++e) again |= (parts_hold(total[i][j][e]) ? 0u : 1u) << (j * 4 + e);
     const int row = row0 + wave_m * WM + i * 16 + r;
-    if (row - r >= m || !__any(!stand)) continue;  // (rows beyond the end, here and below: a valid one, not stored)
+    if (row - r >= m || !__any(again)) continue;  // (rows beyond the end, here and below: a valid one, not stored)
     const float* weights[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int of = weight_row(wave_n * WN + j * 16 + r);
       weights[j] = w + (size_t)(of >= 0 && of < n ? of : 0) * k;
     }
-    f32x4 again[TN];
-    multiply_in_32_bits<TN, 2>(x + (size_t)(row < m ? row : m - 1) * k, weights, k, again);
+    f32x4 sums[TN];
+    multiply_in_32_bits<TN, 2>(x + (size_t)(row < m ? row : m - 1) * k, weights, k, sums);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (!parts_hold(total[i][j][e])) total[i][j][e] = again[j][e];
+        if (again >> (j * 4 + e) & 1u) total[i][j][e] = sums[j][e];
   }
 
 #pragma unroll

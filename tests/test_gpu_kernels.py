@@ -113,10 +113,9 @@ def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
 @pytest.mark.parametrize("k", [36, 100, 612])
 def test_gemm_f32_tiles_split_any_number(k, variant):
     """The tiles multiply the bfloat16 parts that a 32-bit number is the sum of.  Rows of every magnitude come out as
-    accurate as ordinary ones: the bound as above, the smallest 32-bit number for each product that falls below it, and
-    what a last part below bfloat16's smallest number, 2^-133, may lack, half of that times the other operand (which
-    only a far larger other operand lets anyone see; small sums are taken again).  Numbers that are none and sums beyond the largest number come out where the 32-bit chain has them, in their rows and
-    columns alone."""
+    accurate as ordinary ones: the bound as above, and the smallest 32-bit number for each product that falls below
+    it.  Numbers that are none and sums beyond the largest number come out where the 32-bit chain has them, in their
+    rows and columns alone."""
     ops = _ops()
     torch.manual_seed(k)
     m, n = 70, 65
@@ -132,7 +131,7 @@ def test_gemm_f32_tiles_split_any_number(k, variant):
     y = torch.empty(m, n, device="cuda")
     ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
     got = y.cpu().double()
-    scale = 2e-7 * math.sqrt(k) * scale + 1.5e-45 * k + 2.0 ** -134 * (x.double().abs().sum(1)[:, None] + w.double().abs().sum(1))
+    scale = 2e-7 * math.sqrt(k) * scale + 1.5e-45 * k
     fits = scale < 3.4e38 * 2e-7  # (a sum of terms beyond it may be infinite, or cancel, in one order and not in another)
     bad = ((got - want).abs() > scale) & fits
     assert not bad.any() and (got[5] == 0).all(), (bad.nonzero()[:8], (got - want)[bad][:8], scale[bad][:8], want[bad][:8])
@@ -148,6 +147,32 @@ def test_gemm_f32_tiles_split_any_number(k, variant):
     columns = [c for c in range(n) if c != 9]
     # (bits: a sum whose terms are beyond the largest number with either sign is none, in both)
     assert torch.equal(now[rest][:, columns].view(torch.int32), got.float()[rest][:, columns].view(torch.int32))
+
+
+@pytest.mark.parametrize("variant", range(4, 13))
+@pytest.mark.parametrize("m, n, k", [(70, 65, 4), (129, 130, 100), (64, 64, 612)])
+def test_gemm_f32_tiles_keep_every_bit_of_tiny_factors(m, n, k, variant):
+    """Numbers below 2^-110 are not the sum of their bfloat16 parts, and below 2^-134 all of these are zero: times large numbers they
+    come out as accurate as any others, on either side, and change no other row or column."""
+    ops = _ops()
+    torch.manual_seed(k)
+    x, w = torch.randn(m, k), torch.randn(n, k)
+    y, plain = torch.empty(m, n, device="cuda"), torch.empty(m, n, device="cuda")
+    ops.gemm_f32(x.cuda(), w.cuda(), plain, variant)
+    for row, magnitude in ((0, -112), (17, -118), (38, -126), (62, -135), (m - 1, -142)):
+        x[row] *= 2.0 ** magnitude
+    for column, magnitude in ((1, 40), (20, 70), (39, 110), (50, -114), (n - 1, -130)):
+        w[column] *= 2.0 ** magnitude
+    x[40, 1:], x[40, 0], w[40, 1:], w[40, 0] = 0.0, 4e-41, 0.0, 1e20  # (one term, whose sum of parts is zero)
+    x[41, 1:], x[41, 0] = 0.0, 3e35
+    want, scale = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
+    error = (y.cpu().double() - want).abs()
+    bad = (error > 2e-7 * math.sqrt(k) * scale + 1.5e-45 * k) & (scale < 3e38)  # (row 41 beside the large columns is beyond the largest number)
+    assert not bad.any(), (bad.nonzero()[:8], error[bad][:8], want[bad][:8])
+    rows = [r for r in range(m) if r not in (0, 17, 38, 62, m - 1, 40, 41)]
+    columns = [c for c in range(n) if c not in (1, 20, 39, 50, n - 1, 40)]
+    assert torch.equal(y[rows][:, columns], plain[rows][:, columns])
 
 
 @pytest.mark.parametrize("variant", range(4, 13))
