@@ -1569,9 +1569,10 @@ def test_gla_single_tokens(batch, heads, d, e, dtype):
 
 
 @pytest.mark.parametrize("width", [1028, 2048, 4096, 5000, 8192])
-@pytest.mark.parametrize("count", [1, 5, 1023, 1024])
+@pytest.mark.parametrize("count", [1, 5, 1023, 1024, 2046])
 def test_rmsnorm_of_few_rows(width, count):
-    """Rows that a block each norms (up to 1,023) and rows that a wave each does: with a row list, with a sum written back, with
+    """Rows that a block each norms (up to 1,023) and rows that a wave each does, with the weight asked for beside the row (up to 2,048; the
+    last count has 2,049 without a row list) and behind its sum: with a row list, with a sum written back, with
     both, in both types; the last rows of the list out of order."""
     ops = _ops()
     torch.manual_seed(width + count)
