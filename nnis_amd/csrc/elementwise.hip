@@ -49,7 +49,11 @@ extern "C" int nnis_embed(const int* ids, const void* table, int table_dtype, fl
   NNIS_REQUIRE(nnis_dtype_ok(table_dtype), "embed: unknown table dtype %d", table_dtype);
   NNIS_REQUIRE(tokens >= 0 && width > 0 && vocab > 0, "embed: bad sizes tokens=%d width=%d vocab=%d", tokens, width, vocab);
   if (tokens == 0) return 0;
-  hipLaunchKernelGGL(embed_kernel, dim3(tokens), dim3(width >= 2048 ? 512 : 256), 0, (hipStream_t)stream, ids, table, table_dtype, out,
+  // a thread for every four channels, up to 512 (16,384 rows of 64 channels: 6.1 us, in blocks of 256 threads 7.4); where channels are copied one
+  // at a time 256, and 512 for wide rows that are few (2,050 channels of 16 bits, 200 rows 3.7 us with 256 and 3.3 with 512, 16,384 rows 36.4 and 41.0)
+  const bool fours = width % 4 == 0 && ((uintptr_t)table | (uintptr_t)out) % 16 == 0;
+  const int threads = fours ? (width >= 2048 ? 512 : (width + 255) / 256 * 64) : (width >= 2048 && tokens < 1024 ? 512 : 256);
+  hipLaunchKernelGGL(embed_kernel, dim3(tokens), dim3(threads), 0, (hipStream_t)stream, ids, table, table_dtype, out,
                      width, vocab, scale);
   NNIS_LAUNCH_CHECK("embed");
   return 0;

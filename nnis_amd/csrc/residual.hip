@@ -82,7 +82,11 @@ extern "C" int nnis_embed_pair(const int* ids, const int* tok_slot, const int* t
   NNIS_REQUIRE(mul_prev >= 0 && mul_cur >= 0, "embed_pair: the multipliers must not be negative");
   NNIS_REQUIRE(ids && tok_slot && tok_pos && last_token && out, "embed_pair: a pointer is missing");
   if (tokens == 0) return 0;
-  hipLaunchKernelGGL(embed_pair_kernel, dim3(tokens), dim3(width >= 2048 ? 512 : (width >= 1024 ? 256 : 64)), 0, (hipStream_t)stream, ids, tok_slot,
+  const bool fours = width % 4 == 0 && ((uintptr_t)table | (uintptr_t)pairs | (uintptr_t)out) % 16 == 0;
+  // (wide rows whose channels are copied one at a time: 512 threads while they are few; 2,050 channels, 200 rows 4.7 us with 256 and 4.1 with
+  // 512, 16,384 rows of 16 bits 91.7 and 95.0)
+  const int threads = width >= 2048 && (fours || tokens < 1024) ? 512 : (width >= 1024 ? 256 : 64);
+  hipLaunchKernelGGL(embed_pair_kernel, dim3(tokens), dim3(threads), 0, (hipStream_t)stream, ids, tok_slot,
                      tok_pos, tokens, table, table_dtype, vocab, pairs, pairs_dtype, buckets, mul_prev, mul_cur, last_token, out,
                      copies, width);
   NNIS_LAUNCH_CHECK("embed_pair");

@@ -1617,6 +1617,26 @@ def test_embeddings_four_channels_at_a_time(width, shift, dtype):
     assert torch.equal(both.cpu(), want.expand(3, 5, width))
 
 
+@pytest.mark.parametrize("count", [1023, 1024])
+@pytest.mark.parametrize("width", [64, 260, 2050, 2052])
+def test_embeddings_of_many_rows(width, count):
+    """The blocks that few and many rows take, for widths of less than a wave's channels, a few more than one wave's, and wide ones whose
+    channels are copied four and one at a time."""
+    ops = _ops()
+    torch.manual_seed(width)
+    table, pairs = torch.randn(50, width), torch.randn(4, width)
+    ids = torch.randint(-1, 51, (count,), dtype=torch.int32)
+    known = ((ids >= 0) & (ids < 50))[:, None]
+    out = torch.full((count + 1, width), 9.0, device="cuda")
+    ops.embed(ids.cuda(), table.cuda(), out[:count], scale=0.5)
+    assert torch.equal(out[:count].cpu(), torch.where(known, table[ids.clamp(0, 49).long()] * 0.5, 0.0)) and (out[count] == 9).all()
+    both = torch.full((2, count, width), 9.0, device="cuda")
+    slots = torch.zeros(count, dtype=torch.int32)
+    ops.embed_pair(ids.cuda(), slots.cuda(), slots.cuda(), table.cuda(), pairs.cuda(), 3, 5, _i32([-1] * 4), both)  # (each at position 0)
+    want = torch.where(known, table[ids.clamp(0, 49).long()] + pairs[3], 0.0)
+    assert torch.equal(both.cpu(), want.expand(2, count, width))
+
+
 @pytest.mark.parametrize("kernel, heads, kv_heads", [("columns", 16, 2), ("keys", 9, 3)])
 @pytest.mark.parametrize("splits, waves", [(1, 4), (2, 2), (8, 4), (1, 1)])
 def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves):
