@@ -1637,6 +1637,26 @@ def test_embeddings_of_many_rows(width, count):
     assert torch.equal(both.cpu(), want.expand(2, count, width))
 
 
+@pytest.mark.parametrize("rows", [255, 256])
+@pytest.mark.parametrize("streams, width", [(2, 36), (4, 2048), (5, 4096), (2, 4100)])
+def test_streams_of_few_and_many_rows(streams, width, rows):
+    """Rows whose norm's vectors come beside them (up to 255, up to 4,096 channels) and behind their sums, after an update: streams and
+    norms against 64 bits, a few roundings of the largest terms."""
+    ops = _ops()
+    torch.manual_seed(width)
+    x, y, mix, gain, take = torch.randn(streams, rows, width), torch.randn(rows, width), torch.randn(streams, streams), torch.randn(streams), torch.rand(streams) + 0.5
+    w, b = 1 + 0.2 * torch.randn(width), torch.randn(width)
+    want = torch.einsum("st,srw->trw", mix.double(), x.double()) + gain.double()[:, None, None] * y.double()
+    read = (take.double()[:, None, None] * want).sum(0)
+    centred = read - read.mean(1, keepdim=True)
+    normed = centred / torch.sqrt((centred * centred).mean(1, keepdim=True) + 1e-5) * w.double() + b.double()
+    held, h = x.cuda(), torch.full((rows, width), 9.0, device="cuda")
+    ops.stream_step(held, h, y.cuda(), mix.cuda(), gain.cuda(), take.cuda(), w.cuda(), b.cuda(), 1e-5)
+    size = torch.einsum("st,srw->trw", mix.double().abs(), x.double().abs()) + gain.double().abs()[:, None, None] * y.double().abs()
+    assert ((held.cpu().double() - want).abs() <= 1e-6 * size).all()
+    assert ((h.cpu().double() - normed).abs() <= 2e-5 * (1 + normed.abs())).all()
+
+
 @pytest.mark.parametrize("kernel, heads, kv_heads", [("columns", 16, 2), ("keys", 9, 3)])
 @pytest.mark.parametrize("splits, waves", [(1, 4), (2, 2), (8, 4), (1, 1)])
 def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves):
