@@ -1657,6 +1657,45 @@ def test_streams_of_few_and_many_rows(streams, width, rows):
     assert ((h.cpu().double() - normed).abs() <= 2e-5 * (1 + normed.abs())).all()
 
 
+@pytest.mark.parametrize("rows", [5, 1023, 1024])
+@pytest.mark.parametrize("q_rank, kv_rank, rot, gates", [(224, 64, 32, 16), (0, 72, 16, 3), (40, 208, 0, 0)])
+def test_latents_of_few_and_many_rows(q_rank, kv_rank, rot, gates, rows):
+    """A channel a thread (up to 1,023 rows) and fewer threads, for latents whose widths the two part: query latent, cached latent and
+    rotated channels, gates against 64 bits; a row without a slot leaves the cache as it was."""
+    ops = _ops()
+    torch.manual_seed(q_rank + kv_rank)
+    proj = torch.randn(rows, q_rank + kv_rank + rot + gates)
+    q_weight, c_weight = 1 + 0.2 * torch.randn(q_rank), 1 + 0.2 * torch.randn(kv_rank)
+    angle = torch.rand(rows, rot // 2) * 6
+    pages = (rows + 63) // 64
+    k_pages, v_pages = _empty_pages(pages, 1, kv_rank + rot, torch.float32, 7.0, 7.0, "cuda")[0], _empty_pages(pages, 1, kv_rank, torch.float32, 7.0, 7.0, "cuda")[1]
+    slots = torch.zeros(rows, dtype=torch.int32)
+    slots[3] = -1
+    cq = torch.full((rows, q_rank), 9.0, device="cuda") if q_rank else None
+    gate = torch.full((rows, gates), 9.0, device="cuda") if gates else None
+    ops.latent_prepare(proj.cuda(), q_rank, kv_rank, rot, gates, q_weight.cuda() if q_rank else None, c_weight.cuda(), 1e-5,
+                       angle.cos().cuda() if rot else None, angle.sin().cuda() if rot else None, slots.cuda(), _i32(range(rows)), cq, k_pages, v_pages,
+                       torch.arange(pages, dtype=torch.int32).flip(0)[None].cuda(), gate)
+    def normed(x, w):
+        return x.double() / torch.sqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5) * w.double()
+
+    latent = normed(proj[:, q_rank:q_rank + kv_rank], c_weight)
+    u, v = proj[:, q_rank + kv_rank:q_rank + kv_rank + rot].double().view(rows, rot // 2, 2).unbind(2)
+    cos, sin = angle.cos().double(), angle.sin().double()
+    keys = torch.cat([latent, torch.stack([u * cos - v * sin, v * cos + u * sin], 2).view(rows, rot)], 1)
+    held_k = k_pages.cpu().view(pages, -1)[:, _k_index(kv_rank + rot)].flip(0).reshape(pages * 64, -1)
+    held_v = v_pages.cpu().view(pages, -1)[:, _v_index(kv_rank)].flip(0).reshape(pages * 64, -1)
+    kept = [r for r in range(rows) if r != 3]
+    assert ((held_k[:rows] - keys).abs()[kept] <= 2e-6 * (1 + keys.abs()[kept])).all() and ((held_v[:rows] - latent).abs()[kept] <= 2e-6 * (1 + latent.abs()[kept])).all()
+    assert (held_k[3] == 7).all() and (held_k[rows:] == 7).all() and (held_v[rows:] == 7).all()
+    if q_rank:
+        want = normed(proj[:, :q_rank], q_weight)
+        assert ((cq.cpu().double() - want).abs() <= 2e-6 * (1 + want.abs())).all()
+    if gates:
+        want = torch.sigmoid(proj[:, -gates:].double())
+        assert ((gate.cpu().double() - want).abs() <= 1e-6).all()
+
+
 @pytest.mark.parametrize("kernel, heads, kv_heads", [("columns", 16, 2), ("keys", 9, 3)])
 @pytest.mark.parametrize("splits, waves", [(1, 4), (2, 2), (8, 4), (1, 1)])
 def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves):
