@@ -1555,6 +1555,7 @@ def decode_plan(batch: int, kv_heads: int, longest: int, max_waves: int = 4, wid
 # against 13.3), from 1,536 on all three are (9/3: 14.9 against 22.9 with two columns).  Whole prompt steps, ms:
 # TinyLlama shape 128 / 1,024 tokens 1.68 / 4.31 -> 1.60 / 4.19, 135M shape 128 / 256 1.04 / 1.32 -> 0.99 / 1.23.
 PREFILL_MANY_ROWS = 65536  # rows x query heads from which a step has work items enough for the widest tiles
+PREFILL_NARROW_MOST = 4096  # ... up to which short prompts of 65 to 128 channels have items of one column
 PREFILL_SOME_ROWS = 16384  # ... from which a step of 1,024 to 1,279 tokens still gains by two columns
 # Items of four columns (up to 64 channels, any group but 3) merge the states of 8 waves through 72 KB of LDS: worth it
 # while a step's items are few (16 heads of 64 at 2,048 tokens 26 us a layer against 37 with 4 waves, 16/4 heads of 48
@@ -1596,8 +1597,11 @@ def prefill_plan(longest: int, rows: int, heads: int, head_dim: int = 64, kv_hea
     # A short prompt's items are few and each hangs on its first trips to memory: one column an item.  Whole prompt steps, us, widest
     # items and these: 135M shape 24 / 64 / 100 tokens 776 / 804 / 999 -> 748 / 761 / 912, 8 of 100 1,525 -> 1,450; TinyLlama shape 1,322 /
     # 1,339 / 1,679 -> 1,274 / 1,276 / 1,587, 24 of 120 7,012 -> 7,045; 1.7B shape 100 tokens 2,001 -> 1,897, 24 of 120 equal: with
-    # items enough they stay wide.  (Two waves an item gain 1% more from 65 rows on, and lose 1% below.)
-    if plan_class == 0 and kv_heads and size < PREFILL_MANY_ROWS:
+    # items enough they stay wide.  (Two waves an item gain 1% more from 65 rows on, and lose 1% below.)  The attention alone, us a layer,
+    # widest items and these: 32/8 heads of 64, prompts of 100 tokens, 51,200 rows x heads 14.6 -> 10.5, 65,024 15.4 -> 10.8, 102,400 15.9 -> 21.8.
+    # Of 65 to 128 channels the items of two columns fill the chip sooner: 32/8 heads of 128, 4,064 rows x heads 7.5 -> 5.8, 4,096 5.5 -> 4.6, but 6,144
+    # (prompts of 24 tokens) 4.9 -> 6.2, 8,192 5.6 -> 6.7, 65,024 16.7 -> 20.0.  Beyond 128 channels every item has one column.
+    if plan_class == 0 and kv_heads and (size <= PREFILL_NARROW_MOST if 64 < head_dim <= 128 else size < PREFILL_MANY_ROWS):
         return 1, 1
     waves = (1, 2, 4, 8, 8)[plan_class]
     if waves == 8 and head_dim <= 64 and group != 3 and size > PREFILL_EIGHT_WAVES_MOST:

@@ -176,3 +176,13 @@ def test_prefill_plans_of_short_prompts(heads, kv_heads, head_dim):
         assert prefill_plan(longest, 64, heads, head_dim, kv_heads) == prefill_plan(longest, 128, heads, head_dim, kv_heads) == (1, 1)
         assert prefill_plan(longest, 65536, heads, head_dim, kv_heads) == (1, 0)
     assert prefill_plan(128, 128, heads, head_dim, kv_heads) == (2, 1)
+
+
+@pytest.mark.parametrize("heads, kv_heads, head_dim", [(16, 4, 128), (32, 8, 96), (8, 8, 80)])
+def test_prefill_plans_of_short_prompts_of_wide_heads(heads, kv_heads, head_dim):
+    """Heads of 65 to 128 channels: items of one column up to 4,096 rows x heads, where they still find compute units without a block."""
+    from nnis_amd.kernels.ops import prefill_plan
+
+    most = 4096 // heads
+    assert prefill_plan(100, most, heads, head_dim, kv_heads) == prefill_plan(1, 64, heads, head_dim, kv_heads) == (1, 1)
+    assert prefill_plan(100, most + 1, heads, head_dim, kv_heads) == prefill_plan(24, 65024 // heads, heads, head_dim, kv_heads) == (1, 0)
