@@ -1567,7 +1567,7 @@ PREFILL_EIGHT_WAVES_MOST = 40960
 def prefill_plan(longest: int, rows: int, heads: int, head_dim: int = 64, kv_heads: int = 0):
     """(waves of a block, column option) of the prefill attention for a step of ``rows`` rows (what the engine
     plans for: a step's tokens rounded up as a replayed step's are) whose longest sequence has ``longest``
-    (``kv_heads``: 0 for as many as ``heads``, and for the widest items of a short prompt)."""
+    (``kv_heads``: 0 for as many as ``heads``)."""
     plan_class = prefill_plan_class(longest)
     size = rows * heads
     # A step with work items for about twice the waves that the chip holds (two a SIMD up to 64 channels, one
@@ -1601,7 +1601,7 @@ def prefill_plan(longest: int, rows: int, heads: int, head_dim: int = 64, kv_hea
     # widest items and these: 32/8 heads of 64, prompts of 100 tokens, 51,200 rows x heads 14.6 -> 10.5, 65,024 15.4 -> 10.8, 102,400 15.9 -> 21.8.
     # Of 65 to 128 channels the items of two columns fill the chip sooner: 32/8 heads of 128, 4,064 rows x heads 7.5 -> 5.8, 4,096 5.5 -> 4.6, but 6,144
     # (prompts of 24 tokens) 4.9 -> 6.2, 8,192 5.6 -> 6.7, 65,024 16.7 -> 20.0.  Beyond 128 channels every item has one column.
-    if plan_class == 0 and kv_heads and (size <= PREFILL_NARROW_MOST if 64 < head_dim <= 128 else size < PREFILL_MANY_ROWS):
+    if plan_class == 0 and (size <= PREFILL_NARROW_MOST if 64 < head_dim <= 128 else size < PREFILL_MANY_ROWS):
         return 1, 1
     waves = (1, 2, 4, 8, 8)[plan_class]
     if waves == 8 and head_dim <= 64 and group != 3 and size > PREFILL_EIGHT_WAVES_MOST:

@@ -57,7 +57,7 @@ def test_prefill_plan_by_class_and_size():
     assert [prefill_rows(n) for n in (1, 64, 65, 1024, 1025, 2048, 2049, 4000)] == [64, 64, 128, 1024, 1152, 2048, 2304, 4096]
     for n in (1, 64, 100, 1000, 1100, 2000, 3000):
         assert prefill_rows(prefill_rows(n)) == prefill_rows(n)  # a step replayed from a graph's rows plans as the step launched
-    assert prefill_plan(100, 100, 9) == (1, 0)
+    assert prefill_plan(100, 100, 9) == prefill_plan(100, 100, 9, 64, 9) == (1, 1)  # (short prompts: items of one column, however the key heads are given)
     assert prefill_plan(300, 300, 9) == (2, 1)
     assert prefill_plan(700, 700, 9) == (4, 2)
     assert prefill_plan(1024, 1024, 32) == (4, 2) and prefill_plan(1024, 1024, 9) == (8, 0)
