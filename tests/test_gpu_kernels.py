@@ -114,8 +114,8 @@ def test_gemm_f32_on_the_matrix_cores(m, n, k, variant):
 def test_gemm_f32_tiles_split_any_number(k, variant):
     """The tiles multiply the bfloat16 parts that a 32-bit number is the sum of.  Rows of every magnitude come out as
     accurate as ordinary ones: the bound as above, and the smallest 32-bit number for each product that falls below
-    it.  Numbers that are none and sums beyond the largest number come out where the 32-bit chain has them, in their
-    rows and columns alone."""
+    it.  Rows and columns with infinities and numbers that are none come out as the 32-bit chain has them, and change
+    nothing beside them."""
     ops = _ops()
     torch.manual_seed(k)
     m, n = 70, 65
@@ -139,10 +139,11 @@ def test_gemm_f32_tiles_split_any_number(k, variant):
     ops.gemm_f32(x.cuda(), w.cuda(), y, variant)
     now, chain = y.cpu(), torch.empty(m, n, device="cuda")
     ops.gemm_ordered(x.cuda(), w.cuda(), chain)
-    for row in (6, 7):
-        assert torch.equal(now[row].isnan(), chain[row].cpu().isnan()) and torch.equal(now[row].isinf(), chain[row].cpu().isinf())
-        assert torch.equal(now[row].sign()[now[row].isinf()], chain[row].cpu().sign()[now[row].isinf()])
-    assert torch.equal(now[:, 9].nan_to_num(), chain[:, 9].cpu().nan_to_num()) or not now[:, 9].isfinite().any()
+    chain = chain.cpu()
+    for got_line, want_line in ((now[6], chain[6]), (now[7], chain[7]), (now[:, 9], chain[:, 9])):
+        assert torch.equal(got_line.isnan(), want_line.isnan()) and torch.equal(got_line.isinf(), want_line.isinf())
+        assert torch.equal(got_line.sign()[got_line.isinf()], want_line.sign()[got_line.isinf()])
+    assert not now[:, 9].isfinite().any()
     rest = [r for r in range(m) if r not in (6, 7)]
     columns = [c for c in range(n) if c != 9]
     # (bits: a sum whose terms are beyond the largest number with either sign is none, in both)
@@ -742,7 +743,7 @@ def test_residual_projection_with_two_blocks_a_strip(m, n, k):
 
 
 @pytest.mark.parametrize("tile", ["TILE_64x128", "TILE_64x64", "TILE_256x256", "TILE_256x192", "TILE_128x128", "TILE_256x128", "TILE_128x192"])
-@pytest.mark.parametrize("m, n, k", [(70, 600, 136), (530, 300, 72), (300, 1100, 584)])
+@pytest.mark.parametrize("m, n, k", [(70, 600, 136), (530, 300, 72), (300, 1100, 584), (300, 1100, 1800), (70, 600, 1992)])
 def test_residual_projection_with_every_tile(tile, m, n, k):
     """The tiled kernel's residual epilogue with each tile shape (several row
     and column blocks, ragged edges): the stream, the prepared operand and the
@@ -1719,14 +1720,123 @@ def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves
         assert (out.cpu().float().view(len(rows), heads, head_dim) - want).abs().max().item() <= 1e-2
 
 
-@pytest.mark.parametrize("m, n, k", [(70, 576, 576), (128, 700, 1024), (128, 576, 1032), (65, 576, 1208), (130, 2048, 1792), (130, 2000, 1832)])
-def test_products_around_the_k_from_which_it_goes_in_parts(m, n, k):
-    """Products whose K is just too short to go in two, four or eight parts, and just long enough: against 64 bits, and the
-    parts' own rows, as ops.linear and into the stream."""
+# the four-wave tiles: their hint to the products, their columns
+FOUR_WAVE_TILES = [(48, 64), (32, 128)]
+
+
+def _tiled_parts(m, n, k, columns):
+    """Parts of K of a product in tiles of 64 rows: the rule of the kernels' launch, written once more."""
+    col_blocks, steps = -(-n // columns), -(-k // 64)
+    tiles, parts = col_blocks * -(-m // 64), 1
+    while parts < 8 and tiles * parts * 2 <= 256 and steps // (parts * 2) >= 4:
+        parts *= 2
+    while parts > 1 and parts * m * col_blocks * columns * 4 > _ops().GEMM_WORKSPACE_BYTES:
+        parts //= 2
+    return parts if k - k // parts >= 900 else 1
+
+
+class _PartsOfK:
+    """Sees by the workspace in how many parts of ``size`` sums the product inside went (1: K whole, nothing written)."""
+
+    def __init__(self, size):
+        ops = _ops()
+        self.size, self.workspace = size, ops._gemm_workspace(torch.device("cuda", torch.cuda.current_device()))[:ops.GEMM_WORKSPACE_BYTES // 4]
+
+    def __enter__(self):
+        self.workspace.fill_(-7.5e33)
+        return self
+
+    def __exit__(self, *error):
+        written = (self.workspace != -7.5e33).nonzero()
+        self.parts = 1 if written.numel() == 0 else written.max().item() // self.size + 1
+        self.workspace.zero_()
+
+
+# sizes whose tiles of 64 x 64 leave room for 2, 4 and 8 parts: a K just too short for them, and just long enough
+PARTS_OF_K = {(130, 2000, 1792): 1, (130, 2000, 1800): 2, (300, 1500, 1800): 2, (70, 1900, 1192): 1, (70, 1900, 1200): 4, (19, 130, 1200): 4, (70, 500, 1984): 4,
+              (70, 500, 1992): 8}
+
+
+@pytest.mark.parametrize("hint, columns", FOUR_WAVE_TILES)
+@pytest.mark.parametrize("m, n, k", list(PARTS_OF_K))
+def test_products_around_the_k_from_which_it_goes_in_parts(m, n, k, hint, columns):
+    """Products whose K is just too short to go in two, four or eight parts, and just long enough: stored and into the stream, with
+    the sums of squares that either leaves, against 64 bits; that K went in so many parts, or whole, shows in the workspace."""
     ops = _ops()
     torch.manual_seed(m + k)
     x, w = torch.randn(m, k).bfloat16(), (torch.randn(n, k) / math.sqrt(k)).bfloat16()
     want, scale = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
-    y = torch.full((m + 1, n), 7.0, device="cuda")
-    ops.linear(x.cuda(), ops.pack_weight(w.cuda()), y[:m])
-    assert ((y[:m].cpu().double() - want).abs() <= 2e-7 * math.sqrt(k) * scale + 1e-6).all() and (y[m] == 7).all()
+    parts, width = _tiled_parts(m, n, k, columns), -(-n // columns) * columns
+    assert columns != 64 or parts == PARTS_OF_K[m, n, k]
+    packed = ops.pack_weight(w.cuda())
+    for dtype, bound in ((torch.float32, 2e-7 * math.sqrt(k) * scale + 1e-6), (torch.bfloat16, 2.0 ** -8 * want.abs() + 1e-5)):
+        y = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
+        with _PartsOfK(m * width) as seen:
+            ops.gemm_bf16(x.cuda(), packed, y[:m], hint)
+        assert seen.parts == parts
+        assert ((y[:m].cpu().double() - want).abs() <= bound).all() and (y[m] == 7).all()
+    resid, gain = torch.randn(m, n) * 2, (1 + 0.3 * torch.randn(n)).bfloat16()
+    held, scaled = resid.cuda(), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ss = torch.full((ops.gemm_residual_parts(m, n) + 1, m), 7.0, device="cuda")
+    with _PartsOfK(m * width) as seen:
+        squares = ops.gemm_residual(x.cuda(), packed, held, gain.cuda(), scaled, ss, hint // 16)
+    assert seen.parts == parts
+    each = 64 if parts > 1 else columns // 2
+    assert squares == (-(-n // 64) if parts > 1 else 2 * -(-n // columns)) and (ss[squares:] == 7).all()
+    got = held.cpu().double()
+    assert ((got - resid.double() - want).abs() <= 2e-7 * math.sqrt(k) * scale + 2e-6).all()
+    assert torch.equal(scaled.cpu(), (held.cpu() * gain.float()).bfloat16())
+    for part in range(squares):
+        of = got[:, part * each:(part + 1) * each].pow(2).sum(dim=1)
+        assert ((ss[part].cpu().double() - of).abs() <= 1e-5 * (1e-3 + of)).all(), part
+
+
+@pytest.mark.parametrize("hint, columns", FOUR_WAVE_TILES)
+@pytest.mark.parametrize("m, k", [(65, 1200), (19, 1992), (130, 2304)])
+def test_scaled_projection_with_k_in_parts(m, k, hint, columns):
+    """The epilogues of products behind a prepared norm -- stored, gated, rotated with the write into the cache -- where K goes in
+    parts, whose sums a kernel behind the product adds up: against the plain functions one after another."""
+    ops = _ops()
+    torch.manual_seed(hint + m + k)
+    eps = 1e-5
+    scaled = torch.randn(m, k).bfloat16()
+    ss = (torch.rand(3, m) + 0.1) * k
+    normed = scaled.double() / torch.sqrt(ss.double().sum(0) / k + eps)[:, None]
+
+    def run(w, y, epilogue, covered, rope=None):  # (covered: weight rows that the grid has tiles for)
+        with _PartsOfK(m * -(-covered // columns) * columns) as seen:
+            ops.gemm_scaled(scaled.cuda(), ss.cuda(), 3, eps, ops.pack_weight(w.cuda()), y, epilogue, rope, hint)
+        assert seen.parts == _tiled_parts(m, covered, k, columns) > 1
+        return y.cpu().double()
+
+    def close(got, want, what):
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), (what, (got - want).abs().max().item())
+
+    n = 300
+    w = (torch.randn(n, k) / math.sqrt(k)).bfloat16()
+    close(run(w, torch.empty(m, n, dtype=torch.bfloat16, device="cuda"), ops.EPILOGUE_STORE, n), normed @ w.double().t(), "store")
+    inner = 200
+    w = (torch.randn(2 * inner, k) / math.sqrt(k)).bfloat16()
+    both = normed @ w.double().t()
+    close(run(w, torch.empty(m, inner, dtype=torch.bfloat16, device="cuda"), ops.EPILOGUE_SILU, 32 * -(-inner // 16)), P.silu(both[:, :inner]) * both[:, inner:], "silu")
+    heads, kv_heads, head_dim = 5, 2, 64
+    n = (heads + 2 * kv_heads) * head_dim
+    w = (torch.randn(n, k) / math.sqrt(k)).bfloat16()
+    qkv = (normed @ w.double().t()).view(m, heads + 2 * kv_heads, head_dim)
+    cos, sin = (torch.from_numpy(a) for a in P.rope_tables(1024, head_dim, 10000.0))
+    positions = torch.tensor([(i * 37) % 1024 for i in range(m)])
+    table = torch.arange(16, dtype=torch.int32).flip(0)[None]
+    k_pages, v_pages = _empty_pages(16, kv_heads, head_dim, torch.bfloat16, 7.0, 7.0, "cuda")
+    rope = dict(cos=cos.cuda(), sin=sin.cuda(), tok_slot=_i32([0 if i % 11 else -1 for i in range(m)]), tok_pos=positions.int().cuda(), k_pages=k_pages, v_pages=v_pages,
+                block_table=table.cuda(), heads=heads, kv_heads=kv_heads, head_dim=head_dim)
+    got = run(w, torch.empty(m, heads * head_dim, dtype=torch.bfloat16, device="cuda"), ops.EPILOGUE_ROPE, n, rope)
+    turned = P.rope_rotate_half(qkv[:, :heads + kv_heads], cos[positions].double(), sin[positions].double())
+    close(got.view(m, heads, head_dim), turned[:, :heads], "queries")
+    held_k, held_v = _read_pages(k_pages, v_pages, head_dim)
+    for i in range(m):
+        page, inside = table[0, positions[i] // 64].item(), positions[i].item() % 64
+        if i % 11:
+            close(held_k[page, :, inside].double(), turned[i, heads:], "keys")
+            close(held_v[page, :, inside].double(), qkv[i, heads + kv_heads:], "values")
+        else:
+            assert (held_k[page, :, inside] == 7).all() and (held_v[page, :, inside] == 7).all()
