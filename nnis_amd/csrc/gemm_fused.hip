@@ -126,7 +126,8 @@ __global__ __launch_bounds__(KSPLIT > 4 ? 64 * KSPLIT : 256) void gemm_fused_ker
   int tok_slot[MT], tok_pos[MT], tok_page[MT];
   f32x4 tok_cos[MT], tok_sin[MT];
   // Parts of a row's sum of squares a lane keeps in flight (4 lane groups share a row): 9 take the 36 of a row of 576 columns in
-  // one trip to memory (with 8 the last four were another, behind the products: a decode step of 30 layers, 8 sequences, 891 -> 882 us)
+  // one trip to memory (with 8 the last four were another, behind the products: a decode step of 30 layers, 8 sequences, 891 -> 882 us).
+  // Rows of 592 columns on (37 parts and more, up to where DEAL begins) still take a second trip.
   constexpr int kPartRegs = DEAL ? 8 : 9;
   float ss_held[MT][kPartRegs];
   const bool ends_unit = active && part == 0;

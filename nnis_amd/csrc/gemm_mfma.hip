@@ -1070,7 +1070,10 @@ struct Workspace {
 // compute units without a block, a part keeps at least 4 steps of 64, and the parts fit the workspace.
 // The parts' kernel costs 3.6 us and a launch, a step of 64 of a tile's K 0.36: K in parts pays from about 900 saved on (128
 // tokens, gate/up of 3072 x 576 in two parts 5.8 + 3.6 us; whole, a prompt of 100 tokens
-// through 30 such layers 1,060 -> 996, of 250 1,195 -> 1,154).
+// through 30 such layers 1,060 -> 996, of 250 1,195 -> 1,154).  The line was then looked at from both sides over weights of 576 to
+// 11,264 rows, K of 512 to 1,792 and 17 to 600 tokens, microseconds in parts and whole: stored, 64 x 4608 x 1024 8.8 and 7.2, 100 x 4096 x
+// 1152 9.5 and 7.6; into the stream 400 x 1024 x 1024 9.2 and 8.0, 128 x 4096 x 1192 10.8 and 9.4, but 17 x 4096 x 1192 7.6 and 8.4 and
+// 65 x 3072 x 1792 10.3 and 11.0.
 constexpr int kSplitSavesLeast = 900;
 int tiled_ksplit(int tiles, int m, int width, int k, size_t workspace_bytes) {
   const int steps = (k + 63) / 64;
@@ -1272,7 +1275,10 @@ bool nnis_gemm_takes_few_tokens(int m, int n, int k) {
 
 // The same for a product whose tiled kernel may cut K into parts (it stores, or adds to the stream): large
 // weights with few columns still fill the chip then.  Measured with 64 tokens, microseconds: 2048 x 5632
-// 28 for few tokens against 15 in 8 parts, 2048 x 8192 39 against 18.
+// 28 for few tokens against 15 in 8 parts, 2048 x 8192 39 against 18.  `parts` counts a K of 256 and more as a part also
+// where the tiles leave K whole because parts would not pay (tiled_ksplit): they are as fast there with fewer blocks.  Microseconds for few tokens, in
+// tiles with K whole, and in parts: 64 x 4608 x 1024 12.1, 7.2 and 9.1, 64 x 5632 x 768 10.5, 6.4 and 8.7, 33 x 8064 x 576 6.7, 5.7 and 7.7,
+// 33 x 4608 x 1152 8.6, 7.2 and 8.1; 17 x 4608 x 1024 6.2, 6.7 and 7.6.
 static bool takes_few_tokens_with_parts(int m, int n, int k, bool workspace) {
   if (m <= 16 || m > 64 || !workspace) return nnis_gemm_takes_few_tokens(m, n, k);
   const bool large = (size_t)n * k * sizeof(bf16_t) > kRereadWeightBytes;

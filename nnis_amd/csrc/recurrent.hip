@@ -684,7 +684,8 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(GlaArgs a) {
 // takes LANES x 4 value columns of one head of one sequence, a thread 4 neighbouring columns (16 bytes) of every
 // (256 / LANES)-th key row, LANES threads a row's consecutive memory.  (The scan above has 8 lanes of 4 bytes on a row for heads of
 // 128 x 256, and walks its tokens' loop for one.)  The rows' parts of o are added by lane exchanges and through LDS.
-// One sequence, 8 heads of 128 x 256: 10.0 -> 5.2 us, four 10.8 -> 5.9.
+// One sequence, 8 heads of 128 x 256: 10.0 -> 5.2 us, four 10.8 -> 5.9; by themselves 1 / 16 / 64 sequences 8.3 / 12.7 / 30.9 -> 4.0 / 9.4 /
+// 22.4, 4 heads of 256 x 256 8.6 / 14.8 / 40.2 -> 4.5 / 9.9 / 23.4, 16 of 64 x 64 5.8 / 6.4 / 11.0 -> 3.7 / 4.7 / 9.8.
 template <int ROWS, int LANES>
 __global__ __launch_bounds__(256) void gla_step_kernel(GlaArgs a) {
   constexpr int kRowsApart = 256 / LANES;  // ROWS of them a thread: key channels up to ROWS * kRowsApart
@@ -857,7 +858,9 @@ extern "C" int nnis_selective_scan(const void* x, int x_dtype, const float* dt_p
   a.y = y; a.y_dtype = y_dtype; a.piece = piece; a.pieces = pieces; a.carried = carried; a.stepped = stepped;
   const int need = (states + 15) / 16;  // lanes of 16 states (of 8 for up to 8 states)
   hipStream_t s = (hipStream_t)stream;
-  // blocks of one wave while larger ones would leave compute units without any (single tokens, short runs)
+  // blocks of one wave while larger ones would leave compute units without any (single tokens, short runs); with wide loads, channels of 16
+  // states, 1 / 16 / 64 single tokens: 512 channels 8.4 / 8.6 / 9.9 -> 3.3 / 3.5 / 4.1 us, 4,096 8.5 / 12.0 / 39.6 -> 3.4 / 5.2 / 12.0 (the last in
+  // blocks of four waves)
   const int threads = pieces <= 1 && (long long)batch * channels * (need <= 1 ? 1 : (need <= 2 ? 2 : (need <= 4 ? 4 : 8))) < 256 * 1024 ? 64 : 256;
 #define NNIS_SCAN(LANES_, PASS_, PIECES_, PER_, UNIFORM_)                                                                  \
   hipLaunchKernelGGL((selective_scan_kernel<LANES_, PASS_, PER_, UNIFORM_>),                                               \
