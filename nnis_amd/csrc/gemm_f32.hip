@@ -764,7 +764,7 @@ void launch_few(const XT* x, const float* w, const Fused& f, int m, int n, int k
 template <int EPI, int BM, int BN, int WGM, int WGN, int KG>
 int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, int k, hipStream_t stream) {
   constexpr int lds = tile_lds(BM, BN, KG);
-  static_assert(lds <= 160 * 1024 && lds >= BM * BN * 4, "a compute unit has 160 KB; the groups' sums fit");
+  static_assert(lds <= 160 * 1024 && tile_stages(BM, BN, KG) >= BM * BN * 4, "a compute unit has 160 KB; the groups' sums fit before the marks");
   auto kernel = gemm_f32_tiled_kernel<BM, BN, WGM, WGN, KG, EPI>;
   NNIS_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess,
                "gemm_f32: %d bytes of LDS were refused", lds);
