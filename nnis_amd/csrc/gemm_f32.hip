@@ -785,8 +785,8 @@ int launch_tiled(const float* x, const float* w, const Fused& f, int m, int n, i
 // rows of 6144 x 2048 19.3 against 20.6).  Beyond 16 rows a variant's time is close to a start and, for every
 // round of its blocks on 256 compute units, a slope times K: the least of these is taken.  Measured:
 // 64 x 2048 x 2048 13.4 us (two strips, one tile a block), 100 x 2048 x 2048 18.1 (2 x 2; 23.9 in tiles of 32 x 64), 100 x 11264 x 2048
-// 45.6 (tiles of 64 x 96; 52.7 in 128 x 64), 509 x 2048 x 5632 90 (64 x 64; 103 in 32 x 64), 2000 x 11264 x 2048 501 (128 x 128; 558 in 64 x 128).
-// Over 8 weights from 576 x 576 to 11264 x 2048 at 20 to 2,000 rows the form taken is 0.2% slower than the best on average.
+// 47.5 (tiles of 64 x 96; 53.6 in 128 x 64), 509 x 2048 x 5632 94 (64 x 64; 109 in 32 x 64), 2000 x 11264 x 2048 519 (128 x 128; 572 in 64 x 128).
+// Over 7 weights from 960 x 576 to 11264 x 2048 at 20 to 2,000 rows the form taken is 0.2% slower than the best on average.
 struct Variant {
   int rows, columns;  // of a block
   float slope, start; // microseconds: slope * K for each round of blocks, and start
