@@ -1,0 +1,794 @@
+// The layers of a step of few single tokens in one launch (pre-norm blocks of plain attention with heads of 64 channels and a
+// SiLU-gated feed-forward, bfloat16, up to 16 rows).
+//
+// What bounds such a step is neither bytes nor products but its chain of dependent kernels, five to six a layer: each begins
+// 1.6 us after the one before has ended, asks for its weights, and only then has something to multiply.  Here a layer's stages
+// are blocks of one grid, in the order of the chain: a block asks for its weights (or keys and values) first, waits for its
+// operands, and ends with words that the blocks behind it wait for; the chip holds the blocks of two to four layers at a time, so
+// a stage's weights are in registers before its operands exist, and from one stage to the next is a store, a load and a
+// reduction.
+//
+// How words get from block to block: every word of the exchange is kNone (all bits set) before the launch, and is there once it is
+// anything else.  Writers store past the caches and never store kNone (a NaN with that payload goes out as another NaN), readers
+// load past the caches until no word of what they asked for is kNone.  A word carries its own mark, so no order between
+// words is needed, no counter and no fence.
+//
+// Why every wait ends: the stages of a block's operands are blocks of smaller numbers, and a die is handed its blocks in the order
+// of their numbers; so the unfinished block with the smallest number is on the chip, or its die is full of blocks of another
+// kernel.  Should two such launches ever fill a die each for the other, or a fault keep words away, a wait gives up after
+// kWaitTicks: it says so in `fail` (then all others leave too) and in `host_fail`, which the host reads before its next step;
+// what was not written stays kNone, which is no number, so nothing that hangs on it looks like a result.
+#include <hip/hip_runtime.h>
+
+#include "product.h"
+
+thread_local char g_nnis_error[512] = {0};
+extern "C" const char* nnis_last_error() { return g_nnis_error; }
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+
+constexpr unsigned kNone = 0xffffffffu;
+constexpr int kPastCaches = 16;             // a buffer access's cache policy: sc1, agent scope
+constexpr int HD = 64;                      // channels of a head
+constexpr int kMostRows = 16;
+constexpr int kRunRow = HD + 4;             // words of a run: outputs, reference, sum, two unused
+constexpr long long kWaitTicks = 200000000; // of the 100 MHz clock: 2 s
+constexpr float kLazyRise = 8.0f;           // as in attention.hip: a softmax reference moves when a score rises 2^8 above it
+
+struct ChainLayer {
+  const bf16_t *w_qkv, *w_o, *w_gate_up, *w_down;  // packed
+  const void *gain1, *gain2;
+  bf16_t *k_pages, *v_pages;
+};
+
+struct ChainArgs {
+  const ChainLayer* layers;
+  int layer_count, m, width, heads, kv_heads, inner, splits, gain_dtype;
+  float eps, scale_log2;
+  const float* x;  // [m, width]
+  float* x_out;    // [m, width]: the stream behind the last layer
+  const float *tok_cos, *tok_sin;
+  const int *tok_pos, *tok_page, *tok_pages;
+  int max_pages;
+  unsigned *words, *run_words;  // (the runs lie apart: in the scratch that the split decode attention has)
+  unsigned words_bytes, run_bytes, layer_words, layer_runs;
+  // where a layer's words lie: the stream's records before the attention and before the feed-forward; queries, keys, values;
+  // attention rows; gated rows
+  unsigned stream1, stream2, q, k, v, attn, act;
+  int n_strip;        // strips of the stream
+  int n_entry, n_qkv, n_att, n_comb, n_out, n_gate, n_down;  // blocks of a stage
+  unsigned *fail, *host_fail;
+};
+
+// Rows lie by strips of 16 channels: [strip][row][16 bfloat16], 32 bytes that one block writes and that a lane's two pieces of an
+// operand are.  The stream's rows are records of 128 bytes, [strip][row]: 16 channels times the next norm's gain in bfloat16, the
+// strip's part of the row's sum of squares (four times), 16 unused bytes, and the 16 channels in 32 bits: two full stores, and a
+// reader's operand and its share of the sum from one line.  (Parts of 4 bytes from 36 blocks in one line took a reader 1.2 us more.)
+constexpr int kRecord = 32;                 // words
+constexpr int kRecordSum = 8, kRecordStream = 16;
+
+__device__ __forceinline__ unsigned marked(float v) {
+  const unsigned u = __float_as_uint(v);
+  return u == kNone ? 0x7fc00000u : u;
+}
+__device__ __forceinline__ unsigned marked2(bf16_t lo, bf16_t hi) {
+  const unsigned u = (unsigned)__builtin_bit_cast(unsigned short, lo) | ((unsigned)__builtin_bit_cast(unsigned short, hi) << 16);
+  return u == kNone ? 0x7fc07fc0u : u;
+}
+
+// where a lane reads: its own part of a byte offset, and the part that is the wave's
+struct At {
+  unsigned lane, wave;
+};
+
+struct Exchange {
+  __amdgpu_buffer_rsrc_t r;
+  unsigned *fail, *host_fail;
+
+  __device__ __forceinline__ Exchange(const ChainArgs& a, unsigned* words, unsigned bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc(words, 0, bytes, 0x00020000)), fail(a.fail), host_fail(a.host_fail) {}
+
+  // whether a wait is to be left: every 256th look, by the clock and by what others found
+  __device__ __forceinline__ bool leave(int& looks, long long& since) const {
+    if ((++looks & 255) != 0) return false;
+    const long long now = wall_clock64();
+    if (looks == 256) since = now;
+    if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
+    if (now - since < kWaitTicks) return false;
+    __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(host_fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return true;
+  }
+
+  // Until one word of a stage further ahead is there: a block that is on the chip early looks now and then at one word, so that
+  // the words of the stage at work are not asked for by every block of the layers behind it.
+  template <bool ONE>  // the first wave looks for the whole block
+  __device__ __forceinline__ void gate(unsigned word, int wave) const {
+    if (!ONE || wave == 0) {
+      int looks = 0;
+      long long since = 0;
+      while (true) {
+        const unsigned u = __builtin_amdgcn_raw_buffer_load_b32(r, word * 4, 0, kPastCaches);
+        asm volatile("" ::: "memory");  // (asked for anew each time)
+        if (__builtin_amdgcn_readfirstlane(u) != kNone || leave(looks, since)) break;
+        __builtin_amdgcn_s_sleep(4);
+      }
+    }
+    if (ONE) __syncthreads();
+  }
+
+  // 16 bytes a lane N times, and beside each an M-th of 4 or 8 bytes: `ask(i)` gives the i-th's byte offsets, the lane's part and
+  // the wave's; until all of them are there
+  template <int N, typename Ask>
+  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask) const {
+    int looks = 0;
+    long long since = 0;
+    while (true) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
+      asm volatile("" ::: "memory");
+      unsigned top = 0;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
+      if (!__any(top == kNone) || leave(looks, since)) return;
+    }
+  }
+  template <int N, typename Ask, typename T, int M, typename AskBeside>
+  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask, T (&w)[M], AskBeside ask_beside) const {
+    int looks = 0;
+    long long since = 0;
+    while (true) {
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        if constexpr (sizeof(T) == 4) w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
+        else w[i] = __builtin_amdgcn_raw_buffer_load_b64(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
+      asm volatile("" ::: "memory");
+      unsigned top = 0;
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        if constexpr (sizeof(T) == 4) top = max(top, w[i]);
+        else top = max(top, max(w[i][0], w[i][1]));
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
+      if (!__any(top == kNone) || leave(looks, since)) return;
+    }
+  }
+  __device__ __forceinline__ void put(unsigned word, unsigned v) const { __builtin_amdgcn_raw_buffer_store_b32(v, r, word * 4, 0, kPastCaches); }
+  __device__ __forceinline__ void put(unsigned word, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, r, word * 4, 0, kPastCaches); }
+  __device__ __forceinline__ void put(unsigned word, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, r, word * 4, 0, kPastCaches); }
+};
+
+__device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
+
+// STRIPS strips of 16 weight rows times the step's rows; the block's waves share K (chunks of 64, whole).  A wave asks for the
+// weights of its first STEPS chunks when the block begins; XB chunks of the operand are asked for together.  A step of the operand
+// beyond the last chunk reads the last again and is not multiplied.
+template <int WAVES, int STRIPS, int STEPS, int XB>
+struct Product {
+  static_assert(STEPS % XB == 0, "whole trips");
+  bf16x8 w[STEPS][2][STRIPS];
+  f32x4 acc[STRIPS];
+  const bf16_t* strip[STRIPS];
+  int chunks, part, lane;
+
+  __device__ __forceinline__ void ask(int base) {
+#pragma unroll
+    for (int d = 0; d < STEPS; ++d) {
+      if (base + d * WAVES >= chunks) break;  // (the same for the whole wave)
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int j = 0; j < STRIPS; ++j)
+          w[d][half][j] = load_packed(strip[j] + (size_t)(base + d * WAVES) * kPackedChunkElems + half * kPackedHalfElems + lane * 8);
+    }
+  }
+  // row(j): the first row of strip j
+  template <typename Row>
+  __device__ __forceinline__ void begin(const bf16_t* weight, Row row, int k, int lane_, int part_) {
+    part = part_;
+    lane = lane_;
+    chunks = nnis_packed_chunks(k);
+#pragma unroll
+    for (int j = 0; j < STRIPS; ++j) {
+      strip[j] = weight + (size_t)(row(j) / 16) * nnis_packed_strip_elems(k);
+      acc[j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    ask(part);
+  }
+  // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`.  SUM: the strips are the
+  // stream's records; returns the lane's share of its row's sum of squares.
+  template <bool SUM>
+  __device__ __forceinline__ float run(const Exchange& ex, unsigned row_at, unsigned stride) {
+    float ss = 0.0f;
+    const unsigned at = row_at + lane / 16 * stride;
+    for (int base = part; base < chunks; base += WAVES * STEPS) {
+      if (base != part) ask(base);
+#pragma unroll
+      for (int b = 0; b < STEPS; b += XB) {
+        if (base + b * WAVES >= chunks) continue;
+        u32x4 v[XB * 2];
+        unsigned sum[XB];
+        auto step = [&](int d) { return (unsigned)min(base + (b + d) * WAVES, chunks - 1) * 4 * stride; };
+        auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
+        if constexpr (SUM) ex.take(v, pieces, sum, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
+        else ex.take(v, pieces);
+#pragma unroll
+        for (int d = 0; d < XB; ++d) {
+          if (base + (b + d) * WAVES >= chunks) continue;
+          if constexpr (SUM) ss += __uint_as_float(sum[d]);
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int j = 0; j < STRIPS; ++j) acc[j] = mfma(w[b + d][half][j], __builtin_bit_cast(bf16x8, v[2 * d + half]), acc[j]);
+        }
+      }
+    }
+    return ss;
+  }
+};
+
+// a row's 16 channels of a strip into its record, by the wave that ends the strip: lane (row, g) has four of them
+__device__ __forceinline__ void put_record(const Exchange& ex, unsigned word, int g, f32x4 v, f32x4 gain, float sum) {
+  const unsigned lo = marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), hi = marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]));
+  const unsigned next_lo = __shfl_xor(lo, 16, kWave), next_hi = __shfl_xor(hi, 16, kWave), part = marked(sum);
+  // lanes 0 and 2 of a row store 8 channels each, lanes 1 and 3 the sum
+  const u32x4 first = g % 2 == 0 ? (u32x4){lo, hi, next_lo, next_hi} : (u32x4){part, part, part, part};
+  ex.put(word + (g % 2 == 0 ? 2 * g : kRecordSum + 2 * (g - 1)), first);
+  ex.put(word + kRecordStream + 4 * g, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+}
+
+// units that a block of the products takes: wide models' blocks two, whose rows they then read once
+template <int WAVES>
+constexpr int units_of() { return WAVES == 8 ? 2 : 1; }
+
+// ... but down's blocks one: a compute unit reads about 30 GB/s, and half as many blocks of twice the weights are late
+template <int WAVES, bool DOWN>
+constexpr int into_units_of() { return DOWN ? 1 : units_of<WAVES>(); }
+
+template <int WAVES>
+struct Shared {
+  union {
+    struct {
+      float acc[WAVES][WAVES == 8 ? 4 : 2][kWave][4];
+      float ss[WAVES][kWave];
+    } product;
+    struct {
+      __attribute__((aligned(16))) float o[WAVES][4][HD];
+      float m[WAVES][4], l[WAVES][4];
+      bf16x8 heads[WAVES][kWave];
+      __attribute__((aligned(16))) bf16_t stage[WAVES][4][kPageTokens + 8];
+    } attention;
+    float sums[16];
+  };
+};
+
+// The waves' sums added up: of a block's UNITS units of NACC strips, unit u's in wave u (sums[NACC], ss); false for waves that have none.
+template <int WAVES, int UNITS, int NACC>
+__device__ __forceinline__ bool add_waves(Shared<WAVES>& s, const f32x4 (&acc)[UNITS * NACC], f32x4 (&sums)[NACC], float& ss, int wave, int lane) {
+  ss += __shfl_xor(ss, 16, kWave);
+  ss += __shfl_xor(ss, 32, kWave);
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u)
+    if (wave != u) {
+#pragma unroll
+      for (int j = 0; j < NACC; ++j) *(f32x4*)s.product.acc[wave][u * NACC + j][lane] = acc[u * NACC + j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < NACC; ++j) sums[j] = acc[u * NACC + j];
+    }
+  s.product.ss[wave][lane] = ss;
+  __syncthreads();
+  if (wave >= UNITS) return false;
+#pragma unroll
+  for (int i = 1; i < WAVES; ++i) {
+    const int other = (wave + i) % WAVES;
+#pragma unroll
+    for (int j = 0; j < NACC; ++j) sums[j] += *(const f32x4*)s.product.acc[other][wave * NACC + j][lane];
+    ss += s.product.ss[other][lane];
+  }
+  return true;
+}
+
+// a row of the embedding into the first layer's records; its sum of squares is one part
+template <int WAVES>
+__device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int row) {
+  const float* x = a.x + (size_t)row * a.width;
+  float sum = 0.0f;
+  for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
+    const f32x4 v = *(const f32x4*)(x + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum = fmaf(v[e], v[e], sum);
+  }
+  sum = block_sum(sum, s.sums);
+  for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
+    const f32x4 v = *(const f32x4*)(x + c);
+    const f32x4 gain = four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
+    const unsigned word = a.stream1 + (c / 16 * a.m + row) * kRecord, four = c % 16 / 4;
+    ex.put(word + 2 * four, (u32x2){marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]))});
+    if (four == 0) ex.put(word + kRecordSum, marked(c == 0 ? sum : 0.0f));
+    ex.put(word + kRecordStream + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+  }
+}
+
+// queries, keys and values of two strips (a head's channels f .. f + 15 and f + 32 ..), rotated, and the write into the cache
+template <int WAVES>
+__device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int unit) {
+  constexpr bool kNear = WAVES == 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const ChainLayer& L = a.layers[layer];
+  const unsigned here = layer * a.layer_words;
+  // unit 2 h + i of all: channels 16 i .. 16 i + 15 of head h and those half a head on
+  constexpr int kUnits = units_of<WAVES>();
+  Product<WAVES, 2 * kUnits, 4, 4> p;
+  p.begin(L.w_qkv, [&](int j) { const int u = unit * kUnits + j / 2; return u / 2 * HD + u % 2 * 16 + j % 2 * (HD / 2); }, a.width, lane, wave);
+  const int row = r < a.m ? r : a.m - 1, ends = unit * kUnits + (wave < kUnits ? wave : 0), head = ends / 2, f0 = ends % 2 * 16;
+  const f32x4 c = *(const f32x4*)(a.tok_cos + row * (HD / 2) + f0 + 4 * g), sn = *(const f32x4*)(a.tok_sin + row * (HD / 2) + f0 + 4 * g);
+  const int pos = a.tok_pos[row], page = a.tok_page[row];
+  if (kNear) ex.template gate<kNear>(here + a.stream1 + unit * 61 % (a.m * a.n_strip) * kRecord, wave);
+  else if (layer > 0) ex.template gate<kNear>(here - a.layer_words + a.act + unit * 61 % (a.m * a.inner / 2), wave);
+  float ss = p.template run<true>(ex, (here + a.stream1 + row * kRecord) * 4, a.m * kRecord * 4);
+  f32x4 sums[2];
+  if (!add_waves<WAVES, kUnits, 2>(s, p.acc, sums, ss, wave, lane)) return;
+  if (r >= a.m) return;
+  const float scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  const f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
+  f32x4 out_lo = lo, out_hi = hi;
+  if (head < a.heads + a.kv_heads) {
+    out_lo = lo * c - hi * sn;
+    out_hi = hi * c + lo * sn;
+  }
+  bf16x4 b_lo, b_hi;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    b_lo[e] = (__bf16)out_lo[e];
+    b_hi[e] = (__bf16)out_hi[e];
+  }
+  const u32x2 w_lo = {marked2(b_lo[0], b_lo[1]), marked2(b_lo[2], b_lo[3])}, w_hi = {marked2(b_hi[0], b_hi[1]), marked2(b_hi[2], b_hi[3])};
+  const int f = f0 + 4 * g;
+  unsigned to;  // [head][strip][row]
+  if (head < a.heads) to = a.q + head * a.m * (HD / 2);
+  else if (head < a.heads + a.kv_heads) to = a.k + (head - a.heads) * a.m * (HD / 2);
+  else to = a.v + (head - a.heads - a.kv_heads) * a.m * (HD / 2);
+  to += here + (f0 / 16 * a.m + row) * 8 + 2 * g;
+  ex.put(to, w_lo);
+  ex.put(to + HD / 32 * a.m * 8, w_hi);
+  if (page < 0 || head < a.heads) return;
+  if (head < a.heads + a.kv_heads) {
+    bf16_t* dst = L.k_pages + ((size_t)page * a.kv_heads + head - a.heads) * nnis_k_page_elems(HD);
+    *(bf16x4*)(dst + nnis_k_offset(pos % kPageTokens, f)) = b_lo;
+    *(bf16x4*)(dst + nnis_k_offset(pos % kPageTokens, f + HD / 2)) = b_hi;
+  } else {
+    bf16_t* dst = L.v_pages + ((size_t)page * a.kv_heads + head - a.heads - a.kv_heads) * nnis_v_page_elems(HD);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dst[nnis_v_offset(f + e, pos % kPageTokens)] = b_lo[e];
+      dst[nnis_v_offset(f + HD / 2 + e, pos % kPageTokens)] = b_hi[e];
+    }
+  }
+}
+
+struct KeysPage {
+  bf16x8 k[HD / 8];       // this lane's key, all channels
+  bf16x8 v[2][HD / 16];   // value operands of the two halves of the page
+};
+__device__ __forceinline__ void load_keys(KeysPage& f, const bf16_t* page, int lane) {
+#pragma unroll
+  for (int c = 0; c < HD / 8; ++c) f.k[c] = *(const bf16x8*)(page + nnis_k_offset(lane, 8 * c));
+}
+__device__ __forceinline__ void load_values(KeysPage& f, const bf16_t* page, int lane) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int t = 0; t < HD / 16; ++t) f.v[h][t] = *(const bf16x8*)(page + nnis_v_offset(16 * t + lane % 16, 32 * h + 8 * (lane / 16)));
+}
+__device__ __forceinline__ bf16x4 low4(bf16x8 v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); }
+__device__ __forceinline__ bf16x4 high4(bf16x8 v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); }
+
+// A run of a sequence's keys against up to 4 query heads of a key head, keys on lanes (attention.hip,
+// attention_decode_keys_kernel: the same products in the same layouts).  The pages hold every key but the step's own, which the
+// projection's blocks of this launch are still writing: it comes from the exchange and takes its place in the page's operands.
+template <int WAVES>
+__device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int item) {
+  constexpr bool kNear = WAVES == 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const int blk = lane / 4, j = lane % 4;
+  const ChainLayer& L = a.layers[layer];
+  const unsigned here = layer * a.layer_words;
+  const int group = a.heads / a.kv_heads, fours = (group + 3) / 4;
+  const int kv_head = item / fours % a.kv_heads, first_head = kv_head * group + item % fours * 4;
+  const int token = item / (fours * a.kv_heads) % a.m, split = item / (fours * a.kv_heads * a.m);
+  const int heads_here = min(4, kv_head * group + group - first_head);
+  const int pos = a.tok_page[token] < 0 ? 0 : a.tok_pos[token];  // a padding row reads its own key only
+  const int* pages = a.tok_pages + (size_t)token * a.max_pages;
+  const int page_count = pos / kPageTokens + 1;
+  const int per_split = (page_count + a.splits - 1) / a.splits;
+  const int begin = split * per_split, end = min(begin + per_split, page_count);
+  // the run's pages are dealt to the waves from its end, so that the page of the step's own key is its wave's first
+  const int last = end - 1 - wave, mine = last >= begin ? (last - begin) / WAVES + 1 : 0;
+  const bf16_t* k_base = L.k_pages + (size_t)kv_head * nnis_k_page_elems(HD);
+  const bf16_t* v_base = L.v_pages + (size_t)kv_head * nnis_v_page_elems(HD);
+  const size_t k_stride = (size_t)a.kv_heads * nnis_k_page_elems(HD), v_stride = (size_t)a.kv_heads * nnis_v_page_elems(HD);
+  KeysPage f;
+  if (mine > 0) {
+    const size_t page = __builtin_amdgcn_readfirstlane(pages[last]);
+    load_keys(f, k_base + page * k_stride, lane);
+    load_values(f, v_base + page * v_stride, lane);
+  }
+  if (kNear) ex.template gate<kNear>(here + a.q + ((first_head * (HD / 16) + item * 61 % (HD / 16)) * a.m + token) * 8, wave);
+  else ex.template gate<kNear>(here + a.stream1 + item * 61 % (a.m * a.n_strip) * kRecord, wave);
+  // Queries and the step's own key and value in one load of the wave (8 lanes a head's row, [head][strip][row]: two pieces a
+  // strip), and from there through LDS.
+  bf16x8* heads_lds = s.attention.heads[wave];
+  {
+    const int which = lane / 8, piece = lane % 8;  // 0 to 3: the group's queries; 4, 5: key, value
+    const unsigned rows = which < 4 ? a.q + (first_head + (which < heads_here ? which : 0)) * (HD / 2) * a.m : (which == 4 ? a.k : a.v) + kv_head * (HD / 2) * a.m;
+    u32x4 v[1];
+    ex.take(v, [&](int) { return At{(here + rows + (piece / 2 * a.m + token) * 8 + piece % 2 * 4) * 4, 0}; });
+    heads_lds[lane] = which < heads_here || which >= 4 ? __builtin_bit_cast(bf16x8, v[0]) : zero_chunk();
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  bf16x8 q[HD / 8];
+#pragma unroll
+  for (int c = 0; c < HD / 8; ++c) q[c] = heads_lds[8 * j + c];
+  if (mine > 0 && last == pos / kPageTokens) {  // the step's own key and value take their places in the page's operands
+    const int at_key = pos % kPageTokens, h_at = at_key / 32, e_at = at_key % 8;
+    if (lane == at_key) {
+#pragma unroll
+      for (int c = 0; c < HD / 8; ++c) f.k[c] = heads_lds[32 + c];
+    }
+    if (g == at_key % 32 / 8) {
+      const unsigned short* value = (const unsigned short*)(heads_lds + 40) + r;
+#pragma unroll
+      for (int t = 0; t < HD / 16; ++t) {
+        const unsigned short channel = value[16 * t];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          u32x4 words = __builtin_bit_cast(u32x4, f.v[h][t]);
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const unsigned put = e_at % 2 ? (words[w] & 0xffffu) | ((unsigned)channel << 16) : (words[w] & 0xffff0000u) | channel;
+            words[w] = h == h_at && w == e_at / 2 ? put : words[w];
+          }
+          f.v[h][t] = __builtin_bit_cast(bf16x8, words);
+        }
+      }
+    }
+  }
+  f32x4 o[HD / 16];
+#pragma unroll
+  for (int t = 0; t < HD / 16; ++t) o[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  float reference = -INFINITY, sum = 0.0f;
+  bf16_t* stage = &s.attention.stage[wave][0][0];
+  constexpr int kStageRow = kPageTokens + 8;
+  for (int n = 0; n < mine; ++n) {
+    const int index = last - n * WAVES, key0 = index * kPageTokens;
+    f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < HD / 8; ++c) {
+      s0 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(low4(f.k[c]), low4(q[c]), s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(high4(f.k[c]), high4(q[c]), s1, 0, 0, 0);
+    }
+    const bool more = n + 1 < mine;
+    const size_t next = more ? __builtin_amdgcn_readfirstlane(pages[index - WAVES]) : 0;
+    if (more) load_keys(f, k_base + next * k_stride, lane);
+    f32x4 sc = s0 + s1;
+    float top = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sc[e] = key0 + 4 * blk + e <= pos ? sc[e] * a.scale_log2 : -INFINITY;
+      top = fmaxf(top, sc[e]);
+    }
+    if (__any(top > reference + kLazyRise)) {
+      float moved = fmaxf(reference, top);
+#pragma unroll
+      for (int offset = 4; offset < kWave; offset <<= 1) moved = fmaxf(moved, __shfl_xor(moved, offset, kWave));
+      const float shrink = reference == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(reference - moved);
+      sum *= shrink;
+#pragma unroll
+      for (int t = 0; t < HD / 16; ++t) o[t] = o[t] * shrink;
+      reference = moved;
+    }
+    const float base = reference == -INFINITY ? 0.0f : reference;
+    bf16x4 p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float w = __builtin_amdgcn_exp2f(sc[e] - base);
+      sum += w;
+      p[e] = (__bf16)w;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    *(bf16x4*)(stage + j * kStageRow + 4 * blk) = p;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      bf16x8 columns = *(const bf16x8*)(stage + (r < 4 ? r : 0) * kStageRow + 32 * h + 8 * g);
+      if (r >= 4) columns = zero_chunk();
+#pragma unroll
+      for (int t = 0; t < HD / 16; ++t) o[t] = mfma(f.v[h][t], columns, o[t]);
+    }
+    if (more) load_values(f, v_base + next * v_stride, lane);
+  }
+#pragma unroll
+  for (int offset = 4; offset < kWave; offset <<= 1) sum += __shfl_xor(sum, offset, kWave);
+  if (r < 4) {
+#pragma unroll
+    for (int t = 0; t < HD / 16; ++t) *(f32x4*)&s.attention.o[wave][r][16 * t + 4 * g] = o[t];
+  }
+  if (lane < 4) {
+    s.attention.m[wave][lane] = reference;
+    s.attention.l[wave][lane] = sum;
+  }
+  __syncthreads();
+  const Exchange runs(a, a.run_words, a.run_bytes);
+  // four channels of a head a thread, and one thread a head for the run's reference and sum
+  for (int i = threadIdx.x; i < heads_here * (HD / 4 + 1); i += 64 * WAVES) {
+    const int head = i / (HD / 4 + 1), four = i % (HD / 4 + 1);
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, s.attention.m[w][head]);
+    f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
+    float den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float m = s.attention.m[w][head], weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+      num += *(const f32x4*)&s.attention.o[w][head][four < HD / 4 ? 4 * four : 0] * weight;
+      den += s.attention.l[w][head] * weight;
+    }
+    if (a.splits == 1) {
+      num = num / den;
+      if (four < HD / 4)
+        ex.put(here + a.attn + (((first_head + head) * (HD / 16) + four / 4) * a.m + token) * 8 + four % 4 * 2,
+               (u32x2){marked2((bf16_t)num[0], (bf16_t)num[1]), marked2((bf16_t)num[2], (bf16_t)num[3])});
+    } else {
+      if (four == HD / 4) num = (f32x4){top, den, 0.0f, 0.0f};
+      runs.put(layer * a.layer_runs + ((token * a.heads + first_head + head) * a.splits + split) * kRunRow + 4 * four,
+             (u32x4){marked(num[0]), marked(num[1]), marked(num[2]), marked(num[3])});
+    }
+  }
+}
+
+// Four channels of a (row, head) from its runs, RUNS at once: a head is 16 lanes, a wave has four.
+template <int RUNS>
+__device__ __forceinline__ bf16x4 sum_runs(const Exchange& ex, unsigned first_word, int splits, int channel) {
+  u32x4 v[RUNS];
+  u32x2 state[RUNS];
+  ex.take(v, [&](int i) { return At{(first_word + channel) * 4, (unsigned)(i < splits ? i : 0) * kRunRow * 4}; }, state,
+          [&](int i) { return At{(first_word + HD) * 4, (unsigned)(i < splits ? i : 0) * kRunRow * 4}; });
+  float top = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < RUNS; ++i) top = i < splits ? fmaxf(top, __uint_as_float(state[i][0])) : top;
+  f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
+  float den = 0.0f;
+#pragma unroll
+  for (int i = 0; i < RUNS; ++i)
+    if (i < splits) {
+      const float m = __uint_as_float(state[i][0]), weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+      num += __builtin_bit_cast(f32x4, v[i]) * weight;
+      den += __uint_as_float(state[i][1]) * weight;
+    }
+  bf16x4 out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = (__bf16)(num[e] / den);
+  return out;
+}
+template <int WAVES>
+__device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange& ex, int layer, int block) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int items = a.m * a.heads, first = (block * WAVES + wave) * 4;  // head * rows + row, four a wave: whole lines of the rows' strips
+  if (first >= items) return;
+  const unsigned here = layer * a.layer_words;
+  const int item = min(first + lane / 16, items - 1), head = item / a.m, row = item % a.m, channel = lane % 16 * 4;
+  ex.template gate<false>(here + a.q + first * 61 % (items * (HD / 2)), 0);
+  const Exchange runs(a, a.run_words, a.run_bytes);
+  const unsigned first_run = layer * a.layer_runs + (row * a.heads + head) * a.splits * kRunRow;
+  const bf16x4 out = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel)
+                     : a.splits <= 8 ? sum_runs<8>(runs, first_run, a.splits, channel) : sum_runs<16>(runs, first_run, a.splits, channel);
+  ex.put(here + a.attn + ((head * (HD / 16) + channel / 16) * a.m + row) * 8 + channel % 16 / 2,
+         (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
+}
+
+// a strip of 16 columns of the stream: the output projection (down = false) or the feed-forward's down
+template <int WAVES, bool DOWN>
+__device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
+  constexpr bool kNear = WAVES == 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const ChainLayer& L = a.layers[layer];
+  const unsigned here = layer * a.layer_words, next = here + (DOWN ? a.layer_words : 0);
+  const int k = DOWN ? a.inner : a.heads * HD;
+  const bool last = DOWN && layer + 1 == a.layer_count;
+  // a wave's steps whose weights are in registers before the operands exist: 4 waves have 6 of an inner size of 1,536, 8 waves 11 of 5,632
+  constexpr int kUnits = into_units_of<WAVES, DOWN>(), kSteps = WAVES == 4 ? (DOWN ? 6 : 3) : (DOWN ? 16 : 4), kTogether = WAVES == 4 ? kSteps : 4;
+  Product<WAVES, kUnits, kSteps, kTogether> p;
+  p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, lane, wave);
+  const int strip = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1, column = strip * 16 + 4 * g;
+  const void* gain_of = DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2;
+  const f32x4 gain = four_of(gain_of, a.gain_dtype, column, 4, true);
+  if (kNear) ex.template gate<kNear>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
+  else if (DOWN) ex.template gate<kNear>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
+  else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<kNear>(layer * a.layer_runs + (block * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
+  else ex.template gate<kNear>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
+  // (the stream is two stages old and more: it is there)
+  u32x4 held[1];
+  if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + (strip * a.m + row) * kRecord + kRecordStream + 4 * g) * 4, 0}; });
+  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32);
+  float unused = 0.0f;
+  f32x4 sums[1];
+  if (!add_waves<WAVES, kUnits, 1>(s, p.acc, sums, unused, wave, lane)) return;
+  f32x4 v;
+  float sq = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = __uint_as_float(held[0][e]) + sums[0][e];
+    sq = fmaf(v[e], v[e], sq);
+  }
+  sq += __shfl_xor(sq, 16, kWave);
+  sq += __shfl_xor(sq, 32, kWave);
+  if (r >= a.m) return;
+  if (last) {
+    *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
+    return;
+  }
+  put_record(ex, next + (DOWN ? a.stream1 : a.stream2) + (strip * a.m + row) * kRecord, g, v, gain, sq);
+}
+
+template <int WAVES>
+__device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
+  constexpr bool kNear = WAVES == 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const unsigned here = layer * a.layer_words;
+  constexpr int kUnits = units_of<WAVES>();
+  Product<WAVES, 2 * kUnits, 4, 4> p;
+  p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, lane, wave);
+  const int unit = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
+  if (kNear) ex.template gate<kNear>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
+  else ex.template gate<kNear>(here + a.attn + block * 61 % (a.m * a.heads * (HD / 2)), wave);
+  float ss = p.template run<true>(ex, (here + a.stream2 + row * kRecord) * 4, a.m * kRecord * 4);
+  f32x4 sums[2];
+  if (!add_waves<WAVES, kUnits, 2>(s, p.acc, sums, ss, wave, lane)) return;
+  if (r >= a.m) return;
+  const float scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  bf16_t out[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float gate = sums[0][e] * scale, up = sums[1][e] * scale;
+    const float x = __builtin_amdgcn_exp2f(gate * -1.4426950408889634f);  // (as epilogue.h)
+    out[e] = (bf16_t)(gate * __builtin_amdgcn_rcpf(1.0f + x) * up);
+  }
+  ex.put(here + a.act + (unit * a.m + row) * 8 + 2 * g, (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
+}
+
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? 3 : 2))) void chain_kernel(ChainArgs a) {
+  __shared__ Shared<WAVES> s;
+  const Exchange ex(a, a.words, a.words_bytes);
+  int b = blockIdx.x;
+  if (b < a.n_entry) return entry_stage<WAVES>(a, ex, s, b);
+  b -= a.n_entry;
+  const int per_layer = a.n_qkv + a.n_att + a.n_comb + a.n_out + a.n_gate + a.n_down;
+  const int layer = b / per_layer;
+  b -= layer * per_layer;
+  if (b < a.n_qkv) return qkv_stage<WAVES>(a, ex, s, layer, b);
+  b -= a.n_qkv;
+  if (b < a.n_att) return attention_stage<WAVES>(a, ex, s, layer, b);
+  b -= a.n_att;
+  if (b < a.n_comb) return combine_stage<WAVES>(a, ex, layer, b);
+  b -= a.n_comb;
+  if (b < a.n_out) return strip_stage<WAVES, false>(a, ex, s, layer, b);
+  b -= a.n_out;
+  if (b < a.n_gate) return gate_stage<WAVES>(a, ex, s, layer, b);
+  strip_stage<WAVES, true>(a, ex, s, layer, b - a.n_gate);
+}
+
+__global__ __launch_bounds__(256) void chain_clear_kernel(u32x4* words, unsigned n, u32x4* runs, unsigned n_runs, unsigned* fail) {
+  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n + n_runs; i += gridDim.x * 256) {
+    u32x4* at = i < n ? words + i : runs + (i - n);
+    *at = (u32x4){kNone, kNone, kNone, kNone};
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *fail = 0;
+}
+
+// where the words of a layer lie; returns their number
+unsigned lay_out(ChainArgs& a) {
+  unsigned at = 0;
+  auto place = [&](unsigned& where, unsigned words) {
+    where = at;
+    at += (words + 31) / 32 * 32;
+  };
+  const unsigned m = a.m, strips = a.width / 16;
+  place(a.stream1, m * strips * kRecord);
+  place(a.stream2, m * strips * kRecord);
+  place(a.q, m * a.heads * (HD / 2));
+  place(a.k, m * a.kv_heads * (HD / 2));
+  place(a.v, m * a.kv_heads * (HD / 2));
+  place(a.attn, m * a.heads * (HD / 2));
+  place(a.act, m * a.inner / 2);
+  a.layer_runs = a.splits > 1 ? m * a.heads * a.splits * kRunRow : 0;
+  return at;
+}
+
+bool fits(int m, int width, int heads, int kv_heads, int inner, int splits) {
+  return m >= 1 && m <= kMostRows && width > 0 && width % 64 == 0 && width <= 8192 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads * HD <= 8192 &&
+         inner > 0 && inner % 64 == 0 && inner <= 65536 && splits >= 1 && splits <= 16;
+}
+
+}  // namespace
+
+// Words that a step's exchange needs (of 4 bytes; the last 32 are the kernel's own), or 0 for sizes that it does not take; `runs`: the
+// words of the runs beside them.
+extern "C" long long nnis_chain_words(int layers, int m, int width, int heads, int kv_heads, int inner, int splits, long long* runs) {
+  *runs = 0;
+  if (layers <= 0 || !fits(m, width, heads, kv_heads, inner, splits)) return 0;
+  ChainArgs a;
+  a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits;
+  const long long words = (long long)lay_out(a) * layers + 32;
+  *runs = (long long)a.layer_runs * layers;
+  return words * 4 < (1LL << 31) && *runs * 4 < (1LL << 31) ? words : 0;
+}
+
+// The layers of one step of single tokens.  layers: device memory, 8 pointers a layer (packed weights of q/k/v, output, gate/up
+// and down; the gains of its two norms, all of gain_dtype; its key and value pages); x, x_out: [m, width] in 32 bits; tok_cos,
+// tok_sin, tok_page, tok_pages: the step's tables.  words, runs: as nnis_chain_words says, 16-byte aligned.  host_fail: a word of pinned
+// host memory.
+extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width, int heads, int kv_heads, int head_dim, int inner, int splits,
+                          int gain_dtype, float eps, float scale, const float* x, float* x_out, const float* tok_cos, const float* tok_sin,
+                          const int* tok_pos, const int* tok_page, const int* tok_pages, int max_pages, void* words, long long word_count, void* runs, long long run_count,
+                          void* host_fail, void* stream_ptr) {
+  NNIS_REQUIRE(head_dim == HD && fits(m, width, heads, kv_heads, inner, splits), "chain: %d rows, width %d, %d/%d heads of %d, inner %d, %d runs are not taken", m,
+               width, heads, kv_heads, head_dim, inner, splits);
+  NNIS_REQUIRE(layers && x && x_out && tok_cos && tok_sin && tok_pos && tok_page && tok_pages && max_pages > 0 && words && host_fail, "chain: an operand is missing");
+  long long runs_needed;
+  const long long needed = nnis_chain_words(layer_count, m, width, heads, kv_heads, inner, splits, &runs_needed);
+  NNIS_REQUIRE(needed > 0 && word_count == needed && run_count >= runs_needed && (runs || runs_needed == 0), "chain: %lld and %lld words for %d layers", word_count,
+               run_count, layer_count);
+  NNIS_REQUIRE(nnis_dtype_ok(gain_dtype) && eps > 0.0f && scale > 0.0f, "chain: bad gain type, eps or scale");
+  for (const void* p : {(const void*)x, (const void*)x_out, (const void*)tok_cos, (const void*)tok_sin, (const void*)words, (const void*)runs})
+    NNIS_REQUIRE((uintptr_t)p % 16 == 0, "chain: operands must be 16-byte aligned");
+  ChainArgs a;
+  a.layers = (const ChainLayer*)layers; a.layer_count = layer_count;
+  a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits; a.gain_dtype = gain_dtype;
+  a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f;
+  a.x = x; a.x_out = x_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages;
+  a.max_pages = max_pages; a.words = (unsigned*)words; a.words_bytes = (unsigned)(word_count * 4);
+  a.layer_words = lay_out(a);
+  a.run_words = (unsigned*)runs; a.run_bytes = (unsigned)(runs_needed * 4);
+  a.fail = a.words + (word_count - 32);
+  a.host_fail = (unsigned*)host_fail;
+  // wide models' units are large: 8 waves share them
+  const int waves = width > 1024 ? 8 : 4;
+  a.n_entry = m;
+  const int units = waves == 8 ? units_of<8>() : units_of<4>();
+  a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
+  a.n_att = m * kv_heads * ((heads / kv_heads + 3) / 4) * splits;
+  a.n_comb = splits > 1 ? (m * heads + 4 * waves - 1) / (4 * waves) : 0;
+  a.n_strip = width / 16;
+  a.n_out = width / 16 / (waves == 8 ? into_units_of<8, false>() : into_units_of<4, false>());
+  a.n_down = width / 16 / (waves == 8 ? into_units_of<8, true>() : into_units_of<4, true>());
+  a.n_gate = inner / 16 / units;
+  const long long blocks = a.n_entry + (long long)layer_count * (a.n_qkv + a.n_att + a.n_comb + a.n_out + a.n_gate + a.n_down);
+  NNIS_REQUIRE(blocks < (1LL << 30), "chain: too many blocks");
+  hipStream_t stream = (hipStream_t)stream_ptr;
+  const unsigned fours = (unsigned)((word_count - 32) / 4), run_fours = (unsigned)(runs_needed / 4), clears = (fours + run_fours + 255) / 256;
+  hipLaunchKernelGGL(chain_clear_kernel, dim3(clears < 1024 ? clears : 1024), dim3(256), 0, stream, (u32x4*)words, fours, (u32x4*)runs, run_fours, a.fail);
+  NNIS_LAUNCH_CHECK("chain_clear");
+  if (waves == 8) hipLaunchKernelGGL(chain_kernel<8>, dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  else hipLaunchKernelGGL(chain_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  NNIS_LAUNCH_CHECK("chain");
+  return 0;
+}

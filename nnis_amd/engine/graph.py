@@ -59,6 +59,7 @@ class DecodeGraph:
         self.graph = None
         self.logits = None
         self.held = []  # memory the parts' kernels keep between calls, whose addresses the capture baked in: held as long as the graph
+        self.tables = []
 
     def _forward(self) -> torch.Tensor:
         engine = self.engine
@@ -90,11 +91,13 @@ class DecodeGraph:
         # holds what the parts name (``Part.held_buffers``): whatever its keeper does later, a replay never writes
         # into memory that has gone back to the allocator.
         self.held = list(self.engine.model.held_buffers(self.engine.rt))
+        self.tables = list(self.engine.model.held_tables(self.engine.rt))
 
     def run(self, ids, slots: Sequence[int], positions: Sequence[int], ids_device: torch.Tensor = None) -> torch.Tensor:
         """``ids``: the step's token ids, or None when they are on the device
         already: then row j's id is ``ids_device[j]`` (int32)."""
         count = len(slots)
+        self.engine.model.check_steps(self.engine.rt)
         self.copied.synchronize()  # the previous copy has left the pinned buffer
         host = self.host.numpy()
         host[0, :count] = ids if ids is not None else -1

@@ -163,6 +163,8 @@ register_module("core", ["elementwise.hip", "residual.hip", "gemm.hip", "gemm_f3
 register_module_family("attn_hd", _attention_recipe)
 # the mixers that carry a state of fixed size (convolution, selective scan, gated linear attention and retention, minGRU, gated delta rule)
 register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
+# the layers of a step of few single tokens in one launch
+register_module("chain", ["chain.hip"], headers=["common.h", "product.h"], source_flags={"chain.hip": _VECTOR_SUMS})
 # the real-gated linear recurrent unit
 register_module("gated_unit", ["gated_unit.hip"], headers=["common.h"], source_flags={"gated_unit.hip": _VECTOR_SUMS})
 # Mamba-2's state spaces
@@ -348,7 +350,7 @@ def load_module(module: str, build_if_missing: bool = True) -> ctypes.CDLL:
 
 
 def all_prebuilt_modules() -> List[str]:
-    return ["core", "reference", "recurrent", "state_space", "gated_unit", "token_side", "latent", "sublayer", "experts"] + [f"attn_hd{d}" for d in PREBUILT_HEAD_DIMS] + list(PREBUILT_WIDE_VALUES)
+    return ["core", "chain", "reference", "recurrent", "state_space", "gated_unit", "token_side", "latent", "sublayer", "experts"] + [f"attn_hd{d}" for d in PREBUILT_HEAD_DIMS] + list(PREBUILT_WIDE_VALUES)
 
 
 def build_all(force: bool = True, jobs: int = 4) -> List[str]:

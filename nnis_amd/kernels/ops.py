@@ -293,6 +293,19 @@ def latent():
     return _latent
 
 
+_chain = None
+
+
+def chain_module():
+    """The module of a decode step's layers in one launch."""
+    global _chain
+    if _chain is None:
+        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 9 + [_FLT, _FLT] + [_VOID] * 7 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]})
+        _chain.nnis_chain_words.argtypes = [_INT] * 7 + [ctypes.POINTER(_I64)]
+        _chain.nnis_chain_words.restype = _I64
+    return _chain
+
+
 _sublayer = None
 _experts = None
 
@@ -655,6 +668,56 @@ def step_tables(tok_slot: torch.Tensor, tok_pos: torch.Tensor, tokens: int, cos:
     _check(lib, lib.nnis_step_tables(tok_slot.data_ptr(), tok_pos.data_ptr(), tokens, _ptr(cos), _ptr(sin), half, positions,
                                      _ptr(block_table), max_pages, _ptr(out.cos), _ptr(out.sin), _ptr(out.page),
                                      _ptr(out.pages), _stream()))
+    return out
+
+
+CHAIN_MOST_ROWS = 16
+
+
+def chain_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, runs: int = 1) -> bool:
+    """Whether ``chain`` takes layers of these sizes."""
+    return head_dim == 64 and chain_words(layers, rows, width, heads, kv_heads, inner, runs)[0] > 0
+
+
+def chain_words(layers: int, rows: int, width: int, heads: int, kv_heads: int, inner: int, runs: int):
+    """(32-bit words of the exchange, of the runs) that ``chain`` needs; (0, _) for sizes that it does not take."""
+    of_runs = _I64()
+    return chain_module().nnis_chain_words(layers, rows, width, heads, kv_heads, inner, runs, ctypes.byref(of_runs)), of_runs.value
+
+
+def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int):
+    """The runs that ``chain`` cuts a sequence's keys into for a step of ``batch`` single tokens, the longest sequence of
+    ``longest`` tokens; None where the layers' own kernels are faster or do not take the sizes."""
+    if batch > CHAIN_MOST_ROWS:
+        return None
+    pages, waves = (longest + 63) // 64, 8 if width > 1024 else 4
+    each, blocks = 1 if batch <= 4 else 2, batch * kv_heads * ((heads // kv_heads + 3) // 4)
+    runs = 1
+    while runs < 16 and pages > each * runs * waves and 2 * runs * blocks <= 128:
+        runs *= 2
+    return runs if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs) else None
+
+
+def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, runs: int, failed: torch.Tensor,
+          gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int) -> torch.Tensor:
+    """All layers of a step of single tokens; returns the stream behind them.  ``layers``: int64 [8 * count] on the device, the
+    layers' pointers (``LayerChain``); ``runs``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
+    for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page"), (tables.pages, "pages")):
+        _dev(t, f"chain {what}")
+    rows = x.shape[0]
+    if (x.shape != (rows, width) or x.dtype != torch.float32 or tables.cos.shape != (rows, head_dim // 2) or tables.tokens != rows or tok_pos.numel() < rows
+            or tok_pos.dtype != torch.int32 or layers.dtype != torch.int64 or layers.numel() != 8 * count or not failed.is_pinned()):
+        raise KernelError(f"chain: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
+    lib = chain_module()
+    words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs)
+    exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
+    partial = decode_scratch(x.device, run_words) if run_words else None  # (as the split decode attention's)
+    out = torch.empty_like(x)
+    _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, _DTYPE_CODE[gain_dtype], float(eps),
+                               float(scale), x.data_ptr(), out.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
+                               tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial),
+                               run_words, failed.data_ptr(),
+                               _stream()))
     return out
 
 

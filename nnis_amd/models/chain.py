@@ -1,0 +1,81 @@
+"""A step of few single tokens through all layers in one launch (``csrc/chain.hip``).
+
+A part that the launch takes says what of it there is (``chain_link``); a model whose every layer does, over one cache and one
+rotation, runs such steps through it, and all others -- other mixers, options, types, sizes, more rows, longer sequences --
+through the layers' own kernels."""
+
+from __future__ import annotations
+
+from typing import Dict, List, Optional
+
+import torch
+
+from ..errors import KernelError
+
+
+class LayerChain:
+    def __init__(self, links: List[dict], rt):
+        """``links``: what each run of the schedule says of itself (``PreNormBlock.chain_link``)."""
+        self.links = links
+        first = links[0]
+        self.sizes = {name: first[name] for name in ("width", "heads", "kv_heads", "head_dim", "inner")}
+        self.eps, self.scale, self.position, self.gain_dtype = first["eps"], first["scale"], first["position"], first["gains"][0].dtype
+        # where a wait that was given up says so: a word of host memory that the kernel writes and the next step reads
+        self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._failed = self.failed.numpy()
+        self.tables: Dict[tuple, torch.Tensor] = {}  # the layers' pointers -> the same on the device
+
+    @classmethod
+    def of(cls, schedule_layers, rt) -> Optional["LayerChain"]:
+        links = []
+        for layer in schedule_layers:
+            link = layer.chain_link(rt) if hasattr(layer, "chain_link") else None
+            if link is None:
+                return None
+            links.append(link)
+        alike = ("width", "heads", "kv_heads", "head_dim", "inner", "eps", "scale", "position")
+        if not links or any(link[name] != links[0][name] for link in links for name in alike):
+            return None
+        if any(gain.dtype != links[0]["gains"][0].dtype or gain.data_ptr() % 16 for link in links for gain in link["gains"]):
+            return None
+        if not rt.ops.chain_takes(len(links), 1, **{n: links[0][n] for n in ("width", "heads", "kv_heads", "head_dim", "inner")}):
+            return None
+        return cls(links, rt)
+
+    def plan(self, batch: int, longest: int, rt):
+        """The runs of a sequence's keys for a step of these sizes, or None: the layers' own kernels."""
+        return rt.ops.chain_plan(len(self.links), batch, longest, **self.sizes)
+
+    def check(self) -> None:
+        """Raises if a wait of an earlier step was given up."""
+        if self._failed[0]:
+            self._failed[0] = 0
+            raise KernelError("a decode step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
+                              "the logits of the step before this one are not numbers")
+
+    def views_fit(self, views) -> bool:
+        """Whether each layer writes keys and values of its own, through one block table."""
+        return all(not getattr(view, "read_only", True) and view.k_pages.dtype == torch.bfloat16
+                   and view.block_table.data_ptr() == views[0].block_table.data_ptr() for view in views)
+
+    def _table(self, views, device) -> Optional[torch.Tensor]:
+        key = tuple(pointer for link, view in zip(self.links, views)
+                    for pointer in (*(w.data_ptr() for w in link["weights"]), *(g.data_ptr() for g in link["gains"]),
+                                    view.k_pages.data_ptr(), view.v_pages.data_ptr()))
+        table = self.tables.get(key)
+        if table is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None  # (the copy below does not belong into a graph; a graph's eager run comes first)
+            while len(self.tables) >= 16:
+                self.tables.pop(next(iter(self.tables)))  # (graphs hold what they were captured with: ``held_tables``)
+            table = self.tables[key] = torch.tensor(key, dtype=torch.int64).to(device)
+        return table
+
+    def forward(self, x: torch.Tensor, ctx, views, plan, rt) -> Optional[torch.Tensor]:
+        """The stream behind the last layer, [rows, width] in 32 bits; None where the launch cannot be made here."""
+        table = self._table(views, x.device)
+        if table is None:
+            return None
+        tables = ctx.step_tables(rt, self.position.rotary(), views[0].block_table)
+        return rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, gain_dtype=self.gain_dtype, eps=self.eps,
+                            scale=self.scale, **self.sizes)

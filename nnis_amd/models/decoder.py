@@ -11,6 +11,7 @@ import torch
 
 from ..parts import build_part
 from ..parts.base import TensorSpec
+from .chain import LayerChain
 from .spec import ModelSpec
 
 
@@ -54,6 +55,15 @@ class DecoderModel:
                     if part is not owner:
                         part.adopt_packed(source, packed)
         self.bound = True
+        # (made when it is first asked for: it wants the kernels, which a model that is only described does without)
+        self._chain, self._chain_made = None, False
+
+    def layer_chain(self, rt):
+        """What runs a step of few single tokens through all layers in one launch (``LayerChain``), or None."""
+        if not self._chain_made:
+            self._chain = None if self.entries else LayerChain.of([self.layers[entry.layer] for entry in self.spec.schedule], rt)
+            self._chain_made = True
+        return self._chain
 
     def step_weight_bytes(self, rows=None) -> int:
         """Bytes of weights a decode step reads: every layer each time the
@@ -81,6 +91,17 @@ class DecoderModel:
         """What the parts' kernels keep between calls and a captured step has baked in (``Part.held_buffers``)."""
         return [buffer for part in self.parts() for buffer in part.held_buffers(rt)]
 
+    def held_tables(self, rt):
+        """The same of the model's own: what a launch through all layers reads their pointers from."""
+        chain = self.layer_chain(rt)
+        return list(chain.tables.values()) if chain is not None else []
+
+    def check_steps(self, rt) -> None:
+        """Raises if the kernels of an earlier step found something wrong that only the host can report."""
+        chain = self.layer_chain(rt)
+        if chain is not None:
+            chain.check()
+
     def prompt_plan(self, batch: int, rows: int, longest: int, rt, most_new: int = 0):
         """The plans of every run of the schedule for a step of prompts (``Part.prompt_plan``, ``Part.run_plan``);
         ``most_new``: the most tokens that a sequence brings (0: all rows of a step of one, their mean of several)."""
@@ -104,7 +125,11 @@ class DecoderModel:
         if plans is None:
             if len(self._plans) > 4096:
                 self._plans.clear()
-            plans = self._plans[key] = tuple(self.layers[entry.layer].decode_plan(batch, longest, rt) for entry in self.spec.schedule)
+            plans = tuple(self.layers[entry.layer].decode_plan(batch, longest, rt) for entry in self.spec.schedule)
+            chain = self.layer_chain(rt)
+            if chain is not None:
+                plans += (("chain", chain.plan(batch, longest, rt)),)
+            self._plans[key] = plans
         return plans
 
     # ---- cache ---------------------------------------------------------------
@@ -127,6 +152,16 @@ class DecoderModel:
         return requests, shared
 
     # ---- forward -------------------------------------------------------------
+    def _chained(self, x, schedule, ctx, cache, rt):
+        """(the stream behind all layers, nothing left to run) where one launch takes the step, else what it was handed."""
+        chain = self.layer_chain(rt) if ctx.decode and not ctx.options else None
+        plan = chain.plan(ctx.batch, ctx.planned_len, rt) if chain is not None else None
+        if plan is None or x.dim() != 2 or x.dtype != torch.float32 or not x.is_contiguous():
+            return x, schedule
+        views = [cache.view(index) for index in range(len(schedule))]
+        done = chain.forward(x, ctx, views, plan, rt) if chain.views_fit(views) else None
+        return (x, schedule) if done is None else (done, ())
+
     def forward(self, ids: torch.Tensor, ctx, cache, want_rows: torch.Tensor, rt) -> torch.Tensor:
         """ids: int32 [tokens] on the device; want_rows: int32 indices of the
         packed tokens whose logits are asked for.  Returns float32
@@ -145,8 +180,9 @@ class DecoderModel:
             # kept as it is for the entries that add it again: an entry writes a stream that still is this tensor into
             # a new one; a layer that runs first would write into it
             embedded = x if 0 in self.entries else x.clone()
-        stream = (x, None)
         schedule = self.spec.schedule
+        x, schedule = self._chained(x, schedule, ctx, cache, rt)
+        stream = (x, None)
         for index, entry in enumerate(schedule):
             layer = self.layers[entry.layer]
             if index in self.entries:

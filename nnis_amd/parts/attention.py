@@ -226,6 +226,17 @@ class CausalSelfAttention(Mixer):
         held = rt.ops.decode_scratch_held(rt.device)
         return [] if held is None else [held]
 
+    def chain_link(self, rt):
+        """See ``PreNormBlock.chain_link``: the plain formula, whole heads rotated, no window."""
+        tables = self.position.rotary() if self.position is not None else None
+        plain = (type(self) is CausalSelfAttention and self._plain and not self.softcap and not self.window and not self.chunk and not self.extras
+                 and self.gate_name is None and self.unit_eps is None and not any(self.bias_names.values()))
+        if (not plain or tables is None or tables.rot_dim != self.head_dim or getattr(self.position, "pairing", None) == "neighbours"
+                or not all(isinstance(p.weight, rt.ops.PackedWeight) for p in (self.qkv, self.out))):
+            return None
+        return {"heads": self.heads, "kv_heads": self.kv_heads, "head_dim": self.head_dim, "scale": self.scale, "position": self.position,
+                "weights": [self.qkv.weight, self.out.weight]}
+
     takes_pending_norm = True
     adds_to_residual = True
 

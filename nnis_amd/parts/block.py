@@ -89,6 +89,18 @@ class PreNormBlock(Block):
         """The norm a stream meets first here: a block before this one may prepare it."""
         return self.norm1
 
+    def chain_link(self, rt):
+        """What this layer is to a launch of all layers (``models/chain.py``), or None if that does not take it."""
+        if type(self) is not PreNormBlock or self.feed_forward is None or self.side is not None or rt.is_fp32:
+            return None
+        norms = (self.norm1, self.norm2)
+        parts = [part.chain_link(rt) if hasattr(part, "chain_link") else None for part in (self.mixer, self.feed_forward)]
+        if None in parts or not all(getattr(norm, "fusable_rms", False) and norm.width == self.width and norm.eps == norms[0].eps for norm in norms):
+            return None
+        mixer, feed_forward = parts
+        return {**mixer, **feed_forward, "width": self.width, "eps": norms[0].eps, "gains": [norm.weight for norm in norms],
+                "weights": mixer["weights"] + feed_forward["weights"]}
+
     def _run(self, part, normed, args, then, rt):
         """Runs a mixer or feed-forward on a pending norm; returns the pending
         norm ``then`` of the stream with the part's output (or, without

@@ -42,6 +42,13 @@ class GatedFeedForward(FeedForward):
     def weight_bytes(self):
         return self.gate_up.weight_bytes() + self.down.weight_bytes()
 
+    def chain_link(self, rt):
+        """See ``PreNormBlock.chain_link``."""
+        if (type(self) is not GatedFeedForward or self.activation != "silu"
+                or not all(isinstance(p.weight, rt.ops.PackedWeight) for p in (self.gate_up, self.down))):
+            return None
+        return {"inner": self.inner, "weights": [self.gate_up.weight, self.down.weight]}
+
     takes_pending_norm = True
     adds_to_residual = True
 

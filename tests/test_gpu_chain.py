@@ -1,0 +1,119 @@
+"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``) against the layers' own kernels, both
+measured by the 32-bit path on the same weights.  Sizes are those at which the launch changes what it does: a K that leaves
+waves without a chunk or takes them a second round, groups of heads beyond four, four and eight waves, runs of the keys."""
+
+import numpy as np
+import pytest
+import torch
+
+from configs import llama
+from nnis_amd.errors import KernelError
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(width, heads, kv_heads, inner, layers=2):
+    return llama(num_hidden_layers=layers, hidden_size=width, num_attention_heads=heads, num_key_value_heads=kv_heads, head_dim=64,
+                 intermediate_size=inner, vocab_size=509, rope_theta=10000.0, rms_norm_eps=1e-5, tie_word_embeddings=True,
+                 max_position_embeddings=4096, torch_dtype="bfloat16")
+
+
+# width, query heads, key heads, inner size
+SIZES = [
+    (64, 1, 1, 64),        # one chunk of K: three of four waves have no share of it
+    (320, 5, 1, 128),      # a group of five heads
+    (192, 6, 2, 1600),     # down takes 25 chunks: a wave's second round of weights
+    (1024, 14, 2, 448),    # the widest of four waves; the output projection's second round
+    (1088, 8, 8, 576),     # eight waves, 17 chunks; a head a key head
+    (1152, 16, 2, 8256),   # down takes 129 chunks
+]
+# lengths before the step: the first token, pages' ends, runs
+LENGTHS = [1, 63, 64, 65, 200, 1023, 1100, 5, 128, 320, 577, 129, 31, 2000, 90, 447]
+
+
+def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
+    """The logits of ``steps`` steps of single tokens behind prompts of these lengths, [steps, sequences, vocab]."""
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    with monkeypatch.context() as patch:
+        if plan != "own":
+            patch.setattr(ops, "chain_plan", lambda *args, **sizes: plan)
+        engine = load_engine(folder, dtype=dtype, max_tokens=sum(-(-(n + steps + 1) // 64) * 64 for n in lengths))
+        rng = np.random.default_rng(sum(lengths))
+        slots = [engine.start_sequence() for _ in lengths]
+        engine.step([StepEntry(slot, rng.integers(0, 509, size=n).tolist(), None) for slot, n in zip(slots, lengths)])
+        out = []
+        for _ in range(steps):
+            tokens = rng.integers(0, 509, size=len(lengths)).tolist()
+            entries = [StepEntry(slot, [token], None) for slot, token in zip(slots, tokens)]
+            out.append(engine.step(entries).double().cpu())
+            if len(out) == 1:  # the same step again, replayed over what the first left in the exchange
+                for slot, n in zip(slots, lengths):
+                    engine.truncate(slot, n)
+                assert torch.equal(engine.step(entries).double().cpu(), out[0])
+        chain = engine.model.layer_chain(engine.rt)
+        ran = chain is not None and len(chain.tables) > 0
+        return torch.stack(out), ran, engine
+
+
+@pytest.mark.parametrize("batch", [1, 3, 16])
+@pytest.mark.parametrize("sizes", SIZES)
+def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
+    """As far from 32 bits as the layers' kernels: the same roundings in another order.  (Their distances are equal but for
+    which roundings fall together; over a few hundred logits that is within a third.)"""
+    import nnis_amd
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    lengths = LENGTHS[:batch] if batch > 1 else [1100]
+    want, ran, _ = _run(str(tmp_path), "float32", lengths, "own", monkeypatch)
+    assert not ran
+    layers, ran, _ = _run(str(tmp_path), "bfloat16", lengths, None, monkeypatch)
+    assert not ran
+    bound = 1.33 * (layers - want).norm()
+    for plan in ("own", 1, 2, 16):
+        got, ran, _ = _run(str(tmp_path), "bfloat16", lengths, plan, monkeypatch)
+        assert ran, f"plan {plan}: the launch was not made"
+        error = (got - want).norm()
+        assert error <= bound, f"plan {plan}: {error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
+
+
+def test_not_taken(tmp_path, monkeypatch):
+    """Other head sizes, sizes in other steps than 64 and 32 bits stay with the layers' kernels."""
+    import nnis_amd
+
+    for index, change in enumerate(({"head_dim": 32}, {"intermediate_size": 176})):
+        folder = tmp_path / str(index)
+        folder.mkdir()
+        nnis_amd.write_random_model(str(folder), dict(_config(64, 1, 1, 64), **change), 3)
+        assert not _run(str(folder), "bfloat16", [40], "own", monkeypatch)[1]
+
+
+def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
+    """The word that a kernel writes when it gives a wait up (written here by the host) refuses the next step, once."""
+    import nnis_amd
+    from nnis_amd.engine.batch import StepEntry
+
+    nnis_amd.write_random_model(str(tmp_path), _config(64, 1, 1, 64), 3)
+    _, ran, engine = _run(str(tmp_path), "bfloat16", [40], "own", monkeypatch)
+    assert ran
+    slot = next(iter(engine.cache.lengths))
+    length = engine.length(slot)
+    engine.model.layer_chain(engine.rt).failed[0] = 1
+    with pytest.raises(KernelError, match="gave up waiting"):
+        engine.step([StepEntry(slot, [7], None)])
+    assert engine.length(slot) == length
+    assert bool(torch.isfinite(engine.step([StepEntry(slot, [7], None)])).all())
+
+
+def test_sizes_and_words():
+    """The exchange's size is 0 for what the launch refuses, and grows with what it holds."""
+    from nnis_amd.kernels import ops
+
+    words = ops.chain_words
+    assert words(2, 1, 64, 1, 1, 64, 1)[0] > 0 and words(2, 1, 64, 1, 1, 64, 1)[1] == 0
+    assert words(2, 2, 64, 1, 1, 64, 1)[0] > words(2, 1, 64, 1, 1, 64, 1)[0] and words(2, 2, 64, 1, 1, 64, 2)[1] == 2 * 2 * 2 * 68
+    for refused in ((2, 17, 64, 1, 1, 64, 1), (2, 0, 64, 1, 1, 64, 1), (2, 1, 96, 1, 1, 64, 1), (2, 1, 64, 3, 2, 64, 1), (2, 1, 64, 1, 1, 80, 1),
+                    (2, 1, 64, 1, 1, 64, 17), (0, 1, 64, 1, 1, 64, 1)):
+        assert words(*refused)[0] == 0
