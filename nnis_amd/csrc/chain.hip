@@ -48,9 +48,13 @@ struct ChainLayer {
 struct ChainArgs {
   const ChainLayer* layers;
   int layer_count, m, width, heads, kv_heads, inner, splits, gain_dtype;
+  // how many ways K is cut (the first layer's queries, keys and values; the others'; output, gate/up, down), and the waves that
+  // share a run's pages
+  int parts_first, parts_qkv, parts_out, parts_gate, parts_down, page_waves;
   float eps, scale_log2;
   const float* x;  // [m, width]
-  float* x_out;    // [m, width]: the stream behind the last layer
+  float* x_out;    // [m, width]: the stream behind the last attention
+  bf16_t* y_out;   // [m, width]: what the last feed-forward adds to it
   const float *tok_cos, *tok_sin;
   const int *tok_pos, *tok_page, *tok_pages;
   int max_pages;
@@ -172,70 +176,78 @@ struct Exchange {
 
 __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
 
-// STRIPS strips of 16 weight rows times the step's rows; the block's waves share K (chunks of 64, whole).  A wave asks for the
-// weights of its first STEPS chunks when the block begins; XB chunks of the operand are asked for together.  A step of the operand
-// beyond the last chunk reads the last again and is not multiplied.
-template <int WAVES, int STRIPS, int STEPS, int XB>
+// STRIPS strips of 16 weight rows times the step's rows.  K (chunks of 64, whole) is cut `parts` ways: part p has the chunks p, p +
+// parts, ..; a wave has V parts, its own number and those WAVES on.  It asks for the weights of its first STEPS chunks when the
+// block begins; XB chunks of the operand are asked for together.  A step of the operand beyond the last chunk reads the last again
+// and is not multiplied.  The parts and the order of their sums are those of the layers' own kernels for the same product.
+template <int WAVES, int STRIPS, int STEPS, int XB, int V>
 struct Product {
-  static_assert(STEPS % XB == 0, "whole trips");
+  static_assert(STEPS % XB == 0 && STEPS % V == 0, "whole trips");
   bf16x8 w[STEPS][2][STRIPS];
-  f32x4 acc[STRIPS];
+  f32x4 acc[V][STRIPS];
   const bf16_t* strip[STRIPS];
-  int chunks, part, lane;
+  int chunks, parts, wave, lane;
 
-  __device__ __forceinline__ void ask(int base) {
+  // the chunk of step `s` of the round that begins with a part's chunk number `d0`; `chunks` and more: none
+  __device__ __forceinline__ int chunk(int d0, int s) const {
+    const int part = wave + WAVES * (s / (STEPS / V));
+    return V > 1 && part >= parts ? chunks : part + parts * (d0 + s % (STEPS / V));
+  }
+  __device__ __forceinline__ void ask(int d0) {
 #pragma unroll
     for (int d = 0; d < STEPS; ++d) {
-      if (base + d * WAVES >= chunks) break;  // (the same for the whole wave)
+      const int c = chunk(d0, d);
+      if (c >= chunks) continue;  // (the same for the whole wave)
 #pragma unroll
       for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int j = 0; j < STRIPS; ++j)
-          w[d][half][j] = load_packed(strip[j] + (size_t)(base + d * WAVES) * kPackedChunkElems + half * kPackedHalfElems + lane * 8);
+        for (int j = 0; j < STRIPS; ++j) w[d][half][j] = load_packed(strip[j] + (size_t)c * kPackedChunkElems + half * kPackedHalfElems + lane * 8);
     }
   }
   // row(j): the first row of strip j
   template <typename Row>
-  __device__ __forceinline__ void begin(const bf16_t* weight, Row row, int k, int lane_, int part_) {
-    part = part_;
+  __device__ __forceinline__ void begin(const bf16_t* weight, Row row, int k, int parts_, int lane_, int wave_) {
+    parts = parts_;
+    wave = wave_;
     lane = lane_;
     chunks = nnis_packed_chunks(k);
 #pragma unroll
     for (int j = 0; j < STRIPS; ++j) {
       strip[j] = weight + (size_t)(row(j) / 16) * nnis_packed_strip_elems(k);
-      acc[j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
     }
-    ask(part);
+    if (wave < parts) ask(0);
   }
-  // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`.  SUM: the strips are the
-  // stream's records; returns the lane's share of its row's sum of squares.
-  template <bool SUM>
-  __device__ __forceinline__ float run(const Exchange& ex, unsigned row_at, unsigned stride) {
-    float ss = 0.0f;
+  // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
+  // every chunk with the lane's part of its row's sum of squares, if SUM: the strips are then the stream's records.
+  template <bool SUM, typename Sum>
+  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, Sum sum) {
     const unsigned at = row_at + lane / 16 * stride;
-    for (int base = part; base < chunks; base += WAVES * STEPS) {
-      if (base != part) ask(base);
+    for (int d0 = 0; wave < parts && wave + parts * d0 < chunks; d0 += STEPS / V) {
+      if (d0 > 0) ask(d0);
 #pragma unroll
       for (int b = 0; b < STEPS; b += XB) {
-        if (base + b * WAVES >= chunks) continue;
+        if (XB <= STEPS / V && chunk(d0, b) >= chunks) continue;  // (no step of the trip has a chunk)
         u32x4 v[XB * 2];
-        unsigned sum[XB];
-        auto step = [&](int d) { return (unsigned)min(base + (b + d) * WAVES, chunks - 1) * 4 * stride; };
+        unsigned part[XB];
+        auto step = [&](int d) { return (unsigned)min(chunk(d0, b + d), chunks - 1) * 4 * stride; };
         auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
-        if constexpr (SUM) ex.take(v, pieces, sum, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
+        if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
         else ex.take(v, pieces);
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
-          if (base + (b + d) * WAVES >= chunks) continue;
-          if constexpr (SUM) ss += __uint_as_float(sum[d]);
+          const int c = chunk(d0, b + d);
+          if (c >= chunks) continue;
+          if constexpr (SUM) sum(c, __uint_as_float(part[d]));
 #pragma unroll
           for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int j = 0; j < STRIPS; ++j) acc[j] = mfma(w[b + d][half][j], __builtin_bit_cast(bf16x8, v[2 * d + half]), acc[j]);
+            for (int j = 0; j < STRIPS; ++j)
+              acc[(b + d) / (STEPS / V)][j] = mfma(w[b + d][half][j], __builtin_bit_cast(bf16x8, v[2 * d + half]), acc[(b + d) / (STEPS / V)][j]);
         }
       }
     }
-    return ss;
   }
 };
 
@@ -259,14 +271,15 @@ constexpr int into_units_of() { return DOWN ? 1 : units_of<WAVES>(); }
 
 template <int WAVES>
 struct Shared {
+  static constexpr int kSums = WAVES == 4 ? 16 : WAVES;  // four waves: a sum a chunk of K; eight: one a wave
   union {
     struct {
-      float acc[WAVES][WAVES == 8 ? 4 : 2][kWave][4];
-      float ss[WAVES][kWave];
+      float acc[WAVES][4][kWave][4];
+      float ss[kSums][kWave];
     } product;
     struct {
       __attribute__((aligned(16))) float o[WAVES][4][HD];
-      float m[WAVES][4], l[WAVES][4];
+      float m[WAVES][4], l[WAVES][4][4];
       bf16x8 heads[WAVES][kWave];
       __attribute__((aligned(16))) bf16_t stage[WAVES][4][kPageTokens + 8];
     } attention;
@@ -274,44 +287,82 @@ struct Shared {
   };
 };
 
-// The waves' sums added up: of a block's UNITS units of NACC strips, unit u's in wave u (sums[NACC], ss); false for waves that have none.
-template <int WAVES, int UNITS, int NACC>
-__device__ __forceinline__ bool add_waves(Shared<WAVES>& s, const f32x4 (&acc)[UNITS * NACC], f32x4 (&sums)[NACC], float& ss, int wave, int lane) {
-  ss += __shfl_xor(ss, 16, kWave);
-  ss += __shfl_xor(ss, 32, kWave);
+// The parts of K added up, in their order: of a block's UNITS units of NACC strips, unit u's in wave u; false for waves that have none.
+template <int WAVES, int UNITS, int NACC, int V>
+__device__ __forceinline__ bool add_parts(Shared<WAVES>& s, const f32x4 (&acc)[V][UNITS * NACC], f32x4 (&sums)[NACC], int wave, int lane) {
+  static_assert(V * UNITS * NACC <= 4 && (V == 1 || UNITS == 1), "room for the sums");
 #pragma unroll
-  for (int u = 0; u < UNITS; ++u)
-    if (wave != u) {
+  for (int v = 0; v < V; ++v)
 #pragma unroll
-      for (int j = 0; j < NACC; ++j) *(f32x4*)s.product.acc[wave][u * NACC + j][lane] = acc[u * NACC + j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < NACC; ++j) sums[j] = acc[u * NACC + j];
-    }
-  s.product.ss[wave][lane] = ss;
+    for (int j = 0; j < UNITS * NACC; ++j) *(f32x4*)s.product.acc[wave][v * UNITS * NACC + j][lane] = acc[v][j];
   __syncthreads();
   if (wave >= UNITS) return false;
 #pragma unroll
-  for (int i = 1; i < WAVES; ++i) {
-    const int other = (wave + i) % WAVES;
+  for (int j = 0; j < NACC; ++j) {
+    sums[j] = *(const f32x4*)s.product.acc[0][wave * NACC + j][lane];
 #pragma unroll
-    for (int j = 0; j < NACC; ++j) sums[j] += *(const f32x4*)s.product.acc[other][wave * NACC + j][lane];
-    ss += s.product.ss[other][lane];
+    for (int part = 1; part < WAVES * V; ++part) sums[j] += *(const f32x4*)s.product.acc[part % WAVES][part / WAVES * UNITS * NACC + wave * NACC + j][lane];
   }
   return true;
 }
 
-// a row of the embedding into the first layer's records; its sum of squares is one part
+// a product with a row that a norm prepared, from the records at word `first_word`; `sums` and the row's scale in the waves that end a unit
+template <int WAVES, int UNITS, int NACC, int V, typename P>
+__device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, P& p, unsigned first_word, int row, int wave, int lane,
+                                             f32x4 (&sums)[NACC], float& scale) {
+  // The row's sum of squares is added up as the layers' kernels do: four waves' rows (up to 64 parts) chunk by chunk by one wave,
+  // eight waves' each wave's own chunks first.
+  float ss = 0.0f;
+  p.template run<true>(ex, (first_word + row * kRecord) * 4, a.m * kRecord * 4, [&](int c, float part) {
+    if constexpr (WAVES == 4) s.product.ss[c][lane] = part;
+    else ss += part;
+  });
+  if constexpr (WAVES != 4) {
+    ss += __shfl_xor(ss, 16, kWave);
+    ss += __shfl_xor(ss, 32, kWave);
+    s.product.ss[wave][lane] = ss;
+  }
+  if (!add_parts<WAVES, UNITS, NACC, V>(s, p.acc, sums, wave, lane)) return false;
+  ss = 0.0f;
+  if constexpr (WAVES == 4) {
+    float part[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) part[c] = s.product.ss[c][lane];  // (beyond the chunks: whatever is there, not added)
+#pragma unroll
+    for (int c = 0; c < 16; ++c) ss = c < p.chunks ? ss + part[c] : ss;
+    ss += __shfl_xor(ss, 16, kWave);
+    ss += __shfl_xor(ss, 32, kWave);
+  } else {
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) ss += s.product.ss[w][lane];
+  }
+  scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  return true;
+}
+
+// A row of the embedding into the first layer's records.  Its sum of squares is one part, added up as the layers' kernel for a row
+// that no norm has prepared does: a lane per (part of K, 16 of a chunk's 64 channels).
 template <int WAVES>
 __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int row) {
   const float* x = a.x + (size_t)row * a.width;
-  float sum = 0.0f;
-  for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
-    const f32x4 v = *(const f32x4*)(x + c);
+  if (threadIdx.x < kWave) {
+    const int part = threadIdx.x / 4, g = threadIdx.x % 4, parts = a.parts_first;
+    float sum = 0.0f;
+    for (int c = part; part < parts && c < a.width / 64; c += parts) {
+      f32x4 v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sum = fmaf(v[e], v[e], sum);
+      for (int i = 0; i < 4; ++i) v[i] = *(const f32x4*)(x + c * 64 + g * 16 + 4 * i);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum = fmaf(v[i / 4][i % 4], v[i / 4][i % 4], sum);
+    }
+    sum += __shfl_xor(sum, 1, kWave);
+    sum += __shfl_xor(sum, 2, kWave);
+    float total = __shfl(sum, 0, kWave);
+    for (int p = 1; p < parts; ++p) total += __shfl(sum, 4 * p, kWave);
+    if (threadIdx.x == 0) s.sums[0] = total;
   }
-  sum = block_sum(sum, s.sums);
+  __syncthreads();
+  const float sum = s.sums[0];
   for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
     const f32x4 v = *(const f32x4*)(x + c);
     const f32x4 gain = four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
@@ -323,26 +374,26 @@ __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& 
 }
 
 // queries, keys and values of two strips (a head's channels f .. f + 15 and f + 32 ..), rotated, and the write into the cache
-template <int WAVES>
+template <int WAVES, bool FIRST>
 __device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int unit) {
-  constexpr bool kNear = WAVES == 8;
+  constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const ChainLayer& L = a.layers[layer];
   const unsigned here = layer * a.layer_words;
   // unit 2 h + i of all: channels 16 i .. 16 i + 15 of head h and those half a head on
   constexpr int kUnits = units_of<WAVES>();
-  Product<WAVES, 2 * kUnits, 4, 4> p;
-  p.begin(L.w_qkv, [&](int j) { const int u = unit * kUnits + j / 2; return u / 2 * HD + u % 2 * 16 + j % 2 * (HD / 2); }, a.width, lane, wave);
+  constexpr int kParts = FIRST && WAVES == 4 ? 2 : 1;  // (a row that no norm has prepared has K cut up to eight ways)
+  Product<WAVES, 2 * kUnits, 4, 4, kParts> p;
+  p.begin(L.w_qkv, [&](int j) { const int u = unit * kUnits + j / 2; return u / 2 * HD + u % 2 * 16 + j % 2 * (HD / 2); }, a.width,
+          FIRST ? a.parts_first : a.parts_qkv, lane, wave);
   const int row = r < a.m ? r : a.m - 1, ends = unit * kUnits + (wave < kUnits ? wave : 0), head = ends / 2, f0 = ends % 2 * 16;
   const f32x4 c = *(const f32x4*)(a.tok_cos + row * (HD / 2) + f0 + 4 * g), sn = *(const f32x4*)(a.tok_sin + row * (HD / 2) + f0 + 4 * g);
   const int pos = a.tok_pos[row], page = a.tok_page[row];
-  if (kNear) ex.template gate<kNear>(here + a.stream1 + unit * 61 % (a.m * a.n_strip) * kRecord, wave);
-  else if (layer > 0) ex.template gate<kNear>(here - a.layer_words + a.act + unit * 61 % (a.m * a.inner / 2), wave);
-  float ss = p.template run<true>(ex, (here + a.stream1 + row * kRecord) * 4, a.m * kRecord * 4);
+  ex.template gate<kOne>(here + a.stream1 + unit * 61 % (a.m * a.n_strip) * kRecord, wave);
   f32x4 sums[2];
-  if (!add_waves<WAVES, kUnits, 2>(s, p.acc, sums, ss, wave, lane)) return;
+  float scale;
+  if (!run_prepared<WAVES, kUnits, 2, kParts>(a, ex, s, p, here + a.stream1, row, wave, lane, sums, scale)) return;
   if (r >= a.m) return;
-  const float scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
   const f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
   f32x4 out_lo = lo, out_hi = hi;
   if (head < a.heads + a.kv_heads) {
@@ -401,7 +452,7 @@ __device__ __forceinline__ bf16x4 high4(bf16x8 v) { return __builtin_shufflevect
 // projection's blocks of this launch are still writing: it comes from the exchange and takes its place in the page's operands.
 template <int WAVES>
 __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int item) {
-  constexpr bool kNear = WAVES == 8;
+  constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const int blk = lane / 4, j = lane % 4;
   const ChainLayer& L = a.layers[layer];
@@ -415,19 +466,18 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   const int page_count = pos / kPageTokens + 1;
   const int per_split = (page_count + a.splits - 1) / a.splits;
   const int begin = split * per_split, end = min(begin + per_split, page_count);
-  // the run's pages are dealt to the waves from its end, so that the page of the step's own key is its wave's first
-  const int last = end - 1 - wave, mine = last >= begin ? (last - begin) / WAVES + 1 : 0;
+  const int first = begin + wave, stride = a.page_waves, mine = wave < stride && end > first ? (end - first + stride - 1) / stride : 0;
   const bf16_t* k_base = L.k_pages + (size_t)kv_head * nnis_k_page_elems(HD);
   const bf16_t* v_base = L.v_pages + (size_t)kv_head * nnis_v_page_elems(HD);
   const size_t k_stride = (size_t)a.kv_heads * nnis_k_page_elems(HD), v_stride = (size_t)a.kv_heads * nnis_v_page_elems(HD);
   KeysPage f;
   if (mine > 0) {
-    const size_t page = __builtin_amdgcn_readfirstlane(pages[last]);
+    const size_t page = __builtin_amdgcn_readfirstlane(pages[first]);
     load_keys(f, k_base + page * k_stride, lane);
     load_values(f, v_base + page * v_stride, lane);
   }
-  if (kNear) ex.template gate<kNear>(here + a.q + ((first_head * (HD / 16) + item * 61 % (HD / 16)) * a.m + token) * 8, wave);
-  else ex.template gate<kNear>(here + a.stream1 + item * 61 % (a.m * a.n_strip) * kRecord, wave);
+  if (kOne) ex.template gate<kOne>(here + a.q + ((first_head * (HD / 16) + item * 61 % (HD / 16)) * a.m + token) * 8, wave);
+  else ex.template gate<kOne>(here + a.stream1 + item * 61 % (a.m * a.n_strip) * kRecord, wave);
   // Queries and the step's own key and value in one load of the wave (8 lanes a head's row, [head][strip][row]: two pieces a
   // strip), and from there through LDS.
   bf16x8* heads_lds = s.attention.heads[wave];
@@ -444,30 +494,6 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   bf16x8 q[HD / 8];
 #pragma unroll
   for (int c = 0; c < HD / 8; ++c) q[c] = heads_lds[8 * j + c];
-  if (mine > 0 && last == pos / kPageTokens) {  // the step's own key and value take their places in the page's operands
-    const int at_key = pos % kPageTokens, h_at = at_key / 32, e_at = at_key % 8;
-    if (lane == at_key) {
-#pragma unroll
-      for (int c = 0; c < HD / 8; ++c) f.k[c] = heads_lds[32 + c];
-    }
-    if (g == at_key % 32 / 8) {
-      const unsigned short* value = (const unsigned short*)(heads_lds + 40) + r;
-#pragma unroll
-      for (int t = 0; t < HD / 16; ++t) {
-        const unsigned short channel = value[16 * t];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          u32x4 words = __builtin_bit_cast(u32x4, f.v[h][t]);
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const unsigned put = e_at % 2 ? (words[w] & 0xffffu) | ((unsigned)channel << 16) : (words[w] & 0xffff0000u) | channel;
-            words[w] = h == h_at && w == e_at / 2 ? put : words[w];
-          }
-          f.v[h][t] = __builtin_bit_cast(bf16x8, words);
-        }
-      }
-    }
-  }
   f32x4 o[HD / 16];
 #pragma unroll
   for (int t = 0; t < HD / 16; ++t) o[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
@@ -475,7 +501,31 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   bf16_t* stage = &s.attention.stage[wave][0][0];
   constexpr int kStageRow = kPageTokens + 8;
   for (int n = 0; n < mine; ++n) {
-    const int index = last - n * WAVES, key0 = index * kPageTokens;
+    const int index = first + n * stride, key0 = index * kPageTokens;
+    if (index == pos / kPageTokens) {  // the step's own key and value take their places in the page's operands
+      const int at_key = pos % kPageTokens, h_at = at_key / 32, e_at = at_key % 8;
+      if (lane == at_key) {
+  #pragma unroll
+        for (int c = 0; c < HD / 8; ++c) f.k[c] = heads_lds[32 + c];
+      }
+      if (g == at_key % 32 / 8) {
+        const unsigned short* value = (const unsigned short*)(heads_lds + 40) + r;
+  #pragma unroll
+        for (int t = 0; t < HD / 16; ++t) {
+          const unsigned short channel = value[16 * t];
+  #pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            u32x4 words = __builtin_bit_cast(u32x4, f.v[h][t]);
+  #pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const unsigned put = e_at % 2 ? (words[w] & 0xffffu) | ((unsigned)channel << 16) : (words[w] & 0xffff0000u) | channel;
+              words[w] = h == h_at && w == e_at / 2 ? put : words[w];
+            }
+            f.v[h][t] = __builtin_bit_cast(bf16x8, words);
+          }
+        }
+      }
+    }
     f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int c = 0; c < HD / 8; ++c) {
@@ -483,7 +533,7 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
       s1 = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(high4(f.k[c]), high4(q[c]), s1, 0, 0, 0);
     }
     const bool more = n + 1 < mine;
-    const size_t next = more ? __builtin_amdgcn_readfirstlane(pages[index - WAVES]) : 0;
+    const size_t next = more ? __builtin_amdgcn_readfirstlane(pages[index + stride]) : 0;
     if (more) load_keys(f, k_base + next * k_stride, lane);
     f32x4 sc = s0 + s1;
     float top = -INFINITY;
@@ -525,48 +575,72 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
     }
     if (more) load_values(f, v_base + next * v_stride, lane);
   }
-#pragma unroll
-  for (int offset = 4; offset < kWave; offset <<= 1) sum += __shfl_xor(sum, offset, kWave);
+  // the states meet in LDS: a lane group's part of a head's sum is that of the keys 16 g .. 16 g + 15 of its pages
+  sum += __shfl_xor(sum, 4, kWave);
+  sum += __shfl_xor(sum, 8, kWave);
   if (r < 4) {
 #pragma unroll
     for (int t = 0; t < HD / 16; ++t) *(f32x4*)&s.attention.o[wave][r][16 * t + 4 * g] = o[t];
-  }
-  if (lane < 4) {
-    s.attention.m[wave][lane] = reference;
-    s.attention.l[wave][lane] = sum;
+    s.attention.l[wave][r][g] = sum;
+    if (g == 0) s.attention.m[wave][r] = reference;
   }
   __syncthreads();
   const Exchange runs(a, a.run_words, a.run_bytes);
   // four channels of a head a thread, and one thread a head for the run's reference and sum
   for (int i = threadIdx.x; i < heads_here * (HD / 4 + 1); i += 64 * WAVES) {
     const int head = i / (HD / 4 + 1), four = i % (HD / 4 + 1);
-    float top = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, s.attention.m[w][head]);
-    f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
-    float den = 0.0f;
+    // the waves' states in halving rounds, as the layers' kernel has them
+    float m[WAVES];
+    f32x4 l[WAVES], out[WAVES];
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const float m = s.attention.m[w][head], weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
-      num += *(const f32x4*)&s.attention.o[w][head][four < HD / 4 ? 4 * four : 0] * weight;
-      den += s.attention.l[w][head] * weight;
+      m[w] = s.attention.m[w][head];
+      l[w] = *(const f32x4*)s.attention.l[w][head];
+      out[w] = *(const f32x4*)&s.attention.o[w][head][four < HD / 4 ? 4 * four : 0];
     }
+#pragma unroll
+    for (int half = WAVES / 2; half >= 1; half >>= 1) {
+      if (half >= a.page_waves) continue;
+#pragma unroll
+      for (int w = 0; w < half; ++w) {
+        const float m_new = fmaxf(m[w], m[w + half]), m_safe = m_new == -INFINITY ? 0.0f : m_new;
+        const float mine_w = __builtin_amdgcn_exp2f(m[w] - m_safe), their_w = __builtin_amdgcn_exp2f(m[w + half] - m_safe);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // (which of a sum's two products is rounded first is the compiler's choice there: the other one for the last 16 channels)
+          l[w][e] = fmaf(l[w + half][e], their_w, l[w][e] * mine_w);
+          out[w][e] = four >= 12 ? fmaf(out[w][e], mine_w, out[w + half][e] * their_w) : fmaf(out[w + half][e], their_w, out[w][e] * mine_w);
+        }
+        m[w] = m_new;
+      }
+    }
+    const float total = (l[0][0] + l[0][1]) + (l[0][2] + l[0][3]);
+    f32x4 num = out[0];
     if (a.splits == 1) {
-      num = num / den;
+      const float inv = 1.0f / total;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) num[e] = num[e] * inv;
       if (four < HD / 4)
         ex.put(here + a.attn + (((first_head + head) * (HD / 16) + four / 4) * a.m + token) * 8 + four % 4 * 2,
                (u32x2){marked2((bf16_t)num[0], (bf16_t)num[1]), marked2((bf16_t)num[2], (bf16_t)num[3])});
     } else {
-      if (four == HD / 4) num = (f32x4){top, den, 0.0f, 0.0f};
+      if (four == HD / 4) num = (f32x4){m[0], total, 0.0f, 0.0f};
       runs.put(layer * a.layer_runs + ((token * a.heads + first_head + head) * a.splits + split) * kRunRow + 4 * four,
              (u32x4){marked(num[0]), marked(num[1]), marked(num[2]), marked(num[3])});
     }
   }
 }
 
-// Four channels of a (row, head) from its runs, RUNS at once: a head is 16 lanes, a wave has four.
+__device__ __forceinline__ float rounded_sum(float sum, float a, float b) {
+#pragma clang fp contract(off)
+  const float product = a * b;
+  return sum + product;
+}
+
+// Four channels of a (row, head) from its runs, RUNS at once: a head is 16 lanes, a wave has four.  alone: in the roundings of the
+// layers' kernel of its own for this sum (more than four rows), not of the output projection that makes it on the way.
 template <int RUNS>
-__device__ __forceinline__ bf16x4 sum_runs(const Exchange& ex, unsigned first_word, int splits, int channel) {
+__device__ __forceinline__ bf16x4 sum_runs(const Exchange& ex, unsigned first_word, int splits, int channel, bool alone) {
   u32x4 v[RUNS];
   u32x2 state[RUNS];
   ex.take(v, [&](int i) { return At{(first_word + channel) * 4, (unsigned)(i < splits ? i : 0) * kRunRow * 4}; }, state,
@@ -581,7 +655,8 @@ __device__ __forceinline__ bf16x4 sum_runs(const Exchange& ex, unsigned first_wo
     if (i < splits) {
       const float m = __uint_as_float(state[i][0]), weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
       num += __builtin_bit_cast(f32x4, v[i]) * weight;
-      den += __uint_as_float(state[i][1]) * weight;
+      const float add = __uint_as_float(state[i][1]);
+      den = alone ? rounded_sum(den, add, weight) : fmaf(add, weight, den);
     }
   bf16x4 out;
 #pragma unroll
@@ -597,9 +672,10 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
   const int item = min(first + lane / 16, items - 1), head = item / a.m, row = item % a.m, channel = lane % 16 * 4;
   ex.template gate<false>(here + a.q + first * 61 % (items * (HD / 2)), 0);
   const Exchange runs(a, a.run_words, a.run_bytes);
+  const bool alone = a.m > 4;
   const unsigned first_run = layer * a.layer_runs + (row * a.heads + head) * a.splits * kRunRow;
-  const bf16x4 out = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel)
-                     : a.splits <= 8 ? sum_runs<8>(runs, first_run, a.splits, channel) : sum_runs<16>(runs, first_run, a.splits, channel);
+  const bf16x4 out = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, alone)
+                     : a.splits <= 8 ? sum_runs<8>(runs, first_run, a.splits, channel, alone) : sum_runs<16>(runs, first_run, a.splits, channel, alone);
   ex.put(here + a.attn + ((head * (HD / 16) + channel / 16) * a.m + row) * 8 + channel % 16 / 2,
          (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
 }
@@ -607,30 +683,38 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
 // a strip of 16 columns of the stream: the output projection (down = false) or the feed-forward's down
 template <int WAVES, bool DOWN>
 __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
-  constexpr bool kNear = WAVES == 8;
+  constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const ChainLayer& L = a.layers[layer];
   const unsigned here = layer * a.layer_words, next = here + (DOWN ? a.layer_words : 0);
   const int k = DOWN ? a.inner : a.heads * HD;
   const bool last = DOWN && layer + 1 == a.layer_count;
   // a wave's steps whose weights are in registers before the operands exist: 4 waves have 6 of an inner size of 1,536, 8 waves 11 of 5,632
-  constexpr int kUnits = into_units_of<WAVES, DOWN>(), kSteps = WAVES == 4 ? (DOWN ? 6 : 3) : (DOWN ? 16 : 4), kTogether = WAVES == 4 ? kSteps : 4;
-  Product<WAVES, kUnits, kSteps, kTogether> p;
-  p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, lane, wave);
+  constexpr int kUnits = into_units_of<WAVES, DOWN>(), kSteps = WAVES == 4 ? (DOWN ? 6 : 4) : (DOWN ? 16 : 4), kTogether = WAVES == 4 ? kSteps : 4;
+  constexpr int kParts = WAVES == 4 && DOWN ? 2 : 1;
+  Product<WAVES, kUnits, kSteps, kTogether, kParts> p;
+  p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, DOWN ? a.parts_down : a.parts_out, lane, wave);
   const int strip = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1, column = strip * 16 + 4 * g;
   const void* gain_of = DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2;
   const f32x4 gain = four_of(gain_of, a.gain_dtype, column, 4, true);
-  if (kNear) ex.template gate<kNear>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
-  else if (DOWN) ex.template gate<kNear>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
-  else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<kNear>(layer * a.layer_runs + (block * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
-  else ex.template gate<kNear>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
+  if (kOne || DOWN) ex.template gate<kOne>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
+  else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<kOne>(layer * a.layer_runs + (block * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
+  else ex.template gate<kOne>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
   // (the stream is two stages old and more: it is there)
   u32x4 held[1];
   if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + (strip * a.m + row) * kRecord + kRecordStream + 4 * g) * 4, 0}; });
-  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32);
-  float unused = 0.0f;
+  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32, [](int, float) {});
   f32x4 sums[1];
-  if (!add_waves<WAVES, kUnits, 1>(s, p.acc, sums, unused, wave, lane)) return;
+  if (!add_parts<WAVES, kUnits, 1, kParts>(s, p.acc, sums, wave, lane)) return;
+  if (last) {  // (the final norm's kernel adds it to the stream)
+    if (r < a.m) {
+      bf16x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = (__bf16)sums[0][e];
+      *(bf16x4*)(a.y_out + (size_t)row * a.width + column) = y;
+    }
+    return;
+  }
   f32x4 v;
   float sq = 0.0f;
 #pragma unroll
@@ -641,29 +725,24 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   sq += __shfl_xor(sq, 16, kWave);
   sq += __shfl_xor(sq, 32, kWave);
   if (r >= a.m) return;
-  if (last) {
-    *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
-    return;
-  }
+  if (!DOWN && layer + 1 == a.layer_count) *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
   put_record(ex, next + (DOWN ? a.stream1 : a.stream2) + (strip * a.m + row) * kRecord, g, v, gain, sq);
 }
 
 template <int WAVES>
 __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
-  constexpr bool kNear = WAVES == 8;
+  constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const unsigned here = layer * a.layer_words;
   constexpr int kUnits = units_of<WAVES>();
-  Product<WAVES, 2 * kUnits, 4, 4> p;
-  p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, lane, wave);
+  Product<WAVES, 2 * kUnits, 4, 4, 1> p;
+  p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, a.parts_gate, lane, wave);
   const int unit = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
-  if (kNear) ex.template gate<kNear>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
-  else ex.template gate<kNear>(here + a.attn + block * 61 % (a.m * a.heads * (HD / 2)), wave);
-  float ss = p.template run<true>(ex, (here + a.stream2 + row * kRecord) * 4, a.m * kRecord * 4);
+  ex.template gate<kOne>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
   f32x4 sums[2];
-  if (!add_waves<WAVES, kUnits, 2>(s, p.acc, sums, ss, wave, lane)) return;
+  float scale;
+  if (!run_prepared<WAVES, kUnits, 2, 1>(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
   if (r >= a.m) return;
-  const float scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
   bf16_t out[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -684,7 +763,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
   const int per_layer = a.n_qkv + a.n_att + a.n_comb + a.n_out + a.n_gate + a.n_down;
   const int layer = b / per_layer;
   b -= layer * per_layer;
-  if (b < a.n_qkv) return qkv_stage<WAVES>(a, ex, s, layer, b);
+  if (b < a.n_qkv) {
+    if (WAVES == 4 && layer == 0) return qkv_stage<WAVES, true>(a, ex, s, layer, b);
+    return qkv_stage<WAVES, false>(a, ex, s, layer, b);
+  }
   b -= a.n_qkv;
   if (b < a.n_att) return attention_stage<WAVES>(a, ex, s, layer, b);
   b -= a.n_att;
@@ -746,25 +828,25 @@ extern "C" long long nnis_chain_words(int layers, int m, int width, int heads, i
 // and down; the gains of its two norms, all of gain_dtype; its key and value pages); x, x_out: [m, width] in 32 bits; tok_cos,
 // tok_sin, tok_page, tok_pages: the step's tables.  words, runs: as nnis_chain_words says, 16-byte aligned.  host_fail: a word of pinned
 // host memory.
-extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width, int heads, int kv_heads, int head_dim, int inner, int splits,
-                          int gain_dtype, float eps, float scale, const float* x, float* x_out, const float* tok_cos, const float* tok_sin,
+extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width, int heads, int kv_heads, int head_dim, int inner, int splits, int page_waves,
+                          int gain_dtype, float eps, float scale, const float* x, float* x_out, void* y_out, const float* tok_cos, const float* tok_sin,
                           const int* tok_pos, const int* tok_page, const int* tok_pages, int max_pages, void* words, long long word_count, void* runs, long long run_count,
                           void* host_fail, void* stream_ptr) {
   NNIS_REQUIRE(head_dim == HD && fits(m, width, heads, kv_heads, inner, splits), "chain: %d rows, width %d, %d/%d heads of %d, inner %d, %d runs are not taken", m,
                width, heads, kv_heads, head_dim, inner, splits);
-  NNIS_REQUIRE(layers && x && x_out && tok_cos && tok_sin && tok_pos && tok_page && tok_pages && max_pages > 0 && words && host_fail, "chain: an operand is missing");
+  NNIS_REQUIRE(layers && x && x_out && y_out && tok_cos && tok_sin && tok_pos && tok_page && tok_pages && max_pages > 0 && words && host_fail, "chain: an operand is missing");
   long long runs_needed;
   const long long needed = nnis_chain_words(layer_count, m, width, heads, kv_heads, inner, splits, &runs_needed);
   NNIS_REQUIRE(needed > 0 && word_count == needed && run_count >= runs_needed && (runs || runs_needed == 0), "chain: %lld and %lld words for %d layers", word_count,
                run_count, layer_count);
   NNIS_REQUIRE(nnis_dtype_ok(gain_dtype) && eps > 0.0f && scale > 0.0f, "chain: bad gain type, eps or scale");
-  for (const void* p : {(const void*)x, (const void*)x_out, (const void*)tok_cos, (const void*)tok_sin, (const void*)words, (const void*)runs})
+  for (const void* p : {(const void*)x, (const void*)x_out, (const void*)y_out, (const void*)tok_cos, (const void*)tok_sin, (const void*)words, (const void*)runs})
     NNIS_REQUIRE((uintptr_t)p % 16 == 0, "chain: operands must be 16-byte aligned");
   ChainArgs a;
   a.layers = (const ChainLayer*)layers; a.layer_count = layer_count;
   a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits; a.gain_dtype = gain_dtype;
   a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f;
-  a.x = x; a.x_out = x_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages;
+  a.x = x; a.x_out = x_out; a.y_out = (bf16_t*)y_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages;
   a.max_pages = max_pages; a.words = (unsigned*)words; a.words_bytes = (unsigned)(word_count * 4);
   a.layer_words = lay_out(a);
   a.run_words = (unsigned*)runs; a.run_bytes = (unsigned)(runs_needed * 4);
@@ -773,6 +855,20 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   // wide models' units are large: 8 waves share them
   const int waves = width > 1024 ? 8 : 4;
   a.n_entry = m;
+  NNIS_REQUIRE(page_waves == 1 || page_waves == 2 || page_waves == 4 || (page_waves == 8 && waves == 8), "chain: %d waves for a run's pages", page_waves);
+  a.page_waves = page_waves;
+  // The ways that the layers' kernels cut K for so few rows (nnis_gemm_fused, nnis_gemm_residual), so that a step's numbers are the
+  // same bits by either route; eight waves always share K eight ways.
+  auto cut = [&](int k, int depth, int strips, int most) {
+    int parts = 1;
+    while (parts < most && (k + 63) / 64 > parts * depth && strips * parts * 2 <= 4096) parts *= 2;
+    return waves == 8 ? 8 : parts;
+  };
+  a.parts_first = cut(width, 2, 0, 8);
+  a.parts_qkv = cut(width, 4, 0, 4);
+  a.parts_out = cut(heads * HD, 4, 0, 4);
+  a.parts_gate = cut(width, 4, inner / 8, 4);
+  a.parts_down = cut(inner, 4, 0, 8);
   const int units = waves == 8 ? units_of<8>() : units_of<4>();
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
   a.n_att = m * kv_heads * ((heads / kv_heads + 3) / 4) * splits;

@@ -300,7 +300,7 @@ def chain_module():
     """The module of a decode step's layers in one launch."""
     global _chain
     if _chain is None:
-        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 9 + [_FLT, _FLT] + [_VOID] * 7 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]})
+        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 10 + [_FLT, _FLT] + [_VOID] * 8 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]})
         _chain.nnis_chain_words.argtypes = [_INT] * 7 + [ctypes.POINTER(_I64)]
         _chain.nnis_chain_words.restype = _I64
     return _chain
@@ -686,25 +686,33 @@ def chain_words(layers: int, rows: int, width: int, heads: int, kv_heads: int, i
 
 
 def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int):
-    """The runs that ``chain`` cuts a sequence's keys into for a step of ``batch`` single tokens, the longest sequence of
-    ``longest`` tokens; None where the layers' own kernels are faster or do not take the sizes."""
+    """(runs that ``chain`` cuts a sequence's keys into, waves that share a run's pages) for a step of ``batch`` single tokens,
+    the longest sequence of ``longest`` tokens; None where the sizes are not taken.  Up to a width of 1,024 (blocks of four waves)
+    these are the layers' own kernels', whose bits the launch then has.  Beyond, a wave has one page where the blocks are few, two
+    where they are more, and the runs stop at 256 blocks: 32/32 heads, 24 layers, whole steps in microseconds by the layers' kernels
+    and in 1 / 2 / 4 / 8 runs: batch 1 at 1,900 tokens 1,249 and 848 / 763 / 727 / 781, batch 4 at 3,700 1,633 and 1,198 / 1,146 /
+    1,173 / 1,286, batch 16 at 3,700 3,087 and 2,690 / 2,703 / 2,821 / 3,341."""
     if batch > CHAIN_MOST_ROWS:
         return None
-    pages, waves = (longest + 63) // 64, 8 if width > 1024 else 4
-    each, blocks = 1 if batch <= 4 else 2, batch * kv_heads * ((heads // kv_heads + 3) // 4)
-    runs = 1
-    while runs < 16 and pages > each * runs * waves and 2 * runs * blocks <= 128:
-        runs *= 2
-    return runs if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs) else None
+    if width <= 1024:
+        runs, waves = decode_plan(batch, kv_heads, longest, width=heads * head_dim)
+    else:
+        pages, waves = (longest + 63) // 64, 8
+        blocks = batch * kv_heads * ((heads // kv_heads + 3) // 4)
+        each, runs = 1 if blocks <= 32 else 2, 1  # pages a wave
+        while runs < 16 and pages > each * runs * waves and 2 * runs * blocks <= 256:
+            runs *= 2
+    return (runs, waves) if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs) else None
 
 
-def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, runs: int, failed: torch.Tensor,
-          gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int) -> torch.Tensor:
-    """All layers of a step of single tokens; returns the stream behind them.  ``layers``: int64 [8 * count] on the device, the
-    layers' pointers (``LayerChain``); ``runs``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
+def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, plan, failed: torch.Tensor,
+          gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int):
+    """All layers of a step of single tokens; returns the stream behind the last attention [rows, width] in 32 bits and what the
+    last feed-forward adds to it, in bfloat16.  ``layers``: int64 [8 * count] on the device, the
+    layers' pointers (``LayerChain``); ``plan``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
     for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page"), (tables.pages, "pages")):
         _dev(t, f"chain {what}")
-    rows = x.shape[0]
+    rows, (runs, waves) = x.shape[0], plan
     if (x.shape != (rows, width) or x.dtype != torch.float32 or tables.cos.shape != (rows, head_dim // 2) or tables.tokens != rows or tok_pos.numel() < rows
             or tok_pos.dtype != torch.int32 or layers.dtype != torch.int64 or layers.numel() != 8 * count or not failed.is_pinned()):
         raise KernelError(f"chain: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
@@ -712,13 +720,13 @@ def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables,
     words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs)
     exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
     partial = decode_scratch(x.device, run_words) if run_words else None  # (as the split decode attention's)
-    out = torch.empty_like(x)
-    _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, _DTYPE_CODE[gain_dtype], float(eps),
-                               float(scale), x.data_ptr(), out.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
+    out, last = torch.empty_like(x), torch.empty_like(x, dtype=torch.bfloat16)
+    _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, waves, _DTYPE_CODE[gain_dtype], float(eps),
+                               float(scale), x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
                                tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial),
                                run_words, failed.data_ptr(),
                                _stream()))
-    return out
+    return out, last
 
 
 class ScoreExtras:

@@ -43,7 +43,7 @@ class LayerChain:
         return cls(links, rt)
 
     def plan(self, batch: int, longest: int, rt):
-        """The runs of a sequence's keys for a step of these sizes, or None: the layers' own kernels."""
+        """(runs of a sequence's keys, waves of a run) for a step of these sizes, or None: the layers' own kernels."""
         return rt.ops.chain_plan(len(self.links), batch, longest, **self.sizes)
 
     def check(self) -> None:
@@ -71,8 +71,8 @@ class LayerChain:
             table = self.tables[key] = torch.tensor(key, dtype=torch.int64).to(device)
         return table
 
-    def forward(self, x: torch.Tensor, ctx, views, plan, rt) -> Optional[torch.Tensor]:
-        """The stream behind the last layer, [rows, width] in 32 bits; None where the launch cannot be made here."""
+    def forward(self, x: torch.Tensor, ctx, views, plan, rt):
+        """The stream, and what the last layer still adds to it; None where the launch cannot be made here."""
         table = self._table(views, x.device)
         if table is None:
             return None

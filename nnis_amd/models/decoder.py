@@ -152,15 +152,16 @@ class DecoderModel:
         return requests, shared
 
     # ---- forward -------------------------------------------------------------
-    def _chained(self, x, schedule, ctx, cache, rt):
+    def _chained(self, stream, schedule, ctx, cache, rt):
         """(the stream behind all layers, nothing left to run) where one launch takes the step, else what it was handed."""
+        x = stream[0]
         chain = self.layer_chain(rt) if ctx.decode and not ctx.options else None
         plan = chain.plan(ctx.batch, ctx.planned_len, rt) if chain is not None else None
         if plan is None or x.dim() != 2 or x.dtype != torch.float32 or not x.is_contiguous():
-            return x, schedule
+            return stream, schedule
         views = [cache.view(index) for index in range(len(schedule))]
         done = chain.forward(x, ctx, views, plan, rt) if chain.views_fit(views) else None
-        return (x, schedule) if done is None else (done, ())
+        return (stream, schedule) if done is None else (done, ())
 
     def forward(self, ids: torch.Tensor, ctx, cache, want_rows: torch.Tensor, rt) -> torch.Tensor:
         """ids: int32 [tokens] on the device; want_rows: int32 indices of the
@@ -181,8 +182,7 @@ class DecoderModel:
             # a new one; a layer that runs first would write into it
             embedded = x if 0 in self.entries else x.clone()
         schedule = self.spec.schedule
-        x, schedule = self._chained(x, schedule, ctx, cache, rt)
-        stream = (x, None)
+        stream, schedule = self._chained((x, None), schedule, ctx, cache, rt)
         for index, entry in enumerate(schedule):
             layer = self.layers[entry.layer]
             if index in self.entries:

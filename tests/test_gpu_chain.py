@@ -1,5 +1,5 @@
-"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``) against the layers' own kernels, both
-measured by the 32-bit path on the same weights.  Sizes are those at which the launch changes what it does: a K that leaves
+"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``) against the layers' own kernels: the same
+bits up to a width of 1,024 in groups of up to four heads, else both measured by the 32-bit path on the same weights.  Sizes are those at which the launch changes what it does: a K that leaves
 waves without a chunk or takes them a second round, groups of heads beyond four, four and eight waves, runs of the keys."""
 
 import numpy as np
@@ -23,7 +23,8 @@ SIZES = [
     (64, 1, 1, 64),        # one chunk of K: three of four waves have no share of it
     (320, 5, 1, 128),      # a group of five heads
     (192, 6, 2, 1600),     # down takes 25 chunks: a wave's second round of weights
-    (1024, 14, 2, 448),    # the widest of four waves; the output projection's second round
+    (1024, 14, 7, 448),    # the widest of four waves
+    (576, 9, 3, 1536),     # the 135M shape's
     (1088, 8, 8, 576),     # eight waves, 17 chunks; a head a key head
     (1152, 16, 2, 8256),   # down takes 129 chunks
 ]
@@ -61,8 +62,8 @@ def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
 @pytest.mark.parametrize("batch", [1, 3, 16])
 @pytest.mark.parametrize("sizes", SIZES)
 def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
-    """As far from 32 bits as the layers' kernels: the same roundings in another order.  (Their distances are equal but for
-    which roundings fall together; over a few hundred logits that is within a third.)"""
+    """The same bits where the sums are made in the same order, else as far from 32 bits as the layers' kernels.  (The roundings are
+    the same; which of them fall together is not: over a few hundred logits the distances are within a third.)"""
     import nnis_amd
 
     nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
@@ -72,9 +73,12 @@ def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
     layers, ran, _ = _run(str(tmp_path), "bfloat16", lengths, None, monkeypatch)
     assert not ran
     bound = 1.33 * (layers - want).norm()
-    for plan in ("own", 1, 2, 16):
+    waves = 4 if sizes[0] <= 1024 else 8
+    for plan in ("own", (1, waves), (2, waves // 2), (16, waves)):
         got, ran, _ = _run(str(tmp_path), "bfloat16", lengths, plan, monkeypatch)
         assert ran, f"plan {plan}: the launch was not made"
+        if plan == "own" and waves == 4 and sizes[1] // sizes[2] <= 4:
+            assert torch.equal(got, layers)
         error = (got - want).norm()
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
 
