@@ -1,0 +1,144 @@
+// How the blocks of one launch hand each other their results (chain.hip, chain_f32.hip).
+//
+// How words get from block to block: every word of the exchange is kNone (all bits set) before the launch, and is there once it is
+// anything else.  Writers store past the caches and never store kNone (a NaN with that payload goes out as another NaN), readers
+// load past the caches until no word of what they asked for is kNone.  A word carries its own mark, so no order between
+// words is needed, no counter and no fence.
+//
+// Why every wait ends: the stages of a block's operands are blocks of smaller numbers, and a die is handed its blocks in the order
+// of their numbers; so the unfinished block with the smallest number is on the chip, or its die is full of blocks of another
+// kernel.  Should two such launches ever fill a die each for the other, or a fault keep words away, a wait gives up after
+// kWaitTicks: it says so in `fail` (then all others leave too) and in `host_fail`, which the host reads before its next step;
+// what was not written stays kNone, which is no number, so nothing that hangs on it looks like a result.
+#pragma once
+
+#include "common.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+
+constexpr unsigned kNone = 0xffffffffu;
+constexpr int kPastCaches = 16;              // a buffer access's cache policy: sc1, agent scope
+constexpr int kChainHead = 64;               // channels of a head
+constexpr int kMostRows = 16;
+constexpr int kRunRow = kChainHead + 4;      // words of a run of keys: outputs, reference, sum, two unused
+constexpr long long kWaitTicks = 200000000;  // of the 100 MHz clock: 2 s
+
+__device__ __forceinline__ unsigned marked(float v) {
+  const unsigned u = __float_as_uint(v);
+  return u == kNone ? 0x7fc00000u : u;
+}
+__device__ __forceinline__ unsigned marked2(bf16_t lo, bf16_t hi) {
+  const unsigned u = (unsigned)__builtin_bit_cast(unsigned short, lo) | ((unsigned)__builtin_bit_cast(unsigned short, hi) << 16);
+  return u == kNone ? 0x7fc07fc0u : u;
+}
+
+// where a lane reads: its own part of a byte offset, and the part that is the wave's
+struct At {
+  unsigned lane, wave;
+};
+
+struct Exchange {
+  __amdgpu_buffer_rsrc_t r;
+  unsigned *fail, *host_fail;
+
+  template <typename Args>
+  __device__ __forceinline__ Exchange(const Args& a, unsigned* words, unsigned bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc(words, 0, bytes, 0x00020000)), fail(a.fail), host_fail(a.host_fail) {}
+
+  // whether a wait is to be left: every 256th look, by the clock and by what others found
+  __device__ __forceinline__ bool leave(int& looks, long long& since) const {
+    if ((++looks & 255) != 0) return false;
+    const long long now = wall_clock64();
+    if (looks == 256) since = now;
+    if (__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
+    if (now - since < kWaitTicks) return false;
+    __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(host_fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return true;
+  }
+
+  // Until one word of a stage further ahead is there: a block that is on the chip early looks now and then at one word, so that
+  // the words of the stage at work are not asked for by every block of the layers behind it.
+  template <bool ONE>  // the first wave looks for the whole block
+  __device__ __forceinline__ void gate(unsigned word, int wave) const {
+    if (!ONE || wave == 0) {
+      int looks = 0;
+      long long since = 0;
+      while (true) {
+        const unsigned u = __builtin_amdgcn_raw_buffer_load_b32(r, word * 4, 0, kPastCaches);
+        asm volatile("" ::: "memory");  // (asked for anew each time)
+        if (__builtin_amdgcn_readfirstlane(u) != kNone || leave(looks, since)) break;
+        __builtin_amdgcn_s_sleep(4);
+      }
+    }
+    if (ONE) __syncthreads();
+  }
+
+  // 16 bytes a lane N times, and beside each an M-th of 4 or 8 bytes: `ask(i)` gives the i-th's byte offsets, the lane's part and
+  // the wave's; until all of them are there
+  template <int N, typename Ask>
+  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask) const {
+    int looks = 0;
+    long long since = 0;
+    while (true) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
+      asm volatile("" ::: "memory");
+      unsigned top = 0;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
+      if (!__any(top == kNone) || leave(looks, since)) return;
+    }
+  }
+  template <int N, typename Ask, typename T, int M, typename AskBeside>
+  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask, T (&w)[M], AskBeside ask_beside) const {
+    int looks = 0;
+    long long since = 0;
+    while (true) {
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        if constexpr (sizeof(T) == 4) w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
+        else w[i] = __builtin_amdgcn_raw_buffer_load_b64(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
+      asm volatile("" ::: "memory");
+      unsigned top = 0;
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        if constexpr (sizeof(T) == 4) top = max(top, w[i]);
+        else top = max(top, max(w[i][0], w[i][1]));
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
+      if (!__any(top == kNone) || leave(looks, since)) return;
+    }
+  }
+  __device__ __forceinline__ void put(unsigned word, unsigned v) const { __builtin_amdgcn_raw_buffer_store_b32(v, r, word * 4, 0, kPastCaches); }
+  __device__ __forceinline__ void put(unsigned word, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, r, word * 4, 0, kPastCaches); }
+  __device__ __forceinline__ void put(unsigned word, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, r, word * 4, 0, kPastCaches); }
+};
+
+__global__ __launch_bounds__(256) void chain_clear_kernel(u32x4* words, unsigned n, u32x4* runs, unsigned n_runs, unsigned* fail) {
+  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n + n_runs; i += gridDim.x * 256) {
+    u32x4* at = i < n ? words + i : runs + (i - n);
+    *at = (u32x4){kNone, kNone, kNone, kNone};
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *fail = 0;
+}
+
+inline int chain_clear(void* words, long long word_count, void* runs, long long run_count, unsigned* fail, hipStream_t stream) {
+  const unsigned fours = (unsigned)(word_count / 4), run_fours = (unsigned)(run_count / 4), blocks = (fours + run_fours + 255) / 256;
+  hipLaunchKernelGGL(chain_clear_kernel, dim3(blocks < 1024 ? blocks : 1024), dim3(256), 0, stream, (u32x4*)words, fours, (u32x4*)runs, run_fours, fail);
+  NNIS_LAUNCH_CHECK("chain_clear");
+  return 0;
+}
+
+}  // namespace

@@ -300,9 +300,11 @@ def chain_module():
     """The module of a decode step's layers in one launch."""
     global _chain
     if _chain is None:
-        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 10 + [_FLT, _FLT] + [_VOID] * 8 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]})
-        _chain.nnis_chain_words.argtypes = [_INT] * 7 + [ctypes.POINTER(_I64)]
-        _chain.nnis_chain_words.restype = _I64
+        tail = [_VOID] * 8 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]
+        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 10 + [_FLT, _FLT] + tail, "nnis_chain_f32": [_VOID] + [_INT] * 8 + [_FLT, _FLT] + tail})
+        for words in (_chain.nnis_chain_words, _chain.nnis_chain_f32_words):
+            words.argtypes = [_INT] * 7 + [ctypes.POINTER(_I64)]
+            words.restype = _I64
     return _chain
 
 
@@ -674,58 +676,68 @@ def step_tables(tok_slot: torch.Tensor, tok_pos: torch.Tensor, tokens: int, cos:
 CHAIN_MOST_ROWS = 16
 
 
-def chain_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, runs: int = 1) -> bool:
-    """Whether ``chain`` takes layers of these sizes."""
-    return head_dim == 64 and chain_words(layers, rows, width, heads, kv_heads, inner, runs)[0] > 0
-
-
-def chain_words(layers: int, rows: int, width: int, heads: int, kv_heads: int, inner: int, runs: int):
+def chain_words(layers: int, rows: int, width: int, heads: int, kv_heads: int, inner: int, runs: int, dtype=torch.bfloat16):
     """(32-bit words of the exchange, of the runs) that ``chain`` needs; (0, _) for sizes that it does not take."""
-    of_runs = _I64()
-    return chain_module().nnis_chain_words(layers, rows, width, heads, kv_heads, inner, runs, ctypes.byref(of_runs)), of_runs.value
+    of_runs, lib = _I64(), chain_module()
+    words = lib.nnis_chain_f32_words if dtype == torch.float32 else lib.nnis_chain_words
+    return words(layers, rows, width, heads, kv_heads, inner, runs, ctypes.byref(of_runs)), of_runs.value
 
 
-def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int):
+def chain_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, runs: int = 1, dtype=torch.bfloat16) -> bool:
+    """Whether ``chain`` takes layers of these sizes."""
+    return head_dim == 64 and chain_words(layers, rows, width, heads, kv_heads, inner, runs, dtype)[0] > 0
+
+
+def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """(runs that ``chain`` cuts a sequence's keys into, waves that share a run's pages) for a step of ``batch`` single tokens,
-    the longest sequence of ``longest`` tokens; None where the sizes are not taken.  Up to a width of 1,024 (blocks of four waves)
-    these are the layers' own kernels', whose bits the launch then has.  Beyond, a wave has one page where the blocks are few, two
-    where they are more, and the runs stop at 256 blocks: 32/32 heads, 24 layers, whole steps in microseconds by the layers' kernels
-    and in 1 / 2 / 4 / 8 runs: batch 1 at 1,900 tokens 1,249 and 848 / 763 / 727 / 781, batch 4 at 3,700 1,633 and 1,198 / 1,146 /
-    1,173 / 1,286, batch 16 at 3,700 3,087 and 2,690 / 2,703 / 2,821 / 3,341."""
+    the longest sequence of ``longest`` tokens; None where the sizes are not taken.  In bfloat16 up to a width of 1,024 (blocks of
+    four waves) these are the layers' own kernels', whose bits the launch then has.  Beyond, a wave has one page where the blocks are
+    few, two where they are more, and the runs stop at 256 blocks: 32/32 heads, 24 layers, whole steps in microseconds by the layers'
+    kernels and in 1 / 2 / 4 / 8 runs: batch 1 at 1,900 tokens 1,249 and 848 / 763 / 727 / 781, batch 4 at 3,700 1,633 and 1,198 /
+    1,146 / 1,173 / 1,286, batch 16 at 3,700 3,087 and 2,690 / 2,703 / 2,821 / 3,341.  In 32 bits a wave's tiles are 16 keys: up to two
+    tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and 900 / 723 / 623 / 590, in 16 runs 618; batch
+    8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868."""
     if batch > CHAIN_MOST_ROWS:
         return None
-    if width <= 1024:
+    pages, runs, waves = (longest + 63) // 64, 1, 8
+    if dtype == torch.float32:
+        blocks = batch * kv_heads
+        while runs < 16 and 4 * pages > runs * waves and 2 * runs * blocks <= 256:
+            runs *= 2
+    elif width <= 1024:
         runs, waves = decode_plan(batch, kv_heads, longest, width=heads * head_dim)
     else:
-        pages, waves = (longest + 63) // 64, 8
         blocks = batch * kv_heads * ((heads // kv_heads + 3) // 4)
-        each, runs = 1 if blocks <= 32 else 2, 1  # pages a wave
+        each = 1 if blocks <= 32 else 2  # pages a wave
         while runs < 16 and pages > each * runs * waves and 2 * runs * blocks <= 256:
             runs *= 2
-    return (runs, waves) if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs) else None
+    return (runs, waves) if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs, dtype) else None
 
 
 def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, plan, failed: torch.Tensor,
-          gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int):
+          gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """All layers of a step of single tokens; returns the stream behind the last attention [rows, width] in 32 bits and what the
-    last feed-forward adds to it, in bfloat16.  ``layers``: int64 [8 * count] on the device, the
-    layers' pointers (``LayerChain``); ``plan``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
+    last feed-forward adds to it, in ``dtype``, the weights' and the cache's.  ``layers``: int64 [8 * count] on the device, the layers'
+    pointers (``LayerChain``); ``plan``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
     for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page"), (tables.pages, "pages")):
         _dev(t, f"chain {what}")
     rows, (runs, waves) = x.shape[0], plan
     if (x.shape != (rows, width) or x.dtype != torch.float32 or tables.cos.shape != (rows, head_dim // 2) or tables.tokens != rows or tok_pos.numel() < rows
-            or tok_pos.dtype != torch.int32 or layers.dtype != torch.int64 or layers.numel() != 8 * count or not failed.is_pinned()):
+            or tok_pos.dtype != torch.int32 or layers.dtype != torch.int64 or layers.numel() != 8 * count or not failed.is_pinned()
+            or (dtype == torch.float32 and gain_dtype != torch.float32)):
         raise KernelError(f"chain: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
     lib = chain_module()
-    words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs)
+    words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs, dtype)
     exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
     partial = decode_scratch(x.device, run_words) if run_words else None  # (as the split decode attention's)
-    out, last = torch.empty_like(x), torch.empty_like(x, dtype=torch.bfloat16)
-    _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, waves, _DTYPE_CODE[gain_dtype], float(eps),
-                               float(scale), x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
-                               tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial),
-                               run_words, failed.data_ptr(),
-                               _stream()))
+    out, last = torch.empty_like(x), torch.empty_like(x, dtype=dtype)
+    tail = (float(eps), float(scale), x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
+            tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial), run_words, failed.data_ptr(),
+            _stream())
+    if dtype == torch.float32:
+        _check(lib, lib.nnis_chain_f32(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, *tail))
+    else:
+        _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, waves, _DTYPE_CODE[gain_dtype], *tail))
     return out, last
 
 

@@ -19,6 +19,7 @@ class LayerChain:
         self.links = links
         first = links[0]
         self.sizes = {name: first[name] for name in ("width", "heads", "kv_heads", "head_dim", "inner")}
+        self.sizes["dtype"] = rt.dtype
         self.eps, self.scale, self.position, self.gain_dtype = first["eps"], first["scale"], first["position"], first["gains"][0].dtype
         # where a wait that was given up says so: a word of host memory that the kernel writes and the next step reads
         self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
@@ -38,9 +39,11 @@ class LayerChain:
             return None
         if any(gain.dtype != links[0]["gains"][0].dtype or gain.data_ptr() % 16 for link in links for gain in link["gains"]):
             return None
-        if not rt.ops.chain_takes(len(links), 1, **{n: links[0][n] for n in ("width", "heads", "kv_heads", "head_dim", "inner")}):
+        if rt.is_fp32 and any(t.dtype != torch.float32 or not t.is_contiguous() or t.data_ptr() % 16
+                              for link in links for t in (*link["weights"], *link["gains"])):
             return None
-        return cls(links, rt)
+        chain = cls(links, rt)
+        return chain if rt.ops.chain_takes(len(links), 1, **chain.sizes) else None
 
     def plan(self, batch: int, longest: int, rt):
         """(runs of a sequence's keys, waves of a run) for a step of these sizes, or None: the layers' own kernels."""
@@ -55,7 +58,7 @@ class LayerChain:
 
     def views_fit(self, views) -> bool:
         """Whether each layer writes keys and values of its own, through one block table."""
-        return all(not getattr(view, "read_only", True) and view.k_pages.dtype == torch.bfloat16
+        return all(not getattr(view, "read_only", True) and view.k_pages.dtype == self.sizes["dtype"]
                    and view.block_table.data_ptr() == views[0].block_table.data_ptr() for view in views)
 
     def _table(self, views, device) -> Optional[torch.Tensor]:

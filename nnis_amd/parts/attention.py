@@ -232,7 +232,7 @@ class CausalSelfAttention(Mixer):
         plain = (type(self) is CausalSelfAttention and self._plain and not self.softcap and not self.window and not self.chunk and not self.extras
                  and self.gate_name is None and self.unit_eps is None and not any(self.bias_names.values()))
         if (not plain or tables is None or tables.rot_dim != self.head_dim or getattr(self.position, "pairing", None) == "neighbours"
-                or not all(isinstance(p.weight, rt.ops.PackedWeight) for p in (self.qkv, self.out))):
+                or not all(isinstance(p.weight, torch.Tensor if rt.is_fp32 else rt.ops.PackedWeight) for p in (self.qkv, self.out))):
             return None
         return {"heads": self.heads, "kv_heads": self.kv_heads, "head_dim": self.head_dim, "scale": self.scale, "position": self.position,
                 "weights": [self.qkv.weight, self.out.weight]}

@@ -91,7 +91,7 @@ class PreNormBlock(Block):
 
     def chain_link(self, rt):
         """What this layer is to a launch of all layers (``models/chain.py``), or None if that does not take it."""
-        if type(self) is not PreNormBlock or self.feed_forward is None or self.side is not None or rt.is_fp32:
+        if type(self) is not PreNormBlock or self.feed_forward is None or self.side is not None:
             return None
         norms = (self.norm1, self.norm2)
         parts = [part.chain_link(rt) if hasattr(part, "chain_link") else None for part in (self.mixer, self.feed_forward)]

@@ -45,7 +45,7 @@ class GatedFeedForward(FeedForward):
     def chain_link(self, rt):
         """See ``PreNormBlock.chain_link``."""
         if (type(self) is not GatedFeedForward or self.activation != "silu"
-                or not all(isinstance(p.weight, rt.ops.PackedWeight) for p in (self.gate_up, self.down))):
+                or not all(isinstance(p.weight, torch.Tensor if rt.is_fp32 else rt.ops.PackedWeight) for p in (self.gate_up, self.down))):
             return None
         return {"inner": self.inner, "weights": [self.gate_up.weight, self.down.weight]}
 

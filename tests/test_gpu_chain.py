@@ -1,6 +1,7 @@
-"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``) against the layers' own kernels: the same
-bits up to a width of 1,024 in groups of up to four heads, else both measured by the 32-bit path on the same weights.  Sizes are those at which the launch changes what it does: a K that leaves
-waves without a chunk or takes them a second round, groups of heads beyond four, four and eight waves, runs of the keys."""
+"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``, ``chain_f32.hip``) against the layers' own
+kernels: in bfloat16 the same bits up to a width of 1,024 in groups of up to four heads, else both measured by the 32-bit path on the
+same weights; in 32 bits both measured by the oracle in 64.  Sizes are those at which the launch changes what it does: a K that
+leaves waves without a chunk or takes them a second round, groups of heads beyond four, four and eight waves, runs of the keys."""
 
 import numpy as np
 import pytest
@@ -32,6 +33,11 @@ SIZES = [
 LENGTHS = [1, 63, 64, 65, 200, 1023, 1100, 5, 128, 320, 577, 129, 31, 2000, 90, 447]
 
 
+def _tokens(lengths, steps):
+    rng = np.random.default_rng(sum(lengths))
+    return [rng.integers(0, 509, size=n).tolist() for n in lengths], [rng.integers(0, 509, size=len(lengths)).tolist() for _ in range(steps)]
+
+
 def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
     """The logits of ``steps`` steps of single tokens behind prompts of these lengths, [steps, sequences, vocab]."""
     from nnis_amd.api import load_engine
@@ -42,13 +48,12 @@ def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
         if plan != "own":
             patch.setattr(ops, "chain_plan", lambda *args, **sizes: plan)
         engine = load_engine(folder, dtype=dtype, max_tokens=sum(-(-(n + steps + 1) // 64) * 64 for n in lengths))
-        rng = np.random.default_rng(sum(lengths))
+        prompts, tokens = _tokens(lengths, steps)
         slots = [engine.start_sequence() for _ in lengths]
-        engine.step([StepEntry(slot, rng.integers(0, 509, size=n).tolist(), None) for slot, n in zip(slots, lengths)])
+        engine.step([StepEntry(slot, prompt, None) for slot, prompt in zip(slots, prompts)])
         out = []
-        for _ in range(steps):
-            tokens = rng.integers(0, 509, size=len(lengths)).tolist()
-            entries = [StepEntry(slot, [token], None) for slot, token in zip(slots, tokens)]
+        for step in range(steps):
+            entries = [StepEntry(slot, [token], None) for slot, token in zip(slots, tokens[step])]
             out.append(engine.step(entries).double().cpu())
             if len(out) == 1:  # the same step again, replayed over what the first left in the exchange
                 for slot, n in zip(slots, lengths):
@@ -68,7 +73,7 @@ def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
 
     nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
     lengths = LENGTHS[:batch] if batch > 1 else [1100]
-    want, ran, _ = _run(str(tmp_path), "float32", lengths, "own", monkeypatch)
+    want, ran, _ = _run(str(tmp_path), "float32", lengths, None, monkeypatch)
     assert not ran
     layers, ran, _ = _run(str(tmp_path), "bfloat16", lengths, None, monkeypatch)
     assert not ran
@@ -83,15 +88,39 @@ def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
 
 
+@pytest.mark.parametrize("batch", [1, 3, 16])
+@pytest.mark.parametrize("sizes", SIZES + [(128, 12, 1, 192)])  # (twelve heads a key head)
+def test_32_bits_against_the_oracle(tmp_path, sizes, batch, monkeypatch):
+    """As close to 64 bits as the layers' 32-bit kernels.  (Each sum is of the same terms in an order of its own, so the distances are
+    two draws of the same size; over a few hundred logits of a few rows they are within a third.)"""
+    import nnis_amd
+    import plain_llama
+
+    nnis_amd.write_random_model(str(tmp_path), dict(_config(*sizes), torch_dtype="float32"), 3)
+    lengths = LENGTHS[:batch] if batch > 1 else [1100]
+    prompts, tokens = _tokens(lengths, 3)
+    plain = plain_llama.PlainLlama(str(tmp_path), torch.float64)
+    want = torch.stack([plain.logits(prompt + [row[at] for row in tokens])[-3:] for at, prompt in enumerate(prompts)], dim=1)
+    layers, ran, _ = _run(str(tmp_path), "float32", lengths, None, monkeypatch)
+    assert not ran
+    bound = 1.33 * (layers - want).norm()
+    for plan in ("own", (1, 8), (2, 8), (16, 8)):
+        got, ran, _ = _run(str(tmp_path), "float32", lengths, plan, monkeypatch)
+        assert ran, f"plan {plan}: the launch was not made"
+        error = (got - want).norm()
+        assert error <= bound, f"plan {plan}: {error.item():.4g} from 64 bits, the layers' kernels {(layers - want).norm().item():.4g}"
+
+
 def test_not_taken(tmp_path, monkeypatch):
-    """Other head sizes, sizes in other steps than 64 and 32 bits stay with the layers' kernels."""
+    """Other head sizes and sizes in other steps than 64 stay with the layers' kernels."""
     import nnis_amd
 
     for index, change in enumerate(({"head_dim": 32}, {"intermediate_size": 176})):
         folder = tmp_path / str(index)
         folder.mkdir()
         nnis_amd.write_random_model(str(folder), dict(_config(64, 1, 1, 64), **change), 3)
-        assert not _run(str(folder), "bfloat16", [40], "own", monkeypatch)[1]
+        for dtype in ("bfloat16", "float32"):
+            assert not _run(str(folder), dtype, [40], "own", monkeypatch)[1]
 
 
 def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
@@ -120,4 +149,5 @@ def test_sizes_and_words():
     assert words(2, 2, 64, 1, 1, 64, 1)[0] > words(2, 1, 64, 1, 1, 64, 1)[0] and words(2, 2, 64, 1, 1, 64, 2)[1] == 2 * 2 * 2 * 68
     for refused in ((2, 17, 64, 1, 1, 64, 1), (2, 0, 64, 1, 1, 64, 1), (2, 1, 96, 1, 1, 64, 1), (2, 1, 64, 3, 2, 64, 1), (2, 1, 64, 1, 1, 80, 1),
                     (2, 1, 64, 1, 1, 64, 17), (0, 1, 64, 1, 1, 64, 1)):
-        assert words(*refused)[0] == 0
+        assert words(*refused)[0] == 0 and words(*refused, torch.float32)[0] == 0
+    assert words(2, 1, 64, 16, 1, 64, 1, torch.float32)[0] > 0 and words(2, 1, 64, 17, 1, 64, 1, torch.float32)[0] == 0
