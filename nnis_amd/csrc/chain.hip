@@ -35,7 +35,7 @@ struct ChainArgs {
   int layer_count, m, width, heads, kv_heads, inner, splits, gain_dtype;
   // how many ways K is cut (the first layer's queries, keys and values; the others'; output, gate/up, down), and the waves that
   // share a run's pages
-  int parts_first, parts_qkv, parts_out, parts_gate, parts_down, page_waves;
+  int parts_first, parts_qkv, parts_out, parts_gate, parts_down, page_waves, down_paired;
   float eps, scale_log2;
   const float* x;  // [m, width]
   float* x_out;    // [m, width]: the stream behind the last attention
@@ -66,7 +66,8 @@ __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builti
 // parts, ..; a wave has V parts, its own number and those WAVES on.  It asks for the weights of its first STEPS chunks when the
 // block begins; XB chunks of the operand are asked for together.  A step of the operand beyond the last chunk reads the last again
 // and is not multiplied.  The parts and the order of their sums are those of the layers' own kernels for the same product.
-template <int WAVES, int STRIPS, int STEPS, int XB, int V>
+// NEXT: a wave's second part is the one after its first, not the one WAVES on.
+template <int WAVES, int STRIPS, int STEPS, int XB, int V, bool NEXT = false>
 struct Product {
   static_assert(STEPS % XB == 0 && STEPS % V == 0, "whole trips");
   bf16x8 w[STEPS][2][STRIPS];
@@ -76,7 +77,7 @@ struct Product {
 
   // the chunk of step `s` of the round that begins with a part's chunk number `d0`; `chunks` and more: none
   __device__ __forceinline__ int chunk(int d0, int s) const {
-    const int part = wave + WAVES * (s / (STEPS / V));
+    const int part = NEXT ? V * wave + s / (STEPS / V) : wave + WAVES * (s / (STEPS / V));
     return V > 1 && part >= parts ? chunks : part + parts * (d0 + s % (STEPS / V));
   }
   __device__ __forceinline__ void ask(int d0) {
@@ -221,6 +222,31 @@ __device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange&
   } else {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) ss += s.product.ss[w][lane];
+  }
+  scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  return true;
+}
+
+// The same of eight waves that cut K four ways, waves 0 to 3 for the block's first unit and 4 to 7 for its second.
+template <typename P>
+__device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Exchange& ex, Shared<8>& s, P& p, unsigned first_word, int row, int wave, int lane,
+                                                    f32x4 (&sums)[2], float& scale) {
+  float ss = 0.0f;
+  p.template run<true>(ex, (first_word + row * kRecord) * 4, a.m * kRecord * 4, [&](int, float part) { ss += part; });
+  ss += __shfl_xor(ss, 16, kWave);
+  ss += __shfl_xor(ss, 32, kWave);
+  s.product.ss[wave][lane] = ss;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) *(f32x4*)s.product.acc[wave][j][lane] = p.acc[0][j];
+  __syncthreads();
+  if (wave % 4 != 0) return false;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) ss += s.product.ss[wave + w][lane];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    sums[j] = p.acc[0][j];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) sums[j] += *(const f32x4*)s.product.acc[wave + w][j][lane];
   }
   scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
   return true;
@@ -567,7 +593,8 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
 }
 
 // a strip of 16 columns of the stream: the output projection (down = false) or the feed-forward's down
-template <int WAVES, bool DOWN>
+// PAIRED: K cut sixteen ways, the even parts and the odd ones added up apart, as the layers' kernel does in two blocks
+template <int WAVES, bool DOWN, bool PAIRED>
 __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
   constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
@@ -577,9 +604,9 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   const bool last = DOWN && layer + 1 == a.layer_count;
   // a wave's steps whose weights are in registers before the operands exist: 4 waves have 6 of an inner size of 1,536, 8 waves 11 of 5,632
   constexpr int kUnits = into_units_of<WAVES, DOWN>(), kSteps = WAVES == 4 ? (DOWN ? 6 : 4) : (DOWN ? 16 : 4), kTogether = WAVES == 4 ? kSteps : 4;
-  constexpr int kParts = WAVES == 4 && DOWN ? 2 : 1;
-  Product<WAVES, kUnits, kSteps, kTogether, kParts> p;
-  p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, DOWN ? a.parts_down : a.parts_out, lane, wave);
+  constexpr int kParts = (WAVES == 4 && DOWN) || PAIRED ? 2 : 1;
+  Product<WAVES, kUnits, kSteps, kTogether, kParts, PAIRED> p;
+  p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, PAIRED ? 16 : DOWN ? a.parts_down : a.parts_out, lane, wave);
   const int strip = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1, column = strip * 16 + 4 * g;
   const void* gain_of = DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2;
   const f32x4 gain = four_of(gain_of, a.gain_dtype, column, 4, true);
@@ -591,7 +618,17 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + (strip * a.m + row) * kRecord + kRecordStream + 4 * g) * 4, 0}; });
   p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32, [](int, float) {});
   f32x4 sums[1];
-  if (!add_parts<WAVES, kUnits, 1, kParts>(s, p.acc, sums, wave, lane)) return;
+  if constexpr (PAIRED) {
+    const f32x4 even[1][1] = {{p.acc[0][0]}};
+    *(f32x4*)s.product.acc[wave][1][lane] = p.acc[1][0];
+    if (!add_parts<WAVES, 1, 1, 1>(s, even, sums, wave, lane)) return;
+    f32x4 odd = *(const f32x4*)s.product.acc[0][1][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) odd += *(const f32x4*)s.product.acc[w][1][lane];
+    sums[0] += odd;
+  } else {
+    if (!add_parts<WAVES, kUnits, 1, kParts>(s, p.acc, sums, wave, lane)) return;
+  }
   if (last) {  // (the final norm's kernel adds it to the stream)
     if (r < a.m) {
       bf16x4 y;
@@ -615,19 +652,28 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   put_record(ex, next + (DOWN ? a.stream1 : a.stream2) + (strip * a.m + row) * kRecord, g, v, gain, sq);
 }
 
-template <int WAVES>
+// HALVES: eight waves that cut K four ways for each of the block's two units, as the layers' kernel does for this many strips
+template <int WAVES, bool HALVES>
 __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
   constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const unsigned here = layer * a.layer_words;
   constexpr int kUnits = units_of<WAVES>();
-  Product<WAVES, 2 * kUnits, 4, 4, 1> p;
-  p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, a.parts_gate, lane, wave);
-  const int unit = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
-  ex.template gate<kOne>(here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord, wave);
+  const int unit = block * kUnits + (HALVES ? wave / 4 : wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
+  const unsigned one = here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord;
   f32x4 sums[2];
   float scale;
-  if (!run_prepared<WAVES, kUnits, 2, 1>(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
+  if constexpr (HALVES) {
+    Product<4, 2, 8, 4, 1> p;
+    p.begin(a.layers[layer].w_gate_up, [&](int j) { return unit * 16 + j * a.inner; }, a.width, 4, lane, wave % 4);
+    ex.template gate<kOne>(one, wave);
+    if (!run_prepared_halves(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
+  } else {
+    Product<WAVES, 2 * kUnits, 4, 4, 1> p;
+    p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, a.parts_gate, lane, wave);
+    ex.template gate<kOne>(one, wave);
+    if (!run_prepared<WAVES, kUnits, 2, 1>(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
+  }
   if (r >= a.m) return;
   bf16_t out[4];
 #pragma unroll
@@ -658,10 +704,17 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
   b -= a.n_att;
   if (b < a.n_comb) return combine_stage<WAVES>(a, ex, layer, b);
   b -= a.n_comb;
-  if (b < a.n_out) return strip_stage<WAVES, false>(a, ex, s, layer, b);
+  if (b < a.n_out) return strip_stage<WAVES, false, false>(a, ex, s, layer, b);
   b -= a.n_out;
-  if (b < a.n_gate) return gate_stage<WAVES>(a, ex, s, layer, b);
-  strip_stage<WAVES, true>(a, ex, s, layer, b - a.n_gate);
+  if (b < a.n_gate) {
+    if constexpr (WAVES == 8)
+      if (a.parts_gate == 4) return gate_stage<WAVES, true>(a, ex, s, layer, b);
+    return gate_stage<WAVES, false>(a, ex, s, layer, b);
+  }
+  b -= a.n_gate;
+  if constexpr (WAVES == 8)
+    if (a.down_paired && layer + 1 < a.layer_count) return strip_stage<WAVES, true, true>(a, ex, s, layer, b);
+  strip_stage<WAVES, true, false>(a, ex, s, layer, b);
 }
 
 // where the words of a layer lie; returns their number
@@ -736,17 +789,19 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   NNIS_REQUIRE(page_waves == 1 || page_waves == 2 || page_waves == 4 || (page_waves == 8 && waves == 8), "chain: %d waves for a run's pages", page_waves);
   a.page_waves = page_waves;
   // The ways that the layers' kernels cut K for so few rows (nnis_gemm_fused, nnis_gemm_residual), so that a step's numbers are the
-  // same bits by either route; eight waves always share K eight ways.
+  // same bits by either route; four waves take up to four parts (narrow rows' are no more), and down's eight two a wave.
   auto cut = [&](int k, int depth, int strips, int most) {
     int parts = 1;
     while (parts < most && (k + 63) / 64 > parts * depth && strips * parts * 2 <= 4096) parts *= 2;
-    return waves == 8 ? 8 : parts;
+    return parts;
   };
   a.parts_first = cut(width, 2, 0, 8);
-  a.parts_qkv = cut(width, 4, 0, 4);
-  a.parts_out = cut(heads * HD, 4, 0, 4);
-  a.parts_gate = cut(width, 4, inner / 8, 4);
+  a.parts_qkv = cut(width, 4, 0, waves);
+  a.parts_out = cut(heads * HD, 4, 0, waves);
+  a.parts_gate = cut(width, 4, inner / 8, waves);
+  if (waves == 8 && a.parts_gate < 4) a.parts_gate = 8;  // (not the layers' bits there)
   a.parts_down = cut(inner, 4, 0, 8);
+  a.down_paired = waves == 8 && width <= 2048 && inner >= 80 * 64;
   const int units = waves == 8 ? units_of<8>() : units_of<4>();
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
   a.n_att = m * kv_heads * ((heads / kv_heads + 3) / 4) * splits;

@@ -690,22 +690,29 @@ def chain_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, h
 
 def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """(runs that ``chain`` cuts a sequence's keys into, waves that share a run's pages) for a step of ``batch`` single tokens,
-    the longest sequence of ``longest`` tokens; None where the sizes are not taken.  In bfloat16 up to a width of 1,024 (blocks of
-    four waves) these are the layers' own kernels', whose bits the launch then has.  Beyond, a wave has one page where the blocks are
-    few, two where they are more, and the runs stop at 256 blocks: 32/32 heads, 24 layers, whole steps in microseconds by the layers'
-    kernels and in 1 / 2 / 4 / 8 runs: batch 1 at 1,900 tokens 1,249 and 848 / 763 / 727 / 781, batch 4 at 3,700 1,633 and 1,198 /
-    1,146 / 1,173 / 1,286, batch 16 at 3,700 3,087 and 2,690 / 2,703 / 2,821 / 3,341.  In 32 bits a wave's tiles are 16 keys: up to two
-    tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and 900 / 723 / 623 / 590, in 16 runs 618; batch
-    8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868."""
+    the longest sequence of ``longest`` tokens; None where the launch is not to take the step.
+
+    In bfloat16 with up to four query heads a key head these are the layers' own kernels', whose bits the launch then has (the ways
+    that K is cut are theirs too).  Other plans are not faster by much: 32/32 heads, 24 layers, whole steps in microseconds by the
+    layers' kernels, by this plan and by one of 8 waves: batch 2 at 500 tokens 1,173 and 724 and 716, batch 8 at 2,000 1,539 and 1,233 and
+    1,196, batch 12 at 3,000 2,218 and 2,064 and 1,993.
+
+    Larger groups have the scores of four heads a wave here and of sixteen there, so other bits, and a seeded draw over other bits picks
+    other tokens: the launch is theirs up to seven rows.  A wave has one page where the blocks are few, two where they are more, and the
+    runs stop at 256 blocks (32/4 heads, 22 layers, batch 1 at 700 tokens 945 and 480).  In 32 bits a wave's tiles are 16 keys: up to two
+    tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and in 1 / 2 / 4 / 8 runs 900 / 723 / 623 / 590, in
+    16 618; batch 8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868."""
     if batch > CHAIN_MOST_ROWS:
         return None
-    pages, runs, waves = (longest + 63) // 64, 1, 8
+    pages, runs, waves = (longest + 63) // 64, 1, 8 if dtype == torch.float32 or width > 1024 else 4
     if dtype == torch.float32:
         blocks = batch * kv_heads
         while runs < 16 and 4 * pages > runs * waves and 2 * runs * blocks <= 256:
             runs *= 2
-    elif width <= 1024:
+    elif heads // kv_heads <= 4:
         runs, waves = decode_plan(batch, kv_heads, longest, width=heads * head_dim)
+    elif batch >= 8:
+        return None
     else:
         blocks = batch * kv_heads * ((heads // kv_heads + 3) // 4)
         each = 1 if blocks <= 32 else 2  # pages a wave

@@ -27,6 +27,7 @@ SIZES = [
     (1024, 14, 7, 448),    # the widest of four waves
     (576, 9, 3, 1536),     # the 135M shape's
     (1088, 8, 8, 576),     # eight waves, 17 chunks; a head a key head
+    (1152, 16, 4, 5184),   # down takes 81 chunks, the even and the odd apart; gate and up in 4 parts
     (1152, 16, 2, 8256),   # down takes 129 chunks
 ]
 # lengths before the step: the first token, pages' ends, runs
@@ -67,8 +68,8 @@ def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
 @pytest.mark.parametrize("batch", [1, 3, 16])
 @pytest.mark.parametrize("sizes", SIZES)
 def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
-    """The same bits where the sums are made in the same order, else as far from 32 bits as the layers' kernels.  (The roundings are
-    the same; which of them fall together is not: over a few hundred logits the distances are within a third.)"""
+    """The same bits in groups of up to four heads, else as far from 32 bits as the layers' kernels.  (The roundings are the same;
+    which of them fall together is not: over a few hundred logits the distances are within a third.)"""
     import nnis_amd
 
     nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
@@ -78,11 +79,11 @@ def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
     layers, ran, _ = _run(str(tmp_path), "bfloat16", lengths, None, monkeypatch)
     assert not ran
     bound = 1.33 * (layers - want).norm()
-    waves = 4 if sizes[0] <= 1024 else 8
+    waves, group = 4 if sizes[0] <= 1024 else 8, sizes[1] // sizes[2]
     for plan in ("own", (1, waves), (2, waves // 2), (16, waves)):
         got, ran, _ = _run(str(tmp_path), "bfloat16", lengths, plan, monkeypatch)
-        assert ran, f"plan {plan}: the launch was not made"
-        if plan == "own" and waves == 4 and sizes[1] // sizes[2] <= 4:
+        assert ran == (plan != "own" or group <= 4 or batch < 8), f"plan {plan}: whether the launch was made"
+        if plan == "own" and group <= 4:
             assert torch.equal(got, layers)
         error = (got - want).norm()
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
