@@ -188,7 +188,7 @@ class PrefillGraph:
         self.copied.record()
         self.graph = None
         self.logits = None
-        self.held = []
+        self.held, self.tables = [], []
         self._lay_out({})
 
     def _lay_out(self, list_shapes) -> None:
@@ -263,6 +263,7 @@ class PrefillGraph:
                 self.logits = self._forward()
             self.graph = graph
             self.held = list(self.engine.model.held_buffers(self.engine.rt))
+            self.tables = list(self.engine.model.held_tables(self.engine.rt))
         except KernelError:
             # a part that cannot run under capture: the shape goes on being launched
             self.graph = self.logits = None
@@ -273,6 +274,7 @@ class PrefillGraph:
 
     def run(self) -> torch.Tensor:
         """Replays the step on what the buffers hold; the rows returned view the graph's output buffer."""
+        self.engine.model.check_steps(self.engine.rt)
         self.graph.replay()
         return self.logits
 

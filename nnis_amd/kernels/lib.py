@@ -164,8 +164,8 @@ register_module_family("attn_hd", _attention_recipe)
 # the mixers that carry a state of fixed size (convolution, selective scan, gated linear attention and retention, minGRU, gated delta rule)
 register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
 # the layers of a step of few single tokens in one launch
-register_module("chain", ["chain.hip", "chain_f32.hip"], headers=["common.h", "product.h", "chain.h"],
-                source_flags={"chain.hip": _VECTOR_SUMS, "chain_f32.hip": _VECTOR_SUMS})
+register_module("chain", ["chain.hip", "chain_f32.hip", "chain_prompt.hip"], headers=["common.h", "product.h", "chain.h"],
+                source_flags={"chain.hip": _VECTOR_SUMS, "chain_f32.hip": _VECTOR_SUMS, "chain_prompt.hip": _VECTOR_SUMS})
 # the real-gated linear recurrent unit
 register_module("gated_unit", ["gated_unit.hip"], headers=["common.h"], source_flags={"gated_unit.hip": _VECTOR_SUMS})
 # Mamba-2's state spaces

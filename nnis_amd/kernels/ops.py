@@ -301,7 +301,10 @@ def chain_module():
     global _chain
     if _chain is None:
         tail = [_VOID] * 8 + [_INT, _VOID, _I64, _VOID, _I64, _VOID, _VOID]
-        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 10 + [_FLT, _FLT] + tail, "nnis_chain_f32": [_VOID] + [_INT] * 8 + [_FLT, _FLT] + tail})
+        _chain = _bind("chain", {"nnis_chain": [_VOID] + [_INT] * 10 + [_FLT, _FLT] + tail, "nnis_chain_f32": [_VOID] + [_INT] * 8 + [_FLT, _FLT] + tail,
+                                 "nnis_chain_prompt": [_VOID] + [_INT] * 8 + [_FLT, _FLT] + [_VOID] * 8 + [_I64, _VOID, _VOID]})
+        _chain.nnis_chain_prompt_words.argtypes = [_INT] * 6
+        _chain.nnis_chain_prompt_words.restype = _I64
         for words in (_chain.nnis_chain_words, _chain.nnis_chain_f32_words):
             words.argtypes = [_INT] * 7 + [ctypes.POINTER(_I64)]
             words.restype = _I64
@@ -745,6 +748,39 @@ def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables,
         _check(lib, lib.nnis_chain_f32(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, *tail))
     else:
         _check(lib, lib.nnis_chain(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, waves, _DTYPE_CODE[gain_dtype], *tail))
+    return out, last
+
+
+def chain_prompt_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16) -> bool:
+    """Whether ``chain_prompt`` is to run a prompt of ``rows`` rows: up to 1,024 (192 above a width of 1,024, where a block has the unit's
+    weights for fewer rows), an exchange of up to 512 MB, and up to rows x a layer's weights of 5.7e9, beyond which the blocks' reading
+    of weights costs more than the layers' tiled products.  Whole steps in microseconds by the layers' kernels and in one launch, rows x
+    weights in 1e9: width 576, 9/3 heads, 30 layers, 177 rows (0.6) 940 and
+    538, 1,000 (3.5) 1,627 and 1,354; 768, 12/12, 12 layers, 500 (3.6) 601 and 466, 768 (5.5) 684 and 667, 1,000 (7.1) 766 and 894; 1,024, 16/16, 12 layers, 320
+    (5.4) 725 and 625, 500 (8.4) 854 and 936; 1,280, 20/4, 16 layers, 192 (3.3) 903 and 705, 320 (5.4) 1,011 and 1,134; 2,048, 32/4, 22 layers, 60 rows as 64 (2.8) 1,232 and 891, 128 (5.6) 1,514 and 1,260,
+    190 as 192 (8.5) 1,705 and 1,824; 2,048, 32/32, 24 layers, 64 (4.3) 1,490 and 1,321, 128 (8.6) 1,786 and 1,898; 3,072, 48/8, 4 layers, 64
+    (6.2) 343 and 363."""
+    if dtype != torch.bfloat16 or head_dim != 64 or rows > (1024 if width <= 1024 else 192) or rows * width * ((2 * heads + 2 * kv_heads) * head_dim + 3 * inner) > 5.7e9:
+        return False
+    return 0 < chain_module().nnis_chain_prompt_words(layers, rows, width, heads, kv_heads, inner) <= 1 << 27
+
+
+def chain_prompt(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, failed: torch.Tensor, gain_dtype: torch.dtype,
+                 eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
+    """As ``chain``, for the rows of one prompt that begins at its sequence's first position: row i is position i."""
+    for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page")):
+        _dev(t, f"chain_prompt {what}")
+    rows = x.shape[0]
+    if (x.shape != (rows, width) or x.dtype != torch.float32 or tables.cos.shape != (rows, head_dim // 2) or tables.tokens != rows or tok_pos.numel() < rows
+            or tok_pos.dtype != torch.int32 or layers.dtype != torch.int64 or layers.numel() != 8 * count or not failed.is_pinned() or dtype != torch.bfloat16):
+        raise KernelError(f"chain_prompt: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
+    lib = chain_module()
+    words = lib.nnis_chain_prompt_words(count, rows, width, heads, kv_heads, inner)
+    exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
+    out, last = torch.empty_like(x), torch.empty_like(x, dtype=dtype)
+    _check(lib, lib.nnis_chain_prompt(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, _DTYPE_CODE[gain_dtype], float(eps), float(scale),
+                                      x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
+                                      tables.page.data_ptr(), exchange.data_ptr(), words, failed.data_ptr(), _stream()))
     return out, last
 
 

@@ -1,4 +1,4 @@
-"""A step of few single tokens through all layers in one launch (``csrc/chain.hip``).
+"""A step of few single tokens, or of one short prompt, through all layers in one launch (``csrc/chain.hip``, ``chain_prompt.hip``).
 
 A part that the launch takes says what of it there is (``chain_link``); a model whose every layer does, over one cache and one
 rotation, runs such steps through it, and all others -- other mixers, options, types, sizes, more rows, longer sequences --
@@ -49,11 +49,16 @@ class LayerChain:
         """(runs of a sequence's keys, waves of a run) for a step of these sizes, or None: the layers' own kernels."""
         return rt.ops.chain_plan(len(self.links), batch, longest, **self.sizes)
 
+    def takes_prompt(self, batch: int, rows: int, longest: int, most_new: int, rt) -> bool:
+        """Whether a step of ``batch`` sequences, the longest of ``longest`` tokens after it and ``most_new`` of them new, is one
+        short prompt from its sequence's first position on."""
+        return batch == 1 and longest == most_new and rt.ops.chain_prompt_takes(len(self.links), rows, **self.sizes)
+
     def check(self) -> None:
         """Raises if a wait of an earlier step was given up."""
         if self._failed[0]:
             self._failed[0] = 0
-            raise KernelError("a decode step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
+            raise KernelError("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
                               "the logits of the step before this one are not numbers")
 
     def views_fit(self, views) -> bool:
@@ -80,5 +85,7 @@ class LayerChain:
         if table is None:
             return None
         tables = ctx.step_tables(rt, self.position.rotary(), views[0].block_table)
-        return rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, gain_dtype=self.gain_dtype, eps=self.eps,
-                            scale=self.scale, **self.sizes)
+        more = dict(self.sizes, gain_dtype=self.gain_dtype, eps=self.eps, scale=self.scale)
+        if plan == "prompt":
+            return rt.ops.chain_prompt(table, len(self.links), x, tables, ctx.tok_pos, self.failed, **more)
+        return rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, **more)

@@ -114,6 +114,9 @@ class DecoderModel:
             plans = self._prompt_plans[key] = tuple(
                 plan for layer in (self.layers[entry.layer] for entry in self.spec.schedule)
                 for plan in (layer.prompt_plan(batch, rows, longest, rt), layer.run_plan(batch, rows, most_new, rt)))
+            chain = self.layer_chain(rt)
+            if chain is not None and chain.takes_prompt(batch, rows, longest, most_new, rt):
+                plans = self._prompt_plans[key] = plans + (("chain", "prompt"),)
         return plans
 
     def decode_plan(self, batch: int, longest: int, rt):
@@ -155,8 +158,13 @@ class DecoderModel:
     def _chained(self, stream, schedule, ctx, cache, rt):
         """(the stream behind all layers, nothing left to run) where one launch takes the step, else what it was handed."""
         x = stream[0]
-        chain = self.layer_chain(rt) if ctx.decode and not ctx.options else None
-        plan = chain.plan(ctx.batch, ctx.planned_len, rt) if chain is not None else None
+        chain = self.layer_chain(rt) if not ctx.options else None
+        if chain is None:
+            plan = None
+        elif ctx.decode:
+            plan = chain.plan(ctx.batch, ctx.planned_len, rt)
+        else:
+            plan = "prompt" if chain.takes_prompt(ctx.batch, ctx.planned_rows, ctx.planned_len, ctx.planned_new, rt) else None
         if plan is None or x.dim() != 2 or x.dtype != torch.float32 or not x.is_contiguous():
             return stream, schedule
         views = [cache.view(index) for index in range(len(schedule))]

@@ -1,7 +1,8 @@
-"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``, ``chain_f32.hip``) against the layers' own
-kernels: in bfloat16 the same bits up to a width of 1,024 in groups of up to four heads, else both measured by the 32-bit path on the
-same weights; in 32 bits both measured by the oracle in 64.  Sizes are those at which the launch changes what it does: a K that
-leaves waves without a chunk or takes them a second round, groups of heads beyond four, four and eight waves, runs of the keys."""
+"""Steps of few single tokens through all layers in one launch (``csrc/chain.hip``, ``chain_f32.hip``), or of one short prompt
+(``chain_prompt.hip``), against the layers' own kernels: single tokens in bfloat16 the same bits in groups of up to
+four heads, else both measured by the 32-bit path on the same weights; in 32 bits both measured by the oracle in 64.  Sizes are
+those at which the launch changes what it does: a K that leaves waves without a chunk or takes them a second round, groups of heads
+beyond four, four and eight waves, runs of the keys."""
 
 import numpy as np
 import pytest
@@ -110,6 +111,88 @@ def test_32_bits_against_the_oracle(tmp_path, sizes, batch, monkeypatch):
         assert ran, f"plan {plan}: the launch was not made"
         error = (got - want).norm()
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 64 bits, the layers' kernels {(layers - want).norm().item():.4g}"
+
+
+@pytest.mark.parametrize("rows", [2, 16, 33, 177, 600])
+@pytest.mark.parametrize("sizes", SIZES + [(1088, 8, 8, 4160)])  # (eight waves with a second round of down's weights)
+def test_a_prompt_against_the_layers(tmp_path, sizes, rows, monkeypatch):
+    """As far from 32 bits as the layers' kernels, the prompt's last row and the steps behind it (by the layers' kernels, from what
+    the launch left in the cache); launched and replayed the same bits.  (The roundings are the same, the orders of the sums are not.)"""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    rng = np.random.default_rng(rows)
+    prompt, tokens = rng.integers(0, 509, size=rows).tolist(), rng.integers(0, 509, size=2).tolist()
+    places = sorted({0, rows // 3, rows - 1})
+
+    def run(dtype, takes):
+        with monkeypatch.context() as patch:
+            launches = []
+            launch = ops.chain_prompt
+            patch.setattr(ops, "chain_prompt", lambda *args, **more: launches.append(1) or launch(*args, **more))
+            if takes is not None:
+                patch.setattr(ops, "chain_prompt_takes", lambda *args, **more: takes)
+            patch.setattr(ops, "chain_plan", lambda *args, **more: None)
+            engine = load_engine(str(tmp_path), dtype=dtype, max_tokens=1024)
+            slot, out = engine.start_sequence(), None
+            for again in range(4):  # launched, launched and captured, replayed
+                engine.truncate(slot, 0)
+                got = [engine.step([StepEntry(slot, prompt, places)]).double().cpu()]
+                for token in tokens:
+                    got.append(engine.step([StepEntry(slot, [token], None)]).double().cpu())
+                got = torch.cat(got)
+                assert dtype == "float32" or not launches or out is None or torch.equal(out, got)
+                out = got
+            return out, len(launches)
+
+    want, _ = run("float32", None)
+    layers, launched = run("bfloat16", False)
+    assert launched == 0
+    got, launched = run("bfloat16", True)
+    assert launched > 0
+    error, bound = (got - want).norm(), 1.33 * (layers - want).norm()
+    assert error <= bound, f"{error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
+
+
+def test_prompts_that_are_not_taken(tmp_path, monkeypatch):
+    """A prompt behind cached tokens, two prompts in a step, one beyond the rows: the layers' kernels, also where a prompt of the same
+    rows has been captured."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    nnis_amd.write_random_model(str(tmp_path), _config(192, 6, 2, 1600), 3)
+    launches = []
+    launch = ops.chain_prompt
+    monkeypatch.setattr(ops, "chain_prompt", lambda *args, **more: launches.append(1) or launch(*args, **more))
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=4096)
+    plain = load_engine(str(tmp_path), dtype="float32", max_tokens=4096)
+    rng = np.random.default_rng(5)
+    first, second = rng.integers(0, 509, size=40).tolist(), rng.integers(0, 509, size=50).tolist()
+    slot, other = engine.start_sequence(), plain.start_sequence()
+    for _ in range(3):
+        engine.truncate(slot, 0)
+        engine.step([StepEntry(slot, second, None)])
+    taken = len(launches)
+    assert taken > 0
+    engine.truncate(slot, 0)
+    engine.step([StepEntry(slot, first, None)])
+    plain.step([StepEntry(other, first, None)])
+    taken = len(launches)
+    for _ in range(3):  # the same 64 rows as the captured prompt's
+        engine.truncate(slot, len(first))
+        plain.truncate(other, len(first))
+        got, want = engine.step([StepEntry(slot, second, None)]), plain.step([StepEntry(other, second, None)])
+        assert (got.double() - want.double()).norm() <= 0.05 * want.double().norm()  # (a few bfloat16 roundings of 2^-9 over two layers)
+    assert len(launches) == taken
+    slots = [engine.start_sequence() for _ in range(2)]
+    engine.step([StepEntry(s, first, None) for s in slots])
+    engine.step([StepEntry(engine.start_sequence(), rng.integers(0, 509, size=1100).tolist(), None)])
+    assert len(launches) == taken
 
 
 def test_not_taken(tmp_path, monkeypatch):
