@@ -18,7 +18,7 @@
 
 namespace {
 
-constexpr int kSampleThreads = 512;  // 8 waves: a thread may keep up to 128 keys of its row in registers
+constexpr int kSampleThreads = 512, kHeldMost = 128;  // 8 waves: a thread may keep up to 128 keys of its row in registers
 
 __device__ __forceinline__ unsigned ordered_key(float v) {
   if (v == 0.0f) v = 0.0f;  // -0 and +0 compare equal
@@ -81,15 +81,21 @@ __device__ __forceinline__ int load_keys(Keys<PER>& keys, const RowView& r) {
   return bad;
 }
 
+// A row with a top-k of up to kFewMost has its few candidates' weights made by its own block (sample_few), if a thread holds up to
+// kFewHeld keys.  (Beside 128 of them this path's registers push keys of the general one into memory: 11 rows of 65,000, a top-k of 400,
+// 145 us for a draw and 230.)
+constexpr int kFewMost = 256, kFew = kSampleThreads, kFewHeld = 96;
+__device__ __forceinline__ bool takes_few(int k, int vocab) { return k > 0 && k < vocab && k <= kFewMost && vocab <= kFewHeld * kSampleThreads; }
+
 // The weights exp((l - l_max) / T) of every row that samples, 64-bit, with all of the chip (a row's own block
 // would take 49,152 of them 40 us and more).  `best` holds an index of each row's maximum.
 constexpr int kWeightThreads = 256, kWeightsEach = 8;
 __global__ __launch_bounds__(kWeightThreads) void sample_weights_kernel(
     const float* __restrict__ logits, double* __restrict__ weights, int vocab, const int* __restrict__ row_slot,
-    const float* __restrict__ temperature, int by_slot, const int* __restrict__ best) {
+    const float* __restrict__ temperature, const int* __restrict__ top_k, int by_slot, const int* __restrict__ best) {
   const int row = blockIdx.y;
   const int slot = row_slot[row];
-  if (slot < 0) return;
+  if (slot < 0 || takes_few(top_k[by_slot ? slot : row], vocab)) return;
   const float* l = logits + (size_t)row * vocab;
   double* w = weights + (size_t)row * vocab;
   const double inv_t = 1.0 / (double)temperature[by_slot ? slot : row];
@@ -159,6 +165,115 @@ __device__ __forceinline__ int count_at_least(const RowView& r, const Keys<PER>&
   }
 }
 
+// The draw among the k largest of a row, k up to kFewMost: by bits from the top down to a bound that kFew tokens and fewer are at or
+// above (k and more are), those into LDS, each thread's token into its place among them by (logit, id), and the rest by one wave on
+// the running sums of the first k's weights: top-p keeps them up to the first that reaches its threshold, the draw is the first
+// beyond its own.  False, and nothing done, if equal keys leave more than kFew.
+// Bound by the chain of about fourteen counts, half a microsecond each, behind the row's way into one compute unit's registers.  The
+// general search below sums weights from memory for each probe that it cannot decide by counts: a draw from 11 rows of
+// 49,152 with a top-k of 50 and a top-p of 0.9 takes it 123 us with the other three kernels, this 33; of 4,000 78 and 18; 49,152 with a
+// top-k of 256 124 and 38.
+struct FewTokens {
+  unsigned long long order[kFew];  // key, then the smaller id first
+  double weight[kFewMost];
+  int id[kFewMost];
+  int wave_count[kSampleThreads / kWave];
+};
+template <int PER>
+__device__ __forceinline__ bool sample_few(FewTokens& few, const RowView& r, const Keys<PER>& keys, int k, float p, double inv_t, double max_scaled,
+                                           unsigned long long* state_at, int* out, int* scratch) {
+  unsigned t = 0;
+  int below = r.vocab;
+  for (int bit = 31; bit >= 0 && below > kFew; --bit) {
+    const unsigned probe = t | (1u << bit);
+    const int count = count_at_least<PER>(r, keys, probe, scratch);
+    if (count >= k) {
+      t = probe;
+      below = count;
+    }
+  }
+  if (below > kFew) return false;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const unsigned from = t > 1u ? t : 1u;
+  int mine = 0;
+#pragma clang loop unroll(full)
+  for (int i = 0; i < PER; ++i) mine += keys.held[i] >= from ? 1 : 0;
+  int upto = mine;
+#pragma unroll
+  for (int offset = 1; offset < kWave; offset <<= 1) {
+    const int other = __shfl_up(upto, offset, kWave);
+    upto += lane >= offset ? other : 0;
+  }
+  if (lane == kWave - 1) few.wave_count[wave] = upto;
+  __syncthreads();
+  int place = upto - mine;
+  for (int w = 0; w < wave; ++w) place += few.wave_count[w];
+#pragma clang loop unroll(full)
+  for (int i = 0; i < PER; ++i)
+    if (keys.held[i] >= from) few.order[place++] = ((unsigned long long)keys.held[i] << 32) | (unsigned)~(threadIdx.x + i * kSampleThreads);
+  __syncthreads();
+  if ((int)threadIdx.x < below) {
+    const unsigned long long own = few.order[threadIdx.x];
+    int rank = 0;
+    for (int i = 0; i < below; ++i) rank += few.order[i] > own ? 1 : 0;
+    if (rank < k) {
+      const unsigned key = (unsigned)(own >> 32);
+      few.id[rank] = (int)~(unsigned)own;
+      few.weight[rank] = exp((double)__uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key) * inv_t - max_scaled);
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return true;
+  constexpr int kEach = kFewMost / kWave;
+  double sum[kEach];  // up to and with each of the lane's tokens
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    const int at = lane * kEach + i;
+    sum[i] = (i > 0 ? sum[i - 1] : 0.0) + (at < k ? few.weight[at] : 0.0);
+  }
+  double upto_lane = sum[kEach - 1];
+#pragma unroll
+  for (int offset = 1; offset < kWave; offset <<= 1) {
+    const double other = __shfl_up(upto_lane, offset, kWave);
+    upto_lane = lane >= offset ? other + upto_lane : upto_lane;
+  }
+  const double before = __shfl_up(upto_lane, 1, kWave);
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) sum[i] = lane > 0 ? before + sum[i] : sum[i];
+  // how many of the first `kept` tokens' running sums `under` holds for
+  auto count = [&](int kept, auto under) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) n += lane * kEach + i < kept && under(sum[i]) ? 1 : 0;
+#pragma unroll
+    for (int offset = kWave / 2; offset > 0; offset >>= 1) n += __shfl_xor(n, offset, kWave);
+    return n;
+  };
+  auto sum_at = [&](int index) {
+    double v = 0.0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) v = index % kEach == i ? sum[i] : v;
+    return __shfl(v, index / kEach, kWave);
+  };
+  int kept = k;
+  double total = sum_at(k - 1);
+  if (p > 0.0f && p < 1.0f) {
+    const double threshold = (double)p * total;
+    const int reached = count(k, [&](double v) { return v < threshold; }) + 1;
+    kept = reached < k ? reached : k;
+    total = sum_at(kept - 1);
+  }
+  unsigned long long state = *state_at;
+  const unsigned long long raw = splitmix64_next(&state);
+  const double draw = (double)(raw >> 11) * (1.0 / 9007199254740992.0) * total;
+  const int index = count(kept, [&](double v) { return !(v > draw); });
+  if (lane == 0) {
+    *out = few.id[index < kept ? index : kept - 1];
+    *state_at = state;
+  }
+  return true;
+}
+
 template <int PER>
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     const float* __restrict__ logits, double* __restrict__ weights, int vocab, const int* __restrict__ row_slot,
@@ -188,6 +303,15 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   if (top == 0.0f) top = 0.0f;
   const double max_scaled = (double)top * inv_t;
 
+  if constexpr (PER > 0 && PER <= kFewHeld) {
+    __shared__ FewTokens few;
+    if (takes_few(top_k[at], vocab)) {
+      if (sample_few<PER>(few, r, keys, top_k[at], top_p[at], inv_t, max_scaled, rng + slot, out + row, scratch_i)) return;
+      // (many equal keys: the weights that sample_weights_kernel left out)
+      for (int c = threadIdx.x; c < vocab; c += kSampleThreads) w[c] = exp((double)r.logits[c] * inv_t - max_scaled);
+      __syncthreads();
+    }
+  }
   // the kept prefix: everything with key > cut_key plus `cut_ties` tokens at cut_key
   unsigned cut_key = 0;
   int cut_ties = 0;          // meaningful only when limited
@@ -447,15 +571,15 @@ extern "C" int nnis_sample(const float* logits, double* weights, int rows, int v
   const dim3 grid(rows), block(kSampleThreads);
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(sample_weights_kernel, dim3((vocab + kWeightThreads * kWeightsEach - 1) / (kWeightThreads * kWeightsEach), rows),
-                     dim3(kWeightThreads), 0, s, logits, weights, vocab, row_slot, temperature, by_slot, best);
+                     dim3(kWeightThreads), 0, s, logits, weights, vocab, row_slot, temperature, top_k, by_slot, best);
 #define NNIS_SAMPLE(PER) hipLaunchKernelGGL(sample_kernel<PER>, grid, block, 0, s, logits, weights, vocab, row_slot, rng, temperature, top_k, top_p, by_slot, best, out)
   // elements a thread keeps in registers: the least that covers the row
   if (vocab <= 8 * kSampleThreads) NNIS_SAMPLE(8);
   else if (vocab <= 16 * kSampleThreads) NNIS_SAMPLE(16);
   else if (vocab <= 32 * kSampleThreads) NNIS_SAMPLE(32);
   else if (vocab <= 64 * kSampleThreads) NNIS_SAMPLE(64);
-  else if (vocab <= 96 * kSampleThreads) NNIS_SAMPLE(96);
-  else if (vocab <= 128 * kSampleThreads) NNIS_SAMPLE(128);
+  else if (vocab <= kFewHeld * kSampleThreads) NNIS_SAMPLE(kFewHeld);
+  else if (vocab <= kHeldMost * kSampleThreads) NNIS_SAMPLE(kHeldMost);
   else NNIS_SAMPLE(0);
 #undef NNIS_SAMPLE
   NNIS_LAUNCH_CHECK("sample");

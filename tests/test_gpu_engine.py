@@ -552,6 +552,36 @@ def test_device_sampling_matches_the_host_sampler(options, vocab):
     assert out[3].item() == -1 and out[0].item() >= 0
 
 
+@pytest.mark.parametrize("top_k", [1, 64, 255, 256, 257])
+@pytest.mark.parametrize("vocab", [300, 512, 513, 49152, 49153])
+def test_draws_among_few_tokens_match_the_host_sampler(vocab, top_k):
+    """Both sides of what the draw among few tokens takes: a top-k of up to 256, of up to 49,152 logits, no more than 512 of them
+    at or above its bound (with ties at the k-th that leave as many, and more)."""
+    from nnis_amd.kernels import ops
+    from nnis_amd.sampling import HostSampler, SamplingParams
+
+    rng = np.random.default_rng(vocab + top_k)
+    logits = (rng.standard_normal((4, vocab)) * 2.0).astype(np.float32)
+    for row, ties in ((1, 512), (2, 513)):  # this many at the k-th place and above
+        order = np.argsort(-logits[row], kind="stable")
+        logits[row, order[min(top_k, vocab) - 1:min(ties, vocab)]] = logits[row, order[min(top_k, vocab) - 1]]
+    logits[3] = np.abs(logits[3]) * -1.0  # the largest is below zero, or -0
+    logits[3, vocab // 2] = -0.0
+    dev = torch.from_numpy(logits).cuda()
+    slots = [2, 0, 3, 1]
+    state = torch.tensor([5, 6, 7, 8], dtype=torch.int64, device="cuda")
+    hosts = [HostSampler(SamplingParams(seed=5 + slot, temperature=0.7, top_k=top_k, top_p=p), vocab) for slot, p in zip(slots, (0.9, 0.99, 1.0, 0.5))]
+    temperature = torch.full((4,), 0.7, dtype=torch.float32, device="cuda")
+    top_ks = torch.full((4,), top_k, dtype=torch.int32, device="cuda")
+    top_p = torch.tensor([0.9, 0.99, 1.0, 0.5], dtype=torch.float32, device="cuda")
+    weights = torch.full((4, vocab), float("nan"), dtype=torch.float64, device="cuda")
+    row_slot = torch.tensor(slots, dtype=torch.int32, device="cuda")
+    for draw in range(8):
+        out = torch.full((4,), -7, dtype=torch.int32, device="cuda")
+        ops.sample(dev, weights, row_slot, state, temperature, top_ks, top_p, out)
+        assert out.tolist() == [host.sample(row) for host, row in zip(hosts, logits)], draw
+
+
 def test_sampled_generation_is_seeded_and_per_sequence(model_dirs):
     import nnis_amd
     from nnis_amd.api import load_engine
