@@ -2,7 +2,7 @@
 //
 // How words get from block to block: every word of the exchange is kNone (all bits set) before the launch, and is there once it is
 // anything else.  Writers store past the caches and never store kNone (a NaN with that payload goes out as another NaN), readers
-// load past the caches until no word of what they asked for is kNone.  A word carries its own mark, so no order between
+// load until no word of what they asked for is kNone.  A word carries its own mark, so no order between
 // words is needed, no counter and no fence.
 //
 // Why every wait ends: the stages of a block's operands are blocks of smaller numbers, and a die is handed its blocks in the order
@@ -78,48 +78,47 @@ struct Exchange {
   }
 
   // 16 bytes a lane N times, and beside each an M-th of 4 or 8 bytes: `ask(i)` gives the i-th's byte offsets, the lane's part and
-  // the wave's; until all of them are there
-  template <int N, typename Ask>
-  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask) const {
-    int looks = 0;
-    long long since = 0;
-    while (true) {
+  // the wave's; whether all of them are there
+  template <int POLICY, int N, typename Ask>
+  __device__ __forceinline__ bool look(u32x4 (&v)[N], Ask ask) const {
 #pragma unroll
-      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
-      asm volatile("" ::: "memory");
-      unsigned top = 0;
+    for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, POLICY);
+    asm volatile("" ::: "memory");  // (asked for anew each time)
+    unsigned top = 0;
 #pragma unroll
-      for (int i = 0; i < N; ++i)
+    for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
-      if (!__any(top == kNone) || leave(looks, since)) return;
-    }
+      for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
+    return !__any(top == kNone);
   }
-  template <int N, typename Ask, typename T, int M, typename AskBeside>
-  __device__ __forceinline__ void take(u32x4 (&v)[N], Ask ask, T (&w)[M], AskBeside ask_beside) const {
+  template <int POLICY, int N, typename Ask, typename T, int M, typename AskBeside>
+  __device__ __forceinline__ bool look(u32x4 (&v)[N], Ask ask, T (&w)[M], AskBeside ask_beside) const {
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      if constexpr (sizeof(T) == 4) w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, ask_beside(i).lane, ask_beside(i).wave, POLICY);
+      else w[i] = __builtin_amdgcn_raw_buffer_load_b64(r, ask_beside(i).lane, ask_beside(i).wave, POLICY);
+    }
+    const bool all = look<POLICY>(v, ask);
+    unsigned top = 0;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      if constexpr (sizeof(T) == 4) top = max(top, w[i]);
+      else top = max(top, max(w[i][0], w[i][1]));
+    }
+    return !__any(top == kNone) && all;
+  }
+
+  // ... until all of them are there.  The first look goes through the caches, which may have them from a neighbour's: a word is
+  // written once in a launch, so a cached one is what was written or still none; a line that was fetched half written stays
+  // so, and all further looks go past them.  (16 rows of 32 heads and a width of 2,048 1,405 us and 1,259, 8 rows 1,147 and 1,112; a
+  // prompt of 177 rows of width 576, with nothing through the caches 552 and 482; few rows of narrow models alike, whose products
+  // leave it out, NEAR: with it they spill.)
+  template <bool NEAR = true, int N, typename... Rest>
+  __device__ __forceinline__ void take(u32x4 (&v)[N], Rest&&... rest) const {
+    if (NEAR && look<0>(v, rest...)) return;
     int looks = 0;
     long long since = 0;
-    while (true) {
-#pragma unroll
-      for (int i = 0; i < M; ++i) {
-        if constexpr (sizeof(T) == 4) w[i] = __builtin_amdgcn_raw_buffer_load_b32(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
-        else w[i] = __builtin_amdgcn_raw_buffer_load_b64(r, ask_beside(i).lane, ask_beside(i).wave, kPastCaches);
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(r, ask(i).lane, ask(i).wave, kPastCaches);
-      asm volatile("" ::: "memory");
-      unsigned top = 0;
-#pragma unroll
-      for (int i = 0; i < M; ++i) {
-        if constexpr (sizeof(T) == 4) top = max(top, w[i]);
-        else top = max(top, max(w[i][0], w[i][1]));
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
-      if (!__any(top == kNone) || leave(looks, since)) return;
-    }
+    while (!look<kPastCaches>(v, rest...) && !leave(looks, since)) {}
   }
   __device__ __forceinline__ void put(unsigned word, unsigned v) const { __builtin_amdgcn_raw_buffer_store_b32(v, r, word * 4, 0, kPastCaches); }
   __device__ __forceinline__ void put(unsigned word, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, r, word * 4, 0, kPastCaches); }

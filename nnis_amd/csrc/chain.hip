@@ -70,6 +70,7 @@ __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builti
 template <int WAVES, int STRIPS, int STEPS, int XB, int V, bool NEXT = false>
 struct Product {
   static_assert(STEPS % XB == 0 && STEPS % V == 0, "whole trips");
+  static constexpr bool kNear = WAVES == 8 || STEPS == 8;  // (Exchange::take; wide models')
   bf16x8 w[STEPS][2][STRIPS];
   f32x4 acc[V][STRIPS];
   const bf16_t* strip[STRIPS];
@@ -120,8 +121,8 @@ struct Product {
         unsigned part[XB];
         auto step = [&](int d) { return (unsigned)min(chunk(d0, b + d), chunks - 1) * 4 * stride; };
         auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
-        if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
-        else ex.take(v, pieces);
+        if constexpr (SUM) ex.template take<kNear>(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
+        else ex.template take<kNear>(v, pieces);
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
           const int c = chunk(d0, b + d);

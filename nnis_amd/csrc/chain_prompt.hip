@@ -1,14 +1,18 @@
-// The layers of a step of one short prompt in one launch: chain.hip's stages for up to 256 rows that begin at a sequence's first
-// position (pre-norm blocks of plain attention with heads of 64 channels and a SiLU-gated feed-forward, bfloat16).
+// The layers of a step of one short prompt in one launch: chain.hip's stages for up to 1,024 rows that begin at a sequence's first
+// position (pre-norm blocks of plain attention with heads of 64 channels and a SiLU-gated feed-forward, bfloat16).  Where it is
+// taken and what it measures there: kernels/ops.py, chain_prompt_takes.
+//
+// What bounds it is the way from stage to stage, about 3 us of five a layer (30 layers of width 576, 177 rows: 440 of 480 us), and on wide
+// models the weights, of which a compute unit holds one block's.
 //
 // Rows are tiles of 16; a block has a unit of weight rows and 2 or 4 tiles, and 8 waves: K is cut PARTS ways, a wave has a part of K
-// and two tiles.  Tiles come in pairs: rows beyond the step's are computed as rows of zeros, so that every word that is waited for is
-// written.
+// and two tiles (four from 65 rows on where the model is wide, for a unit's weights to be read half as often: 128 rows of width 2,048, 22
+// layers, 1,503 us and 1,250).  Tiles come in pairs: rows beyond the step's are computed as rows of zeros, so that every word that is
+// waited for is written.
 //
-// Words are handed on as in chain.h, but the blocks of a stage read the same words many times over, and past the caches that
-// would be tens of megabytes a stage: a wave looks, past the caches, at one word of each piece that it needs, and then loads through
-// them; what is not yet there after all (a line that was fetched half written stays so in a cache) it asks for past them.  A word
-// is written once in a launch, so a cached one is what was written or still none.
+// Words are handed on as in chain.h.  The blocks of a stage read the same words many times over, and past the caches that would be
+// tens of megabytes a stage: the first look through them finds most.  (With a look, past the caches, at a word of each piece before
+// it: 177 rows of width 576 536 us and not 482.)
 #include <hip/hip_runtime.h>
 
 #include "chain.h"
@@ -75,48 +79,6 @@ __device__ __forceinline__ void place(int block, int units, int groups, int& uni
   unit = (block < whole * groups ? at / (8 * groups) * 8 : whole) + at % apart;
 }
 
-// N words a lane, until all are there
-template <int N>
-__device__ __forceinline__ void near_gate(const Exchange& ex, const unsigned (&word)[N]) {
-  int looks = 0;
-  long long since = 0;
-  while (true) {
-    unsigned top = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) top = max(top, __builtin_amdgcn_raw_buffer_load_b32(ex.r, word[i] * 4, 0, kPastCaches));
-    asm volatile("" ::: "memory");
-    if (!__any(top == kNone) || ex.leave(looks, since)) return;
-  }
-}
-
-// Exchange::take through the caches first
-template <int N, typename Ask, int M, typename AskBeside>
-__device__ __forceinline__ void take_near(const Exchange& ex, u32x4 (&v)[N], Ask ask, unsigned (&w)[M], AskBeside ask_beside) {
-#pragma unroll
-  for (int i = 0; i < M; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(ex.r, ask_beside(i).lane, ask_beside(i).wave, 0);
-#pragma unroll
-  for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(ex.r, ask(i).lane, ask(i).wave, 0);
-  unsigned top = 0;
-#pragma unroll
-  for (int i = 0; i < M; ++i) top = max(top, w[i]);
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
-  if (__any(top == kNone)) ex.take(v, ask, w, ask_beside);
-}
-template <int N, typename Ask>
-__device__ __forceinline__ void take_near(const Exchange& ex, u32x4 (&v)[N], Ask ask) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(ex.r, ask(i).lane, ask(i).wave, 0);
-  unsigned top = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) top = max(top, v[i][e]);
-  if (__any(top == kNone)) ex.take(v, ask);
-}
-
 // STRIPS strips of 16 weight rows times the tiles of a block, TILES a wave, K (chunks of 64) cut PARTS ways: part p has the chunks p, p + PARTS, ..
 // A wave asks for the weights of its first STEPS chunks when the block begins; TRIP chunks of the operand are asked for together.
 template <int STRIPS, int PARTS, int TILES, int STEPS, int TRIP, bool NORM>
@@ -163,16 +125,8 @@ struct PromptProduct {
     if (tile >= a.tiles) return;
     constexpr int kWords = NORM ? kPrepared : kPiece;
     const unsigned at = (words + (lane / 16 * a.tiles + tile) * kWords + lane % 16 * 8) * 4;
-    constexpr int kLooks = (STEPS * 4 * TILES + kWave - 1) / kWave;
     for (int base = part; base < chunks; base += PARTS * STEPS) {
       if (base != part) ask(base);
-      unsigned look[kLooks];
-#pragma unroll
-      for (int n = 0; n < kLooks; ++n) {
-        const int i = min(lane + n * kWave, STEPS * 4 * TILES - 1), c = min(base + i / (4 * TILES) * PARTS, chunks - 1);
-        look[n] = words + ((c * 4 + i % 4) * a.tiles + tile + min(i / 4 % TILES, a.tiles - 1 - tile)) * kWords;
-      }
-      near_gate(ex, look);
 #pragma unroll
       for (int b = 0; b < STEPS; b += TRIP) {
         if (base + b * PARTS >= chunks) continue;
@@ -183,8 +137,8 @@ struct PromptProduct {
           u32x4 v[TRIP * 2];
           unsigned sums[TRIP];
           auto pieces = [&](int i) { return At{at + i % 2 * 16 + t * kWords * 4, chunk(i / 2)}; };
-          if constexpr (NORM) take_near(ex, v, pieces, sums, [&](int i) { return At{at - lane % 16 * 28 + kSums * 4 + t * kWords * 4, chunk(i)}; });
-          else take_near(ex, v, pieces);
+          if constexpr (NORM) ex.take(v, pieces, sums, [&](int i) { return At{at - lane % 16 * 28 + kSums * 4 + t * kWords * 4, chunk(i)}; });
+          else ex.take(v, pieces);
 #pragma unroll
           for (int d = 0; d < TRIP; ++d) {
             if (base + (b + d) * PARTS >= chunks) continue;
@@ -332,13 +286,8 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
   for (int c = 0; c < HD / 16; ++c) o[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   float reference = -INFINITY, sum = 0.0f;
   for (int pair = wave; pair < pairs; pair += kWaves) {
-    const unsigned keys = k + 2 * pair * kPiece, values = v + pair * kValues;
-    const int n = min(lane, 19);
-    const unsigned look[1] = {n < 4 ? q + n * a.tiles * kPiece
-                              : n < 12 ? keys + ((n - 4) / 2 * a.tiles + n % 2) * kPiece : values + (n - 12) / 2 * 256 + n % 2 * 2};
-    near_gate(ex, look);
     u32x4 got[10];
-    take_near(ex, got, [&](int i) {
+    ex.take(got, [&](int i) {
       if (i < 2) return At{(q + g * a.tiles * kPiece + r * 8 + i * 4) * 4, 0};
       if (i < 6) return At{(k + g * a.tiles * kPiece + r * 8 + i % 2 * 4) * 4, (unsigned)((2 * pair + (i - 2) / 2) * kPiece * 4)};
       return At{(v + r * 16 + g * 4) * 4, (unsigned)(pair * kValues * 4 + (i - 6) * 1024)};

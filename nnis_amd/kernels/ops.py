@@ -755,11 +755,11 @@ def chain_prompt_takes(layers: int, rows: int, width: int, heads: int, kv_heads:
     """Whether ``chain_prompt`` is to run a prompt of ``rows`` rows: up to 1,024 (192 above a width of 1,024, where a block has the unit's
     weights for fewer rows), an exchange of up to 512 MB, and up to rows x a layer's weights of 5.7e9, beyond which the blocks' reading
     of weights costs more than the layers' tiled products.  Whole steps in microseconds by the layers' kernels and in one launch, rows x
-    weights in 1e9: width 576, 9/3 heads, 30 layers, 177 rows (0.6) 940 and
-    538, 1,000 (3.5) 1,627 and 1,354; 768, 12/12, 12 layers, 500 (3.6) 601 and 466, 768 (5.5) 684 and 667, 1,000 (7.1) 766 and 894; 1,024, 16/16, 12 layers, 320
-    (5.4) 725 and 625, 500 (8.4) 854 and 936; 1,280, 20/4, 16 layers, 192 (3.3) 903 and 705, 320 (5.4) 1,011 and 1,134; 2,048, 32/4, 22 layers, 60 rows as 64 (2.8) 1,232 and 891, 128 (5.6) 1,514 and 1,260,
-    190 as 192 (8.5) 1,705 and 1,824; 2,048, 32/32, 24 layers, 64 (4.3) 1,490 and 1,321, 128 (8.6) 1,786 and 1,898; 3,072, 48/8, 4 layers, 64
-    (6.2) 343 and 363."""
+    weights in 1e9: width 576, 9/3 heads, 30 layers, 177 rows (0.6) 940 and 483, 1,000 (3.5) 1,627 and 1,232; 768, 12/12, 12 layers, 500
+    (3.6) 598 and 427, 768 (5.5) 673 and 609, 1,000 (7.1) 761 and 835; 1,024, 16/16, 12 layers, 320 (5.4) 723 and 570, 500 (8.4) 851 and
+    873; 1,280, 20/4, 16 layers, 192 (3.3) 900 and 649, 320 (5.4) 1,005 and 1,037; 2,048, 32/4, 22 layers, 60 rows as 64 (2.8) 1,220 and 835,
+    128 (5.6) 1,519 and 1,173, 190 as 192 (8.5) 1,695 and 1,669; 2,048, 32/32, 24 layers, 64 (4.3) 1,479 and 1,246, 128 (8.6) 1,793 and
+    1,759; 3,072, 48/8, 4 layers, 64 (6.2) 338 and 344."""
     if dtype != torch.bfloat16 or head_dim != 64 or rows > (1024 if width <= 1024 else 192) or rows * width * ((2 * heads + 2 * kv_heads) * head_dim + 3 * inner) > 5.7e9:
         return False
     return 0 < chain_module().nnis_chain_prompt_words(layers, rows, width, heads, kv_heads, inner) <= 1 << 27
