@@ -1,5 +1,7 @@
 // The layers of a step of few single tokens in one launch (pre-norm blocks of plain attention with heads of 64 channels and a
-// SiLU-gated feed-forward, bfloat16, up to 16 rows).
+// SiLU-gated feed-forward, bfloat16, up to 16 rows; up to a width of 1,024 32, as two tiles of rows that have nothing to do with
+// one another: 24 rows of 30 layers of width 576 1,037 us by the layers' kernels and 805, 32 rows 968 and 704, but 48 rows of 600 to 2,000
+// tokens 1,153 and 1,380).
 //
 // What bounds such a step is neither bytes nor products but its chain of dependent kernels, five to six a layer: each begins
 // 1.6 us after the one before has ended, asks for its weights, and only then has something to multiply.  Here a layer's stages
@@ -21,7 +23,7 @@ namespace {
 
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 
-constexpr int HD = kChainHead;
+constexpr int HD = kChainHead, kMostNarrowRows = 32;
 constexpr float kLazyRise = 8.0f;  // as in attention.hip: a softmax reference moves when a score rises 2^8 above it
 
 struct ChainLayer {
@@ -32,7 +34,7 @@ struct ChainLayer {
 
 struct ChainArgs {
   const ChainLayer* layers;
-  int layer_count, m, width, heads, kv_heads, inner, splits, gain_dtype;
+  int layer_count, rows, tiles, m, width, heads, kv_heads, inner, splits, gain_dtype;
   // how many ways K is cut (the first layer's queries, keys and values; the others'; output, gate/up, down), and the waves that
   // share a run's pages
   int parts_first, parts_qkv, parts_out, parts_gate, parts_down, page_waves, down_paired;
@@ -44,12 +46,13 @@ struct ChainArgs {
   const int *tok_pos, *tok_page, *tok_pages;
   int max_pages;
   unsigned *words, *run_words;  // (the runs lie apart: in the scratch that the split decode attention has)
-  unsigned words_bytes, run_bytes, layer_words, layer_runs;
+  unsigned words_bytes, run_bytes, layer_words, layer_runs;  // of a tile, as m: at most 16 of the step's rows
   // where a layer's words lie: the stream's records before the attention and before the feed-forward; queries, keys, values;
   // attention rows; gated rows
   unsigned stream1, stream2, q, k, v, attn, act;
   int n_strip;        // strips of the stream
-  int n_entry, n_qkv, n_att, n_comb, n_out, n_gate, n_down;  // blocks of a stage
+  int n_qkv, n_att, n_comb, n_out, n_gate, n_down;  // blocks of a stage for a tile (the last may have fewer of the attention's two)
+  int n_att_all, n_comb_all;
   unsigned *fail, *host_fail;
 };
 
@@ -253,6 +256,31 @@ __device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Ex
   return true;
 }
 
+// A row of the embedding into the first layer's records.  Of a step of more than 16 rows it is normed as the layers' kernel of its own for
+// that does it, a lane per 4 of 256 channels, and its product needs no scale.
+__device__ __forceinline__ void normed_entry_stage(const ChainArgs& a, const Exchange& ex, float& shared_scale, int row) {
+  const float* x = a.x + (size_t)row * a.width;
+  if (threadIdx.x < kWave) {
+    float sum = 0.0f;
+    for (int c = threadIdx.x * 4; c < a.width; c += kWave * 4) {
+      const f32x4 v = *(const f32x4*)(x + c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = fmaf(v[e], v[e], sum);
+    }
+    const float inv_width = 1.0f / (float)a.width, scale = 1.0f / sqrtf(wave_sum(sum) * inv_width + a.eps);
+    if (threadIdx.x == 0) shared_scale = scale;
+  }
+  __syncthreads();
+  const float scale = shared_scale;
+  for (int c = threadIdx.x * 4; c < a.width; c += blockDim.x * 4) {
+    const f32x4 v = *(const f32x4*)(x + c), normed = (v * scale) * four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
+    const unsigned word = a.stream1 + (c / 16 * a.m + row) * kRecord, four = c % 16 / 4;
+    ex.put(word + 2 * four, (u32x2){marked2((bf16_t)normed[0], (bf16_t)normed[1]), marked2((bf16_t)normed[2], (bf16_t)normed[3])});
+    if (four == 0) ex.put(word + kRecordSum, marked(0.0f));
+    ex.put(word + kRecordStream + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+  }
+}
+
 // A row of the embedding into the first layer's records.  Its sum of squares is one part, added up as the layers' kernel for a row
 // that no norm has prepared does: a lane per (part of K, 16 of a chunk's 64 channels).
 template <int WAVES>
@@ -287,7 +315,7 @@ __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& 
 }
 
 // queries, keys and values of two strips (a head's channels f .. f + 15 and f + 32 ..), rotated, and the write into the cache
-template <int WAVES, bool FIRST>
+template <int WAVES, bool FIRST, bool NORMED = false>
 __device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int unit) {
   constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
@@ -307,7 +335,14 @@ __device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex
   float scale;
   if (!run_prepared<WAVES, kUnits, 2, kParts>(a, ex, s, p, here + a.stream1, row, wave, lane, sums, scale)) return;
   if (r >= a.m) return;
-  const f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
+  f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
+  if (NORMED && layer == 0) {  // of a normed row, by way of 16 bits, as the layers' two kernels for that
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      lo[e] = (float)(__bf16)sums[0][e];
+      hi[e] = (float)(__bf16)sums[1][e];
+    }
+  }
   f32x4 out_lo = lo, out_hi = hi;
   if (head < a.heads + a.kv_heads) {
     out_lo = lo * c - hi * sn;
@@ -585,7 +620,7 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
   const int item = min(first + lane / 16, items - 1), head = item / a.m, row = item % a.m, channel = lane % 16 * 4;
   ex.template gate<false>(here + a.q + first * 61 % (items * (HD / 2)), 0);
   const Exchange runs(a, a.run_words, a.run_bytes);
-  const bool alone = a.m > 4;
+  const bool alone = a.rows > 4;
   const unsigned first_run = layer * a.layer_runs + (row * a.heads + head) * a.splits * kRunRow;
   const bf16x4 out = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, alone)
                      : a.splits <= 8 ? sum_runs<8>(runs, first_run, a.splits, channel, alone) : sum_runs<16>(runs, first_run, a.splits, channel, alone);
@@ -686,33 +721,65 @@ __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& e
   ex.put(here + a.act + (unit * a.m + row) * 8 + 2 * g, (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
 }
 
-template <int WAVES>
+// TILED: more than 16 rows (beside its arithmetic steps of up to 16 are half a per cent slower)
+template <int WAVES, bool TILED>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? 3 : 2))) void chain_kernel(ChainArgs a) {
   __shared__ Shared<WAVES> s;
-  const Exchange ex(a, a.words, a.words_bytes);
-  int b = blockIdx.x;
-  if (b < a.n_entry) return entry_stage<WAVES>(a, ex, s, b);
-  b -= a.n_entry;
-  const int per_layer = a.n_qkv + a.n_att + a.n_comb + a.n_out + a.n_gate + a.n_down;
-  const int layer = b / per_layer;
-  b -= layer * per_layer;
-  if (b < a.n_qkv) {
-    if (WAVES == 4 && layer == 0) return qkv_stage<WAVES, true>(a, ex, s, layer, b);
-    return qkv_stage<WAVES, false>(a, ex, s, layer, b);
+  int b = blockIdx.x, layer = -1, stage = -1, tile = 0;
+  auto in = [&](int index, int blocks, int all) {  // the stage with this index has `blocks` for a tile
+    if (stage >= 0) return;
+    if (b < all) {
+      stage = index;
+      if (TILED) {
+        tile = b / blocks;
+        b -= tile * blocks;
+      }
+    } else {
+      b -= all;
+    }
+  };
+  in(0, kMostRows, a.rows);
+  if (stage < 0) {
+    const int per_layer = a.tiles * (a.n_qkv + a.n_out + a.n_gate + a.n_down) + a.n_att_all + a.n_comb_all;
+    layer = b / per_layer;
+    b -= layer * per_layer;
+    in(1, a.n_qkv, a.tiles * a.n_qkv);
+    in(2, a.n_att, a.n_att_all);
+    in(3, a.n_comb, a.n_comb_all);
+    in(4, a.n_out, a.tiles * a.n_out);
+    in(5, a.n_gate, a.tiles * a.n_gate);
+    in(6, a.n_down, a.tiles * a.n_down);
   }
-  b -= a.n_qkv;
-  if (b < a.n_att) return attention_stage<WAVES>(a, ex, s, layer, b);
-  b -= a.n_att;
-  if (b < a.n_comb) return combine_stage<WAVES>(a, ex, layer, b);
-  b -= a.n_comb;
-  if (b < a.n_out) return strip_stage<WAVES, false, false>(a, ex, s, layer, b);
-  b -= a.n_out;
-  if (b < a.n_gate) {
+  if constexpr (TILED) {  // from here on the tile's rows are all there is
+    a.x += (size_t)tile * kMostRows * a.width;
+    a.x_out += (size_t)tile * kMostRows * a.width;
+    a.y_out += (size_t)tile * kMostRows * a.width;
+    a.tok_cos += tile * kMostRows * (HD / 2);
+    a.tok_sin += tile * kMostRows * (HD / 2);
+    a.tok_pos += tile * kMostRows;
+    a.tok_page += tile * kMostRows;
+    a.tok_pages += (size_t)tile * kMostRows * a.max_pages;
+    a.words += (size_t)tile * a.layer_count * a.layer_words;
+    a.run_words += (size_t)tile * a.layer_count * a.layer_runs;
+    a.m = min(kMostRows, a.rows - tile * kMostRows);
+  }
+  const Exchange ex(a, a.words, a.words_bytes);
+  if (stage == 0) {
+    if (TILED) return normed_entry_stage(a, ex, s.sums[0], b);
+    return entry_stage<WAVES>(a, ex, s, b);
+  }
+  if (stage == 1) {
+    if (WAVES == 4 && !TILED && layer == 0) return qkv_stage<WAVES, true>(a, ex, s, layer, b);
+    return qkv_stage<WAVES, false, TILED>(a, ex, s, layer, b);
+  }
+  if (stage == 2) return attention_stage<WAVES>(a, ex, s, layer, b);
+  if (stage == 3) return combine_stage<WAVES>(a, ex, layer, b);
+  if (stage == 4) return strip_stage<WAVES, false, false>(a, ex, s, layer, b);
+  if (stage == 5) {
     if constexpr (WAVES == 8)
       if (a.parts_gate == 4) return gate_stage<WAVES, true>(a, ex, s, layer, b);
     return gate_stage<WAVES, false>(a, ex, s, layer, b);
   }
-  b -= a.n_gate;
   if constexpr (WAVES == 8)
     if (a.down_paired && layer + 1 < a.layer_count) return strip_stage<WAVES, true, true>(a, ex, s, layer, b);
   strip_stage<WAVES, true, false>(a, ex, s, layer, b);
@@ -738,7 +805,7 @@ unsigned lay_out(ChainArgs& a) {
 }
 
 bool fits(int m, int width, int heads, int kv_heads, int inner, int splits) {
-  return m >= 1 && m <= kMostRows && width > 0 && width % 64 == 0 && width <= 8192 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads * HD <= 8192 &&
+  return m >= 1 && m <= (width > 1024 ? kMostRows : kMostNarrowRows) && width > 0 && width % 64 == 0 && width <= 8192 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads * HD <= 8192 &&
          inner > 0 && inner % 64 == 0 && inner <= 65536 && splits >= 1 && splits <= 16;
 }
 
@@ -750,9 +817,10 @@ extern "C" long long nnis_chain_words(int layers, int m, int width, int heads, i
   *runs = 0;
   if (layers <= 0 || !fits(m, width, heads, kv_heads, inner, splits)) return 0;
   ChainArgs a;
-  a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits;
-  const long long words = (long long)lay_out(a) * layers + 32;
-  *runs = (long long)a.layer_runs * layers;
+  const int tiles = (m + kMostRows - 1) / kMostRows;
+  a.m = min(m, kMostRows); a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits;
+  const long long words = (long long)lay_out(a) * layers * tiles + 32;
+  *runs = (long long)a.layer_runs * layers * tiles;
   return words * 4 < (1LL << 31) && *runs * 4 < (1LL << 31) ? words : 0;
 }
 
@@ -776,17 +844,18 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
     NNIS_REQUIRE((uintptr_t)p % 16 == 0, "chain: operands must be 16-byte aligned");
   ChainArgs a;
   a.layers = (const ChainLayer*)layers; a.layer_count = layer_count;
-  a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits; a.gain_dtype = gain_dtype;
+  a.rows = m; a.tiles = (m + kMostRows - 1) / kMostRows; a.m = min(m, kMostRows);
+  a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits; a.gain_dtype = gain_dtype;
   a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f;
   a.x = x; a.x_out = x_out; a.y_out = (bf16_t*)y_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages;
-  a.max_pages = max_pages; a.words = (unsigned*)words; a.words_bytes = (unsigned)(word_count * 4);
+  a.max_pages = max_pages; a.words = (unsigned*)words; a.run_words = (unsigned*)runs;
   a.layer_words = lay_out(a);
-  a.run_words = (unsigned*)runs; a.run_bytes = (unsigned)(runs_needed * 4);
+  a.words_bytes = a.layer_words * layer_count * 4;
+  a.run_bytes = a.layer_runs * layer_count * 4;
   a.fail = a.words + (word_count - 32);
   a.host_fail = (unsigned*)host_fail;
   // wide models' units are large: 8 waves share them
   const int waves = width > 1024 ? 8 : 4;
-  a.n_entry = m;
   NNIS_REQUIRE(page_waves == 1 || page_waves == 2 || page_waves == 4 || (page_waves == 8 && waves == 8), "chain: %d waves for a run's pages", page_waves);
   a.page_waves = page_waves;
   // The ways that the layers' kernels cut K for so few rows (nnis_gemm_fused, nnis_gemm_residual), so that a step's numbers are the
@@ -805,18 +874,24 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   a.down_paired = waves == 8 && width <= 2048 && inner >= 80 * 64;
   const int units = waves == 8 ? units_of<8>() : units_of<4>();
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
-  a.n_att = m * kv_heads * ((heads / kv_heads + 3) / 4) * splits;
-  a.n_comb = splits > 1 ? (m * heads + 4 * waves - 1) / (4 * waves) : 0;
+  const int last = m - (a.tiles - 1) * kMostRows;
+  auto att = [&](int rows) { return rows * kv_heads * ((heads / kv_heads + 3) / 4) * splits; };
+  auto comb = [&](int rows) { return splits > 1 ? (rows * heads + 4 * waves - 1) / (4 * waves) : 0; };
+  a.n_att = att(a.m);
+  a.n_att_all = (a.tiles - 1) * a.n_att + att(last);
+  a.n_comb = comb(a.m);
+  a.n_comb_all = (a.tiles - 1) * a.n_comb + comb(last);
   a.n_strip = width / 16;
   a.n_out = width / 16 / (waves == 8 ? into_units_of<8, false>() : into_units_of<4, false>());
   a.n_down = width / 16 / (waves == 8 ? into_units_of<8, true>() : into_units_of<4, true>());
   a.n_gate = inner / 16 / units;
-  const long long blocks = a.n_entry + (long long)layer_count * (a.n_qkv + a.n_att + a.n_comb + a.n_out + a.n_gate + a.n_down);
+  const long long blocks = m + (long long)layer_count * (a.tiles * (a.n_qkv + a.n_out + a.n_gate + a.n_down) + a.n_att_all + a.n_comb_all);
   NNIS_REQUIRE(blocks < (1LL << 30), "chain: too many blocks");
   hipStream_t stream = (hipStream_t)stream_ptr;
   if (chain_clear(words, word_count - 32, runs, runs_needed, a.fail, stream)) return 1;
-  if (waves == 8) hipLaunchKernelGGL(chain_kernel<8>, dim3((unsigned)blocks), dim3(512), 0, stream, a);
-  else hipLaunchKernelGGL(chain_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, false>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((chain_kernel<4, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   NNIS_LAUNCH_CHECK("chain");
   return 0;
 }

@@ -705,7 +705,10 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
     runs stop at 256 blocks (32/4 heads, 22 layers, batch 1 at 700 tokens 945 and 480).  In 32 bits a wave's tiles are 16 keys: up to two
     tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and in 1 / 2 / 4 / 8 runs 900 / 723 / 623 / 590, in
     16 618; batch 8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868."""
-    if batch > CHAIN_MOST_ROWS:
+    # two tiles of rows where the layers' products are those of few rows, a tile at a time (weights of up to 8 MB)
+    two = (dtype == torch.bfloat16 and width <= 1024 and heads // kv_heads <= 4
+           and 2 * width * max(2 * inner, (heads + 2 * kv_heads) * head_dim) <= 8 << 20)
+    if batch > (2 * CHAIN_MOST_ROWS if two else CHAIN_MOST_ROWS):
         return None
     pages, runs, waves = (longest + 63) // 64, 1, 8 if dtype == torch.float32 or width > 1024 else 4
     if dtype == torch.float32:

@@ -66,6 +66,21 @@ def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
         return torch.stack(out), ran, engine
 
 
+@pytest.mark.parametrize("sizes", [(64, 1, 1, 64), (192, 6, 2, 1600), (576, 9, 3, 1536), (1024, 14, 7, 448), (1024, 16, 16, 2048)])
+def test_two_tiles_of_rows(tmp_path, sizes, monkeypatch):
+    """17 to 32 rows of narrow models: the layers' bits."""
+    import nnis_amd
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    for batch in (17, 20, 32):
+        lengths = (LENGTHS + [n + 1 for n in LENGTHS])[:batch]
+        layers, ran, _ = _run(str(tmp_path), "bfloat16", lengths, None, monkeypatch)
+        assert not ran
+        got, ran, _ = _run(str(tmp_path), "bfloat16", lengths, "own", monkeypatch)
+        assert ran and torch.equal(got, layers), batch
+    assert not _run(str(tmp_path), "bfloat16", LENGTHS * 2 + [7], "own", monkeypatch)[1]
+
+
 @pytest.mark.parametrize("batch", [1, 3, 16])
 @pytest.mark.parametrize("sizes", SIZES)
 def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
@@ -231,7 +246,7 @@ def test_sizes_and_words():
     words = ops.chain_words
     assert words(2, 1, 64, 1, 1, 64, 1)[0] > 0 and words(2, 1, 64, 1, 1, 64, 1)[1] == 0
     assert words(2, 2, 64, 1, 1, 64, 1)[0] > words(2, 1, 64, 1, 1, 64, 1)[0] and words(2, 2, 64, 1, 1, 64, 2)[1] == 2 * 2 * 2 * 68
-    for refused in ((2, 17, 64, 1, 1, 64, 1), (2, 0, 64, 1, 1, 64, 1), (2, 1, 96, 1, 1, 64, 1), (2, 1, 64, 3, 2, 64, 1), (2, 1, 64, 1, 1, 80, 1),
+    for refused in ((2, 33, 64, 1, 1, 64, 1), (2, 17, 1088, 1, 1, 64, 1), (2, 0, 64, 1, 1, 64, 1), (2, 1, 96, 1, 1, 64, 1), (2, 1, 64, 3, 2, 64, 1), (2, 1, 64, 1, 1, 80, 1),
                     (2, 1, 64, 1, 1, 64, 17), (0, 1, 64, 1, 1, 64, 1)):
         assert words(*refused)[0] == 0 and words(*refused, torch.float32)[0] == 0
     assert words(2, 1, 64, 16, 1, 64, 1, torch.float32)[0] > 0 and words(2, 1, 64, 17, 1, 64, 1, torch.float32)[0] == 0
