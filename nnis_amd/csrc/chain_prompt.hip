@@ -1,8 +1,8 @@
-// The layers of a step of one short prompt in one launch: chain.hip's stages for up to 1,024 rows that begin at a sequence's first
+// The layers of a step of short prompts in one launch: chain.hip's stages for up to 1,024 rows of sequences that begin at their first
 // position (pre-norm blocks of plain attention with heads of 64 channels and a SiLU-gated feed-forward, bfloat16).  Where it is
 // taken and what it measures there: kernels/ops.py, chain_prompt_takes.
 //
-// What bounds it is the way from stage to stage, about 3 us of five a layer (30 layers of width 576, 177 rows: 440 of 480 us), and on wide
+// What bounds it is the way from stage to stage, about 3 us of five a layer (30 layers of width 576, 177 rows: 440 of 487 us), and on wide
 // models the weights, of which a compute unit holds one block's.
 //
 // Rows are tiles of 16; a block has a unit of weight rows and 2 or 4 tiles, and 8 waves: K is cut PARTS ways, a wave has a part of K
@@ -12,7 +12,8 @@
 //
 // Words are handed on as in chain.h.  The blocks of a stage read the same words many times over, and past the caches that would be
 // tens of megabytes a stage: the first look through them finds most.  (With a look, past the caches, at a word of each piece before
-// it: 177 rows of width 576 536 us and not 482.)
+// it: 177 rows of width 576 536 us and not 482.)  Rows see their own sequence only; its one segment a tile is the usual case
+// (segments for all: 495 us and not 487).
 #include <hip/hip_runtime.h>
 
 #include "chain.h"
@@ -271,34 +272,44 @@ __device__ __forceinline__ void qkv_stage(const PromptArgs& a, const Exchange& e
   }
 }
 
-// 16 rows of a head against the keys up to their own, 32 keys a wave: scores as [key][row], whose registers are the
+// 16 rows of a head against their sequence's keys up to their own, 32 keys a wave: scores as [key][row], whose registers are the
 // probabilities' operand in the order of keys that the values have (kValues)
 template <int TILES>
 __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Exchange& ex, SharedPrompt<TILES>& s, int layer, int block) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const unsigned here = layer * a.layer_words;
-  const int head = block % a.heads, tile = block / a.heads, kv_head = head / (a.heads / a.kv_heads), pairs = tile / 2 + 1;
+  const int head = block % a.heads, tile = block / a.heads, kv_head = head / (a.heads / a.kv_heads), row = 16 * tile + r;
   const unsigned q = here + a.q + (head * 4 * a.tiles + tile) * kPiece, k = here + a.k + kv_head * 4 * a.tiles * kPiece;
   const unsigned v = here + a.v + kv_head * (a.tiles / 2) * kValues;
+  // where the row's sequence begins (padding rows, the last: one from the first of them in the tile on)
+  const bool real = row < a.m && a.tok_page[min(row, a.m - 1)] >= 0;
+  const int padding = 16 * tile + __popcll(__ballot(real) & 0xffffull);  // (by all lanes)
+  const int start = real ? row - a.tok_pos[row] : padding;
+  const int first = __builtin_amdgcn_readfirstlane(start);  // (starts do not fall from row to row)
+  const bool one = !__any(start != first);
   ex.template gate<true>(q, wave);
   f32x4 o[HD / 16];
 #pragma unroll
   for (int c = 0; c < HD / 16; ++c) o[c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   float reference = -INFINITY, sum = 0.0f;
-  for (int pair = wave; pair < pairs; pair += kWaves) {
+  for (int pair = first / 32 + wave; pair <= tile / 2; pair += kWaves) {
     u32x4 got[10];
     ex.take(got, [&](int i) {
       if (i < 2) return At{(q + g * a.tiles * kPiece + r * 8 + i * 4) * 4, 0};
       if (i < 6) return At{(k + g * a.tiles * kPiece + r * 8 + i % 2 * 4) * 4, (unsigned)((2 * pair + (i - 2) / 2) * kPiece * 4)};
       return At{(v + r * 16 + g * 4) * 4, (unsigned)(pair * kValues * 4 + (i - 6) * 1024)};
     });
+    const int key0 = 32 * pair + 4 * g;  // the lane's eight: key0 + 16 t + e
     f32x4 score[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       score[t] = mfma(__builtin_bit_cast(bf16x8, got[2 + 2 * t]), __builtin_bit_cast(bf16x8, got[0]), (f32x4){0.0f, 0.0f, 0.0f, 0.0f});
       score[t] = mfma(__builtin_bit_cast(bf16x8, got[3 + 2 * t]), __builtin_bit_cast(bf16x8, got[1]), score[t]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) score[t][e] = 32 * pair + 16 * t + 4 * g + e <= 16 * tile + r ? score[t][e] * a.scale_log2 : -INFINITY;
+      for (int e = 0; e < 4; ++e) {
+        const int key = key0 + 16 * t + e;
+        score[t][e] = key >= start && key <= row ? score[t][e] * a.scale_log2 : -INFINITY;
+      }
     }
     float top = reference;
 #pragma unroll
@@ -308,18 +319,44 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
     const float base = top == -INFINITY ? 0.0f : top, shrink = __builtin_amdgcn_exp2f(reference - base);
     reference = top;
     sum *= shrink;
-    bf16x8 p;
+    u32x4 p;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float weight = __builtin_amdgcn_exp2f(score[i / 4][i % 4] - base);
-      sum += weight;
-      p[i] = (__bf16)weight;
+    for (int i = 0; i < 8; i += 2) {
+      const float lo = __builtin_amdgcn_exp2f(score[i / 4][i % 4] - base), hi = __builtin_amdgcn_exp2f(score[i / 4][i % 4 + 1] - base);
+      sum += lo;
+      sum += hi;
+      p[i / 2] = (unsigned)__builtin_bit_cast(unsigned short, (bf16_t)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (bf16_t)hi) << 16);
     }
 #pragma unroll
-    for (int c = 0; c < HD / 16; ++c) {
-      u32x4 value = got[6 + c];
-      if (2 * pair + 1 > tile) value[2] = value[3] = 0;  // (a tile of later rows: whatever they are, no product)
-      o[c] = mfma(__builtin_bit_cast(bf16x8, value), p, o[c] * shrink);
+    for (int c = 0; c < HD / 16; ++c) o[c] *= shrink;
+    // A sequence at a time, with the values of no other and for its rows only: what a value is that a row does not see must not
+    // matter, and zero times infinity would.
+    if (one && 32 * pair >= first) {
+#pragma unroll
+      for (int c = 0; c < HD / 16; ++c) {
+        u32x4 value = got[6 + c];
+        if (2 * pair + 1 > tile) value[2] = value[3] = 0;  // (a tile of later rows)
+        o[c] = mfma(__builtin_bit_cast(bf16x8, value), __builtin_bit_cast(bf16x8, p), o[c]);
+      }
+      continue;
+    }
+    for (int from = first; from >= 0;) {
+      int next = start > from ? start : 0x7fffffff;  // the next sequence's first row
+#pragma unroll
+      for (int offset = 1; offset < 16; offset <<= 1) next = min(next, __shfl_xor(next, offset, kWave));
+      const int end = min(next, 16 * tile + 16);
+      u32x4 keep;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int key = key0 + 16 * (w / 2) + 2 * (w % 2);
+        keep[w] = (key >= from && key < end ? 0xffffu : 0u) | (key + 1 >= from && key + 1 < end ? 0xffff0000u : 0u);
+      }
+#pragma unroll
+      for (int c = 0; c < HD / 16; ++c) {
+        const f32x4 with = mfma(__builtin_bit_cast(bf16x8, got[6 + c] & keep), __builtin_bit_cast(bf16x8, p), o[c]);
+        o[c] = start == from ? with : o[c];
+      }
+      from = next < 16 * tile + 16 ? next : -1;
     }
   }
   sum += __shfl_xor(sum, 16, kWave);
@@ -333,20 +370,20 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
   __syncthreads();
   if (wave >= 4) return;
   // wave c: the head's channels 16 c ..; a lane four of them of a row
-  const int row = lane / 4, four = lane % 4;
+  const int of_row = lane / 4, four = lane % 4, pairs = tile / 2 + 1 - first / 32;
   float top = -INFINITY, den = 0.0f;
   f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int w = 0; w < kWaves; ++w)
-    if (w < pairs) top = fmaxf(top, s.attention.m[w][row]);
+    if (w < pairs) top = fmaxf(top, s.attention.m[w][of_row]);
 #pragma unroll
   for (int w = 0; w < kWaves; ++w)
     if (w < pairs) {
-      const float m = s.attention.m[w][row], weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
-      num += *(const f32x4*)&s.attention.o[w][row][16 * wave + 4 * four] * weight;
-      den = fmaf(s.attention.l[w][row], weight, den);
+      const float m = s.attention.m[w][of_row], weight = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+      num += *(const f32x4*)&s.attention.o[w][of_row][16 * wave + 4 * four] * weight;
+      den = fmaf(s.attention.l[w][of_row], weight, den);
     }
-  ex.put(here + a.attn + ((head * 4 + wave) * a.tiles + tile) * kPiece + row * 8 + four * 2, four_bf16(num * (1.0f / den)));
+  ex.put(here + a.attn + ((head * 4 + wave) * a.tiles + tile) * kPiece + of_row * 8 + four * 2, four_bf16(num * (1.0f / den)));
 }
 
 // a strip of 16 columns of the stream: the output projection or the feed-forward's down
@@ -461,8 +498,8 @@ long long lay_out(PromptArgs& a) {
 
 }  // namespace
 
-// As nnis_chain_words and nnis_chain (chain.hip), for the m rows of one prompt that begins at its sequence's first position: row i is
-// position i.  Rows with a negative page are computed and not kept.
+// As nnis_chain_words and nnis_chain (chain.hip), for the m rows of sequences that each begin at their first position and lie one
+// behind the other.  Rows with a negative page are computed and not kept; they come last.
 extern "C" long long nnis_chain_prompt_words(int layers, int m, int width, int heads, int kv_heads, int inner) {
   if (layers <= 0 || m < 1 || m > kMostPromptRows || width <= 0 || width % 64 != 0 || width > 8192 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 ||
       heads * HD > 8192 || inner <= 0 || inner % 64 != 0 || inner > 65536) return 0;

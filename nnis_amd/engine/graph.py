@@ -175,10 +175,11 @@ def prompt_rows(total: int) -> int:
 
 
 class PrefillGraph:
-    def __init__(self, engine, batch: int, total: int, wanted: int, plan_len: int, plan_new: int = 0):
+    def __init__(self, engine, batch: int, total: int, wanted: int, plan_len: int, plan_new: int = 0, fresh: bool = False):
         """``total``: the rows of the step (``prompt_rows`` of its tokens), ``batch``: its sequences,
         ``plan_len``, ``plan_new``: a longest sequence and a most tokens that one brings for which the parts plan as they do for this
-        shape."""
+        shape; ``fresh``: every sequence begins with the step (those that a plan hangs on it for do so whenever it is replayed)."""
+        self.fresh = fresh
         self.engine = engine if isinstance(engine, weakref.ProxyTypes) else weakref.proxy(engine)
         self.batch, self.total, self.plan_len, self.plan_new = batch, total, plan_len, plan_new
         # the step's arrays in one buffer, in the order the step function stages them
@@ -211,7 +212,7 @@ class PrefillGraph:
         self.ctx = StepContext(
             tokens=self.total, batch=self.batch, tok_slot=views[1], tok_pos=views[2], seq_slot=views[3], seq_start=views[4],
             seq_pos0=views[5], decode=False, max_new=self.total, max_len=self.plan_len, host_new=None, host_pos0=None,
-            plan_len=self.plan_len, plan_rows=self.total, plan_new=self.plan_new, lists=self.lists)
+            plan_len=self.plan_len, plan_rows=self.total, plan_new=self.plan_new, fresh=self.fresh, lists=self.lists)
 
     def fill(self, arrays, counts: Sequence[int], first_positions: Sequence[int]) -> None:
         """The step's data into the buffers: ``arrays`` as the step function stages them (ids, slot and position
@@ -306,7 +307,7 @@ class PrefillGraphs:
         if times < 2:
             return None
         batch, total, wanted, _ = key
-        graph = PrefillGraph(self.engine, batch, total, wanted, longest, max(counts))
+        graph = PrefillGraph(self.engine, batch, total, wanted, longest, max(counts), not any(first_positions))
         logits = graph.first_run(arrays, counts, first_positions)
         if graph.graph is None:
             self.refused.add(key)

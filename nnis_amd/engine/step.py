@@ -181,11 +181,11 @@ class Engine:
 
     def _run_prompts(self, entries, counts, pos0, total, want_rows, arrays) -> torch.Tensor:
         longest = max(p + n for p, n in zip(pos0, counts))
-        rows = prompt_rows(total)
+        rows, fresh = prompt_rows(total), not any(pos0)
         if (self.use_graphs and total <= PREFILL_GRAPH_MOST_TOKENS and want_rows
                 and total * float(self.model.spec.width) ** 2 <= PREFILL_GRAPH_MOST_WORK):
             # a shape that comes again is replayed from a graph (engine/graph.py)
-            shape = (len(counts), rows, len(want_rows), self.model.prompt_plan(len(counts), rows, longest, self.rt, max(counts)))
+            shape = (len(counts), rows, len(want_rows), self.model.prompt_plan(len(counts), rows, longest, self.rt, max(counts), fresh))
             if self._prefill_graphs is None:
                 self._prefill_graphs = PrefillGraphs(self)
             done = self._prefill_graphs.step(shape, arrays, counts, pos0, longest)
@@ -208,6 +208,7 @@ class Engine:
             host_new=counts,
             host_pos0=pos0,
             plan_rows=rows,
+            fresh=fresh,
         )
         return self.model.forward(dev[0], ctx, self.cache, dev[6], self.rt)
 

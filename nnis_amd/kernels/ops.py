@@ -755,10 +755,10 @@ def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables,
 
 
 def chain_prompt_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16) -> bool:
-    """Whether ``chain_prompt`` is to run a prompt of ``rows`` rows: up to 1,024 (192 above a width of 1,024, where a block has the unit's
+    """Whether ``chain_prompt`` is to run prompts of ``rows`` rows in all: up to 1,024 (192 above a width of 1,024, where a block has the unit's
     weights for fewer rows), an exchange of up to 512 MB, and up to rows x a layer's weights of 5.7e9, beyond which the blocks' reading
     of weights costs more than the layers' tiled products.  Whole steps in microseconds by the layers' kernels and in one launch, rows x
-    weights in 1e9: width 576, 9/3 heads, 30 layers, 177 rows (0.6) 940 and 483, 1,000 (3.5) 1,627 and 1,232; 768, 12/12, 12 layers, 500
+    weights in 1e9: width 576, 9/3 heads, 30 layers, 177 rows (0.6) 940 and 487, 1,000 (3.5) 1,627 and 1,232, six prompts of 570 rows 1,321 and 740; 768, 12/12, 12 layers, 500
     (3.6) 598 and 427, 768 (5.5) 673 and 609, 1,000 (7.1) 761 and 835; 1,024, 16/16, 12 layers, 320 (5.4) 723 and 570, 500 (8.4) 851 and
     873; 1,280, 20/4, 16 layers, 192 (3.3) 900 and 649, 320 (5.4) 1,005 and 1,037; 2,048, 32/4, 22 layers, 60 rows as 64 (2.8) 1,220 and 835,
     128 (5.6) 1,519 and 1,173, 190 as 192 (8.5) 1,695 and 1,669; 2,048, 32/32, 24 layers, 64 (4.3) 1,479 and 1,246, 128 (8.6) 1,793 and
@@ -770,7 +770,7 @@ def chain_prompt_takes(layers: int, rows: int, width: int, heads: int, kv_heads:
 
 def chain_prompt(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, failed: torch.Tensor, gain_dtype: torch.dtype,
                  eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
-    """As ``chain``, for the rows of one prompt that begins at its sequence's first position: row i is position i."""
+    """As ``chain``, for the rows of prompts that each begin at their sequence's first position, one behind the other."""
     for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page")):
         _dev(t, f"chain_prompt {what}")
     rows = x.shape[0]

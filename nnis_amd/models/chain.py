@@ -1,4 +1,4 @@
-"""A step of few single tokens, or of one short prompt, through all layers in one launch (``csrc/chain.hip``, ``chain_prompt.hip``).
+"""A step of few single tokens, or of short prompts, through all layers in one launch (``csrc/chain.hip``, ``chain_prompt.hip``).
 
 A part that the launch takes says what of it there is (``chain_link``); a model whose every layer does, over one cache and one
 rotation, runs such steps through it, and all others -- other mixers, options, types, sizes, more rows, longer sequences --
@@ -49,10 +49,9 @@ class LayerChain:
         """(runs of a sequence's keys, waves of a run) for a step of these sizes, or None: the layers' own kernels."""
         return rt.ops.chain_plan(len(self.links), batch, longest, **self.sizes)
 
-    def takes_prompt(self, batch: int, rows: int, longest: int, most_new: int, rt) -> bool:
-        """Whether a step of ``batch`` sequences, the longest of ``longest`` tokens after it and ``most_new`` of them new, is one
-        short prompt from its sequence's first position on."""
-        return batch == 1 and longest == most_new and rt.ops.chain_prompt_takes(len(self.links), rows, **self.sizes)
+    def takes_prompt(self, rows: int, rt) -> bool:
+        """Whether the launch takes a step of prompts of this many rows in all that each begin at their sequence's first position."""
+        return rt.ops.chain_prompt_takes(len(self.links), rows, **self.sizes)
 
     def check(self) -> None:
         """Raises if a wait of an earlier step was given up."""

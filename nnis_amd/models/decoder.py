@@ -5,7 +5,7 @@ architecture; which parts exist and how they are sized is the spec's business.
 
 from __future__ import annotations
 
-from typing import Any, Dict, List, Tuple
+from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
@@ -102,11 +102,13 @@ class DecoderModel:
         if chain is not None:
             chain.check()
 
-    def prompt_plan(self, batch: int, rows: int, longest: int, rt, most_new: int = 0):
+    def prompt_plan(self, batch: int, rows: int, longest: int, rt, most_new: int = 0, fresh: Optional[bool] = None):
         """The plans of every run of the schedule for a step of prompts (``Part.prompt_plan``, ``Part.run_plan``);
-        ``most_new``: the most tokens that a sequence brings (0: all rows of a step of one, their mean of several)."""
+        ``most_new``: the most tokens that a sequence brings (0: all rows of a step of one, their mean of several); ``fresh``: whether
+        every sequence begins with the step (None: what can be said of one)."""
         most_new = most_new or -(-rows // max(batch, 1))
-        key = (batch, rows, longest, most_new)
+        fresh = batch == 1 and longest == most_new if fresh is None else fresh
+        key = (batch, rows, longest, most_new, fresh)
         plans = self._prompt_plans.get(key)
         if plans is None:
             if len(self._prompt_plans) > 4096:
@@ -115,7 +117,7 @@ class DecoderModel:
                 plan for layer in (self.layers[entry.layer] for entry in self.spec.schedule)
                 for plan in (layer.prompt_plan(batch, rows, longest, rt), layer.run_plan(batch, rows, most_new, rt)))
             chain = self.layer_chain(rt)
-            if chain is not None and chain.takes_prompt(batch, rows, longest, most_new, rt):
+            if chain is not None and fresh and chain.takes_prompt(rows, rt):
                 plans = self._prompt_plans[key] = plans + (("chain", "prompt"),)
         return plans
 
@@ -164,7 +166,7 @@ class DecoderModel:
         elif ctx.decode:
             plan = chain.plan(ctx.batch, ctx.planned_len, rt)
         else:
-            plan = "prompt" if chain.takes_prompt(ctx.batch, ctx.planned_rows, ctx.planned_len, ctx.planned_new, rt) else None
+            plan = "prompt" if ctx.fresh and chain.takes_prompt(ctx.planned_rows, rt) else None
         if plan is None or x.dim() != 2 or x.dtype != torch.float32 or not x.is_contiguous():
             return stream, schedule
         views = [cache.view(index) for index in range(len(schedule))]

@@ -47,6 +47,7 @@ def _run(folder, dtype, lengths, plan, monkeypatch, steps=3):
     from nnis_amd.kernels import ops
 
     with monkeypatch.context() as patch:
+        patch.setattr(ops, "chain_prompt_takes", lambda *args, **sizes: False)  # (the same cache for all)
         if plan != "own":
             patch.setattr(ops, "chain_plan", lambda *args, **sizes: plan)
         engine = load_engine(folder, dtype=dtype, max_tokens=sum(-(-(n + steps + 1) // 64) * 64 for n in lengths))
@@ -128,10 +129,10 @@ def test_32_bits_against_the_oracle(tmp_path, sizes, batch, monkeypatch):
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 64 bits, the layers' kernels {(layers - want).norm().item():.4g}"
 
 
-@pytest.mark.parametrize("rows", [2, 16, 33, 177, 600])
+@pytest.mark.parametrize("counts", [(2,), (16,), (33,), (177,), (600,), (1, 1, 15, 16, 1, 30, 33), (100, 3, 260, 2), (9,) * 20])
 @pytest.mark.parametrize("sizes", SIZES + [(1088, 8, 8, 4160)])  # (eight waves with a second round of down's weights)
-def test_a_prompt_against_the_layers(tmp_path, sizes, rows, monkeypatch):
-    """As far from 32 bits as the layers' kernels, the prompt's last row and the steps behind it (by the layers' kernels, from what
+def test_prompts_against_the_layers(tmp_path, sizes, counts, monkeypatch):
+    """As far from 32 bits as the layers' kernels, some rows of each prompt and the steps behind them (by the layers' kernels, from what
     the launch left in the cache); launched and replayed the same bits.  (The roundings are the same, the orders of the sums are not.)"""
     import nnis_amd
     from nnis_amd.api import load_engine
@@ -139,9 +140,9 @@ def test_a_prompt_against_the_layers(tmp_path, sizes, rows, monkeypatch):
     from nnis_amd.kernels import ops
 
     nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
-    rng = np.random.default_rng(rows)
-    prompt, tokens = rng.integers(0, 509, size=rows).tolist(), rng.integers(0, 509, size=2).tolist()
-    places = sorted({0, rows // 3, rows - 1})
+    rng = np.random.default_rng(sum(counts))
+    prompts, tokens = [rng.integers(0, 509, size=n).tolist() for n in counts], rng.integers(0, 509, size=2).tolist()
+    places = [sorted({0, n // 3, n - 1}) for n in counts]
 
     def run(dtype, takes):
         with monkeypatch.context() as patch:
@@ -151,13 +152,14 @@ def test_a_prompt_against_the_layers(tmp_path, sizes, rows, monkeypatch):
             if takes is not None:
                 patch.setattr(ops, "chain_prompt_takes", lambda *args, **more: takes)
             patch.setattr(ops, "chain_plan", lambda *args, **more: None)
-            engine = load_engine(str(tmp_path), dtype=dtype, max_tokens=1024)
-            slot, out = engine.start_sequence(), None
+            engine = load_engine(str(tmp_path), dtype=dtype, max_tokens=2048)
+            slots, out = [engine.start_sequence() for _ in counts], None
             for again in range(4):  # launched, launched and captured, replayed
-                engine.truncate(slot, 0)
-                got = [engine.step([StepEntry(slot, prompt, places)]).double().cpu()]
+                for slot in slots:
+                    engine.truncate(slot, 0)
+                got = [engine.step([StepEntry(*entry) for entry in zip(slots, prompts, places)]).double().cpu()]
                 for token in tokens:
-                    got.append(engine.step([StepEntry(slot, [token], None)]).double().cpu())
+                    got.append(engine.step([StepEntry(slot, [token], None) for slot in slots]).double().cpu())
                 got = torch.cat(got)
                 assert dtype == "float32" or not launches or out is None or torch.equal(out, got)
                 out = got
@@ -173,8 +175,8 @@ def test_a_prompt_against_the_layers(tmp_path, sizes, rows, monkeypatch):
 
 
 def test_prompts_that_are_not_taken(tmp_path, monkeypatch):
-    """A prompt behind cached tokens, two prompts in a step, one beyond the rows: the layers' kernels, also where a prompt of the same
-    rows has been captured."""
+    """A prompt behind cached tokens, also beside one that begins, and one beyond the rows: the layers' kernels, also where a prompt of
+    the same rows has been captured."""
     import nnis_amd
     from nnis_amd.api import load_engine
     from nnis_amd.engine.batch import StepEntry
@@ -204,10 +206,36 @@ def test_prompts_that_are_not_taken(tmp_path, monkeypatch):
         got, want = engine.step([StepEntry(slot, second, None)]), plain.step([StepEntry(other, second, None)])
         assert (got.double() - want.double()).norm() <= 0.05 * want.double().norm()  # (a few bfloat16 roundings of 2^-9 over two layers)
     assert len(launches) == taken
-    slots = [engine.start_sequence() for _ in range(2)]
-    engine.step([StepEntry(s, first, None) for s in slots])
+    engine.truncate(slot, 7)
+    engine.step([StepEntry(engine.start_sequence(), first, None), StepEntry(slot, first, None)])
     engine.step([StepEntry(engine.start_sequence(), rng.integers(0, 509, size=1100).tolist(), None)])
     assert len(launches) == taken
+
+
+def test_prompts_in_a_step_do_not_meet(tmp_path):
+    """What a sequence holds that is not finite stays its own: the others' logits are the same bits as beside finite ones."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+
+    nnis_amd.write_random_model(str(tmp_path), dict(_config(192, 6, 2, 1600), tie_word_embeddings=False), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=2048)
+    rng = np.random.default_rng(7)
+    prompts = [rng.integers(8, 509, size=n).tolist() for n in (5, 20, 3, 40, 17)]
+    prompts[1][9] = prompts[3][0] = 7
+    slots = [engine.start_sequence() for _ in prompts]
+
+    def step():
+        for slot in slots:
+            engine.truncate(slot, 0)
+        return engine.step([StepEntry(slot, prompt, None) for slot, prompt in zip(slots, prompts)])
+
+    finite = step()
+    table = engine.model.embedding.table
+    table[7] = float("inf")
+    for _ in range(3):
+        got = step()
+        assert torch.equal(got[[0, 2, 4]], finite[[0, 2, 4]]) and not bool(torch.isfinite(got[[1, 3]]).any())
 
 
 def test_not_taken(tmp_path, monkeypatch):
