@@ -43,10 +43,11 @@ struct At {
 struct Exchange {
   __amdgpu_buffer_rsrc_t r;
   unsigned *fail, *host_fail;
+  bool near;
 
   template <typename Args>
-  __device__ __forceinline__ Exchange(const Args& a, unsigned* words, unsigned bytes)
-      : r(__builtin_amdgcn_make_buffer_rsrc(words, 0, bytes, 0x00020000)), fail(a.fail), host_fail(a.host_fail) {}
+  __device__ __forceinline__ Exchange(const Args& a, unsigned* words, unsigned bytes, bool near_ = true)
+      : r(__builtin_amdgcn_make_buffer_rsrc(words, 0, bytes, 0x00020000)), fail(a.fail), host_fail(a.host_fail), near(near_) {}
 
   // whether a wait is to be left: every 256th look, by the clock and by what others found
   __device__ __forceinline__ bool leave(int& looks, long long& since) const {
@@ -111,11 +112,10 @@ struct Exchange {
   // ... until all of them are there.  The first look goes through the caches, which may have them from a neighbour's: a word is
   // written once in a launch, so a cached one is what was written or still none; a line that was fetched half written stays
   // so, and all further looks go past them.  (16 rows of 32 heads and a width of 2,048 1,405 us and 1,259, 8 rows 1,147 and 1,112; a
-  // prompt of 177 rows of width 576, with nothing through the caches 552 and 482; few rows of narrow models alike, whose products
-  // leave it out, NEAR: with it they spill.)
-  template <bool NEAR = true, int N, typename... Rest>
+  // prompt of 177 rows of width 576, with nothing through the caches 552 and 482.  `near`: few rows of narrow models leave it out.)
+  template <int N, typename... Rest>
   __device__ __forceinline__ void take(u32x4 (&v)[N], Rest&&... rest) const {
-    if (NEAR && look<0>(v, rest...)) return;
+    if (near && look<0>(v, rest...)) return;
     int looks = 0;
     long long since = 0;
     while (!look<kPastCaches>(v, rest...) && !leave(looks, since)) {}

@@ -1,7 +1,7 @@
 // The layers of a step of few single tokens in one launch (pre-norm blocks of plain attention with heads of 64 channels and a
 // SiLU-gated feed-forward, bfloat16, up to 16 rows; up to a width of 1,024 32, as two tiles of rows that have nothing to do with
-// one another: 24 rows of 30 layers of width 576 1,037 us by the layers' kernels and 805, 32 rows 968 and 704, but 48 rows of 600 to 2,000
-// tokens 1,153 and 1,380).
+// one another: 24 rows of 30 layers of width 576 1,037 us by the layers' kernels and 772, 32 rows 968 and 660, but 48 rows of 600 to 2,000
+// tokens 1,153 and 1,380 when last measured).
 //
 // What bounds such a step is neither bytes nor products but its chain of dependent kernels, five to six a layer: each begins
 // 1.6 us after the one before has ended, asks for its weights, and only then has something to multiply.  Here a layer's stages
@@ -73,7 +73,6 @@ __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builti
 template <int WAVES, int STRIPS, int STEPS, int XB, int V, bool NEXT = false>
 struct Product {
   static_assert(STEPS % XB == 0 && STEPS % V == 0, "whole trips");
-  static constexpr bool kNear = WAVES == 8 || STEPS == 8;  // (Exchange::take; wide models')
   bf16x8 w[STEPS][2][STRIPS];
   f32x4 acc[V][STRIPS];
   const bf16_t* strip[STRIPS];
@@ -124,8 +123,8 @@ struct Product {
         unsigned part[XB];
         auto step = [&](int d) { return (unsigned)min(chunk(d0, b + d), chunks - 1) * 4 * stride; };
         auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
-        if constexpr (SUM) ex.template take<kNear>(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
-        else ex.template take<kNear>(v, pieces);
+        if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
+        else ex.take(v, pieces);
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
           const int c = chunk(d0, b + d);
@@ -721,9 +720,11 @@ __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& e
   ex.put(here + a.act + (unit * a.m + row) * 8 + 2 * g, (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
 }
 
-// TILED: more than 16 rows (beside its arithmetic steps of up to 16 are half a per cent slower)
-template <int WAVES, bool TILED>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? 3 : 2))) void chain_kernel(ChainArgs a) {
+// TILED: more than 16 rows (beside its arithmetic steps of up to 16 are half a per cent slower).  NEAR: the first look through the caches
+// (Exchange::take): it needs registers that fewer than five rows lose more by than they gain (four waves, of 30 layers of width 576, without
+// and with it: 1 row 387 and 391 us, 4 458 and 462, 8 491 and 480, 16 566 and 550, 17 643 and 603).
+template <int WAVES, bool TILED, bool NEAR>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 && (TILED || !NEAR) ? 3 : 2))) void chain_kernel(ChainArgs a) {
   __shared__ Shared<WAVES> s;
   int b = blockIdx.x, layer = -1, stage = -1, tile = 0;
   auto in = [&](int index, int blocks, int all) {  // the stage with this index has `blocks` for a tile
@@ -763,7 +764,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     a.run_words += (size_t)tile * a.layer_count * a.layer_runs;
     a.m = min(kMostRows, a.rows - tile * kMostRows);
   }
-  const Exchange ex(a, a.words, a.words_bytes);
+  const Exchange ex(a, a.words, a.words_bytes, NEAR);
   if (stage == 0) {
     if (TILED) return normed_entry_stage(a, ex, s.sums[0], b);
     return entry_stage<WAVES>(a, ex, s, b);
@@ -889,9 +890,10 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   NNIS_REQUIRE(blocks < (1LL << 30), "chain: too many blocks");
   hipStream_t stream = (hipStream_t)stream_ptr;
   if (chain_clear(words, word_count - 32, runs, runs_needed, a.fail, stream)) return 1;
-  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, false>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
-  else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((chain_kernel<4, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  else if (m <= 4) hipLaunchKernelGGL((chain_kernel<4, false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((chain_kernel<4, true, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   NNIS_LAUNCH_CHECK("chain");
   return 0;
 }
