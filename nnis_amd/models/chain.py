@@ -80,6 +80,7 @@ class LayerChain:
 
     def forward(self, x: torch.Tensor, ctx, views, plan, rt):
         """The stream, and what the last layer still adds to it; None where the launch cannot be made here."""
+        self.check()
         table = self._table(views, x.device)
         if table is None:
             return None

@@ -265,6 +265,11 @@ def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
         engine.step([StepEntry(slot, [7], None)])
     assert engine.length(slot) == length
     assert bool(torch.isfinite(engine.step([StepEntry(slot, [7], None)])).all())
+    engine.use_graphs = False  # launched, not replayed
+    engine.model.layer_chain(engine.rt).failed[0] = 1
+    with pytest.raises(KernelError, match="gave up waiting"):
+        engine.step([StepEntry(slot, [7], None)])
+    assert engine.length(slot) == length + 1
 
 
 def test_sizes_and_words():
