@@ -870,9 +870,10 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   a.parts_qkv = cut(width, 4, 0, waves);
   a.parts_out = cut(heads * HD, 4, 0, waves);
   a.parts_gate = cut(width, 4, inner / 8, waves);
-  if (waves == 8 && a.parts_gate < 4) a.parts_gate = 8;  // (not the layers' bits there)
+  const bool alike = heads / kv_heads <= 4;  // (larger groups' scores are other bits in any case)
+  if (waves == 8 && (a.parts_gate < 4 || !alike)) a.parts_gate = 8;  // (not the layers' bits there)
   a.parts_down = cut(inner, 4, 0, 8);
-  a.down_paired = waves == 8 && width <= 2048 && inner >= 80 * 64;
+  a.down_paired = waves == 8 && alike && width <= 2048 && inner >= 80 * 64;
   const int units = waves == 8 ? units_of<8>() : units_of<4>();
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
   const int last = m - (a.tiles - 1) * kMostRows;

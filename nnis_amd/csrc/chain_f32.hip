@@ -467,7 +467,7 @@ __device__ __forceinline__ void gate_stage(const ChainArgs32& a, const Exchange&
 template <bool WIDE>
 __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 3))) void chain_f32_kernel(ChainArgs32 a) {
   __shared__ Shared32 s;
-  const Exchange ex(a, a.words, a.words_bytes);
+  const Exchange ex(a, a.words, a.words_bytes, !WIDE);  // (22 layers of width 2,048, 8 rows: 1,427 us and 1,435 with the look through the caches)
   int b = blockIdx.x;
   if (b < a.n_entry) return entry_stage(a, ex, b);
   b -= a.n_entry;

@@ -702,7 +702,7 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
 
     Larger groups have the scores of four heads a wave here and of sixteen there, so other bits, and a seeded draw over other bits picks
     other tokens: the launch is theirs up to seven rows.  A wave has one page where the blocks are few, two where they are more, and the
-    runs stop at 256 blocks (32/4 heads, 22 layers, batch 1 at 700 tokens 945 and 480).  In 32 bits a wave's tiles are 16 keys: up to two
+    runs stop at 256 blocks (32/4 heads, 22 layers, batch 1 at 700 tokens 943 and 508, batch 4 at 1,500 998 and 546).  In 32 bits a wave's tiles are 16 keys: up to two
     tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and in 1 / 2 / 4 / 8 runs 900 / 723 / 623 / 590, in
     16 618; batch 8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868."""
     # two tiles of rows where the layers' products are those of few rows, a tile at a time (weights of up to 8 MB)
