@@ -55,6 +55,7 @@ _CORE_SIGNATURES = {
                             _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
     "nnis_gemm_f32": [_VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_ordered": [_VOID, _INT, _VOID, _INT, _VOID, _INT, _INT, _INT, _INT, _VOID],
+    "nnis_gemm_two": [_VOID, _VOID, _VOID, _INT, _VOID, _INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_bf16": [_VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _INT, _VOID, _SIZE, _VOID],
     "nnis_gemm_fused": [_VOID, _VOID, _VOID, _VOID, _INT, _FLT, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT,
                         _VOID, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
@@ -1137,6 +1138,22 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, split: int = 
     _check(lib, lib.nnis_gemm_bf16(x.data_ptr(), w.data_ptr(), out.data_ptr(), _code(out), m, n, k, int(split), _ptr(work),
                                    GEMM_WORKSPACE_BYTES if work is not None else 0, _stream()))
     return out
+
+
+def gemm_two(x: torch.Tensor, w: "PackedWeight", out: torch.Tensor, second: torch.Tensor):
+    """``gemm_bf16`` of up to 16 rows by two weights in one launch: ``w`` holds the first's rows, a multiple of 16, and the second's
+    behind them; ``out``: bfloat16, ``second``: bfloat16 or float32."""
+    _packed(w, "gemm_two")
+    _dev(x, "x"), _dev(out, "out"), _dev(second, "second")
+    m, k = x.shape
+    n, columns = w.shape[0], out.shape[1]
+    if w.shape[1] != k or out.shape[0] != m or second.shape != (m, n - columns) or not (out.is_contiguous() and second.is_contiguous()):
+        raise KernelError(f"gemm_two: x {tuple(x.shape)} w {tuple(w.shape)} out {tuple(out.shape)} and {tuple(second.shape)} do not fit")
+    if x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or not x.is_contiguous():
+        raise KernelError(f"gemm_two takes bfloat16 rows one behind the other and gives the first product in bfloat16, got {x.dtype} and {out.dtype}")
+    lib = core()
+    _check(lib, lib.nnis_gemm_two(x.data_ptr(), w.data_ptr(), out.data_ptr(), columns, second.data_ptr(), _code(second), m, n, k, _stream()))
+    return out, second
 
 
 EPILOGUE_STORE, EPILOGUE_SILU, EPILOGUE_ROPE = 0, 1, 2

@@ -51,3 +51,33 @@ class Projection:
         if x.can_fuse(self.weight):
             return x.fused(self.weight, rt.empty(x.rows, self.out_features), rt.ops.EPILOGUE_STORE)
         return self(x.materialize(), rt)
+
+
+class ProjectionPair:
+    """Two projections of the same rows, whose packed weights lie one behind the other: few rows take both in one launch, with the
+    same results."""
+
+    MOST_ROWS = 16
+
+    def __init__(self, first: torch.Tensor, second: torch.Tensor, rt):
+        self.first, self.second = Projection(first, rt), Projection(second, rt)
+        self.joined = None
+        if rt is None or rt.dtype != torch.bfloat16:
+            return
+        kind, parts = rt.ops.PackedWeight, (self.first.weight, self.second.weight)
+        rows = self.first.out_features, self.second.out_features
+        if all(isinstance(part, kind) for part in parts) and rows[0] % 16 == 0 and sum(rows) < 2048 * 16:
+            data = torch.cat([part.data for part in parts])
+            self.joined = kind(data, sum(rows), first.shape[1])
+            cut = parts[0].data.numel()
+            self.first.weight, self.second.weight = kind(data[:cut], *first.shape), kind(data[cut:], *second.shape)
+
+    def weight_bytes(self) -> int:
+        return self.first.weight_bytes() + self.second.weight_bytes()
+
+    def __call__(self, x: torch.Tensor, rt, second_dtype: Optional[torch.dtype] = None):
+        rows = x.shape[0]
+        if self.joined is None or not 0 < rows <= self.MOST_ROWS or not x.is_contiguous() or x.data_ptr() % 16:
+            return self.first(x, rt), self.second(x, rt, out_dtype=second_dtype)
+        return rt.ops.gemm_two(x, self.joined, rt.empty(rows, self.first.out_features),
+                               rt.empty(rows, self.second.out_features, dtype=second_dtype or rt.dtype))

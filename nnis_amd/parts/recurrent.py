@@ -17,7 +17,7 @@ import torch
 from ..errors import InvalidInput, Unsupported
 from ..weights.random_init import register_init_rule
 from .base import Mixer, StateRequest, TensorSpec, register_part
-from .linear import Projection
+from .linear import Projection, ProjectionPair
 
 
 class SelectiveScan(Mixer):
@@ -65,9 +65,8 @@ class SelectiveScan(Mixer):
         self.w_in = Projection(weights[n["w_in"]], rt)
         self.conv = weights[n["conv"]].contiguous()
         self.conv_bias = weights[n["conv_bias"]].contiguous()
-        # the low-rank step sizes and the read/write vectors leave separate projections: each output is then a matrix of its own
-        self.w_dt_low = Projection(weights[n["w_x"]][:R].contiguous(), rt)
-        self.w_bc = Projection(weights[n["w_x"]][R:].contiguous(), rt)
+        # the low-rank step sizes and the read/write vectors: each output is a matrix of its own
+        self.w_x = ProjectionPair(weights[n["w_x"]][:R].contiguous(), weights[n["w_x"]][R:].contiguous(), rt)
         self.w_dt = Projection(weights[n["w_dt"]], rt)
         self.dt_bias = weights[n["dt_bias"]].float().contiguous()
         self.A = (-torch.exp(weights[n["a_log"]].float())).contiguous()  # the rates, 32-bit, made once
@@ -76,7 +75,7 @@ class SelectiveScan(Mixer):
 
     def weight_bytes(self):
         small = sum(t.numel() * t.element_size() for t in (self.conv, self.conv_bias, self.dt_bias, self.A, self.D))
-        return small + sum(p.weight_bytes() for p in (self.w_in, self.w_dt_low, self.w_bc, self.w_dt, self.w_out))
+        return small + sum(p.weight_bytes() for p in (self.w_in, self.w_x, self.w_dt, self.w_out))
 
     def cache_request(self):
         return (StateRequest((self.channels, self.states)), StateRequest((self.taps - 1, self.channels)))
@@ -88,9 +87,8 @@ class SelectiveScan(Mixer):
         tokens, C = x.shape[0], self.channels
         xz = self.w_in(x, rt)
         xc = rt.ops.conv_silu(xz, C, self.conv, self.conv_bias, conv_state.state if self.taps > 1 else None, ctx, rt.empty(tokens, C))
-        low = self.w_dt_low(xc, rt)
+        low, bc = self.w_x(xc, rt, second_dtype=torch.float32)
         dt_pre = self.w_dt(low, rt, out_dtype=torch.float32)
-        bc = self.w_bc(xc, rt, out_dtype=torch.float32)
         y = rt.ops.selective_scan(xc, dt_pre, bc, xz[:, C:], self.A, self.D, self.dt_bias, scan_state.state, ctx, rt.empty(tokens, C))
         return self.w_out(y, rt)
 
@@ -137,17 +135,16 @@ class GatedLinearAttention(Mixer):
     def bind(self, weights, rt):
         n = self.names
         # queries, keys, values and gates leave one projection; their columns are read in place
-        self.qkvg = Projection(torch.cat([weights[n[key]] for key in ("q", "k", "v", "g")], dim=0), rt)
         if weights[n["a1"]].shape[0] != weights[n["a2"]].shape[1]:
             raise InvalidInput(f"{n['a1']} and {n['a2']} do not meet: {tuple(weights[n['a1']].shape)} and {tuple(weights[n['a2']].shape)}")
-        self.a1 = Projection(weights[n["a1"]], rt)
+        self.qkvg_a1 = ProjectionPair(torch.cat([weights[n[key]] for key in ("q", "k", "v", "g")], dim=0), weights[n["a1"]], rt)
         self.a2 = Projection(weights[n["a2"]], rt)
         self.a2_bias = weights[n["a2_bias"]].float().contiguous()
         self.norm = weights[n["norm"]].contiguous()
         self.out = Projection(weights[n["o"]], rt)
 
     def weight_bytes(self):
-        return (sum(p.weight_bytes() for p in (self.qkvg, self.a1, self.a2, self.out))
+        return (sum(p.weight_bytes() for p in (self.qkvg_a1, self.a2, self.out))
                 + self.a2_bias.numel() * 4 + self.norm.numel() * self.norm.element_size())
 
     def cache_request(self):
@@ -158,8 +155,8 @@ class GatedLinearAttention(Mixer):
             raise Unsupported("gated linear attention cannot read another layer's state")
         H, d, e = self.heads, self.key_dim, self.value_dim
         tokens = x.shape[0]
-        qkvg = self.qkvg(x, rt)
-        logits = self.a2(self.a1(x, rt), rt, out_dtype=torch.float32)
+        qkvg, low = self.qkvg_a1(x, rt)
+        logits = self.a2(low, rt, out_dtype=torch.float32)
         rt.ops.gla_decays(logits, self.a2_bias, self.tau)  # the decays' logarithms, once for all heads' blocks
         q, k = qkvg[:, :H * d], qkvg[:, H * d:2 * H * d]
         v, g = qkvg[:, 2 * H * d:2 * H * d + H * e], qkvg[:, 2 * H * d + H * e:]

@@ -1114,6 +1114,27 @@ def test_silu_mul(dtype):
     assert ((out.cpu().double() - want).abs() <= (1e-6 if dtype == "float32" else 1e-2) * (1 + want.abs())).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("columns, rest, k", [(16, 1, 8), (16, 16, 64), (128, 32, 4096), (48, 33, 200), (3072, 8, 2048)])
+def test_two_products_in_one_launch(columns, rest, k, dtype):
+    """The same numbers as apart."""
+    from nnis_amd.parts.linear import ProjectionPair
+    from nnis_amd.engine.runtime import Runtime
+
+    rt = Runtime(dtype="bfloat16")
+    torch.manual_seed(columns + k)
+    weights = [torch.randn(n, k, device="cuda").bfloat16() for n in (columns, rest)]
+    pair = ProjectionPair(*weights, rt)
+    assert pair.joined is not None
+    for rows in (1, 4, 16, 17):
+        x = torch.randn(rows, k, device="cuda").bfloat16()
+        first, second = pair(x, rt, second_dtype=dtype)
+        assert torch.equal(first, pair.first(x, rt)) and torch.equal(second, pair.second(x, rt, out_dtype=dtype))
+        assert torch.allclose(second.float(), x.float() @ weights[1].float().t(), rtol=0.02, atol=0.02 * k ** 0.5)  # (2^-8 of a result and more)
+    with pytest.raises(KernelError):
+        rt.ops.gemm_two(x, pair.joined, first, second)  # 17 rows
+
+
 @pytest.mark.parametrize("vocab", [1, 63, 1000, 49152, 50001])
 def test_argmax(vocab):
     ops = _ops()
