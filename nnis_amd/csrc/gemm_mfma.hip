@@ -41,22 +41,6 @@ constexpr size_t kStreamWeightBytes = 16u << 20;
 __device__ __forceinline__ bf16x8 load_stream(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
 
 // -----------------------------------------------------------------------------
-// Where a product of two weights on the same rows goes, one behind the other in whole strips: the first's columns, then the second's.
-struct TwoOut {
-  bf16_t* first;  // [m, columns]
-  int columns;
-  void* second;   // [m, n - columns]
-  int second_f32;
-  int n;
-};
-__device__ __forceinline__ void store4(const TwoOut& y, size_t index, f32x4 v, int valid, bool) {
-  const size_t token = index / y.n;
-  const int column = (int)(index - token * y.n), rest = y.n - y.columns;
-  if (column < y.columns) store4(y.first, token * y.columns + column, v, valid, true);
-  else if (y.second_f32) store4((float*)y.second, token * rest + column - y.columns, v, valid, rest % 4 == 0);
-  else store4((bf16_t*)y.second, token * rest + column - y.columns, v, valid, rest % 4 == 0);
-}
-
 // skinny: MT token tiles of 16 (M <= 16 * MT); KSPLIT waves share one strip's K.
 // A decode-sized product is bound by memory latency, not bandwidth: a wave
 // issues the loads of DEPTH steps of 64 k (weights and activations) before the
@@ -1347,22 +1331,6 @@ extern "C" int nnis_gemm_bf16(const void* x, const void* w, void* y, int y_dtype
     else dispatch_tiled<bf16_t*>(xp, wp, (bf16_t*)y, m, n, k, tile_hint, ws, stream);
     NNIS_LAUNCH_CHECK("gemm_tiled");
   }
-  return 0;
-}
-
-// Two products of up to 16 rows in one launch: w [n, k] is two packed weights, the first of `columns` rows (whole strips), whose product goes to
-// y in bfloat16, the other's to second in second_dtype.  The same numbers as apart: a strip's K is cut by K alone.  Two
-// short kernels are a launch and a trip to memory more than one: 4 rows of 4,096 channels into 128 and 32 columns 6.4 and 6.5 us apart, and
-// whole requests of four sequences through six scans and two gated linear attentions 9,796 us and 9,384.  (A large product with 16 columns
-// beside it gained nothing in the gated delta rule: 5,290 and 5,329.)
-extern "C" int nnis_gemm_two(const void* x, const void* w, void* y, int columns, void* second, int second_dtype, int m, int n, int k, void* stream_ptr) {
-  NNIS_REQUIRE(nnis_dtype_ok(second_dtype), "gemm_two: unknown output dtype %d", second_dtype);
-  NNIS_REQUIRE(m > 0 && m <= 16 && columns > 0 && columns % 16 == 0 && columns < n && n < 2048 * 16 && k > 0 && k % 8 == 0,
-               "gemm_two: %d rows, %d of %d columns and K=%d are not taken", m, columns, n, k);
-  for (const void* p : {x, w, (const void*)y, (const void*)second}) NNIS_REQUIRE(p && (uintptr_t)p % 16 == 0, "gemm_two: operands must be there, 16-byte aligned");
-  dispatch_skinny_split<1, TwoOut>((const bf16_t*)x, (const bf16_t*)w, TwoOut{(bf16_t*)y, columns, second, second_dtype == NNIS_F32, n}, m, n, k,
-                                   skinny_split(m, n, k, 0), nullptr, (hipStream_t)stream_ptr);
-  NNIS_LAUNCH_CHECK("gemm_two");
   return 0;
 }
 

@@ -158,8 +158,8 @@ def _attention_recipe(rest: str) -> ModuleRecipe:
 
 
 # the library's own modules: ``core`` holds the kernels whose sizes are run-time arguments; attention is compiled per head size
-register_module("core", ["elementwise.hip", "residual.hip", "gemm.hip", "gemm_f32.hip", "gemm_mfma.hip", "gemm_fused.hip", "sampling.hip"],
-                headers=["common.h", "epilogue.h", "lds_loads.h", "product.h", "nnis_noalloc.h"], source_flags={"gemm_mfma.hip": _VECTOR_SUMS, "gemm_f32.hip": _VECTOR_SUMS})
+register_module("core", ["elementwise.hip", "residual.hip", "gemm.hip", "gemm_f32.hip", "gemm_mfma.hip", "gemm_fused.hip", "gemm_two.hip", "sampling.hip"],
+                headers=["common.h", "epilogue.h", "lds_loads.h", "product.h", "nnis_noalloc.h"], source_flags={"gemm_mfma.hip": _VECTOR_SUMS, "gemm_f32.hip": _VECTOR_SUMS, "gemm_two.hip": _VECTOR_SUMS})
 register_module_family("attn_hd", _attention_recipe)
 # the mixers that carry a state of fixed size (convolution, selective scan, gated linear attention and retention, minGRU, gated delta rule)
 register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
