@@ -64,7 +64,7 @@ void launch_two(const bf16_t* x, const bf16_t* w, const TwoOut& y, int m, int n,
 
 // w [n, k]: two packed weights, the first of `columns` rows (whole strips), whose product goes to y in bfloat16, the other's to second in
 // second_dtype.  Two short kernels are a launch and a trip to memory more than one: 4 rows of 4,096 channels into 128 and 32 columns
-// 6.4 and 6.5 us apart, and whole requests of four sequences through six scans and two gated linear attentions 9,757 us and 9,370.  (A
+// 6.4 and 6.5 us apart, and whole requests of four sequences through six scans and two gated linear attentions 9,794 us and 9,322.  (A
 // large product with 16 columns beside it gained nothing in the gated delta rule: 5,290 and 5,329.)
 extern "C" int nnis_gemm_two(const void* x, const void* w, void* y, int columns, void* second, int second_dtype, int m, int n, int k, void* stream_ptr) {
   NNIS_REQUIRE(nnis_dtype_ok(second_dtype), "gemm_two: unknown output dtype %d", second_dtype);
