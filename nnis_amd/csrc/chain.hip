@@ -585,7 +585,8 @@ __device__ __forceinline__ float rounded_sum(float sum, float a, float b) {
 }
 
 // Four channels of a (row, head) from its runs, RUNS at once: a head is 16 lanes, a wave has four.  alone: in the roundings of the
-// layers' kernel of its own for this sum (more than four rows), not of the output projection that makes it on the way.
+// layers' kernel of its own for this sum, not of the output projection that makes it on the way (up to four rows, of up to 2,040
+// channels: 16 rows of them in its LDS; nnis_gemm_residual_runs_fits).
 template <int RUNS>
 __device__ __forceinline__ bf16x4 sum_runs(const Exchange& ex, unsigned first_word, int splits, int channel, bool alone) {
   u32x4 v[RUNS];
@@ -619,7 +620,7 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
   const int item = min(first + lane / 16, items - 1), head = item / a.m, row = item % a.m, channel = lane % 16 * 4;
   ex.template gate<false>(here + a.q + first * 61 % (items * (HD / 2)), 0);
   const Exchange runs(a, a.run_words, a.run_bytes);
-  const bool alone = a.rows > 4;
+  const bool alone = a.rows > 4 || a.heads * HD > 2040;
   const unsigned first_run = layer * a.layer_runs + (row * a.heads + head) * a.splits * kRunRow;
   const bf16x4 out = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, alone)
                      : a.splits <= 8 ? sum_runs<8>(runs, first_run, a.splits, channel, alone) : sum_runs<16>(runs, first_run, a.splits, channel, alone);

@@ -680,6 +680,16 @@ def step_tables(tok_slot: torch.Tensor, tok_pos: torch.Tensor, tokens: int, cos:
 CHAIN_MOST_ROWS = 16
 
 
+def chain_cuts_alike(batch: int, width: int, heads: int, inner: int) -> bool:
+    """Whether ``chain`` cuts K, heads of 64 channels in groups of up to four, in the ways that the layers' own kernels do, so that a step
+    has the same bits by either.  Where those take ways that the launch does not have, it is not made: more than four parts of
+    the output projection's K on four waves (more than 16 heads), two blocks a strip (``nnis_gemm_takes_pair``: K of 80 chunks and
+    more up to a width of 2,048, up to 16 rows) other than a wide model's down, and less than four parts of gate and up on eight waves."""
+    if width <= 1024:
+        return heads <= 16 and (inner < 80 * 64 or batch > 16)
+    return inner <= 8192 and (width > 2048 or heads < 80)
+
+
 def chain_words(layers: int, rows: int, width: int, heads: int, kv_heads: int, inner: int, runs: int, dtype=torch.bfloat16):
     """(32-bit words of the exchange, of the runs) that ``chain`` needs; (0, _) for sizes that it does not take."""
     of_runs, lib = _I64(), chain_module()
@@ -697,7 +707,7 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
     the longest sequence of ``longest`` tokens; None where the launch is not to take the step.
 
     In bfloat16 with up to four query heads a key head these are the layers' own kernels', whose bits the launch then has (the ways
-    that K is cut are theirs too).  Other plans are not faster by much: 32/32 heads, 24 layers, whole steps in microseconds by the
+    that K is cut are theirs too: ``chain_cuts_alike``).  Other plans are not faster by much: 32/32 heads, 24 layers, whole steps in microseconds by the
     layers' kernels, by this plan and by one of 8 waves: batch 2 at 500 tokens 1,173 and 724 and 716, batch 8 at 2,000 1,539 and 1,233 and
     1,196, batch 12 at 3,000 2,218 and 2,064 and 1,993.
 
@@ -717,6 +727,8 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
         while runs < 16 and 4 * pages > runs * waves and 2 * runs * blocks <= 256:
             runs *= 2
     elif heads // kv_heads <= 4:
+        if not chain_cuts_alike(batch, width, heads, inner):
+            return None
         runs, waves = decode_plan(batch, kv_heads, longest, width=heads * head_dim)
     elif batch >= 8:
         return None

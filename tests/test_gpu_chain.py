@@ -129,6 +129,64 @@ def test_32_bits_against_the_oracle(tmp_path, sizes, batch, monkeypatch):
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 64 bits, the layers' kernels {(layers - want).norm().item():.4g}"
 
 
+def _streams(folder, lengths, plan, monkeypatch):
+    """The 32-bit stream behind the last attention and what the last feed-forward adds to it, of two steps of single tokens, and whether
+    the launch ran.  (Logits are of 16-bit rows, in which most differences of the last bit are gone.)"""
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.kernels import ops
+
+    with monkeypatch.context() as patch:
+        patch.setattr(ops, "chain_prompt_takes", lambda *args, **sizes: False)  # (the same cache for all)
+        if plan != "own":
+            patch.setattr(ops, "chain_plan", lambda *args, **sizes: plan)
+        engine = load_engine(folder, dtype="bfloat16", max_tokens=sum(-(-(n + 3) // 64) * 64 for n in lengths))
+        engine.use_graphs = False  # (launched: what the final norm is handed is seen here)
+        prompts, tokens = _tokens(lengths, 2)
+        slots = [engine.start_sequence() for _ in lengths]
+        engine.step([StepEntry(slot, prompt, None) for slot, prompt in zip(slots, prompts)])
+        seen, norm = [], engine.model.final_norm
+        add = norm.add_forward
+        patch.setattr(norm, "add_forward", lambda x, delta, *args, **more: seen.extend((x.clone(), delta.clone())) or add(x, delta, *args, **more), raising=False)
+        for row in tokens:
+            engine.step([StepEntry(slot, [token], None) for slot, token in zip(slots, row)])
+        chain = engine.model.layer_chain(engine.rt)
+        return seen, chain is not None and len(chain.tables) > 0
+
+
+# ... and whether the launch takes 3, 16 and 20 rows of them: the layers' kernels cut K in ways that it does not have
+CUTS = [
+    ((1024, 16, 4, 2048), (True, True, True)),
+    ((1024, 17, 17, 512), (False, False, False)),   # the output projection in eight parts, four waves
+    ((1024, 32, 8, 512), (False, False, False)),
+    ((192, 6, 2, 5056), (True, True, True)),
+    ((192, 6, 2, 5120), (False, False, True)),      # down by two blocks a strip, up to 16 rows
+    ((2048, 31, 31, 1024), (True, True, False)),    # the runs' sum on the way into the output projection, up to four rows
+    ((2048, 32, 32, 1024), (True, True, False)),    # ... and by a kernel of its own
+    ((2048, 79, 79, 256), (True, True, False)),
+    ((2048, 80, 20, 256), (False, False, False)),   # the output projection by two blocks a strip
+    ((2112, 80, 20, 256), (True, True, False)),     # ... not above a width of 2,048
+    ((3072, 24, 8, 8192), (True, True, False)),
+    ((3072, 24, 8, 8256), (False, False, False)),   # gate and up in two parts
+    ((4096, 64, 16, 4096), (True, True, False)),
+]
+
+
+@pytest.mark.parametrize("sizes, taken", CUTS)
+def test_cuts_of_k(tmp_path, sizes, taken, monkeypatch):
+    """Both sides of each line of ``chain_cuts_alike``: the stream's bits are the layers' kernels' wherever the launch is made."""
+    import nnis_amd
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    for batch, takes in zip((3, 16, 20), taken):
+        lengths = (LENGTHS + [n + 1 for n in LENGTHS])[:batch] if batch != 3 else [1100, 1500, 700]
+        layers, ran = _streams(str(tmp_path), lengths, None, monkeypatch)
+        assert not ran
+        got, ran = _streams(str(tmp_path), lengths, "own", monkeypatch)
+        assert ran == takes, batch
+        assert len(got) == 4 and all(torch.equal(a, b) for a, b in zip(got, layers)), batch
+
+
 @pytest.mark.parametrize("counts", [(2,), (16,), (33,), (177,), (600,), (1, 1, 15, 16, 1, 30, 33), (100, 3, 260, 2), (9,) * 20])
 @pytest.mark.parametrize("sizes", SIZES + [(1088, 8, 8, 4160)])  # (eight waves with a second round of down's weights)
 def test_prompts_against_the_layers(tmp_path, sizes, counts, monkeypatch):
