@@ -702,6 +702,29 @@ def chain_takes(layers: int, rows: int, width: int, heads: int, kv_heads: int, h
     return head_dim == 64 and chain_words(layers, rows, width, heads, kv_heads, inner, runs, dtype)[0] > 0
 
 
+def chain_longest(batch: int, width: int, heads: int, kv_heads: int, dtype=torch.bfloat16) -> float:
+    """The longest sequence with which ``chain`` is to take a step of ``batch`` single tokens: the layers' own attention reads
+    long sequences' keys faster (its waves ask for pages further ahead), and from some length on that is more than the launch saves.
+
+    Whole steps by the layers' kernels over the launch's, at thousands of tokens in every sequence.  In bfloat16 up to a width of 1,024 with
+    groups of up to four heads, by rows x key heads: 9/3 heads, 1 row 1.22 at 32 and 1.01 at 64; 4 rows 1.05 at 32, 0.95 at 64; 6 rows 1.02 at
+    24, 0.92 at 32; 12 rows 1.14 at 8, 0.94 at 16; 16 rows 1.14 at 8, 1.00 at 16; 12/3 heads, 16 rows 1.03 at 16, 0.93 at 32; 16/16 heads, 1 row 1.08 at
+    32, 0.88 at 64; 4 rows 1.11 at 8, 0.96 at 16; 8 rows 1.06 at 16, 0.97 at 32; 16 rows 1.06 at 4, 0.95 at 8.  Of 17 to 32 rows, 9/3 heads 1.02 to
+    1.08 at 4, 0.98 to 1.02 at 5, 0.85 to 0.88 at 8; 16/16 heads 1.00 to 1.03 at 4, 0.97 to 1.00 at 8.  Larger groups: 32/4 heads, 1 row 1.98 at 64, 4 rows
+    1.27 at 32, 0.99 at 64.  In 32 bits up to a width of 1,024: 9/3 heads, 8 rows 1.06 at 32, 0.97 at 64; 16 rows 1.03 at 32, 0.97 at 64; 4 rows
+    1.19 at 64.  Wider models of small groups and of 32 bits do not lose: 32/8 heads, 16 rows 1.12 at 32, 1.07 at 64; 32/32 heads, 16 rows 1.06 at 16,
+    1.02 at 32; in 32 bits 32/4 heads, 16 rows 1.13 at 64."""
+    if dtype == torch.float32:
+        return 400_000 // batch if width <= 1024 else math.inf
+    if heads // kv_heads > 4:
+        return 200_000 // batch
+    if width > 1024:
+        return math.inf
+    if batch > CHAIN_MOST_ROWS:
+        return 4096
+    return max(6144, min(40960, 450_000 // (batch * kv_heads)))
+
+
 def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """(runs that ``chain`` cuts a sequence's keys into, waves that share a run's pages) for a step of ``batch`` single tokens,
     the longest sequence of ``longest`` tokens; None where the launch is not to take the step.
@@ -719,7 +742,7 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
     # two tiles of rows where the layers' products are those of few rows, a tile at a time (weights of up to 8 MB)
     two = (dtype == torch.bfloat16 and width <= 1024 and heads // kv_heads <= 4
            and 2 * width * max(2 * inner, (heads + 2 * kv_heads) * head_dim) <= 8 << 20)
-    if batch > (2 * CHAIN_MOST_ROWS if two else CHAIN_MOST_ROWS):
+    if batch > (2 * CHAIN_MOST_ROWS if two else CHAIN_MOST_ROWS) or longest > chain_longest(batch, width, heads, kv_heads, dtype):
         return None
     pages, runs, waves = (longest + 63) // 64, 1, 8 if dtype == torch.float32 or width > 1024 else 4
     if dtype == torch.float32:

@@ -3,8 +3,9 @@ the step's sizes, checked for their invariants (what a kernel's launch
 assumes) and for the measured cases their docstrings name."""
 
 import pytest
+import torch
 
-from nnis_amd.kernels.ops import PREFILL_CLASS_LENGTH, decode_plan, prefill_plan_class, prefill_tile_items
+from nnis_amd.kernels.ops import PREFILL_CLASS_LENGTH, chain_plan, decode_plan, prefill_plan_class, prefill_tile_items
 
 
 @pytest.mark.parametrize("batch", [1, 2, 8, 33, 64, 256])
@@ -186,3 +187,26 @@ def test_prefill_plans_of_short_prompts_of_wide_heads(heads, kv_heads, head_dim)
     most = 4096 // heads
     assert prefill_plan(100, most, heads, head_dim, kv_heads) == prefill_plan(1, 64, heads, head_dim, kv_heads) == (1, 1)
     assert prefill_plan(100, most + 1, heads, head_dim, kv_heads) == prefill_plan(24, 65024 // heads, heads, head_dim, kv_heads) == (1, 0)
+
+
+@pytest.mark.parametrize("heads, kv_heads, width, dtype, batch, longest", [
+    (9, 3, 576, torch.bfloat16, 1, 40960), (9, 3, 576, torch.bfloat16, 4, 37500), (9, 3, 576, torch.bfloat16, 8, 18750),
+    (16, 16, 1024, torch.bfloat16, 1, 28125), (16, 16, 1024, torch.bfloat16, 4, 7031), (16, 16, 1024, torch.bfloat16, 16, 6144),
+    (9, 3, 576, torch.bfloat16, 17, 4096), (9, 3, 576, torch.bfloat16, 32, 4096), (32, 4, 2048, torch.bfloat16, 4, 50000),
+    (9, 3, 576, torch.float32, 8, 50000), (9, 3, 576, torch.float32, 16, 25000)])
+def test_long_sequences_stay_with_the_layers_kernels(heads, kv_heads, width, dtype, batch, longest):
+    """A step is launched as one up to the measured length and not from the next page on; wider models' at any length."""
+    def taken(tokens):
+        return chain_plan(2, batch, tokens, width=width, heads=heads, kv_heads=kv_heads, head_dim=64, inner=1536, dtype=dtype) is not None
+
+    assert taken(1) and taken(longest) and not taken(longest + 1) and not taken(10 * longest)
+    assert chain_plan(2, 16, 1 << 20, width=2048, heads=32, kv_heads=8, head_dim=64, inner=8192) is not None
+
+
+def test_ways_to_cut_k_that_a_launched_step_does_not_have():
+    def taken(batch, width, heads, inner):
+        return chain_plan(2, batch, 500, width=width, heads=heads, kv_heads=heads, head_dim=64, inner=inner) is not None
+
+    assert taken(16, 1024, 16, 2048) and not taken(1, 1024, 17, 2048) and not taken(16, 1024, 17, 2048)
+    assert taken(16, 192, 4, 5056) and not taken(16, 192, 4, 5120) and taken(17, 192, 4, 5120)
+    assert taken(1, 1088, 79, 8192) and not taken(1, 1088, 79, 8256) and not taken(1, 2048, 80, 2048) and taken(1, 2112, 80, 2048)
