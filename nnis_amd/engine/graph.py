@@ -97,7 +97,6 @@ class DecodeGraph:
         """``ids``: the step's token ids, or None when they are on the device
         already: then row j's id is ``ids_device[j]`` (int32)."""
         count = len(slots)
-        self.engine.model.check_steps(self.engine.rt)
         self.copied.synchronize()  # the previous copy has left the pinned buffer
         host = self.host.numpy()
         host[0, :count] = ids if ids is not None else -1
@@ -275,7 +274,6 @@ class PrefillGraph:
 
     def run(self) -> torch.Tensor:
         """Replays the step on what the buffers hold; the rows returned view the graph's output buffer."""
-        self.engine.model.check_steps(self.engine.rt)
         self.graph.replay()
         return self.logits
 

@@ -144,6 +144,7 @@ class Engine:
         overwrites: for callers that read them at once (the generation loop)."""
         self._borrowed = False
         self.rt.check_current()
+        self.model.check_steps(self.rt)
         if self.use_graphs and entries and all(len(e.tokens) == 1 for e in entries):
             return self._decode_step(entries)
         growth, token_arrays = self._validate(entries)
@@ -239,6 +240,7 @@ class Engine:
             raise InvalidInput("step_from_device: one int32 id per slot is needed")
         self._borrowed = False
         self.rt.check_current()
+        self.model.check_steps(self.rt)
         return self._decode_step([StepEntry(s, (), None) for s in slots], ids_device)
 
     def _decode_step(self, entries: Sequence[StepEntry], ids_device: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -30,3 +30,8 @@ class CacheFull(NnisError):
 
 class KernelError(NnisError, RuntimeError):
     """The HIP extension is missing, failed to build, or refused an argument."""
+
+
+class StepLost(KernelError):
+    """A step's kernel gave up waiting for its own blocks: what the step computed is not numbers.  (No refusal: who goes on by
+    another way where a kernel refuses lets this one through.)"""

@@ -10,7 +10,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-from ..errors import KernelError
+from ..errors import StepLost
 
 
 class LayerChain:
@@ -57,8 +57,8 @@ class LayerChain:
         """Raises if a wait of an earlier step was given up."""
         if self._failed[0]:
             self._failed[0] = 0
-            raise KernelError("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
-                              "the logits of the step before this one are not numbers")
+            raise StepLost("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
+                           "the logits of the step before this one are not numbers")
 
     def views_fit(self, views) -> bool:
         """Whether each layer writes keys and values of its own, through one block table."""
@@ -80,7 +80,6 @@ class LayerChain:
 
     def forward(self, x: torch.Tensor, ctx, views, plan, rt):
         """The stream, and what the last layer still adds to it; None where the launch cannot be made here."""
-        self.check()
         table = self._table(views, x.device)
         if table is None:
             return None

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from configs import llama
-from nnis_amd.errors import KernelError
+from nnis_amd.errors import KernelError, StepLost
 
 pytestmark = pytest.mark.gpu
 
@@ -328,6 +328,32 @@ def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
     with pytest.raises(KernelError, match="gave up waiting"):
         engine.step([StepEntry(slot, [7], None)])
     assert engine.length(slot) == length + 1
+
+
+def test_a_report_is_no_refusal(tmp_path):
+    """The report reaches the caller also at the step with which a shape of prompts would be captured, and the shape is captured later."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+
+    nnis_amd.write_random_model(str(tmp_path), _config(64, 1, 1, 64), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=512)
+    prompt = list(range(20))
+
+    def step():
+        slot = engine.start_sequence()
+        try:
+            return engine.step([StepEntry(slot, prompt, None)])
+        finally:
+            engine.end_sequence(slot)
+
+    want = step()
+    engine.model.layer_chain(engine.rt).failed[0] = 1
+    with pytest.raises(StepLost, match="gave up waiting"):
+        step()
+    for _ in range(3):
+        assert torch.equal(step(), want)
+    assert len(engine._prefill_graphs.graphs) == 1 and not engine._prefill_graphs.refused
 
 
 def test_sizes_and_words():
