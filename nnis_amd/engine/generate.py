@@ -115,6 +115,7 @@ def generate(engine, requests: Sequence[GenerationRequest], selector=None, max_b
     step = getattr(engine, "step_view", engine.step)  # the logits are read at once: no copy needed
     # An engine that takes a step's ids from the device, with a selector that leaves them there, runs a step
     # ahead of the host (below); any other pair runs step by step.
+    check = getattr(engine, "check_steps", lambda: None)
     ahead = getattr(engine, "use_graphs", False) and hasattr(engine, "step_from_device") and hasattr(selector, "select_start")
 
     def take(index: int, token: int, slot_of) -> bool:
@@ -152,6 +153,7 @@ def generate(engine, requests: Sequence[GenerationRequest], selector=None, max_b
                     live = []
                     break
                 tokens = selector.select(logits, [slot_of[i] for i in live], [requests[i].sampling for i in live])
+                check()  # (a selector of another kind may have read logits that are none)
                 still = []
                 for index, token in zip(live, tokens):
                     if take(index, int(token), slot_of):

@@ -16,7 +16,7 @@ import torch
 
 from ..cache import SequenceCache
 from ..cache.allocator import PAGE_TOKENS, pages_for
-from ..errors import InvalidInput
+from ..errors import InvalidInput, StepLost
 from .batch import StepContext, StepEntry
 from .graph import PREFILL_GRAPH_MOST_TOKENS, PREFILL_GRAPH_MOST_WORK, PrefillGraphs, prompt_rows
 
@@ -42,6 +42,7 @@ class Engine:
         self.use_graphs = model.graph_safe() if use_graphs is None else (use_graphs and model.graph_safe())
         self._graphs = None
         self._prefill_graphs = None  # prompt steps whose shape comes again
+        self._lost = model.lost_steps(rt)
         # A step's positions index the rotation tables on the device, where nothing can refuse them: the tables
         # reach as far as the cache lets a sequence grow, so the check of the lengths before a step covers both.
         for name, position in model.positions.items():
@@ -76,6 +77,17 @@ class Engine:
     def free_pages(self) -> int:
         groups = self.cache.kv_groups
         return min(g.table.pool.free for g in groups) if groups else 1 << 30
+
+    # ---- steps that are lost -------------------------------------------------
+    def check_steps(self) -> None:
+        """Raises ``StepLost`` if a step gave up waiting for its own blocks.  Every step asks this when it begins, and every
+        ``PendingTokens`` before it hands its tokens out; a caller that reads a step's logits itself asks once it has them on the
+        host."""
+        lost = self.model.lost_steps(self.rt)
+        if lost != self._lost:
+            self._lost = lost
+            raise StepLost("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); what it computed is "
+                           "not numbers")
 
     # ---- one step ------------------------------------------------------------
     def _validate(self, entries: Sequence[StepEntry]):
@@ -144,7 +156,7 @@ class Engine:
         overwrites: for callers that read them at once (the generation loop)."""
         self._borrowed = False
         self.rt.check_current()
-        self.model.check_steps(self.rt)
+        self.check_steps()
         if self.use_graphs and entries and all(len(e.tokens) == 1 for e in entries):
             return self._decode_step(entries)
         growth, token_arrays = self._validate(entries)
@@ -240,7 +252,7 @@ class Engine:
             raise InvalidInput("step_from_device: one int32 id per slot is needed")
         self._borrowed = False
         self.rt.check_current()
-        self.model.check_steps(self.rt)
+        self.check_steps()
         return self._decode_step([StepEntry(s, (), None) for s in slots], ids_device)
 
     def _decode_step(self, entries: Sequence[StepEntry], ids_device: Optional[torch.Tensor] = None) -> torch.Tensor:

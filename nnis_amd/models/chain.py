@@ -10,8 +10,6 @@ from typing import Dict, List, Optional
 
 import torch
 
-from ..errors import StepLost
-
 
 class LayerChain:
     def __init__(self, links: List[dict], rt):
@@ -21,9 +19,10 @@ class LayerChain:
         self.sizes = {name: first[name] for name in ("width", "heads", "kv_heads", "head_dim", "inner")}
         self.sizes["dtype"] = rt.dtype
         self.eps, self.scale, self.position, self.gain_dtype = first["eps"], first["scale"], first["position"], first["gains"][0].dtype
-        # where a wait that was given up says so: a word of host memory that the kernel writes and the next step reads
+        # where a wait that was given up says so: a word of host memory that the kernel writes
         self.failed = torch.zeros(1, dtype=torch.int32, pin_memory=True)
         self._failed = self.failed.numpy()
+        self._lost = 0
         self.tables: Dict[tuple, torch.Tensor] = {}  # the layers' pointers -> the same on the device
 
     @classmethod
@@ -53,12 +52,14 @@ class LayerChain:
         """Whether the launch takes a step of prompts of this many rows in all that each begin at their sequence's first position."""
         return rt.ops.chain_prompt_takes(len(self.links), rows, **self.sizes)
 
-    def check(self) -> None:
-        """Raises if a wait of an earlier step was given up."""
+    def lost(self) -> int:
+        """How often a report of given-up waits has been found: one more than before if a step that has run since then made one.
+        (Steps still on their way may make another for the same reason: they are waited for, and go with it.)"""
         if self._failed[0]:
+            torch.cuda.current_stream().synchronize()
             self._failed[0] = 0
-            raise StepLost("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); "
-                           "the logits of the step before this one are not numbers")
+            self._lost += 1
+        return self._lost
 
     def views_fit(self, views) -> bool:
         """Whether each layer writes keys and values of its own, through one block table."""

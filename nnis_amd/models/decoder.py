@@ -96,11 +96,10 @@ class DecoderModel:
         chain = self.layer_chain(rt)
         return list(chain.tables.values()) if chain is not None else []
 
-    def check_steps(self, rt) -> None:
-        """Raises if the kernels of an earlier step found something wrong that only the host can report."""
+    def lost_steps(self, rt) -> int:
+        """How often kernels have reported that a step of this model is lost (``LayerChain.lost``)."""
         chain = self.layer_chain(rt)
-        if chain is not None:
-            chain.check()
+        return chain.lost() if chain is not None else 0
 
     def prompt_plan(self, batch: int, rows: int, longest: int, rt, most_new: int = 0, fresh: Optional[bool] = None):
         """The plans of every run of the schedule for a step of prompts (``Part.prompt_plan``, ``Part.run_plan``);

@@ -23,13 +23,17 @@ class PendingTokens:
     """Tokens that a selection kernel has been asked for: on the device at
     once (in stream order), on the host when ``result`` returns."""
 
-    def __init__(self, device: torch.Tensor, host: torch.Tensor, event):
+    def __init__(self, device: torch.Tensor, host: torch.Tensor, event, check=None):
+        """``check``: called once the tokens are on the host, raises if they are none (``Engine.check_steps``)."""
         self.device = device
         self._host = host
         self._event = event
+        self._check = check
 
     def result(self) -> List[int]:
         self._event.synchronize()
+        if self._check is not None:
+            self._check()
         tokens = self._host.tolist()
         for row, token in enumerate(tokens):
             if token < 0:  # what the sampling kernel leaves in place of a token it will not draw
@@ -98,7 +102,7 @@ class DeviceSelector:
                        self.top_p, device[:rows], by_slot=True, best=device[:rows])
         host[:rows].copy_(device[:rows], non_blocking=True)
         event.record()
-        return PendingTokens(device[:rows], host[:rows], event)
+        return PendingTokens(device[:rows], host[:rows], event, self.engine.check_steps)
 
     def select(self, logits: torch.Tensor, slots: Sequence[int], params: Sequence[Optional[SamplingParams]]) -> List[int]:
         """One token per row of ``logits``, on the host."""

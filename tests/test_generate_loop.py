@@ -4,10 +4,11 @@ sequences that end earlier, batches one after another with slots used again."""
 
 import numpy as np
 import pytest
+import torch
 
 from nnis_amd.cache.allocator import FreeList, pages_for
 from nnis_amd.engine.generate import GenerationRequest, generate, plan_batches
-from nnis_amd.errors import CacheFull, InvalidInput
+from nnis_amd.errors import CacheFull, InvalidInput, StepLost
 from nnis_amd.sampling import HostSampler, SamplingParams, greedy_token
 
 VOCAB = 50
@@ -79,6 +80,43 @@ def test_unequal_prompts_stop_tokens_and_early_ends():
     # the last emitted token is not run: 5 decode steps for 6 new tokens
     assert len(engine.steps) == 6 and engine.lengths == {} and engine.free_slots() == 4
     assert engine.ended == [2, 1, 0]  # given back as each ends, not at the batch's end
+
+
+@pytest.mark.parametrize("lost", [1, 2, 4])
+def test_tokens_of_a_lost_step_are_not_handed_out(lost):
+    """An engine that says after a step that it is lost: its tokens reach nobody, and the slots go back."""
+    class LosingEngine(ToyEngine):
+        def check_steps(self):
+            if len(self.steps) == lost:
+                raise StepLost("lost")
+
+    engine, seen = LosingEngine(), []
+    with pytest.raises(StepLost):
+        generate(engine, [GenerationRequest([1], max_new_tokens=4, on_token=lambda i, token: seen.append(token) or True)], HostSelector())
+    assert seen == [2, 3, 4, 5][:lost - 1] and engine.lengths == {} and engine.free_slots() == 4
+
+
+def test_a_result_is_checked_before_it_is_read():
+    from nnis_amd.sampling.device import PendingTokens
+
+    class Event:
+        waited = False
+
+        def synchronize(self):
+            self.waited = True
+
+    event, asked = Event(), []
+
+    def check():
+        asked.append(event.waited)
+        raise StepLost("lost")
+
+    tokens = torch.tensor([0, -1], dtype=torch.int32)
+    with pytest.raises(StepLost):
+        PendingTokens(tokens, tokens, event, check).result()
+    assert asked == [True]  # once the step has run
+    assert PendingTokens(tokens[:1], tokens[:1], event, lambda: None).result() == [0]
+    assert PendingTokens(tokens[:1], tokens[:1], event).result() == [0]
 
 
 def test_batches_follow_one_another_and_reuse_slots():

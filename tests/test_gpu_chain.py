@@ -356,6 +356,65 @@ def test_a_report_is_no_refusal(tmp_path):
     assert len(engine._prefill_graphs.graphs) == 1 and not engine._prefill_graphs.refused
 
 
+def _lose(engine, call, at):
+    """Patches ``engine`` so that the ``at``-th step's launch is followed by the word that a given-up wait writes."""
+    count = [0]
+
+    def wrap(step):
+        def run(*args):
+            out = step(*args)
+            count[0] += 1
+            if count[0] == at:
+                engine.model.layer_chain(engine.rt).failed[0] = 1
+            return out
+        return run
+
+    for name in ("step_view", "step_from_device"):
+        call.setattr(engine, name, wrap(getattr(engine, name)))
+
+
+@pytest.mark.parametrize("new, at", [(1, 1), (6, 1), (6, 3), (6, 6)])
+@pytest.mark.parametrize("ahead", [True, False])
+def test_tokens_of_a_lost_step_go_nowhere(tmp_path, new, at, ahead, monkeypatch):
+    """A request whose step gave a wait up, its only one, its first, a later one or its last, gets an error and no token of that step; the
+    next request gets its tokens."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.generate import GenerationRequest, generate
+
+    nnis_amd.write_random_model(str(tmp_path), _config(64, 1, 1, 64), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=512)
+    engine.use_graphs = ahead
+    prompts = [list(range(20)), list(range(30, 37))]
+    seen = [[], []]
+    want = [r.tokens for r in generate(engine, [GenerationRequest(p, new) for p in prompts])]
+    with monkeypatch.context() as patch:
+        _lose(engine, patch, at)
+        with pytest.raises(StepLost, match="gave up waiting"):
+            generate(engine, [GenerationRequest(p, new, on_token=lambda i, token: seen[i].append(token) or True) for p in prompts])
+    for tokens, right in zip(seen, want):
+        assert tokens == right[:len(tokens)] and len(tokens) < at
+    assert not engine.cache.lengths
+    assert [r.tokens for r in generate(engine, [GenerationRequest(p, new) for p in prompts])] == want
+
+
+def test_pending_tokens_of_a_lost_step(tmp_path):
+    """Written between the selection and its result."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.sampling.device import DeviceSelector
+
+    nnis_amd.write_random_model(str(tmp_path), _config(64, 1, 1, 64), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=512)
+    selector = DeviceSelector(engine)
+    slot = engine.start_sequence()
+    pending = selector.select_start(engine.step_view([StepEntry(slot, [1, 2, 3], None)]), [slot], [None])
+    engine.model.layer_chain(engine.rt).failed[0] = 1
+    with pytest.raises(StepLost):
+        pending.result()
+
+
 def test_sizes_and_words():
     """The exchange's size is 0 for what the launch refuses, and grows with what it holds."""
     from nnis_amd.kernels import ops
