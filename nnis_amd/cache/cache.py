@@ -349,6 +349,14 @@ class SequenceCache:
             lengths[slot] = length + 1
         return before
 
+    def zero_pages_beside(self, slots: Sequence[int]) -> None:
+        """Zeroes every page that none of these slots holds."""
+        for group in self.kv_groups:
+            kept = {page for slot in slots for page in group.table.rows.get(slot, ())}
+            others = torch.tensor([page for page in range(self.pages) if page not in kept], dtype=torch.long, device=self.device)
+            for pages in (group.k, group.v):
+                pages.index_fill_(1, others, 0)
+
     def bytes_per_token(self) -> int:
         return sum(group.bytes_per_token() for group in self.kv_groups)
 

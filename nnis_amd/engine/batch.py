@@ -125,6 +125,7 @@ class StepContext:
     plan_rows: int = 0
     plan_new: int = 0
     fresh: bool = False  # every sequence begins at its first position with this step
+    chained: bool = False  # set by the model: its layers ran as one launch, which may give a wait up (``Engine.check_steps``)
     options: dict = field(default_factory=dict)  # launch options by part kind, for tests and tuning: {"causal_attention": {...}}
     lists: Optional[StepLists] = None  # the parts' host-made work lists (``StepLists``)
     ids: Optional[torch.Tensor] = None  # int32 [tokens]: the step's tokens, for parts that read them beside the stream

@@ -189,6 +189,7 @@ class PrefillGraph:
         self.graph = None
         self.logits = None
         self.held, self.tables = [], []
+        self.chained = False  # whether the first run was (the capture's context says it of the replays)
         self._lay_out({})
 
     def _lay_out(self, list_shapes) -> None:
@@ -250,6 +251,7 @@ class PrefillGraph:
         self.ctx.lists = self.lists
         try:
             logits = self._forward()
+            self.chained = self.ctx.chained
         except KernelError:
             return None  # (a part that needs the host's view of the step: the caller runs the step as any step)
         self._lay_out(dict(self.lists.shapes))
@@ -288,14 +290,14 @@ class PrefillGraphs:
         self.graphs: Dict[tuple, PrefillGraph] = {}  # in the order of their last use
 
     def step(self, key: tuple, arrays, counts: Sequence[int], first_positions: Sequence[int], longest: int):
-        """(logits, borrowed) if this step is replayed or captured; None if it is to run as any step.
+        """(logits, borrowed, chained) if this step is replayed or captured; None if it is to run as any step.
         ``key``: (sequences, rows, wanted logit rows, the parts' plans); ``longest``: the step's longest
         sequence (one for which the parts plan as the key says)."""
         graph = self.graphs.pop(key, None)
         if graph is not None:
             self.graphs[key] = graph  # the most recently used is last
             graph.fill(arrays, counts, first_positions)
-            return graph.run(), True
+            return graph.run(), True, graph.ctx.chained
         if key in self.refused:
             return None
         times = self.seen.get(key, 0) + 1
@@ -309,10 +311,10 @@ class PrefillGraphs:
         logits = graph.first_run(arrays, counts, first_positions)
         if graph.graph is None:
             self.refused.add(key)
-            return None if logits is None else (logits, False)
+            return None if logits is None else (logits, False, graph.chained)
         while len(self.graphs) >= PREFILL_GRAPHS_KEPT:
             # (the stream may still replay the oldest: it is destroyed only when the GPU has left it)
             torch.cuda.synchronize()
             self.graphs.pop(next(iter(self.graphs)))
         self.graphs[key] = graph
-        return logits, False
+        return logits, False, graph.chained

@@ -42,7 +42,11 @@ class Engine:
         self.use_graphs = model.graph_safe() if use_graphs is None else (use_graphs and model.graph_safe())
         self._graphs = None
         self._prefill_graphs = None  # prompt steps whose shape comes again
+        # Steps whose layers ran as one launch (``StepContext.chained``) may turn out lost after they were launched.
+        self.steps = 0  # steps launched so far
         self._lost = model.lost_steps(rt)
+        self._unsure = set()  # sequences that were in such a step since the last one that is known to have ended well
+        self._refused = set()  # sequences of a step that was lost: they have keys and values that are no numbers
         # A step's positions index the rotation tables on the device, where nothing can refuse them: the tables
         # reach as far as the cache lets a sequence grow, so the check of the lengths before a step covers both.
         for name, position in model.positions.items():
@@ -58,6 +62,7 @@ class Engine:
 
     def end_sequence(self, slot: int) -> None:
         self.cache.release(slot)
+        self._forget(slot)
 
     def length(self, slot: int) -> int:
         return self.cache.length(slot)
@@ -66,10 +71,13 @@ class Engine:
         """Shortens a sequence to its first ``length`` tokens; the next step
         appends there.  Pages beyond go back to the cache at once."""
         self.cache.truncate(slot, length)
+        if not length:
+            self._forget(slot)
 
     def reset(self, slot: int) -> None:
         """Empties a sequence's slot without giving the slot back."""
         self.cache.reset(slot)
+        self._forget(slot)
 
     def free_slots(self) -> int:
         return self.cache.slots.free
@@ -79,15 +87,39 @@ class Engine:
         return min(g.table.pool.free for g in groups) if groups else 1 << 30
 
     # ---- steps that are lost -------------------------------------------------
-    def check_steps(self) -> None:
-        """Raises ``StepLost`` if a step gave up waiting for its own blocks.  Every step asks this when it begins, and every
+    def check_steps(self, done: Optional[int] = None) -> None:
+        """Raises ``StepLost`` if a step gave up waiting for its own blocks: then the sequences that were in one since the last step that
+        is known to have ended well are refused until they end or are emptied.  Every step asks this when it begins, and every
         ``PendingTokens`` before it hands its tokens out; a caller that reads a step's logits itself asks once it has them on the
-        host."""
+        host.  ``done``: ``steps`` as it was behind a step that has run by now."""
         lost = self.model.lost_steps(self.rt)
-        if lost != self._lost:
-            self._lost = lost
+        if lost == self._lost:
+            if done == self.steps:
+                self._unsure.clear()
+            return
+        self._lost = lost
+        refused, self._unsure = self._unsure, set()
+        self._refused |= refused
+        # pages hold numbers whoever takes them next (``KVGroup``)
+        self.cache.zero_pages_beside([slot for slot in self.cache.lengths if slot not in self._refused])
+        if refused:
             raise StepLost("a step's kernel gave up waiting for its own blocks (another process may hold part of the GPU); what it computed is "
-                           "not numbers")
+                           f"not numbers, and the sequences of slots {sorted(refused)} have to end or be emptied")
+
+    def _may_step(self, slots) -> None:
+        self.check_steps()
+        for slot in slots if self._refused else ():
+            if slot in self._refused:
+                raise StepLost(f"slot {slot}: a step of this sequence gave up waiting for its own blocks; its keys and values are not numbers")
+
+    def _launched(self, slots, chained: bool) -> None:
+        self.steps += 1
+        if chained:
+            self._unsure.update(slots)
+
+    def _forget(self, slot: int) -> None:
+        self._unsure.discard(slot)
+        self._refused.discard(slot)
 
     # ---- one step ------------------------------------------------------------
     def _validate(self, entries: Sequence[StepEntry]):
@@ -156,7 +188,7 @@ class Engine:
         overwrites: for callers that read them at once (the generation loop)."""
         self._borrowed = False
         self.rt.check_current()
-        self.check_steps()
+        self._may_step([e.slot for e in entries])
         if self.use_graphs and entries and all(len(e.tokens) == 1 for e in entries):
             return self._decode_step(entries)
         growth, token_arrays = self._validate(entries)
@@ -203,7 +235,8 @@ class Engine:
                 self._prefill_graphs = PrefillGraphs(self)
             done = self._prefill_graphs.step(shape, arrays, counts, pos0, longest)
             if done is not None:
-                logits, self._borrowed = done
+                logits, self._borrowed, chained = done
+                self._launched([e.slot for e in entries], chained)
                 return logits
         dev = self._stage(arrays)
         ctx = StepContext(
@@ -223,7 +256,9 @@ class Engine:
             plan_rows=rows,
             fresh=fresh,
         )
-        return self.model.forward(dev[0], ctx, self.cache, dev[6], self.rt)
+        logits = self.model.forward(dev[0], ctx, self.cache, dev[6], self.rt)
+        self._launched(ctx.host_slots, ctx.chained)
+        return logits
 
     def prepare_decode(self, batch: int, longest: int) -> None:
         """Makes the graph that a step of one token for each of ``batch``
@@ -252,7 +287,7 @@ class Engine:
             raise InvalidInput("step_from_device: one int32 id per slot is needed")
         self._borrowed = False
         self.rt.check_current()
-        self.check_steps()
+        self._may_step(slots)
         return self._decode_step([StepEntry(s, (), None) for s in slots], ids_device)
 
     def _decode_step(self, entries: Sequence[StepEntry], ids_device: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -287,6 +322,7 @@ class Engine:
         except BaseException:
             self.cache.roll_back(dict(zip(slots, pos0)))
             raise
+        self._launched(slots, graph.ctx.chained)
         wanted = [i for i, e in enumerate(entries) if e.want is None or len(e.want) > 0]
         if len(wanted) == len(entries):
             self._borrowed = True

@@ -84,6 +84,7 @@ class LayerChain:
         table = self._table(views, x.device)
         if table is None:
             return None
+        ctx.chained = True
         tables = ctx.step_tables(rt, self.position.rotary(), views[0].block_table)
         more = dict(self.sizes, gain_dtype=self.gain_dtype, eps=self.eps, scale=self.scale)
         if plan == "prompt":

@@ -7,6 +7,7 @@ selection needs nothing from the host but the rows' slots."""
 
 from __future__ import annotations
 
+from functools import partial
 from typing import List, Optional, Sequence
 
 import torch
@@ -102,7 +103,7 @@ class DeviceSelector:
                        self.top_p, device[:rows], by_slot=True, best=device[:rows])
         host[:rows].copy_(device[:rows], non_blocking=True)
         event.record()
-        return PendingTokens(device[:rows], host[:rows], event, self.engine.check_steps)
+        return PendingTokens(device[:rows], host[:rows], event, partial(self.engine.check_steps, self.engine.steps))
 
     def select(self, logits: torch.Tensor, slots: Sequence[int], params: Sequence[Optional[SamplingParams]]) -> List[int]:
         """One token per row of ``logits``, on the host."""

@@ -281,6 +281,24 @@ def test_values_may_be_narrower_than_keys():
     assert narrow.bytes_per_token() == 2 * (32 + 16) * 4 and cache.kv_groups[1].bytes_per_token() == 2 * 64 * 4
 
 
+def test_pages_that_others_hold_are_zeroed():
+    cache = SequenceCache([(0, KVRequest(1, 16)), (1, (KVRequest(1, 16), KVRequest(2, 32, 64)))], {}, 640, 640, torch.float32, "cpu")
+    kept, other, gone = (cache.acquire() for _ in range(3))
+    cache.grow({kept: 65, other: 65, gone: 1})
+    cache.release(gone)
+    for group in cache.kv_groups:
+        group.k.fill_(float("nan"))
+        group.v.fill_(float("nan"))
+    cache.zero_pages_beside([kept])
+    for group in cache.kv_groups:
+        held = group.table.rows[kept]
+        for pages in (group.k, group.v):
+            for page in range(cache.pages):
+                assert bool((pages[:, page].isnan() if page in held else pages[:, page] == 0).all())
+    cache.zero_pages_beside([])
+    assert all(not bool(pages.any()) for group in cache.kv_groups for pages in (group.k, group.v))
+
+
 def test_roll_back_returns_what_a_failed_step_took():
     """A step whose launch failed after the cache grew: lengths and pages as
     before, also where fixed-size state makes ``truncate`` refuse; a slot that

@@ -309,7 +309,8 @@ def test_not_taken(tmp_path, monkeypatch):
 
 
 def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
-    """The word that a kernel writes when it gives a wait up (written here by the host) refuses the next step, once."""
+    """The word that a kernel writes when it gives a wait up (written here by the host) refuses the next step, and the sequence until it
+    has been emptied."""
     import nnis_amd
     from nnis_amd.engine.batch import StepEntry
 
@@ -322,12 +323,61 @@ def test_a_wait_given_up_is_reported(tmp_path, monkeypatch):
     with pytest.raises(KernelError, match="gave up waiting"):
         engine.step([StepEntry(slot, [7], None)])
     assert engine.length(slot) == length
+    with pytest.raises(KernelError, match="not numbers"):
+        engine.step([StepEntry(slot, [7], None)])
+    engine.truncate(slot, 0)
     assert bool(torch.isfinite(engine.step([StepEntry(slot, [7], None)])).all())
     engine.use_graphs = False  # launched, not replayed
     engine.model.layer_chain(engine.rt).failed[0] = 1
     with pytest.raises(KernelError, match="gave up waiting"):
         engine.step([StepEntry(slot, [7], None)])
-    assert engine.length(slot) == length + 1
+    assert engine.length(slot) == 1
+
+
+def test_sequences_of_a_lost_step(tmp_path):
+    """Those that were in it are refused until they end, and leave no NaN to whoever takes their pages; the others, and those whose last step
+    is known to have ended well, go on with the same bits."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.sampling.device import DeviceSelector
+
+    nnis_amd.write_random_model(str(tmp_path), _config(64, 1, 1, 64), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=320)
+    selector = DeviceSelector(engine)
+    first, second, third = (engine.start_sequence() for _ in range(3))
+    prompts = {first: [1, 2, 3], second: list(range(70)), third: [9, 8]}
+
+    def step(slots, tokens):
+        logits = engine.step([StepEntry(slot, tokens[slot], None) for slot in slots])
+        return logits, selector.select_start(logits, slots, [None] * len(slots))
+
+    step([first, second, third], prompts)[1].result()  # (known to have ended well)
+    want, _ = step([first], {first: [5]})
+    engine.truncate(first, 3)
+    selector.select_start(want, [first], [None]).result()
+    _, lost = step([second, third], {second: [5], third: [6]})
+    engine.model.layer_chain(engine.rt).failed[0] = 1
+    for view in (engine.cache.view(0), engine.cache.view(1)):  # what such a step leaves, also in pages that have gone back since
+        for slot in (second, third):
+            for page in engine.cache.kv_groups[0].table.rows[slot]:
+                view.k_pages[page] = view.v_pages[page] = float("nan")
+    engine.end_sequence(third)
+    with pytest.raises(StepLost):
+        lost.result()
+    assert torch.equal(step([first], {first: [5]})[0], want)
+    with pytest.raises(StepLost, match="not numbers"):
+        engine.step([StepEntry(second, [5], None)])
+    with pytest.raises(StepLost, match="not numbers"):
+        engine.step([StepEntry(first, [5], None), StepEntry(second, [5], None)])
+    assert engine.length(first) == 4 and engine.length(second) == 71
+    engine.end_sequence(second)
+    for _ in range(2):  # (two pages each of the four that are free: those of the lost step among them)
+        slot = engine.start_sequence()
+        engine.step([StepEntry(slot, list(range(65)), None)])
+        assert bool(torch.isfinite(engine.step([StepEntry(slot, [5], None)])).all())
+    for view in (engine.cache.view(0), engine.cache.view(1)):
+        assert bool(torch.isfinite(view.k_pages).all()) and bool(torch.isfinite(view.v_pages).all())
 
 
 def test_a_report_is_no_refusal(tmp_path):
@@ -341,11 +391,7 @@ def test_a_report_is_no_refusal(tmp_path):
     prompt = list(range(20))
 
     def step():
-        slot = engine.start_sequence()
-        try:
-            return engine.step([StepEntry(slot, prompt, None)])
-        finally:
-            engine.end_sequence(slot)
+        return engine.step([StepEntry(engine.start_sequence(), prompt, None)])
 
     want = step()
     engine.model.layer_chain(engine.rt).failed[0] = 1
