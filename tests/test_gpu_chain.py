@@ -461,6 +461,39 @@ def test_pending_tokens_of_a_lost_step(tmp_path):
         pending.result()
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("sizes", [(192, 6, 2, 192), (1088, 8, 8, 576)])
+def test_what_lies_behind_a_sequence_does_not_matter(tmp_path, sizes, dtype, monkeypatch):
+    """Keys and values from the step's own place in a page on may be no numbers: the same bits as over zeros."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    engine = load_engine(str(tmp_path), dtype=dtype, max_tokens=4096)
+    lengths = [1, 7, 8, 31, 32, 40, 62, 63, 64, 65, 100, 1100]
+    prompts, tokens = _tokens(lengths, 1)
+    slots = [engine.start_sequence() for _ in lengths]
+    for slot, prompt in zip(slots, prompts):
+        engine.step([StepEntry(slot, prompt, None)])
+
+    def step(fill):
+        for slot, n in zip(slots, lengths):
+            engine.truncate(slot, n)
+            row = engine.cache.kv_groups[0].table.rows[slot]
+            for index in range(2) if n % 64 else ():
+                view = engine.cache.view(index)
+                for t in range(n % 64, 64):
+                    view.k_pages[row[-1]][:, :, t] = fill
+                    view.v_pages[row[-1]][:, :, t // 32, t % 32 // 8, :, t % 8] = fill
+        return engine.step([StepEntry(slot, [token], None) for slot, token in zip(slots, tokens[0])])
+
+    want = step(0.0)
+    assert len(engine.model.layer_chain(engine.rt).tables) > 0
+    for fill in (float("nan"), float("inf")):
+        assert torch.equal(step(fill), want)
+
+
 def test_sizes_and_words():
     """The exchange's size is 0 for what the launch refuses, and grows with what it holds."""
     from nnis_amd.kernels import ops
