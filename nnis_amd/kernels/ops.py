@@ -763,11 +763,12 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
     return (runs, waves) if chain_takes(layers, batch, width, heads, kv_heads, head_dim, inner, runs, dtype) else None
 
 
-def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, plan, failed: torch.Tensor,
+def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, plan, failed: torch.Tensor, room,
           gain_dtype: torch.dtype, eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """All layers of a step of single tokens; returns the stream behind the last attention [rows, width] in 32 bits and what the
     last feed-forward adds to it, in ``dtype``, the weights' and the cache's.  ``layers``: int64 [8 * count] on the device, the layers'
-    pointers (``LayerChain``); ``plan``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory."""
+    pointers (``LayerChain``); ``plan``: ``chain_plan``'s; ``failed``: an int32 word of pinned host memory; ``room``: gives at least that many 32-bit
+    words for the exchange, or None, and then nothing is launched and None returned."""
     for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page"), (tables.pages, "pages")):
         _dev(t, f"chain {what}")
     rows, (runs, waves) = x.shape[0], plan
@@ -777,11 +778,14 @@ def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables,
         raise KernelError(f"chain: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
     lib = chain_module()
     words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs, dtype)
-    exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
-    partial = decode_scratch(x.device, run_words) if run_words else None  # (as the split decode attention's)
+    exchange = room(words + run_words)
+    if exchange is None:
+        return None
+    _dev(exchange, "chain exchange")
+    runs_at = exchange.data_ptr() + 4 * words if run_words else None  # (the words are whole lines)
     out, last = torch.empty_like(x), torch.empty_like(x, dtype=dtype)
     tail = (float(eps), float(scale), x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
-            tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial), run_words, failed.data_ptr(),
+            tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, runs_at, run_words, failed.data_ptr(),
             _stream())
     if dtype == torch.float32:
         _check(lib, lib.nnis_chain_f32(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, *tail))
@@ -804,7 +808,7 @@ def chain_prompt_takes(layers: int, rows: int, width: int, heads: int, kv_heads:
     return 0 < chain_module().nnis_chain_prompt_words(layers, rows, width, heads, kv_heads, inner) <= 1 << 27
 
 
-def chain_prompt(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, failed: torch.Tensor, gain_dtype: torch.dtype,
+def chain_prompt(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables, tok_pos: torch.Tensor, failed: torch.Tensor, room, gain_dtype: torch.dtype,
                  eps: float, scale: float, width: int, heads: int, kv_heads: int, head_dim: int, inner: int, dtype=torch.bfloat16):
     """As ``chain``, for the rows of prompts that each begin at their sequence's first position, one behind the other."""
     for t, what in ((layers, "layers"), (x, "x"), (tok_pos, "tok_pos"), (tables.cos, "cos"), (tables.sin, "sin"), (tables.page, "page")):
@@ -815,7 +819,10 @@ def chain_prompt(layers: torch.Tensor, count: int, x: torch.Tensor, tables: Step
         raise KernelError(f"chain_prompt: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
     lib = chain_module()
     words = lib.nnis_chain_prompt_words(count, rows, width, heads, kv_heads, inner)
-    exchange = torch.empty(max(words, 1), dtype=torch.int32, device=x.device)
+    exchange = room(words)
+    if exchange is None:
+        return None
+    _dev(exchange, "chain_prompt exchange")
     out, last = torch.empty_like(x), torch.empty_like(x, dtype=dtype)
     _check(lib, lib.nnis_chain_prompt(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, _DTYPE_CODE[gain_dtype], float(eps), float(scale),
                                       x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),

@@ -14,7 +14,7 @@ import torch
 class LayerChain:
     def __init__(self, links: List[dict], rt):
         """``links``: what each run of the schedule says of itself (``PreNormBlock.chain_link``)."""
-        self.links = links
+        self.links, self.device = links, rt.device
         first = links[0]
         self.sizes = {name: first[name] for name in ("width", "heads", "kv_heads", "head_dim", "inner")}
         self.sizes["dtype"] = rt.dtype
@@ -24,6 +24,7 @@ class LayerChain:
         self._failed = self.failed.numpy()
         self._lost = 0
         self.tables: Dict[tuple, torch.Tensor] = {}  # the layers' pointers -> the same on the device
+        self.exchange: Optional[torch.Tensor] = None  # where a launch's blocks hand on their words; what lies there between launches is nothing
 
     @classmethod
     def of(cls, schedule_layers, rt) -> Optional["LayerChain"]:
@@ -75,18 +76,33 @@ class LayerChain:
             if torch.cuda.is_current_stream_capturing():
                 return None  # (the copy below does not belong into a graph; a graph's eager run comes first)
             while len(self.tables) >= 16:
-                self.tables.pop(next(iter(self.tables)))  # (graphs hold what they were captured with: ``held_tables``)
+                self.tables.pop(next(iter(self.tables)))  # (graphs hold what they were captured with: ``held``)
             table = self.tables[key] = torch.tensor(key, dtype=torch.int64).to(device)
         return table
+
+    def _room(self, words: int) -> Optional[torch.Tensor]:
+        """The exchange, of ``words`` 32-bit words at least: one for all launches, as they follow one another.  It grows by powers of two, and not
+        inside a capture (None; a graph's eager run comes first, and a graph holds the one that it was captured with: ``held``)."""
+        if self.exchange is None or self.exchange.numel() < words:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            self.exchange = torch.empty(1 << (words - 1).bit_length(), dtype=torch.int32, device=self.device)
+        return self.exchange
+
+    def held(self) -> List[torch.Tensor]:
+        """What a captured launch has the addresses of."""
+        return [*self.tables.values(), *([self.exchange] if self.exchange is not None else [])]
 
     def forward(self, x: torch.Tensor, ctx, views, plan, rt):
         """The stream, and what the last layer still adds to it; None where the launch cannot be made here."""
         table = self._table(views, x.device)
         if table is None:
             return None
-        ctx.chained = True
         tables = ctx.step_tables(rt, self.position.rotary(), views[0].block_table)
-        more = dict(self.sizes, gain_dtype=self.gain_dtype, eps=self.eps, scale=self.scale)
+        more = dict(self.sizes, room=self._room, gain_dtype=self.gain_dtype, eps=self.eps, scale=self.scale)
         if plan == "prompt":
-            return rt.ops.chain_prompt(table, len(self.links), x, tables, ctx.tok_pos, self.failed, **more)
-        return rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, **more)
+            done = rt.ops.chain_prompt(table, len(self.links), x, tables, ctx.tok_pos, self.failed, **more)
+        else:
+            done = rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, **more)
+        ctx.chained = done is not None
+        return done

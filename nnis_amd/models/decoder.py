@@ -88,13 +88,10 @@ class DecoderModel:
             part.check(rt)
 
     def held_buffers(self, rt):
-        """What the parts' kernels keep between calls and a captured step has baked in (``Part.held_buffers``)."""
-        return [buffer for part in self.parts() for buffer in part.held_buffers(rt)]
-
-    def held_tables(self, rt):
-        """The same of the model's own: what a launch through all layers reads their pointers from."""
+        """What the parts' kernels, and a launch through all layers, keep between calls and a captured step has baked in
+        (``Part.held_buffers``, ``LayerChain.held``)."""
         chain = self.layer_chain(rt)
-        return list(chain.tables.values()) if chain is not None else []
+        return [buffer for part in self.parts() for buffer in part.held_buffers(rt)] + (chain.held() if chain is not None else [])
 
     def lost_steps(self, rt) -> int:
         """How often kernels have reported that a step of this model is lost (``LayerChain.lost``)."""

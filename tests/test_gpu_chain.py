@@ -494,6 +494,38 @@ def test_what_lies_behind_a_sequence_does_not_matter(tmp_path, sizes, dtype, mon
         assert torch.equal(step(fill), want)
 
 
+def test_one_exchange_for_all_shapes(tmp_path):
+    """Steps of any shape, launched and captured, share the exchange: captured shapes do not add up. A larger shape gets a larger one, and
+    graphs go on with the one that they were captured with."""
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+
+    nnis_amd.write_random_model(str(tmp_path), _config(576, 9, 3, 1536, layers=6), 3)
+    engine = load_engine(str(tmp_path), dtype="bfloat16", max_tokens=2048)
+    rng = np.random.default_rng(3)
+    prompts = [rng.integers(0, 509, size=n).tolist() for n in (40, 1000, 100, 200, 400, 700)]
+
+    def step(prompt):
+        slot = engine.start_sequence()
+        out = [engine.step([StepEntry(slot, prompt, None)]), engine.step([StepEntry(slot, [7], None)])]
+        engine.end_sequence(slot)
+        return torch.cat(out)
+
+    want = [step(prompt) for prompt in prompts]
+    chain = engine.model.layer_chain(engine.rt)
+    largest = chain.exchange
+    words, needed = [], nnis_amd.kernels.ops.chain_module().nnis_chain_prompt_words(6, 1024, 576, 9, 3, 1536)
+    assert needed <= largest.numel() <= 2 * needed
+    for _ in range(3):  # captured, replayed; the shapes in turn
+        for prompt, first in zip(prompts, want):
+            assert torch.equal(step(prompt), first)
+            words.append(chain.exchange)
+    graphs = list(engine._prefill_graphs.graphs.values())
+    assert len(graphs) == len(prompts) and all(word is largest for word in words)
+    assert all(any(buffer is largest for buffer in graph.held) for graph in graphs)
+
+
 def test_sizes_and_words():
     """The exchange's size is 0 for what the launch refuses, and grows with what it holds."""
     from nnis_amd.kernels import ops
