@@ -424,22 +424,21 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
     load_values(f, v_base + page * v_stride, lane);
   }
   // What lies in a page behind the step's own key may be no number, and zero times that would be none: of the page that a wave
-  // has before its operands exist it goes here, where it waits in any case (30 layers of width 576, 1 row: 382 us, all of it below 393,
+  // has before its operands exist it goes here, where it waits in any case (30 layers of width 576, 1 row: 380 us, all of it below 393,
   // without 385).
   const int own_page = pos / kPageTokens, at_key = pos % kPageTokens;
-  u32x4 keep[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int key = 32 * h + 8 * g + 2 * w;
-      keep[h][w] = (key <= at_key ? 0xffffu : 0u) | (key + 1 <= at_key ? 0xffff0000u : 0u);
-    }
   auto drop_behind = [&]() {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      u32x4 keep;
 #pragma unroll
-      for (int t = 0; t < HD / 16; ++t) f.v[h][t] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, f.v[h][t]) & keep[h]);
+      for (int w = 0; w < 4; ++w) {
+        const int key = 32 * h + 8 * g + 2 * w;
+        keep[w] = (key <= at_key ? 0xffffu : 0u) | (key + 1 <= at_key ? 0xffff0000u : 0u);
+      }
+#pragma unroll
+      for (int t = 0; t < HD / 16; ++t) f.v[h][t] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, f.v[h][t]) & keep);
+    }
   };
   if (mine > 0 && first == own_page) drop_behind();
   if (kOne) ex.template gate<kOne>(here + a.q + ((first_head * (HD / 16) + item * 61 % (HD / 16)) * a.m + token) * 8, wave);
