@@ -7,9 +7,10 @@
 //
 // Why every wait ends: the stages of a block's operands are blocks of smaller numbers, and a die is handed its blocks in the order
 // of their numbers; so the unfinished block with the smallest number is on the chip, or its die is full of blocks of another
-// kernel.  Should two such launches ever fill a die each for the other, or a fault keep words away, a wait gives up after
-// kWaitTicks: it says so in `fail` (then all others leave too) and in `host_fail`, which the host reads before its next step;
-// what was not written stays kNone, which is no number, so nothing that hangs on it looks like a result.
+// kernel.  Two such launches could fill a die each for the other: those of one process take turns (models/chain.py, in_turn).  Should
+// another process's meet one, or a fault keep words away, a wait gives up after kWaitTicks: it says so in `fail` (then all others leave
+// too) and in `host_fail`, which the host reads before a step's tokens become the caller's and when a step begins (Engine.check_steps); what was
+// not written stays kNone, which is no number, and what hangs on it is none.
 #pragma once
 
 #include "common.h"

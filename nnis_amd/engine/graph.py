@@ -23,6 +23,7 @@ import torch
 import numpy as np
 
 from ..errors import KernelError
+from ..models.chain import in_turn
 from .batch import RecordedLists, StepContext
 
 BUCKETS = (1, 2, 4, 8, 12, 16, 24, 32, 48, 64)
@@ -107,7 +108,8 @@ class DecodeGraph:
         self.copied.record()
         if ids is None:
             self.meta[0, :count].copy_(ids_device[:count], non_blocking=True)
-        self.graph.replay()
+        with in_turn(self.engine.rt.device, self.ctx.chained):
+            self.graph.replay()
         return self.logits
 
 
@@ -273,7 +275,8 @@ class PrefillGraph:
 
     def run(self) -> torch.Tensor:
         """Replays the step on what the buffers hold; the rows returned view the graph's output buffer."""
-        self.graph.replay()
+        with in_turn(self.engine.rt.device, self.ctx.chained):
+            self.graph.replay()
         return self.logits
 
 

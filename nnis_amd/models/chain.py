@@ -6,9 +6,31 @@ through the layers' own kernels."""
 
 from __future__ import annotations
 
+import threading
+from contextlib import contextmanager
 from typing import Dict, List, Optional
 
 import torch
+
+_turn = threading.Lock()
+_last: Dict[int, torch.cuda.Stream] = {}  # by GPU: the stream of the last launch of all layers
+
+
+@contextmanager
+def in_turn(device: torch.device, launches: bool = True):
+    """Around a launch of all layers, or a replay that holds one: puts it behind the one before it on this GPU, whatever streams and
+    threads the two come from.  Two at once could each fill a die for the other, whose blocks then wait until they give up
+    (``csrc/chain.h``).  One stream's follow one another by themselves; inside a capture nothing runs."""
+    if not launches or torch.cuda.is_current_stream_capturing():
+        yield
+        return
+    with _turn:
+        stream = torch.cuda.current_stream(device)
+        last = _last.get(device.index)
+        if last is not None and last != stream:
+            stream.wait_stream(last)
+        _last[device.index] = stream
+        yield
 
 
 class LayerChain:
@@ -81,12 +103,15 @@ class LayerChain:
         return table
 
     def _room(self, words: int) -> Optional[torch.Tensor]:
-        """The exchange, of ``words`` 32-bit words at least: one for all launches, as they follow one another.  It grows by powers of two, and not
+        """The exchange, of ``words`` 32-bit words at least: one for all launches, as they follow one another (``in_turn``).  It grows by powers of two, and not
         inside a capture (None; a graph's eager run comes first, and a graph holds the one that it was captured with: ``held``)."""
         if self.exchange is None or self.exchange.numel() < words:
             if torch.cuda.is_current_stream_capturing():
                 return None
             self.exchange = torch.empty(1 << (words - 1).bit_length(), dtype=torch.int32, device=self.device)
+            self._exchange_of = torch.cuda.current_stream()
+        elif not torch.cuda.is_current_stream_capturing() and torch.cuda.current_stream() != self._exchange_of:
+            self.exchange.record_stream(torch.cuda.current_stream())  # (it may be let go while that stream's launch runs)
         return self.exchange
 
     def held(self) -> List[torch.Tensor]:
@@ -100,9 +125,10 @@ class LayerChain:
             return None
         tables = ctx.step_tables(rt, self.position.rotary(), views[0].block_table)
         more = dict(self.sizes, room=self._room, gain_dtype=self.gain_dtype, eps=self.eps, scale=self.scale)
-        if plan == "prompt":
-            done = rt.ops.chain_prompt(table, len(self.links), x, tables, ctx.tok_pos, self.failed, **more)
-        else:
-            done = rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, **more)
+        with in_turn(self.device):
+            if plan == "prompt":
+                done = rt.ops.chain_prompt(table, len(self.links), x, tables, ctx.tok_pos, self.failed, **more)
+            else:
+                done = rt.ops.chain(table, len(self.links), x, tables, ctx.tok_pos, plan, self.failed, **more)
         ctx.chained = done is not None
         return done

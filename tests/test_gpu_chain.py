@@ -526,6 +526,63 @@ def test_one_exchange_for_all_shapes(tmp_path):
     assert all(any(buffer is largest for buffer in graph.held) for graph in graphs)
 
 
+@pytest.mark.parametrize("threads", [False, True])
+def test_launches_on_two_streams_take_turns(tmp_path, threads):
+    """Two engines on streams of their own, over one model and over two, from one thread and from two: neither waits for what the other's
+    launch keeps off the chip, and each has the bits that it has alone."""
+    import threading
+
+    import nnis_amd
+    from nnis_amd.api import load_engine
+    from nnis_amd.engine.batch import StepEntry
+    from nnis_amd.engine.step import Engine
+
+    nnis_amd.write_random_model(str(tmp_path), _config(576, 9, 3, 1536, layers=8), 3)
+    first, other = (load_engine(str(tmp_path), dtype="bfloat16", max_tokens=1024) for _ in range(2))
+    engines = [first, Engine(first.model, first.rt, max_tokens=1024), other]
+    rng = np.random.default_rng(11)
+    prompts = [rng.integers(0, 509, size=n).tolist() for n in (150, 90, 33)]
+
+    def steps(engine, prompt):
+        slot, out = engine.start_sequence(), []
+        for number in range(25):
+            if number % 8 == 0:  # (launched, captured, replayed)
+                engine.truncate(slot, 0)
+                out.append(engine.step([StepEntry(slot, prompt, None)]))
+            out.append(engine.step([StepEntry(slot, [number], None)]))
+            yield
+        engine.end_sequence(slot)
+        yield torch.cat(out)
+
+    def alone(engine, prompt):
+        *_, out = steps(engine, prompt)
+        return out
+
+    want = [alone(engine, prompt) for engine, prompt in zip(engines, prompts)]
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream() for _ in engines], [None] * len(engines)
+    if threads:
+        def run(index):
+            with torch.cuda.stream(streams[index]):
+                got[index] = alone(engines[index], prompts[index])
+
+        workers = [threading.Thread(target=run, args=(index,)) for index in range(len(engines))]
+        for worker in workers:
+            worker.start()
+        for worker in workers:
+            worker.join()
+    else:
+        runs = [steps(engine, prompt) for engine, prompt in zip(engines, prompts)]
+        for _ in range(26):
+            for index, run in enumerate(runs):
+                with torch.cuda.stream(streams[index]):
+                    got[index] = next(run)
+    torch.cuda.synchronize()
+    for engine, a, b in zip(engines, got, want):
+        assert torch.equal(a, b)
+        engine.check_steps()
+
+
 def test_sizes_and_words():
     """The exchange's size is 0 for what the launch refuses, and grows with what it holds."""
     from nnis_amd.kernels import ops
