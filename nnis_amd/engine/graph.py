@@ -23,7 +23,7 @@ import torch
 import numpy as np
 
 from ..errors import KernelError
-from ..models.chain import in_turn
+from ..models.chain import in_turn, turns_waited_for
 from .batch import RecordedLists, StepContext
 
 BUCKETS = (1, 2, 4, 8, 12, 16, 24, 32, 48, 64)
@@ -70,10 +70,11 @@ class DecodeGraph:
         # once eagerly on a side stream (loads every kernel), then the capture itself
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            self._forward()
-        torch.cuda.current_stream().wait_stream(side)
-        torch.cuda.synchronize()
+        with turns_waited_for(self.engine.rt.device):
+            with torch.cuda.stream(side):
+                self._forward()
+            torch.cuda.current_stream().wait_stream(side)
+            torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
         # A graph that the cycle collector destroys while another is being captured aborts the process: the
         # collector stays off until the capture ends.  (Graphs hold their engine weakly, so an engine that is

@@ -12,7 +12,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-_turn = threading.Lock()
+_turn = threading.RLock()
 _last: Dict[int, torch.cuda.Stream] = {}  # by GPU: the stream of the last launch of all layers
 
 
@@ -31,6 +31,14 @@ def in_turn(device: torch.device, launches: bool = True):
             stream.wait_stream(last)
         _last[device.index] = stream
         yield
+
+
+@contextmanager
+def turns_waited_for(device: torch.device):
+    """Around launches at whose end the caller waits for the whole GPU: nobody has to get behind them afterwards."""
+    with _turn:
+        yield
+        _last.pop(device.index, None)
 
 
 class LayerChain:
