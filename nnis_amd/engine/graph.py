@@ -60,6 +60,7 @@ class DecodeGraph:
         self.graph = None
         self.logits = None
         self.held = []  # memory the parts' kernels keep between calls, whose addresses the capture baked in: held as long as the graph
+        self.held_of_launches = []  # ... and what a launch through all layers does
 
     def _forward(self) -> torch.Tensor:
         engine = self.engine
@@ -92,6 +93,7 @@ class DecodeGraph:
         # holds what the parts name (``Part.held_buffers``): whatever its keeper does later, a replay never writes
         # into memory that has gone back to the allocator.
         self.held = list(self.engine.model.held_buffers(self.engine.rt))
+        self.held_of_launches = list(self.engine.model.held_of_launches(self.engine.rt))
 
     def run(self, ids, slots: Sequence[int], positions: Sequence[int], ids_device: torch.Tensor = None) -> torch.Tensor:
         """``ids``: the step's token ids, or None when they are on the device
@@ -189,7 +191,7 @@ class PrefillGraph:
         self.copied.record()
         self.graph = None
         self.logits = None
-        self.held = []
+        self.held, self.held_of_launches = [], []
         self.chained = False  # whether the first run was (the capture's context says it of the replays)
         self._lay_out({})
 
@@ -266,6 +268,7 @@ class PrefillGraph:
                 self.logits = self._forward()
             self.graph = graph
             self.held = list(self.engine.model.held_buffers(self.engine.rt))
+            self.held_of_launches = list(self.engine.model.held_of_launches(self.engine.rt))
         except KernelError:
             # a part that cannot run under capture: the shape goes on being launched
             self.graph = self.logits = None

@@ -778,14 +778,16 @@ def chain(layers: torch.Tensor, count: int, x: torch.Tensor, tables: StepTables,
         raise KernelError(f"chain: rows {tuple(x.shape)} {x.dtype}, tables for {tables.tokens} tokens, {layers.numel()} pointers do not fit {count} layers of {width}")
     lib = chain_module()
     words, run_words = chain_words(count, rows, width, heads, kv_heads, inner, runs, dtype)
-    exchange = room(words + run_words)
+    exchange = room(words)
     if exchange is None:
         return None
     _dev(exchange, "chain exchange")
-    runs_at = exchange.data_ptr() + 4 * words if run_words else None  # (the words are whole lines)
+    partial = decode_scratch(x.device, run_words) if run_words else None  # (as the split decode attention's)
+    if partial is not None and not torch.cuda.is_current_stream_capturing():
+        partial.record_stream(torch.cuda.current_stream())  # (launches take turns on streams of their own, and it may be let go meanwhile)
     out, last = torch.empty_like(x), torch.empty_like(x, dtype=dtype)
     tail = (float(eps), float(scale), x.data_ptr(), out.data_ptr(), last.data_ptr(), tables.cos.data_ptr(), tables.sin.data_ptr(), tok_pos.data_ptr(),
-            tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, runs_at, run_words, failed.data_ptr(),
+            tables.page.data_ptr(), tables.pages.data_ptr(), tables.pages.shape[1], exchange.data_ptr(), words, _ptr(partial), run_words, failed.data_ptr(),
             _stream())
     if dtype == torch.float32:
         _check(lib, lib.nnis_chain_f32(layers.data_ptr(), count, rows, width, heads, kv_heads, head_dim, inner, runs, *tail))

@@ -88,10 +88,13 @@ class DecoderModel:
             part.check(rt)
 
     def held_buffers(self, rt):
-        """What the parts' kernels, and a launch through all layers, keep between calls and a captured step has baked in
-        (``Part.held_buffers``, ``LayerChain.held``)."""
+        """What the parts' kernels keep between calls and a captured step has baked in (``Part.held_buffers``)."""
+        return [buffer for part in self.parts() for buffer in part.held_buffers(rt)]
+
+    def held_of_launches(self, rt):
+        """The same of the model's own launches through all layers (``LayerChain.held``)."""
         chain = self.layer_chain(rt)
-        return [buffer for part in self.parts() for buffer in part.held_buffers(rt)] + (chain.held() if chain is not None else [])
+        return chain.held() if chain is not None else []
 
     def lost_steps(self, rt) -> int:
         """How often kernels have reported that a step of this model is lost (``LayerChain.lost``)."""

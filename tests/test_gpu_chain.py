@@ -523,7 +523,7 @@ def test_one_exchange_for_all_shapes(tmp_path):
             words.append(chain.exchange)
     graphs = list(engine._prefill_graphs.graphs.values())
     assert len(graphs) == len(prompts) and all(word is largest for word in words)
-    assert all(any(buffer is largest for buffer in graph.held) for graph in graphs)
+    assert all(any(buffer is largest for buffer in graph.held_of_launches) for graph in graphs)
 
 
 @pytest.mark.parametrize("threads", [False, True])
