@@ -526,8 +526,9 @@ def test_one_exchange_for_all_shapes(tmp_path):
     assert all(any(buffer is largest for buffer in graph.held_of_launches) for graph in graphs)
 
 
+@pytest.mark.parametrize("lengths", [(150, 90, 33), (700, 570, 950)])  # (keys in one run, and in several in the scratch that all have)
 @pytest.mark.parametrize("threads", [False, True])
-def test_launches_on_two_streams_take_turns(tmp_path, threads):
+def test_launches_on_two_streams_take_turns(tmp_path, threads, lengths):
     """Two engines on streams of their own, over one model and over two, from one thread and from two: neither waits for what the other's
     launch keeps off the chip, and each has the bits that it has alone."""
     import threading
@@ -541,7 +542,7 @@ def test_launches_on_two_streams_take_turns(tmp_path, threads):
     first, other = (load_engine(str(tmp_path), dtype="bfloat16", max_tokens=1024) for _ in range(2))
     engines = [first, Engine(first.model, first.rt, max_tokens=1024), other]
     rng = np.random.default_rng(11)
-    prompts = [rng.integers(0, 509, size=n).tolist() for n in (150, 90, 33)]
+    prompts = [rng.integers(0, 509, size=n).tolist() for n in lengths]
 
     def steps(engine, prompt):
         slot, out = engine.start_sequence(), []
