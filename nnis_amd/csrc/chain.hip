@@ -47,9 +47,10 @@ struct ChainArgs {
   int max_pages;
   unsigned *words, *run_words;  // (the runs lie apart: in the scratch that the split decode attention has)
   unsigned words_bytes, run_bytes, layer_words, layer_runs;  // of a tile, as m: at most 16 of the step's rows
-  // where a layer's words lie: the stream's records before the attention and before the feed-forward; queries, keys, values;
-  // attention rows; gated rows
-  unsigned stream1, stream2, q, k, v, attn, act;
+  // where a layer's words lie: the stream's rows before the attention and before the feed-forward, as operands and in 32 bits; queries,
+  // keys, values; attention rows; gated rows
+  unsigned stream1, stream2, plain1, plain2, q, k, v, attn, act;
+  unsigned strip_words;  // of the stream's rows as the next product takes them
   int n_strip;        // strips of the stream
   int n_qkv, n_att, n_comb, n_out, n_gate, n_down;  // blocks of a stage for a tile (the last may have fewer of the attention's two)
   int n_att_all, n_comb_all;
@@ -57,11 +58,12 @@ struct ChainArgs {
 };
 
 // Rows lie by strips of 16 channels: [strip][row][16 bfloat16], 32 bytes that one block writes and that a lane's two pieces of an
-// operand are.  The stream's rows are records of 128 bytes, [strip][row]: 16 channels times the next norm's gain in bfloat16, the
-// strip's part of the row's sum of squares (four times), 16 unused bytes, and the 16 channels in 32 bits: two full stores, and a
-// reader's operand and its share of the sum from one line.  (Parts of 4 bytes from 36 blocks in one line took a reader 1.2 us more.)
-constexpr int kRecord = 32;                 // words
-constexpr int kRecordSum = 8, kRecordStream = 16;
+// operand are.  A strip of the stream's rows, which is times the next norm's gain, has the rows' parts of their sums of squares
+// behind it (a word a row) and begins on 64 bytes; the stream itself, [strip][row][16], lies apart.  (In one record of 128 bytes a row, every
+// piece that a product's block read was a line of its own: a look at 8 rows was 32 lines a load, and the blocks of a stage had their operands
+// 1.4 us after the last of them was written, where rows side by side take 0.7.  Parts of 36 blocks in one line took a reader 1.2 us more.)
+constexpr int kRowWords = 8;     // of a strip of an operand
+constexpr int kPlainWords = 16;  // ... of the stream
 
 __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
 
@@ -110,10 +112,10 @@ struct Product {
     if (wave < parts) ask(0);
   }
   // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
-  // every chunk with the lane's part of its row's sum of squares, if SUM: the strips are then the stream's records.
+  // every chunk with the lane's part of its row's sum of squares, at byte `sum_at` of the strip, if SUM.
   template <bool SUM, typename Sum>
-  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, Sum sum) {
-    const unsigned at = row_at + lane / 16 * stride;
+  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, unsigned sum_at, Sum sum) {
+    const unsigned at = row_at + lane / 16 * stride, sums = sum_at + lane / 16 * stride;
     for (int d0 = 0; wave < parts && wave + parts * d0 < chunks; d0 += STEPS / V) {
       if (d0 > 0) ask(d0);
 #pragma unroll
@@ -123,7 +125,7 @@ struct Product {
         unsigned part[XB];
         auto step = [&](int d) { return (unsigned)min(chunk(d0, b + d), chunks - 1) * 4 * stride; };
         auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
-        if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{at + kRecordSum * 4, step(i)}; });
+        if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{sums, step(i)}; });
         else ex.take(v, pieces);
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
@@ -141,14 +143,17 @@ struct Product {
   }
 };
 
-// a row's 16 channels of a strip into its record, by the wave that ends the strip: lane (row, g) has four of them
-__device__ __forceinline__ void put_record(const Exchange& ex, unsigned word, int g, f32x4 v, f32x4 gain, float sum) {
-  const unsigned lo = marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), hi = marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]));
-  const unsigned next_lo = __shfl_xor(lo, 16, kWave), next_hi = __shfl_xor(hi, 16, kWave), part = marked(sum);
-  // lanes 0 and 2 of a row store 8 channels each, lanes 1 and 3 the sum
-  const u32x4 first = g % 2 == 0 ? (u32x4){lo, hi, next_lo, next_hi} : (u32x4){part, part, part, part};
-  ex.put(word + (g % 2 == 0 ? 2 * g : kRecordSum + 2 * (g - 1)), first);
-  ex.put(word + kRecordStream + 4 * g, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+// a row's 16 channels of a strip by the wave that ends it, lane (row, g) has four of them: as the next product's operand and its part of the sum
+// of squares, the strip at word `word`, and in 32 bits at word `plain`
+__device__ __forceinline__ void put_row(const Exchange& ex, unsigned word, unsigned plain, int m, int row, int g, f32x4 v, f32x4 gain, float sum) {
+  ex.put(word + row * kRowWords + 2 * g, (u32x2){marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]))});
+  if (g == 0) ex.put(word + m * kRowWords + row, marked(sum));
+  ex.put(plain + row * kPlainWords + 4 * g, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+}
+
+// a word of some row of the stream's strips at `first_word`
+__device__ __forceinline__ unsigned a_row(const ChainArgs& a, unsigned first_word, int some) {
+  return first_word + some / a.m % a.n_strip * a.strip_words + some % a.m * kRowWords;
 }
 
 // units that a block of the products takes: wide models' blocks two, whose rows they then read once
@@ -196,14 +201,14 @@ __device__ __forceinline__ bool add_parts(Shared<WAVES>& s, const f32x4 (&acc)[V
   return true;
 }
 
-// a product with a row that a norm prepared, from the records at word `first_word`; `sums` and the row's scale in the waves that end a unit
+// a product with a row that a norm prepared, from the strips at word `first_word`; `sums` and the row's scale in the waves that end a unit
 template <int WAVES, int UNITS, int NACC, int V, typename P>
 __device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, P& p, unsigned first_word, int row, int wave, int lane,
                                              f32x4 (&sums)[NACC], float& scale) {
   // The row's sum of squares is added up as the layers' kernels do: four waves' rows (up to 64 parts) chunk by chunk by one wave,
   // eight waves' each wave's own chunks first.
   float ss = 0.0f;
-  p.template run<true>(ex, (first_word + row * kRecord) * 4, a.m * kRecord * 4, [&](int c, float part) {
+  p.template run<true>(ex, (first_word + row * kRowWords) * 4, a.strip_words * 4, (first_word + a.m * kRowWords + row) * 4, [&](int c, float part) {
     if constexpr (WAVES == 4) s.product.ss[c][lane] = part;
     else ss += part;
   });
@@ -235,7 +240,7 @@ template <typename P>
 __device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Exchange& ex, Shared<8>& s, P& p, unsigned first_word, int row, int wave, int lane,
                                                     f32x4 (&sums)[2], float& scale) {
   float ss = 0.0f;
-  p.template run<true>(ex, (first_word + row * kRecord) * 4, a.m * kRecord * 4, [&](int, float part) { ss += part; });
+  p.template run<true>(ex, (first_word + row * kRowWords) * 4, a.strip_words * 4, (first_word + a.m * kRowWords + row) * 4, [&](int, float part) { ss += part; });
   ss += __shfl_xor(ss, 16, kWave);
   ss += __shfl_xor(ss, 32, kWave);
   s.product.ss[wave][lane] = ss;
@@ -255,7 +260,7 @@ __device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Ex
   return true;
 }
 
-// A row of the embedding into the first layer's records.  Of a step of more than 16 rows it is normed as the layers' kernel of its own for
+// A row of the embedding into the first layer's strips.  Of a step of more than 16 rows it is normed as the layers' kernel of its own for
 // that does it, a lane per 4 of 256 channels, and its product needs no scale.
 __device__ __forceinline__ void normed_entry_stage(const ChainArgs& a, const Exchange& ex, float& shared_scale, int row) {
   const float* x = a.x + (size_t)row * a.width;
@@ -273,14 +278,14 @@ __device__ __forceinline__ void normed_entry_stage(const ChainArgs& a, const Exc
   const float scale = shared_scale;
   for (int c = threadIdx.x * 4; c < a.width; c += blockDim.x * 4) {
     const f32x4 v = *(const f32x4*)(x + c), normed = (v * scale) * four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
-    const unsigned word = a.stream1 + (c / 16 * a.m + row) * kRecord, four = c % 16 / 4;
-    ex.put(word + 2 * four, (u32x2){marked2((bf16_t)normed[0], (bf16_t)normed[1]), marked2((bf16_t)normed[2], (bf16_t)normed[3])});
-    if (four == 0) ex.put(word + kRecordSum, marked(0.0f));
-    ex.put(word + kRecordStream + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+    const unsigned strip = c / 16, word = a.stream1 + strip * a.strip_words, four = c % 16 / 4;
+    ex.put(word + row * kRowWords + 2 * four, (u32x2){marked2((bf16_t)normed[0], (bf16_t)normed[1]), marked2((bf16_t)normed[2], (bf16_t)normed[3])});
+    if (four == 0) ex.put(word + a.m * kRowWords + row, marked(0.0f));
+    ex.put(a.plain1 + (strip * a.m + row) * kPlainWords + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
   }
 }
 
-// A row of the embedding into the first layer's records.  Its sum of squares is one part, added up as the layers' kernel for a row
+// A row of the embedding into the first layer's strips.  Its sum of squares is one part, added up as the layers' kernel for a row
 // that no norm has prepared does: a lane per (part of K, 16 of a chunk's 64 channels).
 template <int WAVES>
 __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int row) {
@@ -306,10 +311,8 @@ __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& 
   for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
     const f32x4 v = *(const f32x4*)(x + c);
     const f32x4 gain = four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
-    const unsigned word = a.stream1 + (c / 16 * a.m + row) * kRecord, four = c % 16 / 4;
-    ex.put(word + 2 * four, (u32x2){marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]))});
-    if (four == 0) ex.put(word + kRecordSum, marked(c == 0 ? sum : 0.0f));
-    ex.put(word + kRecordStream + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+    const unsigned strip = c / 16;
+    put_row(ex, a.stream1 + strip * a.strip_words, a.plain1 + strip * a.m * kPlainWords, a.m, row, c % 16 / 4, v, gain, c == 0 ? sum : 0.0f);
   }
 }
 
@@ -329,7 +332,7 @@ __device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex
   const int row = r < a.m ? r : a.m - 1, ends = unit * kUnits + (wave < kUnits ? wave : 0), head = ends / 2, f0 = ends % 2 * 16;
   const f32x4 c = *(const f32x4*)(a.tok_cos + row * (HD / 2) + f0 + 4 * g), sn = *(const f32x4*)(a.tok_sin + row * (HD / 2) + f0 + 4 * g);
   const int pos = a.tok_pos[row], page = a.tok_page[row];
-  ex.template gate<kOne>(here + a.stream1 + unit * 61 % (a.m * a.n_strip) * kRecord, wave);
+  ex.template gate<kOne>(a_row(a, here + a.stream1, unit * 61), wave);
   f32x4 sums[2];
   float scale;
   if (!run_prepared<WAVES, kUnits, 2, kParts>(a, ex, s, p, here + a.stream1, row, wave, lane, sums, scale)) return;
@@ -442,7 +445,7 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   };
   if (mine > 0 && first == own_page) drop_behind();
   if (kOne) ex.template gate<kOne>(here + a.q + ((first_head * (HD / 16) + item * 61 % (HD / 16)) * a.m + token) * 8, wave);
-  else ex.template gate<kOne>(here + a.stream1 + item * 61 % (a.m * a.n_strip) * kRecord, wave);
+  else ex.template gate<kOne>(a_row(a, here + a.stream1, item * 61), wave);
   // Queries and the step's own key and value in one load of the wave (8 lanes a head's row, [head][strip][row]: two pieces a
   // strip), and from there through LDS.
   bf16x8* heads_lds = s.attention.heads[wave];
@@ -670,8 +673,8 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   else ex.template gate<kOne>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
   // (the stream is two stages old and more: it is there)
   u32x4 held[1];
-  if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + (strip * a.m + row) * kRecord + kRecordStream + 4 * g) * 4, 0}; });
-  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32, [](int, float) {});
+  if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.plain2 : a.plain1) + (strip * a.m + row) * kPlainWords + 4 * g) * 4, 0}; });
+  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32, 0, [](int, float) {});
   f32x4 sums[1];
   if constexpr (PAIRED) {
     const f32x4 even[1][1] = {{p.acc[0][0]}};
@@ -704,7 +707,7 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   sq += __shfl_xor(sq, 32, kWave);
   if (r >= a.m) return;
   if (!DOWN && layer + 1 == a.layer_count) *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
-  put_record(ex, next + (DOWN ? a.stream1 : a.stream2) + (strip * a.m + row) * kRecord, g, v, gain, sq);
+  put_row(ex, next + (DOWN ? a.stream1 : a.stream2) + strip * a.strip_words, next + (DOWN ? a.plain1 : a.plain2) + strip * a.m * kPlainWords, a.m, row, g, v, gain, sq);
 }
 
 // HALVES: eight waves that cut K four ways for each of the block's two units, as the layers' kernel does for this many strips
@@ -715,7 +718,7 @@ __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& e
   const unsigned here = layer * a.layer_words;
   constexpr int kUnits = units_of<WAVES>();
   const int unit = block * kUnits + (HALVES ? wave / 4 : wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
-  const unsigned one = here + a.stream2 + block * 61 % (a.m * a.n_strip) * kRecord;
+  const unsigned one = a_row(a, here + a.stream2, block * 61);
   f32x4 sums[2];
   float scale;
   if constexpr (HALVES) {
@@ -814,8 +817,11 @@ unsigned lay_out(ChainArgs& a) {
     at += (words + 31) / 32 * 32;
   };
   const unsigned m = a.m, strips = a.width / 16;
-  place(a.stream1, m * strips * kRecord);
-  place(a.stream2, m * strips * kRecord);
+  a.strip_words = ((kRowWords + 1) * m + 15) / 16 * 16;
+  place(a.stream1, strips * a.strip_words);
+  place(a.stream2, strips * a.strip_words);
+  place(a.plain1, m * strips * kPlainWords);
+  place(a.plain2, m * strips * kPlainWords);
   place(a.q, m * a.heads * (HD / 2));
   place(a.k, m * a.kv_heads * (HD / 2));
   place(a.v, m * a.kv_heads * (HD / 2));
