@@ -38,7 +38,7 @@ struct ChainArgs {
   // how many ways K is cut (the first layer's queries, keys and values; the others'; output, gate/up, down), and the waves that
   // share a run's pages
   int parts_first, parts_qkv, parts_out, parts_gate, parts_down, page_waves, down_paired;
-  float eps, scale_log2;
+  float eps, scale_log2, inv_width;
   const float* x;  // [m, width]
   float* x_out;    // [m, width]: the stream behind the last attention
   bf16_t* y_out;   // [m, width]: what the last feed-forward adds to it
@@ -59,11 +59,84 @@ struct ChainArgs {
 
 // Rows lie by strips of 16 channels: [strip][row][16 bfloat16], 32 bytes that one block writes and that a lane's two pieces of an
 // operand are.  A strip of the stream's rows, which is times the next norm's gain, has the rows' parts of their sums of squares
-// behind it (a word a row) and begins on 64 bytes; the stream itself, [strip][row][16], lies apart.  (In one record of 128 bytes a row, every
+// behind it (a word a row, 4, 8 or 16 of them) and begins on 64 bytes; the stream itself, [strip][row][16], lies apart.  (In one record of 128 bytes a row, every
 // piece that a product's block read was a line of its own: a look at 8 rows was 32 lines a load, and the blocks of a stage had their operands
 // 1.4 us after the last of them was written, where rows side by side take 0.7.  Parts of 36 blocks in one line took a reader 1.2 us more.)
 constexpr int kRowWords = 8;     // of a strip of an operand
 constexpr int kPlainWords = 16;  // ... of the stream
+__host__ __device__ constexpr int sum_words(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
+
+// What stands between a stage's last operand and its words is a chain of instructions of one wave, four cycles each and more: the
+// ends of the products are kept short.  A lane's partner 16 and 32 lanes on (a row of another lane group) by register, not by LDS:
+__device__ __forceinline__ float sum_16_apart(float v) {
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+}
+__device__ __forceinline__ float sum_32_apart(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+}
+template <int CONTROL>  // a lane of the same 16
+__device__ __forceinline__ float of_row(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CONTROL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ unsigned pack2(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
+}
+__device__ __forceinline__ unsigned marked2(unsigned packed) { return packed == kNone ? 0x7fc07fc0u : packed; }
+
+// Which of a result's elements (16 channels of up to 16 rows) a lane ends.  The matrix instruction leaves a lane four channels of a row;
+// of up to 8 and 4 rows half and three quarters of the lanes would have none, and from LDS each takes two or one.
+template <int ROWS>
+struct Ends {
+  static constexpr int kEach = ROWS <= 4 ? 1 : ROWS <= 8 ? 2 : 4;
+  int row, first, from;  // the first of its channels; the lane that had them
+  __device__ __forceinline__ explicit Ends(int lane)
+      : row(lane % 16 / (4 / kEach)), first(lane / 16 * 4 + lane % (4 / kEach) * kEach), from(lane / 16 * 16 + row) {}
+};
+template <int N>
+struct Floats {
+  float v[N];
+  __device__ __forceinline__ float& operator[](int e) { return v[e]; }
+  __device__ __forceinline__ float operator[](int e) const { return v[e]; }
+};
+template <int N>
+__device__ __forceinline__ Floats<N> load_floats(const float* p) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  Floats<N> out;
+  if constexpr (N == 4) {
+    const f32x4 v = *(const f32x4*)p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = v[e];
+  } else if constexpr (N == 2) {
+    const f32x2 v = *(const f32x2*)p;
+    out[0] = v[0];
+    out[1] = v[1];
+  } else {
+    out[0] = *p;
+  }
+  return out;
+}
+// a lane's channels in 16 bits, two a word: words[0 .. 1], of which `packed_words` are the lane's (with one channel a lane every other lane has a word)
+template <int N>
+__device__ __forceinline__ void pack_row(const Floats<N>& v, unsigned (&words)[2]) {
+  if constexpr (N == 1) words[0] = pack2(v[0], of_row<0xb1>(v[0]));
+  else words[0] = pack2(v[0], v[1]);
+  words[1] = N == 4 ? pack2(v[N == 4 ? 2 : 0], v[N == 4 ? 3 : 0]) : 0;
+}
+template <int N>
+__device__ __forceinline__ void put_packed(const Exchange& ex, unsigned word, int first, const unsigned (&words)[2]) {
+  if constexpr (N == 4) ex.put(word + first / 2, (u32x2){marked2(words[0]), marked2(words[1])});
+  else if (N == 2 || first % 2 == 0) ex.put(word + first / 2, marked2(words[0]));
+}
+template <int N>
+__device__ __forceinline__ void put_floats(const Exchange& ex, unsigned word, const Floats<N>& v) {
+  if constexpr (N == 4) ex.put(word, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+  else if constexpr (N == 2) ex.put(word, (u32x2){marked(v[0]), marked(v[1])});
+  else ex.put(word, marked(v[0]));
+}
 
 __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
 
@@ -113,20 +186,26 @@ struct Product {
   }
   // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
   // every chunk with the lane's part of its row's sum of squares, at byte `sum_at` of the strip, if SUM.
-  template <bool SUM, typename Sum>
-  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, unsigned sum_at, Sum sum) {
+  // MORE further loads go with the first trip's, whose offsets `ask_more` gives; `more` has what they brought.
+  template <bool SUM, int MORE, typename Sum, typename AskMore>
+  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, unsigned sum_at, Sum sum, u32x4 (&more)[MORE > 0 ? MORE : 1], AskMore ask_more) {
+    static_assert(!SUM || MORE == 0, "one or the other");
     const unsigned at = row_at + lane / 16 * stride, sums = sum_at + lane / 16 * stride;
     for (int d0 = 0; wave < parts && wave + parts * d0 < chunks; d0 += STEPS / V) {
       if (d0 > 0) ask(d0);
 #pragma unroll
       for (int b = 0; b < STEPS; b += XB) {
         if (XB <= STEPS / V && chunk(d0, b) >= chunks) continue;  // (no step of the trip has a chunk)
-        u32x4 v[XB * 2];
+        u32x4 v[XB * 2 + MORE];
         unsigned part[XB];
         auto step = [&](int d) { return (unsigned)min(chunk(d0, b + d), chunks - 1) * 4 * stride; };
-        auto pieces = [&](int i) { return At{at + i % 2 * 16, step(i / 2)}; };
+        auto pieces = [&](int i) { return i < XB * 2 ? At{at + i % 2 * 16, step(i / 2)} : ask_more(i - XB * 2); };
         if constexpr (SUM) ex.take(v, pieces, part, [&](int i) { return At{sums, step(i)}; });
         else ex.take(v, pieces);
+        if constexpr (MORE > 0) {
+#pragma unroll
+          for (int i = 0; i < MORE; ++i) more[i] = v[XB * 2 + i];
+        }
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
           const int c = chunk(d0, b + d);
@@ -143,14 +222,6 @@ struct Product {
   }
 };
 
-// a row's 16 channels of a strip by the wave that ends it, lane (row, g) has four of them: as the next product's operand and its part of the sum
-// of squares, the strip at word `word`, and in 32 bits at word `plain`
-__device__ __forceinline__ void put_row(const Exchange& ex, unsigned word, unsigned plain, int m, int row, int g, f32x4 v, f32x4 gain, float sum) {
-  ex.put(word + row * kRowWords + 2 * g, (u32x2){marked2((bf16_t)(v[0] * gain[0]), (bf16_t)(v[1] * gain[1])), marked2((bf16_t)(v[2] * gain[2]), (bf16_t)(v[3] * gain[3]))});
-  if (g == 0) ex.put(word + m * kRowWords + row, marked(sum));
-  ex.put(plain + row * kPlainWords + 4 * g, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
-}
-
 // a word of some row of the stream's strips at `first_word`
 __device__ __forceinline__ unsigned a_row(const ChainArgs& a, unsigned first_word, int some) {
   return first_word + some / a.m % a.n_strip * a.strip_words + some % a.m * kRowWords;
@@ -164,17 +235,18 @@ constexpr int units_of() { return WAVES == 8 ? 2 : 1; }
 template <int WAVES, bool DOWN>
 constexpr int into_units_of() { return DOWN ? 1 : units_of<WAVES>(); }
 
-template <int WAVES>
+template <int WAVES, int ROWS>
 struct Shared {
-  static constexpr int kSums = WAVES == 4 ? 16 : WAVES;  // four waves: a sum a chunk of K; eight: one a wave
   union {
     struct {
       float acc[WAVES][4][kWave][4];
-      float ss[kSums][kWave];
+      float ss[WAVES == 4 ? 1 : WAVES][kWave];  // eight waves: a row's part from each
+      __attribute__((aligned(16))) unsigned parts[WAVES == 4 ? sum_words(ROWS) * kWave : 1];  // four waves: [strip][row]
+      float scale[16];
     } product;
     struct {
-      __attribute__((aligned(16))) float o[WAVES][4][HD];
-      float m[WAVES][4], l[WAVES][4][4];
+      __attribute__((aligned(16))) float o[WAVES][4][HD + 4];  // a head's outputs, then its sum's four parts
+      float m[WAVES][4];
       bf16x8 heads[WAVES][kWave];
       __attribute__((aligned(16))) bf16_t stage[WAVES][4][kPageTokens + 8];
     } attention;
@@ -183,85 +255,127 @@ struct Shared {
 };
 
 // The parts of K added up, in their order: of a block's UNITS units of NACC strips, unit u's in wave u; false for waves that have none.
-template <int WAVES, int UNITS, int NACC, int V>
-__device__ __forceinline__ bool add_parts(Shared<WAVES>& s, const f32x4 (&acc)[V][UNITS * NACC], f32x4 (&sums)[NACC], int wave, int lane) {
+template <int WAVES, int ROWS, int UNITS, int NACC, int V>
+__device__ __forceinline__ bool add_parts(Shared<WAVES, ROWS>& s, const f32x4 (&acc)[V][UNITS * NACC], Floats<Ends<ROWS>::kEach> (&sums)[NACC], int wave, int lane) {
+  constexpr int kEach = Ends<ROWS>::kEach;
   static_assert(V * UNITS * NACC <= 4 && (V == 1 || UNITS == 1), "room for the sums");
 #pragma unroll
   for (int v = 0; v < V; ++v)
 #pragma unroll
     for (int j = 0; j < UNITS * NACC; ++j) *(f32x4*)s.product.acc[wave][v * UNITS * NACC + j][lane] = acc[v][j];
+  const Ends<ROWS> ends(lane);
   __syncthreads();
   if (wave >= UNITS) return false;
 #pragma unroll
   for (int j = 0; j < NACC; ++j) {
-    sums[j] = *(const f32x4*)s.product.acc[0][wave * NACC + j][lane];
+    auto part_at = [&](int part) { return load_floats<kEach>(&s.product.acc[part % WAVES][part / WAVES * UNITS * NACC + wave * NACC + j][ends.from][ends.first % 4]); };
+    sums[j] = part_at(0);
 #pragma unroll
-    for (int part = 1; part < WAVES * V; ++part) sums[j] += *(const f32x4*)s.product.acc[part % WAVES][part / WAVES * UNITS * NACC + wave * NACC + j][lane];
+    for (int part = 1; part < WAVES * V; ++part) {
+      const Floats<kEach> more = part_at(part);
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) sums[j][e] += more[e];
+    }
   }
   return true;
 }
 
 // a product with a row that a norm prepared, from the strips at word `first_word`; `sums` and the row's scale in the waves that end a unit
-template <int WAVES, int UNITS, int NACC, int V, typename P>
-__device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, P& p, unsigned first_word, int row, int wave, int lane,
-                                             f32x4 (&sums)[NACC], float& scale) {
-  // The row's sum of squares is added up as the layers' kernels do: four waves' rows (up to 64 parts) chunk by chunk by one wave,
-  // eight waves' each wave's own chunks first.
-  float ss = 0.0f;
-  p.template run<true>(ex, (first_word + row * kRowWords) * 4, a.strip_words * 4, (first_word + a.m * kRowWords + row) * 4, [&](int c, float part) {
-    if constexpr (WAVES == 4) s.product.ss[c][lane] = part;
-    else ss += part;
-  });
-  if constexpr (WAVES != 4) {
-    ss += __shfl_xor(ss, 16, kWave);
-    ss += __shfl_xor(ss, 32, kWave);
-    s.product.ss[wave][lane] = ss;
-  }
-  if (!add_parts<WAVES, UNITS, NACC, V>(s, p.acc, sums, wave, lane)) return false;
-  ss = 0.0f;
+template <int WAVES, int ROWS, int UNITS, int NACC, int V, typename P>
+__device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, P& p, unsigned first_word, int row, int wave, int lane,
+                                             Floats<Ends<ROWS>::kEach> (&sums)[NACC], float& scale) {
+  const unsigned row_at = (first_word + row * kRowWords) * 4, stride = a.strip_words * 4;
+  u32x4 none[1];
+  // The row's sum of squares is added up as the layers' kernels do: four waves' rows (up to 64 parts) chunk by chunk, all of it by the
+  // last wave beside the products; eight waves' each wave's own chunks first.
   if constexpr (WAVES == 4) {
-    float part[16];
+    constexpr int kFours = sum_words(ROWS) / 4;  // 16 bytes that a strip has of them
+    // (every wave asks for them: with a branch around the products of the one that needs them the kernel keeps 117 registers in scratch memory)
+    u32x4 parts[kFours];
+    auto at = [&](int i) {
+      const int n = i * kWave + lane, strip = min(n / kFours, a.n_strip - 1);
+      return At{(first_word + a.m * kRowWords + n % kFours * 4) * 4 + strip * stride, 0};
+    };
+    p.template run<false, kFours>(ex, row_at, stride, 0, [](int, float) {}, parts, at);
+    if (wave == WAVES - 1) {
+      if (wave >= min(p.parts, p.chunks)) ex.take(parts, at);  // (it had no product)
 #pragma unroll
-    for (int c = 0; c < 16; ++c) part[c] = s.product.ss[c][lane];  // (beyond the chunks: whatever is there, not added)
+      for (int i = 0; i < kFours; ++i) *(u32x4*)&s.product.parts[(i * kWave + lane) * 4] = parts[i];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      float part[16], ss = 0.0f;
 #pragma unroll
-    for (int c = 0; c < 16; ++c) ss = c < p.chunks ? ss + part[c] : ss;
-    ss += __shfl_xor(ss, 16, kWave);
-    ss += __shfl_xor(ss, 32, kWave);
-  } else {
+      for (int c = 0; c < 16; ++c) part[c] = __uint_as_float(s.product.parts[(4 * c + lane / 16) * sum_words(ROWS) + lane % sum_words(ROWS)]);  // (beyond the chunks: not added)
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) ss += s.product.ss[w][lane];
+      for (int c = 0; c < 16; ++c) {
+        if (c >= p.chunks) break;
+        ss += part[c];
+      }
+      ss = sum_32_apart(sum_16_apart(ss));
+      if (lane < sum_words(ROWS)) s.product.scale[lane] = 1.0f / sqrtf(ss * a.inv_width + a.eps);
+    }
+    if (!add_parts<WAVES, ROWS, UNITS, NACC, V>(s, p.acc, sums, wave, lane)) return false;
+    scale = s.product.scale[Ends<ROWS>(lane).row];
+    return true;
   }
-  scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  float ss = 0.0f;
+  p.template run<true, 0>(ex, row_at, stride, (first_word + a.m * kRowWords + row) * 4, [&](int, float part) { ss += part; }, none, [](int) { return At{0, 0}; });
+  s.product.ss[wave][lane] = sum_32_apart(sum_16_apart(ss));
+  if (!add_parts<WAVES, ROWS, UNITS, NACC, V>(s, p.acc, sums, wave, lane)) return false;
+  ss = 0.0f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) ss += s.product.ss[w][Ends<ROWS>(lane).row];
+  scale = 1.0f / sqrtf(ss * a.inv_width + a.eps);
   return true;
 }
 
 // The same of eight waves that cut K four ways, waves 0 to 3 for the block's first unit and 4 to 7 for its second.
-template <typename P>
-__device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Exchange& ex, Shared<8>& s, P& p, unsigned first_word, int row, int wave, int lane,
-                                                    f32x4 (&sums)[2], float& scale) {
+template <int ROWS, typename P>
+__device__ __forceinline__ bool run_prepared_halves(const ChainArgs& a, const Exchange& ex, Shared<8, ROWS>& s, P& p, unsigned first_word, int row, int wave, int lane,
+                                                    Floats<Ends<ROWS>::kEach> (&sums)[2], float& scale) {
+  constexpr int kEach = Ends<ROWS>::kEach;
   float ss = 0.0f;
-  p.template run<true>(ex, (first_word + row * kRowWords) * 4, a.strip_words * 4, (first_word + a.m * kRowWords + row) * 4, [&](int, float part) { ss += part; });
-  ss += __shfl_xor(ss, 16, kWave);
-  ss += __shfl_xor(ss, 32, kWave);
-  s.product.ss[wave][lane] = ss;
+  u32x4 none[1];
+  p.template run<true, 0>(ex, (first_word + row * kRowWords) * 4, a.strip_words * 4, (first_word + a.m * kRowWords + row) * 4, [&](int, float part) { ss += part; }, none,
+                          [](int) { return At{0, 0}; });
+  s.product.ss[wave][lane] = sum_32_apart(sum_16_apart(ss));
 #pragma unroll
   for (int j = 0; j < 2; ++j) *(f32x4*)s.product.acc[wave][j][lane] = p.acc[0][j];
+  const Ends<ROWS> ends(lane);
   __syncthreads();
   if (wave % 4 != 0) return false;
+  ss = s.product.ss[wave][ends.row];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) ss += s.product.ss[wave + w][lane];
+  for (int w = 1; w < 4; ++w) ss += s.product.ss[wave + w][ends.row];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    sums[j] = p.acc[0][j];
+    sums[j] = load_floats<kEach>(&s.product.acc[wave][j][ends.from][ends.first % 4]);
 #pragma unroll
-    for (int w = 1; w < 4; ++w) sums[j] += *(const f32x4*)s.product.acc[wave + w][j][lane];
+    for (int w = 1; w < 4; ++w) {
+      const Floats<kEach> more = load_floats<kEach>(&s.product.acc[wave + w][j][ends.from][ends.first % 4]);
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) sums[j][e] += more[e];
+    }
   }
-  scale = 1.0f / sqrtf(ss * (1.0f / (float)a.width) + a.eps);
+  scale = 1.0f / sqrtf(ss * a.inv_width + a.eps);
   return true;
+}
+
+// four channels of a row of the embedding: `v`, in 16 bits `operand`, and the strip's part of the sum of squares, the last row's also in place of
+// rows that there are none of
+template <int ROWS>
+__device__ __forceinline__ void put_entry(const ChainArgs& a, const Exchange& ex, int c, int row, f32x4 v, f32x4 operand, float sum) {
+  const unsigned strip = c / 16, word = a.stream1 + strip * a.strip_words, four = c % 16 / 4;
+  ex.put(word + row * kRowWords + 2 * four, (u32x2){marked2(pack2(operand[0], operand[1])), marked2(pack2(operand[2], operand[3]))});
+  ex.put(a.plain1 + (strip * a.m + row) * kPlainWords + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+  if (four == 0)
+    for (int to = row; to < (row + 1 < a.m ? row + 1 : sum_words(ROWS)); ++to) ex.put(word + a.m * kRowWords + to, marked(sum));
 }
 
 // A row of the embedding into the first layer's strips.  Of a step of more than 16 rows it is normed as the layers' kernel of its own for
 // that does it, a lane per 4 of 256 channels, and its product needs no scale.
+template <int ROWS>
 __device__ __forceinline__ void normed_entry_stage(const ChainArgs& a, const Exchange& ex, float& shared_scale, int row) {
   const float* x = a.x + (size_t)row * a.width;
   if (threadIdx.x < kWave) {
@@ -278,17 +392,14 @@ __device__ __forceinline__ void normed_entry_stage(const ChainArgs& a, const Exc
   const float scale = shared_scale;
   for (int c = threadIdx.x * 4; c < a.width; c += blockDim.x * 4) {
     const f32x4 v = *(const f32x4*)(x + c), normed = (v * scale) * four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
-    const unsigned strip = c / 16, word = a.stream1 + strip * a.strip_words, four = c % 16 / 4;
-    ex.put(word + row * kRowWords + 2 * four, (u32x2){marked2((bf16_t)normed[0], (bf16_t)normed[1]), marked2((bf16_t)normed[2], (bf16_t)normed[3])});
-    if (four == 0) ex.put(word + a.m * kRowWords + row, marked(0.0f));
-    ex.put(a.plain1 + (strip * a.m + row) * kPlainWords + 4 * four, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+    put_entry<ROWS>(a, ex, c, row, v, normed, 0.0f);
   }
 }
 
 // A row of the embedding into the first layer's strips.  Its sum of squares is one part, added up as the layers' kernel for a row
 // that no norm has prepared does: a lane per (part of K, 16 of a chunk's 64 channels).
-template <int WAVES>
-__device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int row) {
+template <int WAVES, int ROWS>
+__device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, int row) {
   const float* x = a.x + (size_t)row * a.width;
   if (threadIdx.x < kWave) {
     const int part = threadIdx.x / 4, g = threadIdx.x % 4, parts = a.parts_first;
@@ -311,16 +422,16 @@ __device__ __forceinline__ void entry_stage(const ChainArgs& a, const Exchange& 
   for (int c = threadIdx.x * 4; c < a.width; c += 64 * WAVES * 4) {
     const f32x4 v = *(const f32x4*)(x + c);
     const f32x4 gain = four_of(a.layers[0].gain1, a.gain_dtype, c, 4, true);
-    const unsigned strip = c / 16;
-    put_row(ex, a.stream1 + strip * a.strip_words, a.plain1 + strip * a.m * kPlainWords, a.m, row, c % 16 / 4, v, gain, c == 0 ? sum : 0.0f);
+    put_entry<ROWS>(a, ex, c, row, v, v * gain, c == 0 ? sum : 0.0f);
   }
 }
 
 // queries, keys and values of two strips (a head's channels f .. f + 15 and f + 32 ..), rotated, and the write into the cache
-template <int WAVES, bool FIRST, bool NORMED = false>
-__device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int unit) {
+template <int WAVES, int ROWS, bool FIRST, bool NORMED = false>
+__device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, int layer, int unit) {
   constexpr bool kOne = WAVES == 8;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  constexpr int kEach = Ends<ROWS>::kEach;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const ChainLayer& L = a.layers[layer];
   const unsigned here = layer * a.layer_words;
   // unit 2 h + i of all: channels 16 i .. 16 i + 15 of head h and those half a head on
@@ -329,53 +440,57 @@ __device__ __forceinline__ void qkv_stage(const ChainArgs& a, const Exchange& ex
   Product<WAVES, 2 * kUnits, 4, 4, kParts> p;
   p.begin(L.w_qkv, [&](int j) { const int u = unit * kUnits + j / 2; return u / 2 * HD + u % 2 * 16 + j % 2 * (HD / 2); }, a.width,
           FIRST ? a.parts_first : a.parts_qkv, lane, wave);
-  const int row = r < a.m ? r : a.m - 1, ends = unit * kUnits + (wave < kUnits ? wave : 0), head = ends / 2, f0 = ends % 2 * 16;
-  const f32x4 c = *(const f32x4*)(a.tok_cos + row * (HD / 2) + f0 + 4 * g), sn = *(const f32x4*)(a.tok_sin + row * (HD / 2) + f0 + 4 * g);
+  const Ends<ROWS> ends(lane);
+  const int row = min(ends.row, a.m - 1), unit_here = unit * kUnits + (wave < kUnits ? wave : 0), head = unit_here / 2, f = unit_here % 2 * 16 + ends.first;
+  const Floats<kEach> c = load_floats<kEach>(a.tok_cos + row * (HD / 2) + f), sn = load_floats<kEach>(a.tok_sin + row * (HD / 2) + f);
   const int pos = a.tok_pos[row], page = a.tok_page[row];
   ex.template gate<kOne>(a_row(a, here + a.stream1, unit * 61), wave);
-  f32x4 sums[2];
+  Floats<kEach> sums[2];
   float scale;
-  if (!run_prepared<WAVES, kUnits, 2, kParts>(a, ex, s, p, here + a.stream1, row, wave, lane, sums, scale)) return;
-  if (r >= a.m) return;
-  f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
-  if (NORMED && layer == 0) {  // of a normed row, by way of 16 bits, as the layers' two kernels for that
+  if (!run_prepared<WAVES, ROWS, kUnits, 2, kParts>(a, ex, s, p, here + a.stream1, min(r, a.m - 1), wave, lane, sums, scale)) return;
+  if (ends.row >= a.m) return;
+  Floats<kEach> out_lo, out_hi;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      lo[e] = (float)(__bf16)sums[0][e];
-      hi[e] = (float)(__bf16)sums[1][e];
+  for (int e = 0; e < kEach; ++e) {
+    float lo = sums[0][e] * scale, hi = sums[1][e] * scale;
+    if (NORMED && layer == 0) {  // of a normed row, by way of 16 bits, as the layers' two kernels for that
+      lo = (float)(__bf16)sums[0][e];
+      hi = (float)(__bf16)sums[1][e];
+    }
+    out_lo[e] = lo;
+    out_hi[e] = hi;
+    if (head < a.heads + a.kv_heads) {
+      out_lo[e] = lo * c[e] - hi * sn[e];
+      out_hi[e] = hi * c[e] + lo * sn[e];
     }
   }
-  f32x4 out_lo = lo, out_hi = hi;
-  if (head < a.heads + a.kv_heads) {
-    out_lo = lo * c - hi * sn;
-    out_hi = hi * c + lo * sn;
-  }
-  bf16x4 b_lo, b_hi;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    b_lo[e] = (__bf16)out_lo[e];
-    b_hi[e] = (__bf16)out_hi[e];
-  }
-  const u32x2 w_lo = {marked2(b_lo[0], b_lo[1]), marked2(b_lo[2], b_lo[3])}, w_hi = {marked2(b_hi[0], b_hi[1]), marked2(b_hi[2], b_hi[3])};
-  const int f = f0 + 4 * g;
+  unsigned w_lo[2], w_hi[2];
+  pack_row(out_lo, w_lo);
+  pack_row(out_hi, w_hi);
   unsigned to;  // [head][strip][row]
   if (head < a.heads) to = a.q + head * a.m * (HD / 2);
   else if (head < a.heads + a.kv_heads) to = a.k + (head - a.heads) * a.m * (HD / 2);
   else to = a.v + (head - a.heads - a.kv_heads) * a.m * (HD / 2);
-  to += here + (f0 / 16 * a.m + row) * 8 + 2 * g;
-  ex.put(to, w_lo);
-  ex.put(to + HD / 32 * a.m * 8, w_hi);
+  to += here + (f / 16 * a.m + row) * 8;
+  put_packed<kEach>(ex, to, ends.first, w_lo);
+  put_packed<kEach>(ex, to + HD / 32 * a.m * 8, ends.first, w_hi);
   if (page < 0 || head < a.heads) return;
   if (head < a.heads + a.kv_heads) {
     bf16_t* dst = L.k_pages + ((size_t)page * a.kv_heads + head - a.heads) * nnis_k_page_elems(HD);
-    *(bf16x4*)(dst + nnis_k_offset(pos % kPageTokens, f)) = b_lo;
-    *(bf16x4*)(dst + nnis_k_offset(pos % kPageTokens, f + HD / 2)) = b_hi;
+    unsigned *at_lo = (unsigned*)(dst + nnis_k_offset(pos % kPageTokens, f)), *at_hi = (unsigned*)(dst + nnis_k_offset(pos % kPageTokens, f + HD / 2));
+    if constexpr (kEach == 4) {
+      *(u32x2*)at_lo = (u32x2){w_lo[0], w_lo[1]};
+      *(u32x2*)at_hi = (u32x2){w_hi[0], w_hi[1]};
+    } else if (kEach == 2 || f % 2 == 0) {
+      *at_lo = w_lo[0];
+      *at_hi = w_hi[0];
+    }
   } else {
     bf16_t* dst = L.v_pages + ((size_t)page * a.kv_heads + head - a.heads - a.kv_heads) * nnis_v_page_elems(HD);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      dst[nnis_v_offset(f + e, pos % kPageTokens)] = b_lo[e];
-      dst[nnis_v_offset(f + HD / 2 + e, pos % kPageTokens)] = b_hi[e];
+    for (int e = 0; e < kEach; ++e) {
+      dst[nnis_v_offset(f + e, pos % kPageTokens)] = (bf16_t)out_lo[e];
+      dst[nnis_v_offset(f + HD / 2 + e, pos % kPageTokens)] = (bf16_t)out_hi[e];
     }
   }
 }
@@ -397,11 +512,21 @@ __device__ __forceinline__ void load_values(KeysPage& f, const bf16_t* page, int
 __device__ __forceinline__ bf16x4 low4(bf16x8 v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); }
 __device__ __forceinline__ bf16x4 high4(bf16x8 v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); }
 
+// the largest of a head's lanes: every fourth
+__device__ __forceinline__ float top_of_head(float v) {
+  v = fmaxf(v, of_row<0x124>(v));
+  v = fmaxf(v, of_row<0x128>(v));
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+}
+
 // A run of a sequence's keys against up to 4 query heads of a key head, keys on lanes (attention.hip,
 // attention_decode_keys_kernel: the same products in the same layouts).  The pages hold every key but the step's own, which the
 // projection's blocks of this launch are still writing: it comes from the exchange and takes its place in the page's operands.
-template <int WAVES>
-__device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int item) {
+template <int WAVES, int ROWS>
+__device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, int layer, int item) {
   constexpr bool kOne = WAVES == 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const int blk = lane / 4, j = lane % 4;
@@ -471,27 +596,27 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   for (int n = 0; n < mine; ++n) {
     const int index = first + n * stride, key0 = index * kPageTokens;
     if (index == own_page) {  // the step's own key and value take their places in the page's operands
-      const int h_at = at_key / 32, e_at = at_key % 8;
       if (n > 0) drop_behind();
       if (lane == at_key) {
-  #pragma unroll
+#pragma unroll
         for (int c = 0; c < HD / 8; ++c) f.k[c] = heads_lds[32 + c];
       }
-      if (g == at_key % 32 / 8) {
-        const unsigned short* value = (const unsigned short*)(heads_lds + 40) + r;
-  #pragma unroll
+      // (the word that the key's value is half of is the same in all lanes: a branch a word, not a choice a register)
+      const int word_at = __builtin_amdgcn_readfirstlane(at_key / 32 * 4 + at_key % 8 / 2), of_lanes = at_key % 32 / 8;
+      const unsigned keep = at_key % 2 ? 0xffffu : 0xffff0000u, shift = at_key % 2 * 16;
+      const unsigned short* value = (const unsigned short*)(heads_lds + 40) + r;
+      unsigned channel[HD / 16];
+#pragma unroll
+      for (int t = 0; t < HD / 16; ++t) channel[t] = (unsigned)value[16 * t] << shift;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) {
+        if (w != word_at) continue;
+        asm volatile("");  // (a branch)
+#pragma unroll
         for (int t = 0; t < HD / 16; ++t) {
-          const unsigned short channel = value[16 * t];
-  #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            u32x4 words = __builtin_bit_cast(u32x4, f.v[h][t]);
-  #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const unsigned put = e_at % 2 ? (words[w] & 0xffffu) | ((unsigned)channel << 16) : (words[w] & 0xffff0000u) | channel;
-              words[w] = h == h_at && w == e_at / 2 ? put : words[w];
-            }
-            f.v[h][t] = __builtin_bit_cast(bf16x8, words);
-          }
+          u32x4 words = __builtin_bit_cast(u32x4, f.v[w / 4][t]);
+          words[w % 4] = g == of_lanes ? (words[w % 4] & keep) | channel[t] : words[w % 4];
+          f.v[w / 4][t] = __builtin_bit_cast(bf16x8, words);
         }
       }
     }
@@ -512,9 +637,7 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
       top = fmaxf(top, sc[e]);
     }
     if (__any(top > reference + kLazyRise)) {
-      float moved = fmaxf(reference, top);
-#pragma unroll
-      for (int offset = 4; offset < kWave; offset <<= 1) moved = fmaxf(moved, __shfl_xor(moved, offset, kWave));
+      const float moved = top_of_head(fmaxf(reference, top));
       const float shrink = reference == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(reference - moved);
       sum *= shrink;
 #pragma unroll
@@ -545,12 +668,12 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
     if (more) load_values(f, v_base + next * v_stride, lane);
   }
   // the states meet in LDS: a lane group's part of a head's sum is that of the keys 16 g .. 16 g + 15 of its pages
-  sum += __shfl_xor(sum, 4, kWave);
-  sum += __shfl_xor(sum, 8, kWave);
+  sum += of_row<0x12c>(sum);  // (four lanes on; right in the four lanes that are stored)
+  sum += of_row<0x128>(sum);
   if (r < 4) {
 #pragma unroll
     for (int t = 0; t < HD / 16; ++t) *(f32x4*)&s.attention.o[wave][r][16 * t + 4 * g] = o[t];
-    s.attention.l[wave][r][g] = sum;
+    s.attention.o[wave][r][HD + g] = sum;
     if (g == 0) s.attention.m[wave][r] = reference;
   }
   __syncthreads();
@@ -558,14 +681,14 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
   // four channels of a head a thread, and one thread a head for the run's reference and sum
   for (int i = threadIdx.x; i < heads_here * (HD / 4 + 1); i += 64 * WAVES) {
     const int head = i / (HD / 4 + 1), four = i % (HD / 4 + 1);
-    // the waves' states in halving rounds, as the layers' kernel has them
+    // the waves' states in halving rounds, as the layers' kernel has them; the one thread's four are the sum's parts
     float m[WAVES];
-    f32x4 l[WAVES], out[WAVES];
+    f32x4 out[WAVES], l[WAVES];
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       m[w] = s.attention.m[w][head];
-      l[w] = *(const f32x4*)s.attention.l[w][head];
-      out[w] = *(const f32x4*)&s.attention.o[w][head][four < HD / 4 ? 4 * four : 0];
+      out[w] = *(const f32x4*)&s.attention.o[w][head][4 * four];
+      if (a.splits == 1) l[w] = *(const f32x4*)&s.attention.o[w][head][HD];
     }
 #pragma unroll
     for (int half = WAVES / 2; half >= 1; half >>= 1) {
@@ -577,23 +700,24 @@ __device__ __forceinline__ void attention_stage(const ChainArgs& a, const Exchan
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           // (which of a sum's two products is rounded first is the compiler's choice there: the other one for the last 16 channels)
-          l[w][e] = fmaf(l[w + half][e], their_w, l[w][e] * mine_w);
-          out[w][e] = four >= 12 ? fmaf(out[w][e], mine_w, out[w + half][e] * their_w) : fmaf(out[w + half][e], their_w, out[w][e] * mine_w);
+          const bool other = four >= 12 && four < HD / 4;
+          const float first = other ? out[w][e] : out[w + half][e], second = other ? out[w + half][e] : out[w][e];
+          out[w][e] = fmaf(first, other ? mine_w : their_w, second * (other ? their_w : mine_w));
+          if (a.splits == 1) l[w][e] = fmaf(l[w + half][e], their_w, l[w][e] * mine_w);
         }
         m[w] = m_new;
       }
     }
-    const float total = (l[0][0] + l[0][1]) + (l[0][2] + l[0][3]);
     f32x4 num = out[0];
     if (a.splits == 1) {
-      const float inv = 1.0f / total;
+      const float inv = 1.0f / ((l[0][0] + l[0][1]) + (l[0][2] + l[0][3]));
 #pragma unroll
       for (int e = 0; e < 4; ++e) num[e] = num[e] * inv;
       if (four < HD / 4)
         ex.put(here + a.attn + (((first_head + head) * (HD / 16) + four / 4) * a.m + token) * 8 + four % 4 * 2,
                (u32x2){marked2((bf16_t)num[0], (bf16_t)num[1]), marked2((bf16_t)num[2], (bf16_t)num[3])});
     } else {
-      if (four == HD / 4) num = (f32x4){m[0], total, 0.0f, 0.0f};
+      if (four == HD / 4) num = (f32x4){m[0], (num[0] + num[1]) + (num[2] + num[3]), 0.0f, 0.0f};
       runs.put(layer * a.layer_runs + ((token * a.heads + first_head + head) * a.splits + split) * kRunRow + 4 * four,
              (u32x4){marked(num[0]), marked(num[1]), marked(num[2]), marked(num[3])});
     }
@@ -652,10 +776,11 @@ __device__ __forceinline__ void combine_stage(const ChainArgs& a, const Exchange
 
 // a strip of 16 columns of the stream: the output projection (down = false) or the feed-forward's down
 // PAIRED: K cut sixteen ways, the even parts and the odd ones added up apart, as the layers' kernel does in two blocks
-template <int WAVES, bool DOWN, bool PAIRED>
-__device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
+template <int WAVES, int ROWS, bool DOWN, bool PAIRED>
+__device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, int layer, int block) {
   constexpr bool kOne = WAVES == 8;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  constexpr int kEach = Ends<ROWS>::kEach;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const ChainLayer& L = a.layers[layer];
   const unsigned here = layer * a.layer_words, next = here + (DOWN ? a.layer_words : 0);
   const int k = DOWN ? a.inner : a.heads * HD;
@@ -665,61 +790,92 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   constexpr int kParts = (WAVES == 4 && DOWN) || PAIRED ? 2 : 1;
   Product<WAVES, kUnits, kSteps, kTogether, kParts, PAIRED> p;
   p.begin(DOWN ? L.w_down : L.w_o, [&](int j) { return (block * kUnits + j) * 16; }, k, PAIRED ? 16 : DOWN ? a.parts_down : a.parts_out, lane, wave);
-  const int strip = block * kUnits + (wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1, column = strip * 16 + 4 * g;
+  const Ends<ROWS> ends(lane);
+  const int strip = block * kUnits + (wave < kUnits ? wave : 0), row = min(ends.row, a.m - 1), column = strip * 16 + ends.first;
   const void* gain_of = DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2;
-  const f32x4 gain = four_of(gain_of, a.gain_dtype, column, 4, true);
+  const f32x4 gains = four_of(gain_of, a.gain_dtype, column / 4 * 4, 4, true);
+  Floats<kEach> gain;
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) gain[e] = kEach == 4 ? gains[e] : kEach == 2 ? (ends.first % 4 ? gains[2 + e % 2] : gains[e]) : gains[ends.first % 4];
   if (kOne || DOWN) ex.template gate<kOne>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
   else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<kOne>(layer * a.layer_runs + (block * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
   else ex.template gate<kOne>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
-  // (the stream is two stages old and more: it is there)
-  u32x4 held[1];
-  if (wave < kUnits) ex.take(held, [&](int) { return At{(here + (DOWN ? a.plain2 : a.plain1) + (strip * a.m + row) * kPlainWords + 4 * g) * 4, 0}; });
-  p.template run<false>(ex, (here + (DOWN ? a.act : a.attn) + row * 8) * 4, a.m * 32, 0, [](int, float) {});
-  f32x4 sums[1];
+  // (the stream is two stages old and more: it is there, and what is looked at before the products is rarely looked for behind them)
+  const unsigned held_at = here + (DOWN ? a.plain2 : a.plain1) + (strip * a.m + row) * kPlainWords + ends.first / 4 * 4;
+  u32x4 held[1], none[1];
+  auto held_from = [&](int) { return At{held_at * 4, 0}; };
+  const bool held_there = wave >= kUnits || ex.template look<kPastCaches>(held, held_from);
+  p.template run<false, 0>(ex, (here + (DOWN ? a.act : a.attn) + min(r, a.m - 1) * 8) * 4, a.m * 32, 0, [](int, float) {}, none, [](int) { return At{0, 0}; });
+  if (!held_there) ex.take(held, held_from);
+  Floats<kEach> sums[1];
   if constexpr (PAIRED) {
     const f32x4 even[1][1] = {{p.acc[0][0]}};
     *(f32x4*)s.product.acc[wave][1][lane] = p.acc[1][0];
-    if (!add_parts<WAVES, 1, 1, 1>(s, even, sums, wave, lane)) return;
-    f32x4 odd = *(const f32x4*)s.product.acc[0][1][lane];
+    if (!add_parts<WAVES, ROWS, 1, 1, 1>(s, even, sums, wave, lane)) return;
+    auto odd_at = [&](int w) { return load_floats<kEach>(&s.product.acc[w][1][ends.from][ends.first % 4]); };
+    Floats<kEach> odd = odd_at(0);
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) odd += *(const f32x4*)s.product.acc[w][1][lane];
-    sums[0] += odd;
+    for (int w = 1; w < WAVES; ++w) {
+      const Floats<kEach> more = odd_at(w);
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) odd[e] += more[e];
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) sums[0][e] += odd[e];
   } else {
-    if (!add_parts<WAVES, kUnits, 1, kParts>(s, p.acc, sums, wave, lane)) return;
+    if (!add_parts<WAVES, ROWS, kUnits, 1, kParts>(s, p.acc, sums, wave, lane)) return;
   }
   if (last) {  // (the final norm's kernel adds it to the stream)
-    if (r < a.m) {
-      bf16x4 y;
+    if (ends.row < a.m) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = (__bf16)sums[0][e];
-      *(bf16x4*)(a.y_out + (size_t)row * a.width + column) = y;
+      for (int e = 0; e < kEach; ++e) a.y_out[(size_t)row * a.width + column + e] = (bf16_t)sums[0][e];
     }
     return;
   }
-  f32x4 v;
-  float sq = 0.0f;
+  Floats<kEach> v, operand;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = __uint_as_float(held[0][e]) + sums[0][e];
-    sq = fmaf(v[e], v[e], sq);
+  for (int e = 0; e < kEach; ++e) {
+    v[e] = __uint_as_float(kEach == 4 ? held[0][e] : kEach == 2 ? (ends.first % 4 ? held[0][2 + e % 2] : held[0][e]) : held[0][ends.first % 4]) + sums[0][e];
+    operand[e] = v[e] * gain[e];
   }
-  sq += __shfl_xor(sq, 16, kWave);
-  sq += __shfl_xor(sq, 32, kWave);
-  if (r >= a.m) return;
-  if (!DOWN && layer + 1 == a.layer_count) *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
-  put_row(ex, next + (DOWN ? a.stream1 : a.stream2) + strip * a.strip_words, next + (DOWN ? a.plain1 : a.plain2) + strip * a.m * kPlainWords, a.m, row, g, v, gain, sq);
+  unsigned words[2];
+  pack_row(operand, words);
+  // a lane group's four channels in their order
+  float sq = 0.0f;
+  if constexpr (kEach == 1) {
+    const float v0 = of_row<0x00>(v[0]), v1 = of_row<0x55>(v[0]), v2 = of_row<0xaa>(v[0]), v3 = of_row<0xff>(v[0]);
+    sq = fmaf(v3, v3, fmaf(v2, v2, fmaf(v1, v1, fmaf(v0, v0, 0.0f))));
+  } else if constexpr (kEach == 2) {
+    const float v0 = of_row<0xa0>(v[0]), v1 = of_row<0xa0>(v[1]), v2 = of_row<0xf5>(v[0]), v3 = of_row<0xf5>(v[1]);
+    sq = fmaf(v3, v3, fmaf(v2, v2, fmaf(v1, v1, fmaf(v0, v0, 0.0f))));
+  } else {
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) sq = fmaf(v[e], v[e], sq);
+  }
+  sq = sum_32_apart(sum_16_apart(sq));
+  const unsigned to = next + (DOWN ? a.stream1 : a.stream2) + strip * a.strip_words;
+  if (ends.first == 0) ex.put(to + a.m * kRowWords + ends.row, marked(sq));  // (lanes beyond the rows have the last row's)
+  if (ends.row >= a.m) return;
+  put_packed<kEach>(ex, to + row * kRowWords, ends.first, words);
+  put_floats(ex, next + (DOWN ? a.plain1 : a.plain2) + (strip * a.m + row) * kPlainWords + ends.first, v);
+  if (!DOWN && layer + 1 == a.layer_count) {
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) a.x_out[(size_t)row * a.width + column + e] = v[e];
+  }
 }
 
 // HALVES: eight waves that cut K four ways for each of the block's two units, as the layers' kernel does for this many strips
-template <int WAVES, bool HALVES>
-__device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES>& s, int layer, int block) {
+template <int WAVES, int ROWS, bool HALVES>
+__device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& ex, Shared<WAVES, ROWS>& s, int layer, int block) {
   constexpr bool kOne = WAVES == 8;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const unsigned here = layer * a.layer_words;
   constexpr int kUnits = units_of<WAVES>();
-  const int unit = block * kUnits + (HALVES ? wave / 4 : wave < kUnits ? wave : 0), row = r < a.m ? r : a.m - 1;
+  const int unit = block * kUnits + (HALVES ? wave / 4 : wave < kUnits ? wave : 0), row = min(r, a.m - 1);
   const unsigned one = a_row(a, here + a.stream2, block * 61);
-  f32x4 sums[2];
+  constexpr int kEach = Ends<ROWS>::kEach;
+  const Ends<ROWS> ends(lane);
+  Floats<kEach> sums[2];
   float scale;
   if constexpr (HALVES) {
     Product<4, 2, 8, 4, 1> p;
@@ -730,25 +886,27 @@ __device__ __forceinline__ void gate_stage(const ChainArgs& a, const Exchange& e
     Product<WAVES, 2 * kUnits, 4, 4, 1> p;
     p.begin(a.layers[layer].w_gate_up, [&](int j) { return (block * kUnits + j / 2) * 16 + j % 2 * a.inner; }, a.width, a.parts_gate, lane, wave);
     ex.template gate<kOne>(one, wave);
-    if (!run_prepared<WAVES, kUnits, 2, 1>(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
+    if (!run_prepared<WAVES, ROWS, kUnits, 2, 1>(a, ex, s, p, here + a.stream2, row, wave, lane, sums, scale)) return;
   }
-  if (r >= a.m) return;
-  bf16_t out[4];
+  if (ends.row >= a.m) return;
+  Floats<kEach> out;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < kEach; ++e) {
     const float gate = sums[0][e] * scale, up = sums[1][e] * scale;
     const float x = __builtin_amdgcn_exp2f(gate * -1.4426950408889634f);  // (as epilogue.h)
-    out[e] = (bf16_t)(gate * __builtin_amdgcn_rcpf(1.0f + x) * up);
+    out[e] = gate * __builtin_amdgcn_rcpf(1.0f + x) * up;
   }
-  ex.put(here + a.act + (unit * a.m + row) * 8 + 2 * g, (u32x2){marked2(out[0], out[1]), marked2(out[2], out[3])});
+  unsigned words[2];
+  pack_row(out, words);
+  put_packed<kEach>(ex, here + a.act + (unit * a.m + ends.row) * 8, ends.first, words);
 }
 
 // TILED: more than 16 rows (beside its arithmetic steps of up to 16 are half a per cent slower).  NEAR: the first look through the caches
 // (Exchange::take): it needs registers that fewer than five rows lose more by than they gain (four waves, of 30 layers of width 576, without
 // and with it: 1 row 387 and 391 us, 4 458 and 462, 8 491 and 480, 16 566 and 550, 17 643 and 603).
-template <int WAVES, bool TILED, bool NEAR>
+template <int WAVES, int ROWS, bool TILED, bool NEAR>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 4 && (TILED || !NEAR) ? 3 : 2))) void chain_kernel(ChainArgs a) {
-  __shared__ Shared<WAVES> s;
+  __shared__ Shared<WAVES, ROWS> s;
   int b = blockIdx.x, layer = -1, stage = -1, tile = 0;
   auto in = [&](int index, int blocks, int all) {  // the stage with this index has `blocks` for a tile
     if (stage >= 0) return;
@@ -789,24 +947,24 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
   }
   const Exchange ex(a, a.words, a.words_bytes, NEAR);
   if (stage == 0) {
-    if (TILED) return normed_entry_stage(a, ex, s.sums[0], b);
-    return entry_stage<WAVES>(a, ex, s, b);
+    if (TILED) return normed_entry_stage<ROWS>(a, ex, s.sums[0], b);
+    return entry_stage<WAVES, ROWS>(a, ex, s, b);
   }
   if (stage == 1) {
-    if (WAVES == 4 && !TILED && layer == 0) return qkv_stage<WAVES, true>(a, ex, s, layer, b);
-    return qkv_stage<WAVES, false, TILED>(a, ex, s, layer, b);
+    if (WAVES == 4 && !TILED && layer == 0) return qkv_stage<WAVES, ROWS, true>(a, ex, s, layer, b);
+    return qkv_stage<WAVES, ROWS, false, TILED>(a, ex, s, layer, b);
   }
-  if (stage == 2) return attention_stage<WAVES>(a, ex, s, layer, b);
+  if (stage == 2) return attention_stage<WAVES, ROWS>(a, ex, s, layer, b);
   if (stage == 3) return combine_stage<WAVES>(a, ex, layer, b);
-  if (stage == 4) return strip_stage<WAVES, false, false>(a, ex, s, layer, b);
+  if (stage == 4) return strip_stage<WAVES, ROWS, false, false>(a, ex, s, layer, b);
   if (stage == 5) {
     if constexpr (WAVES == 8)
-      if (a.parts_gate == 4) return gate_stage<WAVES, true>(a, ex, s, layer, b);
-    return gate_stage<WAVES, false>(a, ex, s, layer, b);
+      if (a.parts_gate == 4) return gate_stage<WAVES, ROWS, true>(a, ex, s, layer, b);
+    return gate_stage<WAVES, ROWS, false>(a, ex, s, layer, b);
   }
   if constexpr (WAVES == 8)
-    if (a.down_paired && layer + 1 < a.layer_count) return strip_stage<WAVES, true, true>(a, ex, s, layer, b);
-  strip_stage<WAVES, true, false>(a, ex, s, layer, b);
+    if (a.down_paired && layer + 1 < a.layer_count) return strip_stage<WAVES, ROWS, true, true>(a, ex, s, layer, b);
+  strip_stage<WAVES, ROWS, true, false>(a, ex, s, layer, b);
 }
 
 // where the words of a layer lie; returns their number
@@ -817,7 +975,7 @@ unsigned lay_out(ChainArgs& a) {
     at += (words + 31) / 32 * 32;
   };
   const unsigned m = a.m, strips = a.width / 16;
-  a.strip_words = ((kRowWords + 1) * m + 15) / 16 * 16;
+  a.strip_words = (kRowWords * m + sum_words(a.width > 1024 ? kMostRows : m) + 15) / 16 * 16;  // (the kernels' ROWS)
   place(a.stream1, strips * a.strip_words);
   place(a.stream2, strips * a.strip_words);
   place(a.plain1, m * strips * kPlainWords);
@@ -873,7 +1031,7 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   a.layers = (const ChainLayer*)layers; a.layer_count = layer_count;
   a.rows = m; a.tiles = (m + kMostRows - 1) / kMostRows; a.m = min(m, kMostRows);
   a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits; a.gain_dtype = gain_dtype;
-  a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f;
+  a.eps = eps; a.inv_width = 1.0f / (float)width; a.scale_log2 = scale * 1.4426950408889634f;
   a.x = x; a.x_out = x_out; a.y_out = (bf16_t*)y_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages;
   a.max_pages = max_pages; a.words = (unsigned*)words; a.run_words = (unsigned*)runs;
   a.layer_words = lay_out(a);
@@ -917,10 +1075,11 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   NNIS_REQUIRE(blocks < (1LL << 30), "chain: too many blocks");
   hipStream_t stream = (hipStream_t)stream_ptr;
   if (chain_clear(words, word_count - 32, runs, runs_needed, a.fail, stream)) return 1;
-  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
-  else if (m <= 4) hipLaunchKernelGGL((chain_kernel<4, false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-  else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((chain_kernel<4, true, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, 16, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  else if (m <= 4) hipLaunchKernelGGL((chain_kernel<4, 4, false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else if (m <= 8) hipLaunchKernelGGL((chain_kernel<4, 8, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, 16, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((chain_kernel<4, 16, true, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   NNIS_LAUNCH_CHECK("chain");
   return 0;
 }
