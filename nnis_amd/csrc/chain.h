@@ -17,6 +17,7 @@
 
 namespace {
 
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
 
@@ -124,6 +125,101 @@ struct Exchange {
   __device__ __forceinline__ void put(unsigned word, unsigned v) const { __builtin_amdgcn_raw_buffer_store_b32(v, r, word * 4, 0, kPastCaches); }
   __device__ __forceinline__ void put(unsigned word, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, r, word * 4, 0, kPastCaches); }
   __device__ __forceinline__ void put(unsigned word, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, r, word * 4, 0, kPastCaches); }
+};
+
+// words that a strip of the stream has for its rows' parts of their sums of squares
+__host__ __device__ constexpr int sum_words(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
+
+// What stands between a stage's last operand and its words is a chain of instructions of one wave, four cycles each and more: the
+// ends of the products are kept short.  A lane's partner 16 and 32 lanes on (a row of another lane group) by register, not by LDS:
+__device__ __forceinline__ float sum_16_apart(float v) {
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+}
+__device__ __forceinline__ float sum_32_apart(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+}
+__device__ __forceinline__ float most_16_apart(float v) {
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+}
+__device__ __forceinline__ float most_32_apart(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+}
+template <int CONTROL>  // a lane of the same 16
+__device__ __forceinline__ float of_row(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CONTROL, 0xf, 0xf, false));
+}
+
+// Which of a result's elements (16 channels of up to 16 rows) a lane ends.  The matrix instruction leaves a lane four channels of a row;
+// of up to 8 and 4 rows half and three quarters of the lanes would have none, and from LDS each takes two or one.
+template <int ROWS>
+struct Ends {
+  static constexpr int kEach = ROWS <= 4 ? 1 : ROWS <= 8 ? 2 : 4;
+  int row, first, from;  // the first of its channels; the lane that had them
+  __device__ __forceinline__ explicit Ends(int lane)
+      : row(lane % 16 / (4 / kEach)), first(lane / 16 * 4 + lane % (4 / kEach) * kEach), from(lane / 16 * 16 + row) {}
+};
+template <int N>
+struct Floats {
+  float v[N];
+  __device__ __forceinline__ float& operator[](int e) { return v[e]; }
+  __device__ __forceinline__ float operator[](int e) const { return v[e]; }
+};
+template <int N>
+__device__ __forceinline__ Floats<N> load_floats(const float* p) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  Floats<N> out;
+  if constexpr (N == 4) {
+    const f32x4 v = *(const f32x4*)p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = v[e];
+  } else if constexpr (N == 2) {
+    const f32x2 v = *(const f32x2*)p;
+    out[0] = v[0];
+    out[1] = v[1];
+  } else {
+    out[0] = *p;
+  }
+  return out;
+}
+template <int N>
+__device__ __forceinline__ void put_floats(const Exchange& ex, unsigned word, const Floats<N>& v) {
+  if constexpr (N == 4) ex.put(word, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
+  else if constexpr (N == 2) ex.put(word, (u32x2){marked(v[0]), marked(v[1])});
+  else ex.put(word, marked(v[0]));
+}
+
+// The scales of up to ROWS rows that a norm prepared, by one wave of a block beside its products: the parts of a row's sum of squares lie behind
+// each of the stream's strips (up to 64 of them), and are added up strip 4 c + g by strip in lane group g, then over the groups.
+template <int ROWS>
+struct RowScales {
+  static constexpr int kFours = sum_words(ROWS) / 4;  // 16 bytes that a strip has of them: loads of the wave
+  __attribute__((aligned(16))) unsigned parts[kFours * kWave * 4];  // [strip][row]
+  float scale[16];
+
+  // where load i of a lane is, from the first strip's sums on; `stride`: bytes from strip to strip
+  static __device__ __forceinline__ At at(int i, int lane, unsigned first_word, unsigned stride, int strips) {
+    const int n = i * kWave + lane;
+    return At{(first_word + n % kFours * 4) * 4 + min(n / kFours, strips - 1) * stride, 0};
+  }
+  __device__ __forceinline__ void make(const u32x4 (&got)[kFours], int lane, int strips, float inv_width, float eps) {
+#pragma unroll
+    for (int i = 0; i < kFours; ++i) *(u32x4*)&parts[(i * kWave + lane) * 4] = (i * kWave + lane) / kFours < strips ? got[i] : (u32x4){0, 0, 0, 0};
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // (all sixteen, zeros beyond the strips: told to stop there, the compiler goes through its registers in a loop, 0.2 us)
+    float part[16], sum = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) part[c] = __uint_as_float(parts[(4 * c + lane / 16) * sum_words(ROWS) + lane % sum_words(ROWS)]);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) sum += part[c];
+    sum = sum_32_apart(sum_16_apart(sum));
+    if (lane < sum_words(ROWS)) scale[lane] = 1.0f / sqrtf(sum * inv_width + eps);
+  }
 };
 
 __global__ __launch_bounds__(256) void chain_clear_kernel(u32x4* words, unsigned n, u32x4* runs, unsigned n_runs, unsigned* fail) {

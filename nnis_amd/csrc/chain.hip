@@ -64,22 +64,6 @@ struct ChainArgs {
 // 1.4 us after the last of them was written, where rows side by side take 0.7.  Parts of 36 blocks in one line took a reader 1.2 us more.)
 constexpr int kRowWords = 8;     // of a strip of an operand
 constexpr int kPlainWords = 16;  // ... of the stream
-__host__ __device__ constexpr int sum_words(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
-
-// What stands between a stage's last operand and its words is a chain of instructions of one wave, four cycles each and more: the
-// ends of the products are kept short.  A lane's partner 16 and 32 lanes on (a row of another lane group) by register, not by LDS:
-__device__ __forceinline__ float sum_16_apart(float v) {
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
-}
-__device__ __forceinline__ float sum_32_apart(float v) {
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
-}
-template <int CONTROL>  // a lane of the same 16
-__device__ __forceinline__ float of_row(float v) {
-  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CONTROL, 0xf, 0xf, false));
-}
 __device__ __forceinline__ unsigned pack2(float lo, float hi) {
   typedef __attribute__((ext_vector_type(2))) float f32x2;
   typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
@@ -87,38 +71,6 @@ __device__ __forceinline__ unsigned pack2(float lo, float hi) {
 }
 __device__ __forceinline__ unsigned marked2(unsigned packed) { return packed == kNone ? 0x7fc07fc0u : packed; }
 
-// Which of a result's elements (16 channels of up to 16 rows) a lane ends.  The matrix instruction leaves a lane four channels of a row;
-// of up to 8 and 4 rows half and three quarters of the lanes would have none, and from LDS each takes two or one.
-template <int ROWS>
-struct Ends {
-  static constexpr int kEach = ROWS <= 4 ? 1 : ROWS <= 8 ? 2 : 4;
-  int row, first, from;  // the first of its channels; the lane that had them
-  __device__ __forceinline__ explicit Ends(int lane)
-      : row(lane % 16 / (4 / kEach)), first(lane / 16 * 4 + lane % (4 / kEach) * kEach), from(lane / 16 * 16 + row) {}
-};
-template <int N>
-struct Floats {
-  float v[N];
-  __device__ __forceinline__ float& operator[](int e) { return v[e]; }
-  __device__ __forceinline__ float operator[](int e) const { return v[e]; }
-};
-template <int N>
-__device__ __forceinline__ Floats<N> load_floats(const float* p) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2;
-  Floats<N> out;
-  if constexpr (N == 4) {
-    const f32x4 v = *(const f32x4*)p;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = v[e];
-  } else if constexpr (N == 2) {
-    const f32x2 v = *(const f32x2*)p;
-    out[0] = v[0];
-    out[1] = v[1];
-  } else {
-    out[0] = *p;
-  }
-  return out;
-}
 // a lane's channels in 16 bits, two a word: words[0 .. 1], of which `packed_words` are the lane's (with one channel a lane every other lane has a word)
 template <int N>
 __device__ __forceinline__ void pack_row(const Floats<N>& v, unsigned (&words)[2]) {
@@ -131,13 +83,6 @@ __device__ __forceinline__ void put_packed(const Exchange& ex, unsigned word, in
   if constexpr (N == 4) ex.put(word + first / 2, (u32x2){marked2(words[0]), marked2(words[1])});
   else if (N == 2 || first % 2 == 0) ex.put(word + first / 2, marked2(words[0]));
 }
-template <int N>
-__device__ __forceinline__ void put_floats(const Exchange& ex, unsigned word, const Floats<N>& v) {
-  if constexpr (N == 4) ex.put(word, (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])});
-  else if constexpr (N == 2) ex.put(word, (u32x2){marked(v[0]), marked(v[1])});
-  else ex.put(word, marked(v[0]));
-}
-
 __device__ __forceinline__ bf16x8 load_packed(const bf16_t* p) { return __builtin_nontemporal_load((const bf16x8*)p); }
 
 // STRIPS strips of 16 weight rows times the step's rows.  K (chunks of 64, whole) is cut `parts` ways: part p has the chunks p, p +
@@ -241,8 +186,7 @@ struct Shared {
     struct {
       float acc[WAVES][4][kWave][4];
       float ss[WAVES == 4 ? 1 : WAVES][kWave];  // eight waves: a row's part from each
-      __attribute__((aligned(16))) unsigned parts[WAVES == 4 ? sum_words(ROWS) * kWave : 1];  // four waves: [strip][row]
-      float scale[16];
+      RowScales<ROWS> scales;  // four waves
     } product;
     struct {
       __attribute__((aligned(16))) float o[WAVES][4][HD + 4];  // a head's outputs, then its sum's four parts
@@ -289,34 +233,16 @@ __device__ __forceinline__ bool run_prepared(const ChainArgs& a, const Exchange&
   // The row's sum of squares is added up as the layers' kernels do: four waves' rows (up to 64 parts) chunk by chunk, all of it by the
   // last wave beside the products; eight waves' each wave's own chunks first.
   if constexpr (WAVES == 4) {
-    constexpr int kFours = sum_words(ROWS) / 4;  // 16 bytes that a strip has of them
     // (every wave asks for them: with a branch around the products of the one that needs them the kernel keeps 117 registers in scratch memory)
-    u32x4 parts[kFours];
-    auto at = [&](int i) {
-      const int n = i * kWave + lane, strip = min(n / kFours, a.n_strip - 1);
-      return At{(first_word + a.m * kRowWords + n % kFours * 4) * 4 + strip * stride, 0};
-    };
-    p.template run<false, kFours>(ex, row_at, stride, 0, [](int, float) {}, parts, at);
+    u32x4 parts[RowScales<ROWS>::kFours];
+    auto at = [&](int i) { return RowScales<ROWS>::at(i, lane, first_word + a.m * kRowWords, stride, a.n_strip); };
+    p.template run<false, RowScales<ROWS>::kFours>(ex, row_at, stride, 0, [](int, float) {}, parts, at);
     if (wave == WAVES - 1) {
       if (wave >= min(p.parts, p.chunks)) ex.take(parts, at);  // (it had no product)
-#pragma unroll
-      for (int i = 0; i < kFours; ++i) *(u32x4*)&s.product.parts[(i * kWave + lane) * 4] = parts[i];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      float part[16], ss = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) part[c] = __uint_as_float(s.product.parts[(4 * c + lane / 16) * sum_words(ROWS) + lane % sum_words(ROWS)]);  // (beyond the chunks: not added)
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        if (c >= p.chunks) break;
-        ss += part[c];
-      }
-      ss = sum_32_apart(sum_16_apart(ss));
-      if (lane < sum_words(ROWS)) s.product.scale[lane] = 1.0f / sqrtf(ss * a.inv_width + a.eps);
+      s.product.scales.make(parts, lane, a.n_strip, a.inv_width, a.eps);
     }
     if (!add_parts<WAVES, ROWS, UNITS, NACC, V>(s, p.acc, sums, wave, lane)) return false;
-    scale = s.product.scale[Ends<ROWS>(lane).row];
+    scale = s.product.scales.scale[Ends<ROWS>(lane).row];
     return true;
   }
   float ss = 0.0f;
@@ -516,10 +442,7 @@ __device__ __forceinline__ bf16x4 high4(bf16x8 v) { return __builtin_shufflevect
 __device__ __forceinline__ float top_of_head(float v) {
   v = fmaxf(v, of_row<0x124>(v));
   v = fmaxf(v, of_row<0x128>(v));
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+  return most_32_apart(most_16_apart(v));
 }
 
 // A run of a sequence's keys against up to 4 query heads of a key head, keys on lanes (attention.hip,

@@ -1,9 +1,9 @@
 // The layers of a step of few single tokens in one launch, in 32 bits: chain.hip's stages on v_mfma_f32_16x16x4_f32, for weights
 // in the checkpoint's order (as gemm_f32.hip's kernel for few rows takes them: 16 bytes a lane are 16 k of 16 rows).
 //
-// Rows are exchanged by strips of 16 channels, [strip][row][16], 64 bytes that one block writes; the stream's as records of 192: 16
-// channels times the next norm's gain, the strip's part of the row's sum of squares (four times; 48 unused bytes), and the channels
-// themselves.  The row's scale comes behind the product.
+// Rows are exchanged by strips of 16 channels, [strip][row][16], 64 bytes that one block writes.  A strip of the stream's rows, which is
+// times the next norm's gain, has the rows' parts of their sums of squares behind it (a word a row, 4, 8 or 16 of them); the stream
+// itself, [strip][row][16], lies apart.  The row's scale comes behind the product.
 //
 // A block is a unit of a product (a pair of strips of 16 weight rows, or a strip) and has 8 waves, wave w the chunks of 16 k w, w + 8, ..;
 // WIDE (from a width of 1,025 on): more registers of weights a wave, one block a compute unit.  Bound by the way from a stage's
@@ -17,10 +17,8 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 constexpr int HD = kChainHead, kWaves = 8;
-constexpr int kRecord32 = 48, kSum32 = 16, kStream32 = 32;  // words
+constexpr int kRow32 = 16;  // words of a row's strip
 constexpr float kRise = 8.0f;  // as in attention_f32.h: the softmax reference moves when a score rises this far above it
 
 struct ChainLayer32 {
@@ -32,7 +30,7 @@ struct ChainLayer32 {
 struct ChainArgs32 {
   const ChainLayer32* layers;
   int layer_count, m, width, heads, kv_heads, inner, splits;
-  float eps, scale;
+  float eps, scale, inv_width;
   const float* x;  // [m, width]
   float *x_out, *y_out;  // [m, width]: the stream behind the last attention, and what the last feed-forward adds to it
   const float *tok_cos, *tok_sin;
@@ -40,22 +38,25 @@ struct ChainArgs32 {
   int max_pages;
   unsigned *words, *run_words;
   unsigned words_bytes, run_bytes, layer_words, layer_runs;
-  unsigned stream1, stream2, q, k, v, attn, act;  // where a layer's words lie: all [strip][row][16]
+  unsigned stream1, stream2, plain1, plain2, q, k, v, attn, act;  // where a layer's words lie
+  unsigned strip_words;  // of the stream's rows as the next product takes them
   int n_strip, n_entry, n_qkv, n_att, n_comb, n_gate;  // blocks of a stage (the output projection and down: a strip each)
   unsigned *fail, *host_fail;
 };
 
 __device__ __forceinline__ u32x4 marked4(f32x4 v) { return (u32x4){marked(v[0]), marked(v[1]), marked(v[2]), marked(v[3])}; }
 
+template <int ROWS>
 struct Shared32 {
   union {
     struct {
       f32x4 acc[kWaves][2][kWave];
-      float squares[kWaves][kMostRows];
+      float squares[kWaves][kMostRows];  // WIDE
+      RowScales<ROWS> scales;            // not WIDE
     } product;
     struct {
-      __attribute__((aligned(16))) float o[kWaves][16][HD + 4];
-      float m[kWaves][16], l[kWaves][16];
+      __attribute__((aligned(16))) float o[kWaves][16][HD + 4];  // a head's outputs, then its sum
+      float m[kWaves][16], weights[kWaves][16][kWaves];
     } attention;
   };
 };
@@ -63,7 +64,9 @@ struct Shared32 {
 // STRIPS strips of 16 weight rows times the step's rows.  A wave asks for the weights of its first STEPS chunks when the block
 // begins; XB chunks of the operand are asked for together.  A step of the operand beyond the last chunk reads the last again
 // and is not multiplied.
-template <int STRIPS, int STEPS, int XB, bool NORM>
+// NORM: a row that a norm prepared, whose parts of the sum of squares each wave takes with its own chunks (SUMS), or all of them, with
+// its first trip, for the last wave.
+template <int ROWS, int STRIPS, int STEPS, int XB, bool NORM, bool SUMS>
 struct Product32 {
   static_assert(STEPS % XB == 0, "whole trips");
   f32x4 w[STEPS][STRIPS], acc[STRIPS][4];  // a sum for each of a lane's four k: shorter chains (K 8,256: 0.69 to 0.88 of the layers' error
@@ -95,25 +98,32 @@ struct Product32 {
     }
     ask(wave);
   }
-  // the operand: the lane's row begins at byte `row_at`, `stride` bytes from strip to strip
-  __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride) {
-    const unsigned at = row_at + lane / 16 * 16;
+  // the operand: the lane's row begins at byte `row_at`, `stride` bytes from strip to strip; `sums`: the first strip's sums' first word
+  __device__ __forceinline__ void run(const Exchange& ex, Shared32<ROWS>& s, unsigned row_at, unsigned stride, unsigned sums, int row, float inv_width, float eps) {
+    const unsigned at = row_at + lane / 16 * 16, sum_at = (sums + row) * 4;
+    constexpr int kMore = NORM && !SUMS ? RowScales<ROWS>::kFours : 0;
+    u32x4 more[kMore > 0 ? kMore : 1];
+    auto ask_more = [&](int i) { return RowScales<ROWS>::at(i, lane, sums, stride, chunks); };
     for (int base = wave; base < chunks; base += kWaves * STEPS) {
       if (base != wave) ask(base);
 #pragma unroll
       for (int b = 0; b < STEPS; b += XB) {
         if (base + b * kWaves >= chunks) continue;
-        u32x4 v[XB];
+        u32x4 v[XB + kMore];
         unsigned part[XB];
         auto chunk = [&](int d) { return (unsigned)min(base + (b + d) * kWaves, chunks - 1) * stride; };
-        auto pieces = [&](int d) { return At{at, chunk(d)}; };
-        if constexpr (NORM) ex.take(v, pieces, part, [&](int d) { return At{row_at + kSum32 * 4, chunk(d)}; });
+        auto pieces = [&](int d) { return d < XB ? At{at, chunk(d)} : ask_more(d - XB); };
+        if constexpr (NORM && SUMS) ex.take(v, pieces, part, [&](int d) { return At{sum_at, chunk(d)}; });
         else ex.take(v, pieces);
+        if constexpr (kMore > 0) {
+#pragma unroll
+          for (int i = 0; i < kMore; ++i) more[i] = v[XB + i];
+        }
 #pragma unroll
         for (int d = 0; d < XB; ++d) {
           if (base + (b + d) * kWaves >= chunks) continue;
           const f32x4 x = __builtin_bit_cast(f32x4, v[d]);
-          if constexpr (NORM) square += __uint_as_float(part[d]);
+          if constexpr (NORM && SUMS) square += __uint_as_float(part[d]);
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -121,90 +131,117 @@ struct Product32 {
         }
       }
     }
+    if constexpr (kMore > 0) {
+      if (wave == kWaves - 1) {
+        if (wave >= chunks) ex.take(more, ask_more);  // (it had no product)
+        s.product.scales.make(more, lane, chunks, inv_width, eps);
+      }
+    }
   }
   // the waves' sums added up in their order; false for the waves that are done.  scale: of the lane's row (NORM)
-  __device__ __forceinline__ bool finish(Shared32& s, f32x4 (&sums)[STRIPS], float& scale, float eps) {
+  __device__ __forceinline__ bool finish(Shared32<ROWS>& s, const Ends<ROWS>& ends, Floats<Ends<ROWS>::kEach> (&sums)[STRIPS], float& scale, float eps) {
+    constexpr int kEach = Ends<ROWS>::kEach;
 #pragma unroll
     for (int j = 0; j < STRIPS; ++j) s.product.acc[wave][j][lane] = (acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]);
-    if constexpr (NORM) {
+    if constexpr (NORM && SUMS) {
       if (lane < 16) s.product.squares[wave][lane] = square;
     }
     __syncthreads();
     if (wave != 0) return false;
 #pragma unroll
     for (int j = 0; j < STRIPS; ++j) {
-      sums[j] = s.product.acc[0][j][lane];
+      auto part_at = [&](int p) { return load_floats<kEach>((const float*)&s.product.acc[p][j][ends.from] + ends.first % 4); };
+      sums[j] = part_at(0);
 #pragma unroll
-      for (int p = 1; p < kWaves; ++p) sums[j] += s.product.acc[p][j][lane];
+      for (int p = 1; p < kWaves; ++p) {
+        const Floats<kEach> part = part_at(p);
+#pragma unroll
+        for (int e = 0; e < kEach; ++e) sums[j][e] += part[e];
+      }
     }
-    if constexpr (NORM) {
-      float total = s.product.squares[0][lane % 16];
+    if constexpr (NORM && SUMS) {
+      float total = s.product.squares[0][ends.row];
 #pragma unroll
-      for (int p = 1; p < kWaves; ++p) total += s.product.squares[p][lane % 16];
+      for (int p = 1; p < kWaves; ++p) total += s.product.squares[p][ends.row];
       scale = 1.0f / sqrtf(total / (float)(chunks * 16) + eps);
+    } else if constexpr (NORM) {
+      scale = s.product.scales.scale[ends.row];
     }
     return true;
   }
 };
 
-// four channels of a row's strip into its record; `part`: the strip's sum of squares, in all four lanes
-__device__ __forceinline__ void put_record(const Exchange& ex, unsigned word, int four, f32x4 v, f32x4 gain, float part) {
-  ex.put(word + 4 * four, marked4(v * gain));
-  ex.put(word + kStream32 + 4 * four, marked4(v));
-  if (four == 0) ex.put(word + kSum32, (u32x4){marked(part), marked(part), marked(part), marked(part)});
+// a word of some row of the stream's strips at `first_word`
+__device__ __forceinline__ unsigned a_row(const ChainArgs32& a, unsigned first_word, int some) {
+  return first_word + some / a.m % a.n_strip * a.strip_words + some % a.m * kRow32;
 }
 
+template <int ROWS>
 __device__ __forceinline__ void entry_stage(const ChainArgs32& a, const Exchange& ex, int row) {
   for (int c = threadIdx.x * 4; c < a.width; c += kWave * kWaves * 4) {  // (a strip's four lanes come together: the width is whole strips)
     const f32x4 v = *(const f32x4*)(a.x + (size_t)row * a.width + c), gain = *(const f32x4*)(a.layers[0].gain1 + c);
     float part = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
     part += __shfl_xor(part, 1, kWave);
     part += __shfl_xor(part, 2, kWave);
-    put_record(ex, a.stream1 + (c / 16 * a.m + row) * kRecord32, c % 16 / 4, v, gain, part);
+    const int strip = c / 16, four = c % 16 / 4;
+    const unsigned word = a.stream1 + strip * a.strip_words;
+    ex.put(word + row * kRow32 + 4 * four, marked4(v * gain));
+    ex.put(a.plain1 + (strip * a.m + row) * kRow32 + 4 * four, marked4(v));
+    if (four == 0)  // the last row's also in place of rows that there are none of
+      for (int to = row; to < (row + 1 < a.m ? row + 1 : sum_words(ROWS)); ++to) ex.put(word + a.m * kRow32 + to, marked(part));
   }
 }
 
-template <bool WIDE>
-__device__ __forceinline__ void qkv_stage(const ChainArgs32& a, const Exchange& ex, Shared32& s, int layer, int unit) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+template <bool WIDE, int ROWS>
+__device__ __forceinline__ void qkv_stage(const ChainArgs32& a, const Exchange& ex, Shared32<ROWS>& s, int layer, int unit) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const ChainLayer32& L = a.layers[layer];
   const unsigned here = layer * a.layer_words;
   const int head = unit / 2, f0 = unit % 2 * 16;  // channels f0 .. f0 + 15 of the head and those half a head on
   constexpr int kSteps = WIDE ? 16 : 6, kTogether = WIDE ? 8 : 6;
-  Product32<2, kSteps, kTogether, true> p;
+  constexpr int kEach = Ends<ROWS>::kEach;
+  Product32<ROWS, 2, kSteps, kTogether, true, WIDE> p;
   p.begin(L.w_qkv, [&](int j) { return head * HD + f0 + j * (HD / 2); }, a.width, lane, wave);
-  const int row = r < a.m ? r : a.m - 1;
-  const f32x4 c = *(const f32x4*)(a.tok_cos + row * (HD / 2) + f0 + 4 * g), sn = *(const f32x4*)(a.tok_sin + row * (HD / 2) + f0 + 4 * g);
+  const Ends<ROWS> ends(lane);
+  const int row = min(ends.row, a.m - 1), f = f0 + ends.first, operand_row = min(r, a.m - 1);
+  const Floats<kEach> c = load_floats<kEach>(a.tok_cos + row * (HD / 2) + f), sn = load_floats<kEach>(a.tok_sin + row * (HD / 2) + f);
   const int pos = a.tok_pos[row], page = a.tok_page[row];
-  ex.template gate<true>(here + a.stream1 + unit * 61 % (a.m * a.n_strip) * kRecord32, wave);
-  p.run(ex, (here + a.stream1 + row * kRecord32) * 4, a.m * kRecord32 * 4);
-  f32x4 sums[2];
+  ex.template gate<true>(a_row(a, here + a.stream1, unit * 61), wave);
+  p.run(ex, s, (here + a.stream1 + operand_row * kRow32) * 4, a.strip_words * 4, here + a.stream1 + a.m * kRow32, operand_row, a.inv_width, a.eps);
+  Floats<kEach> sums[2], out_lo, out_hi;
   float scale;
-  if (!p.finish(s, sums, scale, a.eps)) return;
-  if (r >= a.m) return;
-  const f32x4 lo = sums[0] * scale, hi = sums[1] * scale;
-  f32x4 out_lo = lo, out_hi = hi;
-  if (head < a.heads + a.kv_heads) {
-    out_lo = lo * c - hi * sn;
-    out_hi = hi * c + lo * sn;
+  if (!p.finish(s, ends, sums, scale, a.eps)) return;
+  if (ends.row >= a.m) return;
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const float lo = sums[0][e] * scale, hi = sums[1][e] * scale;
+    out_lo[e] = lo;
+    out_hi[e] = hi;
+    if (head < a.heads + a.kv_heads) {
+      out_lo[e] = lo * c[e] - hi * sn[e];
+      out_hi[e] = hi * c[e] + lo * sn[e];
+    }
   }
   unsigned to;  // [head][strip][row]
   if (head < a.heads) to = a.q + head * a.m * HD;
   else if (head < a.heads + a.kv_heads) to = a.k + (head - a.heads) * a.m * HD;
   else to = a.v + (head - a.heads - a.kv_heads) * a.m * HD;
-  to += here + (f0 / 16 * a.m + row) * 16 + 4 * g;
-  ex.put(to, marked4(out_lo));
-  ex.put(to + HD / 32 * a.m * 16, marked4(out_hi));
+  to += here + (f0 / 16 * a.m + row) * 16 + ends.first;
+  put_floats(ex, to, out_lo);
+  put_floats(ex, to + HD / 32 * a.m * 16, out_hi);
   if (page < 0 || head < a.heads) return;
-  const int f = f0 + 4 * g, in_page = pos % kPageTokens;
+  const int in_page = pos % kPageTokens;
   if (head < a.heads + a.kv_heads) {
     float* dst = L.k_pages + ((size_t)page * a.kv_heads + head - a.heads) * nnis_k_page_elems(HD);
-    *(f32x4*)(dst + nnis_k_offset(in_page, f)) = out_lo;  // 4 channels lie within a chunk of 8
-    *(f32x4*)(dst + nnis_k_offset(in_page, f + HD / 2)) = out_hi;
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {  // (a lane's channels lie within a chunk of 8)
+      dst[nnis_k_offset(in_page, f) + e] = out_lo[e];
+      dst[nnis_k_offset(in_page, f + HD / 2) + e] = out_hi[e];
+    }
   } else {
     float* dst = L.v_pages + ((size_t)page * a.kv_heads + head - a.heads - a.kv_heads) * nnis_v_page_elems(HD);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < kEach; ++e) {
       dst[nnis_v_offset(f + e, in_page)] = out_lo[e];
       dst[nnis_v_offset(f + HD / 2 + e, in_page)] = out_hi[e];
     }
@@ -214,7 +251,8 @@ __device__ __forceinline__ void qkv_stage(const ChainArgs32& a, const Exchange& 
 // A run of a sequence's keys against the query heads of a key head (up to 16: the columns), in tiles of 16 keys (attention_f32.h:
 // the same products in the same layouts).  The pages hold every key but the step's own, which comes from the exchange and takes
 // its place in its tile's operands.
-__device__ __forceinline__ void attention_stage(const ChainArgs32& a, const Exchange& ex, Shared32& s, int layer, int item) {
+template <int ROWS>
+__device__ __forceinline__ void attention_stage(const ChainArgs32& a, const Exchange& ex, Shared32<ROWS>& s, int layer, int item) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
   const ChainLayer32& L = a.layers[layer];
   const unsigned here = layer * a.layer_words;
@@ -250,7 +288,7 @@ __device__ __forceinline__ void attention_stage(const ChainArgs32& a, const Exch
     load_keys(other, i + stride);
     load_values(other, i + stride);
   }
-  ex.template gate<true>(here + a.stream1 + item * 61 % (a.m * a.n_strip) * kRecord32, wave);
+  ex.template gate<true>(a_row(a, here + a.stream1, item * 61), wave);
   const int head = kv_head * group + (r < group ? r : 0);
   f32x4 q[HD / 16], own_k[HD / 16];
   float own_v[HD / 16];
@@ -309,8 +347,7 @@ __device__ __forceinline__ void attention_stage(const ChainArgs32& a, const Exch
     for (int e = 0; e < 4; ++e) sc[e] = key0 + 4 * g + e <= pos ? sc[e] : -INFINITY;
     const float top = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
     if (__any(top > reference + kRise)) {
-      float m = fmaxf(top, __shfl_xor(top, 16, kWave));
-      m = fmaxf(fmaxf(m, __shfl_xor(m, 32, kWave)), reference);
+      const float m = fmaxf(most_32_apart(most_16_apart(top)), reference);
       const float factor = reference == -INFINITY ? 0.0f : expf(reference - m);
       reference = m;
       sum *= factor;
@@ -332,32 +369,44 @@ __device__ __forceinline__ void attention_stage(const ChainArgs32& a, const Exch
     take_tile(one);
     if (i < tiles) take_tile(other);
   }
-  sum += __shfl_xor(sum, 16, kWave);
-  sum += __shfl_xor(sum, 32, kWave);
+  sum = sum_32_apart(sum_16_apart(sum));
   if (r < group) {
 #pragma unroll
     for (int c = 0; c < HD / 16; ++c) *(f32x4*)&s.attention.o[wave][r][16 * c + 4 * g] = o[c];
   }
   if (g == 0) {
     s.attention.m[wave][r] = reference;
-    s.attention.l[wave][r] = sum;
+    s.attention.o[wave][r][HD] = sum;
   }
   __syncthreads();
   const Exchange runs(a, a.run_words, a.run_bytes);
+  // every wave makes the weights of its states once, a lane a (state, head)
+  float (*weights)[kWaves] = s.attention.weights[wave];
+  for (int at = lane; at < group * kWaves; at += kWave) {
+    const float m = s.attention.m[at % kWaves][at / kWaves];
+    float top = m;
+    top = fmaxf(top, __shfl_xor(top, 1, kWave));
+    top = fmaxf(top, __shfl_xor(top, 2, kWave));
+    top = fmaxf(top, __shfl_xor(top, 4, kWave));
+    weights[at / kWaves][at % kWaves] = m == -INFINITY ? 0.0f : expf(m - top);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   // four channels of a head a thread, and one thread a head for the run's reference and sum
   for (int at = threadIdx.x; at < group * (HD / 4 + 1); at += kWave * kWaves) {
     const int in_group = at / (HD / 4 + 1), four = at % (HD / 4 + 1), of_head = kv_head * group + in_group;
-    float top = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, s.attention.m[w][in_group]);
     f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float m = s.attention.m[w][in_group], weight = m == -INFINITY ? 0.0f : expf(m - top);
+      const float weight = weights[in_group][w];
       num += *(const f32x4*)&s.attention.o[w][in_group][four < HD / 4 ? 4 * four : 0] * weight;
-      den += s.attention.l[w][in_group] * weight;
+      den += s.attention.o[w][in_group][HD] * weight;
     }
+    float top = s.attention.m[0][in_group];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, s.attention.m[w][in_group]);
     if (a.splits == 1) {
       num *= 1.0f / den;
       if (four < HD / 4) ex.put(here + a.attn + ((of_head * (HD / 16) + four / 4) * a.m + token) * 16 + four % 4 * 4, marked4(num));
@@ -404,86 +453,112 @@ __device__ __forceinline__ void combine_stage(const ChainArgs32& a, const Exchan
   ex.put(here + a.attn + ((head * (HD / 16) + channel / 16) * a.m + row) * 16 + channel % 16, marked4(out));
 }
 
-template <bool WIDE, bool DOWN>
-__device__ __forceinline__ void strip_stage(const ChainArgs32& a, const Exchange& ex, Shared32& s, int layer, int strip) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+template <bool WIDE, int ROWS, bool DOWN>
+__device__ __forceinline__ void strip_stage(const ChainArgs32& a, const Exchange& ex, Shared32<ROWS>& s, int layer, int strip) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const ChainLayer32& L = a.layers[layer];
   const unsigned here = layer * a.layer_words, next = here + (DOWN ? a.layer_words : 0);
   const int k = DOWN ? a.inner : a.heads * HD;
   const bool last = layer + 1 == a.layer_count;
   constexpr int kSteps = WIDE ? (DOWN ? 32 : 16) : (DOWN ? 12 : 6), kTogether = WIDE ? 8 : 6;
-  Product32<1, kSteps, kTogether, false> p;
+  constexpr int kEach = Ends<ROWS>::kEach;
+  Product32<ROWS, 1, kSteps, kTogether, false, false> p;
   p.begin(DOWN ? L.w_down : L.w_o, [&](int) { return strip * 16; }, k, lane, wave);
-  const int row = r < a.m ? r : a.m - 1, column = strip * 16 + 4 * g;
-  const f32x4 gain = *(const f32x4*)((DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2) + column);
+  const Ends<ROWS> ends(lane);
+  const int row = min(ends.row, a.m - 1), column = strip * 16 + ends.first;
+  const Floats<kEach> gain = load_floats<kEach>((DOWN ? (last ? L.gain1 : a.layers[layer + 1].gain1) : L.gain2) + column);
   if (WIDE || DOWN) ex.template gate<true>(here + (DOWN ? a.act : a.attn) + strip * 61 % (a.m * k / 16) * 16, wave);
   else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<true>(layer * a.layer_runs + (strip * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
   else ex.template gate<true>(here + a.q + strip * 61 % (a.m * a.heads * HD), wave);
+  // (the stream is two stages old and more: it is there, and what is looked at before the products is rarely looked for behind them)
   u32x4 held[1];
-  if (wave == 0) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + (strip * a.m + row) * kRecord32 + kStream32 + 4 * g) * 4, 0}; });
-  p.run(ex, (here + (DOWN ? a.act : a.attn) + row * 16) * 4, a.m * 64);
-  f32x4 sums[1];
+  auto held_from = [&](int) { return At{(here + (DOWN ? a.plain2 : a.plain1) + (strip * a.m + row) * kRow32 + ends.first / 4 * 4) * 4, 0}; };
+  const bool held_there = wave != 0 || ex.template look<kPastCaches>(held, held_from);
+  p.run(ex, s, (here + (DOWN ? a.act : a.attn) + min(r, a.m - 1) * 16) * 4, a.m * 64, 0, 0, 0.0f, 0.0f);
+  if (!held_there) ex.take(held, held_from);
+  Floats<kEach> sums[1];
   float unused;
-  if (!p.finish(s, sums, unused, 0.0f)) return;
-  if (r >= a.m) return;
+  if (!p.finish(s, ends, sums, unused, 0.0f)) return;
   if (DOWN && last) {  // (the final norm's kernel adds it to the stream)
-    *(f32x4*)(a.y_out + (size_t)row * a.width + column) = sums[0];
+    if (ends.row < a.m) {
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) a.y_out[(size_t)row * a.width + column + e] = sums[0][e];
+    }
     return;
   }
-  const f32x4 v = __builtin_bit_cast(f32x4, held[0]) + sums[0];
-  float part = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-  part += __shfl_xor(part, 16, kWave);
-  part += __shfl_xor(part, 32, kWave);
-  put_record(ex, next + (DOWN ? a.stream1 : a.stream2) + (strip * a.m + row) * kRecord32, g, v, gain, part);
-  if (!DOWN && last) *(f32x4*)(a.x_out + (size_t)row * a.width + column) = v;
+  Floats<kEach> v, operand;
+  float part = 0.0f;
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    v[e] = __uint_as_float(kEach == 4 ? held[0][e] : kEach == 2 ? (ends.first % 4 ? held[0][2 + e % 2] : held[0][e]) : held[0][ends.first % 4]) + sums[0][e];
+    operand[e] = v[e] * gain[e];
+  }
+  if constexpr (kEach == 4) {
+    part = (v[0] * v[0] + v[kEach - 3] * v[kEach - 3]) + (v[kEach - 2] * v[kEach - 2] + v[kEach - 1] * v[kEach - 1]);
+  } else {  // the lane's own, then its neighbours' of the same four channels
+    part = kEach == 2 ? v[0] * v[0] + v[kEach - 1] * v[kEach - 1] : v[0] * v[0];
+    if constexpr (kEach == 1) part += of_row<0xb1>(part) ;
+    part += of_row<kEach == 1 ? 0x4e : 0xb1>(part);
+  }
+  part = sum_32_apart(sum_16_apart(part));
+  const unsigned to = next + (DOWN ? a.stream1 : a.stream2) + strip * a.strip_words;
+  if (ends.first == 0) ex.put(to + a.m * kRow32 + ends.row, marked(part));  // (lanes beyond the rows have the last row's)
+  if (ends.row >= a.m) return;
+  put_floats(ex, to + row * kRow32 + ends.first, operand);
+  put_floats(ex, next + (DOWN ? a.plain1 : a.plain2) + (strip * a.m + row) * kRow32 + ends.first, v);
+  if (!DOWN && last) {
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) a.x_out[(size_t)row * a.width + column + e] = v[e];
+  }
 }
 
-template <bool WIDE>
-__device__ __forceinline__ void gate_stage(const ChainArgs32& a, const Exchange& ex, Shared32& s, int layer, int unit) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16, g = lane / 16;
+template <bool WIDE, int ROWS>
+__device__ __forceinline__ void gate_stage(const ChainArgs32& a, const Exchange& ex, Shared32<ROWS>& s, int layer, int unit) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, r = lane % 16;
   const ChainLayer32& L = a.layers[layer];
   const unsigned here = layer * a.layer_words;
   constexpr int kSteps = WIDE ? 16 : 6, kTogether = WIDE ? 8 : 6;
-  Product32<2, kSteps, kTogether, true> p;
+  constexpr int kEach = Ends<ROWS>::kEach;
+  Product32<ROWS, 2, kSteps, kTogether, true, WIDE> p;
   p.begin(L.w_gate_up, [&](int j) { return j * a.inner + unit * 16; }, a.width, lane, wave);
-  const int row = r < a.m ? r : a.m - 1;
-  ex.template gate<true>(here + a.stream2 + unit * 61 % (a.m * a.n_strip) * kRecord32, wave);
-  p.run(ex, (here + a.stream2 + row * kRecord32) * 4, a.m * kRecord32 * 4);
-  f32x4 sums[2];
+  const Ends<ROWS> ends(lane);
+  const int operand_row = min(r, a.m - 1);
+  ex.template gate<true>(a_row(a, here + a.stream2, unit * 61), wave);
+  p.run(ex, s, (here + a.stream2 + operand_row * kRow32) * 4, a.strip_words * 4, here + a.stream2 + a.m * kRow32, operand_row, a.inv_width, a.eps);
+  Floats<kEach> sums[2], out;
   float scale;
-  if (!p.finish(s, sums, scale, a.eps)) return;
-  if (r >= a.m) return;
-  f32x4 out;
+  if (!p.finish(s, ends, sums, scale, a.eps)) return;
+  if (ends.row >= a.m) return;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < kEach; ++e) {
     const float gate = sums[0][e] * scale, up = sums[1][e] * scale;
     out[e] = gate / (1.0f + expf(-gate)) * up;
   }
-  ex.put(here + a.act + (unit * a.m + row) * 16 + 4 * g, marked4(out));
+  put_floats(ex, here + a.act + (unit * a.m + ends.row) * 16 + ends.first, out);
 }
 
 // Three waves a SIMD: within the 128 registers of four, the attention's two tiles a wave spill 72 of them (batch 8 behind 1,000
 // tokens 770 us and not 672).
-template <bool WIDE>
+template <bool WIDE, int ROWS>
 __global__ __launch_bounds__(kWave* kWaves) __attribute__((amdgpu_waves_per_eu(WIDE ? 2 : 3))) void chain_f32_kernel(ChainArgs32 a) {
-  __shared__ Shared32 s;
+  __shared__ Shared32<ROWS> s;
   const Exchange ex(a, a.words, a.words_bytes, !WIDE);  // (22 layers of width 2,048, 8 rows: 1,427 us and 1,435 with the look through the caches)
   int b = blockIdx.x;
-  if (b < a.n_entry) return entry_stage(a, ex, b);
+  if (b < a.n_entry) return entry_stage<ROWS>(a, ex, b);
   b -= a.n_entry;
   const int per_layer = a.n_qkv + a.n_att + a.n_comb + 2 * a.n_strip + a.n_gate;
   const int layer = b / per_layer;
   b -= layer * per_layer;
-  if (b < a.n_qkv) return qkv_stage<WIDE>(a, ex, s, layer, b);
+  if (b < a.n_qkv) return qkv_stage<WIDE, ROWS>(a, ex, s, layer, b);
   b -= a.n_qkv;
   if (b < a.n_att) return attention_stage(a, ex, s, layer, b);
   b -= a.n_att;
   if (b < a.n_comb) return combine_stage(a, ex, layer, b);
   b -= a.n_comb;
-  if (b < a.n_strip) return strip_stage<WIDE, false>(a, ex, s, layer, b);
+  if (b < a.n_strip) return strip_stage<WIDE, ROWS, false>(a, ex, s, layer, b);
   b -= a.n_strip;
-  if (b < a.n_gate) return gate_stage<WIDE>(a, ex, s, layer, b);
-  strip_stage<WIDE, true>(a, ex, s, layer, b - a.n_gate);
+  if (b < a.n_gate) return gate_stage<WIDE, ROWS>(a, ex, s, layer, b);
+  strip_stage<WIDE, ROWS, true>(a, ex, s, layer, b - a.n_gate);
 }
 
 // where the words of a layer lie; returns their number
@@ -494,8 +569,11 @@ unsigned lay_out(ChainArgs32& a) {
     at += (words + 31) / 32 * 32;
   };
   const unsigned m = a.m;
-  place(a.stream1, m * a.width * 3);
-  place(a.stream2, m * a.width * 3);
+  a.strip_words = (kRow32 * m + sum_words(a.width > 1024 ? kMostRows : m) + 15) / 16 * 16;  // (the kernels' ROWS)
+  place(a.stream1, a.width / 16 * a.strip_words);
+  place(a.stream2, a.width / 16 * a.strip_words);
+  place(a.plain1, m * a.width);
+  place(a.plain2, m * a.width);
   place(a.q, m * a.heads * HD);
   place(a.k, m * a.kv_heads * HD);
   place(a.v, m * a.kv_heads * HD);
@@ -538,7 +616,7 @@ extern "C" int nnis_chain_f32(const void* layers, int layer_count, int m, int wi
   ChainArgs32 a;
   a.layers = (const ChainLayer32*)layers; a.layer_count = layer_count;
   a.m = m; a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.splits = splits;
-  a.eps = eps; a.scale = scale;
+  a.eps = eps; a.scale = scale; a.inv_width = 1.0f / (float)width;
   a.x = x; a.x_out = x_out; a.y_out = y_out;
   a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page; a.tok_pages = tok_pages; a.max_pages = max_pages;
   a.words = (unsigned*)words; a.words_bytes = (unsigned)(word_count * 4);
@@ -556,8 +634,10 @@ extern "C" int nnis_chain_f32(const void* layers, int layer_count, int m, int wi
   NNIS_REQUIRE(blocks < (1LL << 30), "chain_f32: too many blocks");
   hipStream_t stream = (hipStream_t)stream_ptr;
   if (chain_clear(words, word_count - 32, runs, runs_needed, a.fail, stream)) return 1;
-  if (width > 1024) hipLaunchKernelGGL(chain_f32_kernel<true>, dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
-  else hipLaunchKernelGGL(chain_f32_kernel<false>, dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
+  if (width > 1024) hipLaunchKernelGGL((chain_f32_kernel<true, 16>), dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
+  else if (m <= 4) hipLaunchKernelGGL((chain_f32_kernel<false, 4>), dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
+  else if (m <= 8) hipLaunchKernelGGL((chain_f32_kernel<false, 8>), dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
+  else hipLaunchKernelGGL((chain_f32_kernel<false, 16>), dim3((unsigned)blocks), dim3(kWave * kWaves), 0, stream, a);
   NNIS_LAUNCH_CHECK("chain_f32");
   return 0;
 }
