@@ -37,6 +37,13 @@ __device__ __forceinline__ unsigned marked2(bf16_t lo, bf16_t hi) {
   return u == kNone ? 0x7fc07fc0u : u;
 }
 
+__device__ __forceinline__ unsigned pack2(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
+}
+__device__ __forceinline__ unsigned marked2(unsigned packed) { return packed == kNone ? 0x7fc07fc0u : packed; }
+
 // where a lane reads: its own part of a byte offset, and the part that is the wave's
 struct At {
   unsigned lane, wave;

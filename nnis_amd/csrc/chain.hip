@@ -64,13 +64,6 @@ struct ChainArgs {
 // 1.4 us after the last of them was written, where rows side by side take 0.7.  Parts of 36 blocks in one line took a reader 1.2 us more.)
 constexpr int kRowWords = 8;     // of a strip of an operand
 constexpr int kPlainWords = 16;  // ... of the stream
-__device__ __forceinline__ unsigned pack2(float lo, float hi) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2;
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
-}
-__device__ __forceinline__ unsigned marked2(unsigned packed) { return packed == kNone ? 0x7fc07fc0u : packed; }
-
 // a lane's channels in 16 bits, two a word: words[0 .. 1], of which `packed_words` are the lane's (with one channel a lane every other lane has a word)
 template <int N>
 __device__ __forceinline__ void pack_row(const Floats<N>& v, unsigned (&words)[2]) {

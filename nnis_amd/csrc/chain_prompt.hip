@@ -39,7 +39,7 @@ struct PromptLayer {
 struct PromptArgs {
   const PromptLayer* layers;
   int layer_count, m, tiles, width, heads, kv_heads, inner, gain_dtype;
-  float eps, scale_log2;
+  float eps, scale_log2, inv_width;
   const float* x;  // [m, width]
   float* x_out;    // [m, width]: the stream behind the last attention
   bf16_t* y_out;   // [m, width]: what the last feed-forward adds to it
@@ -178,16 +178,14 @@ struct PromptProduct {
       float total = s.product.squares[first][t][lane];
 #pragma unroll
       for (int p = 1; p < PARTS; ++p) total += s.product.squares[first + p][t][lane];
-      total += __shfl_xor(total, 16, kWave);
-      total += __shfl_xor(total, 32, kWave);
-      scale = 1.0f / sqrtf(total * (1.0f / (float)a.width) + a.eps);
+      scale = 1.0f / sqrtf(sum_32_apart(sum_16_apart(total)) * a.inv_width + a.eps);
     }
     return true;
   }
 };
 
 __device__ __forceinline__ u32x2 four_bf16(f32x4 v) {
-  return (u32x2){marked2((bf16_t)v[0], (bf16_t)v[1]), marked2((bf16_t)v[2], (bf16_t)v[3])};
+  return (u32x2){marked2(pack2(v[0], v[1])), marked2(pack2(v[2], v[3]))};
 }
 
 __device__ __forceinline__ void entry_stage(const PromptArgs& a, const Exchange& ex, int tile) {
@@ -314,8 +312,7 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
     float top = reference;
 #pragma unroll
     for (int i = 0; i < 8; ++i) top = fmaxf(top, score[i / 4][i % 4]);
-    top = fmaxf(top, __shfl_xor(top, 16, kWave));
-    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+    top = most_32_apart(most_16_apart(top));
     const float base = top == -INFINITY ? 0.0f : top, shrink = __builtin_amdgcn_exp2f(reference - base);
     reference = top;
     sum *= shrink;
@@ -325,7 +322,7 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
       const float lo = __builtin_amdgcn_exp2f(score[i / 4][i % 4] - base), hi = __builtin_amdgcn_exp2f(score[i / 4][i % 4 + 1] - base);
       sum += lo;
       sum += hi;
-      p[i / 2] = (unsigned)__builtin_bit_cast(unsigned short, (bf16_t)lo) | ((unsigned)__builtin_bit_cast(unsigned short, (bf16_t)hi) << 16);
+      p[i / 2] = pack2(lo, hi);
     }
 #pragma unroll
     for (int c = 0; c < HD / 16; ++c) o[c] *= shrink;
@@ -359,8 +356,7 @@ __device__ __forceinline__ void attention_stage(const PromptArgs& a, const Excha
       from = next < 16 * tile + 16 ? next : -1;
     }
   }
-  sum += __shfl_xor(sum, 16, kWave);
-  sum += __shfl_xor(sum, 32, kWave);
+  sum = sum_32_apart(sum_16_apart(sum));
 #pragma unroll
   for (int c = 0; c < HD / 16; ++c) *(f32x4*)&s.attention.o[wave][r][16 * c + 4 * g] = o[c];
   if (g == 0) {
@@ -404,8 +400,11 @@ __device__ __forceinline__ void strip_stage(const PromptArgs& a, const Exchange&
   const int tile = min(tile0 + wave, a.tiles - 1), row = tile * 16 + r;
   const unsigned piece = strip * a.tiles + tile;
   u32x4 held[1];
-  if (wave < P::kBlockTiles) ex.take(held, [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + piece * kPlain + r * 16 + 4 * g) * 4, 0}; });
+  // (two stages old and more: looked at before the products, and rarely looked for behind them)
+  auto held_from = [&](int) { return At{(here + (DOWN ? a.stream2 : a.stream1) + piece * kPlain + r * 16 + 4 * g) * 4, 0}; };
+  const bool held_there = wave >= P::kBlockTiles || ex.template look<kPastCaches>(held, held_from);
   p.run(a, ex, from);
+  if (!held_there) ex.take(held, held_from);
   f32x4 sums[1];
   float unused;
   if (!p.finish(a, s, tile0, sums, unused)) return;
@@ -425,8 +424,7 @@ __device__ __forceinline__ void strip_stage(const PromptArgs& a, const Exchange&
     v[e] = __uint_as_float(held[0][e]) + sums[0][e];
     sq = fmaf(v[e], v[e], sq);
   }
-  sq += __shfl_xor(sq, 16, kWave);
-  sq += __shfl_xor(sq, 32, kWave);
+  sq = sum_32_apart(sum_16_apart(sq));
   const unsigned ready = next + (DOWN ? a.ready1 : a.ready2) + piece * kPrepared;
   ex.put(ready + r * 8 + 2 * g, four_bf16(v * gain));
   if (g == 0) ex.put(ready + kSums + r, marked(sq));
@@ -522,7 +520,7 @@ extern "C" int nnis_chain_prompt(const void* layers, int layer_count, int m, int
   PromptArgs a;
   a.layers = (const PromptLayer*)layers; a.layer_count = layer_count; a.m = m; a.tiles = (m + 31) / 32 * 2;
   a.width = width; a.heads = heads; a.kv_heads = kv_heads; a.inner = inner; a.gain_dtype = gain_dtype;
-  a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f;
+  a.eps = eps; a.scale_log2 = scale * 1.4426950408889634f; a.inv_width = 1.0f / (float)width;
   a.x = x; a.x_out = x_out; a.y_out = (bf16_t*)y_out; a.tok_cos = tok_cos; a.tok_sin = tok_sin; a.tok_pos = tok_pos; a.tok_page = tok_page;
   a.words = (unsigned*)words; a.words_bytes = (unsigned)(word_count * 4);
   a.layer_words = (unsigned)lay_out(a);
