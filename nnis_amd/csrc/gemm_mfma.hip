@@ -354,10 +354,11 @@ extern __shared__ __align__(16) char tile_lds[];  // NS stages of BM + BN rows o
 // 2048 132 / 120, 12288 x 11264 x 2048 515 / 482, 4096 x 28672 x 4096 835 / 765, 8192 x 8192 x 8192 902 / 820 (1.34 PFLOP/s; without
 // the buffer loads of load_to_lds it was no faster than before).  What bounds it now: the fill of each block, its epilogue,
 // and the clock under matrix load.
-template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2, bool DIRECT = false>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                                    OutT y, int m, int n, int k, int col_blocks, int ksplit,
-                                                                    float* __restrict__ partial) {
+//
+// A block's tile begins at row `row0` and column block `col_block`; of K it has part `part` of `ksplit`.
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM, int WGN, bool DIRECT>
+__device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const OutT& y, int m, int n, int k, int row0,
+                                              int col_block, int col_blocks, int part, int ksplit, float* __restrict__ partial) {
   constexpr int W = WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;  // a wave's part of the tile
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -366,37 +367,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   // One load instruction of a wave moves 64 x 16 bytes into 1 KB of LDS that is contiguous.  Of the activations
   // that is 8 rows of a stage, lane l to row l / 8, place l % 8; the swizzle is made on the way in by the
   // choice of the source: place p of row r holds chunk p ^ (r % 8).
-  constexpr int A_LOADS = BM / (8 * W), B_LOADS = BN / (8 * W);  // a wave's load instructions per step (8 rows each)
-  static_assert(A_LOADS * 8 * W == BM && B_LOADS * 8 * W == BN && (64 * W) % BM == 0, "the tile must divide among the waves");
+  constexpr int A_LOADS = (BM + 8 * W - 1) / (8 * W), B_LOADS = BN / (8 * W);  // a wave's load instructions per step (8 rows each)
+  constexpr int BM_STAGED = A_LOADS * 8 * W;  // rows that a stage has: of a tile of 160 rows 192, the last 32 nobody's
+  static_assert((DIRECT || BM_STAGED == BM) && B_LOADS * 8 * W == BN, "the tile must divide among the waves");
   constexpr int LOADS = A_LOADS + B_LOADS;
-  constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = (BM + (DIRECT ? 0 : BN)) * BK * 2;
+  constexpr int A_BYTES = BM_STAGED * BK * 2, STAGE_BYTES = (BM_STAGED + (DIRECT ? 0 : BN)) * BK * 2;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;  // (the wave's number as a scalar)
   const int wave_m = wave / WGN, wave_n = wave % WGN;
   const int r = lane % 16, g = lane / 16;
-  // Blocks go to the chip's 8 dies in turn (block i to die i % 8), and each die has an L2 of its own: the
-  // tiles are dealt so that a die's blocks cover a band of consecutive rows of X with all their column
-  // blocks, and each die reads its band once instead of every die reading all of X.
-  // With ksplit > 1 the grid holds every tile ksplit times, part p of K for each (tiles of a part together).
-  int col_block, row_block, part;
-  {
-    const int total = gridDim.x, die = blockIdx.x % 8, nth = blockIdx.x / 8;
-    const int each = total / 8, more = total % 8;  // the first `more` dies have one block more
-    const int item = die * each + (die < more ? die : more) + nth;
-    const int tiles = total / ksplit;
-    part = item / tiles;
-    const int tile = item % tiles;
-    // within the order of the tiles, kGroup row blocks go through the column blocks together, rows fastest:
-    // a column block of W serves them all while it is near
-    constexpr int kGroup = (BM >= 256 ? NNIS_LARGE_TILE_GROUP_ROWS : NNIS_TILE_GROUP_ROWS) / BM;
-    const int row_blocks = tiles / col_blocks;
-    const int group = tile / (kGroup * col_blocks), within = tile % (kGroup * col_blocks);
-    const int rows_here = min(kGroup, row_blocks - group * kGroup);
-    row_block = group * kGroup + within % rows_here;
-    col_block = within / rows_here;
-  }
-  const int row0 = row_block * BM, col0 = col_block * BN;
+  const int col0 = col_block * BN;
 
   f32x4 acc[TM][TN];
 #pragma unroll
@@ -487,7 +468,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
 
   // Behind the first steps' loads, so that one wait covers both: a prepared operand's row scales, for the
   // epilogue, and what the rotation needs of each token
-  constexpr int PG = 64 * W / BM;  // threads a row of the tile has for the parts of its sum of squares
+  constexpr int PG = 64 * W >= 4 * BM ? 4 : 64 * W >= 2 * BM ? 2 : 1;  // threads a row of the tile has for the parts of its sum of squares
   __shared__ float row_scale[EPI >= 0 ? PG : 1][EPI >= 0 ? BM : 1];  // each thread's share of a row's sum of squares
   int tok_pos[TM], tok_page[TM];
   auto ask_places = [&](const auto& to) {
@@ -502,7 +483,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   };
   if constexpr (EPI >= 0 && !SPLIT) {  // (with K in parts the reduce kernel does this)
     // a thread takes the parts pg, pg + PG, .. of its row: eight loads at a time, none waiting for another
-    const int tile_row = tid % BM, pg = tid / BM;
+    const int tile_row = tid % BM, pg = min(tid / BM, PG - 1);  // (threads beyond them make the last ones' sums again)
     const int token = row0 + tile_row < m ? row0 + tile_row : m - 1;
     float total = 0.0f;
     if (y.parts <= 8 * PG) {
@@ -564,19 +545,19 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
     // A step in four groups of products, half by half and TM / 2 row tiles each.  A group's rows are read under the
     // products of the group before it, the last group is multiplied behind the step's barrier; the next step's weights are
     // asked for in the first two groups, the activations NS - 1 steps ahead in the third.
-    constexpr int Q = TM / 2;  // rows of a quarter step: a half's tiles in two groups
+    constexpr int Q = (TM + 1) / 2;  // row tiles of a quarter step: a half's in two groups
     bf16x8 a[2][Q];
     auto read = [&](int from, int half, int group, bf16x8 (&into)[Q]) {
       const bf16x8* a_tile = (const bf16x8*)(tile_lds + from * STAGE_BYTES);
 #pragma unroll
-      for (int i = 0; i < Q; ++i) into[i] = a_tile[swizzled<CH>(wave_m * WM + (group * Q + i) * 16 + r, g * 2 + half)];
+      for (int i = 0; i < (group == 0 ? Q : TM - Q); ++i) into[i] = a_tile[swizzled<CH>(wave_m * WM + (group * Q + i) * 16 + r, g * 2 + half)];
     };
     auto multiply = [&](const bf16x8 (&rows)[Q], int group, const bf16x8 (&b)[TN]) {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < Q; ++i) acc[group * Q + i][j] = mfma(b[j], rows[i], acc[group * Q + i][j]);
+        for (int i = 0; i < (group == 0 ? Q : TM - Q); ++i) acc[group * Q + i][j] = mfma(b[j], rows[i], acc[group * Q + i][j]);
       __builtin_amdgcn_s_setprio(0);
     };
     auto run = [&](int step, bf16x8 (&here)[2][TN], bf16x8 (&next)[2][TN]) {
@@ -871,6 +852,54 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   }  // !SPLIT
 }
 
+// The tile, of `tiles` in row blocks of BM and `col_blocks` column blocks, that the block with number `block` of `blocks` has, and its part of K.
+template <int BM>
+__device__ __forceinline__ void deal_tile(int block, int blocks, int col_blocks, int ksplit, int& row_block, int& col_block, int& part) {
+  // Blocks go to the chip's 8 dies in turn (block i to die i % 8), and each die has an L2 of its own: the
+  // tiles are dealt so that a die's blocks cover a band of consecutive rows of X with all their column
+  // blocks, and each die reads its band once instead of every die reading all of X.
+  // With ksplit > 1 the grid holds every tile ksplit times, part p of K for each (tiles of a part together).
+  const int total = blocks, die = block % 8, nth = block / 8;
+  const int each = total / 8, more = total % 8;  // the first `more` dies have one block more
+  const int item = die * each + (die < more ? die : more) + nth;
+  const int tiles = total / ksplit;
+  part = item / tiles;
+  const int tile = item % tiles;
+  // within the order of the tiles, kGroup row blocks go through the column blocks together, rows fastest:
+  // a column block of W serves them all while it is near
+  constexpr int kGroup = (BM >= 256 ? NNIS_LARGE_TILE_GROUP_ROWS : NNIS_TILE_GROUP_ROWS) / BM;
+  const int row_blocks = tiles / col_blocks;
+  const int group = tile / (kGroup * col_blocks), within = tile % (kGroup * col_blocks);
+  const int rows_here = min(kGroup, row_blocks - group * kGroup);
+  row_block = group * kGroup + within % rows_here;
+  col_block = within / rows_here;
+}
+
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                    OutT y, int m, int n, int k, int col_blocks, int ksplit,
+                                                                    float* __restrict__ partial) {
+  int row_block, col_block, part;
+  deal_tile<BM>(blockIdx.x, gridDim.x, col_blocks, ksplit, row_block, col_block, part);
+  multiply_tile<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, false>(x, w, y, m, n, k, row_block * BM, col_block, col_blocks, part, ksplit, partial);
+}
+
+// Tiles of 256 x 256 (DIRECT), the rows from `tail_row` on in tiles of TAIL x 256: where the tiles' last round would leave compute units without
+// one, the same rows in more and lower tiles are that much sooner done (large_tail_rows has the rule and the figures).
+template <int TAIL, typename OutT>
+__global__ __launch_bounds__(512) void gemm_large_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, OutT y, int m, int n, int k, int col_blocks,
+                                                         int tail_row) {
+  int row_block, col_block, part;
+  const int whole = tail_row / 256 * col_blocks;
+  if (TAIL == 256 || (int)blockIdx.x < whole) {
+    deal_tile<256>(blockIdx.x, TAIL == 256 ? gridDim.x : whole, col_blocks, 1, row_block, col_block, part);
+    multiply_tile<256, 256, 64, 4, false, OutT, 2, 4, true>(x, w, y, m, n, k, row_block * 256, col_block, col_blocks, 0, 1, nullptr);
+  } else {
+    deal_tile<TAIL>(blockIdx.x - whole, gridDim.x - whole, col_blocks, 1, row_block, col_block, part);
+    multiply_tile<TAIL, 256, 64, 4, false, OutT, 2, 4, true>(x, w, y, m, n, k, tail_row + row_block * TAIL, col_block, col_blocks, 0, 1, nullptr);
+  }
+}
+
 // The parts of K that gemm_tiled_kernel left in `partial` [ksplit][m][width], added in the order of the parts,
 // and the product's epilogue: stored, or taken into the residual stream with the next norm prepared (a part of
 // a row's sum of squares per 64 columns).  A thread has 4 columns of a token, a block 16 tokens x 64 columns.
@@ -1084,16 +1113,66 @@ int tiled_ksplit(int tiles, int m, int width, int k, size_t workspace_bytes) {
   return ksplit;
 }
 
-template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2, bool DIRECT = false>
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2, int WGN = 2>
 void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int col_blocks, int row_blocks, int ksplit,
                          Workspace ws, hipStream_t stream) {
-  constexpr int lds_bytes = NS * (BM + (DIRECT ? 0 : BN)) * BK * 2;
+  constexpr int lds_bytes = NS * (BM + BN) * BK * 2;
   // beyond 64 KB a kernel has to be told once; a refusal shows as the launch's failure
-  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, DIRECT>,
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN>,
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
   (void)allowed;
-  hipLaunchKernelGGL((gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, DIRECT>), dim3((unsigned)col_blocks * row_blocks * ksplit),
+  hipLaunchKernelGGL((gemm_tiled_kernel<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN>), dim3((unsigned)col_blocks * row_blocks * ksplit),
                      dim3(64 * WGM * WGN), lds_bytes, stream, x, w, y, m, n, k, col_blocks, ksplit, ws.floats);
+}
+
+// How the rows of a product in tiles of 256 x 256 are cut: from `row` on into tiles of `height` rows (256: none lower).
+//
+// 392 tiles are a round of 256 compute units and a half, and take two.  With the last rows in lower tiles they take a round and as much as those
+// need: of 12,480 rows into 2,048 columns 8,192 in 256 tiles of 256 rows and the rest in 216 of 160.  `rounds`: what it comes to in times of a
+// whole tile, by the blocks' times in the order in which compute units are free; a tile costs its rows (lower ones 5% more a row) and
+// its fill and epilogue, `fixed`, measured as 10 us beside 44 at a K of 2,048 and 6 beside 118 at 5,632.
+struct LargeRows {
+  int row, height;
+  double rounds;
+};
+double rounds_of(long long whole, long long lower, double whole_time, double lower_time) {
+  const long long units = 256, busy = whole % units;
+  const double early = (double)(whole / units) * whole_time, late = busy ? early + whole_time : early;
+  if (lower == 0) return late;
+  for (int a = 0, b = 0;;) {  // a tiles on a unit that is free early, b on one that is free late, whichever ends first
+    if (busy == 0 || early + (a + 1) * lower_time <= late + (b + 1) * lower_time) ++a;
+    else ++b;
+    if ((units - busy) * a + busy * b >= lower) {
+      const double end = b > 0 && late + b * lower_time > early + a * lower_time ? late + b * lower_time : early + a * lower_time;
+      return end > late ? end : late;
+    }
+  }
+}
+LargeRows large_rows(int m, int col_blocks, int k) {
+  const double fixed = 450.0 / k, whole_time = 1.0 + fixed;
+  const long long row_blocks = (m + 255) / 256, tiles = row_blocks * col_blocks;
+  LargeRows best = {m, 256, rounds_of(tiles, 0, whole_time, 1.0) / whole_time};
+  const double as_is = best.rounds;
+  const int most = (int)(tiles / 256 * 256 / col_blocks);  // row blocks that whole rounds take
+  for (int whole = most; whole >= 0 && whole > most - 4; --whole)
+    for (const int height : {128, 160, 192}) {
+      const int rest = m - whole * 256;
+      if (rest <= 0) continue;
+      const long long lower = (long long)((rest + height - 1) / height) * col_blocks;
+      if (whole + lower / col_blocks > 65535) continue;
+      const double rounds = rounds_of((long long)whole * col_blocks, lower, whole_time, fixed + 1.05 * height / 256.0) / whole_time;
+      if (rounds < best.rounds && rounds < 0.97 * as_is) best = {whole * 256, height, rounds};
+    }
+  return best;
+}
+
+template <int TAIL, typename OutT>
+void launch_large_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int col_blocks, int tail_row, hipStream_t stream) {
+  constexpr int lds_bytes = 4 * 256 * 64 * 2;
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_large_kernel<TAIL, OutT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+  (void)allowed;
+  const int rows = TAIL == 256 ? (m + 255) / 256 : tail_row / 256 + (m - tail_row + TAIL - 1) / TAIL;
+  hipLaunchKernelGGL((gemm_large_kernel<TAIL, OutT>), dim3((unsigned)rows * col_blocks), dim3(512), lds_bytes, stream, x, w, y, m, n, k, col_blocks, tail_row);
 }
 
 // the tiles of 256 x 256 (DIRECT, 4 stages of 32 KB) and 256 x 192 (2 of 56 KB), 8 waves, one block a compute unit; returns the parts of a row's sum of
@@ -1102,7 +1181,11 @@ template <int BN, typename OutT>
 int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
   const int col_blocks = (columns + BN - 1) / BN, row_blocks = (m + 255) / 256;
   if constexpr (BN == 256) {
-    launch_tiled_kernel<256, 256, 64, 4, false, OutT, 2, 4, true>(x, w, y, m, n, k, col_blocks, row_blocks, 1, {nullptr, 0}, stream);
+    const LargeRows rows = large_rows(m, col_blocks, k);
+    if (rows.height == 128) launch_large_kernel<128, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
+    else if (rows.height == 160) launch_large_kernel<160, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
+    else if (rows.height == 192) launch_large_kernel<192, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
+    else launch_large_kernel<256, OutT>(x, w, y, m, n, k, col_blocks, m, stream);
   } else {
     launch_tiled_kernel<256, BN, 64, 2, false, OutT, 4, 2>(x, w, y, m, n, k, col_blocks, row_blocks, 1, {nullptr, 0}, stream);
   }
@@ -1204,7 +1287,12 @@ int pick_tile(int m, int columns, int k, int tile_hint, bool residual = false) {
       if (k < 1024 || 4LL * m < 3LL * c.rows * row_blocks) continue;
       if (rounds == 1 ? 8 * blocks < 5 * 256 : (rounds == 2 ? 8 * blocks < 7 * 256 * 2 : 2 * blocks < (2 * rounds - 1) * 256)) continue;
     }
-    const long long cost = rounds * c.rows * c.width * 100 / c.rate[depth];
+    double taken = (double)rounds;
+    if (c.tile == 4) {  // cut rows have to be 5% ahead of whole tiles of another shape
+      const LargeRows cut = large_rows(m, (int)((columns + c.width - 1) / c.width), k);
+      if (cut.height != 256) taken = cut.rounds * 1.05 < taken ? cut.rounds * 1.05 : taken;
+    }
+    const long long cost = (long long)(taken * c.rows * c.width * 100 / c.rate[depth]);
     if (best == 0 || cost < best) {
       best = cost;
       tile = c.tile;
@@ -1337,6 +1425,12 @@ extern "C" int nnis_gemm_bf16(const void* x, const void* w, void* y, int y_dtype
 // The tile that the tiled kernel takes for m rows, `columns` weight rows and a depth of k (2: 64 x 128, 3: 64 x 64,
 // 4: 256 x 256, 5: 256 x 192, 6: 128 x 128, 7: 256 x 128, 8: 128 x 192): for tests and tuning.  The second: of a product into the
 // residual stream.
+// How rows in tiles of 256 x 256 are cut (large_rows): the height of the lower tiles, 256 for none, and the row that they begin at.
+extern "C" int nnis_gemm_large_height(int m, int columns, int k, int* row) {
+  const LargeRows rows = large_rows(m, (columns + 255) / 256, k);
+  *row = rows.row;
+  return rows.height;
+}
 extern "C" int nnis_gemm_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0); }
 extern "C" int nnis_gemm_residual_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0, true); }
 

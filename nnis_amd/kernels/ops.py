@@ -61,6 +61,7 @@ _CORE_SIGNATURES = {
                         _VOID, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
     "nnis_gemm_residual_parts": [_INT, _INT],
     "nnis_gemm_tile": [_INT, _INT, _INT],
+    "nnis_gemm_large_height": [_INT, _INT, _INT, _VOID],
     "nnis_gemm_residual_tile": [_INT, _INT, _INT],
     "nnis_gemm_takes_pair": [_INT, _INT, _INT, _SIZE],
     "nnis_gemm_residual": [_VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _VOID, _SIZE, _VOID, _VOID],
@@ -1324,6 +1325,13 @@ def gemm_tile(m: int, n: int, k: int, residual: bool = False) -> int:
     one into the residual stream, which goes by rates of its own."""
     lib = core()
     return (lib.nnis_gemm_residual_tile if residual else lib.nnis_gemm_tile)(int(m), int(n), int(k))
+
+
+def gemm_large_rows(m: int, n: int, k: int):
+    """(row, height): the rows of a product in tiles of 256 x 256 from ``row`` on are cut into tiles of ``height`` x 256 (256: none lower)."""
+    row = ctypes.c_int()
+    height = core().nnis_gemm_large_height(int(m), int(n), int(k), ctypes.addressof(row))
+    return row.value, height
 
 
 def gemm_residual_parts(m: int, n: int) -> int:

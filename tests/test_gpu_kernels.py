@@ -1861,3 +1861,42 @@ def test_scaled_projection_with_k_in_parts(m, k, hint, columns):
             close(held_v[page, :, inside].double(), qkv[i, heads + kv_heads:], "values")
         else:
             assert (held_k[page, :, inside] == 7).all() and (held_v[page, :, inside] == 7).all()
+
+
+@pytest.mark.parametrize("m, n, height", [(300, 4096, 128), (2285, 8192, 128), (621, 16384, 160), (2093, 8192, 160), (741, 16384, 192), (2257, 11264, 192)])
+def test_large_tiles_with_lower_ones_behind_them(m, n, height):
+    """Rows of a product in tiles of 256 x 256 whose last are cut lower, with every epilogue: the bits of tiles of 64 x 128, which add a sum
+    up in the same order, and the parts of the sums of squares."""
+    ops = _ops()
+    torch.manual_seed(m)
+    k = 264
+    assert ops.gemm_large_rows(m, n, k)[1] == height
+    x, weight = torch.randn(m, k).bfloat16().cuda(), ops.pack_weight((torch.randn(n, k) / math.sqrt(k)).bfloat16().cuda())
+    ss = (1.0 + torch.rand(1, m)).cuda() * k
+    head_dim, kv_heads = 64, 4
+    heads = n // head_dim - 2 * kv_heads
+    angle = torch.rand(64, head_dim // 2, device="cuda") * 6
+    rope = dict(cos=torch.cos(angle), sin=torch.sin(angle), tok_slot=_i32([0] * m), tok_pos=_i32([i % 64 for i in range(m)]), heads=heads,
+                kv_heads=kv_heads, head_dim=head_dim)
+    for epilogue, width in ((ops.EPILOGUE_STORE, n), (ops.EPILOGUE_SILU, n // 2), (ops.EPILOGUE_ROPE, heads * head_dim)):
+        rows = []
+        for tile in (ops.TILE_256x256, ops.TILE_64x128):
+            y = torch.full((m, width), 9.0, dtype=torch.bfloat16, device="cuda")
+            ops.gemm_scaled(x, ss, 1, 1e-5, weight, y, epilogue, rope if epilogue == ops.EPILOGUE_ROPE else None, 16 * tile)
+            rows.append(y)
+        assert torch.equal(*rows), epilogue
+    for dtype in (torch.bfloat16, torch.float32):
+        rows = [torch.full((m + 1, n), 9.0, dtype=dtype, device="cuda") for _ in range(2)]
+        for tile, y in zip((ops.TILE_256x256, ops.TILE_64x128), rows):
+            ops.gemm_bf16(x, weight, y[:m], 16 * tile)
+        assert torch.equal(*rows) and (rows[0][m] == 9.0).all(), dtype
+    stream, gain, got = torch.randn(m, n).cuda(), (1 + 0.3 * torch.randn(n)).bfloat16().cuda(), []
+    for tile in (ops.TILE_256x256, ops.TILE_64x128):
+        resid, scaled = stream.clone(), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        parts_of = torch.full((ops.gemm_residual_parts(m, n) + 1, m), 7.0, device="cuda")
+        parts = ops.gemm_residual(x, weight, resid, gain, scaled, parts_of, tile)
+        assert (parts_of[parts:] == 7.0).all()
+        got.append((resid, scaled, parts_of[:parts].double().sum(dim=0)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    # (sums of n squares in 32 bits: sqrt(n) roundings of 2^-24 and a few more)
+    assert ((got[0][2] - got[1][2]).abs() <= 1e-5 * got[1][2]).all()
