@@ -356,7 +356,8 @@ extern __shared__ __align__(16) char tile_lds[];  // NS stages of BM + BN rows o
 // and the clock under matrix load.
 //
 // A block's tile begins at row `row0` and column block `col_block`; of K it has part `part` of `ksplit`.
-template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM, int WGN, bool DIRECT>
+// GROUPS > 1: as many groups of waves, each with a part of K and a ring of its own, whose sums meet in LDS.
+template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM, int WGN, bool DIRECT, int GROUPS = 1>
 __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const OutT& y, int m, int n, int k, int row0,
                                               int col_block, int col_blocks, int part, int ksplit, float* __restrict__ partial) {
   constexpr int W = WGM * WGN;
@@ -373,8 +374,11 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   constexpr int LOADS = A_LOADS + B_LOADS;
   constexpr int A_BYTES = BM_STAGED * BK * 2, STAGE_BYTES = (BM_STAGED + (DIRECT ? 0 : BN)) * BK * 2;
 
-  const int tid = threadIdx.x;
+  static_assert(GROUPS == 1 || (!SPLIT && !DIRECT), "groups of waves end their tile themselves");
+  const int tid = GROUPS == 1 ? threadIdx.x : threadIdx.x % (64 * W);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;  // (the wave's number as a scalar)
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * W));
+  char* const ring = tile_lds + group * NS * STAGE_BYTES;
   const int wave_m = wave / WGN, wave_n = wave % WGN;
   const int r = lane % 16, g = lane / 16;
   const int col0 = col_block * BN;
@@ -435,12 +439,12 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   // they meet the zeros that pad the packed weights' last chunk (finite times zero: the row's own last values).
   const int steps = (k + BK - 1) / BK;
   const int steps_a_part = (steps + ksplit - 1) / ksplit;
-  const int step0 = part * steps_a_part;  // this block multiplies steps step0 .. step1 - 1 (none, for a part beyond the end)
+  const int step0 = (GROUPS == 1 ? part : group) * steps_a_part;  // this block (group) multiplies steps step0 .. step1 - 1 (none, for a part beyond the end)
   const int step1 = step0 + steps_a_part < steps ? step0 + steps_a_part : steps;
   int last_chunk = k - 8 - chunk_k;  // offset of the row's last whole chunk from this lane's first
   last_chunk = last_chunk > -chunk_k ? last_chunk : -chunk_k;
   auto ask = [&](int step, int stage) {
-    char* base = tile_lds + stage * STAGE_BYTES + wave * 1024;
+    char* base = ring + stage * STAGE_BYTES + wave * 1024;
     const int k0 = step * BK;
     const int from = k0 <= last_chunk ? k0 : last_chunk;
 #pragma unroll
@@ -481,7 +485,7 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
       tok_page[i] = rope_page(to.rope, token, slot, tok_pos[i]);
     }
   };
-  if constexpr (EPI >= 0 && !SPLIT) {  // (with K in parts the reduce kernel does this)
+  if constexpr (EPI >= 0 && !SPLIT) if (group == 0) {  // (with K in parts the reduce kernel does this)
     // a thread takes the parts pg, pg + PG, .. of its row: eight loads at a time, none waiting for another
     const int tile_row = tid % BM, pg = min(tid / BM, PG - 1);  // (threads beyond them make the last ones' sums again)
     const int token = row0 + tile_row < m ? row0 + tile_row : m - 1;
@@ -517,7 +521,7 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   constexpr bool kResidual = std::is_same<OutT, ResidualOut>::value;
   constexpr bool kAskEarly = kResidual && TM * TN <= 8;
   ResidualHeld held[kAskEarly ? TM : 1][kAskEarly ? TN : 1];
-  if constexpr (kAskEarly && !SPLIT) {
+  if constexpr (kAskEarly && !SPLIT) if (group == 0) {
     const bool vector_ok = (n % 4) == 0;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -540,7 +544,7 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   // half before it, while the second is read: the operands of a half are in registers one barrier ahead.  Every
   // read of a stage is still waited for before the barrier that lets the stage be filled again, and a sum takes
   // its halves in the same order as before.
-  constexpr bool kCarry = TM * TN <= 16 && W == 8;
+  constexpr bool kCarry = TM * TN <= 16 && W == 8 && GROUPS == 1;
   if constexpr (DIRECT) {
     // A step in four groups of products, half by half and TM / 2 row tiles each.  A group's rows are read under the
     // products of the group before it, the last group is multiplied behind the step's barrier; the next step's weights are
@@ -641,12 +645,14 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
       interleave();
     }
   } else {
-  for (int step = step0; step < step1; ++step) {
+  for (int step = step0; step < (GROUPS == 1 ? step1 : step0 + steps_a_part); ++step) {  // (every group comes to as many barriers)
     ask(step + NS - 1, stage == 0 ? NS - 1 : stage - 1);
-    const bf16x8* a_tile = (const bf16x8*)(tile_lds + stage * STAGE_BYTES);
-    const bf16x8* b_tile = (const bf16x8*)(tile_lds + stage * STAGE_BYTES + A_BYTES);
+    const bf16x8* a_tile = (const bf16x8*)(ring + stage * STAGE_BYTES);
+    const bf16x8* b_tile = (const bf16x8*)(ring + stage * STAGE_BYTES + A_BYTES);
     static_assert(BK == 64, "two halves of 32 k a step");
-    if constexpr (TM * TN <= 16) {
+    if (GROUPS > 1 && step >= step1) {
+      // (a step beyond the end of K: nothing to multiply)
+    } else if constexpr (TM * TN <= 16) {
       bf16x8 a_frag[2][TM], b_frag[2][TN];  // an instruction takes 32 k: the operands of both halves of the step
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
@@ -695,6 +701,26 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   }
   }
   wait_loads_but<0>();  // the steps asked for beyond the end: nothing of this block is in flight when it ends
+  if constexpr (GROUPS > 1) {
+    // the groups' sums, added up in their order by the first
+    f32x4(*sums)[TM][TN][64 * W] = (f32x4(*)[TM][TN][64 * W])tile_lds;  // [group - 1]
+    static_assert((GROUPS - 1) * TM * TN * 64 * W * 16 <= GROUPS * NS * STAGE_BYTES, "the sums lie where the rings were");
+    __syncthreads();
+    if (group > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sums[group - 1][i][j][tid] = acc[i][j];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int other = 1; other < GROUPS; ++other)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += sums[other - 1][i][j][tid];
+  }
 
   // A part of K: the sums go to `partial` [part][token][grid column] as they are; gemm_reduce_kernel adds the
   // parts and does what would follow here.
@@ -882,6 +908,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t
   int row_block, col_block, part;
   deal_tile<BM>(blockIdx.x, gridDim.x, col_blocks, ksplit, row_block, col_block, part);
   multiply_tile<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, false>(x, w, y, m, n, k, row_block * BM, col_block, col_blocks, part, ksplit, partial);
+}
+
+template <int BM, int BN, int NS, int GROUPS, typename OutT, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN * GROUPS) void gemm_grouped_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, OutT y, int m, int n, int k,
+                                                                              int col_blocks) {
+  int row_block, col_block, part;
+  deal_tile<BM>(blockIdx.x, gridDim.x, col_blocks, 1, row_block, col_block, part);
+  multiply_tile<BM, BN, 64, NS, false, OutT, WGM, WGN, false, GROUPS>(x, w, y, m, n, k, row_block * BM, col_block, col_blocks, 0, GROUPS, nullptr);
 }
 
 // Tiles of 256 x 256 (DIRECT), the rows from `tail_row` on in tiles of TAIL x 256: where the tiles' last round would leave compute units without
@@ -1192,6 +1226,30 @@ int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, i
   return 2 * col_blocks;
 }
 
+// Four groups of waves with a quarter of K each: up to 64 rows of a product that a norm prepared, where tiles of 64 x 64 are so few that their K
+// would go in parts through memory and a kernel of its own (5 us of 11).  Tiles of 32 x 32 where a compute unit has one at most, else of
+// 64 x 32.  Microseconds in parts, in tiles of 32 x 32 and of 64 x 32, with the rotation: 64 rows x 2560 x 2048 11.3, 8.9 and 11.1, 17 rows 10.1,
+// 8.1 and 9.1; 64 x 6144 x 2048 14.4, 15.8 (two rounds) and 11.9, 17 rows 11.1, 9.1 and 10.0.  Not for products into the stream, whose long K is
+// one unit's to read: 64 x 2048 x 5632 12.5, 15.9 and 22.0.
+constexpr int kGroups = 4, kGroupedRowsMost = 64;
+int grouped_tile(int m, int columns, int k, bool parts) {
+  if (!parts || m <= 16 || m > kGroupedRowsMost || k < 1024 || k > 4096) return 0;
+  const int strips = (columns + 31) / 32;
+  return strips * ((m + 31) / 32) <= 256 ? 9 : strips <= 256 ? 10 : 0;
+}
+template <int BM, int BN, int NS, int WGM, int WGN, typename OutT>
+int launch_grouped(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
+  constexpr int GROUPS = kGroups;
+  constexpr int lds_bytes = GROUPS * NS * (BM + BN) * 64 * 2;
+  static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_grouped_kernel<BM, BN, NS, GROUPS, OutT, WGM, WGN>,
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+  (void)allowed;
+  const int col_blocks = (columns + BN - 1) / BN, row_blocks = (m + BM - 1) / BM;
+  hipLaunchKernelGGL((gemm_grouped_kernel<BM, BN, NS, GROUPS, OutT, WGM, WGN>), dim3((unsigned)col_blocks * row_blocks), dim3(64 * WGM * WGN * GROUPS), lds_bytes,
+                     stream, x, w, y, m, n, k, col_blocks);
+  return WGN * col_blocks;
+}
+
 // the tiles of 128 x 128, 128 x 192 and 256 x 128 (8 waves as 4 x 2, a wave tile of 32 x 64, 32 x 96 or 64 x 64; 3 stages
 // of 32, 40 or 48 KB:
 // one block a compute unit, whose row blocks share each column block's weights); returns the parts of a row's
@@ -1315,6 +1373,13 @@ int dispatch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k
                    int columns = 0) {
   if (columns <= 0) columns = n;
   const int tile = pick_tile(m, columns, k, tile_hint, std::is_same<OutT, ResidualOut>::value);
+  if constexpr (scaled_epilogue<OutT>::value >= 0) {
+    const int col_blocks = (columns + 63) / 64, row_blocks = (m + 63) / 64;
+    const bool parts = tile == 3 && ws.floats && tiled_ksplit(col_blocks * row_blocks, m, col_blocks * 64, k, ws.bytes) > 1;
+    const int grouped = tile_hint == 9 || tile_hint == 10 ? tile_hint : tile_hint == 0 ? grouped_tile(m, columns, k, parts) : 0;
+    if (grouped == 9) return launch_grouped<32, 32, 4, 2, 1, OutT>(x, w, y, m, n, k, columns, stream);
+    if (grouped == 10) return launch_grouped<64, 32, 3, 4, 1, OutT>(x, w, y, m, n, k, columns, stream);
+  }
   if (tile == 4) return launch_tiled_large<256, OutT>(x, w, y, m, n, k, columns, stream);
   if (tile == 5) return launch_tiled_large<192, OutT>(x, w, y, m, n, k, columns, stream);
   if (tile == 6) return launch_tiled_medium<128, 128, OutT>(x, w, y, m, n, k, columns, stream);

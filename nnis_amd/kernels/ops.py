@@ -1318,6 +1318,7 @@ def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, r
 
 # tiles of the tiled product (``tile`` of gemm_residual; 16 times as much as a ``split`` of gemm_bf16 / gemm_scaled)
 TILE_64x128, TILE_64x64, TILE_256x256, TILE_256x192, TILE_128x128, TILE_256x128, TILE_128x192 = 2, 3, 4, 5, 6, 7, 8
+TILE_32x32_GROUPED, TILE_64x32_GROUPED = 9, 10  # of a product that a norm prepared (``gemm_scaled``): four groups of waves share K
 
 
 def gemm_tile(m: int, n: int, k: int, residual: bool = False) -> int:
