@@ -54,6 +54,7 @@ struct ChainArgs {
   int n_strip;        // strips of the stream
   int n_qkv, n_att, n_comb, n_out, n_gate, n_down;  // blocks of a stage for a tile (the last may have fewer of the attention's two)
   int n_att_all, n_comb_all;
+  int runs_in_out;    // the output projection's blocks add the runs up themselves
   unsigned *fail, *host_fail;
 };
 
@@ -125,6 +126,17 @@ struct Product {
   // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
   // every chunk with the lane's part of its row's sum of squares, at byte `sum_at` of the strip, if SUM.
   // MORE further loads go with the first trip's, whose offsets `ask_more` gives; `more` has what they brought.
+  // the one row from LDS, [step][64], of a K that is one round
+  __device__ __forceinline__ void run_row(const bf16x8* row) {
+#pragma unroll
+    for (int d = 0; d < STEPS; ++d) {
+      if (chunk(0, d) >= chunks) continue;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int j = 0; j < STRIPS; ++j) acc[0][j] = mfma(w[d][half][j], row[d * 8 + lane / 16 * 2 + half], acc[0][j]);
+    }
+  }
   template <bool SUM, int MORE, typename Sum, typename AskMore>
   __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, unsigned sum_at, Sum sum, u32x4 (&more)[MORE > 0 ? MORE : 1], AskMore ask_more) {
     static_assert(!SUM || MORE == 0, "one or the other");
@@ -180,6 +192,7 @@ struct Shared {
       float acc[WAVES][4][kWave][4];
       float ss[WAVES == 4 ? 1 : WAVES][kWave];  // eight waves: a row's part from each
       RowScales<ROWS> scales;  // four waves
+      bf16x8 row[WAVES == 4 && ROWS <= 4 ? WAVES : 1][4 * HD / 8];  // what a wave makes of one row's runs, [step][64]
     } product;
     struct {
       __attribute__((aligned(16))) float o[WAVES][4][HD + 4];  // a head's outputs, then its sum's four parts
@@ -721,7 +734,24 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   u32x4 held[1], none[1];
   auto held_from = [&](int) { return At{held_at * 4, 0}; };
   const bool held_there = wave >= kUnits || ex.template look<kPastCaches>(held, held_from);
-  p.template run<false, 0>(ex, (here + (DOWN ? a.act : a.attn) + min(r, a.m - 1) * 8) * 4, a.m * 32, 0, [](int, float) {}, none, [](int) { return At{0, 0}; });
+  bool from_runs = false;
+  if constexpr (!DOWN && WAVES == 4 && ROWS <= 4) {
+    from_runs = a.runs_in_out;
+    if (from_runs && wave < min(p.parts, p.chunks)) {
+      // One row: a head is a step of K, and 16 lanes of the wave that multiplies it add its runs up (an exchange less: 30 layers of width
+      // 576 behind 700 keys 370 -> 347 us, behind 3,000 in eight runs 403 -> 383; of 2 rows 378 and 380, of 4 382 and 433).
+      const Exchange runs(a, a.run_words, a.run_bytes);
+      const int head = min(p.chunk(0, lane / 16), p.chunks - 1), channel = lane % 16 * 4;
+      const unsigned first_run = layer * a.layer_runs + head * a.splits * kRunRow;
+      ((bf16x4*)s.product.row[wave])[lane] = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, false) : sum_runs<8>(runs, first_run, a.splits, channel, false);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      p.run_row(s.product.row[wave]);
+    }
+  }
+  if (!from_runs)
+    p.template run<false, 0>(ex, (here + (DOWN ? a.act : a.attn) + min(r, a.m - 1) * 8) * 4, a.m * 32, 0, [](int, float) {}, none, [](int) { return At{0, 0}; });
   if (!held_there) ex.take(held, held_from);
   Floats<kEach> sums[1];
   if constexpr (PAIRED) {
@@ -978,7 +1008,8 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
   const int last = m - (a.tiles - 1) * kMostRows;
   auto att = [&](int rows) { return rows * kv_heads * ((heads / kv_heads + 3) / 4) * splits; };
-  auto comb = [&](int rows) { return splits > 1 ? (rows * heads + 4 * waves - 1) / (4 * waves) : 0; };
+  a.runs_in_out = waves == 4 && splits > 1 && splits <= 8 && m == 1 && heads <= 16;  // (16 heads are one round of K)
+  auto comb = [&](int rows) { return splits > 1 && !a.runs_in_out ? (rows * heads + 4 * waves - 1) / (4 * waves) : 0; };
   a.n_att = att(a.m);
   a.n_att_all = (a.tiles - 1) * a.n_att + att(last);
   a.n_comb = comb(a.m);
