@@ -1706,7 +1706,7 @@ def decode_max_waves(heads: int, kv_heads: int, head_dim: int, value_dim=None, s
     return attention_module(head_dim, value_dim, softcap, extras, pooled, terms).nnis_attention_decode_max_waves(heads, kv_heads)
 
 
-def decode_plan(batch: int, kv_heads: int, longest: int, max_waves: int = 4, width: int = 0, columns: bool = False):
+def decode_plan(batch: int, kv_heads: int, longest: int, max_waves: int = 4, width: int = 0):
     """(splits, waves) of a decode step's attention.  A block of 4 waves deals
     a sequence's pages among its waves.  Cutting the keys into runs for more
     blocks costs a second kernel that sums the runs (dearer the more runs), so
@@ -1724,14 +1724,7 @@ def decode_plan(batch: int, kv_heads: int, longest: int, max_waves: int = 4, wid
     4 waves): batch 1 at 1k keys 0.839/0.822/0.790/0.775, at 128 to 2k
     0.957/0.882/0.823/0.790, at 256 keys 0.724/0.742/0.741/0.749; batch 8 at 1k
     0.943/0.952/0.919/0.914, at 128 to 2k 1.051/0.968/0.910/0.890, at 512 keys
-    0.874/0.900/0.881/0.893.
-    ``columns``: groups of more than four heads of up to 64 channels, whose
-    kernel fits two waves a SIMD: eight waves deal a run's pages, in up to four
-    runs (32/4 heads, whole steps of 22 layers in microseconds with four and
-    eight waves: 64 sequences of 17 to 2,000 keys 1,552 and 1,517, of 300 to
-    400 1,304 and 1,297; 32 of 17 to 2,000 in two runs 1,371 and 1,357; 16 of
-    100 to 2,000 in four 1,175 and 1,172; 8 of 17 to 2,000 in four 1,059 and
-    1,050, in eight 1,037 and 1,042)."""
+    0.874/0.900/0.881/0.893."""
     pages = (longest + 63) // 64
     waves = 1
     while waves * 2 <= min(max_waves, pages):
@@ -1748,8 +1741,6 @@ def decode_plan(batch: int, kv_heads: int, longest: int, max_waves: int = 4, wid
         # key-value heads of 64, whole steps: 1,000 to 1,100 keys each 16,230 tokens/s against 15,900, 128 to 2k
         # 15,620 either way); at four blocks a unit four waves are faster (batch 32: 12,010 against 11,600)
         waves = min(waves, 2)
-    if columns and waves == 4 and pages > 4 and splits <= 4:
-        waves = 8
     return splits, waves
 
 
@@ -1903,7 +1894,7 @@ def attention(q: torch.Tensor, out: torch.Tensor, view, ctx, heads: int, kv_head
     fast = attention_on_matrix_cores(q.dtype, view.k_pages.dtype, head_dim, value_dim, softcap, extras)
     size = max(head_dim, value_dim)  # what a wave's registers are sized by
     if fast and ctx.decode and heads // kv_heads <= 16 * (4 if size <= 64 else (2 if size <= 128 else 1)):
-        splits, waves = plan or decode_plan(ctx.batch, kv_heads, ctx.planned_len, width=heads * value_dim, columns=heads // kv_heads > 4 and size <= 64)
+        splits, waves = plan or decode_plan(ctx.batch, kv_heads, ctx.planned_len, width=heads * value_dim)
         waves = min(waves, decode_max_waves(heads, kv_heads, head_dim, value_dim, softcap, extras, pooled, terms))
         partial = None
         if splits > 1:

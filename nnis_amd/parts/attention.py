@@ -208,8 +208,7 @@ class CausalSelfAttention(Mixer):
             return None
         reach = self.window or self.chunk
         if not reach:
-            columns = self.heads // self.kv_heads > 4 and max(self.head_dim, self.value_dim) <= 64
-            return rt.ops.decode_plan(batch, self.kv_heads, longest, width=self.heads * self.value_dim, columns=columns)
+            return rt.ops.decode_plan(batch, self.kv_heads, longest, width=self.heads * self.value_dim)
         longest = min(longest, reach + 63)  # (a window of n tokens touches the pages of at most n + 63)
         runs, waves = rt.ops.decode_plan(batch, self.kv_heads, longest, width=self.heads * self.value_dim)
         # A window's keys in runs of a few pages: two waves a run (16/4 heads of 128 in a window of 1,024, whole steps of eight

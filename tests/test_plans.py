@@ -26,15 +26,6 @@ def test_decode_plan_invariants(batch, kv_heads, longest, width):
     assert decode_plan(batch, kv_heads, longest, max_waves=1, width=width)[1] == 1
 
 
-def test_decode_plan_of_groups_in_columns():
-    """Eight waves where the kernel has two a SIMD and the pages are more than four, the same runs as with four waves."""
-    for batch in (1, 8, 20, 64, 100, 600):
-        for longest in (1, 256, 257, 2000, 40000):
-            splits, waves = decode_plan(batch, 4, longest, width=2048)
-            eight = waves == 4 and longest > 256 and splits <= 4
-            assert decode_plan(batch, 4, longest, width=2048, columns=True) == (splits, 8 if eight else waves)
-
-
 def test_decode_plan_measured_cases():
     assert decode_plan(8, 3, 2048, width=576) == (8, 4)      # a narrow model: a page or two a wave
     assert decode_plan(64, 3, 2048, width=576) == (1, 4)     # no room for runs
