@@ -472,7 +472,8 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
 
   // Behind the first steps' loads, so that one wait covers both: a prepared operand's row scales, for the
   // epilogue, and what the rotation needs of each token
-  constexpr int PG = 64 * W >= 4 * BM ? 4 : 64 * W >= 2 * BM ? 2 : 1;  // threads a row of the tile has for the parts of its sum of squares
+  // threads a row of the tile has for the parts of its sum of squares (of a lower tile of DIRECT as many as of a whole one: the same sum)
+  constexpr int PG = DIRECT ? 2 : 64 * W / BM;
   __shared__ float row_scale[EPI >= 0 ? PG : 1][EPI >= 0 ? BM : 1];  // each thread's share of a row's sum of squares
   int tok_pos[TM], tok_page[TM];
   auto ask_places = [&](const auto& to) {
@@ -485,9 +486,30 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
       tok_page[i] = rope_page(to.rope, token, slot, tok_pos[i]);
     }
   };
-  if constexpr (EPI >= 0 && !SPLIT) if (group == 0) {  // (with K in parts the reduce kernel does this)
+  if constexpr (EPI >= 0 && GROUPS > 1) {
+    // as gemm_reduce_scaled_kernel adds a row's parts up: sixteen threads a row, and theirs in a tree
+    static_assert(64 * W * GROUPS % 16 == 0, "sixteen threads a row");
+    for (int tile_row = threadIdx.x / 16; tile_row < BM; tile_row += 4 * W * GROUPS) {
+      const int sub = threadIdx.x % 16, token = row0 + tile_row < m ? row0 + tile_row : m - 1;
+      float squares = 0.0f;
+      for (int p0 = sub; p0 < y.parts; p0 += 64) {
+        float part[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int p = p0 + 16 * u;
+          part[u] = y.ss_parts[(size_t)(p < y.parts ? p : y.parts - 1) * m + token];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) squares += p0 + 16 * u < y.parts ? part[u] : 0.0f;
+      }
+#pragma unroll
+      for (int offset = 1; offset < 16; offset <<= 1) squares += __shfl_xor(squares, offset, kWave);
+      if (sub == 0) row_scale[0][tile_row] = squares;
+    }
+    if constexpr (EPI == EPI_ROPE) ask_places(y);
+  } else if constexpr (EPI >= 0 && !SPLIT) {  // (with K in parts the reduce kernel does this)
     // a thread takes the parts pg, pg + PG, .. of its row: eight loads at a time, none waiting for another
-    const int tile_row = tid % BM, pg = min(tid / BM, PG - 1);  // (threads beyond them make the last ones' sums again)
+    const int tile_row = tid % BM, pg = DIRECT ? min(tid / BM, PG - 1) : tid / BM;  // (threads beyond them make the last ones' sums again)
     const int token = row0 + tile_row < m ? row0 + tile_row : m - 1;
     float total = 0.0f;
     if (y.parts <= 8 * PG) {
@@ -521,7 +543,7 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   constexpr bool kResidual = std::is_same<OutT, ResidualOut>::value;
   constexpr bool kAskEarly = kResidual && TM * TN <= 8;
   ResidualHeld held[kAskEarly ? TM : 1][kAskEarly ? TN : 1];
-  if constexpr (kAskEarly && !SPLIT) if (group == 0) {
+  if constexpr (kAskEarly && !SPLIT) {
     const bool vector_ok = (n % 4) == 0;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -740,7 +762,8 @@ __device__ __forceinline__ void multiply_tile(const bf16_t* __restrict__ x, cons
   auto scale_of = [&](int row) -> float {
     if constexpr (EPI >= 0) {
       float total;
-      if constexpr (PG == 4) total = (row_scale[0][row] + row_scale[1][row]) + (row_scale[2][row] + row_scale[3][row]);
+      if constexpr (GROUPS > 1) total = row_scale[0][row];
+      else if constexpr (PG == 4) total = (row_scale[0][row] + row_scale[1][row]) + (row_scale[2][row] + row_scale[3][row]);
       else if constexpr (PG == 2) total = row_scale[0][row] + row_scale[1][row];
       else total = row_scale[0][row];
       return 1.0f / sqrtf(total / (float)k + y.eps);
@@ -1226,20 +1249,21 @@ int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, i
   return 2 * col_blocks;
 }
 
-// Four groups of waves with a quarter of K each: up to 64 rows of a product that a norm prepared, where tiles of 64 x 64 are so few that their K
-// would go in parts through memory and a kernel of its own (5 us of 11).  Tiles of 32 x 32 where a compute unit has one at most, else of
-// 64 x 32.  Microseconds in parts, in tiles of 32 x 32 and of 64 x 32, with the rotation: 64 rows x 2560 x 2048 11.3, 8.9 and 11.1, 17 rows 10.1,
-// 8.1 and 9.1; 64 x 6144 x 2048 14.4, 15.8 (two rounds) and 11.9, 17 rows 11.1, 9.1 and 10.0.  Not for products into the stream, whose long K is
-// one unit's to read: 64 x 2048 x 5632 12.5, 15.9 and 22.0.
-constexpr int kGroups = 4, kGroupedRowsMost = 64;
-int grouped_tile(int m, int columns, int k, bool parts) {
-  if (!parts || m <= 16 || m > kGroupedRowsMost || k < 1024 || k > 4096) return 0;
+// Groups of waves with a part of K each: 33 to 64 rows of a product that a norm prepared, where tiles of 64 x 64 are so few that their K
+// would go in two or four parts through memory and a kernel of its own (5 us of 11).  The parts and the order of every sum are the same, and
+// so are the bits.  Tiles of 32 x 32 where a compute unit has one at most, else of 64 x 32; K in two parts only up to 48 rows.  Microseconds in
+// parts and so, of 64 / 48 / 33 rows: 2560 x 2048 with the rotation 11.2 / 10.7 / 10.3 and 9.7 / 9.2 / 8.6, 3072 x 1536 10.8 / 10.3 / 9.7 and 8.6 / 8.6 / 7.8,
+// 4096 x 2048 12.2 / 11.6 / 11.0 and 9.9 / 9.5 / 8.8; in two parts 6144 x 2048 13.6 / 12.9 / 12.2 and 13.9 / 12.1 / 11.0, gate/up 8192 x 2048 14.2 / 13.6 / 13.0
+// and 14.1 / 12.9 / 11.7.  Not for products into the stream, whose long K is one unit's to read: 64 x 2048 x 5632 12.5 in parts, 15.9 and 22.0 in
+// tiles of 32 x 32 and 64 x 32.
+constexpr int kGroupedRowsLeast = 33, kGroupedRowsMost = 64;  // (fewer rows are the kernel's for few tokens)
+int grouped_tile(int m, int columns, int k, int parts) {
+  if ((parts != 2 && parts != 4) || m < kGroupedRowsLeast || m > (parts == 2 ? 48 : kGroupedRowsMost) || k > 4096) return 0;
   const int strips = (columns + 31) / 32;
   return strips * ((m + 31) / 32) <= 256 ? 9 : strips <= 256 ? 10 : 0;
 }
-template <int BM, int BN, int NS, int WGM, int WGN, typename OutT>
+template <int BM, int BN, int NS, int GROUPS, int WGM, int WGN, typename OutT>
 int launch_grouped(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
-  constexpr int GROUPS = kGroups;
   constexpr int lds_bytes = GROUPS * NS * (BM + BN) * 64 * 2;
   static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_grouped_kernel<BM, BN, NS, GROUPS, OutT, WGM, WGN>,
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
@@ -1345,12 +1369,7 @@ int pick_tile(int m, int columns, int k, int tile_hint, bool residual = false) {
       if (k < 1024 || 4LL * m < 3LL * c.rows * row_blocks) continue;
       if (rounds == 1 ? 8 * blocks < 5 * 256 : (rounds == 2 ? 8 * blocks < 7 * 256 * 2 : 2 * blocks < (2 * rounds - 1) * 256)) continue;
     }
-    double taken = (double)rounds;
-    if (c.tile == 4) {  // cut rows have to be 5% ahead of whole tiles of another shape
-      const LargeRows cut = large_rows(m, (int)((columns + c.width - 1) / c.width), k);
-      if (cut.height != 256) taken = cut.rounds * 1.05 < taken ? cut.rounds * 1.05 : taken;
-    }
-    const long long cost = (long long)(taken * c.rows * c.width * 100 / c.rate[depth]);
+    const long long cost = rounds * c.rows * c.width * 100 / c.rate[depth];
     if (best == 0 || cost < best) {
       best = cost;
       tile = c.tile;
@@ -1375,10 +1394,12 @@ int dispatch_tiled(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k
   const int tile = pick_tile(m, columns, k, tile_hint, std::is_same<OutT, ResidualOut>::value);
   if constexpr (scaled_epilogue<OutT>::value >= 0) {
     const int col_blocks = (columns + 63) / 64, row_blocks = (m + 63) / 64;
-    const bool parts = tile == 3 && ws.floats && tiled_ksplit(col_blocks * row_blocks, m, col_blocks * 64, k, ws.bytes) > 1;
-    const int grouped = tile_hint == 9 || tile_hint == 10 ? tile_hint : tile_hint == 0 ? grouped_tile(m, columns, k, parts) : 0;
-    if (grouped == 9) return launch_grouped<32, 32, 4, 2, 1, OutT>(x, w, y, m, n, k, columns, stream);
-    if (grouped == 10) return launch_grouped<64, 32, 3, 4, 1, OutT>(x, w, y, m, n, k, columns, stream);
+    const int parts = tile == 3 && ws.floats ? tiled_ksplit(col_blocks * row_blocks, m, col_blocks * 64, k, ws.bytes) : 1;
+    const int grouped = tile_hint == 0 ? grouped_tile(m, columns, k, parts) : 0;
+    if (grouped == 9 && parts == 2) return launch_grouped<32, 32, 8, 2, 2, 1, OutT>(x, w, y, m, n, k, columns, stream);
+    if (grouped == 9) return launch_grouped<32, 32, 4, 4, 2, 1, OutT>(x, w, y, m, n, k, columns, stream);
+    if (grouped == 10 && parts == 2) return launch_grouped<64, 32, 6, 2, 4, 1, OutT>(x, w, y, m, n, k, columns, stream);
+    if (grouped == 10) return launch_grouped<64, 32, 3, 4, 4, 1, OutT>(x, w, y, m, n, k, columns, stream);
   }
   if (tile == 4) return launch_tiled_large<256, OutT>(x, w, y, m, n, k, columns, stream);
   if (tile == 5) return launch_tiled_large<192, OutT>(x, w, y, m, n, k, columns, stream);
@@ -1490,6 +1511,13 @@ extern "C" int nnis_gemm_bf16(const void* x, const void* w, void* y, int y_dtype
 // The tile that the tiled kernel takes for m rows, `columns` weight rows and a depth of k (2: 64 x 128, 3: 64 x 64,
 // 4: 256 x 256, 5: 256 x 192, 6: 128 x 128, 7: 256 x 128, 8: 128 x 192): for tests and tuning.  The second: of a product into the
 // residual stream.
+// Whether a product that a norm prepared takes groups of waves that share K: the rows of their tiles and, times 1,000, the groups; 0: no.
+extern "C" int nnis_gemm_grouped(int m, int columns, int k, size_t workspace_bytes) {
+  if (pick_tile(m, columns, k, 0) != 3) return 0;
+  const int col_blocks = (columns + 63) / 64, parts = tiled_ksplit(col_blocks * ((m + 63) / 64), m, col_blocks * 64, k, workspace_bytes);
+  const int tile = grouped_tile(m, columns, k, parts);
+  return tile ? (tile == 9 ? 32 : 64) + 1000 * parts : 0;
+}
 // How rows in tiles of 256 x 256 are cut (large_rows): the height of the lower tiles, 256 for none, and the row that they begin at.
 extern "C" int nnis_gemm_large_height(int m, int columns, int k, int* row) {
   const LargeRows rows = large_rows(m, (columns + 255) / 256, k);

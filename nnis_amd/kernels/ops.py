@@ -61,6 +61,7 @@ _CORE_SIGNATURES = {
                         _VOID, _VOID, _VOID, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _VOID, _VOID, _INT, _VOID],
     "nnis_gemm_residual_parts": [_INT, _INT],
     "nnis_gemm_tile": [_INT, _INT, _INT],
+    "nnis_gemm_grouped": [_INT, _INT, _INT, _SIZE],
     "nnis_gemm_large_height": [_INT, _INT, _INT, _VOID],
     "nnis_gemm_residual_tile": [_INT, _INT, _INT],
     "nnis_gemm_takes_pair": [_INT, _INT, _INT, _SIZE],
@@ -1318,7 +1319,6 @@ def _check_epilogue(what: str, m: int, n: int, y: torch.Tensor, epilogue: int, r
 
 # tiles of the tiled product (``tile`` of gemm_residual; 16 times as much as a ``split`` of gemm_bf16 / gemm_scaled)
 TILE_64x128, TILE_64x64, TILE_256x256, TILE_256x192, TILE_128x128, TILE_256x128, TILE_128x192 = 2, 3, 4, 5, 6, 7, 8
-TILE_32x32_GROUPED, TILE_64x32_GROUPED = 9, 10  # of a product that a norm prepared (``gemm_scaled``): four groups of waves share K
 
 
 def gemm_tile(m: int, n: int, k: int, residual: bool = False) -> int:
@@ -1326,6 +1326,12 @@ def gemm_tile(m: int, n: int, k: int, residual: bool = False) -> int:
     one into the residual stream, which goes by rates of its own."""
     lib = core()
     return (lib.nnis_gemm_residual_tile if residual else lib.nnis_gemm_tile)(int(m), int(n), int(k))
+
+
+def gemm_grouped(m: int, n: int, k: int):
+    """(rows of a tile, groups) where ``gemm_scaled`` gives a product of these sizes to groups of waves that share K, or None."""
+    grouped = core().nnis_gemm_grouped(int(m), int(n), int(k), GEMM_WORKSPACE_BYTES)
+    return (grouped % 1000, grouped // 1000) if grouped else None
 
 
 def gemm_large_rows(m: int, n: int, k: int):
