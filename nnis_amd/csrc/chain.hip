@@ -123,9 +123,6 @@ struct Product {
     }
     if (wave < parts) ask(0);
   }
-  // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
-  // every chunk with the lane's part of its row's sum of squares, at byte `sum_at` of the strip, if SUM.
-  // MORE further loads go with the first trip's, whose offsets `ask_more` gives; `more` has what they brought.
   // the one row from LDS, [step][64], of a K that is one round
   __device__ __forceinline__ void run_row(const bf16x8* row) {
 #pragma unroll
@@ -137,6 +134,9 @@ struct Product {
         for (int j = 0; j < STRIPS; ++j) acc[0][j] = mfma(w[d][half][j], row[d * 8 + lane / 16 * 2 + half], acc[0][j]);
     }
   }
+  // the operand from the exchange: strip s of the lane's row begins at byte `row_at` + s * `stride`; sum(c, part) is called for
+  // every chunk with the lane's part of its row's sum of squares, at byte `sum_at` of the strip, if SUM.
+  // MORE further loads go with the first trip's, whose offsets `ask_more` gives; `more` has what they brought.
   template <bool SUM, int MORE, typename Sum, typename AskMore>
   __device__ __forceinline__ void run(const Exchange& ex, unsigned row_at, unsigned stride, unsigned sum_at, Sum sum, u32x4 (&more)[MORE > 0 ? MORE : 1], AskMore ask_more) {
     static_assert(!SUM || MORE == 0, "one or the other");
@@ -192,7 +192,7 @@ struct Shared {
       float acc[WAVES][4][kWave][4];
       float ss[WAVES == 4 ? 1 : WAVES][kWave];  // eight waves: a row's part from each
       RowScales<ROWS> scales;  // four waves
-      bf16x8 row[WAVES == 4 && ROWS <= 4 ? WAVES : 1][4 * HD / 8];  // what a wave makes of one row's runs, [step][64]
+      bf16x8 row[ROWS <= 4 ? WAVES : 1][4 * HD / 8];  // what a wave makes of one row's runs, [step][64]
     } product;
     struct {
       __attribute__((aligned(16))) float o[WAVES][4][HD + 4];  // a head's outputs, then its sum's four parts
@@ -726,7 +726,7 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   Floats<kEach> gain;
 #pragma unroll
   for (int e = 0; e < kEach; ++e) gain[e] = kEach == 4 ? gains[e] : kEach == 2 ? (ends.first % 4 ? gains[2 + e % 2] : gains[e]) : gains[ends.first % 4];
-  if (kOne || DOWN) ex.template gate<kOne>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
+  if (DOWN || (kOne && !(ROWS <= 4 && a.runs_in_out))) ex.template gate<kOne>(here + (DOWN ? a.act : a.attn) + block * 61 % (a.m * k / 16) * 8, wave);
   else if (a.splits > 1) Exchange(a, a.run_words, a.run_bytes).template gate<kOne>(layer * a.layer_runs + (block * 61 % (a.m * a.heads * a.splits)) * kRunRow, wave);
   else ex.template gate<kOne>(here + a.q + block * 61 % (a.m * a.heads * (HD / 2)), wave);
   // (the stream is two stages old and more: it is there, and what is looked at before the products is rarely looked for behind them)
@@ -735,7 +735,7 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
   auto held_from = [&](int) { return At{held_at * 4, 0}; };
   const bool held_there = wave >= kUnits || ex.template look<kPastCaches>(held, held_from);
   bool from_runs = false;
-  if constexpr (!DOWN && WAVES == 4 && ROWS <= 4) {
+  if constexpr (!DOWN && ROWS <= 4) {
     from_runs = a.runs_in_out;
     if (from_runs && wave < min(p.parts, p.chunks)) {
       // One row: a head is a step of K, and 16 lanes of the wave that multiplies it add its runs up (an exchange less: 30 layers of width
@@ -743,7 +743,8 @@ __device__ __forceinline__ void strip_stage(const ChainArgs& a, const Exchange& 
       const Exchange runs(a, a.run_words, a.run_bytes);
       const int head = min(p.chunk(0, lane / 16), p.chunks - 1), channel = lane % 16 * 4;
       const unsigned first_run = layer * a.layer_runs + head * a.splits * kRunRow;
-      ((bf16x4*)s.product.row[wave])[lane] = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, false) : sum_runs<8>(runs, first_run, a.splits, channel, false);
+      const bool alone = WAVES == 8 && a.heads * HD > 2040;  // (as combine_stage)
+      ((bf16x4*)s.product.row[wave])[lane] = a.splits <= 4 ? sum_runs<4>(runs, first_run, a.splits, channel, alone) : sum_runs<8>(runs, first_run, a.splits, channel, alone);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -921,7 +922,7 @@ unsigned lay_out(ChainArgs& a) {
     at += (words + 31) / 32 * 32;
   };
   const unsigned m = a.m, strips = a.width / 16;
-  a.strip_words = (kRowWords * m + sum_words(a.width > 1024 ? kMostRows : m) + 15) / 16 * 16;  // (the kernels' ROWS)
+  a.strip_words = (kRowWords * m + sum_words(a.width > 1024 && m > 4 ? kMostRows : m) + 15) / 16 * 16;  // (the kernels' ROWS)
   place(a.stream1, strips * a.strip_words);
   place(a.stream2, strips * a.strip_words);
   place(a.plain1, m * strips * kPlainWords);
@@ -1008,7 +1009,7 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   a.n_qkv = (heads + 2 * kv_heads) * 2 / units;
   const int last = m - (a.tiles - 1) * kMostRows;
   auto att = [&](int rows) { return rows * kv_heads * ((heads / kv_heads + 3) / 4) * splits; };
-  a.runs_in_out = waves == 4 && splits > 1 && splits <= 8 && m == 1 && heads <= 16;  // (16 heads are one round of K)
+  a.runs_in_out = splits > 1 && splits <= 8 && m == 1 && heads <= 4 * waves;  // (so many heads are one round of K)
   auto comb = [&](int rows) { return splits > 1 && !a.runs_in_out ? (rows * heads + 4 * waves - 1) / (4 * waves) : 0; };
   a.n_att = att(a.m);
   a.n_att_all = (a.tiles - 1) * a.n_att + att(last);
@@ -1022,7 +1023,10 @@ extern "C" int nnis_chain(const void* layers, int layer_count, int m, int width,
   NNIS_REQUIRE(blocks < (1LL << 30), "chain: too many blocks");
   hipStream_t stream = (hipStream_t)stream_ptr;
   if (chain_clear(words, word_count - 32, runs, runs_needed, a.fail, stream)) return 1;
-  if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, 16, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  // (up to four rows a lane ends one element instead of four: 32/4 heads, 22 layers, width 2048, 1 row at 500 tokens 496 -> 475 us and 4 rows
+  // 495 -> 490; 32/32 heads, 24 layers, one row 757 -> 747 and behind 3,000 tokens, whose runs `out` adds up, 847 -> 832)
+  if (waves == 8 && m <= 4) hipLaunchKernelGGL((chain_kernel<8, 4, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
+  else if (waves == 8) hipLaunchKernelGGL((chain_kernel<8, 16, false, true>), dim3((unsigned)blocks), dim3(512), 0, stream, a);
   else if (m <= 4) hipLaunchKernelGGL((chain_kernel<4, 4, false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   else if (m <= 8) hipLaunchKernelGGL((chain_kernel<4, 8, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   else if (a.tiles == 1) hipLaunchKernelGGL((chain_kernel<4, 16, false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
