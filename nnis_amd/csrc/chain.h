@@ -138,27 +138,7 @@ struct Exchange {
 __host__ __device__ constexpr int sum_words(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
 
 // What stands between a stage's last operand and its words is a chain of instructions of one wave, four cycles each and more: the
-// ends of the products are kept short.  A lane's partner 16 and 32 lanes on (a row of another lane group) by register, not by LDS:
-__device__ __forceinline__ float sum_16_apart(float v) {
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
-}
-__device__ __forceinline__ float sum_32_apart(float v) {
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
-}
-__device__ __forceinline__ float most_16_apart(float v) {
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
-}
-__device__ __forceinline__ float most_32_apart(float v) {
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-}
-template <int CONTROL>  // a lane of the same 16
-__device__ __forceinline__ float of_row(float v) {
-  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CONTROL, 0xf, 0xf, false));
-}
+// ends of the products are kept short (lanes meet by the register moves of common.h).
 
 // Which of a result's elements (16 channels of up to 16 rows) a lane ends.  The matrix instruction leaves a lane four channels of a row;
 // of up to 8 and 4 rows half and three quarters of the lanes would have none, and from LDS each takes two or one.
