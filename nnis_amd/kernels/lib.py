@@ -159,10 +159,10 @@ def _attention_recipe(rest: str) -> ModuleRecipe:
 
 # the library's own modules: ``core`` holds the kernels whose sizes are run-time arguments; attention is compiled per head size
 register_module("core", ["elementwise.hip", "residual.hip", "gemm.hip", "gemm_f32.hip", "gemm_mfma.hip", "gemm_fused.hip", "gemm_two.hip", "sampling.hip"],
-                headers=["common.h", "epilogue.h", "lds_loads.h", "product.h", "nnis_noalloc.h"], source_flags={"gemm_mfma.hip": _VECTOR_SUMS, "gemm_f32.hip": _VECTOR_SUMS, "gemm_two.hip": _VECTOR_SUMS})
+                headers=["common.h", "arguments.h", "epilogue.h", "lds_loads.h", "product.h", "nnis_noalloc.h"], source_flags={"gemm_mfma.hip": _VECTOR_SUMS, "gemm_f32.hip": _VECTOR_SUMS, "gemm_two.hip": _VECTOR_SUMS})
 register_module_family("attn_hd", _attention_recipe)
 # the mixers that carry a state of fixed size (convolution, selective scan, gated linear attention and retention, minGRU, gated delta rule)
-register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
+register_module("recurrent", ["recurrent.hip", "chunked_state.hip"], headers=["common.h", "arguments.h"], source_flags={"chunked_state.hip": _VECTOR_SUMS})
 # the layers of a step of few single tokens in one launch
 register_module("chain", ["chain.hip", "chain_f32.hip", "chain_prompt.hip"], headers=["common.h", "product.h", "chain.h"],
                 source_flags={"chain.hip": _VECTOR_SUMS, "chain_f32.hip": _VECTOR_SUMS, "chain_prompt.hip": _VECTOR_SUMS})
@@ -171,7 +171,7 @@ register_module("gated_unit", ["gated_unit.hip"], headers=["common.h"], source_f
 # Mamba-2's state spaces
 register_module("state_space", ["state_space.hip"], headers=["common.h"], source_flags={"state_space.hip": _VECTOR_SUMS})
 # attention over a cached latent: what lies between its projections (norms of the latents, rotation, cache write, gates)
-register_module("latent", ["latent.hip"], headers=["common.h"])
+register_module("latent", ["latent.hip"], headers=["common.h", "arguments.h"])
 # what lies between the projections of sublayers that norm their outputs, gate or pool their heads, or route their tokens
 register_module("sublayer", ["sublayer.hip"], headers=["common.h"])
 # a token's own input to a layer

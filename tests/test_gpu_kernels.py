@@ -1718,6 +1718,55 @@ def test_latents_of_few_and_many_rows(q_rank, kv_rank, rot, gates, rows):
         assert ((gate.cpu().double() - want).abs() <= 1e-6).all()
 
 
+@pytest.mark.parametrize("rows", [1, 5, 300])
+@pytest.mark.parametrize("size", [1, 2, 3, 4])
+def test_rows_in_16_bits_as_in_32(size, rows):
+    """Kernels that know their types when compiled against the same ones on the same values in 32 bits, whose types are branches, around
+    the sizes that part them: the same numbers but for the rounding that is stored, on whose edge a value may fall to either side."""
+    ops = _ops()
+    torch.manual_seed(10 * size + rows)
+    half = lambda *shape: torch.randn(*shape, device="cuda").bfloat16()
+
+    def alike(call, *shapes):  # call(type, outputs): the outputs of each type
+        got, want = ([torch.full(shape, 7.0, device="cuda", dtype=kind) for shape in shapes] for kind in (torch.bfloat16, torch.float32))
+        call(torch.bfloat16, *got)
+        call(torch.float32, *want)
+        for g, w in zip(got, want):
+            assert ((g.float() - w).abs() <= 2.0 ** -7 * w.abs() + 1e-6).all()
+
+    for dim in (64 * size, 64 * size + 1):  # (in registers up to 256 channels a head)
+        o, gate, weight = torch.randn(rows, 3 * dim, device="cuda"), half(rows, 3 * dim + 8)[:, 8:], half(dim)
+        for w in (weight, None):
+            alike(lambda kind, y: ops.head_norm_gate(o, gate.to(kind), None if w is None else w.to(kind), 1e-5, 3, y), (rows, 3 * dim))
+    for width in (4, 260 * size, 1024 * size):
+        ys, ws, b = [half(rows, width) for _ in range(size)], [half(width) for _ in range(size)], half(width)
+        alike(lambda kind, out: ops.branch_mean([y.to(kind) for y in ys], [w.to(kind) for w in ws], [b.to(kind)] + [None] * (size - 1), 1e-5, out), (rows, width))
+        x, mix, gain = torch.randn(size, rows, width, device="cuda"), torch.randn(size, size, device="cuda"), torch.randn(size, device="cuda")
+
+        def stream(kind, h, y, norm):
+            held = x.clone()
+            ops.stream_step(held, h, ys[0].to(kind) if y else None, mix if y else None, gain if y else None, None, ws[0].to(kind) if norm else None,
+                            b.to(kind) if norm else None, 1e-5 if norm else 0.0)
+        for y, norm in ((True, True), (True, False), (False, True)):
+            alike(lambda kind, h: stream(kind, h, y, norm), (rows, width))
+    heads, kv, dim, rot = 5 * size, size, 128, 64 if size % 2 else 128  # (112 to 480 items of four channels)
+    if rows == 5:
+        heads, kv = 16 * size, 8 * size  # (up to 2,560, beyond a block)
+    qkv, angle, pages = half(rows, (heads + 2 * kv) * dim), torch.rand(512, rot // 2, device="cuda") * 6, (rows + 63) // 64
+    slots = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    slots[3:4] = -1
+    table = torch.arange(pages, dtype=torch.int32).flip(0)[None].cuda()
+    places = [(pages, kv, dim // 8, 64, 8), (pages, kv, dim // 16, 2, 4, 16, 8)]
+    alike(lambda kind, q, k, v: ops.rope_kv_write(qkv.to(kind), q, angle.cos(), angle.sin(), rot, slots, _i32(range(rows)), k, v, table, heads, kv, dim),
+          (rows, heads * dim), *places)
+    q_rank, kv_rank, gates = 96 * (size - 1), 72 * size, 3 * (size % 2)  # (up to 288 channels, beyond a block's threads)
+    proj, q_weight, c_weight, gate = torch.randn(rows, q_rank + kv_rank + 32 + gates, device="cuda"), half(q_rank), half(kv_rank), torch.empty(rows, gates, device="cuda")
+    alike(lambda kind, cq, k, v: ops.latent_prepare(proj, q_rank, kv_rank, 32, gates, q_weight.to(kind) if q_rank else None, c_weight.to(kind), 1e-5,
+                                                    angle[:, :16].cos().contiguous(), angle[:, :16].sin().contiguous(), slots, _i32(range(rows)),
+                                                    cq if q_rank else None, k, v, table, gate if gates else None),
+          (rows, q_rank), *[_empty_pages(pages, 1, n, torch.float32, 0.0, 0.0, "cuda")[which].shape for which, n in ((0, kv_rank + 32), (1, kv_rank))])
+
+
 @pytest.mark.parametrize("kernel, heads, kv_heads", [("columns", 16, 2), ("keys", 9, 3)])
 @pytest.mark.parametrize("splits, waves", [(1, 4), (2, 2), (8, 4), (1, 1)])
 def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves):
