@@ -106,6 +106,21 @@ def test_against_the_layers(tmp_path, sizes, batch, monkeypatch):
         assert error <= bound, f"plan {plan}: {error.item():.4g} from 32 bits, the layers' kernels {(layers - want).norm().item():.4g}"
 
 
+@pytest.mark.parametrize("batch", [5, 7, 8])
+@pytest.mark.parametrize("sizes", [(320, 5, 1, 128), (1152, 16, 2, 8256)])
+def test_five_to_seven_rows_of_large_groups(tmp_path, sizes, batch, monkeypatch):
+    """A step's rows are padded to seven, which the launch takes, and not to eight, which it does not: as far from 32 bits as the layers'
+    kernels (``test_against_the_layers``)."""
+    import nnis_amd
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    want = _run(str(tmp_path), "float32", LENGTHS[:batch], None, monkeypatch)[0]
+    layers = _run(str(tmp_path), "bfloat16", LENGTHS[:batch], None, monkeypatch)[0]
+    got, ran, _ = _run(str(tmp_path), "bfloat16", LENGTHS[:batch], "own", monkeypatch)
+    assert ran == (batch < 8)
+    assert (got - want).norm() <= 1.33 * (layers - want).norm()
+
+
 @pytest.mark.parametrize("batch", [1, 3, 16])
 @pytest.mark.parametrize("sizes", SIZES + [(128, 12, 1, 192)])  # (twelve heads a key head)
 def test_32_bits_against_the_oracle(tmp_path, sizes, batch, monkeypatch):

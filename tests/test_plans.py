@@ -210,3 +210,14 @@ def test_ways_to_cut_k_that_a_launched_step_does_not_have():
     assert taken(16, 1024, 16, 2048) and not taken(1, 1024, 17, 2048) and not taken(16, 1024, 17, 2048)
     assert taken(16, 192, 4, 5056) and not taken(16, 192, 4, 5120) and taken(17, 192, 4, 5120)
     assert taken(1, 1088, 79, 8192) and not taken(1, 1088, 79, 8256) and not taken(1, 2048, 80, 2048) and taken(1, 2112, 80, 2048)
+
+
+@pytest.mark.parametrize("batch, padded, taken", [(4, 4, True), (5, 7, True), (7, 7, True), (8, 8, False), (9, 12, False)])
+def test_padding_keeps_large_groups_on_the_launch(batch, padded, taken, monkeypatch):
+    """Five to seven sequences of more than four query heads a key head are padded to the most rows that the launch through all layers takes."""
+    from nnis_amd.engine.graph import bucket
+    from nnis_amd.kernels import ops
+
+    monkeypatch.setattr(ops, "chain_takes", lambda *sizes: True)  # (the native side's sizes)
+    assert bucket(batch) == padded
+    assert (chain_plan(22, padded, 600, 2048, 32, 4, 64, 5632) is not None) == taken
