@@ -1,7 +1,7 @@
 // The layers of a step of few single tokens in one launch (pre-norm blocks of plain attention with heads of 64 channels and a
 // SiLU-gated feed-forward, bfloat16, up to 16 rows; up to a width of 1,024 32, as two tiles of rows that have nothing to do with
-// one another: 24 rows of 30 layers of width 576 1,037 us by the layers' kernels and 772, 32 rows 968 and 660, but 48 rows of 600 to 2,000
-// tokens 1,153 and 1,380 when last measured).  How long the sequences may be: kernels/ops.py, chain_longest.
+// one another: 32 rows of 30 layers of width 576 968 us by the layers' kernels; 24 and 32 rows of 100 to 800 tokens 512 and 541 us here; but
+// 48 rows of 600 to 2,000 tokens 1,153 and 1,380 when last measured).  How long the sequences may be: kernels/ops.py, chain_longest.
 //
 // What bounds such a step is neither bytes nor products but its chain of dependent kernels, five to six a layer: each begins
 // 1.6 us after the one before has ended, asks for its weights, and only then has something to multiply.  Here a layer's stages
