@@ -2128,20 +2128,14 @@ RUN_PIECE_LEAST = 16
 RUN_SCRATCH_BYTES = 256 << 20
 
 
-# Matrix states are large beside a token's work on them: where pieces of RUN_PIECE_LEAST tokens would hand on as many bytes as this, pieces have
-# twice the tokens (microseconds at 16 / 32 tokens, 8 heads of 128 x 256: 700 tokens 94 / 88, 1,500 141 / 133, 90 to 700 on four sequences 159 / 149,
-# six of 400 231 / 196; 4 heads: 700 72 / 77, four of 90 to 700 102 / 107, six of 400 137 / 123).
-RUN_STATE_BYTES = 64 << 20
-
-
-def run_pieces(ctx, state_bytes: int, least: int = RUN_PIECE_LEAST):
+def run_pieces(ctx, state_bytes: int):
     """(tokens of a piece, most pieces of a sequence) for a step whose longest run has ``ctx.max_new`` tokens, where a
     sequence's state takes ``state_bytes``; (0, 1) for a step that is not cut."""
     longest = int(ctx.max_new)
     if longest < RUN_PIECE_FROM:
         return 0, 1
     most = max(1, min(64, RUN_SCRATCH_BYTES // max(1, ctx.batch * state_bytes)))
-    piece = max(least, -(-longest // most))
+    piece = max(RUN_PIECE_LEAST, -(-longest // most))
     pieces = -(-longest // piece)
     return (piece, pieces) if pieces > 1 else (0, 1)
 
@@ -2501,9 +2495,7 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay_logs: Opti
                                               ctx.seq_start.data_ptr(), ctx.batch, tokens, heads, key_dim, value_dim, out.data_ptr(),
                                               chunks.data_ptr(), _stream()))
         return out
-    state_bytes = heads * key_dim * value_dim * 4
-    large = tokens // RUN_PIECE_LEAST * state_bytes >= RUN_STATE_BYTES
-    piece, pieces = run_pieces(ctx, state_bytes, 2 * RUN_PIECE_LEAST if large else RUN_PIECE_LEAST)
+    piece, pieces = run_pieces(ctx, heads * key_dim * value_dim * 4)
     carried = decayed = None
     if pieces > 1:
         carried = torch.empty(ctx.batch * pieces * heads * key_dim * value_dim, dtype=torch.float32, device=out.device)
