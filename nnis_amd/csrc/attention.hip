@@ -521,7 +521,8 @@ __device__ __forceinline__ float sink_term(const float* sink, int head, float re
 // asked for again behind the block).  The compiler's scheduler is told the order inside each stretch of
 // straight-line code, from behind one unit's test of its maximum to the next unit's: one of those matrix
 // instructions, a few vector instructions, and so on.
-// IN_TURN: the test and the sum as attend_block makes them, the same bits (decode, where some blocks go either way by the group's size).
+// IN_TURN: the test and the sum as attend_block makes them, the same bits: a decode group with columns to spare has them whichever of the two its
+// blocks take.  (Eight additions one after the other, where a group that fills its columns has a tree.)
 template <int C, bool AHEAD, bool IN_TURN, int c>
 __device__ __forceinline__ void attend_unit_ahead(AttnState<C>& st, const QFrag (&q)[C], const BlockFrags& f, const BlockFrags& next,
                                                   f32x4 (&s)[2], bf16x8& before, float scale_log2, float (&rise)[C], const ScoreCap& cap,
@@ -534,7 +535,7 @@ __device__ __forceinline__ void attend_unit_ahead(AttnState<C>& st, const QFrag 
   recede(s[1], more.r1[c], more.r2[c], back[c] - 4);
 #endif
   // rise[c]: the raw score (before the scale) above which column c's reference moves, (st.m[c] + kLazyRise) / scale:
-  // the test of every unit is then the scores' maximum against a register
+  // the test of every unit is then the scores' maximum against a register.  (IN_TURN: the scaled score.)
   float block_max = -INFINITY;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -849,7 +850,7 @@ __device__ __forceinline__ void attend_run(AttnState<C>& st, const QFrag (&q)[C]
   }
   // The blocks all of whose keys count for every column of every lane lie together in the middle of the run (in
   // a causal step without a window: at its start): pages n of the run with every_lo <= their keys <= every_hi.
-  // (A dead column has hi = -1: then there are none.)
+  // (A column that reads no key has hi = -1: then there are none.)
   int every_lo = lo[0], every_hi = hi[0];
 #pragma unroll
   for (int c = 1; c < C; ++c) {
@@ -1195,7 +1196,11 @@ __device__ __forceinline__ void finish_decode(AttnState<C>& st, const bool (&liv
 // ---- decode: a block = (token, kv head, split of the keys); columns are the heads of the group; ------
 // the block's waves deal the split's pages among themselves and merge their states through LDS.  With
 // more than one split every block leaves its state in `partial` for the combine kernel.
-template <int C>
+//
+// REPEATS: the group leaves columns without a head, which repeat its first: all see the same keys, and the blocks before the last need no look at
+// theirs (without keys of its own such a column sent every block the way of the masks: 32/4 heads, 64 sequences of 17 to 2,000 tokens, 22 layers
+// 1,575 -> 1,537 us).
+template <int C, bool REPEATS>
 __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(MfmaArgs a, int waves) {
   extern __shared__ __attribute__((aligned(16))) float merge[];  // [waves / 2][C][kTilesD * 4 + 2][64]
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), r = lane % 16, g = lane / 16;  // (the wave's number as a scalar)
@@ -1227,8 +1232,6 @@ __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(Mfma
     gates[c] = ask_gate(a.terms, token, head);
     take_decay(more, a, c, head);
     lo[c] = first_key;
-    // a column without a head repeats the group's first: all see the same keys, and the blocks before the last need no look at theirs (without
-    // keys of its own it sent every block the way of the masks: 32/4 heads, 64 sequences of 17 to 2,000 tokens, 22 layers 1,575 -> 1,537 us)
     hi[c] = pos;
   }
   // pages are dealt to the splits in contiguous runs, and within a split to the waves in turn
@@ -1251,16 +1254,16 @@ __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(Mfma
   const int kept_pages = split == 0 ? min(page_first, (more.keep + kPageTokens - 1) / kPageTokens) : 0;
   if (kept_pages > 0) {
     const int mine_kept = kept_pages > wave ? (kept_pages - wave + waves - 1) / waves : 0;
-    attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), true>(st, q, a, pages, kv_head, wave, waves, mine_kept, more.keep - 1, lo, hi, lane, more);
+    attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), REPEATS>(st, q, a, pages, kv_head, wave, waves, mine_kept, more.keep - 1, lo, hi, lane, more);
   }
 #endif
   const int mine = end > begin + wave ? (end - begin - wave + waves - 1) / waves : 0;  // pages of this wave
-  attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), true>(st, q, a, pages, kv_head, begin + wave, waves, mine, pos, lo, hi, lane, more);
+  attend_run<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), REPEATS>(st, q, a, pages, kv_head, begin + wave, waves, mine, pos, lo, hi, lane, more);
 #if NNIS_POOLED_BLOCKS
   // the pooled blocks go with the first run of the keys (with the step's tables the pooled pages are still the slot's)
   if (a.pool > 0 && split == 0) {
     const int pool_slot = a.rows_by_token ? a.tok_slot[token] : slot;
-    if (pool_slot >= 0) attend_pooled<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), true>(st, q, a, pool_slot, kv_head, wave, waves, lo, hi, lane);
+    if (pool_slot >= 0) attend_pooled<C, (kDecodeRing / C >= 2 ? kDecodeRing / C : 2), REPEATS>(st, q, a, pool_slot, kv_head, wave, waves, lo, hi, lane);
   }
 #endif
   finish_decode<C>(st, live, a, merge, gates, token, kv_head, split, wave, waves, lane);
@@ -1902,9 +1905,15 @@ extern "C" int nnis_attention_decode_bf16_terms(const void* q, void* out, const 
     }
   }
 #endif
-  if (tiles == 1) hipLaunchKernelGGL((attention_decode_kernel<1>), grid, dim3(kWave * waves), lds, s, a, waves);
-  else if (tiles == 2) hipLaunchKernelGGL((attention_decode_kernel<(kMaxColumns >= 2 ? 2 : 1)>), grid, dim3(kWave * waves), lds, s, a, waves);
-  else hipLaunchKernelGGL((attention_decode_kernel<kMaxColumns>), grid, dim3(kWave * waves), lds, s, a, waves);  // 3 or 4 tiles
+#define NNIS_DECODE(C_)                                                                                                         \
+  do {                                                                                                                         \
+    if (group < 16 * (C_)) hipLaunchKernelGGL((attention_decode_kernel<(C_), true>), grid, dim3(kWave * waves), lds, s, a, waves); \
+    else hipLaunchKernelGGL((attention_decode_kernel<(C_), false>), grid, dim3(kWave * waves), lds, s, a, waves);               \
+  } while (0)
+  if (tiles == 1) NNIS_DECODE(1);
+  else if (tiles == 2) NNIS_DECODE(kMaxColumns >= 2 ? 2 : 1);
+  else NNIS_DECODE(kMaxColumns);  // 3 or 4 tiles
+#undef NNIS_DECODE
   NNIS_LAUNCH_CHECK("attention_decode");
   if (splits > 1 && combine) {
     hipLaunchKernelGGL(attention_combine_kernel, dim3(tokens, heads), dim3(HDV < 64 ? 64 : (HDV > 256 ? 256 : HDV)), 0, s, partial,

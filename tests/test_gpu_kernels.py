@@ -1813,6 +1813,27 @@ def test_decode_attention_around_64_pages(kernel, heads, kv_heads, splits, waves
         assert (out.cpu().float().view(len(rows), heads, head_dim) - want).abs().max().item() <= 1e-2
 
 
+@pytest.mark.parametrize("group", [5, 8, 15, 16, 24, 32])
+def test_the_order_of_a_blocks_weights(group):
+    """A lane's eight weights of a block of keys are added one after the other; where every column has a head, the blocks in the middle of a
+    run are added in pairs.  Weights of 1 and seven times 0.92 of half a unit in its last place say which: one after the other they are
+    lost, in pairs they are three units."""
+    ops = _ops()
+    lengths, places = [1536, 1536], [256, 704]  # (a block in the middle of the first of two runs of 24 blocks, and among its last)
+    ks = [torch.zeros(n, 1, 64) for n in lengths]
+    for k, place in zip(ks, places):
+        k[:, 0, 0] = -20000.0  # (a weight of 0 beside the others)
+        k[place:place + 8, 0, 0] = torch.tensor([0.0] + 7 * [-24.125])
+    k_pages, v_pages, table = _paged(ks, ks, torch.bfloat16, 1, 64, pages=50, max_pages=24)
+    q = torch.zeros(2, group, 64, dtype=torch.bfloat16, device="cuda")
+    q[:, :, 0] = 1.0
+    out = torch.empty(2, group * 64, dtype=torch.bfloat16, device="cuda")
+    partial = torch.full((2, group, 2, 68), float("nan"), device="cuda")
+    ops.attention_decode_bf16(q.view(2, -1), out, k_pages, v_pages, table, _i32([0, 1]), _i32([1535, 1535]), group, 1, 64, math.log(2.0), 0, 2, partial, 1, "columns")
+    middle, end = partial[:, :, 0, 65].cpu()
+    assert (middle == (1.0 + 3 * 2.0 ** -23 if group % 16 == 0 else 1.0)).all() and (end == 1.0).all()
+
+
 # the four-wave tiles: their hint to the products, their columns
 FOUR_WAVE_TILES = [(48, 64), (32, 128)]
 
