@@ -1199,7 +1199,8 @@ __device__ __forceinline__ void finish_decode(AttnState<C>& st, const bool (&liv
 //
 // REPEATS: the group leaves columns without a head, which repeat its first: all see the same keys, and the blocks before the last need no look at
 // theirs (without keys of its own such a column sent every block the way of the masks: 32/4 heads, 64 sequences of 17 to 2,000 tokens, 22 layers
-// 1,575 -> 1,537 us).
+// 1,575 -> 1,537 us).  Not with the scores' extras: there the loop without masks takes a far key's bias as a shift of the reference, which
+// rounds otherwise and has no number to shift by where the bias is minus infinity (64 sequences 21.1 us a call, 18.3 with it).
 template <int C, bool REPEATS>
 __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(MfmaArgs a, int waves) {
   extern __shared__ __attribute__((aligned(16))) float merge[];  // [waves / 2][C][kTilesD * 4 + 2][64]
@@ -1232,7 +1233,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void attention_decode_kernel(Mfma
     gates[c] = ask_gate(a.terms, token, head);
     take_decay(more, a, c, head);
     lo[c] = first_key;
-    hi[c] = pos;
+    hi[c] = REPEATS || live[c] ? pos : -1;
   }
   // pages are dealt to the splits in contiguous runs, and within a split to the waves in turn
   const int page_first = first_key / kPageTokens, page_count = pos / kPageTokens + 1 - page_first;
@@ -1905,10 +1906,13 @@ extern "C" int nnis_attention_decode_bf16_terms(const void* q, void* out, const 
     }
   }
 #endif
-#define NNIS_DECODE(C_)                                                                                                         \
-  do {                                                                                                                         \
-    if (group < 16 * (C_)) hipLaunchKernelGGL((attention_decode_kernel<(C_), true>), grid, dim3(kWave * waves), lds, s, a, waves); \
-    else hipLaunchKernelGGL((attention_decode_kernel<(C_), false>), grid, dim3(kWave * waves), lds, s, a, waves);               \
+  constexpr bool kRepeats = !NNIS_SCORE_EXTRAS;
+#define NNIS_DECODE(C_)                                                                                                      \
+  do {                                                                                                                       \
+    if (kRepeats && group < 16 * (C_))                                                                                       \
+      hipLaunchKernelGGL((attention_decode_kernel<(C_), kRepeats>), grid, dim3(kWave * waves), lds, s, a, waves);            \
+    else                                                                                                                     \
+      hipLaunchKernelGGL((attention_decode_kernel<(C_), false>), grid, dim3(kWave * waves), lds, s, a, waves);               \
   } while (0)
   if (tiles == 1) NNIS_DECODE(1);
   else if (tiles == 2) NNIS_DECODE(kMaxColumns >= 2 ? 2 : 1);

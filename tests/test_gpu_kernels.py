@@ -1834,6 +1834,28 @@ def test_the_order_of_a_blocks_weights(group):
     assert (middle == (1.0 + 3 * 2.0 ** -23 if group % 16 == 0 else 1.0)).all() and (end == 1.0).all()
 
 
+@pytest.mark.parametrize("heads", [3, 8, 24])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_a_bias_that_hides_far_keys(heads, splits):
+    """A bias by distance whose last row is minus infinity, or the lowest number, leaves the keys before it out."""
+    ops = _ops()
+    torch.manual_seed(heads)
+    length, reach, scale = 3000, 40, 0.125
+    k, v = (torch.randn(length, 1, 64).bfloat16().float() for _ in range(2))
+    k_pages, v_pages, table = _paged([k], [v], torch.bfloat16, 1, 64, pages=48, max_pages=48)
+    q = torch.randn(1, heads * 64).bfloat16()
+    bias = torch.randn(heads, reach + 1)
+    bias[::2, reach], bias[1::2, reach] = float("-inf"), torch.finfo(torch.float32).min
+    out = torch.empty(1, heads * 64, dtype=torch.bfloat16, device="cuda")
+    partial = torch.empty(heads * splits * 68, device="cuda")
+    ops.attention_decode_bf16(q.cuda(), out, k_pages, v_pages, table, _i32([0]), _i32([length - 1]), heads, 1, 64, scale, 0, splits, partial, 4, "columns",
+                              extras=ops.ScoreExtras(0, bias.cuda(), None))
+    seen = slice(length - reach, length)
+    scores = q.double().view(heads, 64) @ k[seen, 0].double().T * scale + bias[:, :reach].flip(1).double()
+    want = scores.softmax(dim=1) @ v[seen, 0].double()
+    assert (out.cpu().double().view(heads, 64) - want).abs().max().item() <= 2e-2  # (probabilities and outputs in 16 bits, values up to 4)
+
+
 # the four-wave tiles: their hint to the products, their columns
 FOUR_WAVE_TILES = [(48, 64), (32, 128)]
 
