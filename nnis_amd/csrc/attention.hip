@@ -584,8 +584,9 @@ __device__ __forceinline__ void attend_unit_ahead(AttnState<C>& st, const QFrag 
     for (int t = 0; t < kTilesD; ++t)
       st.o[c - 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.values[t], before, st.o[c - 1][t], 0, 0, 0);
   }
-  // (No key of these blocks is masked: behind the test above the reference is a score's own size, never -inf.)
-  const float base = st.m[c];
+  // (No key of these blocks is masked: behind the test above the reference is a score's own size, -inf only where all of a column's scores were so far.
+  // IN_TURN takes such scores as attend_block does: no weight.)
+  const float base = IN_TURN && st.m[c] == -INFINITY ? 0.0f : st.m[c];
   bf16x8 p;
   float w[8];
 #pragma unroll

@@ -1856,6 +1856,25 @@ def test_a_bias_that_hides_far_keys(heads, splits):
     assert (out.cpu().double().view(heads, 64) - want).abs().max().item() <= 2e-2  # (probabilities and outputs in 16 bits, values up to 4)
 
 
+@pytest.mark.parametrize("heads, kv_heads", [(8, 1), (5, 1), (24, 1), (9, 3)])
+def test_keys_whose_scores_are_minus_infinity(heads, kv_heads):
+    """A sequence's first pages of keys score minus infinity: they have no weight, and the others theirs."""
+    ops = _ops()
+    torch.manual_seed(heads)
+    length, hidden = 1500, 200
+    k, v = (torch.randn(length, kv_heads, 64).bfloat16().float() for _ in range(2))
+    k[:, :, 0], k[:hidden, :, 0] = 0.0, -2.0 ** 100
+    k_pages, v_pages, table = _paged([k], [v], torch.bfloat16, kv_heads, 64, pages=24, max_pages=24)
+    q = torch.randn(1, heads, 64).bfloat16()
+    q[:, :, 0] = 2.0 ** 100
+    out = torch.empty(1, heads * 64, dtype=torch.bfloat16, device="cuda")
+    for waves in (1, 4):
+        ops.attention_decode_bf16(q.view(1, -1).cuda(), out, k_pages, v_pages, table, _i32([0]), _i32([length - 1]), heads, kv_heads, 64, 0.125, 0, 1, None, waves)
+        scores = torch.einsum("khd,tkd->kht", q.double().view(kv_heads, -1, 64), k[hidden:].double()) * 0.125
+        want = torch.einsum("kht,tkd->khd", scores.softmax(dim=2), v[hidden:].double()).reshape(heads, 64)
+        assert (out.cpu().double().view(heads, 64) - want).abs().max().item() <= 1e-2, waves  # (probabilities and outputs in 16 bits)
+
+
 # the four-wave tiles: their hint to the products, their columns
 FOUR_WAVE_TILES = [(48, 64), (32, 128)]
 
