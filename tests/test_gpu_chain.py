@@ -202,6 +202,42 @@ def test_cuts_of_k(tmp_path, sizes, taken, monkeypatch):
         assert len(got) == 4 and all(torch.equal(a, b) for a, b in zip(got, layers)), batch
 
 
+@pytest.mark.parametrize("sizes", [(2048, 31, 31, 1024), (2048, 32, 32, 1024), (3072, 24, 8, 8192), (1024, 16, 4, 2048)])
+def test_a_single_rows_runs(tmp_path, sizes, monkeypatch):
+    """A row alone, whose runs of keys the output projection's waves add up: the layers' bits on four waves and on eight, in four and eight
+    parts of K, and where the layers round 32 heads' sums on their way in (two, four and eight runs)."""
+    import nnis_amd
+    from nnis_amd.kernels import ops
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    for length in (1100, 2000, 3700):
+        assert ops.decode_plan(1, sizes[2], length, width=sizes[1] * 64)[0] in (2, 4, 8)
+        layers, ran = _streams(str(tmp_path), [length], None, monkeypatch)
+        assert not ran
+        got, ran = _streams(str(tmp_path), [length], "own", monkeypatch)
+        assert ran and len(got) == 4 and all(torch.equal(a, b) for a, b in zip(got, layers)), length
+
+
+@pytest.mark.parametrize("sizes, plans", [
+    ((2048, 32, 4, 1024), ("own", (2, 8), (8, 8))),           # eight waves, 32 heads: in the output projection
+    ((1024, 17, 17, 512), ((2, 4), (4, 4), (8, 4))),          # four waves and more than 16 heads: by a stage of its own
+    ((1024, 32, 8, 512), ((2, 4), (4, 4), (8, 4))),
+    ((1152, 33, 11, 576), ((2, 8), (8, 8))),                  # eight waves and more than 32
+    ((192, 6, 1, 448), ("own", (8, 4), (16, 4))),             # up to eight runs, and more
+])
+def test_a_single_rows_runs_in_other_bits(tmp_path, sizes, plans, monkeypatch):
+    """... and where the launch has bits of its own, as far from 32 bits as the layers' kernels (``test_against_the_layers``)."""
+    import nnis_amd
+
+    nnis_amd.write_random_model(str(tmp_path), _config(*sizes), 3)
+    for length in (1100, 3700):
+        want = _run(str(tmp_path), "float32", [length], None, monkeypatch)[0]
+        layers = _run(str(tmp_path), "bfloat16", [length], None, monkeypatch)[0]
+        for plan in plans:
+            got, ran, _ = _run(str(tmp_path), "bfloat16", [length], plan, monkeypatch)
+            assert ran and (got - want).norm() <= 1.33 * (layers - want).norm(), (length, plan)
+
+
 @pytest.mark.parametrize("counts", [(2,), (16,), (33,), (177,), (600,), (1, 1, 15, 16, 1, 30, 33), (100, 3, 260, 2), (9,) * 20])
 @pytest.mark.parametrize("sizes", SIZES + [(1088, 8, 8, 4160)])  # (eight waves with a second round of down's weights)
 def test_prompts_against_the_layers(tmp_path, sizes, counts, monkeypatch):
