@@ -1187,7 +1187,18 @@ void launch_tiled_kernel(const bf16_t* x, const bf16_t* w, OutT y, int m, int n,
 // 392 tiles are a round of 256 compute units and a half, and take two.  With the last rows in lower tiles they take a round and as much as those
 // need: of 12,480 rows into 2,048 columns 8,192 in 256 tiles of 256 rows and the rest in 216 of 160.  `rounds`: what it comes to in times of a
 // whole tile, by the blocks' times in the order in which compute units are free; a tile costs its rows (lower ones 5% more a row) and
-// its fill and epilogue, `fixed`, measured as 10 us beside 44 at a K of 2,048 and 6 beside 118 at 5,632.
+// its fill and epilogue, `fixed`: measured as 10 us beside 44 at a K of 2,048, to which 450 / K was set, and 6 beside 118 at 5,632, which it makes 9
+// (too much for a long K, to the disadvantage of lower tiles).
+//
+// The model makes about twice as much of them as they give: blocks do not end together, and units without one let the others' clock rise.
+// Products of 300 to 16,000 rows, K 512 to 28,672, 1,024 to 57,344 columns, from a modelled gain of 3% on, lower tiles against none:
+//   results stored, weights below 128 MB: 241 gain 6.1% on average, at least 0.5
+//   ... from 128 to 256 MB: 36 below 8% lie between -4 and 7, 41 from 8% on gain 6.5%, one loses 0.5 and none more
+//   ... from 256 MB on: 52 lie between -11 and 10 (few lower rows read the weights once more, past the memory-side cache)
+//   gated or rotated behind a norm, whose ends are more of a low tile: 50 below 8% lie between -6 and 6 (the least at a K of 512 and 1,024), 145
+//   from 8% on gain 5.7%, two lose 0.1 and 0.4
+//   into the stream: 57 below 8% lie between -4 and 11, 124 from 8% on gain 7.8%, at least 1.2
+// (By these lines 249 products of other sizes gain 6.5, 4.8 and 7.5, 7.5% on average; one stored loses 2, one into a stream of 16,384 channels 3.)
 struct LargeRows {
   int row, height;
   double rounds;
@@ -1205,20 +1216,21 @@ double rounds_of(long long whole, long long lower, double whole_time, double low
     }
   }
 }
-LargeRows large_rows(int m, int col_blocks, int k) {
+LargeRows large_rows(int m, int col_blocks, int k, bool stored) {
   const double fixed = 450.0 / k, whole_time = 1.0 + fixed;
   const long long row_blocks = (m + 255) / 256, tiles = row_blocks * col_blocks;
   LargeRows best = {m, 256, rounds_of(tiles, 0, whole_time, 1.0) / whole_time};
-  const double as_is = best.rounds;
+  const long long weights = 512LL * col_blocks * k;
+  if (weights >= 256LL << 20) return best;
+  const double most_rounds = (stored && weights < 128LL << 20 ? 0.97 : 0.92) * best.rounds;
   const int most = (int)(tiles / 256 * 256 / col_blocks);  // row blocks that whole rounds take
   for (int whole = most; whole >= 0 && whole > most - 4; --whole)
     for (const int height : {128, 160, 192}) {
       const int rest = m - whole * 256;
       if (rest <= 0) continue;
       const long long lower = (long long)((rest + height - 1) / height) * col_blocks;
-      if (whole + lower / col_blocks > 65535) continue;
       const double rounds = rounds_of((long long)whole * col_blocks, lower, whole_time, fixed + 1.05 * height / 256.0) / whole_time;
-      if (rounds < best.rounds && rounds < 0.97 * as_is) best = {whole * 256, height, rounds};
+      if (rounds < best.rounds && rounds < most_rounds) best = {whole * 256, height, rounds};
     }
   return best;
 }
@@ -1238,7 +1250,7 @@ template <int BN, typename OutT>
 int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, int k, int columns, hipStream_t stream) {
   const int col_blocks = (columns + BN - 1) / BN, row_blocks = (m + 255) / 256;
   if constexpr (BN == 256) {
-    const LargeRows rows = large_rows(m, col_blocks, k);
+    const LargeRows rows = large_rows(m, col_blocks, k, std::is_pointer<OutT>::value);
     if (rows.height == 128) launch_large_kernel<128, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
     else if (rows.height == 160) launch_large_kernel<160, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
     else if (rows.height == 192) launch_large_kernel<192, OutT>(x, w, y, m, n, k, col_blocks, rows.row, stream);
@@ -1511,6 +1523,8 @@ extern "C" int nnis_gemm_bf16(const void* x, const void* w, void* y, int y_dtype
 // The tile that the tiled kernel takes for m rows, `columns` weight rows and a depth of k (2: 64 x 128, 3: 64 x 64,
 // 4: 256 x 256, 5: 256 x 192, 6: 128 x 128, 7: 256 x 128, 8: 128 x 192): for tests and tuning.  The second: of a product into the
 // residual stream.
+extern "C" int nnis_gemm_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0); }
+extern "C" int nnis_gemm_residual_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0, true); }
 // Whether a product that a norm prepared takes groups of waves that share K: the rows of their tiles and, times 1,000, the groups; 0: no.
 extern "C" int nnis_gemm_grouped(int m, int columns, int k, size_t workspace_bytes) {
   if (pick_tile(m, columns, k, 0) != 3) return 0;
@@ -1518,14 +1532,13 @@ extern "C" int nnis_gemm_grouped(int m, int columns, int k, size_t workspace_byt
   const int tile = grouped_tile(m, columns, k, parts);
   return tile ? (tile == 9 ? 32 : 64) + 1000 * parts : 0;
 }
-// How rows in tiles of 256 x 256 are cut (large_rows): the height of the lower tiles, 256 for none, and the row that they begin at.
-extern "C" int nnis_gemm_large_height(int m, int columns, int k, int* row) {
-  const LargeRows rows = large_rows(m, (columns + 255) / 256, k);
+// How rows in tiles of 256 x 256 are cut (large_rows; `stored`: of a product whose results are stored as they are, not one into the stream or
+// behind a norm): the height of the lower tiles, 256 for none, and the row that they begin at.
+extern "C" int nnis_gemm_large_height(int m, int columns, int k, int stored, int* row) {
+  const LargeRows rows = large_rows(m, (columns + 255) / 256, k, stored != 0);
   *row = rows.row;
   return rows.height;
 }
-extern "C" int nnis_gemm_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0); }
-extern "C" int nnis_gemm_residual_tile(int m, int columns, int k) { return pick_tile(m, columns, k, 0, true); }
 
 // 1 if nnis_gemm_residual gives these sizes to two blocks a strip (with a workspace of `workspace_bytes` and counts
 // behind it), 0 if to another kernel: for callers and tests that have to know which kernel ran.

@@ -62,7 +62,7 @@ _CORE_SIGNATURES = {
     "nnis_gemm_residual_parts": [_INT, _INT],
     "nnis_gemm_tile": [_INT, _INT, _INT],
     "nnis_gemm_grouped": [_INT, _INT, _INT, _SIZE],
-    "nnis_gemm_large_height": [_INT, _INT, _INT, _VOID],
+    "nnis_gemm_large_height": [_INT, _INT, _INT, _INT, _VOID],
     "nnis_gemm_residual_tile": [_INT, _INT, _INT],
     "nnis_gemm_takes_pair": [_INT, _INT, _INT, _SIZE],
     "nnis_gemm_residual": [_VOID, _VOID, _VOID, _VOID, _INT, _VOID, _VOID, _INT, _INT, _INT, _INT, _VOID, _INT, _VOID, _SIZE, _VOID, _VOID],
@@ -1338,10 +1338,11 @@ def gemm_grouped(m: int, n: int, k: int):
     return (grouped % 1000, grouped // 1000) if grouped else None
 
 
-def gemm_large_rows(m: int, n: int, k: int):
-    """(row, height): the rows of a product in tiles of 256 x 256 from ``row`` on are cut into tiles of ``height`` x 256 (256: none lower)."""
+def gemm_large_rows(m: int, n: int, k: int, stored: bool = True):
+    """(row, height): the rows of a product in tiles of 256 x 256 from ``row`` on are cut into tiles of ``height`` x 256 (256: none lower);
+    ``stored``: of a product whose results are stored as they are, not one into the stream or behind a norm."""
     row = ctypes.c_int()
-    height = core().nnis_gemm_large_height(int(m), int(n), int(k), ctypes.addressof(row))
+    height = core().nnis_gemm_large_height(int(m), int(n), int(k), int(stored), ctypes.addressof(row))
     return row.value, height
 
 

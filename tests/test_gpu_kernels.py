@@ -1997,14 +1997,14 @@ def test_scaled_projection_with_k_in_parts(m, k, hint, columns):
             assert (held_k[page, :, inside] == 7).all() and (held_v[page, :, inside] == 7).all()
 
 
-@pytest.mark.parametrize("m, n, height", [(300, 4096, 128), (2285, 8192, 128), (621, 16384, 160), (2093, 8192, 160), (741, 16384, 192), (2257, 11264, 192)])
-def test_large_tiles_with_lower_ones_behind_them(m, n, height):
+@pytest.mark.parametrize("m, n, height, k", [(300, 4096, 128, 264), (2285, 8192, 128, 264), (621, 16384, 160, 264), (2093, 8192, 160, 264), (741, 16384, 192, 264), (2257, 11264, 192, 264),
+                                             (741, 16384, 192, 520), (5900, 2048, 192, 1032)])
+def test_large_tiles_with_lower_ones_behind_them(m, n, height, k):
     """Rows of a product in tiles of 256 x 256 whose last are cut lower, with every epilogue: the bits of tiles of 64 x 128, which add a sum
     up in the same order, and the parts of the sums of squares."""
     ops = _ops()
     torch.manual_seed(m)
-    k = 264
-    assert ops.gemm_large_rows(m, n, k)[1] == height
+    assert ops.gemm_large_rows(m, n, k)[1] == height and (height != 192 or k == 264 or ops.gemm_large_rows(m, n, k, False)[1] == 192)
     x, weight = torch.randn(m, k).bfloat16().cuda(), ops.pack_weight((torch.randn(n, k) / math.sqrt(k)).bfloat16().cuda())
     ss = (1.0 + torch.rand(1, m)).cuda() * k
     head_dim, kv_heads = 64, 4

@@ -221,3 +221,16 @@ def test_padding_keeps_large_groups_on_the_launch(batch, padded, taken, monkeypa
     monkeypatch.setattr(ops, "chain_takes", lambda *sizes: True)  # (the native side's sizes)
     assert bucket(batch) == padded
     assert (chain_plan(22, padded, 600, 2048, 32, 4, 64, 5632) is not None) == taken
+
+
+@pytest.mark.parametrize("m, n, k, stored, others", [
+    (12480, 2048, 5632, (8192, 160), (8192, 160)), (12480, 2048, 2048, (8192, 160), (8192, 160)), (12480, 2560, 2048, None, None),
+    (9247, 8192, 5632, (8192, 160), None), (4348, 6144, 512, (2560, 192), None),  # 6% by the rule's model: into the stream 3 lost, behind a norm 6
+    (12480, 11264, 2048, (11776, 128), None), (4862, 22016, 3072, None, None),     # 4%: stored 2 gained, and lost of weights beyond 128 MB
+    (1106, 36864, 8192, None, None), (3862, 36864, 8192, None, None), (1388, 28672, 8192, None, None),  # weights beyond 256 MB: losses of 2 to 11%
+    (8255, 3072, 14336, (5376, 160), (5376, 160)), (1568, 16384, 8128, (1024, 160), (1024, 160)), (1568, 16384, 8192, None, None)])
+def test_lower_tiles_behind_large_ones(m, n, k, stored, others):
+    from nnis_amd.kernels import ops
+
+    for kind, want in ((True, stored), (False, others)):
+        assert ops.gemm_large_rows(m, n, k, kind) == (want or (m, 256))
