@@ -1263,14 +1263,17 @@ int launch_tiled_large(const bf16_t* x, const bf16_t* w, OutT y, int m, int n, i
 
 // Groups of waves with a part of K each: 33 to 64 rows of a product that a norm prepared, where tiles of 64 x 64 are so few that their K
 // would go in two or four parts through memory and a kernel of its own (5 us of 11).  The parts and the order of every sum are the same, and
-// so are the bits.  Tiles of 32 x 32 where a compute unit has one at most, else of 64 x 32; K in two parts only up to 48 rows.  Microseconds in
+// so are the bits.  Tiles of 32 x 32 where a compute unit has one at most, else of 64 x 32.  K in two parts only up to 48 rows and 2,304 channels: a
+// unit then loads all of K for 64 + 32 rows where a part of a 64 x 64 tile loads half of it for 64 + 64, and from 2,560 on that is more than the
+// kernel between costs (40 rows, 5,120 columns, K 2,048 / 2,304 / 2,560 / 3,072 / 4,096: 10.6 / 11.3 / 11.9 / 12.8 / 14.7 in parts, 10.2 / 11.1 / 11.9 / 13.7 / 16.9 so;
+// in four parts 4,096 columns gain 1 to 21% as far as a K of 4,096).  Microseconds in
 // parts and so, of 64 / 48 / 33 rows: 2560 x 2048 with the rotation 11.2 / 10.7 / 10.3 and 9.7 / 9.2 / 8.6, 3072 x 1536 10.8 / 10.3 / 9.7 and 8.6 / 8.6 / 7.8,
 // 4096 x 2048 12.2 / 11.6 / 11.0 and 9.9 / 9.5 / 8.8; in two parts 6144 x 2048 13.6 / 12.9 / 12.2 and 13.9 / 12.1 / 11.0, gate/up 8192 x 2048 14.2 / 13.6 / 13.0
 // and 14.1 / 12.9 / 11.7.  Not for products into the stream, whose long K is one unit's to read: 64 x 2048 x 5632 12.5 in parts, 15.9 and 22.0 in
 // tiles of 32 x 32 and 64 x 32.
 constexpr int kGroupedRowsLeast = 33, kGroupedRowsMost = 64;  // (fewer rows are the kernel's for few tokens)
 int grouped_tile(int m, int columns, int k, int parts) {
-  if ((parts != 2 && parts != 4) || m < kGroupedRowsLeast || m > (parts == 2 ? 48 : kGroupedRowsMost) || k > 4096) return 0;
+  if ((parts != 2 && parts != 4) || m < kGroupedRowsLeast || m > (parts == 2 ? 48 : kGroupedRowsMost) || k > (parts == 2 ? 2304 : 4096)) return 0;
   const int strips = (columns + 31) / 32;
   return strips * ((m + 31) / 32) <= 256 ? 9 : strips <= 256 ? 10 : 0;
 }
