@@ -928,8 +928,9 @@ template <int BM, int BN, int BK, int NS, bool SPLIT, typename OutT, int WGM = 2
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                     OutT y, int m, int n, int k, int col_blocks, int ksplit,
                                                                     float* __restrict__ partial) {
-  int row_block, col_block, part;
-  deal_tile<BM>(blockIdx.x, gridDim.x, col_blocks, ksplit, row_block, col_block, part);
+  int row_block, col_block, part, block = blockIdx.x;
+  asm("" : "+s"(block) : "s"(x), "s"(w));  // (the pointers are asked for with the sizes: behind the tile's number 64 rows, 11264 x 2048, gated, 12.6 and not 12.3 us)
+  deal_tile<BM>(block, gridDim.x, col_blocks, ksplit, row_block, col_block, part);
   multiply_tile<BM, BN, BK, NS, SPLIT, OutT, WGM, WGN, false>(x, w, y, m, n, k, row_block * BM, col_block, col_blocks, part, ksplit, partial);
 }
 
