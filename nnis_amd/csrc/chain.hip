@@ -65,7 +65,8 @@ struct ChainArgs {
 // 1.4 us after the last of them was written, where rows side by side take 0.7.  Parts of 36 blocks in one line took a reader 1.2 us more.)
 constexpr int kRowWords = 8;     // of a strip of an operand
 constexpr int kPlainWords = 16;  // ... of the stream
-// a lane's channels in 16 bits, two a word: words[0 .. 1], of which `packed_words` are the lane's (with one channel a lane every other lane has a word)
+// a lane's channels in 16 bits, two a word: four channels are words[0 .. 1], two are words[0]; with one channel a lane words[0] is a word of every other lane,
+// whose neighbour has its second half (what the other lanes make is not stored)
 template <int N>
 __device__ __forceinline__ void pack_row(const Floats<N>& v, unsigned (&words)[2]) {
   if constexpr (N == 1) words[0] = pack2(v[0], of_row<0xb1>(v[0]));

@@ -497,7 +497,7 @@ __device__ __forceinline__ void strip_stage(const ChainArgs32& a, const Exchange
     part = (v[0] * v[0] + v[kEach - 3] * v[kEach - 3]) + (v[kEach - 2] * v[kEach - 2] + v[kEach - 1] * v[kEach - 1]);
   } else {  // the lane's own, then its neighbours' of the same four channels
     part = kEach == 2 ? v[0] * v[0] + v[kEach - 1] * v[kEach - 1] : v[0] * v[0];
-    if constexpr (kEach == 1) part += of_row<0xb1>(part) ;
+    if constexpr (kEach == 1) part += of_row<0xb1>(part);
     part += of_row<kEach == 1 ? 0x4e : 0xb1>(part);
   }
   part = sum_32_apart(sum_16_apart(part));

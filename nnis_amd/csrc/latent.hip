@@ -46,8 +46,7 @@ struct PrepareArgs {
 // weights, each behind the one before.  What does not hang on the sums is asked for before them (the position's page and
 // rotation through three of the trips, beside the row's): 1 token of 192 + 64 channels 10.0 -> 7.5 us.
 // BF16: the rows in 32 bits, the weights, the query latents and the pages in bfloat16.  (A type that is a branch is converted in the branch, so what
-// is loaded there is waited for there.)1 token of 192 + 64 channels
-// 7.8 -> 6.1 us, 1,500 tokens 15.3 -> 13.0.
+// is loaded there is waited for there.)  1 token of 192 + 64 channels 7.8 -> 6.1 us, 1,500 tokens 15.3 -> 13.0.
 template <bool BF16>
 __global__ __launch_bounds__(256) void latent_prepare_kernel(PrepareArgs given) {
   __shared__ float scratch[16];

@@ -903,7 +903,7 @@ __global__ void gla_carry_kernel(GlaArgs a) {
 // the heads, times silu(gate):  y[t, h, :] = o / sqrt(mean(o^2) + eps) * w * silu(g[t, h, :]).  A wave a (token, head).
 // -----------------------------------------------------------------------------
 // KEEP: channels a lane holds (heads of up to 64 * KEEP), asked for with their gates and the weight before the sum is made; 0: one by one,
-// from memory again behind the sum.  BF16: gate, weight and y.8 heads of 256, 1 row 5.0 -> 2.5 us, 1,500 rows 11.3 -> 6.4.
+// from memory again behind the sum.  BF16: gate, weight and y.  8 heads of 256, 1 row 5.0 -> 2.5 us, 1,500 rows 11.3 -> 6.4.
 template <int KEEP, bool BF16>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __restrict__ o, const void* __restrict__ gate, int gate_dtype,
                                                              int gate_stride, const void* __restrict__ weight, int weight_dtype,
@@ -1341,8 +1341,7 @@ struct DeltaArgs {
 };
 
 // KEEP: channels a lane holds (up to 64 * KEEP key channels).  A token's and a head's numbers, and those of the gates, are asked for
-// before the first sum.  BF16: the rows.8 heads of 128, 1 row 5.6 -> 3.4 us,
-// 1,500 rows 11.2 -> 8.1.
+// before the first sum.  BF16: the rows.  8 heads of 128, 1 row 5.6 -> 3.4 us, 1,500 rows 11.2 -> 8.1.
 template <int KEEP, bool BF16>
 __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs a) {
   const int d = a.key_dim, type = BF16 ? NNIS_BF16 : a.dtype;

@@ -394,8 +394,7 @@ __global__ void branch_mean_kernel(BranchArgs a) {
 }
 
 // with a row in registers (as stream_wide_kernel, BF16 likewise): widths in steps of 4 up to 4096 channels.  COUNT branches, whose sums meet
-// in one exchange.Two branches of 2,048
-// channels, 1 to 6 rows 5.2 -> 3.2 us, 1,580 rows 11.7 -> 9.1.
+// in one exchange.  Two branches of 2,048 channels, 1 to 6 rows 5.2 -> 3.2 us, 1,580 rows 11.7 -> 9.1.
 template <int COUNT, bool BF16>
 __global__ __launch_bounds__(1024) void branch_mean_wide_kernel(BranchArgs a) {
   __shared__ float scratch[COUNT][16];
