@@ -737,12 +737,15 @@ def chain_plan(layers: int, batch: int, longest: int, width: int, heads: int, kv
     1,196, batch 12 at 3,000 2,218 and 2,064 and 1,993.
 
     Larger groups have the scores of four heads a wave here and of sixteen there, so other bits, and a seeded draw over other bits picks
-    other tokens: the launch is theirs up to seven rows.  A wave has one page where the blocks are few, two where they are more, and the
+    other tokens: the launch is theirs up to seven rows.  That line is drawn by the bits and not by the times, which halve on both sides of it (32/4
+    heads, 22 layers, sequences of 100 to 700 tokens, 4 / 7 / 8 / 12 / 16 rows 963 / 992 / 1,002 / 1,053 / 1,102 and 499 / 504 / 500 / 513 / 552; of 600 to 2,000
+    1,000 / 1,036 / 1,051 / 1,109 / 1,172 and 512 / 561 / 564 / 637 / 670): a step of a few rows was given the launch when it came, a batch from eight on keeps the
+    tokens that its seeds have drawn so far, until the attention here adds up in the layers' order.  A wave has one page where the blocks are few, two where they are more, and the
     runs stop at 256 blocks (32/4 heads, 22 layers, batch 1 at 700 tokens 943 and 508, batch 4 at 1,500 998 and 546).  In 32 bits a wave's tiles are 16 keys: up to two
     tiles a wave, within 256 blocks: 9/3 heads, 30 layers, batch 1 at 1,000 tokens 1,018 and in 1 / 2 / 4 / 8 runs 900 / 723 / 623 / 590, in
     16 618; batch 8 1,134 and 1,007 / 791 / 675 / 672 and 706; batch 16 1,425 and 1,077 / 857 / 761 / 868.
 
-    (The launch's times are from before the stream's rows lay side by side in its exchange, which took 2 to 20% off them, most where rows
+    (The launch's other times are from before the stream's rows lay side by side in its exchange, which took 2 to 20% off them, most where rows
     are many, whatever the plan: 32/32 heads, batch 8 at 2,000 tokens 1,126 -> 1,057; 32/4 heads, batch 1 at 700 503 -> 476, batch 4 at 1,500 558 -> 513;
     in 32 bits 9/3 heads, batch 1 / 8 / 16 at 1,000 598 / 681 / 772 -> 542 / 607 / 663.)"""
     # two tiles of rows where the layers' products are those of few rows, a tile at a time (weights of up to 8 MB)
